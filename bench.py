@@ -87,7 +87,7 @@ def exl3_experts(torch, synth_device, seed, kb):
 def exl3_round(torch, sz, synth, synth_device, stream, L, rates, tag, mode=0):
     w = Workload()
     sess = sz.Session(HIDDEN, FF, NE, TOPK, L, VOCAB, 8)
-    sess.set_expert_mode(mode)   # 0: the exact kernels (the default); 1, 2: the matrix-core launches
+    sess.set_expert_mode(mode)   # every mode runs the exact launches
     layers = []
     for l, kb in enumerate(rates):
         buf, stride, gap = exl3_experts(torch, synth_device, 1000 + l, kb)
@@ -135,13 +135,14 @@ def exl3_round(torch, sz, synth, synth_device, stream, L, rates, tag, mode=0):
     moe_bytes = sum((len(sel[l]) + 1) * ebytes[rates[l]] for l in range(L))
     n_sel = {kb: float(np.mean([len(sel[l]) + 1 for l in range(L) if rates[l] == kb])) if kb in rates else 0.0 for kb in (2, 3, 4)}
     pairs = ROWS * (TOPK + 1)                                       # (token, expert) work items, the shared expert included
-    act_gu = ROWS * (HIDDEN + NE) * 4 + pairs * 2 * FF * 2 * 4     # u and logits in; two split-K partials of gate and up out
-    act_dn = pairs * 2 * FF * 2 * 4 + pairs * HIDDEN * 4           # those partials in; one down output per pair out
+    zs = HIDDEN // 512
+    act_gu = ROWS * (HIDDEN + NE) * 4 + pairs * 2 * FF * zs * 4    # u and logits in; a sum for every 512 inputs of gate and up out
+    act_dn = pairs * 2 * FF * zs * 4 + pairs * HIDDEN * 4          # those sums in; one down output per pair out
     w.kernel_bytes = {n: head_bytes + ROWS * HIDDEN * 4 for n in ("head_q8_0_argmax", "head_q8_0_argmax_mfma", "head_q8_0_argmax_mfma_n8")}
     for kb in (2, 3, 4):
-        for form in ("exl3", "mma_exl3", "mmaw_exl3", "lin_exl3", "linw_exl3", "exl3f"):      # the exact launches, the matrix-core ones and the f16-input ones (sz_session_set_expert_mode)
-            w.kernel_bytes["verify_gate_up_%s_%d" % (form, kb)] = n_sel[kb] * gu_bytes[kb] + act_gu
-            w.kernel_bytes["verify_down_%s_%d" % (form, kb)] = n_sel[kb] * dn_bytes[kb] + act_dn
+        for form in ("", "t2_", "t4_", "w_", "t2w_", "t4w_"):      # a launch carries all layers of its rate
+            w.kernel_bytes["verify_gate_up_%sexl3_%d" % (form, kb)] = rates.count(kb) * (n_sel[kb] * gu_bytes[kb] + act_gu)
+            w.kernel_bytes["verify_down_%sexl3_%d" % (form, kb)] = rates.count(kb) * (n_sel[kb] * dn_bytes[kb] + act_dn)
     w.step, w.check, w.set_eager = step, check, (lambda eager: sess.set_graph(not eager))
     w.step_bytes = moe_bytes + head_bytes + act_bytes
     w.counters_key = "config5" if (L == 48 and tag == "config 5" and ROWS == 4) else ("config3" if (tag == "config 3" and ROWS == 4) else None)
@@ -154,8 +155,7 @@ def exl3_round(torch, sz, synth, synth_device, stream, L, rates, tag, mode=0):
                   "layers": L, "rows": ROWS, "resident_GB": round(sum(b.numel() for b, _, _ in layers) / 1e9 + head.numel() / 1e9, 2)}
     w.describe["expert_layout"] = "every trellis on a 128-byte line (sz_layer_spacing)" if SPACED else "contiguous [gate|up|down]"
     if mode:
-        w.describe["expert_mode"] = {1: "matrix cores, the codebook's f16 values", 2: "matrix cores, the linearised codebook",
-                                     3: "the exact decode, inputs rounded to f16, two products an instruction"}[mode]
+        w.describe["expert_mode"] = mode
     w.extra = {"accepted_drafts": wrong}
     w.cpu = ("exl3_token", (layers[0], rates[0], rl_h[0], u[0].cpu().numpy(), sgl[0].cpu().numpy()))
     w.keep = (sess, layers, head, u, rl, sgl, hu, y, out, drafts)

@@ -181,17 +181,10 @@ uint32_t sz_exl3_head_lds_bytes(int32_t type, uint32_t hidden, uint32_t m);
  * values are the exact head's bit for bit, but an output outside the chosen blocks cannot appear.  sz_head_argmax,
  * sz_head_logits and sz_verify_round never use it.  k_blk = 0 turns it off again. */
 int32_t sz_session_set_head_proxy(sz_session*, uint32_t k_blk);
-/* How a layer of EXL3 experts at a whole bit rate multiplies in sz_moe_layer_verify, sz_moe_block_verify and sz_verify_round
- * (the reference's choice between its exact kernels and mma_grouped_exl3_K, kernels/exl3.cu:682-725, which `--exact` and
- * `tensor_prompt` make, session.rs:1741, 1817): 0, the default, the exact kernels (every weight the codebook's f16, f32
- * multiply-adds in input order, a work item a (token, expert) pair); 1 the matrix cores on the codebook's own f16 values, a
- * work item a distinct expert with its tokens on the rows of the matrix instruction (only the order of the f32 additions and
- * the 22 bits kept of an input differ); 2 the matrix cores on the linearised codebook (a weight's rounding to f16 is skipped:
- * outputs within 1e-3 relative L2 of the exact ones, about 4e-4 measured); 3 the exact kernels' launches and decode with
- * the rotated inputs rounded to f16, two products an instruction (about 4e-4 as well).  Routing ids, their order and the
- * weights are the same bits in every mode.  Half-integer rates always take the exact kernels.  On an MI355X modes 1 and 2 are
- * slower than the exact kernels for batches of up to 8 rows and mode 3 is 1.5 % faster.  Environment SHADOWZERO_EXPERT_MODE
- * sets a new session's mode. */
+/* The reference chooses between exact and tensor-core kernels for EXL3 experts (mma_grouped_exl3_K, kernels/exl3.cu:682-725,
+ * `--exact` and `tensor_prompt`, session.rs:1741, 1817).  Modes 0 to 3 are accepted and all run the same launches: the
+ * codebook's own f16 weights against all 24 bits of the inputs on the matrix cores, f32 sums, which is the fastest form on an
+ * MI355X as well as the exact one.  (Modes 1 to 3 once chose forms that kept fewer bits.) */
 int32_t sz_session_set_expert_mode(sz_session*, int32_t mode);
 /* 0: sz_verify_round launches its kernels one by one instead of replaying a captured graph (default 1). */
 int32_t sz_session_set_graph(sz_session*, int32_t enabled);
@@ -278,7 +271,7 @@ typedef struct sz_hc sz_hc;
 sz_hc* sz_hc_new(const sz_hc_config*);           /* resident weights by address; allocates the read's buffers */
 void sz_hc_free(sz_hc*);
 /* u[m][hidden] = the sublayer's input from the residual streams r[m][streams * hidden]; the per-stream gains of the write
- * that follows land in the handle's g[max_rows][streams] (sz_hc_gains).  Four launches: norm, down + inject, up, mix. */
+ * that follows land in the handle's g[max_rows][streams] (sz_hc_gains).  Two launches: norm + down + inject, up + mix. */
 int32_t sz_hc_read(sz_hc*, uint32_t m, uint64_t r, uint64_t u, uint64_t stream);
 uint64_t sz_hc_gains(sz_hc*);
 /* r[j][s * hidden + i] += g[j][s] * y[j][i]. */

@@ -509,7 +509,7 @@ class Session:
         check(lib().sz_session_set_graph(self._h, int(enabled)))
 
     def set_expert_mode(self, mode):
-        """0 (default): the exact EXL3 layer kernels, 1: the matrix cores on the codebook's f16 values, 2: on the linearised codebook."""
+        """0 to 3 are accepted; all run the exact EXL3 launches, which are the fastest."""
         check(lib().sz_session_set_expert_mode(self._h, int(mode)))
 
     def buffer(self, which):

@@ -1,6 +1,7 @@
 // The host side of the verify path above the kernels: Backend::matvec, the device entry points, and the session's MoE /
 // head / acceptance operations.  Mirrors the hot subset of crates/shadowzero-cuda/src/{backend.rs,session.rs}.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -57,14 +58,19 @@ uint32_t rows_per_block(const Format& f, uint32_t cols, uint32_t cap, uint32_t l
     return rpb;
 }
 
-// Workgroups and dynamic LDS of the unquantized-matrix kernels (dense_group in kernels/matvec.hip): a workgroup a row when
-// the rows are longer than 2048, else one for every 4 to 32 rows with the inputs staged in LDS.
-uint32_t dense_groups(uint64_t rows, uint64_t cols) {
-    if (cols > 2048) return (uint32_t) rows;
-    const uint64_t per = 4 * std::min<uint64_t>(8, std::max<uint64_t>(1, rows / 1024));   // dense_rpw
-    return (uint32_t) ((rows + per - 1) / per);
+// How the unquantized-matrix kernels split a row of `cols` columns (dense_waves and dense_lanes in kernels/matvec.hip): waves a
+// row, threads a workgroup and rows a workgroup takes at a time; the kernels' variant for m inputs; their type code.
+struct DenseShape {
+    uint32_t waves, block, pass;
+};
+DenseShape dense_shape(uint64_t cols) {
+    uint32_t g = 64;
+    while (g > 1 && (uint64_t) (g / 2) * 16 >= cols) g /= 2;
+    const uint32_t waves = (uint32_t) std::min<uint64_t>(8, (cols + 1023) / 1024), block = 64 * std::max<uint32_t>(4, waves);
+    return {waves, block, block / 64 / waves * (64 / g)};
 }
-uint32_t dense_lds(uint64_t cols, uint32_t m) { return cols > 2048 ? 128u : (uint32_t) (m * cols * 4); }
+const char* dense_m(uint32_t m) { return m == 1 ? "1" : m <= 4 ? "4" : "8"; }
+uint32_t dense_code(int ty) { return ty == SZ_TYPE_F32 ? 0 : ty == SZ_TYPE_F16 ? 1 : 2; }
 
 // Workgroups of a kernel that loops over its work (the head): a few per compute unit of the MI355X's 256.
 uint32_t persistent_groups() {
@@ -137,9 +143,12 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
     if (f.dense) {
         if (rows == 0) return 0;
         if (cols % 4 || (x & 15) || xs % 4 || (w & (4 * f.bb - 1))) return fail("matvec_cols: unquantized matrices need columns in fours and aligned rows");
-        const std::string kn = "matvec_cols_" + tag;
-        const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m)};
-        return launch(kn.c_str(), dense_groups(rows, cols), 1, 1, 256, dense_lds(cols, m), stream, a);
+        // several passes a workgroup once there are more than about 1024 of them: the inputs stay in its registers
+        const DenseShape d = dense_shape(cols);
+        const uint32_t np = (uint32_t) std::min<uint64_t>(16, std::max<uint64_t>(1, rows / (1024ull * d.pass)));
+        const std::string kn = std::string("matvec_cols_dense_m") + dense_m(m);
+        const sz_arg a[] = {U32(dense_code(ty)), P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m), U32(np)};
+        return launch(kn.c_str(), (uint32_t) ((rows + (uint64_t) d.pass * np - 1) / ((uint64_t) d.pass * np)), 1, 1, d.block, 0, stream, a);
     }
     if (cols % f.qk) return fail("matvec_cols: columns are not whole blocks");
     // fewer rows a workgroup where the launch would otherwise have under about 512 workgroups (two a CU)
@@ -290,24 +299,24 @@ int32_t sz_matvec_cols(int32_t ty, uint64_t w, uint64_t cols, uint64_t rows, uin
 
 }   // extern "C"
 
-// One matrix of a matvec_cols_multi launch (DenseJob of kernels/matvec.hip).
-struct DenseJob {
-    uint64_t w, y;
-    uint32_t ys, rows, type, first, act;
-    float div;
-};
-static_assert(sizeof(DenseJob) == 40, "the kernel reads this layout");
-
 // ---- B2: the session ----------------------------------------------------------------------------------------------------
 struct SzLayer {
     int type = 0, shared_type = 0;
     uint64_t experts = 0, stride = 0, shared = 0;
     uint64_t gap = 0; // bytes between an expert's projections (0: the reference's contiguous [gate|up|down])
     DevBuf eaddr;     // u64[3 * ne] then u64[3] for the shared expert
-    DevBuf jobs;      // the router launch's job table (set_router)
-    uint32_t router_groups = 0;
+    uint64_t router = 0, gate = 0;   // the router and the shared expert's gate row (set_router; gate 0: none)
+    int router_type = 0, gate_type = 0;
+    uint32_t vpos = 0;   // an EXL3 layer's place in the session's table of them
     bool set = false;
 };
+
+// An EXL3 layer as the verify launches see it (VerifyLayer of kernels/exl3.hip).
+struct VerifyLayer {
+    uint64_t experts, stride, shared;
+    uint32_t part, layer;
+};
+static_assert(sizeof(VerifyLayer) == 32, "the kernels read this layout");
 
 struct SzGraphKey {
     uint64_t v[10];
@@ -321,8 +330,11 @@ struct sz_session {
     uint64_t head_w = 0;
     // batch buffers (session.rs `bb`): the plan, the expert products, the split-k partials, the head's scratch
     DevBuf plan, eg, act, eo, part, dn, head_part, logits, topv, topi, ids;
-    DevBuf plans;                 // a plan a layer for the rounds that route every layer up front (sz_verify_round)
+    DevBuf plans;                 // a plan a layer for the rounds (sz_verify_round)
     uint32_t plan_stride = 0;
+    std::vector<VerifyLayer> vtab;   // the EXL3 layers that are set, by type and then in order; its copy on the device
+    DevBuf vtab_dev;
+    uint32_t vchunk = 1;             // EXL3 layers that `part` and `dn` hold at a time
     DevBuf head_xa, head_inv;   // an EXL3 head's rotated inputs as f16 high and low parts (16 rows of 128 a 128-block), and the tokens' scales
     DevBuf rl, sgl;   // the router's outputs for a batch: f32[max_rows][n_expert], f32[max_rows]
     // the optional 2-bit screen of an EXL3 head (HeadProxy of session.rs:428-441): k_blk = 0 is off
@@ -335,10 +347,6 @@ struct sz_session {
     } pf;   // the prefill chunk's buffers, grown on demand
     void* top_host = nullptr;  // pinned host memory the top-64 merge writes to directly (8 rows of 128 words): no copy back
     bool last_fused = false;   // the last layer call left its routing in the fused layout [tidx | w | cnt]
-    // how an EXL3 layer at a whole bit rate multiplies (sz_session_set_expert_mode): 0 the exact kernels, a weight at a time on
-    // the vector unit; 1 the matrix cores with the codebook's own f16 values; 2 the matrix cores with the linearised codebook
-    int expert_mode = 0;
-    DevBuf plan2;              // a round's layers alternate between two plans: the sum of a layer rides the next layer's first launch, which writes that layer's routing
     uint64_t last_plan = 0;    // the plan the last layer call left its routing in
     std::map<SzGraphKey, uint64_t> graphs;
     // plan offsets for the largest batch
@@ -367,47 +375,81 @@ PlanLayout plan_layout(uint32_t m, uint32_t k) {
     return p;
 }
 
-// The matrix-core EXL3 layer's plan behind [tidx | w | cnt] (verify_plan_exl3 in kernels/exl3.hip): byte offset of the item
-// list, item slots (one a pair plus the shared expert's, an even number), bytes of the whole.
-struct MmaPlan {
+// An EXL3 layer's plan behind [tidx | w | cnt] (verify_plan_exl3 in kernels/exl3.hip): byte offset of the item list, item
+// slots (a layer has at most one item a pair plus the shared expert's: the last slot is never an item), bytes of the whole.
+struct VerifyPlan {
     uint32_t ioff, slots, bytes;
 };
-MmaPlan mma_plan(uint32_t m, uint32_t k) {
-    MmaPlan p{};
+VerifyPlan verify_plan(uint32_t m, uint32_t k) {
+    VerifyPlan p{};
     p.ioff = (uint32_t) align16(2ull * m * k * 4 + m * 4);
-    p.slots = (m * k + 3) & ~1u;   // at least one more than the most items there can be: the last slot is never an item
+    p.slots = m * k + 2;
     p.bytes = p.ioff + 16 + p.slots * 32;
     return p;
 }
-// Dynamic LDS of its two product launches: EXL3_MMA_LDS_WORDS there (a 4-row ring, the A rows and the scales of 4 waves).
-uint32_t mma_lds_bytes(int bits, uint32_t nmax) {
-    const uint32_t stride = (bits == 3 || bits == 4) ? 4 : (uint32_t) bits;
-    const uint32_t ring = 4 * 64 * stride;
-    return 4 * (4 * (ring + nmax * 128 + 64 + 16) + 64);
+// What the verify launches leave for one EXL3 layer: launch 2's sums (an f32 for every pair, projection, 512 inputs and ff
+// column) and launch 3's.
+uint64_t verify_part_bytes(const sz_session_config& c, uint32_t m) { return 2ull * m * (c.top_k + 1) * exl3_ksplit(c.hidden) * c.ff * 4; }
+uint64_t verify_dn_bytes(const sz_session_config& c, uint32_t m) { return (uint64_t) m * (c.top_k + 1) * exl3_ksplit(c.ff) * c.hidden * 4; }
+
+// The variant of a verify launch over `cols` output columns: column tiles a wave and the kernel name's prefix.  `waves8` is the
+// number of waves that 8 tiles a wave would give: they do least work for their A rows (a round of 48 layers 931 us, with 4 tiles
+// 957, with 2 1033) but leave SIMDs idle where there are few of them (a layer alone at 4 rows: 51 us with 2 tiles, 63 with 8).
+const char* verify_variant(uint64_t cols, uint64_t waves8, uint32_t m, uint32_t* ct) {
+    *ct = cols % 512 == 0 && waves8 >= 8192 ? 8 : waves8 >= 2048 ? 4 : 2;
+    if (m > 4) return *ct == 8 ? "w_" : *ct == 4 ? "t4w_" : "t2w_";
+    return *ct == 8 ? "" : *ct == 4 ? "t4_" : "t2_";
 }
 
-// The rank-order sum of an EXL3 layer that has not been launched yet: inside sz_verify_round it rides the first launch of
-// the layer after it (whose routing goes to the session's other plan buffer), and the last layer's gets a launch of its own.
-struct PendingSum {
-    bool active = false;
-    uint64_t plan = 0, sgl = 0, y = 0;
-    bool shared = false;
-    // the round's routing launch (verify_route_layers) has filled a plan a layer, `plan_stride` apart from `plans` on: the
-    // exact EXL3 launches of those layers get no logits and read their plan instead of redoing the selection
-    uint64_t plans = 0;
-    uint32_t plan_stride = 0;
-};
-
-int launch_pending_sum(sz_session* s, PendingSum& ps, uint32_t m, uint64_t stream) {
-    if (!ps.active) return 0;
+// The EXL3 layers table[p0 .. p1) for a batch of m rows: u, rl, sgl, y and `plans` are the caller's, layer `base`'s part first.
+int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t plans, uint64_t stream) {
     const sz_session_config& c = s->cfg;
-    ps.active = false;
-    const sz_arg a[] = {P(s->dn.ptr), U64(0), U64(0), U64(ps.shared ? 1 : 0), U32(0), P(ps.plan), P(ps.sgl), P(ps.y),
-                        U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(0)};
-    return launch("verify_combine_exl3", c.hidden / 128, m, 1, 128, 0, stream, a);
+    const VerifyPlan vp = verify_plan(m, c.top_k);
+    const uint32_t zs = exl3_ksplit(c.hidden), zd = exl3_ksplit(c.ff);
+    const bool one = p1 - p0 == 1;   // a single layer's addresses go along as kernel arguments, not through the table
+    auto table = [&](uint32_t p) { return one ? 0 : s->vtab_dev.ptr + (uint64_t) p * sizeof(VerifyLayer); };
+    const VerifyLayer& V = s->vtab[p0];
+    // Layer by layer, tokens that share an expert are worth a launch that finds them only where they are many: about 6 us and
+    // a boundary, against the decode of a fifth of the pairs (measured at 4 rows of top-10 of 512, where they are one in twenty:
+    // 46 us a layer with the plan, 41 without).  A round's plans are one launch for all layers.
+    const double pairs = (double) m * c.top_k, distinct = c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) m));
+    const bool by_pair = one && distinct > 0.8 * pairs;
+    const uint32_t ioff = by_pair ? 0 : vp.ioff, slots = by_pair ? m * c.top_k + 1 : vp.slots;
+    if (!by_pair) {
+        const sz_arg a[] = {P(rl), P(plans), U32(s->plan_stride), U32(vp.ioff), P(table(p0)), U64(V.shared), U32(base), U32(c.n_expert), U32(c.top_k), U32(m)};
+        if (launch("verify_plan_exl3", p1 - p0, 1, 1, 64 * m, 0, stream, a)) return 1;
+    }
+    for (uint32_t q0 = p0; q0 < p1; q0 += s->vchunk) {
+        const uint32_t q1 = std::min(p1, q0 + s->vchunk);
+        for (uint32_t r0 = q0, r1; r0 < q1; r0 = r1) {   // runs of one type
+            const int ty = s->layers[s->vtab[r0].layer].type;
+            for (r1 = r0 + 1; r1 < q1 && s->layers[s->vtab[r1].layer].type == ty;) r1++;
+            Format f;
+            std::string tag;
+            format_of(ty, f, tag);
+            const uint32_t nl = r1 - r0;
+            const uint64_t part = s->part.ptr + (r0 - q0) * verify_part_bytes(c, m), dn = s->dn.ptr + (r0 - q0) * verify_dn_bytes(c, m);
+            uint32_t ct;
+            {
+                const std::string kn = std::string("verify_gate_up_") + verify_variant(c.ff, 2ull * nl * slots * zs * (c.ff / 128), m, &ct) + tag;
+                const sz_arg a[] = {P(rl), P(table(r0)), U64(V.experts), U64(V.stride), U64(V.shared), U32(V.part), U32(base), P(plans), P(plans), U32(s->plan_stride), U32(ioff), P(u), P(part), U32(c.n_expert), U32(c.top_k),
+                                    U32(m), U32(c.hidden), U32(c.ff)};
+                if (launch(kn.c_str(), c.ff / (64 * ct), 2 * slots, nl * zs, 256, 0, stream, a)) return 1;
+            }
+            {
+                const std::string kn = std::string("verify_down_") + verify_variant(c.hidden, (uint64_t) nl * slots * zd * (c.hidden / 128), m, &ct) + tag;
+                const sz_arg a[] = {P(rl), P(table(r0)), U64(V.experts), U64(V.stride), U64(V.shared), U32(V.part), U32(base), P(plans), P(plans), U32(s->plan_stride), U32(ioff), P(part), P(dn),
+                                    U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff)};
+                if (launch(kn.c_str(), c.hidden / (64 * ct), slots, nl * zd, 256, 0, stream, a)) return 1;
+            }
+        }
+        const sz_arg a[] = {P(s->dn.ptr), P(table(q0)), U64(V.experts), U64(V.stride), U64(V.shared), U32(V.part), U32(base), P(plans), U32(s->plan_stride), P(sgl), P(y), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff)};
+        if (launch("verify_combine_exl3", c.hidden / 128, m, q1 - q0, 64 * std::min<uint32_t>(16, c.top_k + 1), 0, stream, a)) return 1;
+    }
+    return 0;
 }
 
-int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t stream, PendingSum* ride = nullptr) {
+int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t stream) {
     const sz_session_config& c = s->cfg;
     if (l >= s->layers.size() || !s->layers[l].set) return fail("sz_moe_layer_verify: layer " + std::to_string(l) + " has no experts set");
     if (m == 0 || m > c.max_rows) return fail("sz_moe_layer_verify: " + std::to_string(m) + " rows (1.." + std::to_string(c.max_rows) + ")");
@@ -419,87 +461,17 @@ int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, ui
     const bool shared = L.shared != 0;
     if (shared && L.shared_type != L.type) return fail("the shared expert must have the routed experts' type (layer " + std::to_string(l) + ")");
     const PlanLayout p = plan_layout(m, c.top_k);
-    // a layer whose sum may ride the next launch takes the plan buffer the pending sum is not reading; a layer routed by the
-    // round's routing launch has a plan of its own
-    const bool f16x = s->expert_mode == 3 && f.exl3 && !f.half;   // the exact launches with f16 inputs and two products an instruction
-    const bool routed = ride && ride->plans && f.exl3 && (s->expert_mode == 0 || s->expert_mode == 3);
-    const uint64_t plan = routed ? ride->plans + (uint64_t) l * ride->plan_stride
-                                 : (ride && ride->active && ride->plan == s->plan.ptr) ? s->plan2.ptr : s->plan.ptr;
+    const uint64_t plan = s->plan.ptr;
     s->last_plan = plan;
+    if (f.exl3) {
+        s->last_fused = true;
+        return verify_layers(s, L.vpos, L.vpos + 1, l, m, u, rl, sgl, y, plan, stream);
+    }
     const uint64_t addr = plan + p.a0, rec = plan + p.r0, wts = plan + p.w_off, cnt = plan + p.counts_off;
     const uint64_t addr_d = addr + 2ull * p.GT * 8, rec_d = rec + 2ull * p.GT * 17 * 4;
     const std::string kn = "matvec_grouped_" + tag;
-    if (ride && ride->active && !f.exl3 && launch_pending_sum(s, *ride, m, stream)) return 1;   // only an EXL3 layer's first launch carries a sum
-    // the sum of the layer before, if it rides this layer's first launch: the workgroups it adds, its arguments
-    const bool carry = f.exl3 && ride && ride->active;
-    const uint32_t carry_groups = carry ? c.hidden / 128 * m : 0;
-    const uint64_t c_plan = carry ? ride->plan : 0, c_sgl = carry ? ride->sgl : 0, c_y = carry ? ride->y : 0;
-    const uint32_t c_mode = carry ? (ride->shared ? 2 : 1) : 0;
-    // this layer's own sum: left for the next launch to carry when the caller takes care of it (launch 2 must have finished the blocks)
-    auto sum = [&](uint32_t zs_d, uint64_t part) -> int {
-        if (ride) ride->active = false;
-        s->last_fused = true;
-        if (ride && zs_d == 1) {
-            ride->active = true;
-            ride->plan = plan;
-            ride->sgl = sgl;
-            ride->y = y;
-            ride->shared = shared;
-            return 0;
-        }
-        const sz_arg a[] = {P(s->dn.ptr), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), P(sgl), P(y),
-                            U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(zs_d == 1 ? 0 : zs_d)};
-        return launch("verify_combine_exl3", c.hidden / 128, m, 1, zs_d == 1 ? 128 : 1024, 0, stream, a);   // zs_d == 1: launch 2 finished the blocks
-    };
-    if (f.exl3 && !f.half && (s->expert_mode == 1 || s->expert_mode == 2)) {
-        // the matrix-core layer: a plan of the batch's distinct experts, then gate/up and down with an item's tokens on the rows
-        // of the matrix instruction, then the rank-order sum (kernels/exl3.hip, "the verify layer on the matrix cores")
-        const MmaPlan mp = mma_plan(m, c.top_k);
-        const uint32_t zs_gu = (c.hidden / 128 + 3) / 4, zs_d = exl3_ksplit(c.ff);
-        const uint64_t part = matrix_bytes(f, c.hidden, c.ff) + L.gap;   // from one projection of an expert to the next
-        if (part >> 32) return fail("sz_moe_layer_verify: a projection of 4 GiB or more");
-        const uint32_t nmax = m > 4 ? 8 : 4;
-        const uint32_t lds = mma_lds_bytes(f.bits, nmax);
-        const std::string variant = std::string(s->expert_mode == 2 ? "lin" : "mma") + (nmax == 8 ? "w" : "");
-        const std::string k1 = "verify_gate_up_" + variant + "_" + tag, k2 = "verify_down_" + variant + "_" + tag;
-        {
-            const sz_arg a[] = {P(rl), P(plan), U32(mp.ioff), U32(c.n_expert), U32(c.top_k), U32(m), U32(shared ? 1 : 0), U32(c.hidden),
-                                P(s->dn.ptr), P(c_plan), P(c_sgl), P(c_y), U32(c_mode)};
-            if (launch("verify_plan_exl3", 1 + carry_groups, 1, 1, 64 * m, 0, stream, a)) return 1;
-        }
-        {
-            const sz_arg a[] = {P(rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(u), P(plan), U32(mp.ioff), P(s->part.ptr),
-                                U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff)};
-            if (launch(k1.c_str(), c.ff / 128, 2 * mp.slots, zs_gu, 256, lds, stream, a)) return 1;
-        }
-        {
-            const sz_arg a[] = {U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), U32(mp.ioff), P(s->part.ptr), P(s->dn.ptr),
-                                U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(zs_gu)};
-            if (launch(k2.c_str(), c.hidden / 128, mp.slots, zs_d, 256, lds, stream, a)) return 1;
-        }
-        return sum(zs_d, part);
-    } else if (f.exl3) {
-        // the fused layer: three launches, the work items are the (token, rank) pairs themselves, no plan.  A wave of
-        // launch 1 takes one 128-block of the input, 4 waves a workgroup (EXL3_GU_WAVES, EXL3_VERIFY_NB in kernels/exl3.hip).
-        const uint32_t S = p.G + m, zs_gu = (c.hidden / 128 + 3) / 4, zs_d = exl3_ksplit(c.ff);
-        const uint64_t part = matrix_bytes(f, c.hidden, c.ff) + L.gap;   // from one projection of an expert to the next
-        if (part >> 32) return fail("sz_moe_layer_verify: a projection of 4 GiB or more");
-        const std::string ftag = f16x ? "exl3f_" + std::to_string(f.bits) : tag;
-        const std::string k1 = "verify_gate_up_" + ftag, k2 = "verify_down_" + ftag;
-        {
-            const uint32_t gx = c.ff / 128, extra = (carry_groups + gx * zs_gu - 1) / (gx * zs_gu);   // rows of the grid for a riding sum
-            const sz_arg a[] = {P(routed ? 0 : rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(u), P(plan), P(s->part.ptr),
-                                U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), P(s->dn.ptr), P(c_plan), P(c_sgl), P(c_y), U32(c_mode)};
-            if (launch(k1.c_str(), gx, 2 * S + extra, zs_gu, 256, 0, stream, a)) return 1;   // 4 waves of one 128-block each: EXL3_GU_WAVES, EXL3_VERIFY_NB
-        }
-        {
-            const sz_arg a[] = {P(routed ? 0 : rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), P(s->part.ptr), P(s->dn.ptr),
-                                U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(zs_gu)};
-            if (launch(k2.c_str(), c.hidden / 128, S, zs_d, 256, 0, stream, a)) return 1;
-        }
-        return sum(zs_d, part);
-    } else if (!std::getenv("SHADOWZERO_GGUF_PLANNED") && c.ff <= 4096) {
-        // the pair form, as the EXL3 layer: routing inside launch 1, SwiGLU inside launch 2, no plan
+    if (!std::getenv("SHADOWZERO_GGUF_PLANNED") && c.ff <= 4096) {
+        // the pair form: routing inside launch 1, SwiGLU inside launch 2, no plan
         const uint32_t S = p.G + m;
         // (one row has few pairs to hand out: 16 and 32 rows a workgroup fill the chip better than 32 and 64, which win from two rows on: measured)
         const uint32_t rpb_gu = rows_per_block(f, c.hidden, m == 1 ? 16 : 32, m == 1 ? 16384 : 32768);
@@ -772,18 +744,13 @@ sz_session* sz_session_new(const sz_session_config* cfg) {
     sz_session* s = new sz_session();
     s->cfg = c;
     s->layers.resize(c.n_layers);
-    if (const char* e = std::getenv("SHADOWZERO_EXPERT_MODE")) s->expert_mode = std::min(3, std::max(0, std::atoi(e)));
     const PlanLayout p = plan_layout(c.max_rows, c.top_k);
     s->GT_max = p.GT;
-    const uint64_t ks_gu = exl3_ksplit(c.hidden), ks_d = exl3_ksplit(c.ff);
-    const uint64_t part = std::max<uint64_t>(2ull * p.GT * ks_gu * 4 * c.ff, (uint64_t) p.GT * ks_d * 4 * c.hidden) * 4;
     const uint64_t nparts = c.vocab / 4 + 1;
-    bool bad = s->plan.need(std::max(p.bytes, mma_plan(c.max_rows, c.top_k).bytes)) || s->plan2.need(std::max(p.bytes, mma_plan(c.max_rows, c.top_k).bytes)) || s->eg.need(2ull * p.R * c.ff * 4) || s->act.need((uint64_t) p.R * c.ff * 4) ||
-               s->eo.need((uint64_t) p.R * c.hidden * 4) || s->part.need(part) || s->ids.need(64) ||
-               s->dn.need((uint64_t) p.GT * ks_d * 4 * c.hidden * 4);
+    s->plan_stride = (verify_plan(c.max_rows, c.top_k).bytes + 255) & ~255u;
+    bool bad = s->plan.need(std::max(p.bytes, s->plan_stride)) || s->eg.need(2ull * p.R * c.ff * 4) || s->act.need((uint64_t) p.R * c.ff * 4) ||
+               s->eo.need((uint64_t) p.R * c.hidden * 4) || s->ids.need(64);
     if (c.vocab) bad = bad || s->head_part.need(nparts * 4 * 2 * 4);
-    s->plan_stride = (uint32_t) ((2ull * c.max_rows * c.top_k * 4 + c.max_rows * 4 + 255) & ~255ull);
-    if (c.n_layers) bad = bad || s->plans.need((uint64_t) c.n_layers * s->plan_stride);
     if (bad) {
         delete s;
         return nullptr;
@@ -796,6 +763,24 @@ void sz_session_free(sz_session* s) {
     if (s->top_host) hip().hipHostFree(s->top_host);
     for (auto& g : s->graphs) sz_graph_destroy(g.second);
     delete s;
+}
+
+// The table of the EXL3 layers that are set, rebuilt and copied to the device.
+static int verify_table(sz_session* s) {
+    std::vector<uint32_t> order;
+    for (uint32_t l = 0; l < s->layers.size(); l++)
+        if (s->layers[l].set && s->layers[l].type > 1020) order.push_back(l);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return s->layers[a].type < s->layers[b].type; });
+    s->vtab.clear();
+    for (uint32_t l : order) {
+        SzLayer& L = s->layers[l];
+        Format f;
+        std::string tag;
+        format_of(L.type, f, tag);
+        L.vpos = (uint32_t) s->vtab.size();
+        s->vtab.push_back({L.experts, L.stride, L.shared, (uint32_t) (matrix_bytes(f, s->cfg.hidden, s->cfg.ff) + L.gap), l});
+    }
+    return s->vtab.empty() ? 0 : sz_upload(s->vtab_dev.ptr, s->vtab.data(), s->vtab.size() * sizeof(VerifyLayer));
 }
 
 int32_t sz_session_set_layer_spaced(sz_session* s, uint32_t l, int32_t ty, uint64_t experts, uint64_t stride, uint64_t gap, int32_t shared_type, uint64_t shared) {
@@ -835,6 +820,15 @@ int32_t sz_session_set_layer_spaced(sz_session* s, uint32_t l, int32_t ty, uint6
     L.shared = shared;
     L.gap = gap;
     L.set = true;
+    if (f.exl3) {
+        // the launches' buffers hold as many layers as take 256 MiB (what the memory-side cache holds), at least one
+        const uint64_t per = verify_part_bytes(c, c.max_rows) + verify_dn_bytes(c, c.max_rows);
+        s->vchunk = (uint32_t) std::min<uint64_t>(c.n_layers, std::max<uint64_t>(1, (256ull << 20) / per));
+        if (s->plans.need((uint64_t) c.n_layers * s->plan_stride) || s->vtab_dev.need(c.n_layers * sizeof(VerifyLayer)) ||
+            s->part.need(s->vchunk * verify_part_bytes(c, c.max_rows)) || s->dn.need(s->vchunk * verify_dn_bytes(c, c.max_rows)))
+            return 1;
+    }
+    if (verify_table(s)) return 1;
     for (auto& g : s->graphs) sz_graph_destroy(g.second);   // captured address tables may be stale
     s->graphs.clear();
     return 0;
@@ -871,14 +865,11 @@ int32_t sz_session_set_router(sz_session* s, uint32_t l, int32_t rty, uint64_t r
     if (gw && (!format_of(gty, fg, tg) || !fg.dense)) return fail("sz_session_set_router: the shared expert's gate must be F32, F16 or BF16");
     if (!rw || (rw & (4 * fr.bb - 1)) || (gw & (4 * (gw ? fg.bb : 1) - 1))) return fail("sz_session_set_router: matrices must be aligned to four weights");
     if (s->rl.need((uint64_t) c.max_rows * c.n_expert * 4) || s->sgl.need((uint64_t) c.max_rows * 4)) return 1;
-    auto code = [](int ty) { return ty == SZ_TYPE_F32 ? 0u : ty == SZ_TYPE_F16 ? 1u : 2u; };
-    DenseJob jobs[2];
-    const uint32_t g0 = dense_groups(c.n_expert, c.hidden);
-    jobs[0] = {rw, s->rl.ptr, c.n_expert, c.n_expert, code(rty), 0, 0, 1.0f};
-    jobs[1] = {gw, s->sgl.ptr, 1, gw ? 1u : 0u, code(gty), g0, 0, 1.0f};
     SzLayer& L = s->layers[l];
-    if (L.jobs.need(sizeof jobs) || sz_upload(L.jobs.ptr, jobs, sizeof jobs)) return 1;
-    L.router_groups = g0 + (gw ? dense_groups(1, c.hidden) : 0);
+    L.router = rw;
+    L.router_type = rty;
+    L.gate = gw;
+    L.gate_type = gty;
     for (auto& g : s->graphs) sz_graph_destroy(g.second);
     s->graphs.clear();
     return 0;
@@ -886,13 +877,15 @@ int32_t sz_session_set_router(sz_session* s, uint32_t l, int32_t rty, uint64_t r
 
 int32_t sz_moe_router_verify(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t stream) {
     clear_error();
-    if (!s || l >= s->layers.size() || !s->layers[l].router_groups) return fail("sz_moe_router_verify: layer " + std::to_string(l) + " has no router set");
+    if (!s || l >= s->layers.size() || !s->layers[l].router) return fail("sz_moe_router_verify: layer " + std::to_string(l) + " has no router set");
     const sz_session_config& c = s->cfg;
     if (m == 0 || m > c.max_rows) return fail("sz_moe_router_verify: " + std::to_string(m) + " rows (1.." + std::to_string(c.max_rows) + ")");
     if (u & 15) return fail("sz_moe_router_verify: activations must be 16-byte aligned");
     const SzLayer& L = s->layers[l];
-    const sz_arg a[] = {P(L.jobs.ptr), U32(2), P(u), U32(c.hidden), U32(c.hidden), U32(m)};
-    return launch("matvec_cols_multi", L.router_groups, 1, 1, 256, dense_lds(c.hidden, m), stream, a);
+    const DenseShape d = dense_shape(c.hidden);
+    const sz_arg a[] = {U32(dense_code(L.router_type)), P(L.router), U32(dense_code(L.gate_type)), P(L.gate), P(u), P(s->rl.ptr), P(s->sgl.ptr),
+                        U32(c.n_expert), U32(c.hidden), U32(m)};
+    return launch((std::string("router_rows_m") + dense_m(m)).c_str(), (c.n_expert + d.pass - 1) / d.pass + (L.gate ? 1 : 0), 1, 1, d.block, 0, stream, a);
 }
 
 int32_t sz_session_router_outputs(sz_session* s, uint64_t* rl, uint64_t* sgl) {
@@ -979,12 +972,7 @@ int32_t sz_session_set_expert_mode(sz_session* s, int32_t mode) {
     clear_error();
     if (!s) return fail("sz_session_set_expert_mode: null session");
     if (mode < 0 || mode > 3)
-        return fail("sz_session_set_expert_mode: mode " + std::to_string(mode) + " (0 exact, 1 matrix cores, 2 matrix cores with the linearised codebook, 3 exact decode with f16 inputs)");
-    if (s->expert_mode != mode) {
-        for (auto& g : s->graphs) sz_graph_destroy(g.second);   // a captured round holds the other mode's launches
-        s->graphs.clear();
-    }
-    s->expert_mode = mode;
+        return fail("sz_session_set_expert_mode: mode " + std::to_string(mode) + " (0 to 3)");
     return 0;
 }
 
@@ -1101,31 +1089,28 @@ int32_t sz_verify_round(sz_session* s, uint32_t m, uint64_t u, uint64_t rl, uint
     const sz_session_config& c = s->cfg;
     // everything that can be refused is refused before a capture begins
     if (head_check(s, m, head_u, "sz_verify_round")) return 1;
-    for (uint32_t l = 0; l < c.n_layers; l++)
-        if (!s->layers[l].set) return fail("sz_verify_round: layer " + std::to_string(l) + " has no experts set");
+    if ((u & 15) || (y & 15)) return fail("sz_verify_round: activations must be 16-byte aligned");
+    for (uint32_t l = 0; l < c.n_layers; l++) {
+        const SzLayer& L = s->layers[l];
+        if (!L.set) return fail("sz_verify_round: layer " + std::to_string(l) + " has no experts set");
+        if (L.shared && L.shared_type != L.type) return fail("the shared expert must have the routed experts' type (layer " + std::to_string(l) + ")");
+    }
     const SzGraphKey key{{m, u, rl, sgl, y, head_u, drafts, out, stream, 0}};
     auto it = s->use_graph ? s->graphs.find(key) : s->graphs.end();
     if (it == s->graphs.end()) {
         static const bool no_graph = std::getenv("SHADOWZERO_NO_GRAPH") != nullptr;
         auto record = [&]() -> int {
-            // an EXL3 layer's rank-order sum rides the first launch of the layer after it; the last layer's gets its own launch
-            PendingSum ps;
-            bool any_exl3 = false;
-            for (uint32_t l = 0; l < c.n_layers; l++) any_exl3 = any_exl3 || (s->layers[l].type >= 1021 && s->layers[l].type <= 1033);
-            static const bool route_in_launch = std::getenv("SHADOWZERO_ROUTE_IN_LAUNCH") != nullptr;   // the form without the routing launch, for comparisons
-            if (any_exl3 && (s->expert_mode == 0 || s->expert_mode == 3) && !route_in_launch && c.n_layers >= 12) {
-                // every layer's router logits are inputs of the round: all of them are routed by one launch before the first layer
-                // (about 10 us, against about 1 us a layer that the selection inside launch 1 costs: not for short rounds)
-                const sz_arg a[] = {P(rl), P(s->plans.ptr), U32(s->plan_stride), U32(c.n_expert), U32(c.top_k), U32(m), U32(c.n_layers)};
-                if (launch("verify_route_layers", (c.n_layers * m + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
-                ps.plans = s->plans.ptr;
-                ps.plan_stride = s->plan_stride;
-            }
+            // every layer's inputs are given: the EXL3 layers go through the verify launches together, whatever their order
+            if (!s->vtab.empty() && verify_layers(s, 0, (uint32_t) s->vtab.size(), 0, m, u, rl, sgl, y, s->plans.ptr, stream)) return 1;
             for (uint32_t l = 0; l < c.n_layers; l++) {
+                if (s->layers[l].type > 1020) {
+                    s->last_plan = s->plans.ptr + (uint64_t) l * s->plan_stride;
+                    s->last_fused = true;
+                    continue;
+                }
                 const uint64_t off = (uint64_t) l * m;
-                if (moe_layer(s, l, m, u + off * c.hidden * 4, rl + off * c.n_expert * 4, sgl + off * 4, y + off * c.hidden * 4, stream, &ps)) return 1;
+                if (moe_layer(s, l, m, u + off * c.hidden * 4, rl + off * c.n_expert * 4, sgl + off * 4, y + off * c.hidden * 4, stream)) return 1;
             }
-            if (launch_pending_sum(s, ps, m, stream)) return 1;
             const Accept acc{drafts, out};
             return head_argmax(s, m, head_u, out + 8, stream, &acc);
         };
@@ -1259,8 +1244,7 @@ uint64_t sz_prefill_buffer(sz_session* s, int32_t which) {
 // ---- the hyper-connection around a sublayer ---------------------------------------------------------------------------------
 struct sz_hc {
     sz_hc_config cfg{};
-    DevBuf rn, down, mix, g, jobs;   // [max_rows][ch], [max_rows][rank], [max_rows][ch], [max_rows][streams], 3 jobs
-    uint32_t groups_di = 0, groups_up = 0;
+    DevBuf scales, down, g;   // f64[max_rows][streams], f32[max_rows][rank], f32[max_rows][streams]
 };
 
 extern "C" {
@@ -1288,20 +1272,7 @@ sz_hc* sz_hc_new(const sz_hc_config* cfg) {
     }
     sz_hc* h = new sz_hc();
     h->cfg = c;
-    if (h->rn.need(c.max_rows * ch * 4) || h->down.need((uint64_t) c.max_rows * c.rank * 4) || h->mix.need(c.max_rows * ch * 4) ||
-        h->g.need((uint64_t) c.max_rows * c.streams * 4) || h->jobs.need(3 * sizeof(DenseJob))) {
-        delete h;
-        return nullptr;
-    }
-    auto code = [](int ty) { return ty == SZ_TYPE_F32 ? 0u : ty == SZ_TYPE_F16 ? 1u : 2u; };
-    const uint32_t gd = dense_groups(c.rank, ch);
-    DenseJob jobs[3];
-    jobs[0] = {c.down_w, h->down.ptr, c.rank, c.rank, code(c.down_type), 0, 1, (float) c.streams};                    // silu(v / cs)
-    jobs[1] = {c.inject_w, h->g.ptr, c.streams, c.inject_w ? c.streams : 0u, code(c.inject_type), gd, 2, (float) c.streams};   // 2 sigmoid(v / cs)
-    jobs[2] = {c.up_w, h->mix.ptr, (uint32_t) ch, (uint32_t) ch, code(c.up_type), 0, 3, 1.0f};                         // sigmoid(v)
-    h->groups_di = gd + (c.inject_w ? dense_groups(c.streams, ch) : 0);
-    h->groups_up = dense_groups(ch, c.rank);
-    if (sz_upload(h->jobs.ptr, jobs, sizeof jobs)) {
+    if (h->scales.need((uint64_t) c.max_rows * c.streams * 8) || h->down.need((uint64_t) c.max_rows * c.rank * 4) || h->g.need((uint64_t) c.max_rows * c.streams * 4)) {
         delete h;
         return nullptr;
     }
@@ -1317,21 +1288,27 @@ int32_t sz_hc_read(sz_hc* h, uint32_t m, uint64_t r, uint64_t u, uint64_t stream
     const sz_hc_config& c = h->cfg;
     if (m == 0 || m > c.max_rows) return fail("sz_hc_read: " + std::to_string(m) + " rows (1.." + std::to_string(c.max_rows) + ")");
     if ((r & 15) || (u & 15)) return fail("sz_hc_read: rows must be 16-byte aligned");
-    const uint32_t ch = c.hidden * c.streams;
-    {
-        const sz_arg a[] = {P(r), P(c.norm_w), P(h->rn.ptr), U32(c.hidden), F32(c.eps), U32(c.streams)};
-        if (launch("rmsnorm_groups_rows", c.streams, m, 1, 256, 0, stream, a)) return 1;
+    const DenseShape d = dense_shape((uint64_t) c.hidden * c.streams);
+    const uint32_t pass = d.block / 64 / d.waves;   // whole rows, a wave or more each
+    const DenseShape du = dense_shape(c.rank);
+    const uint32_t per = 4 * std::max<uint32_t>(1, du.pass / (du.block / 64 / du.waves));   // 4 waves of 64 / G columns
+    // LDS of the first launch: the sums of squares of every stream's spans (of at least 256 columns) and its scale; as many rows
+    // at a time as fit half a compute unit's (all of them, unless the streams are many and long)
+    const bool eight = c.hidden % 8 == 0 && c.down_type != SZ_TYPE_F32 && (!c.inject_w || c.inject_type != SZ_TYPE_F32);
+    const uint64_t lds = (uint64_t) c.streams * (c.hidden / (eight ? 512 : 256) + 3) * 8;
+    const uint32_t lot = (uint32_t) std::min<uint64_t>(m, std::max<uint64_t>(1, 80000 / lds));
+    for (uint32_t j = 0; j < m; j += lot) {
+        const uint32_t n = std::min(lot, m - j);
+        const uint64_t rj = r + (uint64_t) j * c.hidden * c.streams * 4, sc = h->scales.ptr + (uint64_t) j * c.streams * 8, dj = h->down.ptr + (uint64_t) j * c.rank * 4;
+        const sz_arg a[] = {U32(dense_code(c.down_type)), P(c.down_w), U32(c.rank), U32(dense_code(c.inject_type)), P(c.inject_w), P(rj), P(c.norm_w), P(sc),
+                            P(dj), P(h->g.ptr + (uint64_t) j * c.streams * 4), U32(c.hidden), U32(c.streams), U32(n), F32(c.eps)};
+        if (launch((std::string("hc_down_m") + dense_m(n)).c_str(), (c.rank + pass - 1) / pass + (c.inject_w ? (c.streams + pass - 1) / pass : 0), 1, 1, d.block,
+                   (uint32_t) (n * lds), stream, a))
+            return 1;
+        const sz_arg b[] = {U32(dense_code(c.up_type)), P(c.up_w), P(dj), P(rj), P(c.norm_w), P(sc), P(u + (uint64_t) j * c.hidden * 4), U32(c.hidden), U32(c.streams), U32(c.rank), U32(n)};
+        if (launch((std::string("hc_up_m") + dense_m(n)).c_str(), (c.hidden + per - 1) / per, 1, 1, 256, 0, stream, b)) return 1;
     }
-    {
-        const sz_arg a[] = {P(h->jobs.ptr), U32(2), P(h->rn.ptr), U32(ch), U32(ch), U32(m)};
-        if (launch("matvec_cols_multi", h->groups_di, 1, 1, 256, dense_lds(ch, m), stream, a)) return 1;
-    }
-    {
-        const sz_arg a[] = {P(h->jobs.ptr + 2 * sizeof(DenseJob)), U32(1), P(h->down.ptr), U32(c.rank), U32(c.rank), U32(m)};
-        if (launch("matvec_cols_multi", h->groups_up, 1, 1, 256, dense_lds(c.rank, m), stream, a)) return 1;
-    }
-    const sz_arg a[] = {P(h->rn.ptr), P(h->mix.ptr), P(u), U32(c.hidden), U32(c.streams)};
-    return launch("hc_mix_rows", (c.hidden + 255) / 256, m, 1, 256, 0, stream, a);
+    return 0;
 }
 
 int32_t sz_hc_write(uint64_t r, uint64_t g, uint64_t y, uint32_t m, uint32_t hidden, uint32_t streams, uint64_t stream) {

@@ -299,100 +299,6 @@ __device__ __forceinline__ void exl3_rows_wait(u32 t) {
     }
 }
 
-// The decode loop of one wave for one input over a stream of `rows` tile rows (8 a 128-block of inputs, consecutive
-// blocks): the first D rows have been requested by exl3_rows_issue, every later row is requested into the ring slot of
-// the row just decoded, so D rows stay in flight until the stream runs out.  xw holds the rotated input (16 values a
-// row) and receives the wave's partial sums of its 128 output columns.
-// XH: the wave's rotated inputs are f16 (exl3_put_x_f16: pairs of consecutive inputs a word, scaled by a power of two that
-// `unscale` undoes) and two weights meet their two inputs in one v_dot2_f32_f16: 16 instructions a row for the products
-// instead of 32, f32 sums as before, the inputs rounded to 11 bits.
-template <int K, int D = 8, bool H = false, bool XH = false>
-__device__ __forceinline__ void exl3_wave_stream(const u32* __restrict__ row0, u64 pitch, u32 rows, const u32* wb, u32 lds, float* xw, u32 lane,
-                                                 float unscale = 1.0f) {
-    typedef Exl3Rows<K, D, H> R;
-    constexpr int stride = R::stride, ur = R::unit_rows;
-    constexpr int NW = EXL3_NW(K, H);
-    // where the lane's words lie in a row of the ring: an integer rate's K words at the lane's pitch and the word before them
-    // (the tile's last for its first lane); a half rate's NW + 1 words around its bits, cyclic inside the tile (exl3_load_words)
-    const u32 own = lane * stride, prev = ((lane & 7) == 0 ? lane + 7 : lane - 1) * stride + K - 1;
-    u32 off[NW + 1];
-    const u32 odd = lane & 1;
-    if constexpr (H) {
-        constexpr u32 RW = EXL3_TILE_WORDS(K, H);
-        const u32 first = (lane & 7) * EXL3_LANE_BITS(K, H) - 16 * odd;
-        const u32 w0 = first / 32 + RW - 1;
-#pragma unroll
-        for (int n = 0; n <= NW; n++) off[n] = (lane >> 3) * RW + (w0 + n) % RW;
-    }
-    float acc0 = 0.0f, acc1 = 0.0f;
-#pragma unroll 1
-    for (u32 r = 0; r < rows; r++) {
-        exl3_rows_wait<K, D, H>(r + D > rows ? r + D - rows : 0);
-        const u32* row = wb + (r & (D - 1)) * R::row_words;
-        u32 S[NW];
-        if constexpr (H) {
-            u32 L[NW + 1];
-#pragma unroll
-            for (int n = 0; n <= NW; n++) L[n] = row[off[n]];
-#pragma unroll
-            for (int n = 0; n < NW; n++) S[n] = odd ? __builtin_amdgcn_alignbit(L[n], L[n + 1], 16) : L[n];
-        } else {
-            S[0] = row[prev];
-#pragma unroll
-            for (int d = 0; d < K; d++) S[d + 1] = row[own + d];
-        }
-        f16x2 w[16];
-        exl3_decode32<K, H>(S, w);
-        // once the row's words are in registers (the LDS reads have returned, not just been issued: a request that hits
-        // in the cache can land within a few hundred cycles) its slot, with its partner's for two-row units, can take the
-        // row D further on
-        if ((r + 1) % ur == 0 && r + D + 1 - ur < rows) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-            exl3_unit_issue<K, D, H>(row0, pitch, r + D + 1 - ur, lane, lds);
-        }
-        if constexpr (XH) {
-            // the row's 16 inputs as 8 f16 pairs: weights 2 j, 2 j + 1 of the lane meet inputs 2 q + {0, 1} (j even) or 2 q + 8 + {0, 1}
-            // (j odd) of the tile row, q = j / 4
-            typedef u32 u32x4v __attribute__((ext_vector_type(4)));
-            const u32x4v lo = ((const u32x4v*) xw)[2 * r], hi = ((const u32x4v*) xw)[2 * r + 1];
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const f16x2 xp = __builtin_bit_cast(f16x2, (j & 1) ? hi[j >> 2] : lo[j >> 2]);
-                if ((j >> 1) & 1) acc1 = __builtin_amdgcn_fdot2(w[j], xp, acc1, false);
-                else acc0 = __builtin_amdgcn_fdot2(w[j], xp, acc0, false);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float* xr = xw + r * 16 + 2 * q;
-                const float xa[4] = {xr[0], xr[1], xr[8], xr[9]};
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int i = 8 * q + e;
-                    const int rr = (e & 1) + 2 * ((e >> 1) & 1);
-                    if (EXL3_HALF(i)) acc1 = __builtin_fmaf((float) w[i / 2][i % 2], xa[rr], acc1);
-                    else acc0 = __builtin_fmaf((float) w[i / 2][i % 2], xa[rr], acc0);
-                }
-            }
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    const u32 col = (lane >> 3) * 16 + (lane & 7);
-    xw[col] = acc0 * unscale;
-    xw[col + 8] = acc1 * unscale;
-}
-
-// A wave's rotated 128-block (the lane holds elements `lane` and `lane + 64`) as f16 in input order at xh[0..127], scaled by
-// the power of two that takes the block's largest magnitude to [2^14, 2^15); returns what undoes the scale.
-__device__ __forceinline__ float exl3_put_x_f16(u16* xh, float a0, float a1, u32 lane) {
-    const float mx = wave_max_f32(fmaxf(__builtin_fabsf(a0), __builtin_fabsf(a1)));
-    float scale, iv;
-    pow2_scale_of(f32_bits(mx), scale, iv);
-    xh[lane] = __builtin_bit_cast(u16, (_Float16) (a0 * scale));
-    xh[lane + 64] = __builtin_bit_cast(u16, (_Float16) (a1 * scale));
-    return iv;
-}
-
 // Group g = blockIdx.y: blob wtab[g], record gtab[17 g] = {n <= 4 (0: unused slot), xi[8], yi[8]}; wave w of the workgroup
 // takes input block 4 blockIdx.z + w, and the four waves' sums are added in wave order into
 // part[((g * gridDim.z + blockIdx.z) * 4 + j) * out + col], j < n.  grid = (out / 128, groups, ceil(in / 512)), block 256.
@@ -488,395 +394,622 @@ extern "C" __global__ void __launch_bounds__(64) exl3_finish_rows(const float* p
     }
 }
 
-// ------------------------------------------------------------------------------------------- the fused verify layer
-// A resident EXL3 layer for a verify batch (m <= 8 rows) in three launches, none of which needs a plan: the work items are
-// the (token, expert) pairs themselves, one input each: pair p = j k + t of token j and rank t for p < m k, then the shared
-// expert's pair m k + j of every token j.  Tokens that share an expert, and the shared expert for every token, read the
-// same weights again; at 4 rows and top-10 of 512 that is about 10 % more reads, nearly all of them L2 hits, and it buys
-// kernels with one input a wave: few registers, every wave of a launch resident at once.
-// Expert e's three projections sit at ebase + e estride + {0, part, 2 part} (gate, up, down), the shared expert's at
-// shbase + the same offsets (shbase = 0: no shared expert): addresses are computed, not looked up, so no load stands
-// between a routing result and the first request for that expert's weights.
-// pbuf holds u32 tidx[m k] | f32 w[m k] | u32 cnt[m].
+// ------------------------------------------------------------------------------------------- the verify layer
+// Resident EXL3 layers for a verify batch (m <= 8 rows): a plan, gate and up, down, the rank-order sum, each launch for one
+// layer (sz_moe_layer_verify, sz_moe_block_verify) or for all layers of one type of a round at once (sz_verify_round is
+// given every layer's inputs before the first one runs, so the layers do not wait for each other): with 48 layers in a
+// launch the two decode launches are bound by the vector unit and not by 96 prologues, tails and launch boundaries.
+//
+// (1) The work items are the DISTINCT experts of a layer's batch, the shared expert as the first item with all tokens: an
+// expert's weights are decoded once however many tokens chose it (at 4 rows and top-10 of 512 experts 40 items for 44
+// (token, expert) pairs, at 8 rows 75 for 88, of 32 experts 29 for 72).
+// (2) The products run on the matrix cores: a lane decodes 4 consecutive weights of the bit stream, which are four values of
+// operand B of v_mfma_f32_16x16x32_f16 as decoded (two tile rows make one instruction), 15 vector instructions a 16 x 16
+// tile for up to 4 tokens where the vector unit alone needs 19 a token.  The item's tokens ride on the rows of operand A in
+// THREE f16 parts (11 bits each: all 24 bits of an f32), scaled by the power of two that takes the largest magnitude of the
+// token's 512 inputs to [2^14, 2^15): products are exact and sums are f32, as with f32 inputs.
+// (3) A workgroup prepares the A rows of its 512 inputs once (a wave a 128-block: scales, transform, split) and its four
+// waves then take CT column tiles each over all 512 inputs, so there is no sum over waves.  The sums are left as they are:
+// whoever reads them (launch 2 for gate and up, the last launch for down) adds the partials of the 512-input blocks up and
+// applies the output side once.
+//
+// A layer's table entry: where its experts lie (expert e's gate, up and down at experts + e stride + {0, part, 2 part},
+// the shared expert's at shared + the same; shared = 0: none) and its number in the caller's buffers.
+struct VerifyLayer {
+    u64 experts, stride, shared;
+    u32 part, layer;
+};
+// Layer li of a launch: out of the table, or of a one-layer launch its kernel arguments (table 0): a load less ahead of
+// everything else.
+__device__ __forceinline__ VerifyLayer verify_layer(const u8* __restrict__ table, u32 li, u64 experts, u64 stride, u64 shared, u32 part, u32 base) {
+    if (table) return ((const VerifyLayer*) table)[li];
+    return VerifyLayer{experts, stride, shared, part, base};
+}
+// The plan of a layer (route_plan in route.hip.h), grid = layers, block 64 m.  The routing weights are not needed before the
+// last launch and are left to a spare workgroup of launch 2 (verify_route_weights below).
+extern "C" __global__ void __launch_bounds__(512) verify_plan_exl3(const float* logits, u8* plans, u32 plan_stride, u32 ioff, const u8* table, u64 shared0, u32 base, u32 ne,
+                                                                   u32 k, u32 m) {
+    __shared__ RoutePlanLds lds;
+    const VerifyLayer L = verify_layer(table, blockIdx.x, 0, 0, shared0, 0, base);
+    const u32 l = L.layer - base;
+    route_plan(logits + (u64) l * m * ne, plans + (u64) l * plan_stride, ioff, ne, k, m, L.shared != 0, lds);
+}
 
-// The rank-order sum of token j's finished down products for the 128 columns of block ob (launch 2 has finished every
-// pair's block: no split over its inputs), column ob * 128 + tid for tid < 128: y[j] = sum over the cnt[j] experts of
-// w[j, t] * dn[j k + t] + sigmoid(gl[j]) * dn[m k + j] (moe_combine_qwen_rows, kernels/forward.cu:2568).  Every load goes
-// out before the first is waited for.  pbuf = u32 tidx[m k] | f32 w[m k] | u32 cnt[m].
-__device__ __forceinline__ void exl3_combine_finished(const float* __restrict__ dn, const u8* __restrict__ pbuf, const float* __restrict__ gl,
-                                                      float* __restrict__ y, u32 k, u32 m, u32 hidden, bool shared, u32 ob, u32 j, u32 tid) {
+// The renormalised routing weights and the counts of the chosen experts tidx (pbuf, as the plan left it) into w and cnt:
+// a wave a token, for a workgroup that has nothing else to do.
+__device__ __forceinline__ void verify_route_weights(const float* __restrict__ logits, u8* __restrict__ pbuf, u32 ne, u32 k, u32 m, u32 wave, u32 lane) {
     const u32 G = m * k;
-    const float* wts = (const float*) (pbuf + G * 4);
-    const u32* cnt = (const u32*) (pbuf + 2 * G * 4);
-    const u32 col = ob * 128 + tid;
-    float v[17], w[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const u32 pair = j * k + min((u32) i, k - 1);
-        v[i] = dn[(u64) pair * hidden + col];
-        w[i] = wts[pair];
+    for (u32 j = wave; j < m; j += 4) {
+        u32 kk;
+        const float wt = route_weights_chosen(logits + (u64) j * ne, ne, k, lane, (const u32*) pbuf + j * k, &kk);
+        if (lane < k) ((float*) (pbuf + G * 4))[j * k + lane] = wt;
+        if (lane == 0) ((u32*) (pbuf + 2 * G * 4))[j] = kk;
     }
-    v[16] = shared ? dn[(u64) (G + j) * hidden + col] : 0.0f;
-    const float sg = shared ? sigmoidf_ref(gl[j]) : 0.0f;
-    const u32 c = cnt[j];
-    float a = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        if ((u32) i < c) a += w[i] * v[i];
-    if (shared) a += sg * v[16];
-    y[(u64) j * hidden + col] = a;
 }
 
-// The routing of a whole round in one launch, for a caller that has every layer's router logits before the first layer runs
-// (sz_verify_round): wave (l, j) leaves token j's chosen experts, weights and count in layer l's plan, plans + l *
-// plan_stride, in the layout above; launches 1 and 2 of those layers are then given no logits and read the plan instead of
-// redoing the selection in every workgroup.  Same functions as the launches use, so the same bits.
-// logits[l][m][ne]; grid = ceil(L m / 4), block 256; ne <= 512, k <= 16.
-extern "C" __global__ void __launch_bounds__(256) verify_route_layers(const float* logits, u8* plans, u32 plan_stride, u32 ne, u32 k, u32 m, u32 L) {
-    __shared__ double exs[4][512];
-    __shared__ u32 tops[4][16];
-    const u32 lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const u32 i = blockIdx.x * 4 + w;
-    if (i >= L * m) return;
-    const u32 l = i / m, j = i - l * m, G = m * k;
-    const float* lg = logits + (u64) i * ne;
-    u8* pbuf = plans + (u64) l * plan_stride;
-    route_ids(lg, ne, k, lane, exs[w], tops[w]);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    u32 kk;
-    const float wt = route_weights(lg, ne, k, lane, tops[w], &kk);
-    if (lane < k) {
-        ((u32*) pbuf)[j * k + lane] = tops[w][lane];
-        ((float*) (pbuf + G * 4))[j * k + lane] = wt;
-    }
-    if (lane == 0) ((u32*) (pbuf + 2 * G * 4))[j] = kk;
+__device__ __forceinline__ u64 uniform_u64(u64 v) {
+    return ((u64) (u32) __builtin_amdgcn_readfirstlane((u32) (v >> 32)) << 32) | (u32) __builtin_amdgcn_readfirstlane((u32) v);
 }
 
-// Launch 1's workgroup: EXL3_GU_WAVES waves, each takes EXL3_VERIFY_NB consecutive 128-blocks of the input through a ring
-// of EXL3_GU_DEPTH rows (grid z = ceil(hidden / 128 / (waves * blocks))).  One block a wave with a 4-row ring puts twice as
-// many waves on a SIMD as two blocks a wave with an 8-row ring, for the same LDS: the waves spend most of their life
-// waiting (for rows, for LDS, for an issue slot), and more of them hide more of it (24.2 -> 21.5 us a launch).  Four waves
-// a workgroup rather than eight spread a little more evenly over the CUs (another 1 % of the round), at the price of twice
-// the routing passes and partial sums.
-#define EXL3_GU_WAVES 4
-#define EXL3_VERIFY_NB 1
-#define EXL3_GU_DEPTH 4
+// A wave's stream of trellis rows for CT column tiles: units of 16 tiles (16 / CT tile rows, 512 K bytes), each brought
+// into one of D ring slots by NI global-to-LDS loads of 16 bytes a lane.  In LDS a unit lies packed in the order of the
+// bit stream: tile row, column tile, tile word.
+template <int K, bool H, int CT>
+struct VerifyRing {
+    static constexpr int TW = EXL3_TILE_WORDS(K, H), CH = TW / 4;   // words and 16-byte chunks a tile
+    static constexpr int UR = 16 / CT;                              // tile rows a unit
+    static constexpr int NI = (CH + 3) / 4;                         // loads a unit: 16 CH chunks, 64 a load, the last load perhaps partly
+    static constexpr int UW = 64 * CH;                              // words a unit
+    static constexpr int D = CH <= 8 ? 3 : 2;
+    u64 row0;         // the wave's first tile row, at its first column tile (uniform)
+    u32 pitch;        // bytes between tile rows
+    u32 units, lds;
+    u32 off[NI];      // the lane's source offsets inside a unit
+    __device__ __forceinline__ void init(const u8* first, u32 pitch_bytes, u32 n, u32 lds_addr, u32 lane) {
+        row0 = uniform_u64((u64) first);
+        pitch = pitch_bytes;
+        units = n;
+        lds = lds_addr;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const u32 q = 64 * i + lane, row = q / (CT * CH);
+            off[i] = row * pitch + (q - row * (CT * CH)) * 16;
+        }
+    }
+    __device__ __forceinline__ void issue(u32 unit, u32 slot, u32 lane) const {
+        const u64 at = row0 + (u64) unit * ((u64) UR * pitch);
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+            if (64 * (i + 1) <= 16 * CH || 64 * i + lane < 16 * CH) lds_load_at(at, off[i], lds + (slot * UW + i * 256) * 4);
+    }
+    // requests the first D units and returns once everything requested before them has landed
+    __device__ __forceinline__ void fill(u32 lane) const {
+        if (units >= (u32) D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) issue(d, d, lane);
+            wait_vm<D * NI>();
+        } else {
+            for (u32 d = 0; d < units; d++) issue(d, d, lane);
+            wait_vm<0>();
+        }
+    }
+    // returns once at most the loads of `n` units are in flight
+    __device__ __forceinline__ static void wait(u32 n) {
+        switch (n) {
+            case 0: wait_vm<0>(); break;
+            case 1: wait_vm<NI>(); break;
+            default: wait_vm<2 * NI>(); break;
+        }
+    }
+};
 
-// Launch 1: routing (every workgroup of a routed pair redoes its token's selection on one of its waves; the workgroups
-// with blockIdx.x == 0 and blockIdx.z == 0 of the gate half also publish tidx) and the gate and up products' partial
-// sums: gup[((sel * S + pair) * zs + z)][ff], S = m (k + 1), sel 0 = gate, 1 = up, zs = gridDim.z.
-// grid = (ff / 128, 2 S + c, zs), block 64 * EXL3_GU_WAVES; c = 0, or the rows that give (hidden / 128) m more workgroups
-// for the sum of the layer before (cmode).
-template <int K, bool H = false, bool XH = false>
-__device__ __forceinline__ void verify_gate_up_kernel(const float* __restrict__ logits, u64 ebase, u64 estride, u64 shbase, u32 part,
-                                                      const float* __restrict__ u, u8* __restrict__ pbuf, float* __restrict__ gup, u32 ne, u32 k,
-                                                      u32 m, u32 hidden, u32 ff, const float* __restrict__ cdn, const u8* __restrict__ cpbuf,
-                                                      const float* __restrict__ cgl, float* __restrict__ cy, u32 cmode) {
-    if (blockIdx.y >= 2 * (m * k + m)) {
-        // rows of the grid past the pairs (cmode != 0): the rank-order sum of the layer before this one, whose launch 3 rides
-        // here (same batch and shapes; cdn its finished down products, cpbuf its routing, cgl its shared gate logits, cy its
-        // output; cmode 2: it has a shared expert), a workgroup a (token, 128-column block)
-        const u32 ci = ((blockIdx.y - 2 * (m * k + m)) * gridDim.z + blockIdx.z) * gridDim.x + blockIdx.x, nb = hidden / 128;
-        if (cmode && ci < nb * m && threadIdx.x < 128) exl3_combine_finished(cdn, cpbuf, cgl, cy, k, m, hidden, cmode == 2, ci % nb, ci / nb, threadIdx.x);
-        return;
-    }
-    constexpr int NB = EXL3_VERIFY_NB, WA = EXL3_GU_WAVES, D = EXL3_GU_DEPTH;
-    __shared__ __attribute__((aligned(16))) u32 wb_all[WA][Exl3Rows<K, D, H>::words];   // the waves' trellis rows; before that, the routing's scratch
-    __shared__ float xw_all[WA][NB * 128];
-    __shared__ u32 sc_all[WA][NB * 64];   // the wave's f16 input scales
-    __shared__ u32 sv_out[64];            // the f16 output scales of the workgroup's 128 columns (wave 0 requests them)
-    __shared__ u32 s_top[16];
-    static_assert(sizeof(wb_all) >= 512 * sizeof(double), "the exact routing fallback needs 512 doubles");
-    const u32 G = m * k, S = G + m;
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // the wave index as a scalar: the index arithmetic on it is the scalar unit's
-    const u32 sel = blockIdx.y / S, pair = blockIdx.y % S;
-    const u32 kbs = hidden / 128;
-    const u32 kb0 = (blockIdx.z * WA + wave) * NB;
-    const u32 nb = kb0 >= kbs ? 0u : min((u32) NB, kbs - kb0);   // this wave's input blocks: kb0 .. kb0 + nb - 1
-    const u32 j = pair < G ? pair / k : pair - G;
-    // the wave's blocks of its token's row do not depend on the routing: on their way while that is worked out
-    float v[NB][2];
+// Where lane group a reads element q (0..15) of a tile row: slots 4 a .. 4 a + 3 = inputs 2 a, 2 a + 1, 2 a + 8, 2 a + 9.
+__device__ __forceinline__ u32 exl3_aslot(u32 q) { return 4 * ((q & 7) >> 1) + 2 * (q >> 3) + (q & 1); }
+
+// LDS waited for and a workgroup barrier, with no wait for the global-to-LDS loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The A rows of a workgroup's 512 inputs: f16 a_sh[((step * NR + row) * 4 + a) * 8 + 4 (tile row & 1) + slot & 3], step = a
+// pair of tile rows (4 a 128-block), row 3 r + part of token r, NR = 3 NMAX.  The wave holds elements `lane` and `lane + 64` of
+// its 128-block kbl (0..3; 4: none) of every token's rotated inputs.  Ends with the workgroup past a barrier.
+template <int NMAX>
+__device__ __forceinline__ void verify_put_rows(u16* a_sh, float* s_mx, float* s_iv, const float (&rot)[NMAX][2], u32 n, u32 kbl, u32 wave, u32 lane) {
+    constexpr u32 NR = 3 * NMAX;
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-        v[b][0] = v[b][1] = 0.0f;
-        if ((u32) b < nb) {
-            const float* xj = u + (u64) j * hidden + (kb0 + b) * 128;
-            v[b][0] = load_f32_uncounted(xj + lane);      // waited for together with the input scales, behind which the trellis rows are already on their way
-            v[b][1] = load_f32_uncounted(xj + lane + 64);
+    for (int r = 0; r < NMAX; r++) {
+        if ((u32) r < n) {
+            const float mx = wave_max_f32(fmaxf(__builtin_fabsf(rot[r][0]), __builtin_fabsf(rot[r][1])));
+            if (lane == 0) s_mx[4 * r + wave] = mx;
         }
     }
-    u32* tidx = (u32*) pbuf;
-    const u8* bp;
-    if (pair < G && logits == nullptr) {
-        // the round's routing launch has left every layer's chosen experts in its plan (verify_route_layers): one load
-        const u32 e = tidx[pair];
-        if (e == 0xffffffffu) return;
-        bp = (const u8*) (ebase + e * estride + (u64) sel * part);
-    } else if (pair < G) {
-        const u32 t = pair % k;
-        if (wave == (blockIdx.x + blockIdx.y + blockIdx.z) % WA) {   // not always the same wave: the prologues of co-resident workgroups spread over the SIMDs
-            // the selection is a chain of dependent steps that the whole workgroup waits for: it goes ahead of the decoding
-            // waves of other workgroups on its SIMD
-            __builtin_amdgcn_s_setprio(3);
-            route_id_of_rank(logits + (u64) j * ne, ne, k, t, lane, (double*) &wb_all[0][0], s_top);   // only s_top[t] is read
-            __builtin_amdgcn_s_setprio(0);
-            if (sel == 0 && blockIdx.x == 0 && blockIdx.z == 0 && lane == 0) tidx[pair] = s_top[t];
-        }
-        __syncthreads();
-        const u32 e = s_top[t];
-        if (e == 0xffffffffu) return;
-        bp = (const u8*) (ebase + e * estride + (u64) sel * part);
-    } else {
-        if (!shbase) return;
-        bp = (const u8*) (shbase + (u64) sel * part);
-    }
-    float* xw = xw_all[wave];
-    if (nb) {
-        const u32 sc_lds = __builtin_amdgcn_readfirstlane(lds_offset(sc_all[wave]));
-        const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave]));
-        for (u32 b = 0; b < nb; b++) lds_load<4>(bp + (kb0 + b) * 256 + lane * 4, sc_lds + b * 256);
-        if (wave == 0) lds_load<4>(bp + 2 * (u64) hidden + blockIdx.x * 256 + lane * 4, __builtin_amdgcn_readfirstlane(lds_offset(sv_out)));   // the block's output scales, for the end
-        const u32* row0 = (const u32*) (bp + 2 * (u64) hidden + 2 * (u64) ff + 4) + ((u64) kb0 * 8 * (ff / 16) + blockIdx.x * 8) * EXL3_TILE_WORDS(K, H);
-        const u64 pitch = (u64) (ff / 16) * EXL3_TILE_WORDS(K, H);
-        exl3_rows_issue<K, D, H>(row0, pitch, lane, wb_lds);
-        wait_vm<Exl3Rows<K, D, H>::loads>();   // everything requested before the rows: the token's values, the scales
+    lds_barrier();
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            load_landed(v[b][0]);
-            load_landed(v[b][1]);
-        }
-        const u16* sc = (const u16*) sc_all[wave];
-        float unscale = 1.0f;
+    for (int r = 0; r < NMAX; r++) {
+        if ((u32) r < n) {
+            const f32x4 mx = ((const f32x4*) s_mx)[r];
+            float scale, iv;
+            pow2_scale_of(f32_bits(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]))), scale, iv);
+            if (wave == 0 && lane == 0) s_iv[r] = iv;
+            if (kbl < 4) {
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            if ((u32) b < nb) {
-                float a0 = v[b][0] * f16_to_f32(sc[b * 128 + lane]), a1 = v[b][1] * f16_to_f32(sc[b * 128 + lane + 64]);
-                wht128_wave(a0, a1, lane);
-                if constexpr (XH) {
-                    static_assert(!XH || NB == 1, "the f16 inputs of a wave are one 128-block");
-                    unscale = exl3_put_x_f16((u16*) xw, a0, a1, lane);
-                } else {
-                    xw[b * 128 + lane] = a0;
-                    xw[b * 128 + 64 + lane] = a1;
+                for (int h = 0; h < 2; h++) {
+                    const u32 i = lane + 64 * h, t = i >> 4, sl = exl3_aslot(i & 15);
+                    const float v = rot[r][h] * scale;
+                    const _Float16 hi = (_Float16) v;
+                    const float v1 = v - (float) hi;
+                    const _Float16 mid = (_Float16) v1;
+                    const _Float16 lo = (_Float16) (v1 - (float) mid);
+                    u16* at = a_sh + (((kbl * 4 + (t >> 1)) * NR + 3 * r) * 4 + (sl >> 2)) * 8 + 4 * (t & 1) + (sl & 3);
+                    at[0] = __builtin_bit_cast(u16, hi);
+                    at[32] = __builtin_bit_cast(u16, mid);
+                    at[64] = __builtin_bit_cast(u16, lo);
                 }
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        exl3_wave_stream<K, D, H, XH>(row0, pitch, 8 * nb, wb_all[wave], wb_lds, xw, lane, unscale);
     }
-    __syncthreads();
-    const u32 nw = min((u32) WA, (kbs - min(kbs, blockIdx.z * WA * NB) + NB - 1) / NB);   // waves of this workgroup that had blocks
-    if (wave == 0) {
-        // the workgroup's partial of its 128 columns, already through the output-side transform and the output scales (both
-        // are linear, so launch 2 only has to add the zs partials up)
-        float a0 = xw_all[0][lane], a1 = xw_all[0][lane + 64];
-        for (u32 w = 1; w < nw; w++) {
-            a0 += xw_all[w][lane];
-            a1 += xw_all[w][lane + 64];
+    lds_barrier();
+}
+
+// The products of one wave: its ring's units (requested up to D) against the A rows; acc[g][c]: row 4 a + part of lane group
+// a = lane / 16 is part 0..2 of token 4 g + a (row 4 a + 3 belongs to nobody), column lane % 16 of column tile c.
+template <int K, bool H, int CT, int NG, int NMAX>
+__device__ __forceinline__ void verify_products(const VerifyRing<K, H, CT>& ring, const u32* wb, const u16* a_sh, u32 lane, f32x4 (&acc)[NG][CT]) {
+    typedef VerifyRing<K, H, CT> R;
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    typedef u32 u32x4v __attribute__((ext_vector_type(4)));
+    constexpr bool one_shift = 16 + 3 * K + 2 * (int) H <= 32;
+    constexpr u32 NR = 3 * NMAX;
+    const u32 n16 = lane & 15, a = lane >> 4;
+    const u32 t0 = 32 * (n16 & 7) + 8 * a + 4 * (n16 >> 3);
+    // the 32 stream bits that end at bit e (exclusive) of the tile's ring: word jp holds the last of them, word jm the rest
+    auto window = [&](u32 e, u32& om, u32& op, u32& sh) {
+        op = (e - 1) >> 5;
+        om = op == 0 ? R::TW - 1 : op - 1;
+        sh = 31 - ((e - 1) & 31);
+    };
+    u32 om1, op1, sh1, om0 = 0, op0 = 0, sh0 = 0;
+    window(H ? (t0 / 2 + 2) * (2 * K + 1) : (t0 + 4) * K, om1, op1, sh1);
+    if constexpr (!one_shift) window((t0 + 2) * K, om0, op0, sh0);
+    const u16* ar = a_sh + ((n16 >> 2) * 3 + min(n16 & 3, 2u)) * 32 + a * 8;
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int c = 0; c < CT; c++) acc[g][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    u32 slot = 0;
+#pragma unroll 1
+    for (u32 unit = 0; unit < ring.units; unit++) {
+        R::wait(min((u32) R::D - 1, ring.units - 1 - unit));
+        const u32* row = wb + slot * R::UW;
+        u32 w1[16][2], w0[one_shift ? 1 : 16][2];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            w1[i][0] = row[i * R::TW + om1];
+            w1[i][1] = row[i * R::TW + op1];
+            if constexpr (!one_shift) {
+                w0[i][0] = row[i * R::TW + om0];
+                w0[i][1] = row[i * R::TW + op0];
+            }
         }
-        wht128_wave(a0, a1, lane);
-        const u16* sv = (const u16*) sv_out;
-        float* o = gup + ((u64) blockIdx.y * gridDim.z + blockIdx.z) * ff + blockIdx.x * 128;
-        __builtin_nontemporal_store(a0 * f16_to_f32(sv[lane]), &o[lane]);
-        __builtin_nontemporal_store(a1 * f16_to_f32(sv[lane + 64]), &o[lane + 64]);
+        u32x4v av[R::UR / 2][NG];
+#pragma unroll
+        for (int s = 0; s < R::UR / 2; s++)
+#pragma unroll
+            for (int g = 0; g < NG; g++) av[s][g] = *(const u32x4v*) (ar + ((unit * (R::UR / 2) + s) * NR + 12 * g) * 32);
+        if (unit + R::D < ring.units) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the unit's words are in registers, its slot can take the unit D further on
+            ring.issue(unit + R::D, slot, lane);
+        }
+        slot = slot + 1 == (u32) R::D ? 0u : slot + 1;
+#pragma unroll
+        for (int s = 0; s < R::UR / 2; s++) {
+#pragma unroll
+            for (int c = 0; c < CT; c++) {
+                u32 b[2][2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int i = (2 * s + h) * CT + c;
+                    const u32 hi = __builtin_amdgcn_alignbit(w1[i][0], w1[i][1], sh1);
+                    u32 s0, s1;
+                    if constexpr (one_shift) {
+                        s0 = __builtin_amdgcn_ubfe(hi, 3 * K + 2 * (int) H, 16);
+                        s1 = __builtin_amdgcn_ubfe(hi, 2 * K + (int) H, 16);
+                    } else {
+                        const u32 lo = __builtin_amdgcn_alignbit(w0[i][0], w0[i][1], sh0);
+                        s0 = __builtin_amdgcn_ubfe(lo, K, 16);
+                        s1 = lo & 0xffffu;
+                    }
+                    const u32 s2 = __builtin_amdgcn_ubfe(hi, K + (int) H, 16), s3 = hi & 0xffffu;
+                    b[h][0] = __builtin_bit_cast(u32, exl3_cb2_pair(s0, s1));
+                    b[h][1] = __builtin_bit_cast(u32, exl3_cb2_pair(s2, s3));
+                }
+                const f16x8 bv = __builtin_bit_cast(f16x8, u32x4v{b[0][0], b[0][1], b[1][0], b[1][1]});
+#pragma unroll
+                for (int g = 0; g < NG; g++) acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, av[s][g]), bv, acc[g][c], 0, 0, 0);
+            }
+        }
     }
 }
 
-// Launch 2: act = silu(gate) * up of the pair, from the sums of launch 1's zs partials, by every wave for the 128-block of
-// act it is about to use (16-fold redundant work of a hundred operations, instead of a launch), then the down
-// product's partial sums: dn[pair * gridDim.z + z][hidden].  grid = (hidden / 128, S, ceil(ff / 512)), block 256.
-template <int K, bool H = false, bool XH = false>
-__device__ __forceinline__ void verify_down_kernel(const float* __restrict__ logits, u64 ebase, u64 estride, u64 shbase, u32 part,
-                                                   u8* __restrict__ pbuf, const float* __restrict__ gup, float* __restrict__ dn, u32 ne, u32 k, u32 m,
-                                                   u32 hidden, u32 ff, u32 zs) {
-    __shared__ __attribute__((aligned(16))) u32 wb_all[4][Exl3Rows<K, 8, H>::words];
-    __shared__ float xw_all[4][128];
-    __shared__ u32 sc_all[4][64];      // the wave's 128 f16 scales of down's inputs
+// The item's sums out of the accumulators: token 4 g + a of lane group a into out + (its pair) * stride, the wave's columns.
+template <int CT, int NG>
+__device__ __forceinline__ void verify_store(const f32x4 (&acc)[NG][CT], const float* s_iv, const u32 (&pairs)[4], u32 n, u64 stride, float* out, u32 lane) {
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        const u32 r = 4 * g + (lane >> 4);
+        if (r < n) {
+            const float iv = s_iv[r];
+            const u64 four = (u64) pairs[2 * g] | ((u64) pairs[2 * g + 1] << 32);
+            const u32 pair = (u32) (four >> (lane & 48)) & 0xffffu;
+            float* o = out + (u64) pair * stride + (lane & 15);
+#pragma unroll
+            for (int c = 0; c < CT; c++) o[16 * c] = (acc[g][c][0] + acc[g][c][1] + acc[g][c][2]) * iv;
+        }
+    }
+}
+
+// The shared expert's item: every token, pairs m k + j.
+__device__ __forceinline__ void verify_shared_item(u32 G, u64& toks, u32 (&pairs)[4]) {
+    toks = 0x0706050403020100ull;
+#pragma unroll
+    for (int i = 0; i < 4; i++) pairs[i] = (G + 2 * i) | ((G + 2 * i + 1) << 16);
+}
+
+// Launch 2: the gate and up products of every item, gup[(((layer * 2 + sel) * S + pair) * zs + z) * ff + column], S = m (k + 1),
+// sel 0 = gate, 1 = up, z = the block of 512 inputs.  grid = (ff / (64 CT), 2 slots, layers zs), slots = m k + 2: at least one
+// more than a layer can have items.  block 256.
+// ioff = 0 (one layer): there is no plan, launch 1 does not run.  The items are the shared expert and then the (token,
+// rank) pairs, one token each (slots = m k + 1); the workgroups select for themselves and launch 3 works the weights out.  A layer of a
+// call of its own takes this form where few tokens can share an expert: the pairs' weights are decoded once each, which
+// costs less than another launch ahead of everything.  A token's sums do not depend on the other tokens of an item: both
+// forms give the same bits.
+template <int K, bool H, int CT, int NG>
+__device__ __forceinline__ void verify_gate_up_kernel(const float* __restrict__ logits, const u8* __restrict__ table, u64 experts, u64 stride, u64 shared, u32 part,
+                                                      u32 base, const u8* __restrict__ plans, u8* __restrict__ weights, u32 plan_stride, u32 ioff, const float* __restrict__ u, float* __restrict__ gup, u32 ne, u32 k, u32 m,
+                                                      u32 hidden, u32 ff) {
+    constexpr int NMAX = 4 * NG;
+    typedef VerifyRing<K, H, CT> R;
+    __shared__ __attribute__((aligned(16))) u32 wb_all[4][R::D * R::UW];
+    __shared__ __attribute__((aligned(16))) u16 a_sh[16 * 3 * NMAX * 32];
+    __shared__ __attribute__((aligned(16))) float s_mx[4 * NMAX];
+    __shared__ float s_iv[NMAX];
+    __shared__ u32 s_top[16];
+    static_assert(sizeof(a_sh) >= 512 * sizeof(double), "the exact selection's scratch");
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const u32 zs = (hidden / 128 + 3) / 4, li = blockIdx.z / zs, z = blockIdx.z - li * zs;
+    const u32 slots = gridDim.y >> 1, sel = blockIdx.y >= slots ? 1u : 0u, it = blockIdx.y - sel * slots;
+    const VerifyLayer L = verify_layer(table, li, experts, stride, shared, part, base);
+    const u32 l = L.layer - base;
     const u32 G = m * k, S = G + m;
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // the wave index as a scalar: the index arithmetic on it is the scalar unit's
-    // Which (pair, column block) this workgroup takes.  Workgroup i of a launch runs on XCD i % 8, each with an L2 of its own,
-    // and the 16 workgroups of a pair all read the pair's partial sums from launch 1: in launch order they sit on all eight
-    // XCDs and the sums are fetched into eight L2s.  Where the shape allows, sets of 8 column blocks of one pair go to one
-    // XCD instead (unit u = the set; the workgroups i with the same i % 8 and the same i / 64 share it), so two L2s fetch them.
-    u32 pair = blockIdx.y, cbx = blockIdx.x;
-    if (gridDim.z == 1 && gridDim.x % 8 == 0 && (gridDim.x / 8 * gridDim.y) % 8 == 0) {
-        const u32 i = blockIdx.y * gridDim.x + blockIdx.x, unit = (i >> 6) * 8 + (i & 7), per = gridDim.x / 8;   // `per` runs a pair
-        pair = unit / per;
-        cbx = ((i >> 3) & 7) * per + unit % per;   // every per-th column block: the run's rows of the trellis spread over the row as the launch order's would
-    }
-    if (logits != nullptr && pair < G && pair % k == 0 && cbx == 0 && blockIdx.z == 0 && wave == 3) {
-        // one wave a token: the routing weights and the count, for launch 3 (nothing in this launch reads them)
-        const u32 j = pair / k;
-        u32 kk;
-        const float wt = route_weights(logits + (u64) j * ne, ne, k, lane, (const u32*) pbuf + pair, &kk);
-        if (lane < k) ((float*) (pbuf + G * 4))[pair + lane] = wt;
-        if (lane == 0) ((u32*) (pbuf + 2 * G * 4))[j] = kk;
-    }
-    const u32 kb = blockIdx.z * 4 + wave;
-    const u32 kbs = ff / 128;
-    // launch 1's partial sums of the wave's block of gate and up only depend on the pair: requested before its expert is known
-    float g0 = 0.0f, g1 = 0.0f, u0 = 0.0f, u1 = 0.0f;
-    float pv[4][4];
-    u32 e = 0;
-    if (pair < G) e = ((const u32*) pbuf)[pair];
-    if (kb < kbs) {
-        // the first four partials' loads all go out before any is waited for (a loop would take them a round trip at a time),
-        // and without the compiler's count: the wave's rows are requested as soon as its expert is known, behind these loads
-        // and without waiting for them, and the sums are taken once exactly these have landed
+    u32 e, n, pairs[4];
+    u64 toks;
+    if (ioff) {
+        const u32* plan = (const u32*) (plans + (u64) l * plan_stride + ioff);
+        const u32* rec = plan + 4 + 8 * it;   // there for every slot, an item or not: read along with the count
+        e = rec[0];
+        n = __builtin_amdgcn_readfirstlane(min(rec[1], (u32) NMAX));
+        toks = (u64) rec[2] | ((u64) rec[3] << 32);
 #pragma unroll
-        for (int z = 0; z < 4; z++) {
-            const u32 zz = min((u32) z, zs - 1);
-            const float* pg = gup + ((u64) pair * zs + zz) * ff + kb * 128;
-            const float* pu = gup + ((u64) (S + pair) * zs + zz) * ff + kb * 128;
-            pv[z][0] = load_f32_uncounted(pg + lane);
-            pv[z][1] = load_f32_uncounted(pg + lane + 64);
-            pv[z][2] = load_f32_uncounted(pu + lane);
-            pv[z][3] = load_f32_uncounted(pu + lane + 64);
+        for (int i = 0; i < 4; i++) pairs[i] = __builtin_amdgcn_readfirstlane(rec[4 + i]);
+        if (it >= plan[0]) {
+            // the last slot is never an item: one of its workgroups works the layer's routing weights out for the last launch
+            // while the others multiply
+            if (blockIdx.y == gridDim.y - 1 && blockIdx.x == 0 && z == 0)
+                verify_route_weights(logits + (u64) l * m * ne, weights + (u64) l * plan_stride, ne, k, m, wave, lane);
+            return;
         }
+    } else if (it > 0) {
+        // no plan: a workgroup redoes its token's selection on one of its waves (not always the same one: the prologues of
+        // co-resident workgroups spread over the SIMDs), ahead of the decoding waves of other workgroups on its SIMD
+        const u32 pair = it - 1, j = pair / k, t = pair - j * k;
+        if (wave == (blockIdx.x + blockIdx.y + blockIdx.z) % 4) {
+            __builtin_amdgcn_s_setprio(3);
+            route_id_of_rank(logits + (u64) j * ne, ne, k, t, lane, (double*) &a_sh[0], s_top);   // only s_top[t] is read
+            __builtin_amdgcn_s_setprio(0);
+            if (sel == 0 && blockIdx.x == 0 && z == 0 && lane == 0) ((u32*) weights)[pair] = s_top[t];
+        }
+        __syncthreads();
+        e = __builtin_amdgcn_readfirstlane(s_top[t]);
+        if (e == 0xffffffffu) return;
+        n = 1;
+        toks = j;
+        pairs[0] = pair;
+        pairs[1] = pairs[2] = pairs[3] = 0;
+    } else {
+        if (!L.shared) return;
+        e = 0xffffffffu;
+        n = m;
+        verify_shared_item(G, toks, pairs);
     }
-    if (pair < G ? e == 0xffffffffu : shbase == 0) return;
-    const u8* bp = (const u8*) (pair < G ? ebase + e * estride : shbase);
-    float* xw = xw_all[wave];
-    u32 svb0 = 0, svb1 = 0;   // wave 0 of a launch without a split over the inputs: down's output scales of the block (needed at the end)
-    if (gridDim.z == 1 && wave == 0) {
-        const u16* svh = (const u16*) (bp + 2 * (u64) part + 2 * (u64) ff) + cbx * 128;
-        svb0 = load_u16_uncounted(svh + lane);
-        svb1 = load_u16_uncounted(svh + lane + 64);
-    }
-    if (kb < kbs) {
-        // no load the compiler counts is in flight here: what is, is counted by hand
-        const u32 sc_lds = __builtin_amdgcn_readfirstlane(lds_offset(sc_all[wave]));
-        const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave]));
-        const u8* down = bp + 2 * (u64) part;
-        lds_load<4>(down + kb * 256 + lane * 4, sc_lds);                                  // down's input scales
-        const u32* row0 = (const u32*) (down + 2 * (u64) ff + 2 * (u64) hidden + 4) + ((u64) kb * 8 * (hidden / 16) + cbx * 8) * EXL3_TILE_WORDS(K, H);
-        const u64 pitch = (u64) (hidden / 16) * EXL3_TILE_WORDS(K, H);
-        exl3_rows_issue<K, 8, H>(row0, pitch, lane, wb_lds);
-        wait_vm<Exl3Rows<K, 8, H>::loads + 1>();   // the partial sums, requested before the burst, have landed
+    const u8* bp = (const u8*) uniform_u64((e == 0xffffffffu ? L.shared : L.experts + e * L.stride) + (u64) sel * L.part);
+    const u32 kbs = hidden / 128, kb = z * 4 + wave, nkb = min(4u, kbs - z * 4);
+    const u32 c0 = blockIdx.x * 4 * CT + wave * CT;   // the wave's first column tile
+    R ring;
+    ring.init(bp + 2 * (u64) hidden + 2 * (u64) ff + 4 + ((u64) z * 32 * (ff / 16) + c0) * (4 * R::TW), (ff / 16) * (4 * R::TW), nkb * 8 / R::UR,
+              __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave])), lane);
+    // the wave's 128-block of every token and its scales, then the first units of its rows behind them, uncounted.  Every load
+    // is made, past the item's tokens and blocks of an earlier one: a load behind a branch would leave its register to be
+    // copied at the branches' end, before the value is there.
+    float v[NMAX][2];
+    const u32 kbc = min(kb, kbs - 1);
+    const u16* suh = (const u16*) bp + kbc * 128;
+    u32 sc0 = load_u16_uncounted(suh + lane), sc1 = load_u16_uncounted(suh + lane + 64);
 #pragma unroll
-        for (int z = 0; z < 4; z++) {
+    for (int r = 0; r < NMAX; r++) {
+        const u32 tok = (u32) (toks >> (8 * min((u32) r, n - 1))) & 0xffu;
+        const float* xj = u + ((u64) l * m + tok) * hidden + kbc * 128;
+        v[r][0] = load_f32_uncounted(xj + lane);
+        v[r][1] = load_f32_uncounted(xj + lane + 64);
+    }
+    ring.fill(lane);
+    load_landed(sc0);
+    load_landed(sc1);
 #pragma unroll
-            for (int c = 0; c < 4; c++) load_landed(pv[z][c]);
-            if ((u32) z < zs) {
-                g0 += pv[z][0];
-                g1 += pv[z][1];
-                u0 += pv[z][2];
-                u1 += pv[z][3];
-            }
-        }
-        for (u32 z = 4; z < zs; z++) {   // (hidden above 2048: these wait for the burst too)
-            const float* pg = gup + ((u64) pair * zs + z) * ff + kb * 128;
-            const float* pu = gup + ((u64) (S + pair) * zs + z) * ff + kb * 128;
-            g0 += pg[lane];
-            g1 += pg[lane + 64];
-            u0 += pu[lane];
-            u1 += pu[lane + 64];
-        }
-        // the wave's 128-block of act = silu(gate) * up (launch 1 left gate and up finished but for the sum over its
-        // partials), rotated into the down projection's basis, into its strip
-        wait_vm<Exl3Rows<K, 8, H>::loads>();
-        const u16* suh = (const u16*) sc_all[wave];
-        float a0 = (siluf_ref(g0) * u0) * f16_to_f32(suh[lane]);
-        float a1 = (siluf_ref(g1) * u1) * f16_to_f32(suh[lane + 64]);
-        wht128_wave(a0, a1, lane);
-        float unscale = 1.0f;
-        if constexpr (XH) {
-            unscale = exl3_put_x_f16((u16*) xw, a0, a1, lane);
-        } else {
-            xw[lane] = a0;
-            xw[64 + lane] = a1;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        exl3_wave_stream<K, 8, H, XH>(row0, pitch, 8, wb_all[wave], wb_lds, xw, lane, unscale);
+    for (int r = 0; r < NMAX; r++) {
+        load_landed(v[r][0]);
+        load_landed(v[r][1]);
     }
-    __syncthreads();
-    const u32 nw = min(4u, kbs - blockIdx.z * 4);
-    if (gridDim.z == 1) {
-        // the workgroup holds the whole sum over the inputs: it finishes its block here (output-side transform, scales), and
-        // launch 3 only weights and adds
-        if (wave == 0) {
-            wait_vm<0>();
-            load_landed(svb0);
-            load_landed(svb1);
-            const float sv0 = f16_to_f32((u16) svb0), sv1 = f16_to_f32((u16) svb1);
-            float a0 = xw_all[0][lane], a1 = xw_all[0][lane + 64];
-            for (u32 w = 1; w < nw; w++) {
-                a0 += xw_all[w][lane];
-                a1 += xw_all[w][lane + 64];
-            }
-            wht128_wave(a0, a1, lane);
-            float* o = dn + (u64) pair * hidden + cbx * 128;
-            __builtin_nontemporal_store(a0 * sv0, &o[lane]);
-            __builtin_nontemporal_store(a1 * sv1, &o[lane + 64]);
+#pragma unroll
+    for (int r = 0; r < NMAX; r++) {
+        if ((u32) r < n) {
+            v[r][0] *= f16_to_f32((u16) sc0);
+            v[r][1] *= f16_to_f32((u16) sc1);
+            wht128_wave(v[r][0], v[r][1], lane);
+            if (kb >= kbs) v[r][0] = v[r][1] = 0.0f;
         }
-    } else if (threadIdx.x < 128) {
-        float a = xw_all[0][threadIdx.x];
-        for (u32 w = 1; w < nw; w++) a += xw_all[w][threadIdx.x];
-        dn[((u64) pair * gridDim.z + blockIdx.z) * hidden + cbx * 128 + threadIdx.x] = a;
     }
+    verify_put_rows<NMAX>(a_sh, s_mx, s_iv, v, n, kb < kbs ? wave : 4u, wave, lane);
+    f32x4 acc[NG][CT];
+    verify_products<K, H, CT, NG, NMAX>(ring, wb_all[wave], a_sh, lane, acc);
+    verify_store<CT, NG>(acc, s_iv, pairs, n, (u64) zs * ff, gup + (((u64) (li * 2 + sel) * S) * zs + z) * ff + c0 * 16, lane);
 }
 
-// workgroups of 4 waves a CU that the LDS buffers leave room for (160 KiB a CU): the register budget follows it
-#define EXL3_VERIFY_WAVES(K) ((K) <= 1 ? 8 : (K) == 2 ? 7 : (K) <= 4 ? 4 : (K) <= 5 ? 3 : 2)
-// waves a SIMD of launch 1 that its LDS leaves room for (4-row rings)
-#define EXL3_GU_OCC(K) ((K) <= 4 ? 8 : (K) == 5 ? 6 : 4)
-#define EXL3_VERIFY_ENTRIES(K)                                                                                                            \
-    extern "C" __global__ void __launch_bounds__(64 * EXL3_GU_WAVES, EXL3_GU_OCC(K)) verify_gate_up_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, \
-                                                                                  const float* u, u8* pbuf, float* gup, u32 ne, u32 k, u32 m, \
-                                                                                  u32 hidden, u32 ff, const float* cdn, const u8* cpbuf,      \
-                                                                                  const float* cgl, float* cy, u32 cmode) {                   \
-        verify_gate_up_kernel<K>(logits, ebase, estride, shbase, part, u, pbuf, gup, ne, k, m, hidden, ff, cdn, cpbuf, cgl, cy, cmode);   \
-    }                                                                                                                                     \
-    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_WAVES(K)) verify_down_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part,   \
-                                                                               u8* pbuf, const float* gup, float* dn, u32 ne, u32 k, u32 m,   \
-                                                                               u32 hidden, u32 ff, u32 zs) {                                  \
-        verify_down_kernel<K>(logits, ebase, estride, shbase, part, pbuf, gup, dn, ne, k, m, hidden, ff, zs);                             \
+// Launch 3: act = silu(gate) * up of every token of the item out of launch 2's sums (partials added, output side of the two
+// projections), rotated into the down projection's basis as A rows, then its products: dn[((layer * S + pair) * zd + z) *
+// hidden + column], zd = ceil(ff / 512).  grid = (hidden / (64 CT), slots, layers zd), block 256.
+template <int K, bool H, int CT, int NG>
+__device__ __forceinline__ void verify_down_kernel(const float* __restrict__ logits, const u8* __restrict__ table, u64 experts, u64 stride, u64 shared, u32 part0, u32 base,
+                                                   const u8* __restrict__ plans, u8* __restrict__ weights, u32 plan_stride, u32 ioff, const float* __restrict__ gup, float* __restrict__ dn,
+                                                   u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    constexpr int NMAX = 4 * NG;
+    typedef VerifyRing<K, H, CT> R;
+    __shared__ __attribute__((aligned(16))) u32 wb_all[4][R::D * R::UW];
+    __shared__ __attribute__((aligned(16))) u16 a_sh[16 * 3 * NMAX * 32];
+    __shared__ __attribute__((aligned(16))) float s_mx[4 * NMAX];
+    __shared__ float s_iv[NMAX];
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const u32 zs = (hidden / 128 + 3) / 4, zd = (ff / 128 + 3) / 4, li = blockIdx.z / zd, z = blockIdx.z - li * zd, it = blockIdx.y;
+    const VerifyLayer L = verify_layer(table, li, experts, stride, shared, part0, base);
+    const u8* pbuf = plans + (u64) (L.layer - base) * plan_stride;
+    const u32 G = m * k, S = G + m;
+    u32 e, n, pairs[4];
+    if (ioff) {
+        const u32* plan = (const u32*) (pbuf + ioff);
+        const u32* rec = plan + 4 + 8 * it;
+        e = rec[0];
+        n = __builtin_amdgcn_readfirstlane(min(rec[1], (u32) NMAX));
+#pragma unroll
+        for (int i = 0; i < 4; i++) pairs[i] = __builtin_amdgcn_readfirstlane(rec[4 + i]);
+        if (it >= plan[0]) return;
+    } else if (it > 0) {
+        const u32 pair = it - 1;
+        if (pair % k == 0 && blockIdx.x == 0 && z == 0 && wave == 3) {
+            // one wave a token: the routing weights and the count, for launch 4 (nothing in this launch reads them)
+            const u32 j = pair / k;
+            u32 kk;
+            const float wt = route_weights_chosen(logits + (u64) j * ne, ne, k, lane, (const u32*) pbuf + pair, &kk);
+            if (lane < k) ((float*) (weights + G * 4))[pair + lane] = wt;
+            if (lane == 0) ((u32*) (weights + 2 * G * 4))[j] = kk;
+        }
+        e = ((const u32*) pbuf)[pair];
+        if (e == 0xffffffffu) return;
+        n = 1;
+        pairs[0] = pair;
+        pairs[1] = pairs[2] = pairs[3] = 0;
+    } else {
+        if (!L.shared) return;
+        u64 toks;
+        e = 0xffffffffu;
+        n = m;
+        verify_shared_item(G, toks, pairs);
     }
-
-// The same launches with the rotated inputs rounded to f16 and two products an instruction (session expert mode 3).
-#define EXL3_VERIFY_F16_ENTRIES(K)                                                                                                        \
-    extern "C" __global__ void __launch_bounds__(64 * EXL3_GU_WAVES, EXL3_GU_OCC(K)) verify_gate_up_exl3f_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, \
-                                                                                  const float* u, u8* pbuf, float* gup, u32 ne, u32 k, u32 m, \
-                                                                                  u32 hidden, u32 ff, const float* cdn, const u8* cpbuf,      \
-                                                                                  const float* cgl, float* cy, u32 cmode) {                   \
-        verify_gate_up_kernel<K, false, true>(logits, ebase, estride, shbase, part, u, pbuf, gup, ne, k, m, hidden, ff, cdn, cpbuf, cgl, cy, cmode); \
-    }                                                                                                                                     \
-    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_WAVES(K)) verify_down_exl3f_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part,   \
-                                                                               u8* pbuf, const float* gup, float* dn, u32 ne, u32 k, u32 m,   \
-                                                                               u32 hidden, u32 ff, u32 zs) {                                  \
-        verify_down_kernel<K, false, true>(logits, ebase, estride, shbase, part, pbuf, gup, dn, ne, k, m, hidden, ff, zs);                \
+    const u8* bp = (const u8*) uniform_u64(e == 0xffffffffu ? L.shared : L.experts + e * L.stride);
+    const u64 part = L.part;
+    const u32 kbs = ff / 128, kb = z * 4 + wave, nkb = min(4u, kbs - z * 4);
+    float rot[NMAX][2];
+#pragma unroll
+    for (int r = 0; r < NMAX; r++) rot[r][0] = rot[r][1] = 0.0f;
+    const u32 c0 = blockIdx.x * 4 * CT + wave * CT;
+    R ring;
+    ring.init(bp + 2 * part + 2 * (u64) ff + 2 * (u64) hidden + 4 + ((u64) z * 32 * (hidden / 16) + c0) * (4 * R::TW), (hidden / 16) * (4 * R::TW),
+              nkb * 8 / R::UR, __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave])), lane);
+    if (kb < kbs) {
+        const float* g0 = gup + ((u64) li * 2 * S * zs) * ff + kb * 128 + lane;
+        // gate's and up's output scales and down's input scales of the block
+        u32 sc[6];
+        const u16* svg = (const u16*) (bp + 2 * (u64) hidden) + kb * 128 + lane;
+        const u16* svu = (const u16*) (bp + part + 2 * (u64) hidden) + kb * 128 + lane;
+        const u16* sud = (const u16*) (bp + 2 * part) + kb * 128 + lane;
+        sc[0] = load_u16_uncounted(svg);
+        sc[1] = load_u16_uncounted(svg + 64);
+        sc[2] = load_u16_uncounted(svu);
+        sc[3] = load_u16_uncounted(svu + 64);
+        sc[4] = load_u16_uncounted(sud);
+        sc[5] = load_u16_uncounted(sud + 64);
+#pragma unroll
+        for (int r0 = 0; r0 < NMAX; r0 += 2) {
+            if ((u32) r0 < n) {
+                // two tokens at a time, the first four partials of each requested together; the first lot goes out ahead of the rows
+                float pv[2][4][4];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    // (a lot's second token past the item's: its first again, so that no load stands behind a branch)
+                    const u32 pair = ((u32) (r0 + q) < n ? pairs[r0 / 2] >> (16 * q) : pairs[r0 / 2]) & 0xffffu;
+                    const float* pg = g0 + (u64) pair * zs * ff;
+                    const float* pu = g0 + (u64) (S + pair) * zs * ff;
+#pragma unroll
+                    for (int zz = 0; zz < 4; zz++) {
+                        const u64 o = (u64) min((u32) zz, zs - 1) * ff;
+                        pv[q][zz][0] = load_f32_uncounted(pg + o);
+                        pv[q][zz][1] = load_f32_uncounted(pg + o + 64);
+                        pv[q][zz][2] = load_f32_uncounted(pu + o);
+                        pv[q][zz][3] = load_f32_uncounted(pu + o + 64);
+                    }
+                }
+                if (r0 == 0) {
+                    ring.fill(lane);
+#pragma unroll
+                    for (int i = 0; i < 6; i++) load_landed(sc[i]);
+                } else {
+                    wait_vm<0>();
+                }
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+#pragma unroll
+                    for (int zz = 0; zz < 4; zz++)
+#pragma unroll
+                        for (int c = 0; c < 4; c++) load_landed(pv[q][zz][c]);
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const int r = r0 + q;
+                    if ((u32) r < n) {
+                        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int zz = 0; zz < 4; zz++)
+#pragma unroll
+                            for (int c = 0; c < 4; c++) t[c] += (u32) zz < zs ? pv[q][zz][c] : 0.0f;
+                        if (zs > 4) {
+                            const u32 pair = (pairs[r / 2] >> (16 * (r & 1))) & 0xffffu;
+                            for (u32 zz = 4; zz < zs; zz++) {
+                                const float* pg = g0 + ((u64) pair * zs + zz) * ff;
+                                const float* pu = g0 + ((u64) (S + pair) * zs + zz) * ff;
+                                t[0] += pg[0];
+                                t[1] += pg[64];
+                                t[2] += pu[0];
+                                t[3] += pu[64];
+                            }
+                        }
+                        wht128_wave(t[0], t[1], lane);
+                        wht128_wave(t[2], t[3], lane);
+                        rot[r][0] = siluf_ref(t[0] * f16_to_f32((u16) sc[0])) * (t[2] * f16_to_f32((u16) sc[2])) * f16_to_f32((u16) sc[4]);
+                        rot[r][1] = siluf_ref(t[1] * f16_to_f32((u16) sc[1])) * (t[3] * f16_to_f32((u16) sc[3])) * f16_to_f32((u16) sc[5]);
+                        wht128_wave(rot[r][0], rot[r][1], lane);
+                    }
+                }
+            }
+        }
+    } else {
+        ring.fill(lane);
     }
+    verify_put_rows<NMAX>(a_sh, s_mx, s_iv, rot, n, kb < kbs ? wave : 4u, wave, lane);
+    f32x4 acc[NG][CT];
+    verify_products<K, H, CT, NG, NMAX>(ring, wb_all[wave], a_sh, lane, acc);
+    verify_store<CT, NG>(acc, s_iv, pairs, n, (u64) zd * hidden, dn + ((u64) li * S * zd + z) * hidden + c0 * 16, lane);
+}
 
-// K + 1/2 bits a weight: the LDS and register budget of the next whole rate
-#define EXL3_VERIFY_HALF_ENTRIES(K)                                                                                                       \
-    extern "C" __global__ void __launch_bounds__(64 * EXL3_GU_WAVES, EXL3_GU_OCC(K + 1)) verify_gate_up_exl3h_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, \
-                                                                                  const float* u, u8* pbuf, float* gup, u32 ne, u32 k, u32 m, \
-                                                                                  u32 hidden, u32 ff, const float* cdn, const u8* cpbuf,      \
-                                                                                  const float* cgl, float* cy, u32 cmode) {                   \
-        verify_gate_up_kernel<K, true>(logits, ebase, estride, shbase, part, u, pbuf, gup, ne, k, m, hidden, ff, cdn, cpbuf, cgl, cy, cmode); \
-    }                                                                                                                                     \
-    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_WAVES(K + 1)) verify_down_exl3h_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, \
-                                                                               u8* pbuf, const float* gup, float* dn, u32 ne, u32 k, u32 m,   \
-                                                                               u32 hidden, u32 ff, u32 zs) {                                  \
-        verify_down_kernel<K, true>(logits, ebase, estride, shbase, part, pbuf, gup, dn, ne, k, m, hidden, ff, zs);                       \
+// Occupancy: workgroups a compute unit's LDS (160 KiB) holds; the register budget follows it.
+#define EXL3_VERIFY_OCC(K, NG) ((NG) == 1 ? ((K) <= 2 ? 6 : (K) == 3 ? 5 : (K) <= 6 ? 4 : 3) : ((K) <= 2 ? 4 : 3))
+// CT = 8 column tiles a wave (plain name), or 4 or 2 (t4, t2: shorter waves, for launches that would leave the chip idle);
+// w: batches of more than 4 rows.
+#define EXL3_VERIFY_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_gate_up_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 8, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 8, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_gate_up_t4_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 4, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_t4_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 4, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_gate_up_t2_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 2, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_t2_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 2, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_gate_up_w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 8, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 8, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_gate_up_t4w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 4, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_t4w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 4, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_gate_up_t2w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, false, 2, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_t2w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 2, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
     }
-
-EXL3_VERIFY_HALF_ENTRIES(1)
-EXL3_VERIFY_HALF_ENTRIES(2)
-EXL3_VERIFY_HALF_ENTRIES(3)
-
-EXL3_VERIFY_F16_ENTRIES(1)
-EXL3_VERIFY_F16_ENTRIES(2)
-EXL3_VERIFY_F16_ENTRIES(3)
-EXL3_VERIFY_F16_ENTRIES(4)
-EXL3_VERIFY_F16_ENTRIES(5)
-EXL3_VERIFY_F16_ENTRIES(6)
-EXL3_VERIFY_F16_ENTRIES(7)
-EXL3_VERIFY_F16_ENTRIES(8)
-
+#define EXL3_VERIFY_HALF_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_gate_up_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 8, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 8, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_gate_up_t4_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 4, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_t4_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 4, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_gate_up_t2_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 2, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_t2_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 2, 1>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_gate_up_w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 8, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 8, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_gate_up_t4w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 4, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_t4w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 4, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_gate_up_t2w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* u, float* gup, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_gate_up_kernel<K, true, 2, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, u, gup, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_t2w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 2, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    }
 EXL3_VERIFY_ENTRIES(1)
 EXL3_VERIFY_ENTRIES(2)
 EXL3_VERIFY_ENTRIES(3)
@@ -885,39 +1018,39 @@ EXL3_VERIFY_ENTRIES(5)
 EXL3_VERIFY_ENTRIES(6)
 EXL3_VERIFY_ENTRIES(7)
 EXL3_VERIFY_ENTRIES(8)
+EXL3_VERIFY_HALF_ENTRIES(1)
+EXL3_VERIFY_HALF_ENTRIES(2)
+EXL3_VERIFY_HALF_ENTRIES(3)
 
-// Launch 3: token j = blockIdx.y, output block blockIdx.x: y[j] = sum over its cnt[j] experts t, in rank order, of
-// w[j,t] * (the finished down product of pair j k + t) + sigmoid(gl[j]) * (the shared expert's).  Wave t finishes expert t
-// (wave k the shared one), then the first two waves add them up in rank order (moe_combine_qwen_rows,
-// kernels/forward.cu:2568).  zs = launch 2's gridDim.z, or 0 when that was 1 and launch 2 has left finished blocks in dn:
-// then 128 threads a workgroup do.  grid = (hidden / 128, m), block 1024 (k <= 16) or 128.
-extern "C" __global__ void __launch_bounds__(1024) verify_combine_exl3(const float* dn, u64 ebase, u64 estride, u64 shbase, u32 part, const u8* pbuf,
-                                                                       const float* gl, float* y, u32 k, u32 m, u32 hidden, u32 ff, u32 zs) {
+// Launch 4: token j = blockIdx.y of layer blockIdx.z, output block blockIdx.x: y[j] = sum over its cnt[j] experts t, in rank order,
+// of w[j,t] * (the down product of pair j k + t) + sigmoid(gl[j]) * (the shared expert's).  Wave t finishes expert t (partials
+// added, output-side transform, scales; the shared one on a wave of its own, or on wave 0 at k = 16), then the first two waves
+// add them up in rank order (moe_combine_qwen_rows, kernels/forward.cu:2568).  grid = (hidden / 128, m, layers), block 64 times
+// the experts of a token (at most 1024).
+extern "C" __global__ void __launch_bounds__(1024) verify_combine_exl3(const float* dn, const u8* table, u64 experts, u64 stride, u64 shared0, u32 part, u32 base, const u8* plans,
+                                                                       u32 plan_stride, const float* gl, float* y, u32 k, u32 m, u32 hidden, u32 ff) {
     __shared__ float sums[17][128];
-    const u32 lane = threadIdx.x & 63, t = threadIdx.x >> 6, ob = blockIdx.x, j = blockIdx.y;
-    const u32 G = m * k;
+    const u32 lane = threadIdx.x & 63, t = threadIdx.x >> 6, ob = blockIdx.x, j = blockIdx.y, li = blockIdx.z;
+    const VerifyLayer L = verify_layer(table, li, experts, stride, shared0, part, base);
+    const u32 l = L.layer - base, G = m * k, S = G + m, zd = (ff / 128 + 3) / 4;
+    const u64 shared = L.shared;
+    const u8* pbuf = plans + (u64) l * plan_stride;
     const u32* tidx = (const u32*) pbuf;
     const float* wts = (const float*) (pbuf + G * 4);
-    const u32* cnt = (const u32*) (pbuf + 2 * G * 4);
-    if (zs == 0) {
-        if (t < 2) exl3_combine_finished(dn, pbuf, gl, y, k, m, hidden, shbase != 0, ob, j, threadIdx.x);
-        return;
-    }
-    const u32 c = cnt[j];
-    // one source's block: sum of its partials, output-side transform, scales, weight
+    const u32 c = ((const u32*) (pbuf + 2 * G * 4))[j];
     auto finish = [&](bool routed) {
         // everything that does not depend on the expert is requested first, all at once: the partial sums, the weight, the id
         const u32 pair = routed ? j * k + t : G + j;
         float v0 = 0.0f, v1 = 0.0f;
-        for (u32 z = 0; z < zs; z++) {
-            const float* p = dn + ((u64) pair * zs + z) * hidden + ob * 128;
+        for (u32 z = 0; z < zd; z++) {
+            const float* p = dn + (((u64) li * S + pair) * zd + z) * hidden + ob * 128;
             v0 += p[lane];
             v1 += p[lane + 64];
         }
         const u32 e = routed ? tidx[pair] : 0u;
-        const float wt = routed ? wts[pair] : sigmoidf_ref(gl[j]);
+        const float wt = routed ? wts[pair] : sigmoidf_ref(gl[(u64) l * m + j]);
         if (routed && t >= c) return;
-        const u8* down = (const u8*) (routed ? ebase + e * estride : shbase) + 2 * (u64) part;
+        const u8* down = (const u8*) (routed ? L.experts + e * L.stride : shared) + 2 * (u64) L.part;
         const u16* svh = (const u16*) (down + 2 * (u64) ff) + ob * 128;
         const float s0 = f16_to_f32(svh[lane]), s1 = f16_to_f32(svh[lane + 64]);
         wht128_wave(v0, v1, lane);
@@ -926,13 +1059,13 @@ extern "C" __global__ void __launch_bounds__(1024) verify_combine_exl3(const flo
         o[lane + 64] = wt * (v1 * s1);
     };
     if (t < k) finish(true);
-    if (shbase && t == (k < 16 ? k : 0)) finish(false);   // the shared expert on a wave of its own when there is one to spare
+    if (shared && t == (k < 16 ? k : 0)) finish(false);
     __syncthreads();
     if (threadIdx.x < 128) {
         float a = 0.0f;
         for (u32 i = 0; i < c; i++) a += sums[i][threadIdx.x];
-        if (shbase) a += sums[16][threadIdx.x];
-        y[(u64) j * hidden + ob * 128 + threadIdx.x] = a;
+        if (shared) a += sums[16][threadIdx.x];
+        y[((u64) l * m + j) * hidden + ob * 128 + threadIdx.x] = a;
     }
 }
 
@@ -948,10 +1081,6 @@ extern "C" __global__ void __launch_bounds__(1024) verify_combine_exl3(const flo
 // power of two that takes the token's largest rotated magnitude to [2^14, 2^15), in the same k order: every product with
 // an f16 weight is exact, the matrix core adds in f32, and 8 tokens cost what one costs.
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-
-// Where element q (0..15) of a tile row's 16 inputs sits in the row's 16 slots of an A row: lane group a reads the slots
-// 4 a .. 4 a + 3 = inputs 2 a, 2 a + 1, 2 a + 8, 2 a + 9 as one 8-byte word.
-__device__ __forceinline__ u32 exl3_aslot(u32 q) { return 4 * ((q & 7) >> 1) + 2 * (q >> 3) + (q & 1); }
 
 // Launch 1 of the head: token j = blockIdx.x.  Wave w rotates the 128-blocks w, w + waves, .. of x_j (x * suh, the
 // transform), the largest magnitude over the row gives the token's scale, and the scaled values go out as f16 high and
@@ -1380,552 +1509,6 @@ extern "C" __global__ void __launch_bounds__(64) cols_plan(u64* wtab, u32* gtab,
         r[9 + j] = 4 * g + (j < 4 ? j : 0);
     }
 }
-
-// --------------------------------------------------------------------------------- the verify layer on the matrix cores
-// The same layer as verify_gate_up / verify_down above, for callers that accept f32 outputs within a tolerance instead of
-// the exact per-weight arithmetic (the reference's mma_grouped_exl3_K beside its exact kernels, kernels/exl3.cu:682-725,
-// held to 3e-3 of the largest output by crates/shadowzero-cuda/tests/exl3.rs:201).  Two things change.
-// (1) The work items are the DISTINCT experts of the batch, not the (token, rank) pairs: a small first launch selects every
-// token's experts and lists each expert once with the tokens that chose it, the shared expert as the first item with all of
-// them, so an expert's weights are decoded once however many tokens use it.
-// (2) The dot products run on the matrix cores, as in the head above: a lane decodes 4 consecutive weights of the bit stream,
-// a 16 x 16 tile is one B operand of v_mfma_f32_16x16x16_f16, the item's tokens ride on the A rows as f16 high and low
-// parts (8 tokens cost what one costs).  With LIN the codebook's last step is left to the end of the sum: a weight is
-// f16(h k_inv + k_bias) with h = 1024 + the byte sum, an integer that IS an f16 as the byte-sum instruction leaves it, so
-// the B operand is h itself and sum x w = k_inv sum x h + k_bias sum x, off from the exact value only by the rounding of
-// each weight to f16 that is skipped (half a unit in the last place of a weight, about 1.5e-4 of an output, relative); the
-// sum of a rotated block is sqrt(128) times the block's first element before the rotation.  Without LIN the weights are the
-// codebook's bits and only the order of the f32 additions and the 22 bits kept of an input differ from the exact kernels.
-// The plan: pbuf holds u32 tidx[m k] | f32 w[m k] | u32 cnt[m] as for the exact kernels, then at byte ioff (16-byte
-// aligned) u32 n_items, 3 unused words, and 8 words an item: expert (0xffffffff: the shared one), n tokens, their rows as
-// 8 bytes, their pair numbers as 8 u16 (pair j k + t of token j and rank t, m k + j for the shared expert: the row of the
-// partial sums and of launch 2's output, which verify_combine_exl3 reads as it does after the exact launches).
-
-// grid 1 (+ the workgroups of a riding sum), block 64 m.  Wave j selects token j's experts (lane t < k then holds rank t's); the items come out of three tables
-// in LDS indexed by expert: the lowest pair that chose it (that pair's thread writes the item), the tokens that chose it as
-// a bit mask, and each such token's rank.  The routing weights are not needed before launch 3 and are left to a spare
-// workgroup of launch 1 (verify_route_weights below).
-// Workgroups 1 .. (hidden / 128) m (cmode != 0): the rank-order sum of the layer before, as in verify_gate_up_kernel.
-extern "C" __global__ void __launch_bounds__(512) verify_plan_exl3(const float* logits, u8* pbuf, u32 ioff, u32 ne, u32 k, u32 m, u32 shared, u32 hidden,
-                                                                   const float* cdn, const u8* cpbuf, const float* cgl, float* cy, u32 cmode) {
-    if (blockIdx.x > 0) {
-        const u32 ci = blockIdx.x - 1, nb = hidden / 128;
-        if (cmode && ci < nb * m)
-            for (u32 t = threadIdx.x; t < 128; t += blockDim.x) exl3_combine_finished(cdn, cpbuf, cgl, cy, k, m, hidden, cmode == 2, ci % nb, ci / nb, t);
-        return;
-    }
-    __shared__ double ex[8 * 512];   // the exact selection's scratch, a wave's 512 doubles
-    __shared__ u32 top[8][16];
-    __shared__ u32 lowest[512];      // expert -> the lowest pair number that chose it
-    __shared__ u32 tokens[512];      // expert -> bit j: token j chose it
-    __shared__ u8 rank[512 * 8];     // expert, token -> the token's rank of it
-    __shared__ u32 wave_items[8];
-    const u32 lane = threadIdx.x & 63, j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = m * k;
-    u32* tidx = (u32*) pbuf;
-    u32* plan = (u32*) (pbuf + ioff);
-    for (u32 i = threadIdx.x; i < 512; i += blockDim.x) {
-        lowest[i] = 0xffffffffu;
-        tokens[i] = 0;
-    }
-    route_ids(logits + (u64) j * ne, ne, k, lane, ex + j * 512, top[j]);
-    __syncthreads();
-    const u32 e = lane < k ? top[j][lane] : 0xffffffffu;
-    const u32 p = j * k + lane;
-    if (lane < k) tidx[p] = e;
-    if (e != 0xffffffffu) {
-        atomicMin(&lowest[e], p);
-        atomicOr(&tokens[e], 1u << j);
-        rank[e * 8 + j] = (u8) lane;
-    }
-    __syncthreads();
-    const bool isf = e != 0xffffffffu && lowest[e] == p;
-    const u64 firsts = __builtin_amdgcn_ballot_w64(isf);
-    if (lane == 0) wave_items[j] = __builtin_popcountll(firsts);
-    __syncthreads();
-    u32 slot = shared ? 1u : 0u;
-    for (u32 w = 0; w < j; w++) slot += wave_items[w];
-    if (isf) {
-        slot += __builtin_popcountll(firsts & ((1ull << lane) - 1));
-        u32 n = 0;
-        u64 toks = 0, pr0 = 0, pr1 = 0;
-        for (u32 mask = tokens[e]; mask; mask &= mask - 1) {
-            const u32 jj = __builtin_ctz(mask);
-            toks |= (u64) jj << (8 * n);
-            const u64 pv = jj * k + rank[e * 8 + jj];
-            if (n < 4) pr0 |= pv << (16 * n);
-            else pr1 |= pv << (16 * (n - 4));
-            n++;
-        }
-        u32x4* rec = (u32x4*) (plan + 4 + 8 * slot);
-        rec[0] = u32x4{e, n, (u32) toks, (u32) (toks >> 32)};
-        rec[1] = u32x4{(u32) pr0, (u32) (pr0 >> 32), (u32) pr1, (u32) (pr1 >> 32)};
-    }
-    if (threadIdx.x == 0) {
-        u32 count = shared ? 1u : 0u;
-        for (u32 w = 0; w < m; w++) count += wave_items[w];
-        plan[0] = count;
-        if (shared) {
-            u64 toks = 0, pr0 = 0, pr1 = 0;
-            for (u32 jj = 0; jj < m; jj++) {
-                toks |= (u64) jj << (8 * jj);
-                const u64 pv = G + jj;
-                if (jj < 4) pr0 |= pv << (16 * jj);
-                else pr1 |= pv << (16 * (jj - 4));
-            }
-            u32x4* rec = (u32x4*) (plan + 4);
-            rec[0] = u32x4{0xffffffffu, m, (u32) toks, (u32) (toks >> 32)};
-            rec[1] = u32x4{(u32) pr0, (u32) (pr0 >> 32), (u32) pr1, (u32) (pr1 >> 32)};
-        }
-    }
-}
-
-// The renormalised routing weights and the counts of the chosen experts tidx (pbuf, as the plan left it) into w and cnt:
-// a wave a token, for a workgroup that has nothing else to do.
-__device__ __forceinline__ void verify_route_weights(const float* __restrict__ logits, u8* __restrict__ pbuf, u32 ne, u32 k, u32 m, u32 wave, u32 lane) {
-    const u32 G = m * k;
-    for (u32 j = wave; j < m; j += 4) {
-        u32 kk;
-        const float wt = route_weights(logits + (u64) j * ne, ne, k, lane, (const u32*) pbuf + j * k, &kk);
-        if (lane < k) ((float*) (pbuf + G * 4))[j * k + lane] = wt;
-        if (lane == 0) ((u32*) (pbuf + 2 * G * 4))[j] = kk;
-    }
-}
-
-// Two states to the f16 pair (1024 + byte sum) that the codebook's multiply-add would start from.
-__device__ __forceinline__ f16x2 exl3_h_pair(u32 sa, u32 sb) {
-    const u32 lo = __builtin_amdgcn_sad_u8(exl3_mul(sa), 0u, 0x64006400u);
-    return __builtin_bit_cast(f16x2, __builtin_amdgcn_sad_hi_u8(exl3_mul(sb), 0u, lo));
-}
-
-#define EXL3_KINV 0.0067672729f    /* f16 0x1eee */
-#define EXL3_KBIAS (-10.3828125f)  /* f16 0xc931 */
-
-// A wave's A rows in LDS: f16 astrip[(tile row * 2 NMAX + A row) * 16 + slot], A row 2 r the high and 2 r + 1 the low part
-// of token r.  The lane holds elements `lane` (a0) and `lane + 64` (a1) of the token's rotated 128-block; they are scaled
-// by the power of two that takes the block's largest magnitude to [2^14, 2^15) (returned inverse undoes it).
-template <int NMAX>
-__device__ __forceinline__ float exl3_put_a_rows(u16* astrip, u32 r, float a0, float a1, u32 lane) {
-    const float mx = wave_max_f32(fmaxf(__builtin_fabsf(a0), __builtin_fabsf(a1)));
-    float scale, iv;
-    pow2_scale_of(f32_bits(mx), scale, iv);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const u32 i = lane + 64 * h;
-        const float v = (h ? a1 : a0) * scale;
-        const _Float16 hi = (_Float16) v;
-        const _Float16 lo = (_Float16) (v - (float) hi);
-        u16* at = astrip + ((i >> 4) * (2 * NMAX) + 2 * r) * 16 + exl3_aslot(i & 15);
-        at[0] = __builtin_bit_cast(u16, hi);
-        at[16] = __builtin_bit_cast(u16, lo);
-    }
-    return iv;
-}
-
-// The decode loop of one wave on the matrix cores: the 8 tile rows of one 128-input block (requested into the ring by
-// exl3_rows_issue) against the A rows in astrip; acc[c] = the 16 x 16 sums of column tile c (row 4 a + q of the lane group
-// a = lane / 16: token 2 a high, low, token 2 a + 1 high, low; column lane % 16).
-template <int K, bool LIN, int NMAX>
-__device__ __forceinline__ void exl3_wave_mma(const u32* __restrict__ row0, u64 pitch, const u32* wb, u32 lds, const u16* astrip, u32 n, u32 lane,
-                                              f32x4 (&acc)[8]) {
-    constexpr int D = 4;
-    typedef Exl3Rows<K, D> R;
-    constexpr int stride = R::stride, ur = R::unit_rows;
-    constexpr bool one_shift = 16 + 3 * K <= 32;
-    const u32 n16 = lane & 15, a = lane >> 4;
-    const u32 t0 = 32 * (n16 & 7) + 8 * a + 4 * (n16 >> 3);
-    auto window = [&](u32 e, u32& om, u32& op, u32& sh) {
-        const u32 jp = (e - 1) >> 5, jm = (jp + 8 * K - 1) % (8 * K);
-        sh = 31 - ((e - 1) & 31);
-        om = (jm / K) * stride + jm % K;
-        op = (jp / K) * stride + jp % K;
-    };
-    u32 om1, op1, sh1, om0 = 0, op0 = 0, sh0 = 0;
-    window((t0 + 4) * K, om1, op1, sh1);
-    if constexpr (!one_shift) window((t0 + 2) * K, om0, op0, sh0);
-#pragma unroll
-    for (int c = 0; c < 8; c++) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bool fed = n16 < 2 * n;                          // this lane supplies A row n16
-    const u16* xa0 = astrip + (fed ? n16 : 0) * 16 + 4 * a;
-#pragma unroll 1
-    for (u32 i = 0; i < 8; i++) {
-        exl3_rows_wait<K, D>(i + D > 8 ? i + D - 8 : 0);
-        const u32* row = wb + (i & (D - 1)) * R::row_words;
-        u32 w1[8][2], w0[8][2];
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            w1[c][0] = row[c * 8 * stride + om1];
-            w1[c][1] = row[c * 8 * stride + op1];
-            if constexpr (!one_shift) {
-                w0[c][0] = row[c * 8 * stride + om0];
-                w0[c][1] = row[c * 8 * stride + op0];
-            }
-        }
-        typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-        u32x2 xv = *(const u32x2*) (xa0 + i * (2 * NMAX * 16));
-        if (!fed) xv = u32x2{0u, 0u};
-        if ((i + 1) % ur == 0 && i + D + 1 - ur < 8) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the row's words are in registers, its slot can take the row D further on
-            exl3_unit_issue<K, D>(row0, pitch, i + D + 1 - ur, lane, lds);
-        }
-        const f16x4 av = __builtin_bit_cast(f16x4, xv);
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const u32 hi = __builtin_amdgcn_alignbit(w1[c][0], w1[c][1], sh1);
-            u32 s0, s1;
-            if constexpr (one_shift) {
-                s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16);
-                s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
-            } else {
-                const u32 lo = __builtin_amdgcn_alignbit(w0[c][0], w0[c][1], sh0);
-                s0 = __builtin_amdgcn_ubfe(lo, K, 16);
-                s1 = lo & 0xffffu;
-            }
-            const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
-            const f16x2 b01 = LIN ? exl3_h_pair(s0, s1) : exl3_cb2_pair(s0, s1), b23 = LIN ? exl3_h_pair(s2, s3) : exl3_cb2_pair(s2, s3);
-            const f16x4 bv = {b01[0], b01[1], b23[0], b23[1]};
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, acc[c], 0, 0, 0);
-        }
-    }
-}
-
-// What a wave leaves for the workgroup's sum: red[(wave * NMAX + r) * 128 + column] = token r's partial sum of the wave's
-// 128 inputs (high + low part, scale undone; with LIN times k_inv plus the token's k_bias term).  iv[h], cr[h]: the inverse
-// scale and the k_bias term of the lane group's tokens 2 a + h.
-template <bool LIN, int NMAX>
-__device__ __forceinline__ void exl3_mma_to_red(float* red, u32 wave, u32 n, u32 lane, const f32x4 (&acc)[8], const float (&iv)[2], const float (&cr)[2]) {
-    const u32 n16 = lane & 15, a = lane >> 4;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const u32 r = 2 * a + h;
-        if (r < n && r < (u32) NMAX) {
-            const float f = iv[h] * (LIN ? EXL3_KINV : 1.0f), c0 = LIN ? cr[h] : 0.0f;
-            float* o = red + (wave * NMAX + r) * 128 + n16;
-#pragma unroll
-            for (int c = 0; c < 8; c++) o[16 * c] = __builtin_fmaf(acc[c][2 * h] + acc[c][2 * h + 1], f, c0);
-        }
-    }
-}
-
-// The LDS a workgroup of the two launches needs, in words, for ring rows of `ring` words a wave (Exl3Rows<K, 4>::words).
-#define EXL3_MMA_WAVE_WORDS(ring, NMAX) ((ring) + (NMAX) * 128 + 64 + 16)   /* ring, A rows, input scales, the tokens' inverse scales and k_bias terms */
-#define EXL3_MMA_LDS_WORDS(ring, NMAX) (4 * EXL3_MMA_WAVE_WORDS(ring, NMAX) + 64)
-
-// Launch 1: the gate and up products of every item, partial sums gup[((sel * S + pair) * zs + z)][ff] as the exact launch
-// leaves them (already through the output-side transform and scales).  grid = (ff / 128, 2 IT, zs), IT = the item slots
-// (an even number above m k + 1), zs = ceil(hidden / 512); block 256; dynamic LDS EXL3_MMA_LDS_WORDS.
-template <int K, bool LIN, int NMAX>
-__device__ __forceinline__ void verify_gate_up_mma_kernel(const float* __restrict__ logits, u64 ebase, u64 estride, u64 shbase, u32 part,
-                                                          const float* __restrict__ u, u8* __restrict__ pbuf, u32 ioff, float* __restrict__ gup, u32 ne,
-                                                          u32 k, u32 m, u32 hidden, u32 ff) {
-    constexpr int D = 4;
-    typedef Exl3Rows<K, D> R;
-    constexpr int WW = EXL3_MMA_WAVE_WORDS(R::words, NMAX);
-    extern __shared__ __attribute__((aligned(16))) u32 dyn[];
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 IT = gridDim.y >> 1, sel = blockIdx.y >= IT ? 1u : 0u, it = blockIdx.y - sel * IT;
-    const u32* plan = (const u32*) (pbuf + ioff);
-    if (it >= plan[0]) {
-        // the last item slot is never an item (there are at most m k + 1): one of its workgroups works the routing weights out
-        // for launch 3 while the others multiply
-        if (blockIdx.y == gridDim.y - 1 && blockIdx.x == 0 && blockIdx.z == 0) verify_route_weights(logits, pbuf, ne, k, m, wave, lane);
-        return;
-    }
-    const u32* rec = plan + 4 + 8 * it;
-    const u32 e = rec[0], n = min(rec[1], (u32) NMAX);
-    const u64 toks = (u64) rec[2] | ((u64) rec[3] << 32);
-    const u32 S = m * k + m;
-    const u8* bp = (const u8*) (e == 0xffffffffu ? shbase : ebase + e * estride) + (u64) sel * part;
-    const u32 kbs = hidden / 128, kb = blockIdx.z * 4 + wave;
-    const bool live = kb < kbs;
-    u32* wring = dyn + wave * WW;
-    u16* astrip = (u16*) (wring + R::words);
-    u32* sc = wring + R::words + NMAX * 128;
-    u32* sv_out = dyn + 4 * WW;
-    float iv[2] = {0.0f, 0.0f}, cr[2] = {0.0f, 0.0f};   // the inverse scales and the k_bias terms of the lane group's two tokens
-    f32x4 acc[8];
-    if (live) {
-        float v[NMAX][2];
-#pragma unroll
-        for (int r = 0; r < NMAX; r++) {
-            const u32 tok = (u32) (toks >> (8 * min((u32) r, n - 1))) & 0xffu;
-            const float* xj = u + (u64) tok * hidden + kb * 128;
-            v[r][0] = xj[lane];
-            v[r][1] = xj[lane + 64];
-        }
-#pragma unroll
-        for (int r = 0; r < NMAX; r++) asm volatile("" : "+v"(v[r][0]), "+v"(v[r][1]));   // no ordinary load is in flight from now on
-        const u32 sc_lds = __builtin_amdgcn_readfirstlane(lds_offset(sc));
-        const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wring));
-        lds_load<4>(bp + kb * 256 + lane * 4, sc_lds);
-        if (wave == 0) lds_load<4>(bp + 2 * (u64) hidden + blockIdx.x * 256 + lane * 4, __builtin_amdgcn_readfirstlane(lds_offset(sv_out)));
-        const u32* row0 = (const u32*) (bp + 2 * (u64) hidden + 2 * (u64) ff + 4) + ((u64) kb * 8 * (ff / 16) + blockIdx.x * 8) * EXL3_TILE_WORDS(K, false);
-        const u64 pitch = (u64) (ff / 16) * EXL3_TILE_WORDS(K, false);
-        exl3_rows_issue<K, D>(row0, pitch, lane, wb_lds);
-        wait_vm<R::loads>();
-        const u16* sch = (const u16*) sc;
-        const float s0 = f16_to_f32(sch[lane]), s1 = f16_to_f32(sch[lane + 64]);
-        // a token's inverse scale and k_bias term wait in LDS for the lanes that hold the token's sums at the end
-        float* ivs = (float*) (sc + 64);
-#pragma unroll
-        for (int r = 0; r < NMAX; r++) {
-            if ((u32) r < n) {
-                float a0 = v[r][0] * s0, a1 = v[r][1] * s1;
-                const float c0 = (EXL3_KBIAS * 11.3137085f) * bits_f32(__builtin_amdgcn_readlane(f32_bits(a0), 0));
-                wht128_wave(a0, a1, lane);
-                const float i0 = exl3_put_a_rows<NMAX>(astrip, r, a0, a1, lane);
-                if (lane == 0) {
-                    ivs[r] = i0;
-                    ivs[NMAX + r] = c0;
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        exl3_wave_mma<K, LIN, NMAX>(row0, pitch, wring, wb_lds, astrip, n, lane, acc);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const u32 r = min(2 * (lane >> 4) + h, (u32) NMAX - 1);
-            iv[h] = ivs[r];
-            cr[h] = ivs[NMAX + r];
-        }
-    }
-    __syncthreads();   // every wave is done with its ring and A rows: the space takes the sums
-    float* red = (float*) dyn;
-    if (live) exl3_mma_to_red<LIN, NMAX>(red, wave, n, lane, acc, iv, cr);
-    __syncthreads();
-    const u32 nw = min(4u, kbs - blockIdx.z * 4);
-    const u16* sv = (const u16*) sv_out;
-    for (u32 r = wave; r < n; r += 4) {
-        float a0 = 0.0f, a1 = 0.0f;
-        for (u32 w = 0; w < nw; w++) {
-            a0 += red[(w * NMAX + r) * 128 + lane];
-            a1 += red[(w * NMAX + r) * 128 + lane + 64];
-        }
-        wht128_wave(a0, a1, lane);
-        const u32 pair = (rec[4 + (r >> 1)] >> (16 * (r & 1))) & 0xffffu;
-        float* o = gup + (((u64) sel * S + pair) * gridDim.z + blockIdx.z) * ff + blockIdx.x * 128;
-        __builtin_nontemporal_store(a0 * f16_to_f32(sv[lane]), &o[lane]);
-        __builtin_nontemporal_store(a1 * f16_to_f32(sv[lane + 64]), &o[lane + 64]);
-    }
-}
-
-// Launch 2: act = silu(gate) * up of every token of the item from launch 1's partial sums (by every wave for its own
-// 128-block, as the exact launch does), then the down product: finished blocks dn[pair][hidden] when one workgroup holds
-// the whole sum over the inputs (ff <= 512), else partial sums dn[pair * gridDim.z + z][hidden] for verify_combine_exl3.
-// grid = (hidden / 128, IT, ceil(ff / 512)), block 256, dynamic LDS as launch 1.
-template <int K, bool LIN, int NMAX>
-__device__ __forceinline__ void verify_down_mma_kernel(u64 ebase, u64 estride, u64 shbase, u32 part, const u8* __restrict__ pbuf, u32 ioff,
-                                                       const float* __restrict__ gup, float* __restrict__ dn, u32 k, u32 m, u32 hidden, u32 ff, u32 zs) {
-    constexpr int D = 4;
-    typedef Exl3Rows<K, D> R;
-    constexpr int WW = EXL3_MMA_WAVE_WORDS(R::words, NMAX);
-    extern __shared__ __attribute__((aligned(16))) u32 dyn[];
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 it = blockIdx.y;
-    const u32* plan = (const u32*) (pbuf + ioff);
-    if (it >= plan[0]) return;
-    const u32* rec = plan + 4 + 8 * it;
-    const u32 e = rec[0], n = min(rec[1], (u32) NMAX);
-    const u32 S = m * k + m;
-    const u8* down = (const u8*) (e == 0xffffffffu ? shbase : ebase + e * estride) + 2 * (u64) part;
-    const u32 kbs = ff / 128, kb = blockIdx.z * 4 + wave;
-    const bool live = kb < kbs;
-    u32* wring = dyn + wave * WW;
-    u16* astrip = (u16*) (wring + R::words);
-    u32* sc = wring + R::words + NMAX * 128;
-    u32* sv_out = dyn + 4 * WW;
-    float iv[2] = {0.0f, 0.0f}, cr[2] = {0.0f, 0.0f};   // the inverse scales and the k_bias terms of the lane group's two tokens
-    f32x4 acc[8];
-    if (live) {
-        // the sums of launch 1's partials of the wave's block of gate and up, every token's loads on their way at once (in
-        // two lots of four tokens when there may be more)
-        float gu[NMAX][4];
-#pragma unroll
-        for (int r0 = 0; r0 < NMAX; r0 += 4) {
-            if (r0 > 0 && n <= (u32) r0) break;
-            float pv[4][4][4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const u32 r = min((u32) (r0 + q), n - 1);
-                const u32 pair = (rec[4 + (r >> 1)] >> (16 * (r & 1))) & 0xffffu;
-#pragma unroll
-                for (int z = 0; z < 4; z++) {
-                    const u32 zz = min((u32) z, zs - 1);
-                    const float* pg = gup + ((u64) pair * zs + zz) * ff + kb * 128;
-                    const float* pu = gup + ((u64) (S + pair) * zs + zz) * ff + kb * 128;
-                    pv[q][z][0] = pg[lane];
-                    pv[q][z][1] = pg[lane + 64];
-                    pv[q][z][2] = pu[lane];
-                    pv[q][z][3] = pu[lane + 64];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    float t = pv[q][0][c];
-#pragma unroll
-                    for (int z = 1; z < 4; z++)
-                        if ((u32) z < zs) t += pv[q][z][c];
-                    gu[r0 + q][c] = t;
-                }
-                if (zs > 4) {
-                    const u32 r = min((u32) (r0 + q), n - 1);
-                    const u32 pair = (rec[4 + (r >> 1)] >> (16 * (r & 1))) & 0xffffu;
-                    for (u32 z = 4; z < zs; z++) {
-                        const float* pg = gup + ((u64) pair * zs + z) * ff + kb * 128;
-                        const float* pu = gup + ((u64) (S + pair) * zs + z) * ff + kb * 128;
-                        gu[r0 + q][0] += pg[lane];
-                        gu[r0 + q][1] += pg[lane + 64];
-                        gu[r0 + q][2] += pu[lane];
-                        gu[r0 + q][3] += pu[lane + 64];
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < NMAX; r++) asm volatile("" : "+v"(gu[r][0]), "+v"(gu[r][1]), "+v"(gu[r][2]), "+v"(gu[r][3]));   // no ordinary load is in flight from now on
-        const u32 sc_lds = __builtin_amdgcn_readfirstlane(lds_offset(sc));
-        const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wring));
-        lds_load<4>(down + kb * 256 + lane * 4, sc_lds);
-        if (wave == 0) lds_load<4>(down + 2 * (u64) ff + blockIdx.x * 256 + lane * 4, __builtin_amdgcn_readfirstlane(lds_offset(sv_out)));
-        const u32* row0 = (const u32*) (down + 2 * (u64) ff + 2 * (u64) hidden + 4) + ((u64) kb * 8 * (hidden / 16) + blockIdx.x * 8) * EXL3_TILE_WORDS(K, false);
-        const u64 pitch = (u64) (hidden / 16) * EXL3_TILE_WORDS(K, false);
-        exl3_rows_issue<K, D>(row0, pitch, lane, wb_lds);
-        wait_vm<R::loads>();
-        const u16* sch = (const u16*) sc;
-        const float s0 = f16_to_f32(sch[lane]), s1 = f16_to_f32(sch[lane + 64]);
-        // a token's inverse scale and k_bias term wait in LDS for the lanes that hold the token's sums at the end
-        float* ivs = (float*) (sc + 64);
-#pragma unroll
-        for (int r = 0; r < NMAX; r++) {
-            if ((u32) r < n) {
-                float a0 = (siluf_ref(gu[r][0]) * gu[r][2]) * s0, a1 = (siluf_ref(gu[r][1]) * gu[r][3]) * s1;
-                const float c0 = (EXL3_KBIAS * 11.3137085f) * bits_f32(__builtin_amdgcn_readlane(f32_bits(a0), 0));
-                wht128_wave(a0, a1, lane);
-                const float i0 = exl3_put_a_rows<NMAX>(astrip, r, a0, a1, lane);
-                if (lane == 0) {
-                    ivs[r] = i0;
-                    ivs[NMAX + r] = c0;
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        exl3_wave_mma<K, LIN, NMAX>(row0, pitch, wring, wb_lds, astrip, n, lane, acc);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const u32 r = min(2 * (lane >> 4) + h, (u32) NMAX - 1);
-            iv[h] = ivs[r];
-            cr[h] = ivs[NMAX + r];
-        }
-    }
-    __syncthreads();
-    float* red = (float*) dyn;
-    if (live) exl3_mma_to_red<LIN, NMAX>(red, wave, n, lane, acc, iv, cr);
-    __syncthreads();
-    const u32 nw = min(4u, kbs - blockIdx.z * 4);
-    const u16* sv = (const u16*) sv_out;
-    for (u32 r = wave; r < n; r += 4) {
-        float a0 = 0.0f, a1 = 0.0f;
-        for (u32 w = 0; w < nw; w++) {
-            a0 += red[(w * NMAX + r) * 128 + lane];
-            a1 += red[(w * NMAX + r) * 128 + lane + 64];
-        }
-        const u32 pair = (rec[4 + (r >> 1)] >> (16 * (r & 1))) & 0xffffu;
-        if (gridDim.z == 1) {
-            wht128_wave(a0, a1, lane);
-            float* o = dn + (u64) pair * hidden + blockIdx.x * 128;
-            __builtin_nontemporal_store(a0 * f16_to_f32(sv[lane]), &o[lane]);
-            __builtin_nontemporal_store(a1 * f16_to_f32(sv[lane + 64]), &o[lane + 64]);
-        } else {
-            float* o = dn + ((u64) pair * gridDim.z + blockIdx.z) * hidden + blockIdx.x * 128;
-            o[lane] = a0;
-            o[lane + 64] = a1;
-        }
-    }
-}
-
-// Entry points: _mma_ the codebook's own f16 values, _lin_ the linearised form; the w variants take up to 8 tokens an item
-// (batches of more than 4 rows), the others 4.  5 workgroups of 4 waves a CU: the register budget follows it.
-#define EXL3_MMA_ENTRIES(K)                                                                                                            \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_gate_up_mma_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, const float* u, \
-                                                                                          u8* pbuf, u32 ioff, float* gup, u32 ne, u32 k, u32 m, u32 hidden, \
-                                                                                          u32 ff) {                                      \
-        verify_gate_up_mma_kernel<K, false, 4>(logits, ebase, estride, shbase, part, u, pbuf, ioff, gup, ne, k, m, hidden, ff);                     \
-    }                                                                                                                                    \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_down_mma_exl3_##K(u64 ebase, u64 estride, u64 shbase, u32 part, const u8* pbuf, \
-                                                                                       u32 ioff, const float* gup, float* dn, u32 k, u32 m, u32 hidden, \
-                                                                                       u32 ff, u32 zs) {                                 \
-        verify_down_mma_kernel<K, false, 4>(ebase, estride, shbase, part, pbuf, ioff, gup, dn, k, m, hidden, ff, zs);                   \
-    }
-#define EXL3_MMAW_ENTRIES(K)                                                                                                            \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_gate_up_mmaw_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, const float* u, \
-                                                                                          u8* pbuf, u32 ioff, float* gup, u32 ne, u32 k, u32 m, u32 hidden, \
-                                                                                          u32 ff) {                                      \
-        verify_gate_up_mma_kernel<K, false, 8>(logits, ebase, estride, shbase, part, u, pbuf, ioff, gup, ne, k, m, hidden, ff);                     \
-    }                                                                                                                                    \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_down_mmaw_exl3_##K(u64 ebase, u64 estride, u64 shbase, u32 part, const u8* pbuf, \
-                                                                                       u32 ioff, const float* gup, float* dn, u32 k, u32 m, u32 hidden, \
-                                                                                       u32 ff, u32 zs) {                                 \
-        verify_down_mma_kernel<K, false, 8>(ebase, estride, shbase, part, pbuf, ioff, gup, dn, k, m, hidden, ff, zs);                   \
-    }
-#define EXL3_LIN_ENTRIES(K)                                                                                                            \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_gate_up_lin_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, const float* u, \
-                                                                                          u8* pbuf, u32 ioff, float* gup, u32 ne, u32 k, u32 m, u32 hidden, \
-                                                                                          u32 ff) {                                      \
-        verify_gate_up_mma_kernel<K, true, 4>(logits, ebase, estride, shbase, part, u, pbuf, ioff, gup, ne, k, m, hidden, ff);                     \
-    }                                                                                                                                    \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_down_lin_exl3_##K(u64 ebase, u64 estride, u64 shbase, u32 part, const u8* pbuf, \
-                                                                                       u32 ioff, const float* gup, float* dn, u32 k, u32 m, u32 hidden, \
-                                                                                       u32 ff, u32 zs) {                                 \
-        verify_down_mma_kernel<K, true, 4>(ebase, estride, shbase, part, pbuf, ioff, gup, dn, k, m, hidden, ff, zs);                   \
-    }
-#define EXL3_LINW_ENTRIES(K)                                                                                                            \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_gate_up_linw_exl3_##K(const float* logits, u64 ebase, u64 estride, u64 shbase, u32 part, const float* u, \
-                                                                                          u8* pbuf, u32 ioff, float* gup, u32 ne, u32 k, u32 m, u32 hidden, \
-                                                                                          u32 ff) {                                      \
-        verify_gate_up_mma_kernel<K, true, 8>(logits, ebase, estride, shbase, part, u, pbuf, ioff, gup, ne, k, m, hidden, ff);                     \
-    }                                                                                                                                    \
-    extern "C" __global__ void __launch_bounds__(256, 5) verify_down_linw_exl3_##K(u64 ebase, u64 estride, u64 shbase, u32 part, const u8* pbuf, \
-                                                                                       u32 ioff, const float* gup, float* dn, u32 k, u32 m, u32 hidden, \
-                                                                                       u32 ff, u32 zs) {                                 \
-        verify_down_mma_kernel<K, true, 8>(ebase, estride, shbase, part, pbuf, ioff, gup, dn, k, m, hidden, ff, zs);                   \
-    }
-EXL3_MMA_ENTRIES(1)
-EXL3_MMA_ENTRIES(2)
-EXL3_MMA_ENTRIES(3)
-EXL3_MMA_ENTRIES(4)
-EXL3_MMA_ENTRIES(5)
-EXL3_MMA_ENTRIES(6)
-EXL3_MMA_ENTRIES(7)
-EXL3_MMA_ENTRIES(8)
-EXL3_MMAW_ENTRIES(1)
-EXL3_MMAW_ENTRIES(2)
-EXL3_MMAW_ENTRIES(3)
-EXL3_MMAW_ENTRIES(4)
-EXL3_MMAW_ENTRIES(5)
-EXL3_MMAW_ENTRIES(6)
-EXL3_MMAW_ENTRIES(7)
-EXL3_MMAW_ENTRIES(8)
-EXL3_LIN_ENTRIES(1)
-EXL3_LIN_ENTRIES(2)
-EXL3_LIN_ENTRIES(3)
-EXL3_LIN_ENTRIES(4)
-EXL3_LIN_ENTRIES(5)
-EXL3_LIN_ENTRIES(6)
-EXL3_LIN_ENTRIES(7)
-EXL3_LIN_ENTRIES(8)
-EXL3_LINW_ENTRIES(1)
-EXL3_LINW_ENTRIES(2)
-EXL3_LINW_ENTRIES(3)
-EXL3_LINW_ENTRIES(4)
-EXL3_LINW_ENTRIES(5)
-EXL3_LINW_ENTRIES(6)
-EXL3_LINW_ENTRIES(7)
-EXL3_LINW_ENTRIES(8)
 
 // ------------------------------------------------------------------------ the prefill chunk of an EXL3 layer (matrix cores)
 // A chunk's tokens grouped by expert (prefill_group in kernels/prefill.hip: runs of up to XPF_TOK(K) (token, rank) pairs of

@@ -871,26 +871,42 @@ extern "C" __global__ void __launch_bounds__(256) verify_down_iq3_s(const float*
 }
 
 // ------------------------------------------------------------------------------- unquantized matrices (F32, F16, BF16)
-// The router, the shared expert's gate and the other small projections are stored unquantized (quant.rs:237-239).  One wave
-// a row: a lane takes 4 consecutive columns a step (one 16- or 8-byte load), 256 columns a step for the wave, the row's
-// products are added in f32 lane by lane and then over the wave; every input of the batch (m <= 8) reuses the loaded
-// weights.  cols is a multiple of 4, rows of x are 16-byte aligned, rows of w are aligned to 4 weights, rows >= 1.
+// The router, the shared expert's gate, the hyper-connection's and other small projections are stored unquantized
+// (quant.rs:237-239).  These products are small: what bounds them is the number of memory round trips one after the other,
+// so everything a wave needs is requested at once and straight into registers: its share of the inputs (16 columns a lane of
+// every row of the batch, kept over all of its rows) and its rows' weights, the next rows' while these are multiplied.
+// A row of up to 1024 columns is G lanes' work (64 / G rows a wave at once), a longer one that of several waves of the
+// workgroup, whose sums meet in LDS.  Which lane adds which columns, and in which order, depends on the number of columns
+// and the type alone: every input of a batch has the bits of a launch of its own.
+// cols is a multiple of 4, rows of x are 16-byte aligned, rows of w are aligned to 4 weights, rows >= 1.
+typedef u32 u32x4h __attribute__((ext_vector_type(4), aligned(8)));   // 8 two-byte weights, aligned as 4 are
+typedef u32 u32x2h __attribute__((ext_vector_type(2), aligned(8)));
+
 struct DenseF32 {
-    static constexpr u32 BYTES = 4;
-    static __device__ __forceinline__ f32x4 load4(const u8* p) { return *(const f32x4*) p; }
+    static constexpr u32 BYTES = 4, C = 4;   // columns a load
+    typedef f32x4 Raw;
+    static __device__ __forceinline__ Raw load(const u8* p) { return *(const f32x4*) p; }
+    static __device__ __forceinline__ Raw none() { return f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+    static __device__ __forceinline__ float get(const Raw& r, int i) { return r[i]; }
 };
-struct DenseF16 {
-    static constexpr u32 BYTES = 2;
-    static __device__ __forceinline__ f32x4 load4(const u8* p) {
-        const uint2 v = *(const uint2*) p;
-        return f32x4{f16_to_f32((u16) v.x), f16_to_f32((u16) (v.x >> 16)), f16_to_f32((u16) v.y), f16_to_f32((u16) (v.y >> 16))};
+template <bool BF, int C_>
+struct Dense16 {   // F16, or BF16: the upper half of an f32 (half.rs)
+    static constexpr u32 BYTES = 2, C = C_;
+    typedef u32 Raw __attribute__((ext_vector_type(C_ / 2)));
+    static __device__ __forceinline__ Raw load(const u8* p) {
+        if constexpr (C_ == 8) return *(const u32x4h*) p;
+        else return *(const u32x2h*) p;
     }
-};
-struct DenseBF16 {
-    static constexpr u32 BYTES = 2;
-    static __device__ __forceinline__ f32x4 load4(const u8* p) {   // half.rs: a bf16 is the upper half of the f32
-        const uint2 v = *(const uint2*) p;
-        return f32x4{bits_f32(v.x << 16), bits_f32(v.x & 0xffff0000u), bits_f32(v.y << 16), bits_f32(v.y & 0xffff0000u)};
+    static __device__ __forceinline__ Raw none() {
+        Raw r;
+#pragma unroll
+        for (int i = 0; i < C_ / 2; i++) r[i] = 0;
+        return r;
+    }
+    static __device__ __forceinline__ float get(const Raw& r, int i) {
+        const u32 w = r[i / 2];
+        if constexpr (BF) return bits_f32((i & 1) ? w & 0xffff0000u : w << 16);
+        else return f16_to_f32((u16) ((i & 1) ? w >> 16 : w));
     }
 };
 
@@ -903,177 +919,465 @@ __device__ __forceinline__ float dense_act(float t, u32 act, float div) {
     return t;
 }
 
-#define DENSE_CHUNK 2048u   // columns a wave takes at a time: 8 loads of 4 a lane
-// rows a wave takes in turn when the rows are short: up to 8, fewer while that would leave CUs without a workgroup
-__device__ __forceinline__ u32 dense_rpw(u32 rows) { return min(8u, max(1u, rows / 1024u)); }
+#define DENSE_LANE_COLS 16u   // columns a lane keeps of every input
 
-// The wave's weights of columns [c0, c0 + chunk) of the row at wr, 4 a lane a load, all 8 loads in flight together.
-template <class T>
-__device__ __forceinline__ void dense_load_w(const u8* __restrict__ wr, u32 c0, u32 chunk, bool live, u32 lane, f32x4 (&wv)[8]) {
+// Lanes a row of `cols` columns takes in a wave (a power of two), and waves.
+__device__ __forceinline__ u32 dense_lanes(u32 cols) {
+    u32 g = 64;
+    while (g > 1 && (g / 2) * DENSE_LANE_COLS >= cols) g /= 2;
+    return g;
+}
+__device__ __forceinline__ u32 dense_waves(u32 cols) { return min(8u, (cols + 64 * DENSE_LANE_COLS - 1) / (64 * DENSE_LANE_COLS)); }
+
+// Sums v[j] over the G lanes of a row.  Where G >= M the first log2 M steps halve the number of values a lane carries: lane
+// gl then returns output gl % M; else every lane gets every output (v).  The tree of additions is the same for every M.
+template <int M>
+__device__ __forceinline__ float dense_reduce(float (&v)[M], u32 G, u32 lane) {
+    if (G >= (u32) M) {
+        if constexpr (M >= 2) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const u32 c = 4 * lane + 256 * i;
-        wv[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (live && c < chunk) wv[i] = T::load4(wr + (u64) (c0 + c) * T::BYTES);
+            for (int p = 0; p < M / 2; p++) {
+                const bool up = lane & 1;
+                v[p] = (up ? v[2 * p + 1] : v[2 * p]) + lane_xor<1>(up ? v[2 * p] : v[2 * p + 1], lane);
+            }
+        }
+        if constexpr (M >= 4) {
+#pragma unroll
+            for (int p = 0; p < M / 4; p++) {
+                const bool up = lane & 2;
+                v[p] = (up ? v[2 * p + 1] : v[2 * p]) + lane_xor<2>(up ? v[2 * p] : v[2 * p + 1], lane);
+            }
+        }
+        if constexpr (M >= 8) {
+            const bool up = lane & 4;
+            v[0] = (up ? v[1] : v[0]) + lane_xor<4>(up ? v[0] : v[1], lane);
+        }
+        float t = v[0];
+        if (M < 2 && G > 1) t += lane_xor<1>(t, lane);
+        if (M < 4 && G > 2) t += lane_xor<2>(t, lane);
+        if (M < 8 && G > 4) t += lane_xor<4>(t, lane);
+        if (G > 8) t += lane_xor<8>(t, lane);
+        if (G > 16) t += lane_xor<16>(t, lane);
+        if (G > 32) t += lane_xor<32>(t, lane);
+        return t;
     }
+#pragma unroll
+    for (int j = 0; j < M; j++) v[j] = seg_sum_rt(v[j], G, lane);
+    return 0.0f;
 }
 
-__device__ __forceinline__ float dense_dot8(const f32x4 (&wv)[8], const f32x4 (&xv)[8], float acc) {
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        acc = __builtin_fmaf(wv[i].x, xv[i].x, acc);
-        acc = __builtin_fmaf(wv[i].y, xv[i].y, acc);
-        acc = __builtin_fmaf(wv[i].z, xv[i].z, acc);
-        acc = __builtin_fmaf(wv[i].w, xv[i].w, acc);
-    }
-    return acc;
-}
-
-// Long rows (cols > 2048): one row a workgroup, wave v takes the chunks v, v + 4, .. of it; the inputs' chunks come
-// straight from memory (they are shared by every workgroup and stay in cache), an input at a time; the four waves' sums
-// are added in wave order.  `row` < rows for every workgroup that calls it.
+// One lane's columns of a row or of the inputs: chunk i starts at column ((o * NCH + i) * kw_n + kw) * G * C + gl * C.
 template <class T>
-__device__ __forceinline__ void dense_wide(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 row,
-                                           u32 cols, u32 m, u32 act, float div) {
-    float (*red)[8] = (float (*)[8]) sz_dyn_lds;   // 4 x 8 floats of dynamic LDS
-    const u32 tid = threadIdx.x, lane = tid % 64, wv_ = tid / 64;
-    float acc[8];
+struct DenseSlice {
+    static constexpr int NCH = DENSE_LANE_COLS / T::C;
+    u32 kw, kwn, G, gl, cols;
+    __device__ __forceinline__ u32 col(u32 o, int i) const { return (((o * NCH + i) * kwn + kw) * G + gl) * T::C; }
+    __device__ __forceinline__ void weights(const u8* row, u32 o, bool live, typename T::Raw (&w)[NCH]) const {
 #pragma unroll
-    for (int j = 0; j < 8; j++) acc[j] = 0.0f;
-    const u8* wr = w + (u64) row * cols * T::BYTES;
-    for (u32 c0 = wv_ * DENSE_CHUNK; c0 < cols; c0 += 4 * DENSE_CHUNK) {
-        const u32 chunk = min(DENSE_CHUNK, cols - c0);
-        f32x4 wv[8];
-        dense_load_w<T>(wr, c0, chunk, true, lane, wv);
+        for (int i = 0; i < NCH; i++) {
+            const u32 c = col(o, i);
+            w[i] = T::none();
+            if (live && c < cols) w[i] = T::load(row + (u64) c * T::BYTES);
+        }
+    }
+    template <int M>
+    __device__ __forceinline__ void inputs(const float* x, u32 xs, u32 m, u32 o, float (&xv)[M][DENSE_LANE_COLS]) const {
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if ((u32) j < m) {
-                f32x4 xv[8];
+        for (int j = 0; j < M; j++) {
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const u32 c = 4 * lane + 256 * i;
-                    xv[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    if (c < chunk) xv[i] = *(const f32x4*) (x + (u64) j * xs + c0 + c);
+            for (int i = 0; i < NCH; i++) {
+                const u32 c = col(o, i);
+#pragma unroll
+                for (u32 q = 0; q < T::C; q += 4) {
+                    f32x4 t = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    if ((u32) j < m && c < cols) t = *(const f32x4*) (x + (u64) j * xs + c + q);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) xv[j][i * T::C + q + e] = t[e];
                 }
-                acc[j] = dense_dot8(wv, xv, acc[j]);
             }
         }
     }
+    template <int M>
+    __device__ __forceinline__ void dot(const typename T::Raw (&w)[NCH], const float (&xv)[M][DENSE_LANE_COLS], float (&acc)[M]) const {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        if ((u32) j < m) {
-            const float t = seg_sum<64>(acc[j], lane);
-            if (lane == 0) red[wv_][j] = t;
-        }
+        for (int i = 0; i < NCH; i++)
+#pragma unroll
+            for (int e = 0; e < (int) T::C; e++) {
+                const float wv = T::get(w[i], e);
+#pragma unroll
+                for (int j = 0; j < M; j++) acc[j] = __builtin_fmaf(wv, xv[j][i * T::C + e], acc[j]);
+            }
     }
-    __syncthreads();
-    if (tid < m) y[(u64) tid * ys + row] = dense_act(((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid], act, div);
+};
+
+// Rows [first, first + np * rows a pass) of W against the m inputs by the workgroup (256 threads, or 64 dense_waves(cols) where
+// that is more): emit(row, j, sum) once for every output.  red: 2 * 8 * 8 floats of LDS.
+template <class T, int M, class Emit>
+__device__ __forceinline__ void dense_rows(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, u32 rows, u32 cols, u32 m, u32 first, u32 np,
+                                           float* red, Emit emit) {
+    typedef DenseSlice<T> S;
+    const u32 tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32 kwn = dense_waves(cols), G = dense_lanes(cols), rw = (blockDim.x >> 6) / kwn, rg = wave / kwn, per = 64 / G;
+    const S sl{wave - rg * kwn, kwn, G, lane & (G - 1), cols};
+    const u32 outer = (cols + kwn * G * DENSE_LANE_COLS - 1) / (kwn * G * DENSE_LANE_COLS);
+    const bool live = rg < rw;
+    u32 row = first + rg * per + lane / G;
+    const u32 step = rw * per;
+    float xv[M][DENSE_LANE_COLS];
+    typename T::Raw wv[S::NCH], wn[S::NCH];
+    sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, 0, live && row < rows, wv);
+    sl.inputs(x, xs, m, 0, xv);
+    for (u32 p = 0; p < np; p++, row += step) {
+        const u32 next = row + step;
+        const bool more = p + 1 < np;
+        if (more) sl.weights(w + (u64) min(next, rows - 1) * cols * T::BYTES, 0, live && next < rows, wn);
+        float acc[M];
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[j] = 0.0f;
+        for (u32 o = 0; o < outer; o++) {
+            if (outer > 1 && o + p > 0) {   // (rows of more than 8192 columns: the inputs do not stay)
+                if (o) sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, o, live && row < rows, wv);
+                sl.inputs(x, xs, m, o, xv);
+            }
+            sl.dot(wv, xv, acc);
+        }
+        const float t = dense_reduce<M>(acc, G, lane);
+        if (kwn == 1) {
+            if (live && row < rows) {
+                if (G >= (u32) M) {
+                    if (sl.gl < m && sl.gl < (u32) M) emit(row, sl.gl, t);
+                } else if (sl.gl == 0) {
+#pragma unroll
+                    for (int j = 0; j < M; j++)
+                        if ((u32) j < m) emit(row, (u32) j, acc[j]);
+                }
+            }
+        } else {
+            // (a row is at least one whole wave here: G = 64)
+            float* r = red + (p & 1) * 64;
+            if (live && lane < (u32) M) r[wave * 8 + lane] = t;
+            __syncthreads();
+            const u32 q = tid / 8, j = tid & 7, orow = first + p * step + q;
+            if (q < rw && j < m && orow < rows) {
+                float s = r[q * kwn * 8 + j];
+                for (u32 v = 1; v < kwn; v++) s += r[(q * kwn + v) * 8 + j];
+                emit(orow, j, s);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < S::NCH; i++) wv[i] = wn[i];
+    }
 }
 
-// Short rows (cols <= 2048): the inputs are staged into LDS once a workgroup (xl: m * cols floats of dynamic LDS), then
-// wave v takes rows r0 + v, r0 + v + 4, .. (rpw of them), the next row's weights on their way while this one is
-// multiplied.  Lane 0 writes y[j * ys + row].
-template <class T>
-__device__ __forceinline__ void dense_narrow(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 r0,
-                                             u32 rpw, u32 rows, u32 cols, u32 m, u32 act, float div) {
-    float* xl = (float*) sz_dyn_lds;
-    const u32 tid = threadIdx.x, lane = tid % 64, wv_ = tid / 64;
-    const u32 q4 = cols / 4, total = m * q4;   // 16-byte pieces of the inputs: at most 16 a thread
-    f32x4 wv[8], wn[8];
-    u32 row = r0 + wv_;
-    dense_load_w<T>(w + (u64) min(row, rows - 1) * cols * T::BYTES, 0, cols, row < rows, lane, wv);
-    {
-        f32x4 t[16];
+// The same with the matrix's type picked at run time; two-byte rows that are no multiple of 8 columns are read 4 at a time.
+template <int M, class Emit>
+__device__ __forceinline__ void dense_rows_of(u32 type, const u8* w, const float* x, u32 xs, u32 rows, u32 cols, u32 m, u32 first, u32 np, float* red, Emit emit) {
+    if (type == 0) dense_rows<DenseF32, M>(w, x, xs, rows, cols, m, first, np, red, emit);
+    else if (type == 1) {
+        if (cols % 8 == 0) dense_rows<Dense16<false, 8>, M>(w, x, xs, rows, cols, m, first, np, red, emit);
+        else dense_rows<Dense16<false, 4>, M>(w, x, xs, rows, cols, m, first, np, red, emit);
+    } else {
+        if (cols % 8 == 0) dense_rows<Dense16<true, 8>, M>(w, x, xs, rows, cols, m, first, np, red, emit);
+        else dense_rows<Dense16<true, 4>, M>(w, x, xs, rows, cols, m, first, np, red, emit);
+    }
+}
+
+// y_j = W x_j for an unquantized row-major W[rows][cols], j < m (matvec_cols_*, kernels/matvec.cu:677): m1, m4 and m8 for
+// batches of 1, up to 4 and up to 8, whose inputs take 16, 64 and 128 registers.  type 0 F32, 1 F16, 2 BF16.
+// grid = ceil(rows / (np * rows a pass)), block max(256, 64 dense_waves(cols)); a pass is (waves / dense_waves) * 64 / G rows.
+template <int M>
+__device__ __forceinline__ void dense_cols(u32 type, const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 np) {
+    __shared__ float red[128];
+    const u32 pass = (blockDim.x >> 6) / dense_waves(cols) * (64 / dense_lanes(cols));
+    dense_rows_of<M>(type, w, x, xs, rows, cols, m, blockIdx.x * np * pass, np, red, [&](u32 row, u32 j, float t) { y[(u64) j * ys + row] = t; });
+}
+extern "C" __global__ void __launch_bounds__(512) matvec_cols_dense_m1(u32 type, const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 np) {
+    dense_cols<1>(type, w, x, xs, y, ys, rows, cols, m, np);
+}
+extern "C" __global__ void __launch_bounds__(512) matvec_cols_dense_m4(u32 type, const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 np) {
+    dense_cols<4>(type, w, x, xs, y, ys, rows, cols, m, np);
+}
+extern "C" __global__ void __launch_bounds__(512) matvec_cols_dense_m8(u32 type, const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 np) {
+    dense_cols<8>(type, w, x, xs, y, ys, rows, cols, m, np);
+}
+
+// The router and the shared expert's gate logit on the same inputs in one launch (moe_router_batch of the reference): the
+// router's ne rows into rl[j * ne + row], then, in workgroups of their own, the gate's one row into sgl[j] (gate_w 0: none).
+// grid = ceil(ne / pass) (+ 1), block as above, one pass a workgroup.
+template <int M>
+__device__ __forceinline__ void router_rows(u32 type, const u8* w, u32 gate_type, const u8* gate_w, const float* x, float* rl, float* sgl, u32 ne, u32 cols, u32 m) {
+    __shared__ float red[128];
+    const u32 pass = (blockDim.x >> 6) / dense_waves(cols) * (64 / dense_lanes(cols)), groups = (ne + pass - 1) / pass;
+    if (blockIdx.x < groups) dense_rows_of<M>(type, w, x, cols, ne, cols, m, blockIdx.x * pass, 1, red, [&](u32 row, u32 j, float t) { rl[(u64) j * ne + row] = t; });
+    else if (gate_w) dense_rows_of<M>(gate_type, gate_w, x, cols, 1, cols, m, 0, 1, red, [&](u32, u32 j, float t) { sgl[j] = t; });
+}
+extern "C" __global__ void __launch_bounds__(512) router_rows_m1(u32 type, const u8* w, u32 gate_type, const u8* gate_w, const float* x, float* rl, float* sgl, u32 ne, u32 cols,
+                                                                 u32 m) {
+    router_rows<1>(type, w, gate_type, gate_w, x, rl, sgl, ne, cols, m);
+}
+extern "C" __global__ void __launch_bounds__(512) router_rows_m4(u32 type, const u8* w, u32 gate_type, const u8* gate_w, const float* x, float* rl, float* sgl, u32 ne, u32 cols,
+                                                                 u32 m) {
+    router_rows<4>(type, w, gate_type, gate_w, x, rl, sgl, ne, cols, m);
+}
+extern "C" __global__ void __launch_bounds__(512) router_rows_m8(u32 type, const u8* w, u32 gate_type, const u8* gate_w, const float* x, float* rl, float* sgl, u32 ne, u32 cols,
+                                                                 u32 m) {
+    router_rows<8>(type, w, gate_type, gate_w, x, rl, sgl, ne, cols, m);
+}
+
+// The hyper-connection's read (forward.rs:797-812) in two launches.  The first: every stream of every row normalised (the mean
+// of squares in f64 as the CPU path has it), and the down and inject products of that: a stream's scale 1/sqrt(ms + eps) is a
+// factor of the sum over its columns and multiplies that.  A workgroup owns `pass` rows of the two matrices (down's first) and normalises the inputs for itself: it
+// has to read all of them anyway, and the arithmetic is less than another launch costs.  Workgroup 0 leaves the scales
+// 1/sqrt(ms + eps) for the second launch.
+// r: [m][streams * h]; down, g: silu(t / streams), 2 sigmoid(t / streams).  grid = ceil(rank / pass) + ceil(streams / pass) (inject),
+// block 64 max(4, dense_waves(ch)), dynamic LDS = m * streams * (1 + chunks of ch) doubles.
+__device__ __forceinline__ double lane_xor_f64(double v, u32 lane, int h) {
+    const u64 b = __builtin_bit_cast(u64, v);
+    float lo = bits_f32((u32) b), hi = bits_f32((u32) (b >> 32));
+    switch (h) {
+        case 1: lo = lane_xor<1>(lo, lane); hi = lane_xor<1>(hi, lane); break;
+        case 2: lo = lane_xor<2>(lo, lane); hi = lane_xor<2>(hi, lane); break;
+        case 4: lo = lane_xor<4>(lo, lane); hi = lane_xor<4>(hi, lane); break;
+        case 8: lo = lane_xor<8>(lo, lane); hi = lane_xor<8>(hi, lane); break;
+        case 16: lo = lane_xor<16>(lo, lane); hi = lane_xor<16>(hi, lane); break;
+        default: lo = lane_xor<32>(lo, lane); hi = lane_xor<32>(hi, lane); break;
+    }
+    return __builtin_bit_cast(double, (u64) f32_bits(lo) | ((u64) f32_bits(hi) << 32));
+}
+__device__ __forceinline__ double wave_sum_f64(double v, u32 lane) {
+    v += lane_xor_f64(v, lane, 1);
+    v += lane_xor_f64(v, lane, 2);
+    v += lane_xor_f64(v, lane, 4);
+    v += lane_xor_f64(v, lane, 8);
+    v += lane_xor_f64(v, lane, 16);
+    v += lane_xor_f64(v, lane, 32);
+    return v;
+}
+
+// A lane's sums of w * (norm_w * r), one for each of its chunks (which lies in one stream), before the streams' scales.
+template <class T, int M>
+__device__ __forceinline__ void hc_products(const DenseSlice<T>& sl, const typename T::Raw (&wv)[DenseSlice<T>::NCH], const float (&xv)[M][DENSE_LANE_COLS],
+                                            const float* __restrict__ nw, u32 o, float (&raw)[DenseSlice<T>::NCH][M]) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const u32 idx = tid + 256 * i;
-            if (idx < total) t[i] = *(const f32x4*) (x + (u64) (idx / q4) * xs + 4 * (idx % q4));
-        }
+    for (int i = 0; i < DenseSlice<T>::NCH; i++) {
+        const u32 c = sl.col(o, i);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const u32 idx = tid + 256 * i;
-            if (idx < total) *(f32x4*) (xl + (idx / q4) * cols + 4 * (idx % q4)) = t[i];
+        for (int j = 0; j < M; j++) raw[i][j] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < (int) T::C; q += 4) {
+            f32x4 n = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (c < sl.cols) n = *(const f32x4*) (nw + c + q);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float wv_ = T::get(wv[i], q + e);
+#pragma unroll
+                for (int j = 0; j < M; j++) raw[i][j] = __builtin_fmaf(wv_, xv[j][i * T::C + q + e] * n[e], raw[i][j]);
+            }
         }
     }
+}
+
+template <class T, int M>
+__device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows, u32 first, const float* __restrict__ r, const float* __restrict__ nw, double* __restrict__ scales,
+                                             u32 h, u32 cs, u32 m, float eps, float* red, u32 act, float* y, u32 ys) {
+    typedef DenseSlice<T> S;
+    const u32 tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32 cols = h * cs, kwn = dense_waves(cols), rw = (blockDim.x >> 6) / kwn, rg = wave / kwn;
+    const S sl{wave - rg * kwn, kwn, 64, lane, cols};
+    const u32 span = 64 * T::C, outer = (cols + kwn * span * S::NCH - 1) / (kwn * span * S::NCH);
+    const u32 pieces = outer * S::NCH * kwn;   // spans of 64 C columns, each one wave's
+    double* part = (double*) sz_dyn_lds;       // [m][cs][pieces of the widest stream]: the spans' sums of squares, in order
+    const u32 wide = h / span + 2;
+    float* scl = (float*) (part + (u64) m * cs * wide);
+    const bool live = rg < rw;
+    const u32 row = first + rg;
+    float xv[M][DENSE_LANE_COLS];
+    typename T::Raw wv[S::NCH];
+    sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, 0, live && row < rows, wv);
+    sl.inputs(r, cols, m, 0, xv);
+    for (u32 i = tid; i < m * cs * wide; i += blockDim.x) part[i] = 0.0;
     __syncthreads();
-#pragma unroll 1
-    for (u32 it = 0; it < rpw; it++, row += 4) {
-        if (row >= rows) break;   // the same for every lane of the wave
-        const u32 next = row + 4;
-        if (it + 1 < rpw) dense_load_w<T>(w + (u64) min(next, rows - 1) * cols * T::BYTES, 0, cols, next < rows, lane, wn);
-        float acc[8];
+    float acc[M];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            acc[j] = 0.0f;
-            if ((u32) j < m) {
+    for (int j = 0; j < M; j++) acc[j] = 0.0f;
+    // pass 0: the spans' sums of squares and, while all of the inputs are in registers (outer == 1), the products without the
+    // streams' scales, which are factored out of a lane's sums over one chunk; pass 1 (longer rows): the products
+    float raw[S::NCH][M];
+    for (u32 o = 0; o < outer; o++) {
+        if (o) sl.inputs(r, cols, m, o, xv);
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const u32 c = 4 * lane + 256 * i;
-                    if (c < cols) {
-                        const f32x4 xv = *(const f32x4*) (xl + j * cols + c);
-                        acc[j] = __builtin_fmaf(wv[i].x, xv.x, acc[j]);
-                        acc[j] = __builtin_fmaf(wv[i].y, xv.y, acc[j]);
-                        acc[j] = __builtin_fmaf(wv[i].z, xv.z, acc[j]);
-                        acc[j] = __builtin_fmaf(wv[i].w, xv.w, acc[j]);
+        for (int i = 0; i < S::NCH; i++) {
+            const u32 c0 = ((o * S::NCH + i) * kwn + sl.kw) * span;   // the span's first column: a span touches one stream, or several where h is small
+            const u32 c = c0 + lane * T::C, mine = c / h;
+            if (rg == 0 && c0 < cols) {
+                double sq[M];
+#pragma unroll
+                for (int j = 0; j < M; j++) {
+                    sq[j] = 0.0;
+                    if (c < cols)
+#pragma unroll
+                        for (int e = 0; e < (int) T::C; e++) sq[j] = __builtin_fma((double) xv[j][i * T::C + e], (double) xv[j][i * T::C + e], sq[j]);
+                }
+                for (u32 s = c0 / h; s <= (min(c0 + span, cols) - 1) / h; s++) {
+#pragma unroll
+                    for (int j = 0; j < M; j++) {
+                        if ((u32) j < m) {
+                            const double ss = wave_sum_f64(mine == s ? sq[j] : 0.0, lane);
+                            if (lane == 0) part[((u64) j * cs + s) * wide + (c0 / span - s * h / span)] = ss;
+                        }
                     }
                 }
             }
         }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if ((u32) j < m) {
-                const float t = seg_sum<64>(acc[j], lane);
-                if (lane == 0) y[(u64) j * ys + row] = dense_act(t, act, div);
-            }
+        if (outer == 1) hc_products<T, M>(sl, wv, xv, nw, 0, raw);
+    }
+    __syncthreads();
+    for (u32 i = tid; i < m * cs; i += blockDim.x) {
+        double ss = 0.0;
+        for (u32 q = 0; q < wide; q++) ss += part[i * wide + q];
+        const double sc = 1.0 / sqrt(ss / (double) h + (double) eps);
+        scl[i] = (float) sc;
+        if (blockIdx.x == 0) scales[i] = sc;
+    }
+    __syncthreads();
+    for (u32 o = 0; o < outer; o++) {
+        if (outer > 1) {
+            sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, o, live && row < rows, wv);
+            sl.inputs(r, cols, m, o, xv);
+            hc_products<T, M>(sl, wv, xv, nw, o, raw);
         }
 #pragma unroll
-        for (int i = 0; i < 8; i++) wv[i] = wn[i];
+        for (int i = 0; i < S::NCH; i++) {
+            const u32 s = min(sl.col(o, i), cols - 1) / h;
+#pragma unroll
+            for (int j = 0; j < M; j++) acc[j] = __builtin_fmaf(raw[i][j], scl[min((u32) j, m - 1) * cs + s], acc[j]);
+        }
+    }
+    const float t = dense_reduce<M>(acc, 64, lane);
+    if (live && lane < (u32) M) red[wave * 8 + lane] = t;
+    __syncthreads();
+    const u32 q = tid / 8, j = tid & 7, orow = first + q;
+    if (q < rw && j < m && orow < rows) {
+        float s = red[q * kwn * 8 + j];
+        for (u32 v = 1; v < kwn; v++) s += red[(q * kwn + v) * 8 + j];
+        y[(u64) j * ys + orow] = dense_act(s, act, (float) cs);
     }
 }
-
-// Workgroups a matrix of `rows` rows needs: one a row when the rows are long, one for every 4 * dense_rpw(rows) rows otherwise.
-// Workgroup g (counted from the matrix's first) of the launch:
-template <class T>
-__device__ __forceinline__ void dense_group(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 g, u32 act,
-                                            float div) {
-    if (cols > DENSE_CHUNK) {
-        if (g < rows) dense_wide<T>(w, x, xs, y, ys, g, cols, m, act, div);
+template <int M>
+__device__ __forceinline__ void hc_down_of(u32 type, const u8* w, u32 rows, u32 first, const float* r, const float* nw, double* scales, u32 h, u32 cs, u32 m, float eps, float* red,
+                                           u32 act, float* y, u32 ys) {
+    // spans stay whole inside a stream's 4-column groups: 8 columns a load only where a stream is a multiple of 8
+    if (type == 0) hc_down_rows<DenseF32, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+    else if (type == 1) {
+        if (h % 8 == 0) hc_down_rows<Dense16<false, 8>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+        else hc_down_rows<Dense16<false, 4>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
     } else {
-        const u32 rpw = dense_rpw(rows);
-        dense_narrow<T>(w, x, xs, y, ys, g * 4 * rpw, rpw, rows, cols, m, act, div);
+        if (h % 8 == 0) hc_down_rows<Dense16<true, 8>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+        else hc_down_rows<Dense16<true, 4>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
     }
 }
+template <int M>
+__device__ __forceinline__ void hc_down(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down, float* g, u32 h,
+                                        u32 cs, u32 m, float eps) {
+    __shared__ float red[64];
+    const u32 pass = (blockDim.x >> 6) / dense_waves(h * cs), groups = (rank + pass - 1) / pass;
+    if (blockIdx.x < groups) hc_down_of<M>(type, w, rank, blockIdx.x * pass, r, nw, (double*) scales, h, cs, m, eps, red, 1, down, rank);
+    else hc_down_of<M>(gate_type, gate_w, cs, (blockIdx.x - groups) * pass, r, nw, (double*) scales, h, cs, m, eps, red, 2, g, cs);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_m1(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
+    hc_down<1>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_m4(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
+    hc_down<4>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_m8(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
+    hc_down<8>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+}
 
-// y_j = W x_j for an unquantized row-major W[rows][cols], j < m <= 8 (matvec_cols_*, kernels/matvec.cu:677).
-// cols <= 2048: grid = ceil(rows / (4 * dense_rpw(rows))), dynamic LDS = m * cols * 4; longer rows: grid = rows, dynamic LDS = 128.  block 256.
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_f32(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {
-    dense_group<DenseF32>(w, x, xs, y, ys, rows, cols, m, blockIdx.x, 0, 1.0f);
+// The second: u[j][i] = (sum over the streams s, in order, of sigmoid(up row s h + i . down_j) * the normalised r[j][s h + i]) / streams.
+// A wave takes 64 / G columns i at a time and the streams' rows of them one after the other, the next row's weights on their
+// way, so that the sum over the streams needs nobody else.  grid = ceil(h / (4 * 64 / G)), block 256.
+template <class T, int M>
+__device__ __forceinline__ void hc_up_rows(const u8* __restrict__ w, const float* __restrict__ down, const float* __restrict__ r, const float* __restrict__ nw,
+                                           const double* __restrict__ scales, float* __restrict__ u, u32 h, u32 cs, u32 rank, u32 m) {
+    typedef DenseSlice<T> S;
+    const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const u32 G = dense_lanes(rank), per = 64 / G;
+    const S sl{0, 1, G, lane & (G - 1), rank};
+    const u32 i0 = (blockIdx.x * 4 + wave) * per + lane / G, i = min(i0, h - 1);
+    const u32 outer = (rank + G * DENSE_LANE_COLS - 1) / (G * DENSE_LANE_COLS);
+    // the lane that ends up with output j holds its terms too
+    const bool spread = G >= (u32) M;
+    const u32 j0 = spread ? min(sl.gl & (M - 1), m - 1) : 0;
+    float xv[M][DENSE_LANE_COLS];
+    typename T::Raw wv[S::NCH], wn[S::NCH];
+    sl.weights(w + (u64) i * rank * T::BYTES, 0, true, wv);
+    sl.inputs(down, rank, m, 0, xv);
+    float a[M];
+#pragma unroll
+    for (int j = 0; j < M; j++) a[j] = 0.0f;
+    for (u32 s = 0; s < cs; s++) {
+        const u64 at = (u64) s * h + i;
+        if (s + 1 < cs) sl.weights(w + (at + h) * rank * T::BYTES, 0, true, wn);
+        const float n = nw[at], rv = r[(u64) j0 * cs * h + at];
+        const double sc = scales[j0 * cs + s];
+        float acc[M];
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[j] = 0.0f;
+        for (u32 o = 0; o < outer; o++) {
+            if (outer > 1 && o + s > 0) {
+                if (o) sl.weights(w + at * rank * T::BYTES, o, true, wv);
+                sl.inputs(down, rank, m, o, xv);
+            }
+            sl.dot(wv, xv, acc);
+        }
+        const float t = dense_reduce<M>(acc, G, lane);
+        if (spread) {
+            a[0] += sigmoidf_ref(t) * ((float) ((double) rv * sc) * n);
+        } else {
+#pragma unroll
+            for (int j = 0; j < M; j++)
+                if ((u32) j < m) a[j] += sigmoidf_ref(acc[j]) * ((float) ((double) r[(u64) j * cs * h + at] * scales[j * cs + s]) * n);
+        }
+#pragma unroll
+        for (int q = 0; q < S::NCH; q++) wv[q] = wn[q];
+    }
+    if (i0 < h) {
+        if (spread) {
+            if (sl.gl < m && sl.gl < (u32) M) u[(u64) sl.gl * h + i] = a[0] / (float) cs;
+        } else if (sl.gl == 0) {
+#pragma unroll
+            for (int j = 0; j < M; j++)
+                if ((u32) j < m) u[(u64) j * h + i] = a[j] / (float) cs;
+        }
+    }
 }
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_f16(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {
-    dense_group<DenseF16>(w, x, xs, y, ys, rows, cols, m, blockIdx.x, 0, 1.0f);
+template <int M>
+__device__ __forceinline__ void hc_up(u32 type, const u8* w, const float* down, const float* r, const float* nw, const u8* scales, float* u, u32 h, u32 cs, u32 rank, u32 m) {
+    const double* sc = (const double*) scales;
+    if (type == 0) hc_up_rows<DenseF32, M>(w, down, r, nw, sc, u, h, cs, rank, m);
+    else if (type == 1) {
+        if (rank % 8 == 0) hc_up_rows<Dense16<false, 8>, M>(w, down, r, nw, sc, u, h, cs, rank, m);
+        else hc_up_rows<Dense16<false, 4>, M>(w, down, r, nw, sc, u, h, cs, rank, m);
+    } else {
+        if (rank % 8 == 0) hc_up_rows<Dense16<true, 8>, M>(w, down, r, nw, sc, u, h, cs, rank, m);
+        else hc_up_rows<Dense16<true, 4>, M>(w, down, r, nw, sc, u, h, cs, rank, m);
+    }
 }
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_bf16(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {
-    dense_group<DenseBF16>(w, x, xs, y, ys, rows, cols, m, blockIdx.x, 0, 1.0f);
+extern "C" __global__ void __launch_bounds__(256) hc_up_m1(u32 type, const u8* w, const float* down, const float* r, const float* nw, const u8* scales, float* u, u32 h, u32 cs,
+                                                           u32 rank, u32 m) {
+    hc_up<1>(type, w, down, r, nw, scales, u, h, cs, rank, m);
 }
-
-// Several unquantized matrices on the same inputs in one launch (matvec_cols_multi, kernels/matvec.cu:1958: the router and
-// the shared expert's gate logit).  jobs[i] = {u64 w, u64 y, u32 ys, u32 rows, u32 type (0 F32, 1 F16, 2 BF16), u32 first, u32 act, f32 div} (dense_act):
-// job i owns workgroups [first_i, first_{i+1}), as many as its matrix needs on its own (dense_group); every output is the
-// one-matrix kernel's bit for bit.  block 256, dynamic LDS as for one matrix.
-struct DenseJob {
-    u64 w, y;
-    u32 ys, rows, type, first, act;
-    float div;
-};
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_multi(const u8* jobs, u32 njobs, const float* x, u32 xs, u32 cols, u32 m) {
-    const DenseJob* jt = (const DenseJob*) jobs;
-    u32 i = 0;
-    while (i + 1 < njobs && blockIdx.x >= jt[i + 1].first) i++;
-    const DenseJob jb = jt[i];
-    const u32 g = blockIdx.x - jb.first;
-    if (jb.type == 0) dense_group<DenseF32>((const u8*) jb.w, x, xs, (float*) jb.y, jb.ys, jb.rows, cols, m, g, jb.act, jb.div);
-    else if (jb.type == 1) dense_group<DenseF16>((const u8*) jb.w, x, xs, (float*) jb.y, jb.ys, jb.rows, cols, m, g, jb.act, jb.div);
-    else dense_group<DenseBF16>((const u8*) jb.w, x, xs, (float*) jb.y, jb.ys, jb.rows, cols, m, g, jb.act, jb.div);
+extern "C" __global__ void __launch_bounds__(256) hc_up_m4(u32 type, const u8* w, const float* down, const float* r, const float* nw, const u8* scales, float* u, u32 h, u32 cs,
+                                                           u32 rank, u32 m) {
+    hc_up<4>(type, w, down, r, nw, scales, u, h, cs, rank, m);
+}
+extern "C" __global__ void __launch_bounds__(256) hc_up_m8(u32 type, const u8* w, const float* down, const float* r, const float* nw, const u8* scales, float* u, u32 h, u32 cs,
+                                                           u32 rank, u32 m) {
+    hc_up<8>(type, w, down, r, nw, scales, u, h, cs, rank, m);
 }
 
 // ------------------------------------------------------------------------------------------------ lm_head + argmax

@@ -643,35 +643,6 @@ extern "C" __global__ void __launch_bounds__(256) copy_ranges(const u64* table, 
 }
 
 // ------------------------------------------------------------------------ the hyper-connection around a sublayer
-// rmsnorm over every stream of every row on its own (forward.rs:251-260; rmsnorm_groups_rows of the reference): the mean
-// of squares and the scaling in f64 as the CPU path has them, out = (float) (x * 1/sqrt(ms + eps)) * w.
-// r, rn: [m][cs * h]; w: [cs * h].  grid = (cs, m), block 256.
-extern "C" __global__ void __launch_bounds__(256) rmsnorm_groups_rows(const float* r, const float* w, float* rn, u32 h, float eps, u32 cs) {
-    __shared__ double red[4];
-    const u32 s = blockIdx.x, j = blockIdx.y, tid = threadIdx.x;
-    const float* x = r + ((u64) j * cs + s) * h;
-    double ss = 0.0;
-    for (u32 i = tid; i < h; i += 256) ss += (double) x[i] * (double) x[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, SZ_WAVE);
-    if (tid % 64 == 0) red[tid / 64] = ss;
-    __syncthreads();
-    const double ms = (((red[0] + red[1]) + red[2]) + red[3]) / (double) h;
-    const double sc = 1.0 / sqrt(ms + (double) eps);
-    float* o = rn + ((u64) j * cs + s) * h;
-    for (u32 i = tid; i < h; i += 256) o[i] = (float) ((double) x[i] * sc) * w[s * h + i];
-}
-
-// u[j][i] = (sum over streams s, in order, of mix[j][s h + i] * rn[j][s h + i]) / cs (forward.rs:806-812; hc_mix_rows).
-// grid = (ceil(h / 256), m), block 256.
-extern "C" __global__ void __launch_bounds__(256) hc_mix_rows(const float* rn, const float* mix, float* u, u32 h, u32 cs) {
-    const u32 i = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y;
-    if (i >= h) return;
-    float a = 0.0f;
-    for (u32 s = 0; s < cs; s++) a += mix[((u64) j * cs + s) * h + i] * rn[((u64) j * cs + s) * h + i];
-    u[(u64) j * h + i] = a / (float) cs;
-}
-
 // hc_write (forward.rs:1078-1084): r[j][s h + i] += g[j][s] * y[j][i].  grid = (ceil(h / 256), cs, m), block 256.
 extern "C" __global__ void __launch_bounds__(256) hc_write_rows(float* r, const float* g, const float* y, u32 h, u32 cs) {
     const u32 i = blockIdx.x * 256 + threadIdx.x, s = blockIdx.y, j = blockIdx.z;

@@ -114,6 +114,13 @@ __device__ __forceinline__ void lds_load(const void* g, u32 lds) {
 #undef SZ_LDS_LOAD
 }
 
+// The 16-byte form from a wave-uniform address plus the lane's 32-bit offset: no 64-bit address arithmetic a lane.
+__device__ __forceinline__ void lds_load_at(u64 base, u32 off, u32 lds) {
+    u32 keep;
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(lds), "s"(base) : "memory");
+}
+
 // A 4-byte global load the compiler keeps no count of (as lds_load's): the caller orders it with wait_vm and must pass the
 // value through load_landed() after the wait and before its first use, which keeps the compiler from moving a use ahead.
 __device__ __forceinline__ float load_f32_uncounted(const float* p) {

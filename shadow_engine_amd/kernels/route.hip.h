@@ -294,3 +294,86 @@ __device__ __forceinline__ float route_weights_chosen(const float* lg, u32 ne, u
     *count = kk;
     return e != 0xffffffffu ? (float) (mine / tz) : 0.0f;
 }
+
+// The plan of a verify batch of m <= 8 tokens: pbuf holds u32 tidx[m k] | f32 w[m k] | u32 cnt[m] (w and cnt are filled in
+// later), then at byte ioff (16-byte aligned) u32 n_items, 3 unused words, and 8 words an item, an item being a DISTINCT
+// expert: expert (0xffffffff: the shared one, with every token, the first item), n tokens, their rows as 8 bytes, their pair
+// numbers as 8 u16 (pair j k + t of token j and rank t, m k + j for the shared expert).
+// Made by one workgroup of any number of waves (up to 8), a wave a token.  The items come out of three tables in LDS indexed
+// by expert: the lowest pair that chose it (that pair's lane writes the item), the tokens that chose it as a bit mask, and
+// each such token's rank.  logits: m rows of ne, in memory or in LDS.
+struct RoutePlanLds {
+    double ex[8 * 512];   // the exact selection's scratch, a wave's 512 doubles
+    u32 top[8][16];
+    u32 lowest[512];      // expert -> the lowest pair number that chose it
+    u32 tokens[512];      // expert -> bit j: token j chose it
+    u8 rank[512 * 8];     // expert, token -> the token's rank of it
+    u32 items[8];         // token -> items its pairs write
+};
+__device__ __forceinline__ void route_plan(const float* logits, u8* pbuf, u32 ioff, u32 ne, u32 k, u32 m, bool shared, RoutePlanLds& s) {
+    const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6, G = m * k;
+    u32* tidx = (u32*) pbuf;
+    u32* plan = (u32*) (pbuf + ioff);
+    for (u32 i = threadIdx.x; i < 512; i += blockDim.x) {
+        s.lowest[i] = 0xffffffffu;
+        s.tokens[i] = 0;
+    }
+    for (u32 j = wave; j < m; j += nw) route_ids(logits + (u64) j * ne, ne, k, lane, s.ex + wave * 512, s.top[j]);
+    __syncthreads();
+    for (u32 j = wave; j < m; j += nw) {
+        const u32 e = lane < k ? s.top[j][lane] : 0xffffffffu;
+        if (lane < k) tidx[j * k + lane] = e;
+        if (e != 0xffffffffu) {
+            atomicMin(&s.lowest[e], j * k + lane);
+            atomicOr(&s.tokens[e], 1u << j);
+            s.rank[e * 8 + j] = (u8) lane;
+        }
+    }
+    __syncthreads();
+    for (u32 j = wave; j < m; j += nw) {
+        const u32 e = lane < k ? s.top[j][lane] : 0xffffffffu;
+        const u64 firsts = __builtin_amdgcn_ballot_w64(e != 0xffffffffu && s.lowest[e] == j * k + lane);
+        if (lane == 0) s.items[j] = __builtin_popcountll(firsts);
+    }
+    __syncthreads();
+    for (u32 j = wave; j < m; j += nw) {
+        const u32 e = lane < k ? s.top[j][lane] : 0xffffffffu;
+        const bool isf = e != 0xffffffffu && s.lowest[e] == j * k + lane;
+        const u64 firsts = __builtin_amdgcn_ballot_w64(isf);
+        u32 slot = shared ? 1u : 0u;
+        for (u32 w = 0; w < j; w++) slot += s.items[w];
+        if (isf) {
+            slot += __builtin_popcountll(firsts & ((1ull << lane) - 1));
+            u32 n = 0;
+            u64 toks = 0, pr0 = 0, pr1 = 0;
+            for (u32 mask = s.tokens[e]; mask; mask &= mask - 1) {
+                const u32 jj = __builtin_ctz(mask);
+                toks |= (u64) jj << (8 * n);
+                const u64 pv = jj * k + s.rank[e * 8 + jj];
+                if (n < 4) pr0 |= pv << (16 * n);
+                else pr1 |= pv << (16 * (n - 4));
+                n++;
+            }
+            u32x4* rec = (u32x4*) (plan + 4 + 8 * slot);
+            rec[0] = u32x4{e, n, (u32) toks, (u32) (toks >> 32)};
+            rec[1] = u32x4{(u32) pr0, (u32) (pr0 >> 32), (u32) pr1, (u32) (pr1 >> 32)};
+        }
+    }
+    if (threadIdx.x == 0) {
+        u32 count = shared ? 1u : 0u;
+        for (u32 w = 0; w < m; w++) count += s.items[w];
+        plan[0] = count;
+        if (shared) {
+            u64 toks = 0, pr0 = 0, pr1 = 0;
+            for (u32 jj = 0; jj < m; jj++) {
+                toks |= (u64) jj << (8 * jj);
+                const u64 pv = G + jj;
+                if (jj < 4) pr0 |= pv << (16 * jj);
+                else pr1 |= pv << (16 * (jj - 4));
+            }
+            u32x4* rec = (u32x4*) (plan + 4);
+            rec[0] = u32x4{0xffffffffu, m, (u32) toks, (u32) (toks >> 32)};
+            rec[1] = u32x4{(u32) pr0, (u32) (pr0 >> 32), (u32) pr1, (u32) (pr1 >> 32)};
+        }
+    }
+}
