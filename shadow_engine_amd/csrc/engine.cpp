@@ -108,8 +108,17 @@ struct DevBuf {
     }
 };
 
+// The variant of a verify launch over `cols` output columns: column tiles a wave and the kernel name's prefix.  `waves8` is the
+// number of waves that 8 tiles a wave would give: they do least work for their A rows (a round of 48 layers 931 us, with 4 tiles
+// 957, with 2 1033) but leave SIMDs idle where there are few of them (a layer alone at 4 rows: 51 us with 2 tiles, 63 with 8).
+static const char* verify_variant(uint64_t cols, uint64_t waves8, uint32_t m, uint32_t* ct) {
+    *ct = cols % 512 == 0 && waves8 >= 8192 ? 8 : cols % 256 == 0 && waves8 >= 2048 ? 4 : 2;
+    if (m > 4) return *ct == 8 ? "w_" : *ct == 4 ? "t4w_" : "t2w_";
+    return *ct == 8 ? "" : *ct == 4 ? "t4_" : "t2_";
+}
+
 // ---- one product y_j = W x_j, j < m, on device pointers ---------------------------------------------------------------
-// EXL3 workspace layout: u64 wtab[ng] | u32 gtab[17 ng] (16-byte aligned) | f32 part[ng * ks * 4 * rows]
+// EXL3 workspace: f32 part[m][ks][rows] (callers have always been asked for more: the size they know stays)
 static uint64_t align16(uint64_t v) { return (v + 15) & ~15ull; }
 
 static uint64_t cols_scratch_bytes(const Format& f, uint64_t cols, uint64_t rows, uint32_t m) {
@@ -129,16 +138,14 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
     if (f.exl3) {
         if (check_exl3_shape(cols, rows)) return 1;
         if (xs % 4 || (x & 15)) return fail("matvec_cols: inputs must be 16-byte aligned");
-        const uint32_t ng = (m + 3) / 4, ks = exl3_ksplit((uint32_t) cols);
         if (scratch_bytes < cols_scratch_bytes(f, cols, rows, m) || !scratch) return fail("matvec_cols: workspace too small for EXL3");
-        const uint64_t wtab = scratch, gtab = scratch + align16(ng * 8), part = gtab + align16(ng * 17 * 4);
-        const sz_arg a0[] = {P(wtab), P(gtab), U64(w), U32(m)};
-        if (launch("cols_plan", 1, 1, 1, 64, 0, stream, a0)) return 1;
-        const std::string kn = "matvec_grouped_" + tag;
-        const sz_arg a1[] = {P(wtab), P(gtab), P(x), U32(xs), P(part), U32((uint32_t) cols), U32((uint32_t) rows)};
-        if (launch(kn.c_str(), (uint32_t) rows / 128, ng, ks, 256, 0, stream, a1)) return 1;
-        const sz_arg a2[] = {P(part), P(wtab), P(gtab), P(y), U32(ys), U32((uint32_t) cols), U32((uint32_t) rows)};
-        return launch("exl3_finish_rows", (uint32_t) rows / 128, ng, 1, 64, 0, stream, a2);
+        const uint32_t zs = exl3_ksplit((uint32_t) cols);
+        uint32_t ct;
+        const std::string kn = std::string("matvec_grouped_") + verify_variant(rows, rows / 128 * zs, m, &ct) + tag;
+        const sz_arg a0[] = {P(w), P(x), U32(xs), P(scratch), U32((uint32_t) cols), U32((uint32_t) rows), U32(m)};
+        if (launch(kn.c_str(), (uint32_t) rows / (64 * ct), zs, 1, 256, 0, stream, a0)) return 1;
+        const sz_arg a1[] = {P(scratch), P(w), P(y), U32(ys), U32((uint32_t) cols), U32((uint32_t) rows)};
+        return launch("exl3_finish_rows", (uint32_t) rows / 128, m, 1, 64, 0, stream, a1);
     }
     if (f.dense) {
         if (rows == 0) return 0;
@@ -391,15 +398,6 @@ VerifyPlan verify_plan(uint32_t m, uint32_t k) {
 // column) and launch 3's.
 uint64_t verify_part_bytes(const sz_session_config& c, uint32_t m) { return 2ull * m * (c.top_k + 1) * exl3_ksplit(c.hidden) * c.ff * 4; }
 uint64_t verify_dn_bytes(const sz_session_config& c, uint32_t m) { return (uint64_t) m * (c.top_k + 1) * exl3_ksplit(c.ff) * c.hidden * 4; }
-
-// The variant of a verify launch over `cols` output columns: column tiles a wave and the kernel name's prefix.  `waves8` is the
-// number of waves that 8 tiles a wave would give: they do least work for their A rows (a round of 48 layers 931 us, with 4 tiles
-// 957, with 2 1033) but leave SIMDs idle where there are few of them (a layer alone at 4 rows: 51 us with 2 tiles, 63 with 8).
-const char* verify_variant(uint64_t cols, uint64_t waves8, uint32_t m, uint32_t* ct) {
-    *ct = cols % 512 == 0 && waves8 >= 8192 ? 8 : waves8 >= 2048 ? 4 : 2;
-    if (m > 4) return *ct == 8 ? "w_" : *ct == 4 ? "t4w_" : "t2w_";
-    return *ct == 8 ? "" : *ct == 4 ? "t4_" : "t2_";
-}
 
 // The EXL3 layers table[p0 .. p1) for a batch of m rows: u, rl, sgl, y and `plans` are the caller's, layer `base`'s part first.
 int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t plans, uint64_t stream) {

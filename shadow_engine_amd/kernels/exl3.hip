@@ -126,6 +126,26 @@ __device__ __forceinline__ void exl3_decode_kernel(const u8* blob, float* what, 
     for (int i = 0; i < 32; i++) what[(u64) (kt * 16 + EXL3_ROW(i)) * out_f + col + 8 * EXL3_HALF(i)] = (float) w[i / 2][i % 2];
 }
 
+#define EXL3_ENTRIES(K)                                                                                                              \
+    extern "C" __global__ void __launch_bounds__(64) exl3_decode_##K(const u8* blob, float* what, u32 in_f, u32 out_f) {             \
+        exl3_decode_kernel<K>(blob, what, in_f, out_f);                                                                              \
+    }
+#define EXL3_HALF_ENTRIES(K)                                                                                                         \
+    extern "C" __global__ void __launch_bounds__(64) exl3_decode_h##K(const u8* blob, float* what, u32 in_f, u32 out_f) {            \
+        exl3_decode_kernel<K, true>(blob, what, in_f, out_f);                                                                        \
+    }
+EXL3_ENTRIES(1)
+EXL3_ENTRIES(2)
+EXL3_ENTRIES(3)
+EXL3_ENTRIES(4)
+EXL3_ENTRIES(5)
+EXL3_ENTRIES(6)
+EXL3_ENTRIES(7)
+EXL3_ENTRIES(8)
+EXL3_HALF_ENTRIES(1)
+EXL3_HALF_ENTRIES(2)
+EXL3_HALF_ENTRIES(3)
+
 template <int h>
 __device__ __forceinline__ void wht_stage(float& v0, float& v1, u32 lane) {
     const float p0 = lane_xor<h>(v0, lane), p1 = lane_xor<h>(v1, lane);
@@ -155,80 +175,6 @@ __device__ __forceinline__ void wht128_wave(float& v0, float& v1, u32 lane) {
     v0 *= 0.08838835f;
     v1 *= 0.08838835f;
 }
-
-// The decode loop of one wave: the 8 tile rows of input block kb against the M rotated inputs in the wave's strip xw
-// (input j at xw[j * 128 ..]); on return the strip holds the partial sums instead (column c of input j at xw[j * 128 + c]).
-template <int K, int M, bool H = false>
-__device__ __forceinline__ void exl3_wave_main(const u8* __restrict__ blob, u32 in_f, u32 out_f, u32 ob, u32 kb, float* xw, u32 lane) {
-    const u32* tr = (const u32*) (blob + 2 * (u64) in_f + 2 * (u64) out_f + 4);
-    const u32 nt = out_f / 16;
-    u32 S[EXL3_NW(K, H)], Sn[EXL3_NW(K, H)];
-    exl3_load_words<K, H>(tr, nt, kb * 8, ob, lane, S);
-    float acc[2][M];
-#pragma unroll
-    for (int j = 0; j < M; j++) acc[0][j] = acc[1][j] = 0.0f;
-#pragma unroll 1
-    for (u32 t = 0; t < 8; t++) {
-        if (t < 7) exl3_load_words<K, H>(tr, nt, kb * 8 + t + 1, ob, lane, Sn);   // the next tile row's words, in flight while this one decodes
-        f16x2 w[16];
-        exl3_decode32<K, H>(S, w);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            // weights 8 q .. 8 q + 7 sit on input rows 2 q, 2 q + 1, 2 q + 8, 2 q + 9 of the tile row
-            float xa[M][4];
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                const float* xr = xw + j * 128 + t * 16 + 2 * q;
-                xa[j][0] = xr[0];
-                xa[j][1] = xr[1];
-                xa[j][2] = xr[8];
-                xa[j][3] = xr[9];
-            }
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int i = 8 * q + e;
-                const int r = (e & 1) + 2 * ((e >> 1) & 1);
-#pragma unroll
-                for (int j = 0; j < M; j++) acc[EXL3_HALF(i)][j] = __builtin_fmaf((float) w[i / 2][i % 2], xa[j][r], acc[EXL3_HALF(i)][j]);
-            }
-        }
-#pragma unroll
-        for (int d = 0; d < EXL3_NW(K, H); d++) S[d] = Sn[d];
-    }
-    __builtin_amdgcn_wave_barrier();
-    const u32 col = (lane >> 3) * 16 + (lane & 7);
-#pragma unroll
-    for (int j = 0; j < M; j++) {
-        xw[j * 128 + col] = acc[0][j];
-        xw[j * 128 + col + 8] = acc[1][j];
-    }
-}
-
-// One wave = one 128-block of inputs (8 tile rows) of one 128-output block of one group: it rotates its block of every
-// input (x * suh, then the transform) into a wave-private strip of LDS, decodes its 8 x 8 tiles into the partial sums of
-// (x * suh) H W_hat for its two output columns a lane, and leaves them in its strip for the workgroup to add up.
-template <int K, int M, bool H = false>
-__device__ __forceinline__ void exl3_wave_body(const u8* __restrict__ blob, const float* __restrict__ x, u32 xs, const u32* __restrict__ rec,
-                                               u32 n, u32 in_f, u32 out_f, u32 ob, u32 kb, float* xw, u32 lane) {
-    const u16* suh = (const u16*) blob;
-    const float s0 = f16_to_f32(suh[kb * 128 + lane]), s1 = f16_to_f32(suh[kb * 128 + 64 + lane]);
-#pragma unroll
-    for (int j = 0; j < M; j++) {
-        float v0 = 0.0f, v1 = 0.0f;
-        if ((u32) j < n) {
-            const float* xj = x + (u64) rec[1 + j] * xs + kb * 128;
-            v0 = xj[lane] * s0;
-            v1 = xj[lane + 64] * s1;
-            wht128_wave(v0, v1, lane);
-        }
-        xw[j * 128 + lane] = v0;
-        xw[j * 128 + 64 + lane] = v1;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    exl3_wave_main<K, M, H>(blob, in_f, out_f, ob, kb, xw, lane);
-}
-
 
 // ------------------------------------------------------------------------------------- trellis rows through the LDS
 // A wave's whole share of a projection (the 8 tile rows of its 128 x 128 block, 2 K KiB) is requested in one burst of
@@ -296,101 +242,6 @@ __device__ __forceinline__ void exl3_rows_wait(u32 t) {
         case 5: wait_vm<Exl3Rows<K, D, H>::after(5)>(); break;
         case 6: wait_vm<Exl3Rows<K, D, H>::after(6)>(); break;
         default: wait_vm<0>(); break;
-    }
-}
-
-// Group g = blockIdx.y: blob wtab[g], record gtab[17 g] = {n <= 4 (0: unused slot), xi[8], yi[8]}; wave w of the workgroup
-// takes input block 4 blockIdx.z + w, and the four waves' sums are added in wave order into
-// part[((g * gridDim.z + blockIdx.z) * 4 + j) * out + col], j < n.  grid = (out / 128, groups, ceil(in / 512)), block 256.
-template <int K, bool H = false>
-__device__ __forceinline__ void exl3_grouped_kernel(const u64* __restrict__ wtab, const u32* __restrict__ gtab, const float* __restrict__ x, u32 xs,
-                                                    float* __restrict__ part, u32 in_f, u32 out_f) {
-    __shared__ float xw_all[4][4 * 128];
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // the wave index as a scalar: the index arithmetic on it is the scalar unit's
-    const u32 kb = blockIdx.z * 4 + wave;
-    const u32* rec = gtab + 17 * (u64) blockIdx.y;
-    const u32 n = min(rec[0], 4u);
-    if (n == 0) return;
-    const u8* blob = (const u8*) wtab[blockIdx.y];
-    float* xw = xw_all[wave];
-    const bool live = kb < in_f / 128;
-    if (live) {
-        if (n == 1) exl3_wave_body<K, 1, H>(blob, x, xs, rec, n, in_f, out_f, blockIdx.x, kb, xw, lane);
-        else if (n == 2) exl3_wave_body<K, 2, H>(blob, x, xs, rec, n, in_f, out_f, blockIdx.x, kb, xw, lane);
-        else exl3_wave_body<K, 4, H>(blob, x, xs, rec, n, in_f, out_f, blockIdx.x, kb, xw, lane);
-    }
-    __syncthreads();
-    const u32 nw = min(4u, in_f / 128 - blockIdx.z * 4);   // waves of this workgroup that had a block
-    for (u32 p = threadIdx.x; p < n * 128; p += 256) {
-        float v = xw_all[0][p];
-        for (u32 w = 1; w < nw; w++) v += xw_all[w][p];
-        part[(((u64) blockIdx.y * gridDim.z + blockIdx.z) * 4 + (p >> 7)) * out_f + blockIdx.x * 128 + (p & 127)] = v;
-    }
-}
-
-#define EXL3_ENTRIES(K)                                                                                                              \
-    extern "C" __global__ void __launch_bounds__(64) exl3_decode_##K(const u8* blob, float* what, u32 in_f, u32 out_f) {             \
-        exl3_decode_kernel<K>(blob, what, in_f, out_f);                                                                              \
-    }                                                                                                                                \
-    extern "C" __global__ void __launch_bounds__(256) matvec_grouped_exl3_##K(const u64* wtab, const u32* gtab, const float* x, u32 xs, \
-                                                                               float* part, u32 in_f, u32 out_f) {                     \
-        exl3_grouped_kernel<K>(wtab, gtab, x, xs, part, in_f, out_f);                                                                \
-    }
-
-// K + 1/2 bits a weight (type ids 1030 + K, K = 1..3)
-#define EXL3_HALF_ENTRIES(K)                                                                                                         \
-    extern "C" __global__ void __launch_bounds__(64) exl3_decode_h##K(const u8* blob, float* what, u32 in_f, u32 out_f) {            \
-        exl3_decode_kernel<K, true>(blob, what, in_f, out_f);                                                                        \
-    }                                                                                                                                \
-    extern "C" __global__ void __launch_bounds__(256) matvec_grouped_exl3h_##K(const u64* wtab, const u32* gtab, const float* x, u32 xs, \
-                                                                                float* part, u32 in_f, u32 out_f) {                    \
-        exl3_grouped_kernel<K, true>(wtab, gtab, x, xs, part, in_f, out_f);                                                          \
-    }
-
-EXL3_HALF_ENTRIES(1)
-EXL3_HALF_ENTRIES(2)
-EXL3_HALF_ENTRIES(3)
-
-EXL3_ENTRIES(1)
-EXL3_ENTRIES(2)
-EXL3_ENTRIES(3)
-EXL3_ENTRIES(4)
-EXL3_ENTRIES(5)
-EXL3_ENTRIES(6)
-EXL3_ENTRIES(7)
-EXL3_ENTRIES(8)
-
-// The lane's two elements (`lane`, `lane + 64` of the 128-output block starting at `base`) of the sum over the zs partials
-// of (group g, input j), in order.
-__device__ __forceinline__ void exl3_part_sum2(const float* __restrict__ part, u32 g, u32 j, u32 zs, u32 out_f, u32 base, u32 lane, float& v0,
-                                               float& v1) {
-    v0 = 0.0f;
-    v1 = 0.0f;
-    for (u32 z = 0; z < zs; z++) {
-        const float* p = part + (((u64) g * zs + z) * 4 + j) * out_f + base;
-        v0 += p[lane];
-        v1 += p[lane + 64];
-    }
-}
-
-// y[yi[j]] = (sum of partials) H * svh for every input of every group: the output half of exl3.rs:557-564.
-// grid = (out / 128, groups), block 64.
-extern "C" __global__ void __launch_bounds__(64) exl3_finish_rows(const float* part, const u64* wtab, const u32* gtab, float* y, u32 ys,
-                                                                  u32 in_f, u32 out_f) {
-    const u32 lane = threadIdx.x, ob = blockIdx.x, g = blockIdx.y;
-    const u32* rec = gtab + 17 * (u64) g;
-    const u32 n = min(rec[0], 4u);
-    if (n == 0) return;
-    const u32 zs = (in_f / 128 + 3) / 4;
-    const u16* svh = (const u16*) ((const u8*) wtab[g] + 2 * (u64) in_f) + ob * 128;
-    const float s0 = f16_to_f32(svh[lane]), s1 = f16_to_f32(svh[lane + 64]);
-    for (u32 j = 0; j < n; j++) {
-        float v0, v1;
-        exl3_part_sum2(part, g, j, zs, out_f, ob * 128, lane, v0, v1);
-        wht128_wave(v0, v1, lane);
-        float* o = y + (u64) rec[9 + j] * ys + ob * 128;
-        o[lane] = v0 * s0;
-        o[lane + 64] = v1 * s1;
     }
 }
 
@@ -649,6 +500,54 @@ __device__ __forceinline__ void verify_store(const f32x4 (&acc)[NG][CT], const f
     }
 }
 
+// One projection's products for the 512 inputs of block z and the workgroup's 64 CT columns: token r's inputs start at row(r),
+// its sums go to out + (its pair) * stride + column.
+template <int K, bool H, int CT, int NG, class Row>
+__device__ __forceinline__ void exl3_product(const u8* bp, u32 in_f, u32 out_f, u32 z, Row row, u32 n, const u32 (&pairs)[4], u64 stride, float* __restrict__ out, u32 wave, u32 lane,
+                                             u32* wb, u16* a_sh, float* s_mx, float* s_iv) {
+    constexpr int NMAX = 4 * NG;
+    typedef VerifyRing<K, H, CT> R;
+    const u32 kbs = in_f / 128, kb = z * 4 + wave, nkb = min(4u, kbs - z * 4);
+    const u32 c0 = blockIdx.x * 4 * CT + wave * CT;   // the wave's first column tile
+    R ring;
+    ring.init(bp + 2 * (u64) in_f + 2 * (u64) out_f + 4 + ((u64) z * 32 * (out_f / 16) + c0) * (4 * R::TW), (out_f / 16) * (4 * R::TW), nkb * 8 / R::UR,
+              __builtin_amdgcn_readfirstlane(lds_offset(wb)), lane);
+    // the wave's 128-block of every token and its scales, then the first units of its rows behind them, uncounted.  Every load
+    // is made, past the item's tokens and blocks of an earlier one: a load behind a branch would leave its register to be
+    // copied at the branches' end, before the value is there.
+    float v[NMAX][2];
+    const u32 kbc = min(kb, kbs - 1);
+    const u16* suh = (const u16*) bp + kbc * 128;
+    u32 sc0 = load_u16_uncounted(suh + lane), sc1 = load_u16_uncounted(suh + lane + 64);
+#pragma unroll
+    for (int r = 0; r < NMAX; r++) {
+        const float* xj = row(min((u32) r, n - 1)) + kbc * 128;
+        v[r][0] = load_f32_uncounted(xj + lane);
+        v[r][1] = load_f32_uncounted(xj + lane + 64);
+    }
+    ring.fill(lane);
+    load_landed(sc0);
+    load_landed(sc1);
+#pragma unroll
+    for (int r = 0; r < NMAX; r++) {
+        load_landed(v[r][0]);
+        load_landed(v[r][1]);
+    }
+#pragma unroll
+    for (int r = 0; r < NMAX; r++) {
+        if ((u32) r < n) {
+            v[r][0] *= f16_to_f32((u16) sc0);
+            v[r][1] *= f16_to_f32((u16) sc1);
+            wht128_wave(v[r][0], v[r][1], lane);
+            if (kb >= kbs) v[r][0] = v[r][1] = 0.0f;
+        }
+    }
+    verify_put_rows<NMAX>(a_sh, s_mx, s_iv, v, n, kb < kbs ? wave : 4u, wave, lane);
+    f32x4 acc[NG][CT];
+    verify_products<K, H, CT, NG, NMAX>(ring, wb, a_sh, lane, acc);
+    verify_store<CT, NG>(acc, s_iv, pairs, n, stride, out + c0 * 16, lane);
+}
+
 // The shared expert's item: every token, pairs m k + j.
 __device__ __forceinline__ void verify_shared_item(u32 G, u64& toks, u32 (&pairs)[4]) {
     toks = 0x0706050403020100ull;
@@ -723,46 +622,8 @@ __device__ __forceinline__ void verify_gate_up_kernel(const float* __restrict__ 
         verify_shared_item(G, toks, pairs);
     }
     const u8* bp = (const u8*) uniform_u64((e == 0xffffffffu ? L.shared : L.experts + e * L.stride) + (u64) sel * L.part);
-    const u32 kbs = hidden / 128, kb = z * 4 + wave, nkb = min(4u, kbs - z * 4);
-    const u32 c0 = blockIdx.x * 4 * CT + wave * CT;   // the wave's first column tile
-    R ring;
-    ring.init(bp + 2 * (u64) hidden + 2 * (u64) ff + 4 + ((u64) z * 32 * (ff / 16) + c0) * (4 * R::TW), (ff / 16) * (4 * R::TW), nkb * 8 / R::UR,
-              __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave])), lane);
-    // the wave's 128-block of every token and its scales, then the first units of its rows behind them, uncounted.  Every load
-    // is made, past the item's tokens and blocks of an earlier one: a load behind a branch would leave its register to be
-    // copied at the branches' end, before the value is there.
-    float v[NMAX][2];
-    const u32 kbc = min(kb, kbs - 1);
-    const u16* suh = (const u16*) bp + kbc * 128;
-    u32 sc0 = load_u16_uncounted(suh + lane), sc1 = load_u16_uncounted(suh + lane + 64);
-#pragma unroll
-    for (int r = 0; r < NMAX; r++) {
-        const u32 tok = (u32) (toks >> (8 * min((u32) r, n - 1))) & 0xffu;
-        const float* xj = u + ((u64) l * m + tok) * hidden + kbc * 128;
-        v[r][0] = load_f32_uncounted(xj + lane);
-        v[r][1] = load_f32_uncounted(xj + lane + 64);
-    }
-    ring.fill(lane);
-    load_landed(sc0);
-    load_landed(sc1);
-#pragma unroll
-    for (int r = 0; r < NMAX; r++) {
-        load_landed(v[r][0]);
-        load_landed(v[r][1]);
-    }
-#pragma unroll
-    for (int r = 0; r < NMAX; r++) {
-        if ((u32) r < n) {
-            v[r][0] *= f16_to_f32((u16) sc0);
-            v[r][1] *= f16_to_f32((u16) sc1);
-            wht128_wave(v[r][0], v[r][1], lane);
-            if (kb >= kbs) v[r][0] = v[r][1] = 0.0f;
-        }
-    }
-    verify_put_rows<NMAX>(a_sh, s_mx, s_iv, v, n, kb < kbs ? wave : 4u, wave, lane);
-    f32x4 acc[NG][CT];
-    verify_products<K, H, CT, NG, NMAX>(ring, wb_all[wave], a_sh, lane, acc);
-    verify_store<CT, NG>(acc, s_iv, pairs, n, (u64) zs * ff, gup + (((u64) (li * 2 + sel) * S) * zs + z) * ff + c0 * 16, lane);
+    exl3_product<K, H, CT, NG>(bp, hidden, ff, z, [&](u32 r) { return u + ((u64) l * m + ((u32) (toks >> (8 * r)) & 0xffu)) * hidden; }, n, pairs, (u64) zs * ff,
+                               gup + (((u64) (li * 2 + sel) * S) * zs + z) * ff, wave, lane, wb_all[wave], a_sh, s_mx, s_iv);
 }
 
 // Launch 3: act = silu(gate) * up of every token of the item out of launch 2's sums (partials added, output side of the two
@@ -1068,6 +929,102 @@ extern "C" __global__ void __launch_bounds__(1024) verify_combine_exl3(const flo
         y[((u64) l * m + j) * hidden + ob * 128 + threadIdx.x] = a;
     }
 }
+
+// ------------------------------------------------------------------------------------------- one projection for m <= 8 inputs
+// y_j = ((x_j * suh) H) W_hat H * svh (matvec_cols_exl3_K, kernels/exl3.cu:260) in two launches: the products of the verify
+// layer, 512 inputs and 64 CT columns a workgroup, and the sums' output side.  part: [j][z][out_f].
+// grid = (out / (64 CT), ceil(in / 512)), block 256; the inputs are 4 NG at most.
+template <int K, bool H, int CT, int NG>
+__device__ __forceinline__ void exl3_cols_kernel(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ part, u32 in_f, u32 out_f, u32 m) {
+    constexpr int NMAX = 4 * NG;
+    typedef VerifyRing<K, H, CT> R;
+    __shared__ __attribute__((aligned(16))) u32 wb_all[4][R::D * R::UW];
+    __shared__ __attribute__((aligned(16))) u16 a_sh[16 * 3 * NMAX * 32];
+    __shared__ __attribute__((aligned(16))) float s_mx[4 * NMAX];
+    __shared__ float s_iv[NMAX];
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, z = blockIdx.y;
+    u64 toks;
+    u32 pairs[4];
+    verify_shared_item(0, toks, pairs);
+    exl3_product<K, H, CT, NG>(w, in_f, out_f, z, [&](u32 r) { return x + (u64) r * xs; }, m, pairs, (u64) gridDim.y * out_f, part + (u64) z * out_f, wave, lane, wb_all[wave], a_sh,
+                               s_mx, s_iv);
+}
+
+// y_j's 128-output block ob: the partial sums added up, the output-side transform, the scales.  grid = (out / 128, m), block 64.
+extern "C" __global__ void __launch_bounds__(64) exl3_finish_rows(const float* part, const u8* w, float* y, u32 ys, u32 in_f, u32 out_f) {
+    const u32 lane = threadIdx.x, ob = blockIdx.x, j = blockIdx.y, zs = (in_f / 128 + 3) / 4;
+    const u16* svh = (const u16*) (w + 2 * (u64) in_f) + ob * 128;
+    const float s0 = f16_to_f32(svh[lane]), s1 = f16_to_f32(svh[lane + 64]);
+    float v0 = 0.0f, v1 = 0.0f;
+    for (u32 z0 = 0; z0 < zs; z0 += 4) {
+        float a[4][2];   // four partials' loads in flight together
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float* p = part + ((u64) j * zs + min(z0 + q, zs - 1)) * out_f + ob * 128;
+            a[q][0] = p[lane];
+            a[q][1] = p[lane + 64];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (z0 + q < zs) {
+                v0 += a[q][0];
+                v1 += a[q][1];
+            }
+    }
+    wht128_wave(v0, v1, lane);
+    float* o = y + (u64) j * ys + ob * 128;
+    o[lane] = v0 * s0;
+    o[lane + 64] = v1 * s1;
+}
+#define EXL3_COLS_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) matvec_grouped_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 8, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) matvec_grouped_t4_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 4, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) matvec_grouped_t2_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 2, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) matvec_grouped_w_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 8, 2>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) matvec_grouped_t4w_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 4, 2>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) matvec_grouped_t2w_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 2, 2>(w, x, xs, part, in_f, out_f, m); \
+    }
+#define EXL3_COLS_HALF_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) matvec_grouped_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 8, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) matvec_grouped_t4_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 4, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) matvec_grouped_t2_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 2, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) matvec_grouped_w_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 8, 2>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) matvec_grouped_t4w_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 4, 2>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) matvec_grouped_t2w_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, true, 2, 2>(w, x, xs, part, in_f, out_f, m); \
+    }
+EXL3_COLS_ENTRIES(1)
+EXL3_COLS_ENTRIES(2)
+EXL3_COLS_ENTRIES(3)
+EXL3_COLS_ENTRIES(4)
+EXL3_COLS_ENTRIES(5)
+EXL3_COLS_ENTRIES(6)
+EXL3_COLS_ENTRIES(7)
+EXL3_COLS_ENTRIES(8)
+EXL3_COLS_HALF_ENTRIES(1)
+EXL3_COLS_HALF_ENTRIES(2)
+EXL3_COLS_HALF_ENTRIES(3)
 
 // ------------------------------------------------------------------------------------- the EXL3 head on the matrix cores
 // The lm_head of an EXL3 checkpoint (in = hidden, out = vocabulary; kernels/exl3.cu:349-461, 610-625: exl3_rotate_rows_f32 and
@@ -1495,20 +1452,6 @@ EXL3_HEAD_ENTRIES(5)
 EXL3_HEAD_ENTRIES(6)
 EXL3_HEAD_ENTRIES(7)
 EXL3_HEAD_ENTRIES(8)
-
-// The one-matrix plan of a plain y_j = W x_j product for m <= 8 inputs: groups of 4 inputs, input row = output row = j.
-// grid 1, block 64.
-extern "C" __global__ void __launch_bounds__(64) cols_plan(u64* wtab, u32* gtab, u64 w, u32 m) {
-    const u32 g = threadIdx.x;
-    if (g * 4 >= m) return;
-    wtab[g] = w;
-    u32* r = gtab + 17 * g;
-    r[0] = min(4u, m - 4 * g);
-    for (u32 j = 0; j < 8; j++) {
-        r[1 + j] = 4 * g + (j < 4 ? j : 0);
-        r[9 + j] = 4 * g + (j < 4 ? j : 0);
-    }
-}
 
 // ------------------------------------------------------------------------ the prefill chunk of an EXL3 layer (matrix cores)
 // A chunk's tokens grouped by expert (prefill_group in kernels/prefill.hip: runs of up to XPF_TOK(K) (token, rank) pairs of
