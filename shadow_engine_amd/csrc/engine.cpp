@@ -158,10 +158,8 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         return launch(kn.c_str(), (uint32_t) ((rows + (uint64_t) d.pass * np - 1) / ((uint64_t) d.pass * np)), 1, 1, d.block, 0, stream, a);
     }
     if (cols % f.qk) return fail("matvec_cols: columns are not whole blocks");
-    // fewer rows a workgroup where the launch would otherwise have under about 512 workgroups (two a CU)
-    const uint32_t rpb = rows_per_block(f, (uint32_t) cols, (uint32_t) std::max<uint64_t>(1, rows * ((m + 3) / 4) / 512));
-    if (rpb == 0 || (x & 15) || xs % 4) {
-        // any shape: the one-weight-at-a-time kernel, an input at a time
+    if ((x & 15) || xs % 4) {
+        // any alignment: the one-weight-at-a-time kernel, an input at a time
         const std::string kn = "matvec_" + tag;
         for (uint32_t j = 0; j < m; j++) {
             const sz_arg a[] = {P(w), P(x + (uint64_t) j * xs * 4), P(y + (uint64_t) j * ys * 4), U32((uint32_t) rows), U32((uint32_t) cols)};
@@ -169,10 +167,11 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         }
         return 0;
     }
-    const uint32_t rb = (uint32_t) cols / f.qk * f.bb;
-    const std::string kn = "matvec_cols_" + tag;
-    const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m), U32(rpb)};
-    return launch(kn.c_str(), ((uint32_t) rows + rpb - 1) / rpb, (m + 3) / 4, 1, 256, rpb * rb + 32, stream, a);
+    // waves that share a row: as many as it has 256-column chunks, up to the workgroup's four
+    const uint32_t chunks = (uint32_t) ((cols + 255) / 256), ks = chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
+    const std::string kn = std::string("matvec_cols_") + (m > 4 ? "w_" : "") + tag;
+    const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m), U32(ks)};
+    return launch(kn.c_str(), (uint32_t) ((rows + 128 / ks - 1) / (128 / ks)), 1, 1, 256, 0, stream, a);
 }
 
 }   // namespace sz

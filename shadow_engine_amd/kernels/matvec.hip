@@ -397,32 +397,6 @@ __device__ __forceinline__ void rows_dispatch(const u8* w, u32 rows, u32 cols, u
     }
 }
 
-// y_j = W x_j for inputs j = 4 blockIdx.y .. +4 (< m): x rows xs floats apart, y rows ys apart (matvec.cu:677-756).
-// grid = (ceil(rows / rpb), ceil(m / 4)), block 256, dynamic LDS = rpb * row bytes + 32.
-template <class F>
-__device__ __forceinline__ void cols_kernel(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m, u32 rpb) {
-    const u32 j0 = blockIdx.y * 4;
-    const u32 n = min(4u, m - j0);
-    const float* xp[4];
-    float* yp[4];
-    for (u32 j = 0; j < 4; j++) {
-        const u32 jj = j0 + (j < n ? j : 0);
-        xp[j] = x + (u64) jj * xs;
-        yp[j] = j < n ? y + (u64) jj * ys : nullptr;
-    }
-    rows_dispatch<F>(w, rows, cols, rpb, n, xp, yp, nullptr, NoAfter());
-}
-
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_q8_0(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows,
-                                                                   u32 cols, u32 m, u32 rpb) {
-    cols_kernel<Q80>(w, x, xs, y, ys, rows, cols, m, rpb);
-}
-
-extern "C" __global__ void __launch_bounds__(256) matvec_cols_iq3_s(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows,
-                                                                    u32 cols, u32 m, u32 rpb) {
-    cols_kernel<IQ3S>(w, x, xs, y, ys, rows, cols, m, rpb);
-}
-
 // Group g = blockIdx.y: matrix wtab[g] (device address), record gtab[17 g] = {n <= 4 (0: unused slot), xi[8], yi[8]};
 // y[yi[j]] = W x[xi[j]] (matvec.cu:1576-1677).  grid = (ceil(rows / rpb), groups).
 template <class F>

@@ -1,0 +1,40 @@
+"""The kernels' edges on the GPU: sizes at the ends of tiles, chunks and dispatch ranges, each against the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import shadow_engine_amd as sz
+from shadow_engine_amd import synth
+from test_gpu_path import REL_L2, bits, dev, gguf_bound, gpu  # noqa: F401 (gpu: the fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ty,rows,cols", [(sz.Q8_0, 1, 32), (sz.Q8_0, 33, 288), (sz.Q8_0, 127, 736), (sz.Q8_0, 65, 1056), (sz.Q8_0, 8201, 256),
+                                          (sz.IQ3_S, 1, 256), (sz.IQ3_S, 129, 512), (sz.IQ3_S, 47, 1280)])
+@pytest.mark.parametrize("m", [1, 4, 5, 8])
+def test_gguf_products_at_the_edges_of_tiles_and_chunks(gpu, ty, rows, cols, m):  # noqa: F811
+    """Row counts around the 16-row tiles and 32-row groups, one to more than four 256-column chunks (one, two and four waves a
+    row) with a short last one, both widths of the input tile; inputs of very different sizes in one chunk; values past the
+    last row stay untouched."""
+    rng = np.random.default_rng(rows * 13 + cols + m)
+    w = synth.q8_0_matrix(rng, rows, cols) if ty == sz.Q8_0 else synth.iq3_s_matrix(rng, rows, cols)
+    x = rng.normal(size=(m, cols)).astype(np.float32) * np.exp2(rng.integers(-12, 12, size=(m, cols))).astype(np.float32)
+    ys = rows + 5
+    dw, dx = dev(gpu, w), dev(gpu, x)
+    y = gpu.full((m, ys), 7.5, dtype=gpu.float32, device="cuda")
+    sz.matvec_cols(ty, dw.data_ptr(), cols, rows, dx.data_ptr(), cols, y.data_ptr(), ys, m)
+    gpu.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.all(got[:, rows:] == 7.5)
+    for j in range(m):
+        want = O.matvec(ty, cols, rows, w, x[j])
+        assert np.all(np.abs(got[j, :rows] - want) <= gguf_bound(ty, cols, rows, w, x[j]))
+        assert np.linalg.norm(got[j, :rows] - want) <= REL_L2 * np.linalg.norm(want)
+    # inputs that do not start on 16 bytes take the one-weight-at-a-time kernel
+    d4 = gpu.empty(m * cols + 1, dtype=gpu.float32, device="cuda")
+    d4[1:] = dx.flatten()
+    sz.matvec_cols(ty, dw.data_ptr(), cols, rows, d4.data_ptr() + 4, cols, y.data_ptr(), ys, m)
+    gpu.cuda.synchronize()
+    for j in range(m):
+        assert np.all(np.abs(y[j, :rows].cpu().numpy() - got[j, :rows]) <= 2 * gguf_bound(ty, cols, rows, w, x[j]))
