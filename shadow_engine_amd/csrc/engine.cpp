@@ -167,11 +167,14 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         }
         return 0;
     }
-    // waves that share a row: as many as it has 256-column chunks, up to the workgroup's four
-    const uint32_t chunks = (uint32_t) ((cols + 255) / 256), ks = chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
+    // a wave a 256-column chunk, the same number of chunks a wave as far as they divide, up to 16 waves; as many workgroups as
+    // the chip holds at a time (16 waves a CU), each with up to four tiles of 16 rows, which share the work on the inputs
+    const uint32_t chunks = (uint32_t) ((cols + 255) / 256), each = (chunks + 15) / 16, waves = (chunks + each - 1) / each;
+    const uint32_t n16 = (uint32_t) ((rows + 15) / 16), slots = 256 * (16 / waves), rounds = (n16 + 4 * slots - 1) / (4 * slots);
+    const uint32_t ng = m > 4 ? 2 : 1;
     const std::string kn = std::string("matvec_cols_") + (m > 4 ? "w_" : "") + tag;
-    const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m), U32(ks)};
-    return launch(kn.c_str(), (uint32_t) ((rows + 128 / ks - 1) / (128 / ks)), 1, 1, 256, 0, stream, a);
+    const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m)};
+    return launch(kn.c_str(), std::min(n16, rounds * slots), 1, 1, 64 * waves, waves * (1584 * 4 + 4 * ng * 64 * 4), stream, a);
 }
 
 }   // namespace sz
@@ -257,7 +260,12 @@ int32_t sz_matvec(sz_backend* b, int32_t ty, uint64_t cols, uint64_t rows, const
     if (hip_check(hip().hipMemcpyHtoDAsync((void*) b->x.ptr, b->hx.ptr, cols * 4, nullptr), "hipMemcpyHtoDAsync")) return 1;
     const uint64_t sb = cols_scratch_bytes(f, cols, rows, 1);
     if (sb && b->scratch.need(sb)) return 1;
-    if (matvec_cols_dev(ty, wp, cols, rows, b->x.ptr, (uint32_t) cols, (uint64_t) b->hy.ptr, (uint32_t) rows, 1, b->scratch.ptr, b->scratch.bytes, 0)) return 1;
+    // fewer rows a workgroup where the launch would otherwise have under about 512 workgroups (two a CU)
+    const uint32_t rpb = rows_per_block(f, (uint32_t) cols, (uint32_t) std::max<uint64_t>(1, rows / 512));
+    if (rpb) {
+        const sz_arg a[] = {P(wp), P(b->x.ptr), P((uint64_t) b->hy.ptr), U32((uint32_t) rows), U32((uint32_t) cols), U32(rpb)};
+        if (launch(("matvec_one_" + tag).c_str(), ((uint32_t) rows + rpb - 1) / rpb, 1, 1, 256, rpb * (uint32_t) (cols / f.qk * f.bb) + 32, 0, a)) return 1;
+    } else if (matvec_cols_dev(ty, wp, cols, rows, b->x.ptr, (uint32_t) cols, (uint64_t) b->hy.ptr, (uint32_t) rows, 1, b->scratch.ptr, b->scratch.bytes, 0)) return 1;
     if (sz_stream_synchronize(0)) return 1;   // synchronous, as the reference's backend: waits for the kernels
     std::memcpy(y, b->hy.ptr, rows * 4);
     return 0;

@@ -10,13 +10,13 @@ from test_gpu_path import REL_L2, bits, dev, gguf_bound, gpu  # noqa: F401 (gpu:
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ty,rows,cols", [(sz.Q8_0, 1, 32), (sz.Q8_0, 33, 288), (sz.Q8_0, 127, 736), (sz.Q8_0, 65, 1056), (sz.Q8_0, 8201, 256),
-                                          (sz.IQ3_S, 1, 256), (sz.IQ3_S, 129, 512), (sz.IQ3_S, 47, 1280)])
+@pytest.mark.parametrize("ty,rows,cols", [(sz.Q8_0, 1, 32), (sz.Q8_0, 33, 288), (sz.Q8_0, 127, 736), (sz.Q8_0, 65, 1056), (sz.Q8_0, 8201, 256), (sz.Q8_0, 70, 4384),
+                                          (sz.IQ3_S, 1, 256), (sz.IQ3_S, 129, 512), (sz.IQ3_S, 47, 1280), (sz.IQ3_S, 4200, 4352)])
 @pytest.mark.parametrize("m", [1, 4, 5, 8])
 def test_gguf_products_at_the_edges_of_tiles_and_chunks(gpu, ty, rows, cols, m):  # noqa: F811
-    """Row counts around the 16-row tiles and 32-row groups, one to more than four 256-column chunks (one, two and four waves a
-    row) with a short last one, both widths of the input tile; inputs of very different sizes in one chunk; values past the
-    last row stay untouched."""
+    """Row counts around the 16-row tiles and past one tile a workgroup, rows shorter than a 256-column chunk, of one to more than
+    sixteen chunks (two a wave), with a short last one, both widths of the input tile; inputs of very different sizes in one
+    chunk; values past the last row stay untouched."""
     rng = np.random.default_rng(rows * 13 + cols + m)
     w = synth.q8_0_matrix(rng, rows, cols) if ty == sz.Q8_0 else synth.iq3_s_matrix(rng, rows, cols)
     x = rng.normal(size=(m, cols)).astype(np.float32) * np.exp2(rng.integers(-12, 12, size=(m, cols))).astype(np.float32)
