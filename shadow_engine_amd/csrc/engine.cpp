@@ -414,6 +414,17 @@ int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32
     const bool one = p1 - p0 == 1;   // a single layer's addresses go along as kernel arguments, not through the table
     auto table = [&](uint32_t p) { return one ? 0 : s->vtab_dev.ptr + (uint64_t) p * sizeof(VerifyLayer); };
     const VerifyLayer& V = s->vtab[p0];
+    if (one) {
+        // its part of the buffers, wherever the caller's begin: without a table the kernels take it to be layer `base`, and without a
+        // plan (below) they leave ids and weights at `plans` itself
+        const uint64_t l = V.layer - base;
+        u += l * m * c.hidden * 4;
+        rl += l * m * c.n_expert * 4;
+        sgl += l * m * 4;
+        y += l * m * c.hidden * 4;
+        plans += l * s->plan_stride;
+        base = V.layer;
+    }
     // Layer by layer, tokens that share an expert are worth a launch that finds them only where they are many: about 6 us and
     // a boundary, against the decode of a fifth of the pairs (measured at 4 rows of top-10 of 512, where they are one in twenty:
     // 46 us a layer with the plan, 41 without).  A round's plans are one launch for all layers.

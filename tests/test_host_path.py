@@ -1,0 +1,121 @@
+"""The library's host side without a GPU: which launches a call makes, with which addresses, and what a failure leaves behind.
+The library binds its HIP runtime at run time, so a child process binds hip_stub.cpp instead, which runs nothing and reports
+every launch."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = '''
+import ctypes as C, os
+import numpy as np
+import shadow_engine_amd as sz
+from shadow_engine_amd import synth
+stub = C.CDLL(os.environ["SHADOWZERO_HIP_LIB"])
+stub.stub_fail_allocations_over.argtypes = [C.c_size_t]
+stub.stub_fail_copy_after.argtypes = [C.c_long]
+sz.init(0)
+PARAMS = {n: k for n, _, k in sz.kernels()}   # kinds: 0, 1 pointers, 2 u32, 3 i32, 4 u64, 5 f32
+launches = []
+@C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_uint), C.POINTER(C.c_void_p))
+def on_launch(name, shape, params):
+    name = name.decode()
+    ty = {0: C.c_uint64, 1: C.c_uint64, 2: C.c_uint32, 3: C.c_int32, 4: C.c_uint64, 5: C.c_float}
+    launches.append((name, tuple(shape[:7]), [ty[k].from_address(params[i]).value for i, k in enumerate(PARAMS[name])]))
+stub.stub_on_launch(on_launch)
+def taken():
+    out = list(launches)
+    launches.clear()
+    return out
+def address(n):   # host memory with room to look like a device buffer
+    keep.append(np.zeros(n + 256, np.uint8))
+    return (keep[-1].ctypes.data + 255) // 256 * 256
+keep = []
+'''
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = tmp_path_factory.mktemp("stub") / "libhipstub.so"
+    subprocess.run(["g++", "-O1", "-fPIC", "-shared", "-o", str(so), os.path.join(HERE, "hip_stub.cpp")], check=True)
+
+    def run(body):
+        env = dict(os.environ, SHADOWZERO_HIP_LIB=str(so), PYTHONPATH=ROOT)
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body], env=env, capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+MIXED = '''
+class Layer(C.Structure):
+    _fields_ = [("experts", C.c_uint64), ("stride", C.c_uint64), ("shared", C.c_uint64), ("part", C.c_uint32), ("layer", C.c_uint32)]
+H, FF, NE, K, M, L, V = 512, 256, 32, 4, 3, 4, 1024
+def seen_by(name, shape, a):
+    """The layers one of an EXL3 layer's launches works on, as (experts, logits or gate logits, inputs or outputs, plan) each."""
+    out = []
+    per = {"verify_plan_exl3": 1, "verify_combine_exl3": 1}.get(name, (H + 511) // 512 if "gate_up" in name else (FF + 511) // 512)
+    if name == "verify_plan_exl3":
+        rl, plans, ps, ioff, table, shared, base = a[:7]
+        first, second, e = rl, None, None
+    elif name == "verify_combine_exl3":
+        dn, table, e, stride, shared, part, base, plans, ps, first, second = a[:11]
+    else:
+        rl, table, e, stride, shared, part, base, plans, weights, ps, ioff, second = a[:12]
+        assert weights == plans
+        first = rl
+    n = shape[0] if name == "verify_plan_exl3" else shape[2] // per
+    for i in range(n):
+        lay = Layer.from_address(table + 32 * i) if table else Layer(e or 0, 0, 0, 0, base)
+        l = lay.layer - base
+        wide = 1 if name == "verify_combine_exl3" else NE
+        # without a plan (ioff 0) the ids and weights go to the very place that is given
+        assert "combine" in name or ioff or l == 0
+        out.append((lay.experts or None, first + l * M * wide * 4, None if "down" in name or second is None else second + l * M * H * 4, plans + l * ps))
+    return out
+def check(exl3):
+    s = sz.Session(H, FF, NE, K, L, V, 8)
+    buf = address(1 << 20)                       # nothing reads it
+    base = {l: buf + 4096 * l for l in range(L)}
+    for l in range(L):
+        ty = sz.EXL3(2 + l % 2) if l in exl3 else sz.Q8_0
+        s.set_layer(l, ty, base[l], 1 << 20, ty, base[l] + 64)
+    s.set_head(sz.Q8_0, address(1024))
+    u, rl, sgl, y, hu, dr, out = (address(1 << 16) for _ in range(7))
+    taken()
+    for replay in range(2):
+        s.verify_round(M, u, rl, sgl, y, hu, dr, out, 16)
+        got = taken()
+        if replay:
+            assert not got                       # a graph's replay
+            break
+        plans = {}
+        for name in ("verify_plan_exl3", "verify_gate_up_", "verify_down_", "verify_combine_exl3"):
+            done = [x for g in got if g[0].startswith(name) and "q8_0" not in g[0] for x in seen_by(*g)]
+            if name == "verify_plan_exl3" and len(exl3) == 1:
+                continue                         # a lone layer may do without
+            per_layer = {}
+            for experts, first, second, plan in done:
+                at = (first - (sgl if "combine" in name else rl)) // (M * (1 if "combine" in name else NE) * 4)
+                assert at not in per_layer
+                per_layer[at] = plan
+                assert experts in (None, base[at])
+                if second is not None:
+                    assert second == (y if "combine" in name else u) + at * M * H * 4
+                assert plans.setdefault(at, plan) == plan
+            assert sorted(per_layer) == sorted(exl3), (name, per_layer, exl3)
+        assert len(set(plans.values())) == len(exl3)
+        if L - 1 in exl3:
+            assert sz.lib().sz_session_buffer(s._h, 0) == plans[L - 1]
+    return s, plans, (u, rl, sgl, y, hu, dr, out)
+'''
+
+
+@pytest.mark.parametrize("exl3", [[0], [1], [3], [1, 2], [0, 3], [0, 1, 2, 3]])
+def test_a_round_over_mixed_formats_gives_every_exl3_layer_its_own_buffers(stub, exl3):
+    """A round's launches for its EXL3 layers read and write these layers' inputs, plans and outputs, wherever the layers lie among
+    GGUF ones and however many there are."""
+    stub(MIXED + f"check({exl3})\n")

@@ -5,7 +5,7 @@ import pytest
 import oracle_lib as O
 import shadow_engine_amd as sz
 from shadow_engine_amd import synth
-from test_gpu_path import REL_L2, bits, dev, gguf_bound, gpu  # noqa: F401 (gpu: the fixture)
+from test_gpu_path import REL_L2, bits, build_layer, dev, gguf_bound, gpu, oracle_layer, rel_l2  # noqa: F401 (gpu: the fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,42 @@ def test_gguf_products_at_the_edges_of_tiles_and_chunks(gpu, ty, rows, cols, m):
     gpu.cuda.synchronize()
     for j in range(m):
         assert np.all(np.abs(y[j, :rows].cpu().numpy() - got[j, :rows]) <= 2 * gguf_bound(ty, cols, rows, w, x[j]))
+
+
+@pytest.mark.parametrize("types,m", [((3, 0, 0), 4), ((0, 3, 0), 4), ((0, 0, 3), 1), ((0, 3, 0), 8), ((2, 0, 4, 0, 3), 4)])
+def test_a_round_over_gguf_and_exl3_layers(gpu, types, m):  # noqa: F811
+    """One or several EXL3 layers (the numbers: bits a weight) at any place among Q8_0 ones: a round gives the bits of the
+    layer-by-layer calls, which the oracle checks, and the last layer's routing; so do its graph's replays."""
+    rng = np.random.default_rng(sum(types) + m)
+    hidden, ff, ne, k, vocab, L = 512, 256, 24, 3, 1024, len(types)
+    s = sz.Session(hidden, ff, ne, k, L, vocab, 8)
+    keep, want = [], []
+    u, rl = rng.normal(size=(L, m, hidden)).astype(np.float32), rng.normal(size=(L, m, ne)).astype(np.float32)
+    sgl, hu = rng.normal(size=(L, m)).astype(np.float32), rng.normal(size=(m, hidden)).astype(np.float32)
+    for l, kb in enumerate(types):
+        ty = sz.EXL3(kb) if kb else sz.Q8_0
+        dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, True)
+        keep.append(dbuf)
+        s.set_layer(l, ty, dbuf.data_ptr(), stride, ty, dbuf.data_ptr() + ne * stride)
+        want.append(oracle_layer(ty, hidden, ff, k, blobs, sh, rl[l], sgl[l], u[l]))
+    dhead = dev(gpu, synth.q8_0_matrix(rng, vocab, hidden))
+    s.set_head(sz.Q8_0, dhead.data_ptr())
+    du, drl, dsgl, dhu = dev(gpu, u), dev(gpu, rl), dev(gpu, sgl), dev(gpu, hu)
+    drafts, out = gpu.zeros(8, dtype=gpu.int32, device="cuda"), gpu.zeros(10, dtype=gpu.int32, device="cuda")
+    one = gpu.zeros((L, m, hidden), dtype=gpu.float32, device="cuda")
+    for l in range(L):
+        s.moe_layer_verify(l, m, du[l].data_ptr(), drl[l].data_ptr(), dsgl[l].data_ptr(), one[l].data_ptr())
+    gpu.cuda.synchronize()
+    one = one.cpu().numpy()
+    for l in range(L):
+        for j in range(m):
+            assert rel_l2(one[l, j], want[l][0][j]) <= REL_L2
+    stream, y = sz.Stream(), gpu.zeros((L, m, hidden), dtype=gpu.float32, device="cuda")
+    for replay in range(3):
+        y.zero_()
+        gpu.cuda.synchronize()
+        s.verify_round(m, du.data_ptr(), drl.data_ptr(), dsgl.data_ptr(), y.data_ptr(), dhu.data_ptr(), drafts.data_ptr(), out.data_ptr(), stream.handle)
+        stream.synchronize()
+        assert np.array_equal(bits(y.cpu().numpy()), bits(one)), f"replay {replay}"
+        idx, _ = s.last_route(m, stream.handle)
+        assert np.array_equal(idx, want[-1][1])
