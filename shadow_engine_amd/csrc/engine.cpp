@@ -337,6 +337,12 @@ struct SzGraphKey {
     bool operator<(const SzGraphKey& o) const { return std::memcmp(v, o.v, sizeof v) < 0; }
 };
 
+// A captured round: its graph, and where its last layer leaves its routing (last_plan, last_fused below).
+struct SzRoundGraph {
+    uint64_t exec, plan;
+    bool fused;
+};
+
 struct sz_session {
     sz_session_config cfg{};
     std::vector<SzLayer> layers;
@@ -362,7 +368,7 @@ struct sz_session {
     void* top_host = nullptr;  // pinned host memory the top-64 merge writes to directly (8 rows of 128 words): no copy back
     bool last_fused = false;   // the last layer call left its routing in the fused layout [tidx | w | cnt]
     uint64_t last_plan = 0;    // the plan the last layer call left its routing in
-    std::map<SzGraphKey, uint64_t> graphs;
+    std::map<SzGraphKey, SzRoundGraph> graphs;
     // plan offsets for the largest batch
     uint32_t GT_max = 0;
     bool use_graph = true;
@@ -777,7 +783,7 @@ sz_session* sz_session_new(const sz_session_config* cfg) {
 void sz_session_free(sz_session* s) {
     if (!s) return;
     if (s->top_host) hip().hipHostFree(s->top_host);
-    for (auto& g : s->graphs) sz_graph_destroy(g.second);
+    for (auto& g : s->graphs) sz_graph_destroy(g.second.exec);
     delete s;
 }
 
@@ -845,7 +851,7 @@ int32_t sz_session_set_layer_spaced(sz_session* s, uint32_t l, int32_t ty, uint6
             return 1;
     }
     if (verify_table(s)) return 1;
-    for (auto& g : s->graphs) sz_graph_destroy(g.second);   // captured address tables may be stale
+    for (auto& g : s->graphs) sz_graph_destroy(g.second.exec);   // captured address tables may be stale
     s->graphs.clear();
     return 0;
 }
@@ -886,7 +892,7 @@ int32_t sz_session_set_router(sz_session* s, uint32_t l, int32_t rty, uint64_t r
     L.router_type = rty;
     L.gate = gw;
     L.gate_type = gty;
-    for (auto& g : s->graphs) sz_graph_destroy(g.second);
+    for (auto& g : s->graphs) sz_graph_destroy(g.second.exec);
     s->graphs.clear();
     return 0;
 }
@@ -938,7 +944,7 @@ int32_t sz_session_set_head(sz_session* s, int32_t ty, uint64_t w) {
     s->head_type = ty;
     s->head_w = w;
     s->hp.k_blk = 0;   // a screen belongs to the head it was built from
-    for (auto& g : s->graphs) sz_graph_destroy(g.second);
+    for (auto& g : s->graphs) sz_graph_destroy(g.second.exec);
     s->graphs.clear();
     return 0;
 }
@@ -1141,9 +1147,11 @@ int32_t sz_verify_round(sz_session* s, uint32_t m, uint64_t u, uint64_t rl, uint
             return fail(err);
         }
         if (e) return 1;
-        it = s->graphs.emplace(key, exec).first;
+        it = s->graphs.emplace(key, SzRoundGraph{exec, s->last_plan, s->last_fused}).first;
     }
-    return sz_graph_launch(it->second, stream);
+    s->last_plan = it->second.plan;
+    s->last_fused = it->second.fused;
+    return sz_graph_launch(it->second.exec, stream);
 }
 
 int32_t sz_quantize_act(uint64_t x, uint64_t n, uint64_t q, uint64_t d, uint64_t stream) {

@@ -119,3 +119,17 @@ def test_a_round_over_mixed_formats_gives_every_exl3_layer_its_own_buffers(stub,
     """A round's launches for its EXL3 layers read and write these layers' inputs, plans and outputs, wherever the layers lie among
     GGUF ones and however many there are."""
     stub(MIXED + f"check({exl3})\n")
+
+
+def test_the_last_routing_after_a_replayed_round_is_the_rounds(stub):
+    """Between a round's capture and its replay a single layer's call leaves its own routing; after the replay the last routing is
+    the round's last layer's again."""
+    stub(MIXED + '''
+s, plans, bufs = check([0, 1, 2, 3])
+u, rl, sgl, y = bufs[:4]
+s.moe_layer_verify(0, M, u, rl, sgl, y, 16)
+assert sz.lib().sz_session_buffer(s._h, 0) != plans[L - 1]
+taken()
+s.verify_round(M, *bufs, 16)
+assert not taken() and sz.lib().sz_session_buffer(s._h, 0) == plans[L - 1]
+''')
