@@ -787,7 +787,8 @@ void sz_session_free(sz_session* s) {
     delete s;
 }
 
-// The table of the EXL3 layers that are set, rebuilt and copied to the device.
+// The table of the EXL3 layers that are set, rebuilt and copied to the device.  (After a failed copy the caller unsets its layer:
+// rounds, which alone read the device's copy, are refused until a later call has made it whole.)
 static int verify_table(sz_session* s) {
     std::vector<uint32_t> order;
     for (uint32_t l = 0; l < s->layers.size(); l++)
@@ -834,14 +835,7 @@ int32_t sz_session_set_layer_spaced(sz_session* s, uint32_t l, int32_t ty, uint6
         tab[3ull * c.n_expert + 1] = shared + sgu;
         tab[3ull * c.n_expert + 2] = shared + 2 * sgu;
     }
-    if (L.eaddr.need(tab.size() * 8) || sz_upload(L.eaddr.ptr, tab.data(), tab.size() * 8)) return 1;
-    L.type = ty;
-    L.shared_type = shared_type;
-    L.experts = experts;
-    L.stride = stride;
-    L.shared = shared;
-    L.gap = gap;
-    L.set = true;
+    // the allocations first: one that fails leaves the layer as it was
     if (f.exl3) {
         // the launches' buffers hold as many layers as take 256 MiB (what the memory-side cache holds), at least one
         const uint64_t per = verify_part_bytes(c, c.max_rows) + verify_dn_bytes(c, c.max_rows);
@@ -850,7 +844,21 @@ int32_t sz_session_set_layer_spaced(sz_session* s, uint32_t l, int32_t ty, uint6
             s->part.need(s->vchunk * verify_part_bytes(c, c.max_rows)) || s->dn.need(s->vchunk * verify_dn_bytes(c, c.max_rows)))
             return 1;
     }
-    if (verify_table(s)) return 1;
+    if (L.eaddr.need(tab.size() * 8)) return 1;
+    // then the copies: the layer is unset while one of its tables may be half written
+    L.set = false;
+    if (sz_upload(L.eaddr.ptr, tab.data(), tab.size() * 8)) return 1;
+    L.type = ty;
+    L.shared_type = shared_type;
+    L.experts = experts;
+    L.stride = stride;
+    L.shared = shared;
+    L.gap = gap;
+    L.set = true;
+    if (verify_table(s)) {
+        L.set = false;
+        return 1;
+    }
     for (auto& g : s->graphs) sz_graph_destroy(g.second.exec);   // captured address tables may be stale
     s->graphs.clear();
     return 0;

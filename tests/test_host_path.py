@@ -133,3 +133,50 @@ taken()
 s.verify_round(M, *bufs, 16)
 assert not taken() and sz.lib().sz_session_buffer(s._h, 0) == plans[L - 1]
 ''')
+
+
+def test_a_layer_that_could_not_be_set_is_not_used(stub):
+    """A failed allocation leaves a layer as it was, a failed copy leaves it unset; both are refused by the calls that would run it,
+    and setting the layer again mends it."""
+    stub(MIXED + '''
+s = sz.Session(H, FF, NE, K, L, V, 8)
+buf = address(1 << 20)
+s.set_head(sz.Q8_0, address(1024))
+u, rl, sgl, y, hu, dr, out = (address(1 << 16) for _ in range(7))
+def fails(what, f):
+    try:
+        f()
+    except sz.SzError as e:
+        assert what in str(e), e
+    else:
+        raise AssertionError("not refused")
+set_layer = lambda l, ty: s.set_layer(l, ty, buf + 4096 * l, 1 << 20, ty, buf + 64)
+layer = lambda l: s.moe_layer_verify(l, M, u, rl, sgl, y, 16)
+def launched(l, kind):
+    taken()
+    layer(l)
+    got = taken()
+    assert got and all(kind in g[0] or g[0].startswith("moe_combine") or g[0].startswith("verify_combine") for g in got), got
+set_layer(0, sz.Q8_0)
+stub.stub_fail_allocations_over(1 << 16)     # the EXL3 launches' buffers
+fails("hipMalloc", lambda: set_layer(0, sz.EXL3(3)))
+fails("hipMalloc", lambda: set_layer(1, sz.EXL3(3)))
+launched(0, "q8_0")
+fails("no experts set", lambda: layer(1))
+stub.stub_fail_allocations_over(1 << 62)
+for n in (0, 1):                             # the address table's copy, the table of EXL3 layers
+    stub.stub_fail_copy_after(n)
+    fails("hipMemcpyHtoD", lambda: set_layer(1, sz.EXL3(3)))
+    stub.stub_fail_copy_after(-1)
+    fails("no experts set", lambda: layer(1))
+for l, ty in enumerate((sz.EXL3(4), sz.EXL3(3), sz.Q8_0, sz.EXL3(2))):
+    set_layer(l, ty)
+    launched(l, "q8_0" if ty == sz.Q8_0 else "exl3")
+stub.stub_fail_copy_after(1)
+fails("hipMemcpyHtoD", lambda: set_layer(1, sz.EXL3(2)))
+stub.stub_fail_copy_after(-1)
+fails("layer 1 has no experts set", lambda: s.verify_round(M, u, rl, sgl, y, hu, dr, out, 16))
+launched(3, "exl3_2")
+set_layer(1, sz.EXL3(2))
+s.verify_round(M, u, rl, sgl, y, hu, dr, out, 16)
+''')
