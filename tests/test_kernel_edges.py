@@ -77,3 +77,48 @@ def test_a_round_over_gguf_and_exl3_layers(gpu, types, m):  # noqa: F811
         assert np.array_equal(bits(y.cpu().numpy()), bits(one)), f"replay {replay}"
         idx, _ = s.last_route(m, stream.handle)
         assert np.array_equal(idx, want[-1][1])
+
+
+def products(gpu, ty, rows, cols, w, x):  # noqa: F811
+    """W x_j for the rows of x, through matvec_cols."""
+    m = x.shape[0]
+    nsb = sz.matvec_cols_scratch(ty, cols, rows, m)
+    dw, dx = dev(gpu, w), dev(gpu, x)
+    scratch = gpu.empty(max(nsb, 16), dtype=gpu.uint8, device="cuda")
+    y = gpu.zeros((m, rows), dtype=gpu.float32, device="cuda")
+    sz.matvec_cols(ty, dw.data_ptr(), cols, rows, dx.data_ptr(), cols, y.data_ptr(), rows, m, scratch.data_ptr(), nsb)
+    gpu.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+def set_scales(ty, w, value):
+    """The block scales (of an EXL3 blob of 512 inputs the output scales of 128) of w as one f16 value."""
+    if ty >= 1000:
+        w[1024:1024 + 256] = np.full(128, value, np.float16).view(np.uint8)
+    else:
+        w.reshape(-1, 34 if ty == sz.Q8_0 else 110)[:, :2] = np.array([value], np.float16).view(np.uint8)
+    return w
+
+
+@pytest.mark.parametrize("ty", [sz.Q8_0, sz.IQ3_S, sz.EXL3(3)])
+@pytest.mark.parametrize("m", [1, 3, 8])
+def test_products_of_subnormal_inputs(gpu, ty, m):  # noqa: F811
+    """Inputs that are all subnormal, down to single units of 2^-149, are not lost.  Against f64 sums; the GGUF products of such
+    inputs are exact up to f32 sums, an EXL3 one's transform rounds to multiples of 2^-149: nine additions and a scale for
+    values of about 2^-130, under 2^-15 together, and as much again for its output side."""
+    rng = np.random.default_rng(m)
+    rows, cols = 128, 512
+    w = synth.exl3_blob(rng, cols, rows, 3) if ty >= 1000 else synth.q8_0_matrix(rng, rows, cols) if ty == sz.Q8_0 else synth.iq3_s_matrix(rng, rows, cols)
+    set_scales(ty, w, 16384.0)
+    x = (rng.normal(size=(m, cols)) * 2.0 ** -130).astype(np.float32)
+    if m > 2:
+        x[2] = rng.integers(-3, 4, cols) * 2.0 ** -149 if ty < 1000 else 0.0
+    assert np.abs(x).max() < 2.0 ** -126
+    got = products(gpu, ty, rows, cols, w, x).astype(np.float64)
+    for j in range(m):
+        if ty >= 1000:
+            want = O.exl3_matvec(cols, rows, 3, w, (x[j].astype(np.float64) * 2.0 ** 60).astype(np.float32)).astype(np.float64) * 2.0 ** -60
+            assert np.linalg.norm(got[j] - want) <= 2.0 ** -14 * np.linalg.norm(want)
+        else:
+            want = O.dequantize(ty, w).reshape(rows, cols).astype(np.float64) @ x[j].astype(np.float64)
+            assert np.linalg.norm(want) > 2.0 ** -126 and np.linalg.norm(got[j] - want) <= 1e-5 * np.linalg.norm(want)
