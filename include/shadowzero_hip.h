@@ -183,8 +183,8 @@ uint32_t sz_exl3_head_lds_bytes(int32_t type, uint32_t hidden, uint32_t m);
 int32_t sz_session_set_head_proxy(sz_session*, uint32_t k_blk);
 /* The reference chooses between exact and tensor-core kernels for EXL3 experts (mma_grouped_exl3_K, kernels/exl3.cu:682-725,
  * `--exact` and `tensor_prompt`, session.rs:1741, 1817).  Modes 0 to 3 are accepted and all run the same launches: the
- * codebook's own f16 weights against all 24 bits of the inputs on the matrix cores, f32 sums, which is the fastest form on an
- * MI355X as well as the exact one.  (Modes 1 to 3 once chose forms that kept fewer bits.) */
+ * codebook's own f16 weights against all 24 bits of the inputs (of those down to 2^-37 of the largest of 512; no less than 2^-61
+ * of it of the others) on the matrix cores, f32 sums, which is the fastest form on an MI355X as well as the exact one.  (Modes 1 to 3 once chose forms that kept fewer bits.) */
 int32_t sz_session_set_expert_mode(sz_session*, int32_t mode);
 /* 0: sz_verify_round launches its kernels one by one instead of replaying a captured graph (default 1). */
 int32_t sz_session_set_graph(sz_session*, int32_t enabled);

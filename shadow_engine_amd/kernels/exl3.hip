@@ -257,8 +257,11 @@ __device__ __forceinline__ void exl3_rows_wait(u32 t) {
 // (2) The products run on the matrix cores: a lane decodes 4 consecutive weights of the bit stream, which are four values of
 // operand B of v_mfma_f32_16x16x32_f16 as decoded (two tile rows make one instruction), 15 vector instructions a 16 x 16
 // tile for up to 4 tokens where the vector unit alone needs 19 a token.  The item's tokens ride on the rows of operand A in
-// THREE f16 parts (11 bits each: all 24 bits of an f32), scaled by the power of two that takes the largest magnitude of the
-// token's 512 inputs to [2^14, 2^15): products are exact and sums are f32, as with f32 inputs.
+// THREE f16 parts of 11 bits, scaled by the power of two that takes the largest magnitude of the token's 512 inputs to
+// [2^14, 2^15), the second and third part 2^11 and 2^22 times more: all 24 bits of an f32 down to 2^-37 of that largest, and an
+// error under 2^-61 of it below.  No codebook weight is smaller than 2^-10, so f32 inputs would lose as much in the f32 sums
+// that the largest input is part of.  Products are exact and sums are f32, as with f32 inputs.  (An infinite input gives no
+// finite output: the transform spreads it over 128 inputs of either sign.)
 // (3) A workgroup prepares the A rows of its 512 inputs once (a wave a 128-block: scales, transform, split) and its four
 // waves then take CT column tiles each over all 512 inputs, so there is no sum over waves.  The sums are left as they are:
 // whoever reads them (launch 2 for gate and up, the last launch for down) adds the partials of the 512-input blocks up and
@@ -389,9 +392,9 @@ __device__ __forceinline__ void verify_put_rows(u16* a_sh, float* s_mx, float* s
                     const u32 i = lane + 64 * h, t = i >> 4, sl = exl3_aslot(i & 15);
                     const float v = rot[r][h] * scale;
                     const _Float16 hi = (_Float16) v;
-                    const float v1 = v - (float) hi;
+                    const float v1 = (v - (float) hi) * 0x1p11f;
                     const _Float16 mid = (_Float16) v1;
-                    const _Float16 lo = (_Float16) (v1 - (float) mid);
+                    const _Float16 lo = (_Float16) ((v1 - (float) mid) * 0x1p11f);
                     u16* at = a_sh + (((kbl * 4 + (t >> 1)) * NR + 3 * r) * 4 + (sl >> 2)) * 8 + 4 * (t & 1) + (sl & 3);
                     at[0] = __builtin_bit_cast(u16, hi);
                     at[32] = __builtin_bit_cast(u16, mid);
@@ -495,7 +498,7 @@ __device__ __forceinline__ void verify_store(const f32x4 (&acc)[NG][CT], const f
             const u32 pair = (u32) (four >> (lane & 48)) & 0xffffu;
             float* o = out + (u64) pair * stride + (lane & 15);
 #pragma unroll
-            for (int c = 0; c < CT; c++) o[16 * c] = (acc[g][c][0] + acc[g][c][1] + acc[g][c][2]) * iv;
+            for (int c = 0; c < CT; c++) o[16 * c] = __builtin_fmaf(__builtin_fmaf(acc[g][c][2], 0x1p-11f, acc[g][c][1]), 0x1p-11f, acc[g][c][0]) * iv;
         }
     }
 }

@@ -3,10 +3,15 @@
 // Both formats' weights are a scale times small integers (Q8_0: codes of 8 bits, a scale a 32-block; IQ3_S: grid value * sign *
 // (1 + 2 s), at most 465, one scale a 256-block), which f16 holds exactly.  A row of W is a column of operand B of
 // v_mfma_f32_16x16x32_f16: lane 16 g + r holds 8 weights of row r.  The inputs ride on the rows of operand A in three f16
-// parts (11 bits each: all 24 bits of an f32), scaled by the power of two that takes the largest magnitude of their 256
-// columns to [2^14, 2^15): token t's parts are rows 4 t .. 4 t + 2, so its three sums come out in one lane (16 t + r) and the
-// block's scale is one multiply-add there.  Products are exact and sums are f32; an integer is decoded once for up to 8 inputs
-// (1.3 vector instructions a Q8_0 weight, 4 an IQ3_S one, where the vector unit alone takes 2 and 8 and one more a token).
+// parts of 11 bits, scaled by the power of two that takes the largest magnitude of their 256 columns to [2^14, 2^15), and the
+// second and third part 2^11 and 2^22 times more, so that they do not run under f16's smallest value: together they are the
+// f32 exactly down to 2^-37 of the largest, and within 2^-61 of the largest below.  An IQ3_S block's weights are between 1 and
+// 465 times its scale, so that is far under the rounding of the f32 sums which the largest input is part of; a Q8_0 code may be
+// zero where the largest input meets it, so what the parts leave is multiplied on the vector unit (gg_rest): no size of one
+// input costs another a bit, as with f32 multiply-adds.  Token t's parts are rows 4 t .. 4 t + 2, so its three sums come out in
+// one lane (16 t + r), where two multiply-adds and the block's scale, one more, put them together.  Products are exact and
+// sums are f32; an integer is decoded once for up to 8 inputs (1.3 vector instructions a Q8_0 weight, 4 an IQ3_S one, where
+// the vector unit alone takes 2 and 8 and one more a token).
 //
 // A wave takes 256-column chunks and keeps a chunk's input parts in registers while it goes over the workgroup's tiles of 16
 // rows: the parts are made once a chunk, not once a chunk and row group, and a matrix of few rows still spreads over all its
@@ -27,6 +32,9 @@ typedef u32 u32x4b __attribute__((ext_vector_type(4), aligned(2)));
 __device__ __forceinline__ f16x2 gg_pair(u32 v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ u32 gg_bits(f16x2 v) { return __builtin_bit_cast(u32, v); }
 
+// The three parts' sums put together, in units of the first one's.
+__device__ __forceinline__ float gg_sum(const f32x4& s) { return __builtin_fmaf(__builtin_fmaf(s[2], 0x1p-11f, s[1]), 0x1p-11f, s[0]); }
+
 // What a wave's LDS stores and loads of its own strip need between them: the compiler keeps their order, the chip does anyway.
 __device__ __forceinline__ void gg_order() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -39,26 +47,29 @@ __device__ __forceinline__ void gg_order() {
 struct GgQ8 {
     static constexpr u32 QK = 32, BB = 34, CHUNK = 272;   // bytes of a 256-column chunk: 17 pieces of 16
     static constexpr u32 PITCH = 72;                      // words of a row in the strip: 68 and a shift of four banks
-    static constexpr bool grid = false;
+    static constexpr bool grid = false, zeros = true;     // a table to look weights up in; weights that may be zero
     static constexpr u32 part_at(u32 q, u32 g) { return 32 * q + 8 * g; }   // first column of the lane's 8 in instruction q
     u32x4b v[5];
-    u32 at[5];   // the piece's row * 32 + its place in the row
+    u32 at[2];   // the pieces' rows and places in their rows, five bits each, three pieces a word
     __device__ __forceinline__ void init(u32 lane) {
+        at[0] = at[1] = 0;
 #pragma unroll
         for (u32 i = 0; i < 5; i++) {
             const u32 p = lane + 64 * i;
-            at[i] = p / 17 * 32 + p % 17;
+            at[i / 3] |= (p % 17 + p / 17 * 32) << (10 * (i % 3));
         }
     }
+    __device__ __forceinline__ u32 place(int i) const { return __builtin_amdgcn_ubfe(at[i / 3], 10 * (i % 3), 5); }
+    __device__ __forceinline__ u32 row(int i) const { return __builtin_amdgcn_ubfe(at[i / 3], 10 * (i % 3) + 5, 5); }
     __device__ __forceinline__ void load(const u8* __restrict__ w, u32 rb, u32 first, u32 rows, u32 col, u32 lane) {
         if (rb < CHUNK) return;
         const u8* base = w + (u64) first * rb + col / 32 * 34;
         const u32 rmost = rows - 1 - first;
 #pragma unroll
-        for (int i = 0; i < 5; i++) asm volatile("" : "+v"(at[i]));   // the addresses are a few operations: not kept
+        for (int i = 0; i < 2; i++) asm volatile("" : "+v"(at[i]));   // the addresses are a few operations: not kept
 #pragma unroll
         for (int i = 0; i < 5; i++)
-            if (i < 4 || lane < 16) v[i] = *(const u32x4b*) (base + (u64) min(at[i] >> 5, rmost) * rb + (at[i] & 31) * 16);
+            if (i < 4 || lane < 16) v[i] = *(const u32x4b*) (base + (u64) min(row(i), rmost) * rb + place(i) * 16);
     }
     __device__ __forceinline__ void stage(u32* strip, const u8* __restrict__ w, u32 rb, u32 first, u32 rows, u32 lane) const {
         if (rb < CHUNK) {
@@ -71,9 +82,17 @@ struct GgQ8 {
         } else {
 #pragma unroll
             for (int i = 0; i < 5; i++)
-                if (i < 4 || lane < 16) *(u32x4*) (strip + (at[i] >> 5) * PITCH + (at[i] & 31) * 4) = u32x4{v[i][0], v[i][1], v[i][2], v[i][3]};
+                if (i < 4 || lane < 16) *(u32x4*) (strip + row(i) * PITCH + place(i) * 4) = u32x4{v[i][0], v[i][1], v[i][2], v[i][3]};
         }
         gg_order();
+    }
+    // the product of x with the weights at columns c .. c + 3 (c a multiple of 4) after a row's first block
+    static __device__ __forceinline__ float four(const u8* row, u32 c, const f32x4& x) {
+        const u8* b = row + c / 32 * 34;
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) s = __builtin_fmaf((float) (i8) b[2 + c % 32 + i], x[i], s);
+        return s * f16_to_f32(*(const u16*) b);
     }
     // four codes to f16: 0x6400 | (code ^ 0x80) is 1024 + code + 128
     static __device__ __forceinline__ void codes(u32 v, u32& lo, u32& hi) {
@@ -110,7 +129,7 @@ struct GgQ8 {
 #pragma unroll
                 for (int G = 0; G < NG; G++) {
                     const f32x4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[G][b]), wv, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    out[G] = __builtin_fmaf((s[0] + s[1]) + s[2], dd, out[G]);
+                    out[G] = __builtin_fmaf(gg_sum(s), dd, out[G]);
                 }
             }
             if (b & 1) __builtin_amdgcn_sched_barrier(0);   // two blocks' words in registers at a time, not eight
@@ -121,7 +140,7 @@ struct GgQ8 {
 // eight matrix instructions is the lane's own (instruction i: columns 64 g + 8 i ..), the same on both operands.
 struct GgIq3 {
     static constexpr u32 QK = 256, BB = 110;
-    static constexpr bool grid = true;
+    static constexpr bool grid = true, zeros = false;
     static constexpr u32 part_at(u32 q, u32 g) { return 64 * g + 8 * q; }
     u32 qs[4], sg[2], qh, sc, d;
     __device__ __forceinline__ void init(u32) {}
@@ -172,33 +191,48 @@ struct GgIq3 {
         }
         const float dd = f16_to_f32((u16) d);
 #pragma unroll
-        for (int G = 0; G < NG; G++) out[G] = __builtin_fmaf((s[G][0] + s[G][1]) + s[G][2], dd, out[G]);
+        for (int G = 0; G < NG; G++) out[G] = __builtin_fmaf(gg_sum(s[G]), dd, out[G]);
     }
 };
 
+// The largest magnitude among the chunk's columns of one input (a lane has four).
+__device__ __forceinline__ float gg_most(const f32x4& v) {
+    return wave_max_f32(fmaxf(fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3]))));
+}
+// What is left of an input, scaled, after one f16 part of it, 2^11 times.  Exact: the difference fits an f32.
+__device__ __forceinline__ float gg_left(float x, _Float16 part) { return __builtin_fmaf((float) part, -0x1p11f, x * 0x1p11f); }
+
 // 256 columns of the inputs 4 G .. 4 G + 3 (v[r]: the lane's four columns of each; zero past the last input), as the lane's
-// operand registers: their three parts go through the strip.  iv undoes the scale of input 4 G + lane / 16.
+// operand registers: their three parts go through the strip.  iv undoes the scale of input 4 G + lane / 16.  Returns whether
+// some input is under 2^-37 times the largest, so that the parts may not be all of it.
 template <class F>
-__device__ __forceinline__ void gg_split(const f32x4 (&v)[4], u32 n, u32* strip, u32 lane, u32x4 (&a)[8], float& iv) {
+__device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip, u32 lane, u32x4 (&a)[8], float& iv) {
     u16* st = (u16*) strip;
+    bool small = false;
     iv = 1.0f;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         u32 part[3][2] = {{0, 0}, {0, 0}, {0, 0}};
         if ((u32) r < n) {
-            const float mx = wave_max_f32(fmaxf(fmaxf(__builtin_fabsf(v[r][0]), __builtin_fabsf(v[r][1])), fmaxf(__builtin_fabsf(v[r][2]), __builtin_fabsf(v[r][3]))));
+            const float mx = gg_most(v[r]);
             float scale, inv;
             pow2_scale_of(f32_bits(mx), scale, inv);
             if (lane >> 4 == (u32) r) iv = inv;
+            if constexpr (F::zeros) {
+                u32 least = 0xffffffffu;   // of the bits without the sign, less one: a zero counts as the largest
+#pragma unroll
+                for (int i = 0; i < 4; i++) least = min(least, 2 * f32_bits(v[r][i]) - 1u);
+                small = small || least < max(2 * f32_bits(mx * 0x1p-37f), 1u) - 1u;
+            }
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 const float x0 = v[r][2 * i] * scale, y0 = v[r][2 * i + 1] * scale;
                 const _Float16 xh = (_Float16) x0, yh = (_Float16) y0;
-                const float x1 = x0 - (float) xh, y1 = y0 - (float) yh;
+                const float x1 = gg_left(x0, xh), y1 = gg_left(y0, yh);
                 const _Float16 xm = (_Float16) x1, ym = (_Float16) y1;
                 part[0][i] = gg_bits(f16x2{xh, yh});
                 part[1][i] = gg_bits(f16x2{xm, ym});
-                part[2][i] = gg_bits(f16x2{(_Float16) (x1 - (float) xm), (_Float16) (y1 - (float) ym)});
+                part[2][i] = gg_bits(f16x2{(_Float16) gg_left(x1, xm), (_Float16) gg_left(y1, ym)});
             }
         }
 #pragma unroll
@@ -210,6 +244,41 @@ __device__ __forceinline__ void gg_split(const f32x4 (&v)[4], u32 n, u32* strip,
 #pragma unroll
     for (u32 q = 0; q < 8; q++) a[q] = *(const u32x4*) (rowp + F::part_at(q, lane >> 4));
     gg_order();
+    return F::zeros && __builtin_amdgcn_ballot_w64(small) != 0;
+}
+
+// The products of what the three parts leave of a chunk's inputs, on the vector unit and a row at a time, into the sums of the
+// workgroup's tiles: rare, so short rather than fast.  x: the chunk's columns of input 0 (the lane's four at 4 * lane), if
+// they are `mine` to add; w: the chunk's first block of row 0.
+template <class F, int NG>
+__device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 rows, u32 nt, const float* __restrict__ x, u32 xs, u32 m, bool mine, u32 lane, float* tot) {
+#pragma unroll 1
+    for (u32 j = 0; j < m; j++) {
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (mine) v = *(const f32x4*) (x + (u64) j * xs + 4 * lane);
+        float scale, inv;
+        pow2_scale_of(f32_bits(gg_most(v)), scale, inv);
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float x0 = v[i] * scale;
+            const _Float16 xh = (_Float16) x0;
+            const float x1 = gg_left(x0, xh);
+            const _Float16 xm = (_Float16) x1;
+            const float x2 = gg_left(x1, xm);
+            v[i] = (x2 - (float) (_Float16) x2) * 0x1p-22f;   // in units of the scale
+            any = any || v[i] != 0.0f;
+        }
+        if (!__builtin_amdgcn_ballot_w64(any)) continue;
+#pragma unroll 1
+        for (u32 i = 0; i < 16 * nt; i++) {
+            const u32 row = 16 * (blockIdx.x + i / 16 * gridDim.x) + i % 16;
+            float s = mine && row < rows ? F::four(w + (u64) row * rb, 4 * lane, v) : 0.0f;
+            s = seg_sum<64>(s, lane);
+            float* at = tot + (i / 16 * NG + j / 4) * 64;
+            if (lane == 16 * (j & 3) + i % 16) *at = __builtin_fmaf(s, inv, *at);
+        }
+    }
 }
 
 __device__ __forceinline__ void gg_table(u32* table) {
@@ -236,6 +305,7 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
     F cur;
     cur.init(lane);
     for (u32 t = 0; t < nt * NG; t++) tot[64 * t] = 0.0f;
+    bool left = false;
     for (u32 c = wave; c < nc; c += W) {
         const u32 col = start(c) + 4 * lane;
         f32x4 v[NG][4];
@@ -254,7 +324,7 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
         u32x4 a[NG][8];
         float iv[NG];
 #pragma unroll
-        for (int G = 0; G < NG; G++) gg_split<F>(v[G], m - min(m, 4u * G), strip, lane, a[G], iv[G]);
+        for (int G = 0; G < NG; G++) left = gg_split<F>(v[G], m - min(m, 4u * G), strip, lane, a[G], iv[G]) || left;
 #pragma unroll 1
         for (u32 t = 0; t < nt; t++) {
             const u32 first = 16 * (blockIdx.x + t * gridDim.x);
@@ -270,6 +340,11 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
             for (int G = 0; G < NG; G++) tot[(t * NG + G) * 64] = __builtin_fmaf(out[G], iv[G], tot[(t * NG + G) * 64]);
             gg_order();   // the strip is read before the next tile goes there (LDS is in order within a wave)
         }
+    }
+    if constexpr (F::zeros) {
+        if (left)
+            for (u32 c = wave; c < nc; c += W)
+                gg_rest<F, NG>(w + start(c) / F::QK * F::BB, rb, rows, nt, x + start(c), xs, m, start(c) + 4 * lane >= 256 * c && start(c) + 4 * lane < cols, lane, tot);
     }
     __syncthreads();
     for (u32 i = threadIdx.x; i < nt * NG * 64; i += blockDim.x) {

@@ -122,3 +122,27 @@ def test_products_of_subnormal_inputs(gpu, ty, m):  # noqa: F811
         else:
             want = O.dequantize(ty, w).reshape(rows, cols).astype(np.float64) @ x[j].astype(np.float64)
             assert np.linalg.norm(want) > 2.0 ** -126 and np.linalg.norm(got[j] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("m", [1, 3, 8])
+@pytest.mark.parametrize("cols", [256, 800, 4352])
+def test_a_large_input_costs_the_others_no_bits(gpu, m, cols):  # noqa: F811
+    """Inputs of four sizes from 2^-100 to 2^40 in every 32-block, and rows whose codes are zero but for the inputs of one size: every
+    row's product is as good as f32 sums of its own terms, whatever lies beside them.  (512 terms and less a sum, in chunks:
+    1e-5 of the sum of magnitudes is far above their rounding.)"""
+    rng = np.random.default_rng(m + cols)
+    rows = 96
+    w = synth.q8_0_matrix(rng, rows, cols)
+    size = rng.integers(0, 4, cols)
+    size[:32:8] = [3, 0, 1, 2]
+    codes = w.reshape(rows, cols // 32, 34)[:, :, 2:].reshape(rows, cols)
+    codes[size[None, :] != (np.arange(rows) % 4)[:, None]] = 0
+    w.reshape(rows, cols // 32, 34)[:, :, 2:] = codes.reshape(rows, cols // 32, 32)
+    x = (rng.normal(size=(m, cols)) * np.array([1.0, 2.0 ** -50, 2.0 ** -100, 2.0 ** 40])[size]).astype(np.float32)
+    if m > 2:
+        x[2] = rng.normal(size=cols)             # an input without any such spread between others that have one
+    got = products(gpu, sz.Q8_0, rows, cols, w, x).astype(np.float64)
+    dense = O.dequantize(sz.Q8_0, w).reshape(rows, cols).astype(np.float64)
+    for j in range(m):
+        terms = dense * x[j].astype(np.float64)
+        assert np.all(np.abs(got[j] - terms.sum(axis=1)) <= 1e-5 * np.abs(terms).sum(axis=1)), j
