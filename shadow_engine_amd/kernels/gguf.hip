@@ -224,6 +224,8 @@ __device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip,
                 for (int i = 0; i < 4; i++) least = min(least, 2 * f32_bits(v[r][i]) - 1u);
                 small = small || least < max(2 * f32_bits(mx * 0x1p-37f), 1u) - 1u;
             }
+            // an infinity is all in its first part: what it leaves would be a NaN
+            const u32 keep = f32_bits(mx) == 0x7f800000u ? 0u : ~0u;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 const float x0 = v[r][2 * i] * scale, y0 = v[r][2 * i + 1] * scale;
@@ -231,8 +233,8 @@ __device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip,
                 const float x1 = gg_left(x0, xh), y1 = gg_left(y0, yh);
                 const _Float16 xm = (_Float16) x1, ym = (_Float16) y1;
                 part[0][i] = gg_bits(f16x2{xh, yh});
-                part[1][i] = gg_bits(f16x2{xm, ym});
-                part[2][i] = gg_bits(f16x2{(_Float16) gg_left(x1, xm), (_Float16) gg_left(y1, ym)});
+                part[1][i] = gg_bits(f16x2{xm, ym}) & keep;
+                part[2][i] = gg_bits(f16x2{(_Float16) gg_left(x1, xm), (_Float16) gg_left(y1, ym)}) & keep;
             }
         }
 #pragma unroll
@@ -257,7 +259,9 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (mine) v = *(const f32x4*) (x + (u64) j * xs + 4 * lane);
         float scale, inv;
-        pow2_scale_of(f32_bits(gg_most(v)), scale, inv);
+        const float mx = gg_most(v);
+        if (f32_bits(mx) == 0x7f800000u) continue;   // nothing finite comes of it
+        pow2_scale_of(f32_bits(mx), scale, inv);
         bool any = false;
 #pragma unroll
         for (int i = 0; i < 4; i++) {

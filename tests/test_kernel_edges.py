@@ -146,3 +146,34 @@ def test_a_large_input_costs_the_others_no_bits(gpu, m, cols):  # noqa: F811
     for j in range(m):
         terms = dense * x[j].astype(np.float64)
         assert np.all(np.abs(got[j] - terms.sum(axis=1)) <= 1e-5 * np.abs(terms).sum(axis=1)), j
+
+
+@pytest.mark.parametrize("ty", [sz.Q8_0, sz.IQ3_S])
+@pytest.mark.parametrize("m", [1, 3, 8])
+def test_an_infinite_input_gives_what_multiply_adds_give(gpu, ty, m):  # noqa: F811
+    """One infinity: the sign of its weight's infinity, a NaN where that weight is zero; two that meet weights of opposite signs: a
+    NaN; a NaN: a NaN; the inputs beside them in the batch, the largest floats among them, as without."""
+    rng = np.random.default_rng(m)
+    rows, cols = 48, 768
+    w = synth.q8_0_matrix(rng, rows, cols) if ty == sz.Q8_0 else synth.iq3_s_matrix(rng, rows, cols)
+    if ty == sz.Q8_0:
+        w.reshape(rows, cols // 32, 34)[::3, 300 // 32, 2 + 300 % 32] = 0
+    dense = O.dequantize(ty, w).reshape(rows, cols).astype(np.float64)
+    assert ty == sz.Q8_0 or np.all(dense != 0.0)
+    x = rng.normal(size=(m, cols)).astype(np.float32)
+    x[0, 300] = np.inf
+    if m > 2:
+        x[1, [5, 300]] = -np.inf
+        x[1, 6] = 3.0e38
+    if m > 3:
+        x[3, 700] = np.nan
+        x[4, 300] = 1.0e38
+        x[5] *= np.float32(1.0e-38)
+    got = products(gpu, ty, rows, cols, w, x)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for j in range(m):
+            want = (dense * x[j].astype(np.float64)).sum(axis=1)
+            assert np.array_equal(np.isnan(got[j]), np.isnan(want)), j
+            ok = np.isfinite(want)
+            assert np.array_equal(got[j][~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)]), j
+            assert np.all(np.abs(got[j][ok] - want[ok]) <= 1e-5 * (np.abs(dense) * np.abs(x[j].astype(np.float64))).sum(axis=1)[ok]), j
