@@ -1114,11 +1114,11 @@ extern "C" __global__ void __launch_bounds__(512) router_rows_m8(u32 type, const
     router_rows<8>(type, w, gate_type, gate_w, x, rl, sgl, ne, cols, m);
 }
 
-// The hyper-connection's read (forward.rs:797-812) in two launches.  The first: every stream of every row normalised (the mean
-// of squares in f64 as the CPU path has it), and the down and inject products of that: a stream's scale 1/sqrt(ms + eps) is a
-// factor of the sum over its columns and multiplies that.  A workgroup owns `pass` rows of the two matrices (down's first) and normalises the inputs for itself: it
-// has to read all of them anyway, and the arithmetic is less than another launch costs.  Workgroup 0 leaves the scales
-// 1/sqrt(ms + eps) for the second launch.
+// The hyper-connection's read (forward.rs:797-812) in two launches.  The first: every stream of every row normalised, the mean
+// of squares and the scaling of every input in f64 as the CPU path has them, and the down and inject products of that.  A
+// workgroup owns `pass` rows of the two matrices (down's first) and normalises the inputs for itself: it has to read all of them
+// anyway, and the arithmetic is less than another launch costs.  Workgroup 0 leaves the scales 1/sqrt(ms + eps) for the second
+// launch.
 // r: [m][streams * h]; down, g: silu(t / streams), 2 sigmoid(t / streams).  grid = ceil(rank / pass) + ceil(streams / pass) (inject),
 // block 64 max(4, dense_waves(ch)), dynamic LDS = m * streams * (1 + chunks of ch) doubles.
 __device__ __forceinline__ double lane_xor_f64(double v, u32 lane, int h) {
@@ -1144,24 +1144,19 @@ __device__ __forceinline__ double wave_sum_f64(double v, u32 lane) {
     return v;
 }
 
-// A lane's sums of w * (norm_w * r), one for each of its chunks (which lies in one stream), before the streams' scales.
+// The lane's inputs normalised: (float) (r * scale) * norm weight, a chunk of them in one stream.
 template <class T, int M>
-__device__ __forceinline__ void hc_products(const DenseSlice<T>& sl, const typename T::Raw (&wv)[DenseSlice<T>::NCH], const float (&xv)[M][DENSE_LANE_COLS],
-                                            const float* __restrict__ nw, u32 o, float (&raw)[DenseSlice<T>::NCH][M]) {
+__device__ __forceinline__ void hc_normalise(const DenseSlice<T>& sl, float (&xv)[M][DENSE_LANE_COLS], const float (&nv)[1][DENSE_LANE_COLS], const double* scl, u32 h, u32 cs, u32 m,
+                                             u32 o) {
 #pragma unroll
     for (int i = 0; i < DenseSlice<T>::NCH; i++) {
-        const u32 c = sl.col(o, i);
+        const u32 s = min(sl.col(o, i), sl.cols - 1) / h;
 #pragma unroll
-        for (int j = 0; j < M; j++) raw[i][j] = 0.0f;
+        for (int j = 0; j < M; j++) {
+            if ((u32) j < m) {
+                const double sc = scl[(u32) j * cs + s];
 #pragma unroll
-        for (int q = 0; q < (int) T::C; q += 4) {
-            f32x4 n = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (c < sl.cols) n = *(const f32x4*) (nw + c + q);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float wv_ = T::get(wv[i], q + e);
-#pragma unroll
-                for (int j = 0; j < M; j++) raw[i][j] = __builtin_fmaf(wv_, xv[j][i * T::C + q + e] * n[e], raw[i][j]);
+                for (int e = 0; e < (int) T::C; e++) xv[j][i * T::C + e] = (float) ((double) xv[j][i * T::C + e] * sc) * nv[0][i * T::C + e];
             }
         }
     }
@@ -1178,7 +1173,7 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     const u32 pieces = outer * S::NCH * kwn;   // spans of 64 C columns, each one wave's
     double* part = (double*) sz_dyn_lds;       // [m][cs][pieces of the widest stream]: the spans' sums of squares, in order
     const u32 wide = h / span + 2;
-    float* scl = (float*) (part + (u64) m * cs * wide);
+    double* scl = part + (u64) m * cs * wide;
     const bool live = rg < rw;
     const u32 row = first + rg;
     float xv[M][DENSE_LANE_COLS];
@@ -1190,9 +1185,7 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     float acc[M];
 #pragma unroll
     for (int j = 0; j < M; j++) acc[j] = 0.0f;
-    // pass 0: the spans' sums of squares and, while all of the inputs are in registers (outer == 1), the products without the
-    // streams' scales, which are factored out of a lane's sums over one chunk; pass 1 (longer rows): the products
-    float raw[S::NCH][M];
+    // the spans' sums of squares first, then the products (of inputs that are still in registers where outer == 1)
     for (u32 o = 0; o < outer; o++) {
         if (o) sl.inputs(r, cols, m, o, xv);
 #pragma unroll
@@ -1219,14 +1212,15 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
                 }
             }
         }
-        if (outer == 1) hc_products<T, M>(sl, wv, xv, nw, 0, raw);
     }
+    float nv[1][DENSE_LANE_COLS];   // the norm weights come while the scales are made
+    sl.inputs(nw, 0, 1, 0, nv);
     __syncthreads();
     for (u32 i = tid; i < m * cs; i += blockDim.x) {
         double ss = 0.0;
         for (u32 q = 0; q < wide; q++) ss += part[i * wide + q];
         const double sc = 1.0 / sqrt(ss / (double) h + (double) eps);
-        scl[i] = (float) sc;
+        scl[i] = sc;
         if (blockIdx.x == 0) scales[i] = sc;
     }
     __syncthreads();
@@ -1234,14 +1228,10 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
         if (outer > 1) {
             sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, o, live && row < rows, wv);
             sl.inputs(r, cols, m, o, xv);
-            hc_products<T, M>(sl, wv, xv, nw, o, raw);
+            sl.inputs(nw, 0, 1, o, nv);
         }
-#pragma unroll
-        for (int i = 0; i < S::NCH; i++) {
-            const u32 s = min(sl.col(o, i), cols - 1) / h;
-#pragma unroll
-            for (int j = 0; j < M; j++) acc[j] = __builtin_fmaf(raw[i][j], scl[min((u32) j, m - 1) * cs + s], acc[j]);
-        }
+        hc_normalise<T, M>(sl, xv, nv, scl, h, cs, m, o);
+        sl.dot(wv, xv, acc);
     }
     const float t = dense_reduce<M>(acc, 64, lane);
     if (live && lane < (u32) M) red[wave * 8 + lane] = t;
@@ -1278,7 +1268,7 @@ extern "C" __global__ void __launch_bounds__(512) hc_down_m1(u32 type, const u8*
                                                              float* g, u32 h, u32 cs, u32 m, float eps) {
     hc_down<1>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
 }
-extern "C" __global__ void __launch_bounds__(512) hc_down_m4(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+extern "C" __global__ void __launch_bounds__(512, 4) hc_down_m4(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
                                                              float* g, u32 h, u32 cs, u32 m, float eps) {
     hc_down<4>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
 }

@@ -5,7 +5,7 @@ import pytest
 import oracle_lib as O
 import shadow_engine_amd as sz
 from shadow_engine_amd import synth
-from test_gpu_path import REL_L2, bits, build_layer, dev, gguf_bound, gpu, oracle_layer, rel_l2  # noqa: F401 (gpu: the fixture)
+from test_gpu_path import REL_L2, bits, build_layer, dense_matrix, dev, gguf_bound, gpu, oracle_layer, rel_l2  # noqa: F401 (gpu: the fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -177,3 +177,42 @@ def test_an_infinite_input_gives_what_multiply_adds_give(gpu, ty, m):  # noqa: F
             ok = np.isfinite(want)
             assert np.array_equal(got[j][~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)]), j
             assert np.all(np.abs(got[j][ok] - want[ok]) <= 1e-5 * (np.abs(dense) * np.abs(x[j].astype(np.float64))).sum(axis=1)[ok]), j
+
+
+@pytest.mark.parametrize("ty,h,cs,rank,m,size", [
+    (sz.BF16, 2048, 4, 320, 4, 1.2e38), (sz.F32, 256, 2, 24, 8, 1.2e38), (sz.F16, 512, 4, 64, 1, 1e-30),   # streams near the largest f32, and tiny ones
+    (sz.F16, 1024, 3, 64, 3, 1.0), (sz.BF16, 1280, 4, 64, 5, 1.0), (sz.F32, 1792, 4, 64, 8, 1.0),      # a row over 3, 5 and 7 waves
+    (sz.BF16, 4096, 4, 128, 4, 1.0),                                                                   # rows that do not stay in registers
+    (sz.F16, 100, 64, 24, 8, 1.0),                                                                     # a wave's span over several streams
+    (sz.BF16, 9216, 64, 8, 8, 1.0)])                                                                   # rows in lots: seven, then one
+def test_hyper_connection_at_its_edges(gpu, ty, h, cs, rank, m, size):  # noqa: F811
+    """hc_read over sizes of streams, of the matrices' rows and of the values, against the oracle."""
+    rng = np.random.default_rng(h + cs + m)
+    ch, eps = h * cs, 1e-6 if size >= 1.0 else 0.0
+    r = np.clip(rng.normal(size=(m, ch)) * size, -3.3e38, 3.3e38).astype(np.float32)
+    nw = (1 + 0.1 * rng.normal(size=ch)).astype(np.float32)
+    wd, wu, wi = dense_matrix(rng, ty, rank, ch), dense_matrix(rng, ty, ch, rank), dense_matrix(rng, ty, cs, ch)
+    dr, dnw, dwd, dwu, dwi = dev(gpu, r), dev(gpu, nw), dev(gpu, wd), dev(gpu, wu), dev(gpu, wi)
+    hc = sz.HyperConnection(h, cs, rank, eps, dnw.data_ptr(), ty, dwd.data_ptr(), ty, dwu.data_ptr(), ty, dwi.data_ptr())
+    du = gpu.zeros((m, h), dtype=gpu.float32, device="cuda")
+    hc.read(m, dr.data_ptr(), du.data_ptr())
+    gpu.cuda.synchronize()
+    u, g = du.cpu().numpy(), np.empty((m, cs), np.float32)
+    sz.download(g, hc.gains)
+    for j in range(m):
+        wu_, wg_ = O.hc_read(r[j], h, cs, rank, eps, nw, (ty, wd), (ty, wu), (ty, wi))
+        assert np.all(np.isfinite(wu_)) and rel_l2(u[j], wu_) <= 1e-5, rel_l2(u[j], wu_)
+        assert np.allclose(g[j], wg_, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("ty", [sz.F32, sz.F16, sz.BF16])
+@pytest.mark.parametrize("rows,cols,m", [(9, 3072, 4), (5, 5000, 8), (6, 7168, 1), (17, 8192, 5), (3, 8196, 8), (1100, 9220, 3), (4, 20480, 4)])
+def test_unquantized_rows_of_several_waves_and_longer(gpu, ty, rows, cols, m):  # noqa: F811
+    """Rows over 3, 5, 7 and 8 waves of a workgroup, rows of more than 8192 columns, whose inputs do not stay in registers, and
+    several passes of such rows a workgroup; every input has the bits of a launch of its own."""
+    rng = np.random.default_rng(rows + cols + m)
+    w, x = dense_matrix(rng, ty, rows, cols), rng.normal(size=(m, cols)).astype(np.float32)
+    got = products(gpu, ty, rows, cols, w, x)
+    for j in range(m):
+        assert rel_l2(got[j], O.matvec(ty, cols, rows, w, x[j])) <= 1e-5
+    assert np.array_equal(bits(products(gpu, ty, rows, cols, w, x[m - 1:])), bits(got[m - 1:]))
