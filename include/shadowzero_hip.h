@@ -108,7 +108,8 @@ sz_backend* sz_backend_new(uint64_t resident_budget_bytes);      /* GpuBackend::
 void sz_backend_free(sz_backend*);
 /* y[rows] = W x.  GGUF types: `bytes` is rows whole rows of `cols` weights; EXL3: a blob with in = cols, out = rows.  A
  * non-null `key` names bytes that never change: uploaded once and kept resident within the budget.  Host pointers in,
- * host pointers out, synchronous, like the reference's. */
+ * host pointers out, synchronous, like the reference's.  EXL3 and unquantized products have the bits sz_matvec_cols gives;
+ * GGUF ones are f32 sums in another order (the kernel that answers a single input soonest), equal to it to rounding. */
 int32_t sz_matvec(sz_backend*, int32_t ggml_type, uint64_t cols, uint64_t rows, const void* bytes, uint64_t nbytes, const char* key,
                   const float* x, float* y);
 uint64_t sz_backend_resident_bytes(const sz_backend*);
@@ -120,7 +121,8 @@ uint64_t sz_backend_uploads(const sz_backend*);
 int32_t sz_dequantize(int32_t ggml_type, uint64_t w, uint64_t out_f32, uint64_t cols, uint64_t rows, uint64_t stream);
 int32_t sz_exl3_codebook(uint64_t out_f32_65536, uint64_t stream);
 /* y_j = W x_j, j < m <= 8 (matvec_cols_*, kernels/matvec.cu:677; matvec_cols_exl3_*, kernels/exl3.cu:260): x rows xs floats
- * apart, y rows ys floats apart.  `scratch`/`scratch_bytes`: device workspace, sz_matvec_cols_scratch() bytes. */
+ * apart, y rows ys floats apart.  `scratch`/`scratch_bytes`: device workspace, sz_matvec_cols_scratch() bytes.  Every y_j has the
+ * bits a launch for x_j alone gives. */
 uint64_t sz_matvec_cols_scratch(int32_t ggml_type, uint64_t cols, uint64_t rows, uint32_t m);
 int32_t sz_matvec_cols(int32_t ggml_type, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x, uint32_t xs, uint64_t y, uint32_t ys,
                        uint32_t m, uint64_t scratch, uint64_t scratch_bytes, uint64_t stream);

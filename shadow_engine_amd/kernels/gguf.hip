@@ -17,9 +17,11 @@
 // rows: the parts are made once a chunk, not once a chunk and row group, and a matrix of few rows still spreads over all its
 // chunks.  A Q8_0 tile's chunk comes in 16-byte loads along the rows and is turned round in a strip of LDS of the wave's own
 // (loads of a lane's own 8 codes, 16 rows apart, stopped at 2.2 TB/s without any product).
-// Measured: Q8_0, 8201 rows of 3072 columns, 5 inputs: 11.8 us (2.3 TB/s; 25 with the parts made for every 32 rows and loads of
-// a lane's own codes, 41 on the vector unit).  What is left is the chain of a workgroup's start, an input's parts and two or three
-// tiles, not the memory: a CU runs one such workgroup at a time.
+// Measured: Q8_0, 8201 rows of 3072 columns, 5 inputs: 10.9 us a call (2.5 TB/s; 25 with the parts made for every 32 rows and
+// loads of a lane's own codes, 41 on the vector unit).  What is left is the chain of a workgroup's start, an input's parts and two
+// or three tiles, not the memory: a CU runs one such workgroup at a time.  So the parts take few instructions: the largest
+// magnitude by whole-number DPP steps into a scalar, then five mixed-precision multiply-adds an input (2048 x 8192, 3 inputs: 11.4
+// -> 10.7 us), and their rest for free.  Tiles of 8 or 4 rows for matrices of few rows measured the same as 16.
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef u32 u32x2b __attribute__((ext_vector_type(2), aligned(2)));   // GGUF rows are only 2-byte aligned
@@ -195,50 +197,62 @@ struct GgIq3 {
     }
 };
 
-// The largest magnitude among the chunk's columns of one input (a lane has four).
-__device__ __forceinline__ float gg_most(const f32x4& v) {
-    return wave_max_f32(fmaxf(fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3]))));
+// The bits of the largest magnitude among the chunk's columns of one input (a lane has four): as whole numbers, which order
+// like the floats, over the lanes of a row, the rows, and out of the last lane.
+template <int ctrl, int rows>
+__device__ __forceinline__ u32 gg_max_step(u32 v) { return max(v, (u32) __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, true)); }
+__device__ __forceinline__ u32 gg_most(const f32x4& x) {
+    u32 v = f32_bits(fmaxf(fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])), fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])))) & 0x7fffffffu;
+    v = gg_max_step<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v = gg_max_step<0x112, 0xf>(v);
+    v = gg_max_step<0x114, 0xf>(v);
+    v = gg_max_step<0x118, 0xf>(v);
+    v = gg_max_step<0x142, 0xa>(v);   // row_bcast 15, 31
+    v = gg_max_step<0x143, 0xc>(v);
+    return __builtin_amdgcn_readlane(v, 63);
 }
-// What is left of an input, scaled, after one f16 part of it, 2^11 times.  Exact: the difference fits an f32.
-__device__ __forceinline__ float gg_left(float x, _Float16 part) { return __builtin_fmaf((float) part, -0x1p11f, x * 0x1p11f); }
 
-// 256 columns of the inputs 4 G .. 4 G + 3 (v[r]: the lane's four columns of each; zero past the last input), as the lane's
-// operand registers: their three parts go through the strip.  iv undoes the scale of input 4 G + lane / 16.  Returns whether
-// some input is under 2^-37 times the largest, so that the parts may not be all of it.
+// An input's three parts at a scale, and what they leave of it (in units of the scale, exact like the differences on the way).
+__device__ __forceinline__ float gg_parts(float x, float scale, _Float16& p0, _Float16& p1, _Float16& p2) {
+    p0 = (_Float16) (x * scale);
+    const float r1 = __builtin_fmaf(x, scale, -(float) p0);
+    p1 = (_Float16) (r1 * 0x1p11f);
+    const float r2 = __builtin_fmaf((float) p1, -0x1p-11f, r1);
+    p2 = (_Float16) (r2 * 0x1p22f);
+    return __builtin_fmaf((float) p2, -0x1p-22f, r2);
+}
+
+// 256 columns of the inputs 4 G .. 4 G + 3 (v[r]: the lane's four columns of each), as the lane's operand registers: the three
+// parts of the n that there are go through the strip (the rows of others hold what lay there: their sums go nowhere).  iv undoes
+// the scale of input 4 G + lane / 16.  Returns whether the parts are not all of some input (which is then under 2^-37 times the
+// largest).
 template <class F>
 __device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip, u32 lane, u32x4 (&a)[8], float& iv) {
     u16* st = (u16*) strip;
-    bool small = false;
+    u32 rest = 0;
     iv = 1.0f;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        u32 part[3][2] = {{0, 0}, {0, 0}, {0, 0}};
         if ((u32) r < n) {
-            const float mx = gg_most(v[r]);
+            u32 part[3][2];
+            const u32 mx = gg_most(v[r]);
             float scale, inv;
-            pow2_scale_of(f32_bits(mx), scale, inv);
+            pow2_scale_of(mx, scale, inv);
             if (lane >> 4 == (u32) r) iv = inv;
-            if constexpr (F::zeros) {
-                u32 least = 0xffffffffu;   // of the bits without the sign, less one: a zero counts as the largest
-#pragma unroll
-                for (int i = 0; i < 4; i++) least = min(least, 2 * f32_bits(v[r][i]) - 1u);
-                small = small || least < max(2 * f32_bits(mx * 0x1p-37f), 1u) - 1u;
-            }
             // an infinity is all in its first part: what it leaves would be a NaN
-            const u32 keep = f32_bits(mx) == 0x7f800000u ? 0u : ~0u;
+            const u32 keep = mx == 0x7f800000u ? 0u : ~0u;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                const float x0 = v[r][2 * i] * scale, y0 = v[r][2 * i + 1] * scale;
-                const _Float16 xh = (_Float16) x0, yh = (_Float16) y0;
-                const float x1 = gg_left(x0, xh), y1 = gg_left(y0, yh);
-                const _Float16 xm = (_Float16) x1, ym = (_Float16) y1;
-                part[0][i] = gg_bits(f16x2{xh, yh});
-                part[1][i] = gg_bits(f16x2{xm, ym}) & keep;
-                part[2][i] = gg_bits(f16x2{(_Float16) gg_left(x1, xm), (_Float16) gg_left(y1, ym)}) & keep;
-            }
-        }
+                _Float16 t[2][3];
 #pragma unroll
-        for (int p = 0; p < 3; p++) *(uint2*) (st + (3 * r + p) * GG_PITCH + 4 * lane) = uint2{part[p][0], part[p][1]};
+                for (int e = 0; e < 2; e++) rest |= f32_bits(gg_parts(v[r][2 * i + e], scale, t[e][0], t[e][1], t[e][2]));
+                part[0][i] = gg_bits(f16x2{t[0][0], t[1][0]});
+                part[1][i] = gg_bits(f16x2{t[0][1], t[1][1]}) & keep;
+                part[2][i] = gg_bits(f16x2{t[0][2], t[1][2]}) & keep;
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) *(uint2*) (st + (3 * r + p) * GG_PITCH + 4 * lane) = uint2{part[p][0], part[p][1]};
+        }
     }
     gg_order();
     const u32 ar = lane & 15;
@@ -246,7 +260,7 @@ __device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip,
 #pragma unroll
     for (u32 q = 0; q < 8; q++) a[q] = *(const u32x4*) (rowp + F::part_at(q, lane >> 4));
     gg_order();
-    return F::zeros && __builtin_amdgcn_ballot_w64(small) != 0;
+    return F::zeros && __builtin_amdgcn_ballot_w64(rest != 0) != 0;
 }
 
 // The products of what the three parts leave of a chunk's inputs, on the vector unit and a row at a time, into the sums of the
@@ -259,18 +273,14 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (mine) v = *(const f32x4*) (x + (u64) j * xs + 4 * lane);
         float scale, inv;
-        const float mx = gg_most(v);
-        if (f32_bits(mx) == 0x7f800000u) continue;   // nothing finite comes of it
-        pow2_scale_of(f32_bits(mx), scale, inv);
+        const u32 mx = gg_most(v);
+        if (mx >= 0x7f800000u) continue;   // nothing finite comes of it
+        pow2_scale_of(mx, scale, inv);
         bool any = false;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const float x0 = v[i] * scale;
-            const _Float16 xh = (_Float16) x0;
-            const float x1 = gg_left(x0, xh);
-            const _Float16 xm = (_Float16) x1;
-            const float x2 = gg_left(x1, xm);
-            v[i] = (x2 - (float) (_Float16) x2) * 0x1p-22f;   // in units of the scale
+            _Float16 p0, p1, p2;
+            v[i] = gg_parts(v[i], scale, p0, p1, p2);
             any = any || v[i] != 0.0f;
         }
         if (!__builtin_amdgcn_ballot_w64(any)) continue;
@@ -285,9 +295,6 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
     }
 }
 
-__device__ __forceinline__ void gg_table(u32* table) {
-    for (u32 i = threadIdx.x; i < 512; i += blockDim.x) table[i] = IQ3S_GRID[i];
-}
 
 // y_j = W x_j, j < m: x rows xs floats apart, y rows ys apart (matvec_cols_*, kernels/matvec.cu:677).  A workgroup takes the
 // tiles blockIdx.x, blockIdx.x + gridDim.x, .. of 16 rows (at most GG_TILES); its W waves take the chunks w, w + W, .. of the row
@@ -321,7 +328,7 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
         if (c == wave) {
             cur.load(w, rb, 16 * blockIdx.x, rows, start(c), lane);   // W <= nc
             if constexpr (F::grid) {
-                gg_table(table);
+                for (u32 i = threadIdx.x; i < 512; i += blockDim.x) table[i] = IQ3S_GRID[i];
                 __syncthreads();
             }
         }
@@ -353,10 +360,11 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
     __syncthreads();
     for (u32 i = threadIdx.x; i < nt * NG * 64; i += blockDim.x) {
         const u32 t = i / (NG * 64), G = i / 64 % NG, l = i & 63;
+        const u32 r = 16 * (blockIdx.x + t * gridDim.x) + (l & 15), j = 4 * G + (l >> 4);
+        if (r >= rows || j >= m) continue;
         float s = sums[i];
         for (u32 k = 1; k < W; k++) s += sums[k * SUMS + i];
-        const u32 r = 16 * (blockIdx.x + t * gridDim.x) + (l & 15), j = 4 * G + (l >> 4);
-        if (r < rows && j < m) y[(u64) j * ys + r] = s;
+        y[(u64) j * ys + r] = s;
     }
 }
 extern "C" __global__ void __launch_bounds__(1024, 4) matvec_cols_q8_0(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {

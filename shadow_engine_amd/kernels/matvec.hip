@@ -382,8 +382,11 @@ struct NoAfter {
 };
 
 // y = W x for the one input of GpuBackend::matvec: with a single input there is no decoded weight to share, so the vector unit alone
-// (no parts of the input to make first) answers sooner than the matrix cores: 3.6 us for 1024 rows of 2048 columns where
-// matvec_cols_q8_0 takes 5.5.  grid = ceil(rows / rpb), block 256, dynamic LDS rpb * row bytes + 32.
+// (no parts of the input to make first) answers a small product sooner than the matrix cores: 4.1 us from begin to end for 1024
+// rows of 2048 Q8_0 columns where matvec_cols_q8_0 takes 4.5, 8.4 and 9.5 for 2048 x 8192 (IQ3_S 4.3 and 5.3, 8.0 and 10.3; for
+// 8201 rows of 3072 it is 11.4 and 9.5).  matvec_cols has one form for every number of inputs all the same: an input's bits
+// must not depend on what it is batched with, and these sums are in another order.  grid = ceil(rows / rpb), block 256, dynamic
+// LDS rpb * row bytes + 32.
 template <class F>
 __device__ __forceinline__ void one_kernel(const u8* w, const float* x, float* y, u32 rows, u32 cols, u32 rpb) {
     const float* xp[1] = {x};
