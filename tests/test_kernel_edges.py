@@ -4,7 +4,7 @@ import pytest
 
 import oracle_lib as O
 import shadow_engine_amd as sz
-from shadow_engine_amd import synth
+from shadow_engine_amd import synth, synth_device
 from test_gpu_path import REL_L2, bits, build_layer, dense_matrix, dev, gguf_bound, gpu, oracle_layer, rel_l2  # noqa: F401 (gpu: the fixture)
 
 pytestmark = pytest.mark.gpu
@@ -216,3 +216,35 @@ def test_unquantized_rows_of_several_waves_and_longer(gpu, ty, rows, cols, m):  
     for j in range(m):
         assert rel_l2(got[j], O.matvec(ty, cols, rows, w, x[j])) <= 1e-5
     assert np.array_equal(bits(products(gpu, ty, rows, cols, w, x[m - 1:])), bits(got[m - 1:]))
+
+
+@pytest.mark.parametrize("m", [3, 8])
+def test_a_round_of_more_layers_than_its_buffers_hold(gpu, m):  # noqa: F811
+    """The EXL3 launches' sums are kept for as many layers as take 256 MiB (13 of this size): a round of 29 goes in three lots, whose
+    bounds lie inside the runs of one bit rate, and gives the bits of the layer-by-layer calls, which use the buffers' start."""
+    hidden, ff, ne, k, rates = 4096, 1536, 16, 16, [1, 2] * 14 + [2]
+    per = 2 * 8 * (k + 1) * (hidden // 512) * ff * 4 + 8 * (k + 1) * (ff // 512) * hidden * 4
+    assert (256 << 20) // per == 13
+    L, g = len(rates), gpu.Generator(device="cuda")
+    g.manual_seed(m)
+    s = sz.Session(hidden, ff, ne, k, L, 1024, 8)
+    bufs = {r: synth_device.exl3_layer(gpu, 7 + r, hidden, ff, ne, r, spaced=True) for r in (1, 2)}   # the layers differ by their inputs
+    for l, r in enumerate(rates):
+        buf, stride, gap = bufs[r]
+        s.set_layer(l, sz.EXL3(r), buf.data_ptr(), stride, sz.EXL3(r), buf.data_ptr() + ne * stride, gap=gap)
+    dhead = dev(gpu, synth.q8_0_matrix(np.random.default_rng(1), 1024, hidden))
+    s.set_head(sz.Q8_0, dhead.data_ptr())
+    u, rl, sgl, hu = (gpu.randn(sh, device="cuda", generator=g) for sh in ((L, m, hidden), (L, m, ne), (L, m), (m, hidden)))
+    one, y = (gpu.zeros((L, m, hidden), dtype=gpu.float32, device="cuda") for _ in range(2))
+    drafts, out = gpu.zeros(8, dtype=gpu.int32, device="cuda"), gpu.zeros(10, dtype=gpu.int32, device="cuda")
+    gpu.cuda.synchronize()
+    stream = sz.Stream()
+    for l in range(L):
+        s.moe_layer_verify(l, m, u[l].data_ptr(), rl[l].data_ptr(), sgl[l].data_ptr(), one[l].data_ptr(), stream.handle)
+    for replay in range(3):
+        s.verify_round(m, u.data_ptr(), rl.data_ptr(), sgl.data_ptr(), y.data_ptr(), hu.data_ptr(), drafts.data_ptr(), out.data_ptr(), stream.handle)
+        stream.synchronize()
+        assert gpu.all(gpu.isfinite(one)) and gpu.all(one.abs().amax(dim=2) > 0)
+        assert gpu.equal(y.view(gpu.int32), one.view(gpu.int32)), f"replay {replay}"
+        y.zero_()
+        gpu.cuda.synchronize()
