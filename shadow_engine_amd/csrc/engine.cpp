@@ -147,8 +147,17 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         const sz_arg a1[] = {P(scratch), P(w), P(y), U32(ys), U32((uint32_t) cols), U32((uint32_t) rows)};
         return launch("exl3_finish_rows", (uint32_t) rows / 128, m, 1, 64, 0, stream, a1);
     }
+    auto each_alone = [&]() -> int {   // a weight at a time, an input at a time
+        const std::string kn = "matvec_" + tag;
+        for (uint32_t j = 0; j < m; j++) {
+            const sz_arg a[] = {P(w), P(x + (uint64_t) j * xs * 4), P(y + (uint64_t) j * ys * 4), U32((uint32_t) rows), U32((uint32_t) cols)};
+            if (launch(cols ? kn.c_str() : "matvec_q8_0", ((uint32_t) rows + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
+        }
+        return 0;
+    };
+    if (f.dense && rows == 0) return 0;
+    if (cols == 0) return each_alone();   // empty sums, whatever the type: the launches below divide the columns up
     if (f.dense) {
-        if (rows == 0) return 0;
         if (cols % 4 || (x & 15) || xs % 4 || (w & (4 * f.bb - 1))) return fail("matvec_cols: unquantized matrices need columns in fours and aligned rows");
         // several passes a workgroup once there are more than about 1024 of them: the inputs stay in its registers
         const DenseShape d = dense_shape(cols);
@@ -158,15 +167,7 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         return launch(kn.c_str(), (uint32_t) ((rows + (uint64_t) d.pass * np - 1) / ((uint64_t) d.pass * np)), 1, 1, d.block, 0, stream, a);
     }
     if (cols % f.qk) return fail("matvec_cols: columns are not whole blocks");
-    if ((x & 15) || xs % 4) {
-        // any alignment: the one-weight-at-a-time kernel, an input at a time
-        const std::string kn = "matvec_" + tag;
-        for (uint32_t j = 0; j < m; j++) {
-            const sz_arg a[] = {P(w), P(x + (uint64_t) j * xs * 4), P(y + (uint64_t) j * ys * 4), U32((uint32_t) rows), U32((uint32_t) cols)};
-            if (launch(kn.c_str(), ((uint32_t) rows + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
-        }
-        return 0;
-    }
+    if ((x & 15) || xs % 4) return each_alone();   // any alignment
     // a wave a 256-column chunk, the same number of chunks a wave as far as they divide, up to 16 waves; as many workgroups as
     // the chip holds at a time (16 waves a CU), each with up to four tiles of 16 rows, which share the work on the inputs
     const uint32_t chunks = (uint32_t) ((cols + 255) / 256), each = (chunks + 15) / 16, waves = (chunks + each - 1) / each;

@@ -180,3 +180,13 @@ launched(3, "exl3_2")
 set_layer(1, sz.EXL3(2))
 s.verify_round(M, u, rl, sgl, y, hu, dr, out, 16)
 ''')
+
+
+@pytest.mark.parametrize("ty", ["sz.Q8_0", "sz.IQ3_S", "sz.F32", "sz.BF16"])
+def test_a_product_over_no_columns_is_launched_as_one(stub, ty):
+    """Rows of no columns are taken: every output is the empty sum, written by the kernel that takes a weight at a time."""
+    stub(f"""
+sz.matvec_cols({ty}, 256, 0, 100, 512, 0, 1024, 128, 3, 0, 0, 16)
+got = taken()
+assert [g[0] for g in got] == ["matvec_q8_0"] * 3 and [g[2][2:] for g in got] == [[1024 + 512 * j, 100, 0] for j in range(3)], got
+""")

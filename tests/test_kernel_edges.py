@@ -248,3 +248,11 @@ def test_a_round_of_more_layers_than_its_buffers_hold(gpu, m):  # noqa: F811
         assert gpu.equal(y.view(gpu.int32), one.view(gpu.int32)), f"replay {replay}"
         y.zero_()
         gpu.cuda.synchronize()
+
+
+@pytest.mark.parametrize("ty", [sz.Q8_0, sz.BF16])
+def test_products_over_no_columns_are_zero(gpu, ty):  # noqa: F811
+    y = gpu.full((3, 128), 7.5, dtype=gpu.float32, device="cuda")
+    sz.matvec_cols(ty, 0, 0, 100, 0, 0, y.data_ptr(), 128, 3)
+    gpu.cuda.synchronize()
+    assert gpu.all(y[:, :100] == 0.0) and gpu.all(y[:, 100:] == 7.5)
