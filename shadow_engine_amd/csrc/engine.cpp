@@ -109,8 +109,13 @@ struct DevBuf {
 };
 
 // The variant of a verify launch over `cols` output columns: column tiles a wave and the kernel name's prefix.  `waves8` is the
-// number of waves that 8 tiles a wave would give: they do least work for their A rows (a round of 48 layers 931 us, with 4 tiles
-// 957, with 2 1033) but leave SIMDs idle where there are few of them (a layer alone at 4 rows: 51 us with 2 tiles, 63 with 8).
+// number of waves that 8 tiles a wave would give: they do least work for their A rows but leave SIMDs idle where there are few of
+// them.  Measured with 2, 4 and 8 tiles throughout, at K = 3 and 1 to 8 rows, over layers of 512 experts of 512 (top-10), 128 of
+// 768 (top-8) and 32 of 1536 (top-4), and rounds of 4 and 16 of them: this choice is within 1.5 % of the best (at 8 rows of 4
+// layers of 512: 3 %).  E.g. 4 layers alone at 1, 4 and 8 rows of 512 experts: 97, 167 and 289 us with 2, 115, 172 and 274 with 4,
+// 162, 204 and 282 with 8, 97, 166 and 272 here; a round of 16 at 8 rows 734, 658, 617, 617 here; of 32 experts of 1536 1418,
+// 1214, 1100, 1095 here.  A projection alone (EXL3 at 4 bits) wants 2 tiles up to 8192 x 2048; at 8 inputs of 16384 x 4096 or 32768
+// x 2048 4 tiles would take 22 us a call where this takes 26.
 static const char* verify_variant(uint64_t cols, uint64_t waves8, uint32_t m, uint32_t* ct) {
     *ct = cols % 512 == 0 && waves8 >= 8192 ? 8 : cols % 256 == 0 && waves8 >= 2048 ? 4 : 2;
     if (m > 4) return *ct == 8 ? "w_" : *ct == 4 ? "t4w_" : "t2w_";
@@ -432,9 +437,10 @@ int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32
         plans += l * s->plan_stride;
         base = V.layer;
     }
-    // Layer by layer, tokens that share an expert are worth a launch that finds them only where they are many: about 6 us and
-    // a boundary, against the decode of a fifth of the pairs (measured at 4 rows of top-10 of 512, where they are one in twenty:
-    // 46 us a layer with the plan, 41 without).  A round's plans are one launch for all layers.
+    // Layer by layer, tokens that share an expert are worth a launch that finds them only where they are many: about 3 to 6 us
+    // and a boundary, against the decode of a fifth of the pairs.  Measured a layer with and without the plan: 45 and 42 us at 4
+    // rows of top-10 of 512 (distinct / pairs 0.97), 46.4 and 45.9 of top-8 of 128 (0.91), 68.7 and 70 of top-4 of 32 (0.83), 72
+    // and 75 at 8 rows of top-8 of 128 (0.80), 104 and 128 of top-4 of 32 (0.66).  A round's plans are one launch for all layers.
     const double pairs = (double) m * c.top_k, distinct = c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) m));
     const bool by_pair = one && distinct > 0.8 * pairs;
     const uint32_t ioff = by_pair ? 0 : vp.ioff, slots = by_pair ? m * c.top_k + 1 : vp.slots;

@@ -53,12 +53,12 @@ extern "C" int32_t sz_matvec_cols_static(int32_t ggml_type, uint64_t w, uint64_t
     int device = -1;
     if (hipGetDevice(&device) != hipSuccess) return sz::fail("sz_matvec_cols_static: hipGetDevice failed");
     if (sz::static_workspace_setup(device)) return 1;
-    // the size check comes before any launch: a product whose plan and partial sums do not fit the array is refused
+    // the size check comes before any launch: a product whose partial sums do not fit the array is refused
     const uint64_t need = sz_matvec_cols_scratch(ggml_type, cols, rows, m);
     if (need > SZ_STATIC_WORKSPACE_BYTES)
         return sz::fail("sz_matvec_cols_static: this product needs " + std::to_string(need) + " bytes of workspace, the static one holds " +
                         std::to_string((uint64_t) SZ_STATIC_WORKSPACE_BYTES) + "; use sz_matvec_cols with a workspace of the caller's");
-    // nothing in the workspace has to start at zero: the plan launch writes every table entry it reads and the partial sums
-    // are all written before the finishing launch adds them, so the last call's contents are simply overwritten
+    // nothing in the workspace has to start at zero: the partial sums are all written before the finishing launch adds them, so
+    // the last call's contents are simply overwritten
     return sz::matvec_cols_dev(ggml_type, w, cols, rows, x, xs, y, ys, m, (uint64_t) g_workspace[device].load(std::memory_order_acquire), SZ_STATIC_WORKSPACE_BYTES, stream);
 }

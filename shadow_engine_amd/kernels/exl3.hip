@@ -1,4 +1,4 @@
-// EXL3 (trellis-coded, Hadamard-rotated) matrix-vector products for 1..4 inputs, integer bit rates K = 1..8, codebook
+// EXL3 (trellis-coded, Hadamard-rotated) matrix-vector products for 1..8 inputs, bit rates K = 1..8 and K + 1/2 (K = 1..3), codebook
 // "mul1".  Format and arithmetic follow the CPU reference (crates/shadowzero-model/src/exl3.rs): a projection is a blob
 // [suh f16[in] | svh f16[out] | 4-byte marker | trellis], the trellis is [in/16][out/16] tiles of 16 K u16 words, a tile is
 // a ring of 256 K bits (most significant bit first inside little-endian u32 words) and weight t's 16-bit state ends at

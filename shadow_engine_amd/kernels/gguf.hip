@@ -300,7 +300,7 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
 // tiles blockIdx.x, blockIdx.x + gridDim.x, .. of 16 rows (at most GG_TILES); its W waves take the chunks w, w + W, .. of the row
 // (W by the number of chunks alone: the sums' order, so the bits, do not depend on m).  A row's last chunk, where it is short,
 // is its last 256 columns, the inputs of the ones that the chunk before has taken as zeros.  block 64 W, at most 1024; dynamic
-// LDS gg_cols_lds.
+// LDS: GG_STRIP and GG_TILES * NG * 64 words a wave.
 extern __shared__ __attribute__((aligned(16))) u32 sz_dyn_lds[];
 template <class F, int NG>
 __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 rows, u32 cols, u32 m) {
