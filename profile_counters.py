@@ -5,7 +5,9 @@ those keys are the keys of the sources it runs, so a kernel edit turns the quote
 have been run again.
 
 The passes, each a run of its own from the repository root after `cd /tmp && export TMPDIR=/tmp && cd <repo>`; W is a
-workload of bench.py, ARGS its flags (`--workload W`, nothing for the default one), D = PROF/W for a scratch directory PROF:
+workload of bench.py, ARGS its flags (`--workload W`, nothing for the default one), D = PROF/W for a scratch directory PROF
+(for a W that is a listed case of perf/cases.py the program is `profile_counters.py --run W N`: N passes through it, 100 for a trace,
+3 for counters, and there is no plain run and no memory pass):
 
     python3 bench.py ARGS --no-cpu-baseline --no-other-configs > D/plain.json                      (no profiler: the timings)
     rocprofv3 --kernel-trace --stats -d D/trace -o run -- python3 bench.py ARGS --steps 20 --warmup 3 --no-cpu-baseline --no-other-configs
@@ -28,12 +30,8 @@ import sqlite3
 import sys
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
-OURS = ("verify_", "decode_", "head_", "argmax_merge", "copy_", "matvec_", "route_", "swiglu", "moe_", "prefill_", "quant_act", "scatter_", "exl3_", "topk_", "proxy_")
+OURS = ("verify_", "decode_", "head_", "argmax_merge", "copy_", "matvec_", "route_", "swiglu", "moe_", "prefill_", "quant_act", "scatter_", "exl3_", "topk_", "proxy_", "router_", "hc_")
 NAMES = {"config5": ("verify_round_config5", "the default benchmark workload (config 5: 48-layer verify round on a 4-row batch, mixed EXL3 K in {2,3,4}, Q8_0 lm_head)", ""),
-         "config5_mode2": ("verify_round_config5_matrix_cores", "bench.py --expert-mode 2 (the config-5 round with the experts on the matrix cores: plan of distinct experts, f16 products, the linearised codebook)",
-                           " --expert-mode 2"),
-         "config5_mode3": ("verify_round_config5_f16_inputs", "bench.py --expert-mode 3 (the config-5 round with the exact launches' inputs rounded to f16, two products an instruction)",
-                           " --expert-mode 3"),
          "exl3prefill": ("prefill_chunk_exl3_k3", "bench.py --workload exl3prefill (prefill chunk: 512 tokens through 512 EXL3 K=3 experts + the shared one, f16 matrix cores)", " --workload exl3prefill"),
          "config3": ("verify_layer_and_head_config3", "bench.py --workload config3 (one EXL3 K=3 MoE layer for 4 tokens + Q8_0 head + acceptance)", " --workload config3"),
          "config1": ("matvec_q8_0_config1", "bench.py --workload config1 (one Q8_0 1024 x 2048 matrix-vector product)", " --workload config1"),
@@ -44,7 +42,12 @@ NAMES = {"config5": ("verify_round_config5", "the default benchmark workload (co
          "exl3top_screen": ("head_exl3_k4_top64_screened", "bench.py --workload exl3top --screen 128 (the same hand-off through the inexact 2-bit screen, 128 blocks a row)",
                             " --workload exl3top --screen 128"),
          "stage": ("stage_exl3_layer", "bench.py --workload stage (one EXL3 layer of a safetensors checkpoint staged into HBM)", " --workload stage"),
-         "snapshot": ("copy_ranges_snapshot", "bench.py --workload snapshot (73 device ranges saved and put back)", " --workload snapshot")}
+         "snapshot": ("copy_ranges_snapshot", "bench.py --workload snapshot (73 device ranges saved and put back)", " --workload snapshot"),
+         "cols-q8_0-5rows": ("matvec_cols_q8_0_5rows", "the case cols-q8_0-5rows of perf/cases.py (two Q8_0 products of 8201 x 3072 for 5 inputs a pass)", None),
+         "cols-exl3_4-4rows": ("matvec_cols_exl3_k4_4rows", "the case cols-exl3_4-4rows of perf/cases.py (four EXL3 K=4 projections of 4096 x 2048 for 4 inputs a pass)", None),
+         "block-q8_0-8rows": ("moe_block_q8_0_8rows", "the case block-q8_0-8rows of perf/cases.py (router and MoE block of four Q8_0 layers for 8 tokens a pass)", None),
+         "block-exl3_3-4rows": ("moe_block_exl3_k3_4rows", "the case block-exl3_3-4rows of perf/cases.py (router and MoE block of six EXL3 K=3 layers for 4 tokens a pass)", None),
+         "hyper-bf16-4rows": ("hyper_connection_bf16_4rows", "the case hyper-bf16-4rows of perf/cases.py (hyper-connection read and write, BF16, 4 streams of 2048, rank 320, 4 rows)", None)}
 SQ1 = "SQ_INSTS_VALU SQ_ACTIVE_INST_VALU SQ_BUSY_CYCLES SQ_WAVES SQ_WAVE_CYCLES SQ_WAIT_INST_ANY SQ_INSTS_SALU SQ_INSTS_LDS"
 SQ2 = "SQ_INSTS_MFMA SQ_VALU_MFMA_BUSY_CYCLES SQ_LDS_BANK_CONFLICT SQ_ACTIVE_INST_LDS SQ_INSTS_VMEM_RD SQ_WAIT_ANY SQ_ACTIVE_INST_ANY SQ_INSTS_VMEM_WR"
 L2 = "TCC_HIT_sum TCC_MISS_sum TCC_REQ_sum TCC_EA0_RDREQ_sum"
@@ -52,6 +55,23 @@ TAIL = " --no-cpu-baseline --no-other-configs"
 SHADER_ENGINES = 32          # SQ_BUSY_CYCLES is summed over the 32 shader engines (8 XCDs x 4)
 SIMDS = 1024
 PROF = "PROF"              # the directory the passes wrote to, as the summaries quote it in their commands
+
+
+def program(wl, args, steps, warmup, more=""):
+    """The program under the profiler, as the summaries quote it."""
+    if args is None:
+        return "python3 profile_counters.py --run %s %d" % (wl, 100 if steps == 20 else 3)
+    return "python3 bench.py%s --steps %d --warmup %d%s%s" % (args, steps, warmup, TAIL, more)
+
+
+def run_case(name, passes):
+    """`passes` passes through a listed case of perf/cases.py."""
+    import torch
+    from perf import cases
+    state = cases.prepare(next(c for c in cases.listed() if c["name"] == name), 1)
+    for _ in range(passes):
+        cases.run(state)
+    torch.cuda.synchronize()
 
 
 def rows(db, sql):
@@ -70,7 +90,7 @@ def clean(name):
     return name[:-3] if name.endswith(".kd") else name
 
 
-def trace_summary(d, plain, title, args):
+def trace_summary(d, plain, title, args, wl):
     r = rows(os.path.join(d, "trace", "run_results.db"),
              "select name, count(*), sum(duration), avg(duration), min(duration), max(duration) from kernels group by name order by 3 desc")
     r = [(clean(n), c, t, a, mn, mx) for n, c, t, a, mn, mx in r if ours(clean(n))]
@@ -78,7 +98,7 @@ def trace_summary(d, plain, title, args):
     out = ["Kernel trace of %s on one MI355X." % title,
            "Command (from the repository root after cd /tmp && export TMPDIR=/tmp && cd <repo>; the rocpd database it writes is summarised by",
            "python3 profile_counters.py with: select name, count(*), sum(duration), avg, min, max from kernels group by name):",
-           "  rocprofv3 --kernel-trace --stats -d %s/W/trace -o run -- python3 bench.py%s --steps 20 --warmup 3%s" % (PROF, args, TAIL), "",
+           "  rocprofv3 --kernel-trace --stats -d %s/W/trace -o run -- %s" % (PROF, program(wl, args, 20, 3)), "",
            "%-28s %7s %12s %10s %10s %10s %7s" % ("kernel (this library's only)", "calls", "total_us", "avg_us", "min_us", "max_us", "pct")]
     for n, c, t, a, mn, mx in r:
         out.append("%-28s %7d %12.1f %10.2f %10.2f %10.2f %7.2f" % (n, c, t / 1e3, a / 1e3, mn / 1e3, mx / 1e3, 100 * t / tot))
@@ -133,16 +153,16 @@ def traffic_summary(d, plain, title, args):
     return "\n".join(out) + "\n", traffic, {"FETCH_SIZE": fs, "WRITE_SIZE": ws}
 
 
-def sq_summary(d, title, args):
+def sq_summary(d, title, args, wl):
     c = pmc(os.path.join(d, "sq", "run_results.db"))
     second = os.path.join(d, "sq2", "run_results.db")
     c2 = pmc(second) if os.path.exists(second) else {}
     out = ["Shader counters per launch of the kernels of %s on one MI355X." % title,
            "Commands (each from the repository root, after cd /tmp && export TMPDIR=/tmp && cd <repo>; averaged over a kernel's launches with",
            "select kernel_name, counter_name, count(*), avg(value), avg(duration) from counters_collection group by 1, 2):",
-           "  rocprofv3 --pmc %s -d %s/W/sq -o run -- python3 bench.py%s --steps 2 --warmup 1%s" % (SQ1, PROF, args, TAIL)]
+           "  rocprofv3 --pmc %s -d %s/W/sq -o run -- %s" % (SQ1, PROF, program(wl, args, 2, 1))]
     if c2:
-        out.append("  rocprofv3 --pmc %s -d %s/W/sq2 -o run -- python3 bench.py%s --steps 2 --warmup 1%s" % (SQ2, PROF, args, TAIL))
+        out.append("  rocprofv3 --pmc %s -d %s/W/sq2 -o run -- %s" % (SQ2, PROF, program(wl, args, 2, 1)))
     out += ["", "%-26s %6s %9s %12s %12s %10s %9s %7s %9s %10s" % ("kernel", "calls", "waves", "INSTS_VALU", "ACTIVE_VALU", "cycles", "us (pmc)", "GHz", "VALU busy", "wait-issue")]
     kernels = {}
     for k in sorted(c, key=lambda k: -c[k].get("SQ_INSTS_VALU", (0, 0, 0))[1] * c[k].get("SQ_INSTS_VALU", (0, 0, 0))[0]):
@@ -175,7 +195,7 @@ def sq_summary(d, title, args):
     if os.path.exists(third):
         c3 = pmc(third)
         out += ["", "The L2 caches (summed over the 8 XCDs' channels), averages a launch:",
-                "  rocprofv3 --pmc %s -d %s/W/l2 -o run -- python3 bench.py%s --steps 2 --warmup 1%s" % (L2, PROF, args, TAIL),
+                "  rocprofv3 --pmc %s -d %s/W/l2 -o run -- %s" % (L2, PROF, program(wl, args, 2, 1)),
                 "%-26s %14s %14s %14s %14s %9s" % ("kernel", "TCC_REQ", "TCC_HIT", "TCC_MISS", "EA0_RDREQ", "hit rate")]
         for k in kernels:
             v = c3.get(k)
@@ -214,12 +234,12 @@ def main(prof, out_dir):
             pass
         entry = {"kernels": {}}
         if os.path.exists(os.path.join(d, "trace", "run_results.db")):
-            text, durations = trace_summary(d, plain, title, args)
+            text, durations = trace_summary(d, plain, title, args, wl)
             open(os.path.join(out_dir, stem + "_kernel_trace.txt"), "w").write(text.replace("/W/", "/%s/" % wl))
             for k, us in durations.items():
                 entry["kernels"].setdefault(k, {})["trace_avg_us"] = round(us, 2)
         if os.path.exists(os.path.join(d, "sq", "run_results.db")):
-            text, ks = sq_summary(d, title, args)
+            text, ks = sq_summary(d, title, args, wl)
             open(os.path.join(out_dir, stem + "_shader_counters.txt"), "w").write(text.replace("/W/", "/%s/" % wl))
             for k, e in ks.items():
                 entry["kernels"].setdefault(k, {}).update(e)
@@ -242,4 +262,7 @@ if __name__ == "__main__":
     if len(sys.argv) < 2:
         print(__doc__)
         sys.exit(2)
+    if sys.argv[1] == "--run":
+        run_case(sys.argv[2], int(sys.argv[3]))
+        sys.exit(0)
     main(sys.argv[1], sys.argv[2] if len(sys.argv) > 2 else os.path.join(ROOT, "profiles"))
