@@ -1137,14 +1137,19 @@ __device__ __forceinline__ double lane_xor_f64(double v, u32 lane, int h) {
     }
     return __builtin_bit_cast(double, (u64) f32_bits(lo) | ((u64) f32_bits(hi) << 32));
 }
-__device__ __forceinline__ double wave_sum_f64(double v, u32 lane) {
-    v += lane_xor_f64(v, lane, 1);
-    v += lane_xor_f64(v, lane, 2);
-    v += lane_xor_f64(v, lane, 4);
-    v += lane_xor_f64(v, lane, 8);
-    v += lane_xor_f64(v, lane, 16);
-    v += lane_xor_f64(v, lane, 32);
-    return v;
+// Sums v[j] over the wave: lane l returns the sum of input l % M (the first log2 M steps halve the number of values a lane carries).
+template <int M>
+__device__ __forceinline__ double wave_sums_f64(double (&v)[M], u32 lane) {
+#pragma unroll
+    for (int h = 1; h < M; h *= 2) {
+        const bool up = lane & h;
+#pragma unroll
+        for (int p = 0; p < M / (2 * h); p++) v[p] = (up ? v[2 * p + 1] : v[2 * p]) + lane_xor_f64(up ? v[2 * p] : v[2 * p + 1], lane, h);
+    }
+    double t = v[0];
+#pragma unroll
+    for (int h = M; h < 64; h *= 2) t += lane_xor_f64(t, lane, h);
+    return t;
 }
 
 // The lane's inputs normalised: (float) (r * scale) * norm weight, a chunk of them in one stream.
@@ -1173,8 +1178,7 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     const u32 cols = h * cs, kwn = dense_waves(cols), rw = (blockDim.x >> 6) / kwn, rg = wave / kwn;
     const S sl{wave - rg * kwn, kwn, 64, lane, cols};
     const u32 span = 64 * T::C, outer = (cols + kwn * span * S::NCH - 1) / (kwn * span * S::NCH);
-    const u32 pieces = outer * S::NCH * kwn;   // spans of 64 C columns, each one wave's
-    double* part = (double*) sz_dyn_lds;       // [m][cs][pieces of the widest stream]: the spans' sums of squares, in order
+    double* part = (double*) sz_dyn_lds;       // [m][cs][spans of 64 C columns a stream can touch]: their sums of squares, a span one wave's, in order
     const u32 wide = h / span + 2;
     double* scl = part + (u64) m * cs * wide;
     const bool live = rg < rw;
@@ -1205,13 +1209,11 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
                         for (int e = 0; e < (int) T::C; e++) sq[j] = __builtin_fma((double) xv[j][i * T::C + e], (double) xv[j][i * T::C + e], sq[j]);
                 }
                 for (u32 s = c0 / h; s <= (min(c0 + span, cols) - 1) / h; s++) {
+                    double of[M];
 #pragma unroll
-                    for (int j = 0; j < M; j++) {
-                        if ((u32) j < m) {
-                            const double ss = wave_sum_f64(mine == s ? sq[j] : 0.0, lane);
-                            if (lane == 0) part[((u64) j * cs + s) * wide + (c0 / span - s * h / span)] = ss;
-                        }
-                    }
+                    for (int j = 0; j < M; j++) of[j] = mine == s ? sq[j] : 0.0;
+                    const double ss = wave_sums_f64<M>(of, lane);
+                    if (lane < (u32) M && lane < m) part[((u64) lane * cs + s) * wide + (c0 / span - s * h / span)] = ss;
                 }
             }
         }
