@@ -146,8 +146,6 @@ def exl3_round(torch, sz, synth, synth_device, stream, L, rates, tag, mode=0):
     w.step, w.check, w.set_eager = step, check, (lambda eager: sess.set_graph(not eager))
     w.step_bytes = moe_bytes + head_bytes + act_bytes
     w.counters_key = "config5" if (L == 48 and tag == "config 5" and ROWS == 4) else ("config3" if (tag == "config 3" and ROWS == 4) else None)
-    if mode:
-        w.counters_key = "config5_mode%d" % mode if w.counters_key == "config5" else None
     w.cold_variant = tag == "config 3"
     w.dtype = "f32 accumulate over EXL3 f16 codebook weights / Q8_0 int8"
     w.describe = {"workload": "%s: verify round, %d MoE layer%s (hidden 2048, 512 experts + shared, top-10, EXL3 K in %s), %d-token batch, "
@@ -660,8 +658,7 @@ def main():
     ap.add_argument("--tokens", type=int, default=512, help="tokens of the prefill chunk (config4, exl3prefill; the configuration names 512)")
     ap.add_argument("--bits", type=int, default=0, help="bits a weight of the EXL3 head (exl3head, exl3top: 4 unless given) or of the chunk's experts (exl3prefill: 3)")
     ap.add_argument("--expert-mode", type=int, default=0, choices=[0, 1, 2, 3],
-                    help="config3, config5: 0 the exact EXL3 expert kernels (the library's default), 1 the matrix-core launches with the codebook's f16 values, "
-                         "2 with the linearised codebook, 3 the exact launches with their inputs rounded to f16 (two products an instruction)")
+                    help="config3, config5: the number given to sz_session_set_expert_mode (all of them run the same exact launches)")
     ap.add_argument("--screen", type=int, default=0, help="exl3top: blocks a row of the inexact 2-bit screen (0: the exact hand-off)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-other-configs", action="store_true", help="default workload only: do not time configurations 1-4 after it")
