@@ -256,3 +256,69 @@ def test_products_over_no_columns_are_zero(gpu, ty):  # noqa: F811
     sz.matvec_cols(ty, 0, 0, 100, 0, 0, y.data_ptr(), 128, 3)
     gpu.cuda.synchronize()
     assert gpu.all(y[:, :100] == 0.0) and gpu.all(y[:, 100:] == 7.5)
+
+
+@pytest.mark.parametrize("kb,half", [(k, False) for k in range(1, 9)] + [(k, True) for k in range(1, 4)])
+def test_every_tile_count_of_an_exl3_product_gives_the_same_bits(gpu, kb, half):  # noqa: F811
+    """2, 4 and 8 column tiles a wave and both widths of the input tile, launched by name (which one a call takes follows from its
+    size), on inputs that fill one block of 512 and a quarter of the next: the sums' order is the same, so are the bits; the
+    oracle's values."""
+    rng = np.random.default_rng(kb + 50 * half)
+    cols, rows, m = 640, 1024, 8
+    ty = sz.EXL3_HALF(kb) if half else sz.EXL3(kb)
+    tag = ("exl3h_%d" if half else "exl3_%d") % kb
+    w, x = synth.exl3_blob(rng, cols, rows, kb, half), rng.normal(size=(m, cols)).astype(np.float32)
+    dw, dx = dev(gpu, w), dev(gpu, x)
+    zs = (cols // 128 + 3) // 4
+    P, U = sz.Arg.ptr, sz.Arg.u32
+
+    def launched(form, ct, n):
+        part = gpu.full((n, zs, rows), float("nan"), dtype=gpu.float32, device="cuda")
+        y = gpu.zeros((n, rows), dtype=gpu.float32, device="cuda")
+        sz.launch("matvec_grouped_" + form + tag, (rows // (64 * ct), zs, 1), (256, 1, 1), 0, 0,
+                  [P(dw.data_ptr()), P(dx.data_ptr()), U(cols), P(part.data_ptr()), U(cols), U(rows), U(n)])
+        sz.launch("exl3_finish_rows", (rows // 128, n, 1), (64, 1, 1), 0, 0, [P(part.data_ptr()), P(dw.data_ptr()), P(y.data_ptr()), U(rows), U(cols), U(rows)])
+        gpu.cuda.synchronize()
+        return y.cpu().numpy()
+
+    first = launched("t2_", 2, 4)
+    for j in range(4):
+        assert rel_l2(first[j], O.exl3_matvec(cols, rows, kb, w, x[j], half=half)) <= 2e-6
+    for form, ct in (("t4_", 4), ("", 8)):
+        for n in (1, 3, 4):
+            assert np.array_equal(bits(launched(form, ct, n)), bits(first[:n])), (form, n)
+    for form, ct in (("t2w_", 2), ("t4w_", 4), ("w_", 8)):
+        for n in (5, 8):
+            got = launched(form, ct, n)
+            assert np.array_equal(bits(got[:4]), bits(first)), (form, n)
+            assert all(rel_l2(got[j], O.exl3_matvec(cols, rows, kb, w, x[j], half=half)) <= 2e-6 for j in range(4, n)), (form, n)
+
+
+@pytest.mark.parametrize("m", [4, 8])
+def test_a_deep_rounds_wide_tiles_give_the_bits_of_single_layers(gpu, m):  # noqa: F811
+    """64 layers of one rate: enough waves for 8 column tiles each (at 4 rows 4 in the down launch), where a single layer takes 2.
+    The bits agree in every layer, a sample of layers with the oracle."""
+    rng = np.random.default_rng(m)
+    hidden, ff, ne, k, L = 512, 512, 12, 4, 64
+    s = sz.Session(hidden, ff, ne, k, L, 1024, 8)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, sz.EXL3(3), hidden, ff, ne, True)      # the layers differ by their inputs
+    for l in range(L):
+        s.set_layer(l, sz.EXL3(3), dbuf.data_ptr(), stride, sz.EXL3(3), dbuf.data_ptr() + ne * stride)
+    dhead = dev(gpu, synth.q8_0_matrix(rng, 1024, hidden))
+    s.set_head(sz.Q8_0, dhead.data_ptr())
+    u, rl = rng.normal(size=(L, m, hidden)).astype(np.float32), rng.normal(size=(L, m, ne)).astype(np.float32)
+    sgl, hu = rng.normal(size=(L, m)).astype(np.float32), rng.normal(size=(m, hidden)).astype(np.float32)
+    du, drl, dsgl, dhu = dev(gpu, u), dev(gpu, rl), dev(gpu, sgl), dev(gpu, hu)
+    one, y = (gpu.zeros((L, m, hidden), dtype=gpu.float32, device="cuda") for _ in range(2))
+    drafts, out = gpu.zeros(8, dtype=gpu.int32, device="cuda"), gpu.zeros(10, dtype=gpu.int32, device="cuda")
+    gpu.cuda.synchronize()
+    stream = sz.Stream()
+    for l in range(L):
+        s.moe_layer_verify(l, m, du[l].data_ptr(), drl[l].data_ptr(), dsgl[l].data_ptr(), one[l].data_ptr(), stream.handle)
+    s.verify_round(m, du.data_ptr(), drl.data_ptr(), dsgl.data_ptr(), y.data_ptr(), dhu.data_ptr(), drafts.data_ptr(), out.data_ptr(), stream.handle)
+    stream.synchronize()
+    got = y.cpu().numpy()
+    assert np.array_equal(bits(got), bits(one.cpu().numpy()))
+    for l in (0, 31, 63):
+        want, _, _ = oracle_layer(sz.EXL3(3), hidden, ff, k, blobs, sh, rl[l], sgl[l], u[l])
+        assert all(rel_l2(got[l, j], want[j]) <= 2e-6 for j in range(m))
