@@ -72,6 +72,9 @@ DenseShape dense_shape(uint64_t cols) {
 const char* dense_m(uint32_t m) { return m == 1 ? "1" : m <= 4 ? "4" : "8"; }
 uint32_t dense_code(int ty) { return ty == SZ_TYPE_F32 ? 0 : ty == SZ_TYPE_F16 ? 1 : 2; }
 
+// Bytes of LDS a compute unit of the MI355X has.
+const uint32_t CU_LDS_BYTES = 160 * 1024;
+
 // Workgroups of a kernel that loops over its work (the head): a few per compute unit of the MI355X's 256.
 uint32_t persistent_groups() {
     static const uint32_t n = [] {
@@ -132,6 +135,14 @@ static uint64_t cols_scratch_bytes(const Format& f, uint64_t cols, uint64_t rows
     return align16(ng * 8) + align16(ng * 17 * 4) + ng * exl3_ksplit((uint32_t) cols) * 4 * rows * 4;
 }
 
+// The GGUF products of kernels/gguf.hip: a wave a 256-column chunk, the same number of chunks a wave as far as they divide, up to
+// 16 waves; the dynamic LDS of a workgroup of so many waves for `tiles` row tiles and 4 ng inputs.
+static uint32_t gguf_waves(uint64_t cols) {
+    const uint32_t chunks = (uint32_t) ((cols + 255) / 256), each = (chunks + 15) / 16;
+    return (chunks + each - 1) / each;
+}
+static uint32_t gguf_lds(uint32_t waves, uint32_t tiles, uint32_t ng) { return waves * (1584 * 4 + tiles * ng * 64 * 4); }
+
 int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x, uint32_t xs, uint64_t y, uint32_t ys, uint32_t m,
                            uint64_t scratch, uint64_t scratch_bytes, uint64_t stream) {
     Format f;
@@ -173,14 +184,14 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
     }
     if (cols % f.qk) return fail("matvec_cols: columns are not whole blocks");
     if ((x & 15) || xs % 4) return each_alone();   // any alignment
-    // a wave a 256-column chunk, the same number of chunks a wave as far as they divide, up to 16 waves; as many workgroups as
-    // the chip holds at a time (16 waves a CU), each with up to four tiles of 16 rows, which share the work on the inputs
-    const uint32_t chunks = (uint32_t) ((cols + 255) / 256), each = (chunks + 15) / 16, waves = (chunks + each - 1) / each;
+    // as many workgroups as the chip holds at a time (16 waves a CU), each with up to four tiles of 16 rows, which share the work
+    // on the inputs
+    const uint32_t waves = gguf_waves(cols);
     const uint32_t n16 = (uint32_t) ((rows + 15) / 16), slots = 256 * (16 / waves), rounds = (n16 + 4 * slots - 1) / (4 * slots);
     const uint32_t ng = m > 4 ? 2 : 1;
     const std::string kn = std::string("matvec_cols_") + (m > 4 ? "w_" : "") + tag;
     const sz_arg a[] = {P(w), P(x), U32(xs), P(y), U32(ys), U32((uint32_t) rows), U32((uint32_t) cols), U32(m)};
-    return launch(kn.c_str(), std::min(n16, rounds * slots), 1, 1, 64 * waves, waves * (1584 * 4 + 4 * ng * 64 * 4), stream, a);
+    return launch(kn.c_str(), std::min(n16, rounds * slots), 1, 1, 64 * waves, gguf_lds(waves, 4, ng), stream, a);
 }
 
 }   // namespace sz
@@ -478,6 +489,53 @@ int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32
     return 0;
 }
 
+// A layer of GGUF experts for several tokens, by distinct expert on the matrix cores (verify_items_* in kernels/gguf.hip).
+int verify_items(sz_session* s, const SzLayer& L, const std::string& tag, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t plan, uint64_t stream) {
+    const sz_session_config& c = s->cfg;
+    Format f;
+    std::string t;
+    format_of(L.type, f, t);
+    const uint64_t part = matrix_bytes(f, c.hidden, c.ff) + L.gap;   // from one projection of an expert to the next
+    if (part >> 32) return fail("sz_moe_layer_verify: a projection of 4 GiB or more");
+    // The plan is a launch of 4.5 us: worth it where it saves the decode of about 30 M weights (expected, for independent choices).
+    // Measured, us a layer with and without: 78.5 and 80.6 at 8 rows of top-10 of 512 Q8_0 experts of 2048 x 512 (17 M saved), 98.2
+    // and 92.9 at 6 rows of top-8 of 256 of 3072 x 768 (25 M), 87.5 and 87.2 at 8 rows of top-8 of 128 of 2560 x 768 (73 M), 296
+    // and 309 at 8 rows of top-12 of 512 of 3328 x 1536 (113 M), 55.6 and 85.5 at 8 rows of top-12 of 32 of 2048 x 512 (203 M).
+    const double pairs = (double) m * c.top_k, distinct = c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) m));
+    const char* form = std::getenv("SHADOWZERO_GGUF_ITEMS");
+    const bool by_pair = form ? std::strcmp(form, "pairs") == 0 : (pairs - distinct) * 3.0 * c.hidden * c.ff < 30e6;
+    const VerifyPlan vp = verify_plan(m, c.top_k);
+    const uint32_t ioff = by_pair ? 0 : vp.ioff, ng = m > 4 ? 2 : 1;
+    if (!by_pair) {
+        const sz_arg a[] = {P(rl), P(plan), U32(s->plan_stride), U32(vp.ioff), P(0), U64(L.shared), U32(0), U32(c.n_expert), U32(c.top_k), U32(m)};
+        if (launch("verify_plan_exl3", 1, 1, 1, 64 * m, 0, stream, a)) return 1;
+    }
+    // Row tiles a workgroup: more of them share the inputs' parts and a start worth about 5.5 tiles, fewer fill the chip.  Over 14
+    // layers of both formats the choice is within 5 % of the best of 2, 4 and 8 (8 rows of top-8 of 128 Q8_0 experts of 2560 x 768: 100,
+    // 88.1 and 87.5 us; 2 rows of top-10 of 512 IQ3_S experts of 2048 x 512: 33.3, 31.9 and 32.7).
+    const double items = (by_pair ? pairs : distinct) + (L.shared ? 1 : 0);
+    auto product = [&](const char* name, uint64_t in, uint64_t out, uint32_t tiles, uint32_t slots, uint32_t cols) {
+        const uint32_t waves = gguf_waves(cols);
+        uint32_t each = 0;
+        double best = 1e30;
+        for (uint32_t e = 8; e >= 2; e /= 2) {
+            if (gguf_lds(waves, e, ng) > CU_LDS_BYTES - 4096) continue;
+            const double cost = std::max(1.0, items * ((tiles + e - 1) / e) / (256 * (16 / waves))) * (e + 5.5);
+            if (cost < best) best = cost, each = e;
+        }
+        const sz_arg a[] = {P(rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), U32(ioff), P(in), P(out), U32(c.n_expert), U32(c.top_k), U32(m),
+                            U32(c.hidden), U32(c.ff)};
+        return launch((name + std::string(m > 4 ? "w_" : "") + tag).c_str(), (tiles + each - 1) / each, slots, 1, 64 * waves, gguf_lds(waves, each, ng), stream, a);
+    };
+    // a slot past the items has the routing weights worked out: in the first launch behind a plan, else in the second
+    if (product("verify_items_gate_up_", u, s->eg.ptr, 2 * c.ff / 16, m * c.top_k + (by_pair ? 1 : 2), c.hidden)) return 1;
+    if (product("verify_items_down_", s->eg.ptr, s->eo.ptr, c.hidden / 16, m * c.top_k + (by_pair ? 2 : 1), c.ff)) return 1;
+    s->last_fused = true;
+    const uint64_t G4 = 4ull * m * c.top_k;
+    const sz_arg a[] = {P(y), P(s->eo.ptr), P(plan + G4), P(L.shared ? s->eo.ptr + (uint64_t) m * c.top_k * c.hidden * 4 : 0), P(sgl), P(plan + 2 * G4), U32(c.hidden), U32(c.top_k)};
+    return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, m, 1, 256, 0, stream, a);
+}
+
 int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t stream) {
     const sz_session_config& c = s->cfg;
     if (l >= s->layers.size() || !s->layers[l].set) return fail("sz_moe_layer_verify: layer " + std::to_string(l) + " has no experts set");
@@ -496,6 +554,15 @@ int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, ui
         s->last_fused = true;
         return verify_layers(s, L.vpos, L.vpos + 1, l, m, u, rl, sgl, y, plan, stream);
     }
+    // Several tokens: by distinct expert on the matrix cores (kernels/gguf.hip), unless the layer is so small that the vector kernels'
+    // shorter chains are over first.  Measured, us a layer of four in a row, vector kernels and matrix cores: Q8_0 at 31 M weights of
+    // (token, expert) pairs (128 experts of 2048 x 512, top-4, 2 rows) 22.4 and 21.3, at 19 M 18.6 and 22.7; IQ3_S at 71 M (60 of 3072 x
+    // 768, top-4, 2 rows) 35.3 and 29.1, at 69 M (512 of 2048 x 512, top-10, 2 rows) 30.3 and 31.6, at 104 M 40.1 and 32.7; 8 rows of
+    // top-8 of 128 Q8_0 experts of 2560 x 768 167 and 87.5.
+    const double pairs = (double) m * c.top_k, weights = 3.0 * c.hidden * c.ff;
+    const bool small = (pairs + (shared ? m : 0)) * weights < (L.type == SZ_TYPE_Q8_0 ? 25e6 : 70e6) && c.ff <= 4096;
+    const char* items = std::getenv("SHADOWZERO_GGUF_ITEMS");   // "plan" or "pairs": that form at any size
+    if (m > 1 && (!small || items) && !std::getenv("SHADOWZERO_GGUF_PLANNED")) return verify_items(s, L, tag, m, u, rl, sgl, y, plan, stream);
     const uint64_t addr = plan + p.a0, rec = plan + p.r0, wts = plan + p.w_off, cnt = plan + p.counts_off;
     const uint64_t addr_d = addr + 2ull * p.GT * 8, rec_d = rec + 2ull * p.GT * 17 * 4;
     const std::string kn = "matvec_grouped_" + tag;
@@ -638,9 +705,7 @@ int head_argmax_mfma(sz_session* s, uint32_t m, uint64_t u, uint64_t logits, uin
 bool head_is_exl3(const sz_session* s) { return s->head_type >= 1021 && s->head_type <= 1028; }
 
 // LDS of a workgroup of head_exl3_K for m rows: the four waves' 4-row rings (static; a row is 64 lanes x 4 words at K = 3 and
-// 4, x K words otherwise) and the A rows, 4 KiB for every 512 inputs and every two rows (dynamic).  A compute unit of the
-// MI355X has 160 KiB.
-const uint32_t CU_LDS_BYTES = 160 * 1024;
+// 4, x K words otherwise) and the A rows, 4 KiB for every 512 inputs and every two rows (dynamic).
 uint32_t exl3_head_lds_dynamic(uint32_t hidden, uint32_t m) { return 4 * ((hidden / 128 + 3) / 4) * ((m + 1) / 2) * 1024; }
 uint32_t exl3_head_lds(uint32_t bits, uint32_t hidden, uint32_t m) {
     const uint32_t stride = (bits == 3 || bits == 4) ? 4 : bits;

@@ -29,7 +29,6 @@ typedef u32 u32x4b __attribute__((ext_vector_type(4), aligned(2)));
 
 #define GG_PITCH 264                 /* f16 from one A row of the parts to the next: 256 and a shift of four banks */
 #define GG_STRIP (12 * GG_PITCH / 2) /* words of a wave's strip: four inputs' parts, then the weights */
-#define GG_TILES 4                   /* most row tiles of a workgroup */
 
 __device__ __forceinline__ f16x2 gg_pair(u32 v) { return __builtin_bit_cast(f16x2, v); }
 __device__ __forceinline__ u32 gg_bits(f16x2 v) { return __builtin_bit_cast(u32, v); }
@@ -263,15 +262,21 @@ __device__ __forceinline__ bool gg_split(const f32x4 (&v)[4], u32 n, u32* strip,
     return F::zeros && __builtin_amdgcn_ballot_w64(rest != 0) != 0;
 }
 
+// Sixteen rows of a matrix.
+struct GgTile {
+    const u8* w;
+    u32 first;
+};
+
 // The products of what the three parts leave of a chunk's inputs, on the vector unit and a row at a time, into the sums of the
-// workgroup's tiles: rare, so short rather than fast.  x: the chunk's columns of input 0 (the lane's four at 4 * lane), if
-// they are `mine` to add; w: the chunk's first block of row 0.
-template <class F, int NG>
-__device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 rows, u32 nt, const float* __restrict__ x, u32 xs, u32 m, bool mine, u32 lane, float* tot) {
+// workgroup's tiles: rare, so short rather than fast.  col: the lane's four columns, if they are `mine` to add; off: from a row's
+// first byte to the chunk's first block.
+template <class F, int NG, class Tile, class Input>
+__device__ __forceinline__ void gg_rest(Tile tile, u32 off, u32 rb, u32 rows, u32 nt, Input input, u32 col, u32 m, bool mine, u32 lane, float* tot) {
 #pragma unroll 1
     for (u32 j = 0; j < m; j++) {
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (mine) v = *(const f32x4*) (x + (u64) j * xs + 4 * lane);
+        if (mine) v = *(const f32x4*) (input(j) + col);
         float scale, inv;
         const u32 mx = gg_most(v);
         if (mx >= 0x7f800000u) continue;   // nothing finite comes of it
@@ -286,8 +291,9 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
         if (!__builtin_amdgcn_ballot_w64(any)) continue;
 #pragma unroll 1
         for (u32 i = 0; i < 16 * nt; i++) {
-            const u32 row = 16 * (blockIdx.x + i / 16 * gridDim.x) + i % 16;
-            float s = mine && row < rows ? F::four(w + (u64) row * rb, 4 * lane, v) : 0.0f;
+            const GgTile t = tile(i / 16);
+            const u32 row = t.first + i % 16;
+            float s = mine && row < rows ? F::four(t.w + (u64) row * rb + off, 4 * lane, v) : 0.0f;
             s = seg_sum<64>(s, lane);
             float* at = tot + (i / 16 * NG + j / 4) * 64;
             if (lane == 16 * (j & 3) + i % 16) *at = __builtin_fmaf(s, inv, *at);
@@ -295,23 +301,19 @@ __device__ __forceinline__ void gg_rest(const u8* __restrict__ w, u32 rb, u32 ro
     }
 }
 
-
-// y_j = W x_j, j < m: x rows xs floats apart, y rows ys apart (matvec_cols_*, kernels/matvec.cu:677).  A workgroup takes the
-// tiles blockIdx.x, blockIdx.x + gridDim.x, .. of 16 rows (at most GG_TILES); its W waves take the chunks w, w + W, .. of the row
-// (W by the number of chunks alone: the sums' order, so the bits, do not depend on m).  A row's last chunk, where it is short,
-// is its last 256 columns, the inputs of the ones that the chunk before has taken as zeros.  block 64 W, at most 1024; dynamic
-// LDS: GG_STRIP and GG_TILES * NG * 64 words a wave.
 extern __shared__ __attribute__((aligned(16))) u32 sz_dyn_lds[];
-template <class F, int NG>
-__device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 rows, u32 cols, u32 m) {
-    __shared__ u32 table[F::grid ? 512 : 1];
-    constexpr u32 SUMS = GG_TILES * NG * 64;
+
+// The sums of a workgroup: nt tiles of 16 rows (tile(t): the matrix and the first of the 16) for m inputs of `cols`
+// columns (input(j): its first).  Its W waves take the chunks w, w + W, .. of the row (W by the number of chunks alone: the sums'
+// order, so the bits, do not depend on m).  A row's last chunk, where it is short, is its last 256 columns, the inputs of the ones
+// that the chunk before has taken as zeros.  Ends with the waves' sums in LDS behind a barrier; gg_total adds them up.
+// Dynamic LDS: GG_STRIP and nt * NG * 64 words a wave; table: 512 words of a format with a grid.
+template <class F, int NG, class Tile, class Input>
+__device__ __forceinline__ void gg_sums(Tile tile, u32 nt, u32 rows, Input input, u32 m, u32 cols, u32* table) {
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, W = blockDim.x >> 6;
-    const u32 rb = cols / F::QK * F::BB, nc = (cols + 255) / 256, n16 = (rows + 15) / 16;
-    const u32 nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
+    const u32 rb = cols / F::QK * F::BB, nc = (cols + 255) / 256;
     u32* strip = sz_dyn_lds + wave * GG_STRIP;
-    float* sums = (float*) (sz_dyn_lds + W * GG_STRIP);   // [wave][tile][G][lane]
-    float* tot = sums + wave * SUMS + lane;               // a lane adds to its own places
+    float* tot = (float*) (sz_dyn_lds + W * GG_STRIP) + wave * (nt * NG * 64) + lane;   // [wave][tile][G][lane]: a lane adds to its own places
     auto start = [&](u32 c) { return cols < 256 ? 0u : min(256 * c, cols - 256); };
     F cur;
     cur.init(lane);
@@ -323,10 +325,11 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
 #pragma unroll
         for (int r = 0; r < 4 * NG; r++) {
             v[r >> 2][r & 3] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if ((u32) r < m && col >= 256 * c && col < cols) v[r >> 2][r & 3] = *(const f32x4*) (x + (u64) r * xs + col);
+            if ((u32) r < m && col >= 256 * c && col < cols) v[r >> 2][r & 3] = *(const f32x4*) (input(r) + col);
         }
         if (c == wave) {
-            cur.load(w, rb, 16 * blockIdx.x, rows, start(c), lane);   // W <= nc
+            const GgTile t0 = tile(0);
+            cur.load(t0.w, rb, t0.first, rows, start(c), lane);   // W <= nc
             if constexpr (F::grid) {
                 for (u32 i = threadIdx.x; i < 512; i += blockDim.x) table[i] = IQ3S_GRID[i];
                 __syncthreads();
@@ -338,11 +341,13 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
         for (int G = 0; G < NG; G++) left = gg_split<F>(v[G], m - min(m, 4u * G), strip, lane, a[G], iv[G]) || left;
 #pragma unroll 1
         for (u32 t = 0; t < nt; t++) {
-            const u32 first = 16 * (blockIdx.x + t * gridDim.x);
+            const GgTile tt = tile(t);
             F now = cur;
-            now.stage(strip, w, rb, first, rows, lane);
-            if (t + 1 < nt) cur.load(w, rb, first + 16 * gridDim.x, rows, start(c), lane);
-            else if (c + W < nc) cur.load(w, rb, 16 * blockIdx.x, rows, start(c + W), lane);
+            now.stage(strip, tt.w, rb, tt.first, rows, lane);
+            if (t + 1 < nt || c + W < nc) {
+                const GgTile next = tile(t + 1 < nt ? t + 1 : 0);
+                cur.load(next.w, rb, next.first, rows, start(t + 1 < nt ? c : c + W), lane);
+            }
             float out[NG];
 #pragma unroll
             for (int G = 0; G < NG; G++) out[G] = 0.0f;
@@ -354,17 +359,34 @@ __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* _
     }
     if constexpr (F::zeros) {
         if (left)
-            for (u32 c = wave; c < nc; c += W)
-                gg_rest<F, NG>(w + start(c) / F::QK * F::BB, rb, rows, nt, x + start(c), xs, m, start(c) + 4 * lane >= 256 * c && start(c) + 4 * lane < cols, lane, tot);
+            for (u32 c = wave; c < nc; c += W) {
+                const u32 col = start(c) + 4 * lane;
+                gg_rest<F, NG>(tile, start(c) / F::QK * F::BB, rb, rows, nt, input, col, m, col >= 256 * c && col < cols, lane, tot);
+            }
     }
     __syncthreads();
+}
+// Place i (tile * NG + G) * 64 + lane of the sums: row lane % 16 of the tile, input 4 G + lane / 16.
+template <int NG>
+__device__ __forceinline__ float gg_total(u32 i, u32 nt) {
+    const u32 W = blockDim.x >> 6;
+    const float* sums = (const float*) (sz_dyn_lds + W * GG_STRIP);
+    float s = sums[i];
+    for (u32 k = 1; k < W; k++) s += sums[k * (nt * NG * 64) + i];
+    return s;
+}
+
+// y_j = W x_j, j < m: x rows xs floats apart, y rows ys apart (matvec_cols_*, kernels/matvec.cu:677).  A workgroup takes the
+// tiles blockIdx.x, blockIdx.x + gridDim.x, .. of 16 rows (at most 4).  block 64 W, at most 1024.
+template <class F, int NG>
+__device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 rows, u32 cols, u32 m) {
+    __shared__ u32 table[F::grid ? 512 : 1];
+    const u32 n16 = (rows + 15) / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
+    gg_sums<F, NG>([&](u32 t) { return GgTile{w, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, rows, [&](u32 j) { return x + (u64) j * xs; }, m, cols, table);
     for (u32 i = threadIdx.x; i < nt * NG * 64; i += blockDim.x) {
         const u32 t = i / (NG * 64), G = i / 64 % NG, l = i & 63;
         const u32 r = 16 * (blockIdx.x + t * gridDim.x) + (l & 15), j = 4 * G + (l >> 4);
-        if (r >= rows || j >= m) continue;
-        float s = sums[i];
-        for (u32 k = 1; k < W; k++) s += sums[k * SUMS + i];
-        y[(u64) j * ys + r] = s;
+        if (r < rows && j < m) y[(u64) j * ys + r] = gg_total<NG>(i, nt);
     }
 }
 extern "C" __global__ void __launch_bounds__(1024, 4) matvec_cols_q8_0(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {
@@ -378,4 +400,174 @@ extern "C" __global__ void __launch_bounds__(1024, 4) matvec_cols_iq3_s(const u8
 }
 extern "C" __global__ void __launch_bounds__(1024, 4) matvec_cols_w_iq3_s(const u8* w, const float* x, u32 xs, float* y, u32 ys, u32 rows, u32 cols, u32 m) {
     gg_cols<GgIq3, 2>(w, x, xs, y, ys, rows, cols, m);
+}
+
+// ------------------------------------------------------------------------------------- MoE layers for a batch, by distinct expert
+// The verify layer of GGUF experts for several tokens, on the products above: every distinct expert's weights are decoded once for
+// the tokens that chose it (route_plan in route.hip.h lists them).  Expert e's gate, up and down lie at experts + e stride + {0, part,
+// 2 part}, the shared one's at shared + the same.  A workgroup takes 2 to 8 row tiles of one expert (the host's choice), a wave a
+// 256-column chunk; the first launch has the same rows of gate and up and leaves silu(gate) * up.  Measured, 8 tokens of top-8 of 128
+// Q8_0 experts of 2560 x 768 (52 distinct): 49 us (4.4 TB/s) and 23 us (4.7 TB/s), where the vector unit took 110 and 50 pair by
+// pair: bound by the weights' way from memory.  The same layers of IQ3_S experts take 91 us (148), bound by the decode and its table
+// look-ups.  Requesting the inputs ahead of a pair's selection kept values across it in registers (78 -> 113) and lost 3 to 6 %.
+template <int N>
+struct GgInt {
+    static constexpr int value = N;
+};
+// An item of the plan: its expert's first byte, its tokens' rows and pair numbers.
+struct GgItem {
+    const u8* w;
+    u32 n;
+    u64 toks, pairs[2];
+    __device__ __forceinline__ u32 token(u32 r) const { return (u32) (toks >> (8 * r)) & 0xffu; }
+    __device__ __forceinline__ u32 pair(u32 r) const { return (u32) ((r < 4 ? pairs[0] : pairs[1]) >> (16 * (r & 3))) & 0xffffu; }
+};
+__device__ __forceinline__ u64 gg_uniform(u32 lo, u32 hi) { return (u64) (u32) __builtin_amdgcn_readfirstlane(lo) | ((u64) (u32) __builtin_amdgcn_readfirstlane(hi) << 32); }
+// Item `it` of the launch, if there is one.  ioff = 0: there is no plan; the items are the shared expert with all m tokens (0) and then
+// the (token, rank) pairs, whose expert select(pair) gives.  A token's sums do not depend on the other tokens of its item: both forms
+// give the same bits.
+template <class Select>
+__device__ __forceinline__ bool gg_item(const u8* __restrict__ pbuf, u32 ioff, u32 it, u64 experts, u64 stride, u64 shared, u32 k, u32 m, Select select, GgItem& item) {
+    u32 e = 0xffffffffu;
+    if (ioff) {
+        const u32* plan = (const u32*) (pbuf + ioff);
+        const u32x4 lo = *(const u32x4*) (plan + 4 + 8 * it), hi = *(const u32x4*) (plan + 8 + 8 * it);   // there for every slot, an item or not
+        if (it >= plan[0]) return false;
+        e = __builtin_amdgcn_readfirstlane(lo[0]);
+        item.n = __builtin_amdgcn_readfirstlane(lo[1]);
+        item.toks = gg_uniform(lo[2], lo[3]);
+        item.pairs[0] = gg_uniform(hi[0], hi[1]);
+        item.pairs[1] = gg_uniform(hi[2], hi[3]);
+    } else if (it > 0) {
+        e = __builtin_amdgcn_readfirstlane(select(it - 1));
+        if (e == 0xffffffffu) return false;
+        item.n = 1;
+        item.toks = (it - 1) / k;
+        item.pairs[0] = it - 1;
+        item.pairs[1] = 0;
+    } else {
+        if (!shared) return false;
+        const u64 ones = 0x0001000100010001ull, first = 0x0003000200010000ull + ones * (m * k);
+        item.n = m;
+        item.toks = 0x0706050403020100ull;
+        item.pairs[0] = first;
+        item.pairs[1] = first + 4 * ones;
+    }
+    item.w = (const u8*) (e == 0xffffffffu ? shared : experts + e * stride);
+    return true;
+}
+
+// The routing weights and counts of the chosen experts, by a workgroup that has nothing else to do.
+__device__ __forceinline__ void gg_route_weights(const float* __restrict__ logits, u8* __restrict__ pbuf, u32 ne, u32 k, u32 m) {
+    const u32 lane = threadIdx.x & 63;
+    for (u32 j = threadIdx.x >> 6; j < m; j += blockDim.x >> 6) {
+        u32 kk;
+        const float wt = route_weights(logits + (u64) j * ne, ne, k, lane, (const u32*) pbuf + j * k, &kk);
+        if (lane < k) ((float*) (pbuf + m * k * 4))[j * k + lane] = wt;
+        if (lane == 0) ((u32*) (pbuf + 2 * m * k * 4))[j] = kk;
+    }
+}
+
+// Launch 2 (the plan is launch 1): act[pair][ff] = silu(gate) * up.  grid = (workgroups a projection, slots = m k + 2:
+// the last is never an item and has the routing weights and counts worked out instead), block 64 W as for gg_sums.
+// Without a plan (slots = m k + 1) a workgroup selects its pair's expert on one of its waves and launch 3 works the weights out.
+template <class F, int NG>
+__device__ __forceinline__ void gg_gate_up(const float* __restrict__ logits, u64 experts, u64 stride, u64 shared, u32 part, u8* __restrict__ pbuf, u32 ioff, const float* __restrict__ u,
+                                           float* __restrict__ act, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    __shared__ u32 table[F::grid ? 512 : 1];
+    __shared__ u32 top[16];
+    const u32 lane = threadIdx.x & 63;
+    if (ioff && blockIdx.y == gridDim.y - 1) {
+        if (blockIdx.x == 0) gg_route_weights(logits, pbuf, ne, k, m);
+        return;
+    }
+    GgItem it;
+    auto select = [&](u32 pair) {
+        const u32 j = pair / k, t = pair - j * k;
+        if (threadIdx.x < 64) {
+            __builtin_amdgcn_s_setprio(3);   // every other wave of the workgroup waits for this one
+            route_id_of_rank(logits + (u64) j * ne, ne, k, t, lane, (double*) sz_dyn_lds, top);   // only top[t] is read
+            __builtin_amdgcn_s_setprio(0);
+            if (blockIdx.x == 0 && lane == 0) ((u32*) pbuf)[pair] = top[t];
+        }
+        __syncthreads();
+        return top[t];
+    };
+    if (!gg_item(pbuf, ioff, blockIdx.y, experts, stride, shared, k, m, select, it)) return;
+    const u32 n16 = ff / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
+    auto run = [&](auto ng) {
+        constexpr int N = decltype(ng)::value;
+        gg_sums<F, N>([&](u32 t) { return GgTile{it.w + (t & 1 ? part : 0u), 16 * (blockIdx.x + (t >> 1) * gridDim.x)}; }, 2 * nt, ff,
+                      [&](u32 r) { return u + (u64) it.token(r) * hidden; }, it.n, hidden, table);
+        for (u32 i = threadIdx.x; i < nt * N * 64; i += blockDim.x) {
+            const u32 t = i / (N * 64), l = i % (N * 64), r = l >> 4;
+            if (r >= it.n) continue;
+            const float g = gg_total<N>(2 * t * N * 64 + l, 2 * nt), up = gg_total<N>((2 * t + 1) * N * 64 + l, 2 * nt);
+            act[(u64) it.pair(r) * ff + 16 * (blockIdx.x + t * gridDim.x) + (l & 15)] = siluf_ref(g) * up;
+        }
+    };
+    if constexpr (NG > 1) {
+        if (it.n > 4) return run(GgInt<NG>());
+    }
+    run(GgInt<1>());
+}
+
+// Launch 3: eo[pair][hidden] = down act.  grid = (workgroups, slots = m k + 1, or without a plan m k + 2, the last one for the
+// weights), block as for gg_sums.
+template <class F, int NG>
+__device__ __forceinline__ void gg_down(const float* __restrict__ logits, u64 experts, u64 stride, u64 shared, u32 part, u8* __restrict__ pbuf, u32 ioff, const float* __restrict__ act,
+                                        float* __restrict__ eo, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    __shared__ u32 table[F::grid ? 512 : 1];
+    if (!ioff && blockIdx.y == gridDim.y - 1) {
+        if (blockIdx.x == 0) gg_route_weights(logits, pbuf, ne, k, m);
+        return;
+    }
+    GgItem it;
+    if (!gg_item(pbuf, ioff, blockIdx.y, experts, stride, shared, k, m, [&](u32 pair) { return ((const u32*) pbuf)[pair]; }, it)) return;
+    const u32 n16 = hidden / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
+    auto run = [&](auto ng) {
+        constexpr int N = decltype(ng)::value;
+        gg_sums<F, N>([&](u32 t) { return GgTile{it.w + 2 * (u64) part, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, hidden,
+                      [&](u32 r) { return act + (u64) it.pair(r) * ff; }, it.n, ff, table);
+        for (u32 i = threadIdx.x; i < nt * N * 64; i += blockDim.x) {
+            const u32 t = i / (N * 64), l = i % (N * 64), r = l >> 4;
+            if (r < it.n) eo[(u64) it.pair(r) * hidden + 16 * (blockIdx.x + t * gridDim.x) + (l & 15)] = gg_total<N>(i, nt);
+        }
+    };
+    if constexpr (NG > 1) {
+        if (it.n > 4) return run(GgInt<NG>());
+    }
+    run(GgInt<1>());
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_gate_up_q8_0(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* u, float* act,
+                                                                              u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    gg_gate_up<GgQ8, 1>(logits, experts, stride, shared, part, pbuf, ioff, u, act, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_down_q8_0(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* act, float* eo, u32 ne, u32 k,
+                                                                           u32 m, u32 hidden, u32 ff) {
+    gg_down<GgQ8, 1>(logits, experts, stride, shared, part, pbuf, ioff, act, eo, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_gate_up_w_q8_0(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* u, float* act,
+                                                                              u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    gg_gate_up<GgQ8, 2>(logits, experts, stride, shared, part, pbuf, ioff, u, act, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_down_w_q8_0(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* act, float* eo, u32 ne, u32 k,
+                                                                           u32 m, u32 hidden, u32 ff) {
+    gg_down<GgQ8, 2>(logits, experts, stride, shared, part, pbuf, ioff, act, eo, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_gate_up_iq3_s(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* u, float* act,
+                                                                              u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    gg_gate_up<GgIq3, 1>(logits, experts, stride, shared, part, pbuf, ioff, u, act, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_down_iq3_s(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* act, float* eo, u32 ne, u32 k,
+                                                                           u32 m, u32 hidden, u32 ff) {
+    gg_down<GgIq3, 1>(logits, experts, stride, shared, part, pbuf, ioff, act, eo, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_gate_up_w_iq3_s(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* u, float* act,
+                                                                              u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
+    gg_gate_up<GgIq3, 2>(logits, experts, stride, shared, part, pbuf, ioff, u, act, ne, k, m, hidden, ff);
+}
+extern "C" __global__ void __launch_bounds__(1024, 4) verify_items_down_w_iq3_s(const float* logits, u64 experts, u64 stride, u64 shared, u32 part, u8* pbuf, u32 ioff, const float* act, float* eo, u32 ne, u32 k,
+                                                                           u32 m, u32 hidden, u32 ff) {
+    gg_down<GgIq3, 2>(logits, experts, stride, shared, part, pbuf, ioff, act, eo, ne, k, m, hidden, ff);
 }

@@ -322,3 +322,36 @@ def test_a_deep_rounds_wide_tiles_give_the_bits_of_single_layers(gpu, m):  # noq
     for l in (0, 31, 63):
         want, _, _ = oracle_layer(sz.EXL3(3), hidden, ff, k, blobs, sh, rl[l], sgl[l], u[l])
         assert all(rel_l2(got[l, j], want[j]) <= 2e-6 for j in range(m))
+
+
+@pytest.mark.parametrize("ty", [sz.Q8_0, sz.IQ3_S])
+@pytest.mark.parametrize("hidden,ff,ne,k,m,shared,finite", [
+    (256, 256, 6, 2, 2, True, 6),       # one chunk a row: one wave a workgroup
+    (2560, 768, 12, 4, 8, False, 12),   # experts of more than four tokens beside experts of one
+    (4096, 512, 5, 3, 7, True, 5),      # 16 waves of 8 inputs: the most LDS a workgroup takes
+    (4352, 1280, 4, 2, 3, True, 4),     # 17 chunks on 9 waves, tiles that do not divide among the workgroups
+    (512, 4608, 4, 2, 5, True, 4),      # ff > 4096, and chunks on 9 waves in the down product
+    (768, 256, 24, 16, 4, True, 11),    # the most experts a token, some of them masked: ranks without one
+])
+def test_gguf_layers_by_distinct_expert(gpu, monkeypatch, ty, hidden, ff, ne, k, m, shared, finite):  # noqa: F811
+    """The layer on the matrix cores at the edges of its chunks, tiles and items, with a plan and pair by pair: the same bits, within
+    2e-6 relative L2 of the oracle (f32 sums in another order: 2^-24 of a term for each of a few dozen partial sums)."""
+    rng = np.random.default_rng(ty * 31 + hidden + m)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, shared)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty if shared else 0, dbuf.data_ptr() + ne * stride if shared else 0)
+    u, logits, sgl = rng.normal(size=(m, hidden)).astype(np.float32), rng.normal(size=(m, ne)).astype(np.float32), rng.normal(size=m).astype(np.float32)
+    logits[0, finite:] = -np.inf
+    du, dl, dg = dev(gpu, u), dev(gpu, logits), dev(gpu, sgl)
+    want, widx, ww = oracle_layer(ty, hidden, ff, k, blobs, sh, logits, sgl, u)
+    outs = []
+    for form in ("plan", "pairs"):
+        monkeypatch.setenv("SHADOWZERO_GGUF_ITEMS", form)
+        dy = gpu.zeros((m, hidden), dtype=gpu.float32, device="cuda")
+        s.moe_layer_verify(0, m, du.data_ptr(), dl.data_ptr(), dg.data_ptr(), dy.data_ptr())
+        gpu.cuda.synchronize()
+        outs.append(dy.cpu().numpy())
+        idx, w = s.last_route(m)
+        assert np.array_equal(idx, widx) and np.allclose(w, ww, rtol=2e-6, atol=0)
+        assert max(rel_l2(outs[-1][j], want[j]) for j in range(m)) <= 2e-6
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
