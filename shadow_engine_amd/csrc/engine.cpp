@@ -4,9 +4,11 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "sz_internal.hpp"
@@ -379,9 +381,25 @@ struct sz_session {
         uint32_t k_blk = 0;
         DevBuf w_q2, w_sc, xq, x_sc, x_corr, bmax, seen, sel, logits;
     } hp;
+    // The prefill chunk's buffers: parts of one allocation, grown on demand and laid out anew by every chunk.
     struct {
-        DevBuf xq, xd, tidx, w, cnt, offs, list, items, hq, hd, eo, gup, arows, ainv;
-    } pf;   // the prefill chunk's buffers, grown on demand
+        struct Part {
+            uint64_t ptr = 0;
+        };
+        DevBuf mem;
+        Part xq, xd, tidx, w, cnt, offs, list, items, hq, hd, eo, amax, arows, ainv, drows, dinv;
+        int lay(std::initializer_list<std::pair<Part*, uint64_t>> parts) {
+            uint64_t n = 0;
+            for (const auto& p : parts) n += (p.second + 255) & ~255ull;
+            if (mem.need(n)) return 1;
+            n = mem.ptr;
+            for (const auto& p : parts) {
+                p.first->ptr = n;
+                n += (p.second + 255) & ~255ull;
+            }
+            return 0;
+        }
+    } pf;
     void* top_host = nullptr;  // pinned host memory the top-64 merge writes to directly (8 rows of 128 words): no copy back
     bool last_fused = false;   // the last layer call left its routing in the fused layout [tidx | w | cnt]
     uint64_t last_plan = 0;    // the plan the last layer call left its routing in
@@ -1066,7 +1084,7 @@ int32_t sz_session_set_head_proxy(sz_session* s, uint32_t k_blk) {
 uint64_t sz_session_buffer(sz_session* s, int32_t which) {
     if (!s) return 0;
     const uint64_t at[] = {s->last_plan ? s->last_plan : s->plan.ptr, s->part.ptr, s->dn.ptr, s->eg.ptr, s->eo.ptr, s->hp.w_q2.ptr, s->hp.w_sc.ptr, s->hp.xq.ptr, s->hp.x_sc.ptr,
-                           s->hp.x_corr.ptr, s->hp.bmax.ptr, s->hp.sel.ptr, s->hp.logits.ptr, s->pf.gup.ptr, s->pf.eo.ptr, s->pf.arows.ptr, s->pf.ainv.ptr, s->pf.items.ptr};
+                           s->hp.x_corr.ptr, s->hp.bmax.ptr, s->hp.sel.ptr, s->hp.logits.ptr, s->pf.arows.ptr, s->pf.eo.ptr, s->pf.drows.ptr, s->pf.dinv.ptr, s->pf.items.ptr};
     return which >= 0 && which < (int32_t) (sizeof at / sizeof at[0]) ? at[which] : 0;
 }
 
@@ -1260,61 +1278,74 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
     const uint64_t T = tokens, k = c.top_k, np = T * k, rows = np + (shared ? T : 0);
     auto& pb = s->pf;
     if (exl3) {
-        // EXL3 experts: f16 activations on the columns of the matrix instruction, the rotations on the matrix cores too, items of
-        // up to `tok` pairs (kernels/exl3.hip, "the prefill chunk of an EXL3 layer": XPF_NT, XPF_TOK, XPF_LDS_WORDS)
+        // EXL3 experts: f16 activations on the columns of the matrix instruction, items of up to 128 pairs, of 64 for the down
+        // products (kernels/exl3.hip, "the prefill chunk of an EXL3 layer": XPF_NT, XPF_DOWN_NT, XPF_ROWS_U16, XPF_RING)
         if (c.ff > 512) return fail("sz_moe_prefill_chunk: EXL3 experts of more than 512 intermediate features are not built (a workgroup keeps four 128-blocks of a token)");
-        const uint32_t zs = (c.hidden / 128 + 3) / 4;
-        const uint32_t tok = 16 * (f.bits <= 7 ? 3 : 2), depth = f.bits <= 2 ? 8 : f.bits <= 5 ? 6 : 4;   // XPF_NT, XPF_D
-        const uint64_t max_items = c.n_expert + 1 + rows / tok;
-        if (pb.tidx.need(np * 4) || pb.w.need(np * 4) || pb.cnt.need(T * 4) || pb.offs.need((c.n_expert + 2) * 4ull) || pb.list.need(rows * 4) ||
-            pb.items.need((2 + 4 * max_items) * 4) || pb.gup.need(2ull * rows * zs * c.ff * 4) || pb.eo.need(rows * c.hidden * 4) ||
-            pb.arows.need(max_items * tok * 1024) || pb.ainv.need(max_items * tok * 4))
+        const uint32_t most = f.bits <= 5 ? 8 : 6, tok = 16 * most, kbs = c.hidden / 128, fbs = c.ff / 128, ntl = std::min<uint32_t>(most, (tokens + 15) / 16);
+        const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1, max_items = some + rows / tok, max_down = some + rows / 64, tiles = rows / 16 + c.n_expert + 2;
+        const uint32_t bound = (uint32_t) ((max_items + 7) / 8 * 8), bound_d = (uint32_t) ((max_down + 7) / 8 * 8);   // workgroups an item's part (xpf_place)
+        if (pb.lay({{&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4}, {&pb.items, (2 + 2 * max_items + 2 * max_down) * 4},
+                    {&pb.eo, rows * c.hidden * 4}, {&pb.amax, T * 4}, {&pb.arows, tiles * 2 * kbs * 4096}, {&pb.ainv, tiles * 2 * 64}, {&pb.drows, tiles * fbs * 4096}, {&pb.dinv, tiles * fbs * 64}}))
             return 1;
         const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0, items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
         {
-            const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
+            const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens), P(x), P(pb.amax.ptr), U32(c.hidden)};
             if (launch("route_topk_rows", (tokens + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
         }
         {
-            const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.cnt.ptr),
-                                P(pb.items.ptr), P(items_d), U32(tok), U32(tok)};
+            const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr),
+                                P(pb.items.ptr), P(items_d), U32(tok), U32(64)};
             if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
         }
-        const uint32_t stride = (f.bits == 3 || f.bits == 4) ? 4 : (uint32_t) f.bits;
-        const uint32_t lds = 4 * (tok / 16 * 4096 + 4 * (depth * 64 * stride) + 2 * tok + 4 * tok + tok);   // XPF_LDS_WORDS
         {
-            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(x), P(pb.gup.ptr), U32(c.n_expert), U32(c.top_k),
-                                U32((uint32_t) np), U32((uint32_t) rows), U32(c.hidden), U32(c.ff)};
-            if (launch(("prefill_gate_up_" + tag).c_str(), (uint32_t) max_items, 2 * zs, 1, 256, lds, stream, a)) return 1;
+            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(x), P(pb.amax.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), U32(c.n_expert),
+                                U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(tok), U32(ntl)};
+            if (launch("prefill_rotate_exl3", bound * ntl, 1, 1, 256, 0, stream, a)) return 1;
+        }
+        const uint32_t nt = ntl <= 2 ? ntl : ntl + ntl % 2, bits = (uint32_t) f.bits, wide_ring = bits <= 7 ? 3 : 2;
+        {
+            // two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, where the items are few, fills the
+            // chip (3 bits, 512 experts of 2048 x 512, top-10: 45 tokens 102 and 120 us, 200 tokens 183 and 179, 512 262 and 256, 1024 381
+            // and 346; 600 tokens through 60 of 1024 x 256, top-8: 106 and 120; 1500 through 32 of 2048 x 512, top-4: 226 and 212)
+            const bool wide = rows * fbs >= 16000;
+            const uint32_t ncb = wide ? 2 : 1;
+            // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING, XPF_RING_N), afterwards the exchange of four tiles' sums
+            uint32_t lds = ncb * 2 * std::min(4u, nt) * 8192;
+            for (uint32_t n = 1; n <= nt; n += n == 1 ? 1 : 2) {
+                const uint32_t deep = n <= 2 ? (bits <= 4 ? 8 : 12 - bits) : n == 4 ? (bits <= 5 ? 5 : 4) : wide_ring, ring = wide ? wide_ring : deep;
+                lds = std::max(lds, (wide ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
+            }
+            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff)};
+            if (launch(((wide ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 256 * ncb, lds, stream, a)) return 1;
         }
         {
-            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.gup.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), U32(c.n_expert),
-                                U32(c.top_k), U32((uint32_t) np), U32((uint32_t) rows), U32(c.hidden), U32(c.ff), U32(zs), U32(tok)};
-            if (launch("prefill_act_exl3", (uint32_t) max_items, tok / 16, 1, 256, 0, stream, a)) return 1;
-        }
-        {
-            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.eo.ptr), U32(c.n_expert),
-                                U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(c.ff)};
-            if (launch(("prefill_down_" + tag).c_str(), (uint32_t) max_items, (c.hidden / 128 + 3) / 4, 1, 256, lds, stream, a)) return 1;
+            // shares of an item: one wave a column block in the end where items are few, all blocks on eight waves, whose start then counts
+            // once, where they fill the chip (1, 2 shares of 8 waves, 4 of 4: 45 tokens as above 138, 111, 102 us, 512 tokens 261, 256, 272,
+            // 4096 at 4 bits 968, 986, 1059)
+            const bool wide = rows >= 1800;
+            const uint32_t waves = std::min(wide ? 8u : 4u, kbs), parts = std::max((kbs + 4 * waves - 1) / (4 * waves), std::min(rows >= 20000 ? 1u : wide ? 2u : 4u, kbs / waves)), nd = std::min(4u, nt);
+            const uint32_t ring = wide ? wide_ring : bits <= 4 ? 8 : bits <= 6 ? 6 : 4;   // XPF_RING, XPF_RING_DOWN_N
+            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(items_d), P(pb.drows.ptr), P(pb.dinv.ptr), P(pb.eo.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff),
+                                U32(nd), U32(parts)};
+            if (launch(((wide ? "prefill_down_" : "prefill_down_n_") + tag).c_str(), bound_d * parts, 1, 1, 64 * waves, 4 * (nd * fbs * 1040 + 256 * waves) + waves * ring * 512 * bits, stream, a)) return 1;
         }
         const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden), U32(c.top_k)};
         return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, tokens, 1, 256, 0, stream, a);
     }
     const uint64_t max_items = c.n_expert + 1 + rows / 64, max_items_d = c.n_expert + 1 + rows / 32;   // every expert's runs of up to 64 (32) pairs: PF_TOK, PF_TOK_D in kernels/prefill.hip
-    if (pb.xq.need(T * c.hidden) || pb.xd.need(T * c.hidden / 32 * 4) || pb.tidx.need(np * 4) || pb.w.need(np * 4) || pb.cnt.need(T * 4) ||
-        pb.offs.need((c.n_expert + 2) * 4ull) || pb.list.need(rows * 4) || pb.items.need((2 + 2 * max_items + 2 * max_items_d) * 4) || pb.hq.need(rows * c.ff) || pb.hd.need(rows * (c.ff / 32) * 4) ||
-        pb.eo.need(rows * c.hidden * 4))
+    if (pb.lay({{&pb.xq, T * c.hidden}, {&pb.xd, T * c.hidden / 32 * 4}, {&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4},
+                {&pb.items, (2 + 2 * max_items + 2 * max_items_d) * 4}, {&pb.hq, rows * c.ff}, {&pb.hd, rows * (c.ff / 32) * 4}, {&pb.eo, rows * c.hidden * 4}}))
         return 1;
     const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0;
     {
         // routing and quantization do not depend on each other: one launch
         const uint64_t n = T * c.hidden;
-        const sz_arg a[] = {P(x), U64(n), P(pb.xq.ptr), P(pb.xd.ptr), P(rl), P(pb.tidx.ptr), P(pb.w.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
+        const sz_arg a[] = {P(x), U64(n), P(pb.xq.ptr), P(pb.xd.ptr), P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
         if (launch("prefill_front", (tokens + 3) / 4 + (uint32_t) ((n / 32 + 255) / 256), 1, 1, 256, 0, stream, a)) return 1;
     }
     const uint64_t items_d = pb.items.ptr + (1 + 2 * max_items) * 4;   // the down kernel's items: runs of up to 32 pairs (PF_TOK_D)
     {
-        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.cnt.ptr), P(pb.items.ptr), P(items_d), U32(64), U32(32)};
+        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(items_d), U32(64), U32(32)};
         if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
     }
     {

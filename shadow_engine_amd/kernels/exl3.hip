@@ -308,13 +308,13 @@ __device__ __forceinline__ u64 uniform_u64(u64 v) {
 // A wave's stream of trellis rows for CT column tiles: units of 16 tiles (16 / CT tile rows, 512 K bytes), each brought
 // into one of D ring slots by NI global-to-LDS loads of 16 bytes a lane.  In LDS a unit lies packed in the order of the
 // bit stream: tile row, column tile, tile word.
-template <int K, bool H, int CT>
+template <int K, bool H, int CT, int DEPTH = 0>
 struct VerifyRing {
     static constexpr int TW = EXL3_TILE_WORDS(K, H), CH = TW / 4;   // words and 16-byte chunks a tile
     static constexpr int UR = 16 / CT;                              // tile rows a unit
     static constexpr int NI = (CH + 3) / 4;                         // loads a unit: 16 CH chunks, 64 a load, the last load perhaps partly
     static constexpr int UW = 64 * CH;                              // words a unit
-    static constexpr int D = CH <= 8 ? 3 : 2;
+    static constexpr int D = DEPTH ? DEPTH : CH <= 8 ? 3 : 2;
     u64 row0;         // the wave's first tile row, at its first column tile (uniform)
     u32 pitch;        // bytes between tile rows
     u32 units, lds;
@@ -1457,70 +1457,41 @@ EXL3_HEAD_ENTRIES(7)
 EXL3_HEAD_ENTRIES(8)
 
 // ------------------------------------------------------------------------ the prefill chunk of an EXL3 layer (matrix cores)
-// A chunk's tokens grouped by expert (prefill_group in kernels/prefill.hip: runs of up to XPF_TOK(K) (token, rank) pairs of
+// A chunk's tokens grouped by expert (prefill_group in kernels/prefill.hip: runs of up to 16 XPF_NT (token, rank) pairs of
 // one expert are a work item) through gate/up, the activation and down with the item's tokens on the columns of the matrix
 // instruction: an expert's weights are decoded once for all tokens of an item (the reference's mma_grouped_exl3_pre_K,
-// kernels/exl3.cu:684,704,724, with groups of 64, session.rs:5159-5189).  The rotations of the format run on the matrix
-// cores too: H (x * suh) is a product with the 128 x 128 matrix of signs, whose 16 x 16 x 16 operands a lane makes from
-// its own lane number (H[i][j] = (-1)^popcount(i & j): a tile of it is a per-lane pattern times the parity of the two
-// tile numbers).  Every product here has the tokens on the columns (operand B, lane 16 a + n: token n, inputs 4 a .. 4 a
-// + 3) and its result on the same lanes as (token n, outputs 4 a .. 4 a + 3): a result is the next product's operand as
-// it lies, nothing is transposed.  Inputs of a rotation ride as an f16 high and an f16 low part, scaled by a power of two
-// per token; the rotated values as single f16 values (the reference converts to f16 unscaled); weights are the
-// codebook's own f16 values; sums are f32.  Against the exact arithmetic the f16 roundings of the activations cost about
-// 4e-4 relative L2 of a layer's output (bound of the path: 1e-3).
+// kernels/exl3.cu:684,704,724, with groups of 64, session.rs:5159-5189).  Every product has the tokens on the columns (operand
+// B, lane 16 a + n: token n) and its result on the same lanes as (token n, outputs 4 a .. 4 a + 3).  Inputs ride as single f16
+// values after their rotation, scaled by a power of two per token (the reference converts to f16 unscaled); weights are the
+// codebook's own f16 values; sums are f32.  Against the exact arithmetic the f16 roundings of the activations cost about 4e-4
+// relative L2 of a layer's output (bound of the path: 1e-3).
 //
-// Three launches a layer.  1: (item, gate | up, share z of the inputs): the x rotation and the products, raw partial sums
-// to memory.  2: (item, tile of 16 tokens): the partial sums added up, the output-side transforms and scales of gate and
-// up, act = silu(gate) * up, its rotation into the down projection's basis, left as the f16 operand rows of launch 3.
-// 3: (item, four 128-column blocks of hidden): the products, the output side, the pairs' rows of the layer's result.
+// Three launches a layer.  1 (prefill_rotate_exl3): the inputs of every item through the input sides of its expert's gate and
+// up, left as operand rows.  2 (prefill_gate_up_exl3_K): the products over all inputs, both output sides, act = silu(gate) * up and
+// its rotation into the down projection's basis, as operand rows again.  3 (prefill_down_exl3_K): the products, the output
+// side, the pairs' rows of the layer's result.
+// What a token's numbers are does not depend on the item, the workgroup's shape or the other tokens: the sums over the inputs are
+// one chain, in the order of the tile rows, and a power of two is a token's (launch 1) or a token's and 128-block's (launch 2).
+//
+// What bounds it: the decode, 60 vector cycles for four weights a lane, an expert again for every item, and 9 more for each matrix instruction
+// (measured: of its 16 cycles a SIMD issues nothing else for 9, whichever wave it comes from), so few, large items; then the ends of a
+// workgroup, a third of launch 2's time.  4096 tokens through 512 experts of 2048 x 512 and the shared one at 4 bits, top-10: 130 + 385 +
+// 265 us, 456 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
+// and 738 MB of partial sums in between, took 674 + 213 + 285; the chunk 1288 -> 968 us, of 45 tokens at 3 bits 121 -> 102.
+// Tried: launch 2 by waves of 128 columns for 64 tokens (460 us), its matrix instructions placed among the decode (no change), its two
+// waves of a SIMD half a unit apart (2 %), an expert's items on one XCD (less traffic, same time); launch 3 in launch 2's form (272 to 312).
 
-// Tokens of a work item: as many tiles of 16 as leave room for two workgroups' LDS on a compute unit (the operand rows of four
-// 128-blocks, 1 KiB a token, and the four waves' rings of trellis rows).
-#define XPF_NT(K) ((K) <= 7 ? 3 : 2)
-// Rows of a wave's ring: what is left of half a compute unit's LDS (rows of 256, 512, 1024 (K = 3, 4) or 256 K bytes)
-#define XPF_D(K) ((K) <= 2 ? 8 : (K) <= 5 ? 6 : 4)
-#define XPF_TOK(K) (16 * XPF_NT(K))
-
-// The lane's share of a sign tile of H: element q of the pair is H[16 i + n][16 j + 4 a + q] (= H[16 j + 4 a + q][16 i + n])
-// for tile numbers of even popcount(i & j) (a = lane / 16, n = lane % 16); the other tiles are the negative.
-__device__ __forceinline__ void xpf_sign_tile(u32 lane, u32 (&hop)[2]) {
-    const u32 n = lane & 15, a = lane >> 4;
-    u32 h[4];
-#pragma unroll
-    for (u32 q = 0; q < 4; q++) h[q] = (__builtin_popcount((4 * a + q) & n) & 1) ? 0xbc00u : 0x3c00u;   // -1.0 : +1.0
-    hop[0] = h[0] | (h[1] << 16);
-    hop[1] = h[2] | (h[3] << 16);
-}
-
-// rot[ct][q] = sum over the 128 inputs i of H[16 ct + 4 a + q][i] v[i] for the lane's token (n = lane % 16 of the tile): v
-// comes as load4(ks) = the token's inputs 16 ks + 4 a .. + 3 (already times the input scales and the token's power of two).
-// An input goes in as an f16 high and an f16 low part (22 bits of it; the signs are exact, the sums f32): the rotation
-// itself adds no rounding that matters.
-template <class F>
-__device__ __forceinline__ void xpf_rotate_tile(F&& load4, const u32 (&hop)[2], f32x4 (&rot)[8]) {
-#pragma unroll
-    for (int ct = 0; ct < 8; ct++) rot[ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // the high and the low parts share one 32-deep matrix instruction: its operands are the sign tile twice and the two parts
-    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-    typedef u32 u32x4v __attribute__((ext_vector_type(4)));
-    typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-    const f16x8 hp = __builtin_bit_cast(f16x8, u32x4v{hop[0], hop[1], hop[0], hop[1]});
-    const f16x8 hn = __builtin_bit_cast(f16x8, u32x4v{hop[0] ^ 0x80008000u, hop[1] ^ 0x80008000u, hop[0] ^ 0x80008000u, hop[1] ^ 0x80008000u});
-#pragma unroll
-    for (int ks = 0; ks < 8; ks++) {
-        const f32x4 v = load4(ks);
-        const f16x4 av = {(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
-        const f16x4 al = {(_Float16) (v[0] - (float) av[0]), (_Float16) (v[1] - (float) av[1]), (_Float16) (v[2] - (float) av[2]), (_Float16) (v[3] - (float) av[3])};
-        const u32x2 ab = __builtin_bit_cast(u32x2, av), lb = __builtin_bit_cast(u32x2, al);
-        const f16x8 parts = __builtin_bit_cast(f16x8, u32x4v{ab[0], ab[1], lb[0], lb[1]});
-#pragma unroll
-        for (int ct = 0; ct < 8; ct++) {
-            const bool neg = __builtin_popcount(ks & ct) & 1;
-            rot[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(neg ? hn : hp, parts, rot[ct], 0, 0, 0);
-        }
-    }
-}
+// Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for.
+#define XPF_NT(K) ((K) <= 5 ? 8 : 6)
+// Units of a wave's ring of trellis rows: what eight waves have room for, and in workgroups of four waves (few items, whose weights come
+// from memory rather than a cache: their trip is what the launch waits for) as deep as the operand rows of NT tiles leave room.
+#define XPF_RING(K) ((K) <= 7 ? 3 : 2)
+#define XPF_RING_N(K, NT) ((NT) <= 2 ? ((K) <= 4 ? 8 : 12 - (K)) : (NT) == 4 ? ((K) <= 5 ? 5 : 4) : XPF_RING(K))
+#define XPF_RING_DOWN_N(K) ((K) <= 4 ? 8 : (K) <= 6 ? 6 : 4)
+// What undoes the 1 / 128 that the stored values carry and applies the transform's 1 / sqrt(128)
+#define XPF_UNSCALE 11.3137085f
+typedef u16 u16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // The largest magnitude of the lane's token's 128 values: the lane's 32 of them, then the lanes + 16, + 32, + 48.
 __device__ __forceinline__ float xpf_token_max(const f32x4 (&v)[8], u32 lane) {
@@ -1533,166 +1504,12 @@ __device__ __forceinline__ float xpf_token_max(const f32x4 (&v)[8], u32 lane) {
     return fmaxf(m, lane_xor<32>(m, lane));
 }
 
-// A 128-block of the lane's token through H, its values brought into f16's range for the product by the token's own power
-// of two and back afterwards (exact both ways): rot = H v.
-__device__ __forceinline__ void xpf_rotate_scaled(const f32x4 (&v)[8], const u32 (&hop)[2], f32x4 (&rot)[8], u32 lane) {
-    float scale, inv;
-    pow2_scale_of(f32_bits(xpf_token_max(v, lane)), scale, inv);
-    xpf_rotate_tile([&](int ks) { return v[ks] * scale; }, hop, rot);
-#pragma unroll
-    for (int ct = 0; ct < 8; ct++) rot[ct] *= inv;
-}
-
-// The operand rows of the products.  A token tile's rows: [tile row i of the item's up to 32 (block * 8 + ct)][token n][16
-// values in the order the decode lanes take them], 512 bytes a tile row; the tiles of an item follow each other.  The lane
-// holds the values 4 a + q of tile row ct of its token: slots 8 (a & 1) + 2 (a >> 1) + {0, 1} and + 4 of that (exl3_aslot).
-// rot must be bounded by 2^22 (inputs scaled to below 2^15, 128 terms): the stored value is f16(rot / 128).
-#define XPF_TILE_U16 (32 * 256)      // u16 of a token tile's operand rows (four 128-blocks)
-__device__ __forceinline__ void xpf_put_rows(u16* tile, u32 block, const f32x4 (&rot)[8], u32 lane) {
-    const u32 n = lane & 15, a = lane >> 4;
-    u32* at = (u32*) (tile + (block * 8) * 256 + n * 16 + 8 * (a & 1) + 2 * (a >> 1));
-#pragma unroll
-    for (int ct = 0; ct < 8; ct++) {
-        const f16x2 lo = {(_Float16) (rot[ct][0] * 0.0078125f), (_Float16) (rot[ct][1] * 0.0078125f)};
-        const f16x2 hi = {(_Float16) (rot[ct][2] * 0.0078125f), (_Float16) (rot[ct][3] * 0.0078125f)};
-        at[ct * 128] = __builtin_bit_cast(u32, lo);
-        at[ct * 128 + 2] = __builtin_bit_cast(u32, hi);
-    }
-}
-// what undoes the 1 / 128 of the stored values and applies the transform's 1 / sqrt(128)
-#define XPF_UNSCALE 11.3137085f
-
-// The products of one wave: `nrows` tile rows of its 128-column block (the stream starts at row0, its first rows already
-// requested) against the operand rows of NT token tiles at xa; acc[T][c][q] = output 16 c + 4 a + q of token 16 T + n.
-template <int K, int NT>
-__device__ __forceinline__ void xpf_wave_products_of(const u32* __restrict__ row0, u64 pitch, u32 nrows, const u32* wb, u32 lds, const u16* xa, u32 lane,
-                                                     f32x4 (&acc)[XPF_NT(K)][8]) {
-    constexpr int D = XPF_D(K);
-    typedef Exl3Rows<K, D> R;
-    constexpr int stride = R::stride, ur = R::unit_rows;
-    constexpr bool one_shift = 16 + 3 * K <= 32;
-    const u32 n16 = lane & 15, a = lane >> 4;
-    const u32 t0 = 32 * (n16 & 7) + 8 * a + 4 * (n16 >> 3);
-    auto window = [&](u32 e, u32& om, u32& op, u32& sh) {
-        const u32 jp = (e - 1) >> 5, jm = (jp + 8 * K - 1) % (8 * K);
-        sh = 31 - ((e - 1) & 31);
-        om = (jm / K) * stride + jm % K;
-        op = (jp / K) * stride + jp % K;
-    };
-    u32 om1, op1, sh1, om0 = 0, op0 = 0, sh0 = 0;
-    window((t0 + 4) * K, om1, op1, sh1);
-    if constexpr (!one_shift) window((t0 + 2) * K, om0, op0, sh0);
-#pragma unroll
-    for (int T = 0; T < NT; T++)
-#pragma unroll
-        for (int c = 0; c < 8; c++) acc[T][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const u16* xa0 = xa + n16 * 16 + 4 * a;
-    typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-    if constexpr (one_shift && ur == 1) {
-        // Two tile rows a step: a lane's 4 + 4 weights of the rows' tiles are one operand of the 32-deep matrix instruction
-        // (the contraction runs over both rows' 16 inputs; which of them a lane holds does not matter as long as the token
-        // operand is put together the same way), which halves the matrix instructions and their issue slots.
-        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-        typedef u32 u32x4v __attribute__((ext_vector_type(4)));
-#pragma unroll 1
-        for (u32 i = 0; i < nrows; i += 2) {   // a stream is a whole number of 8-row blocks
-            u32 w1[2][8][2];
-            u32x2 xv[2][NT];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const u32 r = i + h;
-                exl3_rows_wait<K, D>(r + D > nrows ? r + D - nrows : 0);
-                const u32* row = wb + (r % D) * R::row_words;
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    w1[h][c][0] = row[c * 8 * stride + om1];
-                    w1[h][c][1] = row[c * 8 * stride + op1];
-                }
-#pragma unroll
-                for (int T = 0; T < NT; T++) xv[h][T] = *(const u32x2*) (xa0 + T * XPF_TILE_U16 + r * 256);
-                if (r + D < nrows) {
-                    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the row's words are in registers, its slot can take the row D further on
-                    exl3_unit_issue<K, D>(row0, pitch, r + D, lane, lds);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                u32 b[2][2];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const u32 hi = __builtin_amdgcn_alignbit(w1[h][c][0], w1[h][c][1], sh1);
-                    const u32 s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16), s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
-                    const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
-                    b[h][0] = __builtin_bit_cast(u32, exl3_cb2_pair(s0, s1));
-                    b[h][1] = __builtin_bit_cast(u32, exl3_cb2_pair(s2, s3));
-                }
-                const f16x8 bv = __builtin_bit_cast(f16x8, u32x4v{b[0][0], b[0][1], b[1][0], b[1][1]});
-#pragma unroll
-                for (int T = 0; T < NT; T++) {
-                    const f16x8 tv = __builtin_bit_cast(f16x8, u32x4v{xv[0][T][0], xv[0][T][1], xv[1][T][0], xv[1][T][1]});
-                    acc[T][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv, tv, acc[T][c], 0, 0, 0);
-                }
-            }
-        }
-        return;
-    }
-#pragma unroll 1
-    for (u32 i = 0; i < nrows; i++) {
-        exl3_rows_wait<K, D>(i + D > nrows ? i + D - nrows : 0);
-        const u32* row = wb + (i % D) * R::row_words;
-        u32 w1[8][2], w0[8][2];
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            w1[c][0] = row[c * 8 * stride + om1];
-            w1[c][1] = row[c * 8 * stride + op1];
-            if constexpr (!one_shift) {
-                w0[c][0] = row[c * 8 * stride + om0];
-                w0[c][1] = row[c * 8 * stride + op0];
-            }
-        }
-        f16x4 xv[NT];
-#pragma unroll
-        for (int T = 0; T < NT; T++) xv[T] = __builtin_bit_cast(f16x4, *(const u32x2*) (xa0 + T * XPF_TILE_U16 + i * 256));
-        if ((i + 1) % ur == 0 && i + D + 1 - ur < nrows) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the row's words are in registers, its slot can take the row D further on
-            exl3_unit_issue<K, D>(row0, pitch, i + D + 1 - ur, lane, lds);
-        }
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const u32 hi = __builtin_amdgcn_alignbit(w1[c][0], w1[c][1], sh1);
-            u32 s0, s1;
-            if constexpr (one_shift) {
-                s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16);
-                s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
-            } else {
-                const u32 lo = __builtin_amdgcn_alignbit(w0[c][0], w0[c][1], sh0);
-                s0 = __builtin_amdgcn_ubfe(lo, K, 16);
-                s1 = lo & 0xffffu;
-            }
-            const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
-            const f16x2 b01 = exl3_cb2_pair(s0, s1), b23 = exl3_cb2_pair(s2, s3);
-            const f16x4 bv = {b01[0], b01[1], b23[0], b23[1]};
-#pragma unroll
-            for (int T = 0; T < NT; T++) acc[T][c] = __builtin_amdgcn_mfma_f32_16x16x16f16(bv, xv[T], acc[T][c], 0, 0, 0);
-        }
-    }
-}
-
-// One loop for every number of token tiles: the choice is made once, outside the loop.
-template <int K>
-__device__ __forceinline__ void xpf_wave_products(const u32* __restrict__ row0, u64 pitch, u32 nrows, const u32* wb, u32 lds, const u16* xa, u32 ntiles,
-                                                  u32 lane, f32x4 (&acc)[XPF_NT(K)][8]) {
-    if (ntiles == 1) xpf_wave_products_of<K, 1>(row0, pitch, nrows, wb, lds, xa, lane, acc);
-    else if (ntiles == 2) xpf_wave_products_of<K, 2>(row0, pitch, nrows, wb, lds, xa, lane, acc);
-    else if constexpr (XPF_NT(K) >= 3) xpf_wave_products_of<K, 3>(row0, pitch, nrows, wb, lds, xa, lane, acc);
-}
-
-// The output side of a wave's block for the lane's token: v[c][q] = output 16 c + 4 a + q goes through the 128-point
-// transform.  Five of its seven stages are between the lane's own registers; the two over the lane number's bits 4 and 5 are
-// swaps of register halves between the lanes (one swap serves two registers), after which the lane holds OTHER outputs of
-// its token: register c, element q is output xpf_out_col(c, lane) + q.
+// The 128-point transform of the lane's token: v[c][q] = value 16 c + 4 a + q (a = lane / 16).  Five of its seven stages are
+// between the lane's own registers; the two over the lane number's bits 4 and 5 are swaps of register halves between the lanes
+// (one swap serves two registers), after which the lane holds OTHER values of its token: register c, element q is value
+// xpf_out_col(c, lane) + q.  Done twice, the values lie as they did at first.
 __device__ __forceinline__ u32 xpf_out_col(u32 c, u32 lane) { return 64 * (c >> 2) + 32 * ((lane >> 4) & 1) + 16 * (lane >> 5) + 8 * (c & 1) + 4 * ((c >> 1) & 1); }
-__device__ __forceinline__ void xpf_output_side(f32x4 (&v)[8]) {
+__device__ __forceinline__ void xpf_transform(f32x4 (&v)[8]) {
 #pragma unroll
     for (int c = 0; c < 8; c++) {
         const float t0 = v[c][0] + v[c][1], t1 = v[c][0] - v[c][1], t2 = v[c][2] + v[c][3], t3 = v[c][2] - v[c][3];
@@ -1707,9 +1524,9 @@ __device__ __forceinline__ void xpf_output_side(f32x4 (&v)[8]) {
                 v[c] = s;
                 v[c + h] = d;
             }
-    // lane bit 5 (output bit 3): the upper half of register c and the lower half of register c + 1 change places; then both lanes
+    // lane bit 5 (value bit 3): the upper half of register c and the lower half of register c + 1 change places; then both lanes
     // of a pair hold the two ends of one butterfly.  Register c keeps the sum (bit 3 clear), c + 1 the difference; the lane's
-    // bit 5 now says which of the two registers' outputs (output bit 4) it holds.
+    // bit 5 now says which of the two registers' values (value bit 4) it holds.
 #pragma unroll
     for (int c = 0; c < 8; c += 2)
 #pragma unroll
@@ -1718,7 +1535,7 @@ __device__ __forceinline__ void xpf_output_side(f32x4 (&v)[8]) {
             v[c][q] = bits_f32(r[0]) + bits_f32(r[1]);
             v[c + 1][q] = bits_f32(r[0]) - bits_f32(r[1]);
         }
-    // lane bit 4 (output bit 2) with the registers c and c + 2 (output bit 5) likewise
+    // lane bit 4 (value bit 2) with the registers c and c + 2 (value bit 5) likewise
 #pragma unroll
     for (int c = 0; c < 8; c++)
         if (!(c & 2)) {
@@ -1731,276 +1548,532 @@ __device__ __forceinline__ void xpf_output_side(f32x4 (&v)[8]) {
         }
 }
 
-// Shared set-up of the launches: the item, its pairs and rows (tok = the most pairs of an item).  Returns the number of the
-// item's pairs (0: no such item).
-__device__ __forceinline__ u32 xpf_item(const u32* __restrict__ offs, const u32* __restrict__ list, const u32* __restrict__ items, u32 item, u32 ne, bool has_shared,
-                                        u32 k, u32 npairs, u32 tok, u32* s_pairs, u32* s_rows, u32& e) {
-    if (item >= items[0]) return 0;
-    e = items[1 + 2 * item];
-    const u32 t0 = items[2 + 2 * item];
-    if (e == ne && !has_shared) return 0;
-    const u32 first = offs[e], nt = min(tok, offs[e + 1] - first - t0);
-    if (threadIdx.x < tok) {
-        const u32 p = list[first + t0 + min(threadIdx.x, nt - 1)];   // a place past the item's end repeats its last pair: loads stay in bounds, results are dropped
-        s_pairs[threadIdx.x] = p;
-        s_rows[threadIdx.x] = p < npairs ? p / k : p - npairs;
+// The operand rows of 16 tokens and one 128-block: a 32-deep matrix instruction takes two tile rows, lane 16 a + n holds of either the
+// inputs 2 a, 2 a + 1, 2 a + 8, 2 a + 9 of token n (the order in which the decode yields weights).  [pair of tile rows][lane][8], as the
+// lanes read them: 4 KiB, in two halves of 64 inputs half_step u16 apart.
+#define XPF_ROWS_U16 2048
+#define XPF_HALF_U16 1024     // of the first or the last 64 inputs: how the operand rows are laid out, [64-block][tile]
+__device__ __forceinline__ u32 xpf_f16_pair(float a, float b) { return __builtin_bit_cast(u32, f16x2{(_Float16) a, (_Float16) b}); }
+// The values after one transform (xpf_out_col): a lane holds whole tile rows; the lanes 32 on hold the other row of each pair.
+__device__ __forceinline__ void xpf_put_transformed(u16* rows, u32 half_step, const f32x4 (&v)[8], u32 lane) {
+    const u32 n = lane & 15, b4 = (lane >> 4) & 1, b5 = lane >> 5;
+#pragma unroll
+    for (u32 h = 0; h < 2; h++)
+#pragma unroll
+        for (u32 a = 0; a < 2; a++) {
+            u32 w[2][2];
+#pragma unroll
+            for (u32 j = 0; j < 2; j++) {
+                // words of place a (register 4 h + j, elements 2 a, 2 a + 1) and of place a + 2 (register 4 h + 2 + j)
+                const auto r = __builtin_amdgcn_permlane32_swap(xpf_f16_pair(v[4 * h + j][2 * a], v[4 * h + j][2 * a + 1]), xpf_f16_pair(v[4 * h + 2 + j][2 * a], v[4 * h + 2 + j][2 * a + 1]), false, false);
+                w[0][j] = r[0];
+                w[1][j] = r[1];
+            }
+            *(u32x4*) (rows + h * half_step + ((b4 * 4 + a + 2 * b5) * 16 + n) * 8) = u32x4{w[0][0], w[0][1], w[1][0], w[1][1]};
+        }
+}
+// The values as they lie before a transform or after two.
+__device__ __forceinline__ void xpf_put_plain(u16* rows, u32 half_step, const f32x4 (&v)[8], u32 lane) {
+    const u32 n = lane & 15, b4 = (lane >> 4) & 1, b5 = lane >> 5;
+#pragma unroll
+    for (u32 p = 0; p < 4; p++) {
+        u32 w[2][2];
+#pragma unroll
+        for (u32 h = 0; h < 2; h++) {
+            const auto r = __builtin_amdgcn_permlane32_swap(xpf_f16_pair(v[2 * p + h][0], v[2 * p + h][1]), xpf_f16_pair(v[2 * p + h][2], v[2 * p + h][3]), false, false);
+            w[h][0] = r[0];
+            w[h][1] = r[1];
+        }
+        *(u32x4*) (rows + (p >> 1) * half_step + (((p & 1) * 4 + 2 * b4 + b5) * 16 + n) * 8) = u32x4{w[0][0], w[0][1], w[1][0], w[1][1]};
     }
-    return nt;
 }
 
-// LDS of a workgroup of launches 1 and 3, in words: the operand rows of the item's token tiles, the four waves' rings, the
-// item's pairs and rows, the waves' token maxima, the tokens' factors.
-#define XPF_LDS_WORDS(ring, tok) ((tok) / 16 * (XPF_TILE_U16 / 2) + 4 * (ring) + 2 * (tok) + 4 * (tok) + (tok))
+// An item: its expert (ne: the shared one), the number n of its pairs (0: there is no such item), its first pair's place in `list`, its
+// tiles of 16 tokens and the number of the first of them: the operand rows lie behind each other by tiles, an expert's from a place on
+// that its first pair's and its number tell.
+struct XpfItem {
+    u32 e, n, first, tiles, base;
+};
+__device__ __forceinline__ XpfItem xpf_item(const u32* __restrict__ offs, const u32* __restrict__ items, u32 item, u32 ne, bool has_shared, u32 tok) {
+    XpfItem it{0, 0, 0, 0, 0};
+    if (item >= items[0]) return it;
+    it.e = items[1 + 2 * item];
+    if (it.e == ne && !has_shared) return it;
+    it.first = offs[it.e] + items[2 + 2 * item];
+    it.n = min(tok, offs[it.e + 1] - it.first);
+    it.tiles = (it.n + 15) / 16;
+    it.base = offs[it.e] / 16 + it.e + items[2 + 2 * item] / 16;
+    return it;
+}
+// The item of a workgroup of a launch of 8 ceil(bound / 8) parts workgroups, and which of the item's parts it takes.  Workgroup i runs on
+// XCD i mod 8: the parts of an item follow each other on one of them, so that its operand rows come from memory once.
+__device__ __forceinline__ u32 xpf_place(u32 parts, u32& part) {
+    part = blockIdx.x / 8 % parts;
+    return blockIdx.x / 8 / parts * 8 + (blockIdx.x & 7);
+}
+// The products are compiled for 1, 2, 4, 6 and 8 token tiles: an item of 3, 5 or 7 has the next one's do for it, the last tile's
+// operand rows being whatever lies there.
+template <int N>
+struct XpfInt {
+    static constexpr int value = N;
+};
+template <int MOST, class F>
+__device__ __forceinline__ void xpf_tiles(u32 tiles, F&& run) {
+    if (tiles == 1) return run(XpfInt<1>());
+    if (tiles == 2) return run(XpfInt<2>());
+    if constexpr (MOST > 6) {
+        if (tiles > 6) return run(XpfInt<8>());
+    }
+    if constexpr (MOST > 4) {
+        if (tiles > 4) return run(XpfInt<6>());
+    }
+    run(XpfInt<4>());
+}
 
-// Launch 1: item blockIdx.x, sel = blockIdx.y / zs (gate, up), z = blockIdx.y % zs: the inputs' 128-blocks 4 z .. 4 z + 3.
-// Wave w rotates block 4 z + w of the item's tokens, then takes the 128-column blocks w, w + 4, .. of ff over the four input
-// blocks; raw partial sums gup[((sel * NP + pair) * zs + z)][ff] (NP = npairs + the shared expert's rows): the output side
-// is launch 2's.  grid = (bound on the items, 2 zs), block 256, dynamic LDS 4 XPF_LDS_WORDS.
-template <int K>
-__device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs,
-                                                            const u32* __restrict__ list, const u32* __restrict__ items, const float* __restrict__ x,
-                                                            float* __restrict__ gup, u32 ne, u32 k, u32 npairs, u32 NP, u32 hidden, u32 ff) {
-    typedef Exl3Rows<K, XPF_D(K)> R;
-    constexpr u32 TOK = XPF_TOK(K);
-    extern __shared__ __attribute__((aligned(16))) u32 dyn[];
-    u16* arows = (u16*) dyn;                                  // [token tile][block of the four][tile row][token][16]
-    u32* rings = dyn + XPF_NT(K) * (XPF_TILE_U16 / 2);
-    u32* s_pairs = rings + 4 * R::words;
-    u32* s_rows = s_pairs + TOK;
-    float* s_max = (float*) (s_rows + TOK);                   // [wave][token]
-    float* s_inv = s_max + 4 * TOK;                           // [token]
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 kbs = hidden / 128, zs = (kbs + 3) / 4, sel = blockIdx.y / zs, z = blockIdx.y - sel * zs;
-    u32 e;
-    const u32 nt = xpf_item(offs, list, items, blockIdx.x, ne, sh_addr != nullptr, k, npairs, TOK, s_pairs, s_rows, e);
-    if (nt == 0) return;
-    const u32 ntiles = (nt + 15) / 16;
-    const u8* bp = (const u8*) (e < ne ? eaddr[(u64) sel * ne + e] : sh_addr[sel]);
-    const u32 kb = 4 * z + wave, nkb = min(4u, kbs - 4 * z);
-    __syncthreads();                                          // the item's pairs and rows are written
-    typedef u16 u16x4 __attribute__((ext_vector_type(4)));
-    float sc[8][4];
-    if (wave < nkb) {
-        // the largest input of every token over the block: the token's power of two must be one for the workgroup's four blocks
-        const u16* suh = (const u16*) bp + kb * 128 + 4 * (lane >> 4);
+// Launch 1: a tile (16 tokens) of an item; wave w takes the 128-blocks w, w + 4, .. of the inputs.  A token's power of
+// two takes the product of its largest input (amax, from the routing launch) and the projection's largest input scale to [2^7, 2^8):
+// no value passes 2^15 in the transform.  rows: an item's [gate, up][64-block][tile], inv: [gate, up][tile][16].
+// Bound by the rows it writes (8 bytes an input and pair).  grid = xpf_place's, of `tiles` parts, block 256.
+extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const float* x,
+                                                                      const float* amax, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles) {
+    __shared__ u32 s_scale[2][4];
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, kbs = hidden / 128;
+    u32 T;
+    const u32 item = xpf_place(tiles, T);
+    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, tok);
+    if (T >= it.tiles) return;
+    const u32 e = it.e, pair = list[it.first + min(16 * T + (lane & 15), it.n - 1)];   // places past the item's end repeat its last pair: nothing reads them
+    const u32 token = pair < npairs ? pair / k : pair - npairs;
+    const float am = amax[token];
+    const u16* suh[2] = {(const u16*) (e < ne ? eaddr[e] : sh_addr[0]), (const u16*) (e < ne ? eaddr[(u64) ne + e] : sh_addr[1])};
 #pragma unroll
-        for (int ks = 0; ks < 8; ks++) {
-            const u16x4 s4 = *(const u16x4*) (suh + 16 * ks);
+    for (int s = 0; s < 2; s++) {
+        u32 m = 0;
+        for (u32 i = threadIdx.x; i < hidden / 8; i += 256) {
+            const u32x4a v = ((const u32x4a*) suh[s])[i];
 #pragma unroll
-            for (int q = 0; q < 4; q++) sc[ks][q] = f16_to_f32(s4[q]);
+            for (int q = 0; q < 4; q++) m = max(m, max(v[q] & 0x7fffu, (v[q] >> 16) & 0x7fffu));
         }
-        for (u32 T = 0; T < ntiles; T++) {
-            const float* xr = x + (u64) s_rows[16 * T + (lane & 15)] * hidden + kb * 128 + 4 * (lane >> 4);
-            f32x4 xv[8];
+        m = wave_max_u32(m);
+        if (lane == 0) s_scale[s][wave] = m;
+    }
+    __syncthreads();
+    float scale[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const u32 m = max(max(s_scale[s][0], s_scale[s][1]), max(s_scale[s][2], s_scale[s][3]));
+        float iv;
+        pow2_scale_of(f32_bits(am * f16_to_f32((u16) m)), scale[s], iv);
+        scale[s] *= 0.0078125f;
+        if (wave == 0 && lane < 16) inv[(it.base * 2 + s * it.tiles + T) * 16 + lane] = iv * XPF_UNSCALE;
+    }
+    const float* xr = x + (u64) token * hidden + 4 * (lane >> 4);
+    for (u32 kb = wave; kb < kbs; kb += 4) {
+        f32x4 xv[8];
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) xv[ks] = *(const f32x4*) (xr + kb * 128 + 16 * ks);
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            f32x4 v[8];
 #pragma unroll
             for (int ks = 0; ks < 8; ks++) {
-                xv[ks] = *(const f32x4*) (xr + 16 * ks);
+                const u16x4 s4 = *(const u16x4*) (suh[s] + kb * 128 + 16 * ks + 4 * (lane >> 4));
 #pragma unroll
-                for (int q = 0; q < 4; q++) xv[ks][q] *= sc[ks][q];
+                for (int q = 0; q < 4; q++) v[ks][q] = (xv[ks][q] * f16_to_f32(s4[q])) * scale[s];
             }
-            const float m = xpf_token_max(xv, lane);
-            if (lane < 16) s_max[wave * TOK + 16 * T + lane] = m;
-        }
-    }
-    __syncthreads();
-    if (wave < nkb) {
-        u32 hop[2];
-        xpf_sign_tile(lane, hop);
-        for (u32 T = 0; T < ntiles; T++) {
-            const u32 t = 16 * T + (lane & 15);
-            float m = 0.0f;
-            for (u32 w = 0; w < nkb; w++) m = fmaxf(m, s_max[w * TOK + t]);
-            float scale, iv;
-            pow2_scale_of(f32_bits(m), scale, iv);
-            if (wave == 0 && lane < 16) s_inv[t] = iv * XPF_UNSCALE;
-            const float* xr = x + (u64) s_rows[t] * hidden + kb * 128 + 4 * (lane >> 4);   // the second read comes from the caches
-            f32x4 rot[8];
-            xpf_rotate_tile(
-                [&](int ks) {
-                    f32x4 v = *(const f32x4*) (xr + 16 * ks);
-#pragma unroll
-                    for (int q = 0; q < 4; q++) v[q] = (v[q] * sc[ks][q]) * scale;
-                    return v;
-                },
-                hop, rot);
-            xpf_put_rows(arows + T * XPF_TILE_U16, wave, rot, lane);
-        }
-    }
-    __syncthreads();
-    const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(rings + wave * R::words));
-    const u64 pitch = (u64) (ff / 16) * EXL3_TILE_WORDS(K, false);
-    for (u32 cb = wave; cb < ff / 128; cb += 4) {
-        const u32* row0 = (const u32*) (bp + 2 * (u64) hidden + 2 * (u64) ff + 4) + ((u64) (4 * z) * 8 * (ff / 16) + cb * 8) * EXL3_TILE_WORDS(K, false);
-        exl3_rows_issue<K, XPF_D(K)>(row0, pitch, lane, wb_lds);     // a stream has at least 8 rows
-        f32x4 acc[XPF_NT(K)][8];
-        xpf_wave_products<K>(row0, pitch, 8 * nkb, rings + wave * R::words, wb_lds, arows, ntiles, lane, acc);
-#pragma unroll
-        for (int T = 0; T < XPF_NT(K); T++) {
-            if ((u32) T >= ntiles) break;
-            const u32 t = 16 * T + (lane & 15);
-            const float iv = s_inv[t];
-            if (t < nt) {
-                float* o = gup + (((u64) sel * NP + s_pairs[t]) * zs + z) * ff + cb * 128 + 4 * (lane >> 4);
-#pragma unroll
-                for (int c = 0; c < 8; c++) *(f32x4*) (o + 16 * c) = acc[T][c] * iv;
-            }
+            xpf_transform(v);
+            xpf_put_transformed(rows + ((u64) it.base * 2 + s * it.tiles) * kbs * XPF_ROWS_U16 + (2 * kb * it.tiles + T) * XPF_HALF_U16, it.tiles * XPF_HALF_U16, v, lane);
         }
     }
 }
 
-// Launch 2 (one kernel for every rate): tile blockIdx.y (16 tokens) of item blockIdx.x.  Wave w takes block w of ff (ff <=
-// 512: four blocks): adds up launch 1's partial sums of gate and up, puts both through their output sides (transform, output
-// scales), act = silu(gate) * up times the down projection's input scales, rotated, and leaves it as operand rows for
-// launch 3: arows[item * tok / 16 + tile] = a token tile's rows (XPF_TILE_U16), ainv[item * tok + token] = what undoes the
-// token's power of two.  grid = (bound on the items, tok / 16), block 256.
-extern "C" __global__ void __launch_bounds__(256, 2) prefill_act_exl3(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items,
-                                                                      const float* gup, u16* arows, float* ainv, u32 ne, u32 k, u32 npairs, u32 NP,
-                                                                      u32 hidden, u32 ff, u32 zs, u32 tok) {
-    __shared__ u32 s_pairs[64], s_rows[64];
-    __shared__ float s_max[4 * 16];
+// What a wave multiplies at a time: two tile rows of four column tiles (the words of their windows) with the operand rows of NT token
+// tiles, `step` u16 from one to the next.  read() and rows() ask LDS for them, products() adds acc[T][c][q] = output 16 c + 4 a + q of token 16 T + n.
+template <int K, int CT, int NT>
+struct XpfStep {
+    static constexpr int TW = EXL3_TILE_WORDS(K, false);
+    static constexpr bool one_shift = 16 + 3 * K <= 32;
+    u32 w1[8][2], w0[one_shift ? 1 : 8][2];
+    static __device__ __forceinline__ void window(u32 e, u32& om, u32& op, u32& sh) {
+        op = (e - 1) >> 5;
+        om = op == 0 ? TW - 1 : op - 1;
+        sh = 31 - ((e - 1) & 31);
+    }
+    static __device__ __forceinline__ u32 first(u32 lane) { return 32 * (lane & 7) + 8 * (lane >> 4) + 4 * ((lane & 15) >> 3); }   // the lane's first weight
+    // step s of the unit at `row`: its tile rows 2 s and 2 s + 1 (CT = 4: the unit has four), or their column tiles 4 s .. 4 s + 3 (CT = 8)
+    __device__ __forceinline__ void read(const u32* row, u32 s, u32 lane) {
+        u32 om, op, sh;
+        row += s * (CT == 4 ? 8 : 4) * TW;
+        window((first(lane) + 4) * K, om, op, sh);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            w1[i][0] = row[(i / 4 * CT + i % 4) * TW + om];
+            w1[i][1] = row[(i / 4 * CT + i % 4) * TW + op];
+        }
+        if constexpr (!one_shift) {
+            window((first(lane) + 2) * K, om, op, sh);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                w0[i][0] = row[(i / 4 * CT + i % 4) * TW + om];
+                w0[i][1] = row[(i / 4 * CT + i % 4) * TW + op];
+            }
+        }
+    }
+    static __device__ __forceinline__ void rows(u32x4 (&xv)[NT], const u16* xa, u32 step) {
+#pragma unroll
+        for (int T = 0; T < NT; T++) xv[T] = *(const u32x4*) (xa + T * step);
+    }
+    // adds to acc[T][c0 ..]
+    template <int c0>
+    __device__ __forceinline__ void products(const u32x4 (&xv)[NT], f32x4 (&acc)[NT][CT], u32 lane) const {
+        u32 om, op, sh1, sh0 = 0;
+        window((first(lane) + 4) * K, om, op, sh1);
+        if constexpr (!one_shift) window((first(lane) + 2) * K, om, op, sh0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            u32 b[2][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int i = 4 * h + c;
+                const u32 hi = __builtin_amdgcn_alignbit(w1[i][0], w1[i][1], sh1);
+                u32 s0, s1;
+                if constexpr (one_shift) {
+                    s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16);
+                    s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
+                } else {
+                    const u32 lo = __builtin_amdgcn_alignbit(w0[i][0], w0[i][1], sh0);
+                    s0 = __builtin_amdgcn_ubfe(lo, K, 16);
+                    s1 = lo & 0xffffu;
+                }
+                const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
+                b[h][0] = __builtin_bit_cast(u32, exl3_cb2_pair(s0, s1));
+                b[h][1] = __builtin_bit_cast(u32, exl3_cb2_pair(s2, s3));
+            }
+            const f16x8 bv = __builtin_bit_cast(f16x8, u32x4{b[0][0], b[0][1], b[1][0], b[1][1]});
+#pragma unroll
+            for (int T = 0; T < NT; T++) acc[T][c0 + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bv, __builtin_bit_cast(f16x8, xv[T]), acc[T][c0 + c], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
+// The products of a wave (64 columns) over the `ring.units` 64-blocks of the inputs.  The operand rows (src: [64-block][tiles], whole
+// item) come through a ring of NB slots of NT tiles in LDS (`stage`, slots `slot_u16` apart) that the NW waves of one projection share, of
+// which this is number `part`: requested NB - 1 units ahead, each wave its share, a barrier a unit.  A step's words and
+// operand rows are read while the one before is multiplied. The whole workgroup calls this with the same number of units.  D + 1 >= NB; units >= D.
+template <int K, int NT, int NB, int NW, class R>
+__device__ __forceinline__ void xpf_stream(const R& ring, const u32* wb, const u16* __restrict__ src, u16* stage, u32 slot_u16, u32 tiles, u32 part, u32 lane,
+                                           f32x4 (&acc)[NT][4]) {
+    constexpr int D = R::D, LEAST = NT <= 2 ? NT : NT - 1, A = 2 * LEAST / NW;   // A: loads of a unit's operand rows that every wave makes at least
+    static_assert(D + 1 >= NB && R::UR == 4, "operand rows are requested no earlier than the trellis rows of their unit");
+    auto request = [&](u32 unit, u32 slot) {
+        const u8* from = (const u8*) (src + (u64) unit * tiles * XPF_HALF_U16) + lane * 16;
+        const u32 to = __builtin_amdgcn_readfirstlane(lds_offset(stage + slot * slot_u16));
+        for (u32 i = part; i < 2 * tiles; i += NW) lds_load<16>(from + i * 1024, to + i * 1024);
+    };
+#pragma unroll
+    for (int T = 0; T < NT; T++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[T][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = -D; i < 0; i++) {
+        ring.issue(i + D, i + D, lane);
+        if (i + NB - 1 >= 0) request(i + NB - 1, i + NB - 1);
+    }
+    // this wave's share of a unit's operand rows has landed (behind it: NB - 2 times a unit's trellis rows and operand rows, but for the
+    // stream's end); every wave's, and the slot of the unit before has been read
+    auto ready = [&](u32 unit) {
+        if (unit + D <= ring.units) wait_vm<(NB - 2) * (R::NI + A)>();
+        else wait_vm<0>();
+        lds_barrier();
+    };
+    typedef XpfStep<K, 4, NT> Step;
+    Step s0, s1;
+    u32x4 x0[NT], x1[NT];
+    ready(0);
+    s0.read(wb, 0, lane);
+    Step::rows(x0, stage + lane * 8, XPF_HALF_U16);
+    u32 slot = 0, at = 0;
+#pragma unroll 1
+    for (u32 unit = 0; unit < ring.units; unit++) {
+        s1.read(wb + slot * R::UW, 1, lane);
+        Step::rows(x1, stage + at * slot_u16 + 512 + lane * 8, XPF_HALF_U16);
+        __builtin_amdgcn_sched_barrier(0);
+        s0.template products<0>(x0, acc, lane);
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the unit's words are in registers, its slot can take the unit D further on
+        if (unit + D < ring.units) ring.issue(unit + D, slot, lane);
+        if (unit + NB - 1 < ring.units) request(unit + NB - 1, at == 0 ? NB - 1 : at - 1);
+        slot = slot + 1 == (u32) D ? 0u : slot + 1;
+        at = at + 1 == (u32) NB ? 0u : at + 1;
+        if (unit + 1 < ring.units) {
+            ready(unit + 1);
+            s0.read(wb + slot * R::UW, 0, lane);
+            Step::rows(x0, stage + at * slot_u16 + lane * 8, XPF_HALF_U16);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        s1.template products<0>(x1, acc, lane);
+    }
+}
+
+// What launch 2 makes of a token tile's sums over the inputs (g, u: gate and up of a 128-block, in true units but for the output side):
+// output sides, act = silu(gate) * up times the down projection's input scales, its rotation, as operand rows.  The token's power of
+// two for this block is a multiple of 8 in the exponent, so that blocks mostly share one; inv undoes it.
+__device__ __forceinline__ void xpf_activate(f32x4 (&g)[8], f32x4 (&u)[8], const u16* svg, const u16* svu, const u16* suh, u16* rows, u32 half_step, float* inv, u32 lane) {
+    xpf_transform(g);
+    xpf_transform(u);
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const u32 at = xpf_out_col(c, lane);
+        const u16x4 a4 = *(const u16x4*) (svg + at), b4 = *(const u16x4*) (svu + at), c4 = *(const u16x4*) (suh + at);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float gate = g[c][q] * (f16_to_f32(a4[q]) * 0.08838835f), up = u[c][q] * (f16_to_f32(b4[q]) * 0.08838835f);
+            g[c][q] = (siluf_ref(gate) * up) * f16_to_f32(c4[q]);
+        }
+    }
+    float scale, all;
+    pow2_scale_of(f32_bits(xpf_token_max(g, lane)), scale, all);
+    const u32 sb = max((f32_bits(scale) >> 23) & ~7u, 8u);
+    scale = bits_f32(sb << 23) * 0.0078125f;
+    if (lane < 16) inv[lane] = bits_f32((254u - sb) << 23) * XPF_UNSCALE;
+#pragma unroll
+    for (int c = 0; c < 8; c++) g[c] *= scale;
+    xpf_transform(g);
+    xpf_put_plain(rows, half_step, g, lane);
+}
+
+// A workgroup's sums through LDS (x: [block of 128 columns][of R tiles][register][lane]), so that a wave has all 128 columns of a
+// token tile: the wave of columns 64 half .. of block `at` leaves tile T in place R at + i.
+__device__ __forceinline__ void xpf_leave(f32x4* x, u32 place, u32 half, const f32x4 (&acc)[4], u32 lane) {
+#pragma unroll
+    for (u32 c = 0; c < 4; c++) x[(place * 8 + half * 4 + c) * 64 + lane] = acc[c];
+}
+__device__ __forceinline__ void xpf_take(const f32x4* x, u32 place, f32x4 (&v)[8], u32 lane) {
+#pragma unroll
+    for (u32 c = 0; c < 8; c++) v[c] = x[(place * 8 + c) * 64 + lane];
+}
+
+// Launch 2: an item and NCB 128-column blocks of ff, four waves a block (gate's two halves, up's).  rows2:
+// [tile][128-block of ff], inv2: [tile][128-block][16].  grid = xpf_place's, of ff / 128 / NCB parts, block 256 NCB; dynamic LDS: NB
+// slots of two projections' NT tiles and the waves' rings (for the NT of 1, 2, 4, 6, 8 that takes most), or the exchange of the sums, 64
+// KiB NCB for four tiles.
+template <int K, int NCB>
+__device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs, const u32* __restrict__ items,
+                                                            const u16* __restrict__ rows, const float* __restrict__ inv, u16* __restrict__ rows2, float* __restrict__ inv2, u32 ne, u32 hidden,
+                                                            u32 ff) {
+    extern __shared__ __attribute__((aligned(16))) u32 dyn[];
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 kbs = ff / 128, T = blockIdx.y;                  // kbs: at most 4
-    u32 e;
-    const u32 nt = xpf_item(offs, list, items, blockIdx.x, ne, sh_addr != nullptr, k, npairs, tok, s_pairs, s_rows, e);
-    if (16 * T >= nt) return;
-    __syncthreads();
+    const u32 sel = wave / (2 * NCB), part = wave % (2 * NCB), b = part / 2, half = part & 1;
+    const u32 kbs = hidden / 128, fbs = ff / 128;
+    u32 group;
+    const u32 item = xpf_place(fbs / NCB, group), cb = group * NCB + b;
+    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, 16 * XPF_NT(K));
+    if (it.n == 0) return;
+    const u32 e = it.e;
     const u8* bg = (const u8*) (e < ne ? eaddr[e] : sh_addr[0]);
     const u8* bu = (const u8*) (e < ne ? eaddr[(u64) ne + e] : sh_addr[1]);
     const u8* bd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
-    typedef u16 u16x4 __attribute__((ext_vector_type(4)));
-    u32 hop[2];
-    xpf_sign_tile(lane, hop);
-    f32x4 act[8];
-    float m = 0.0f;
-    if (wave < kbs) {
-        const u32 pair = s_pairs[16 * T + (lane & 15)], at = wave * 128 + 4 * (lane >> 4);
-        const float* pg = gup + ((u64) pair * zs) * ff + at;
-        const float* pu = gup + (((u64) NP + pair) * zs) * ff + at;
-        f32x4 g[8], u[8];
+    xpf_tiles<XPF_NT(K)>(it.tiles, [&](auto n) {
+        constexpr int NT = decltype(n)::value, G = NT < 4 ? NT : 4;
+        typedef VerifyRing<K, false, 4, NCB == 2 ? XPF_RING(K) : XPF_RING_N(K, NT)> R;
+        constexpr int NB = NCB == 2 ? 3 : R::D + 1;
+        u32* wb = dyn + NB * 2 * NT * (XPF_HALF_U16 / 2) + wave * (R::D * R::UW);
+        R ring;
+        ring.init((sel ? bu : bg) + 2 * (u64) hidden + 2 * (u64) ff + 4 + (u64) (cb * 8 + half * 4) * (4 * R::TW), (ff / 16) * (4 * R::TW), 2 * kbs,
+                  __builtin_amdgcn_readfirstlane(lds_offset(wb)), lane);
+        f32x4 acc[NT][4];
+        xpf_stream<K, NT, NB, 2 * NCB>(ring, wb, rows + ((u64) it.base * 2 + sel * it.tiles) * kbs * XPF_ROWS_U16, (u16*) dyn + sel * NT * XPF_HALF_U16, 2 * NT * XPF_HALF_U16, it.tiles, part, lane,
+                                       acc);
+        const float* iv = inv + (it.base * 2 + sel * it.tiles) * 16 + (lane & 15);
+        f32x4* x = (f32x4*) dyn;
 #pragma unroll
-        for (int ks = 0; ks < 8; ks++) {
-            g[ks] = *(const f32x4*) (pg + 16 * ks);
-            u[ks] = *(const f32x4*) (pu + 16 * ks);
-        }
-        for (u32 zz = 1; zz < zs; zz++)
+        for (int T0 = 0; T0 < NT; T0 += G) {
+            lds_barrier();
 #pragma unroll
-            for (int ks = 0; ks < 8; ks++) {
-                g[ks] += *(const f32x4*) (pg + (u64) zz * ff + 16 * ks);
-                u[ks] += *(const f32x4*) (pu + (u64) zz * ff + 16 * ks);
+            for (int i = 0; i < G && T0 + i < NT; i++) {
+                const float f = iv[16 * min((u32) (T0 + i), it.tiles - 1)];
+#pragma unroll
+                for (int c = 0; c < 4; c++) acc[T0 + i][c] *= f;
+                xpf_leave(x, (b * 2 + sel) * G + i, half, acc[T0 + i], lane);
             }
-        f32x4 gr[8];
-        xpf_rotate_scaled(g, hop, gr, lane);
-        xpf_rotate_scaled(u, hop, g, lane);                    // g: the rotated up from here on
-        const u16* svg = (const u16*) (bg + 2 * (u64) hidden) + at;
-        const u16* svu = (const u16*) (bu + 2 * (u64) hidden) + at;
-        const u16* suh = (const u16*) bd + at;
-#pragma unroll
-        for (int ct = 0; ct < 8; ct++) {
-            const u16x4 a4 = *(const u16x4*) (svg + 16 * ct), b4 = *(const u16x4*) (svu + 16 * ct), c4 = *(const u16x4*) (suh + 16 * ct);
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float gate = gr[ct][q] * (f16_to_f32(a4[q]) * 0.08838835f), up = g[ct][q] * (f16_to_f32(b4[q]) * 0.08838835f);
-                act[ct][q] = (siluf_ref(gate) * up) * f16_to_f32(c4[q]);
+            lds_barrier();
+            // four waves a block: one a tile
+            const u32 i = part - 2 * b + 2 * sel, T = T0 + i;
+            if (i < (u32) G && T < it.tiles) {
+                f32x4 g[8], u[8];
+                xpf_take(x, (b * 2) * G + i, g, lane);
+                xpf_take(x, (b * 2 + 1) * G + i, u, lane);
+                xpf_activate(g, u, (const u16*) (bg + 2 * (u64) hidden) + cb * 128, (const u16*) (bu + 2 * (u64) hidden) + cb * 128, (const u16*) bd + cb * 128,
+                             rows2 + ((u64) (it.base + T) * fbs + cb) * XPF_ROWS_U16, XPF_HALF_U16, inv2 + ((it.base + T) * fbs + cb) * 16, lane);
             }
         }
-        m = xpf_token_max(act, lane);
-        if (lane < 16) s_max[wave * 16 + lane] = m;
-    }
-    __syncthreads();
-    if (wave >= kbs) return;
-    m = 0.0f;
-    for (u32 w = 0; w < kbs; w++) m = fmaxf(m, s_max[w * 16 + (lane & 15)]);
-    float scale, iv;
-    pow2_scale_of(f32_bits(m), scale, iv);
-    if (wave == 0 && lane < 16) ainv[(u64) blockIdx.x * tok + 16 * T + lane] = iv * XPF_UNSCALE;
-    f32x4 rot[8];
-    xpf_rotate_tile([&](int ks) { return act[ks] * scale; }, hop, rot);
-    xpf_put_rows(arows + ((u64) blockIdx.x * (tok / 16) + T) * XPF_TILE_U16, wave, rot, lane);
+    });
 }
 
-// Launch 3: item blockIdx.x, 128-column blocks 4 blockIdx.y + w of hidden for wave w: the products of the item's operand rows
-// (copied from launch 2's into LDS, wave w its block w of every tile) over the ff / 128 input blocks and the output side:
-// eo[pair][hidden].  grid = (bound on the items, ceil(hidden / 512)), block 256, dynamic LDS 4 XPF_LDS_WORDS.
-template <int K>
-__device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs,
-                                                         const u32* __restrict__ list, const u32* __restrict__ items, const u16* __restrict__ arows_g,
-                                                         const float* __restrict__ ainv, float* __restrict__ eo, u32 ne, u32 k, u32 npairs, u32 hidden, u32 ff) {
-    typedef Exl3Rows<K, XPF_D(K)> R;
-    constexpr u32 TOK = XPF_TOK(K);
+// Launch 3: an item of up to XPF_DOWN_NT tiles and one of `parts` shares of the 128-column blocks of hidden, a wave a block at a time: the
+// products of the item's operand rows over ff and the output side: eo[pair][hidden].  The rows, their factors and the output scales are copied
+// to LDS once; from then on every wave goes its own way, its ring of trellis rows filled from one block to the next.
+// grid = xpf_place's, block 64 W; dynamic LDS in words: NTL tiles' rows (fbs * 1024 each), factors (fbs * 16 each), 64
+// XPF_DOWN_BLOCKS a wave for the output scales, the waves' rings.
+#define XPF_DOWN_NT 4
+#define XPF_DOWN_BLOCKS 4   /* most column blocks of a wave: parts * W * 4 >= hidden / 128 */
+template <int K, int DEPTH>
+__device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs, const u32* __restrict__ list,
+                                                         const u32* __restrict__ items, const u16* __restrict__ rows, const float* __restrict__ inv, float* __restrict__ eo, u32 ne, u32 hidden,
+                                                         u32 ff, u32 ntl, u32 parts) {
+    typedef VerifyRing<K, false, 8, DEPTH> R;
+    constexpr int D = R::D;
     extern __shared__ __attribute__((aligned(16))) u32 dyn[];
-    u16* arows = (u16*) dyn;
-    u32* rings = dyn + XPF_NT(K) * (XPF_TILE_U16 / 2);
-    u32* s_pairs = rings + 4 * R::words;
-    u32* s_rows = s_pairs + TOK;
-    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 kbs = ff / 128;                                  // at most 4
-    u32 e;
-    const u32 nt = xpf_item(offs, list, items, blockIdx.x, ne, sh_addr != nullptr, k, npairs, TOK, s_pairs, s_rows, e);
-    if (nt == 0) return;
-    const u32 ntiles = (nt + 15) / 16;
-    const u8* down = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
-    const u32 cb = 4 * blockIdx.y + wave;
-    const bool live = cb < hidden / 128;
-    // what undoes the powers of two of the lane's tokens (the only ordinary loads: consumed before the burst)
-    float iv[XPF_NT(K)];
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, W = blockDim.x >> 6;
+    const u32 fbs = ff / 128, cbs = hidden / 128, U = 4 * fbs;   // U: units a column block
+    u32 share;
+    const u32 item = xpf_place(parts, share);
+    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, 16 * XPF_DOWN_NT);
+    if (it.n == 0) return;
+    const u8* down = (const u8*) uniform_u64(it.e < ne ? eaddr[2ull * ne + it.e] : sh_addr[2]);
+    const u32 cb0 = share * W + wave, stride = parts * W;        // the wave's column blocks: cb0, cb0 + stride, ..
+    u16* xrows = (u16*) dyn;
+    float* fac = (float*) (dyn + ntl * fbs * 1024);
+    u16* scales = (u16*) (fac + ntl * fbs * 16) + wave * XPF_DOWN_BLOCKS * 128;   // of the wave's column blocks
+    u32* wb = dyn + ntl * fbs * 1040 + W * XPF_DOWN_BLOCKS * 64 + wave * (D * R::UW);
+    const u32 blocks = cb0 < cbs ? (cbs - cb0 + stride - 1) / stride : 0u, total = blocks * U;
+    R ring;
+    ring.init(down + 2 * (u64) ff + 2 * (u64) hidden + 4 + (u64) (cb0 < cbs ? cb0 : 0) * 8 * (4 * R::TW), (hidden / 16) * (4 * R::TW), U, __builtin_amdgcn_readfirstlane(lds_offset(wb)), lane);
+    xpf_tiles<XPF_DOWN_NT>(it.tiles, [&](auto n) {
+        constexpr int NT = decltype(n)::value < XPF_DOWN_NT ? decltype(n)::value : XPF_DOWN_NT;
+        u32 pair[NT];
 #pragma unroll
-    for (int T = 0; T < XPF_NT(K); T++) iv[T] = (u32) T < ntiles ? ainv[(u64) blockIdx.x * TOK + 16 * T + (lane & 15)] : 0.0f;
+        for (int T = 0; T < NT; T++) pair[T] = list[it.first + min(16 * T + (lane & 15), it.n - 1)];
 #pragma unroll
-    for (int T = 0; T < XPF_NT(K); T++) asm volatile("" : "+v"(iv[T]));
-    const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(rings + wave * R::words));
-    if (wave < kbs) {
-        // block `wave` of every live tile: 8 tile rows of 512 bytes, 1 KiB a load
-        for (u32 T = 0; T < ntiles; T++) {
-            const u8* src = (const u8*) (arows_g + ((u64) blockIdx.x * XPF_NT(K) + T) * XPF_TILE_U16 + wave * 8 * 256);
-            const u32 dst = __builtin_amdgcn_readfirstlane(lds_offset(arows + T * XPF_TILE_U16 + wave * 8 * 256));
+        for (int T = 0; T < NT; T++) load_landed(pair[T]);
+        for (u32 i = wave; i < it.tiles * fbs * 4; i += W) lds_load<16>((const u8*) (rows + (u64) it.base * fbs * XPF_ROWS_U16) + i * 1024 + lane * 16, lds_offset(xrows) + i * 1024);
+        for (u32 i = wave; 64 * i < it.tiles * fbs * 16; i += W)
+            if (64 * i + lane < it.tiles * fbs * 16) lds_load<4>(inv + it.base * fbs * 16 + 64 * i + lane, lds_offset(fac) + 256 * i);
+        for (u32 i = 0; i < blocks; i++) lds_load<4>(down + 2 * (u64) ff + 256 * (cb0 + i * stride) + 4 * lane, lds_offset(scales) + 256 * i);
+        // the unit after the last one requested: where it lies
+        u32 ahead = 0, unit = 0;
+        auto request = [&](u32 slot) {
+            ring.issue(unit, slot, lane);
+            ahead++;
+            if (++unit == U) {
+                unit = 0;
+                ring.row0 += (u64) stride * 8 * (4 * R::TW);
+            }
+        };
+        if (total) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) lds_load<16>(src + i * 1024 + lane * 16, dst + i * 1024);
+            for (int d = 0; d < D; d++)
+                if ((u32) d < total) request(d);
+            if (total >= (u32) D) wait_vm<D * R::NI>();
+            else wait_vm<0>();
+        } else wait_vm<0>();
+        lds_barrier();
+        // A block whose values are nothing beside the sums of the blocks before it (2^-88) would take the sums out of range with its power
+        // of two: zeros in its place, and the power of two of the one before.
+        if (threadIdx.x < 16 * it.tiles) {
+            const u32 T = threadIdx.x / 16, t = threadIdx.x % 16;
+            for (u32 b = 1; b < fbs; b++) {
+                float* f = fac + (T * fbs + b) * 16 + t;
+                if (f[-16] / f[0] > 0x1p88f) {
+                    f[0] = f[-16];
+                    for (u32 i = 0; i < 16; i++) *(u32x4*) (xrows + (T * fbs + b) * XPF_ROWS_U16 + (16 * i + t) * 8) = u32x4{0, 0, 0, 0};
+                }
+            }
         }
-    }
-    const u64 pitch = (u64) (hidden / 16) * EXL3_TILE_WORDS(K, false);
-    const u32* row0 = (const u32*) (down + 2 * (u64) ff + 2 * (u64) hidden + 4) + (u64) (live ? cb : 0) * 8 * EXL3_TILE_WORDS(K, false);
-    if (live) {
-        exl3_rows_issue<K, XPF_D(K)>(row0, pitch, lane, wb_lds);
-        wait_vm<R::loads>();                                  // this wave's operand rows have landed (its ring may still be on its way)
-    } else wait_vm<0>();
-    __syncthreads();                                          // every wave's operand rows, and the item's pairs
-    if (!live) return;
-    f32x4 acc[XPF_NT(K)][8];
-    xpf_wave_products<K>(row0, pitch, 8 * kbs, rings + wave * R::words, wb_lds, arows, ntiles, lane, acc);
-    typedef u16 u16x4 __attribute__((ext_vector_type(4)));
-    const u16* svh = (const u16*) (down + 2 * (u64) ff) + cb * 128;
-    f32x4 sv[8];
+        lds_barrier();
+        if (!total) return;
+        typedef XpfStep<K, 8, NT> Step;
+        const u32 tstep = fbs * XPF_ROWS_U16;
+        Step s0, s1;
+        u32x4 xv[NT], xn[NT];
+        f32x4 acc[NT][8];
+        auto reset = [&] {
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const u16x4 s4 = *(const u16x4*) (svh + xpf_out_col(c, lane));
+            for (int T = 0; T < NT; T++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) sv[c][q] = f16_to_f32(s4[q]) * 0.08838835f;
-    }
+                for (int c = 0; c < 8; c++) acc[T][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        };
+        auto factor = [&](int T, u32 b) { return fac[(min((u32) T, it.tiles - 1) * fbs + b) * 16 + (lane & 15)]; };   // what undoes the power of two
+        reset();
+        if (total >= (u32) D) wait_vm<(D - 1) * R::NI>();
+        s0.read(wb, 0, lane);
+        Step::rows(xv, xrows + lane * 8, tstep);
+        u32 slot = 0, u = 0, done = 0;   // done: column blocks finished
+#pragma unroll 1
+        for (u32 g = 0; g < total; g++) {
+            s1.read(wb + slot * R::UW, 1, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            if ((u & 3) == 0 && u > 0) {
+                // another 128-block of the inputs: its tokens' powers of two mostly are the ones before
 #pragma unroll
-    for (int T = 0; T < XPF_NT(K); T++) {
-        if ((u32) T >= ntiles) break;
+                for (int T = 0; T < NT; T++) {
+                    const float r = factor(T, u / 4 - 1) / factor(T, u / 4);   // a power of two
+                    if (__builtin_amdgcn_ballot_w64(r != 1.0f)) {
 #pragma unroll
-        for (int c = 0; c < 8; c++) acc[T][c] *= iv[T];
-        xpf_output_side(acc[T]);
-        const u32 t = 16 * T + (lane & 15);
-        if (t < nt) {
-            float* o = eo + (u64) s_pairs[t] * hidden + cb * 128;
+                        for (int c = 0; c < 8; c++) acc[T][c] *= r;
+                    }
+                }
+            }
+            s0.template products<0>(xv, acc, lane);
+            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the unit's words are in registers, its slot can take the unit D further on
+            if (ahead < total) request(slot);
+            slot = slot + 1 == (u32) D ? 0u : slot + 1;
+            const u32 un = u + 1 == U ? 0u : u + 1;
+            if (g + 1 < total) {
+                // behind the next unit: D - 1 units, but for the stream's end, and the stores of a finished block, which count too
+                if (g + 1 + D > total) wait_vm<0>();
+                else if (done > 0 && u + 1 < (u32) D) wait_vm<(D - 1) * R::NI + 8 * (NT <= 2 ? NT : NT - 1)>();
+                else wait_vm<(D - 1) * R::NI>();
+                s0.read(wb + slot * R::UW, 0, lane);
+                Step::rows(xn, xrows + un * 512 + lane * 8, tstep);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            s1.template products<4>(xv, acc, lane);
+            u = un;
+            if (u == 0) {
 #pragma unroll
-            for (int c = 0; c < 8; c++) *(f32x4*) (o + xpf_out_col(c, lane)) = acc[T][c] * sv[c];
+                for (int T = 0; T < NT; T++) {
+                    const float f = factor(T, fbs - 1);
+#pragma unroll
+                    for (int c = 0; c < 8; c++) acc[T][c] *= f;
+                    xpf_transform(acc[T]);
+                    if (16 * T + (lane & 15) < it.n) {
+                        float* o = eo + (u64) pair[T] * hidden + (cb0 + done * stride) * 128;
+#pragma unroll
+                        for (int c = 0; c < 8; c++) {
+                            const u16x4 s4 = *(const u16x4*) (scales + done * 128 + xpf_out_col(c, lane));
+                            f32x4 v;
+#pragma unroll
+                            for (int q = 0; q < 4; q++) v[q] = acc[T][c][q] * (f16_to_f32(s4[q]) * 0.08838835f);
+                            *(f32x4*) (o + xpf_out_col(c, lane)) = v;
+                        }
+                    }
+                }
+                reset();
+                done++;
+            }
+#pragma unroll
+            for (int T = 0; T < NT; T++) xv[T] = xn[T];
         }
-    }
+    });
 }
 
-#define EXL3_PREFILL_ENTRIES(K)                                                                                                          \
-    extern "C" __global__ void __launch_bounds__(256, 2) prefill_gate_up_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, \
-                                                                                   const u32* items, const float* x, float* gup, u32 ne, u32 k, u32 npairs, \
-                                                                                   u32 NP, u32 hidden, u32 ff) {                         \
-        prefill_gate_up_exl3_kernel<K>(eaddr, sh_addr, offs, list, items, x, gup, ne, k, npairs, NP, hidden, ff);                        \
-    }                                                                                                                                    \
-    extern "C" __global__ void __launch_bounds__(256, 2) prefill_down_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, \
-                                                                                const u32* items, const u16* arows, const float* ainv, float* eo, u32 ne, \
-                                                                                u32 k, u32 npairs, u32 hidden, u32 ff) {                 \
-        prefill_down_exl3_kernel<K>(eaddr, sh_addr, offs, list, items, arows, ainv, eo, ne, k, npairs, hidden, ff);                      \
+#define EXL3_PREFILL_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(512, 2) prefill_gate_up_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
+                                                                                  float* inv2, u32 ne, u32 hidden, u32 ff) { \
+        prefill_gate_up_exl3_kernel<K, 2>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, 2) prefill_gate_up_n_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
+                                                                                    float* inv2, u32 ne, u32 hidden, u32 ff) { \
+        prefill_gate_up_exl3_kernel<K, 1>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(512, 2) prefill_down_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const u16* rows, const float* inv, \
+                                                                               float* eo, u32 ne, u32 hidden, u32 ff, u32 ntl, u32 parts) { \
+        prefill_down_exl3_kernel<K, XPF_RING(K)>(eaddr, sh_addr, offs, list, items, rows, inv, eo, ne, hidden, ff, ntl, parts); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, 2) prefill_down_n_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const u16* rows, const float* inv, \
+                                                                                 float* eo, u32 ne, u32 hidden, u32 ff, u32 ntl, u32 parts) { \
+        prefill_down_exl3_kernel<K, XPF_RING_DOWN_N(K)>(eaddr, sh_addr, offs, list, items, rows, inv, eo, ne, hidden, ff, ntl, parts); \
     }
 EXL3_PREFILL_ENTRIES(1)
 EXL3_PREFILL_ENTRIES(2)

@@ -63,7 +63,7 @@ extern "C" __global__ void __launch_bounds__(256) quant_act_q8(const float* x, u
 // The two things a chunk needs before its tokens can be grouped, in one launch (they do not depend on each other): the
 // routing of its m tokens (workgroups [0, ceil(m / 4)): a wave a token, as route_topk_rows) and the quantization of its
 // activations (the workgroups after them, as quant_act_q8).  grid = ceil(m / 4) + ceil(n / 32 / 256), block 256.
-extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, u64 n, i8* q, float* d, const float* logits, u32* tidx, float* weights,
+extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, u64 n, i8* q, float* d, const float* logits, u32* tidx, float* weights, u32* cnt,
                                                                 u32 ne, u32 k, u32 m) {
     __shared__ double exs[4][512];
     __shared__ u32 tops[4][16];
@@ -85,6 +85,7 @@ extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, 
         tidx[(u64) j * k + lane] = tops[w][lane];
         weights[(u64) j * k + lane] = wt;
     }
+    if (lane == 0) cnt[j] = count;
 }
 
 #define PF_TOK 64      // tokens of one work item: PF_TOK / 16 MFMA tiles of 16
@@ -92,44 +93,49 @@ extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, 
 #define PF_TOK_D 32    // tokens of one work item of the down kernel: with half the activations in LDS twice the workgroups fit a CU
 
 // Groups the chunk's (token, rank) pairs by expert: offs[e] .. offs[e + 1] are the positions in list[] of expert e's pairs
-// (pair = token * k + rank; the shared expert, index ne, takes the pairs npairs + token when nshared = tokens).  Also
-// cnt[token] = its number of valid experts.  The order of an expert's pairs in list[] is arbitrary; every pair owns its
+// (pair = token * k + rank; the shared expert, index ne, takes the pairs npairs + token when nshared = tokens).  The order of an expert's pairs in list[] is arbitrary; every pair owns its
 // output rows, so the results do not depend on it.  items[0] = the number of work items, items[1 + 2 i], items[2 + 2 i] =
 // (expert, first position) of item i: every run of up to unit_gu pairs of an expert is one item of the gate/up kernel (at most
-// ne + 1 + rows / unit_gu of them; PF_TOK for the int8 kernels below); items_d likewise with runs of up to unit_d pairs, for the down kernel.  The items that
-// exist come first in both lists, so the workgroups launched for the rest of the bound run at the launches' ends, out of
-// the way.  One workgroup.  grid 1, block 1024; ne <= 512.
+// ne + 1 + rows / unit_gu of them); items_d likewise with runs of up to unit_d pairs, for the down kernel.  The longest items come
+// first, so that the launches end on short ones, and all ahead of the workgroups launched for the rest of the bound (int8 chunk of 512
+// tokens: 239 -> 226 us with the order alone).  Bound by the round trips of its loads: 41 us for 40960 pairs when a thread had one in
+// flight, 37 with eight.  One workgroup.  grid 1, block 1024; ne <= 512.
 extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list,
-                                                                 u32* cnt, u32* items, u32* items_d, u32 unit_gu, u32 unit_d) {
-    __shared__ u32 s_cnt[513], s_off[514], s_fill[513], s_fill_d[513];
+                                                                 u32* items, u32* items_d, u32 unit_gu, u32 unit_d) {
+    __shared__ u32 s_cnt[513], s_off[514], s_fill[513], s_full[2][513], s_class[2][9];
     const u32 tid = threadIdx.x, npairs = tokens * k, nexp = ne + 1;
     for (u32 i = tid; i < nexp; i += 1024) {
         s_cnt[i] = 0;
         s_fill[i] = 0;
     }
+    if (tid < 18) s_class[tid / 9][tid % 9] = 0;
     __syncthreads();
-    for (u32 p = tid; p < npairs; p += 1024) {
-        const u32 e = tidx[p];
-        if (e < ne) atomicAdd(&s_cnt[e], 1u);
-    }
+    // 32 pairs of a thread's in flight at a time: the loads' round trips are what this launch is made of
+    auto pairs = [&](auto each) {
+        for (u32 p0 = tid; p0 < npairs; p0 += 32 * 1024) {
+            u32 e[32];
+#pragma unroll
+            for (int q = 0; q < 32; q++) e[q] = tidx[min(p0 + 1024 * q, npairs - 1)];
+#pragma unroll
+            for (int q = 0; q < 32; q++)
+                if (p0 + 1024 * q < npairs && e[q] < ne) each(p0 + 1024 * q, e[q]);
+        }
+    };
+    pairs([&](u32, u32 e) { atomicAdd(&s_cnt[e], 1u); });
     if (tid == 0) s_cnt[ne] = nshared;
-    for (u32 j = tid; j < tokens; j += 1024) {
-        u32 c = 0;
-        for (u32 t = 0; t < k; t++) c += tidx[j * k + t] < ne ? 1u : 0u;
-        cnt[j] = c;
-    }
     __syncthreads();
     // three running sums over the experts, each by a wave of its own: lane L takes the experts [9 L, 9 L + 9) (ne <= 512), the
-    // lanes' totals are scanned across the wave, and every lane writes its experts' starts
+    // lanes' totals are scanned across the wave, and every lane writes its experts' starts: of the pairs, of the full items of
+    // either list
     {
         const u32 w = tid >> 6, lane = tid & 63;
         if (w < 3) {
-            const u32 unit = w == 0 ? 1u : w == 1 ? unit_gu : unit_d;   // pairs; gate/up items; down items
+            const u32 unit = w == 0 ? 1u : w == 1 ? unit_gu : unit_d;
             u32 v[9], sum = 0;
 #pragma unroll
             for (int q = 0; q < 9; q++) {
                 const u32 i = 9 * lane + q;
-                v[q] = i < nexp ? (s_cnt[i] + unit - 1) / unit : 0u;
+                v[q] = i < nexp ? s_cnt[i] / unit : 0u;
                 sum += v[q];
             }
             u32 incl = sum;
@@ -139,7 +145,7 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
                 if (lane >= (u32) o) incl += up;
             }
             u32 run = incl - sum;
-            u32* dst = w == 0 ? s_off : w == 1 ? s_fill : s_fill_d;   // s_fill is borrowed until the barrier below; it is cleared again before the fill
+            u32* dst = w == 0 ? s_off : s_full[w - 1];
 #pragma unroll
             for (int q = 0; q < 9; q++) {
                 const u32 i = 9 * lane + q;
@@ -148,32 +154,43 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
             }
             if (lane == 63) {
                 if (w == 0) s_off[nexp] = incl;
-                else if (w == 1) items[0] = incl;
-                else items_d[0] = incl;
+                else s_class[w - 1][0] = incl;
+            }
+        } else {
+            // the items that are not full, by the number of their tiles of 16 pairs
+            for (u32 i = tid - 192; i < 2 * nexp; i += 1024 - 192) {
+                const u32 l = i >= nexp ? 1u : 0u, unit = l ? unit_d : unit_gu, rest = s_cnt[i - l * nexp] % unit;
+                if (rest) atomicAdd(&s_class[l][1 + min((unit - rest) / 16, 7u)], 1u);
             }
         }
     }
     __syncthreads();
-    for (u32 i = tid; i < nexp; i += 1024) {
-        u32 ni = s_fill[i];
-        for (u32 t0 = 0; t0 < s_cnt[i]; t0 += unit_gu, ni++) {
-            items[1 + 2 * ni] = i;
-            items[2 + 2 * ni] = t0;
+    if (tid < 2) {   // where the full ones end and each class begins, the longest first
+        u32 run = 0;
+        for (u32 c = 0; c < 9; c++) {
+            const u32 n = s_class[tid][c];
+            s_class[tid][c] = run;
+            run += n;
         }
-        ni = s_fill_d[i];
-        for (u32 t0 = 0; t0 < s_cnt[i]; t0 += unit_d, ni++) {
-            items_d[1 + 2 * ni] = i;
-            items_d[2 + 2 * ni] = t0;
-        }
+        (tid ? items_d : items)[0] = run;
     }
     __syncthreads();
-    for (u32 i = tid; i < nexp; i += 1024) s_fill[i] = 0;
-    __syncthreads();
+    for (u32 i = tid; i < 2 * nexp; i += 1024) {
+        const u32 l = i >= nexp ? 1u : 0u, e = i - l * nexp, unit = l ? unit_d : unit_gu, n = s_cnt[e], rest = n % unit;
+        u32* to = l ? items_d : items;
+        u32 at = s_full[l][e], t0 = 0;
+        for (; t0 + unit <= n; t0 += unit, at++) {
+            to[1 + 2 * at] = e;
+            to[2 + 2 * at] = t0;
+        }
+        if (rest) {
+            at = atomicAdd(&s_class[l][1 + min((unit - rest) / 16, 7u)], 1u);
+            to[1 + 2 * at] = e;
+            to[2 + 2 * at] = t0;
+        }
+    }
     for (u32 i = tid; i <= nexp; i += 1024) offs[i] = s_off[i];
-    for (u32 p = tid; p < npairs; p += 1024) {
-        const u32 e = tidx[p];
-        if (e < ne) list[s_off[e] + atomicAdd(&s_fill[e], 1u)] = p;
-    }
+    pairs([&](u32 p, u32 e) { list[s_off[e] + atomicAdd(&s_fill[e], 1u)] = p; });
     for (u32 j = tid; j < nshared; j += 1024) list[s_off[ne] + j] = npairs + j;
 }
 
