@@ -722,8 +722,9 @@ int head_argmax_mfma(sz_session* s, uint32_t m, uint64_t u, uint64_t logits, uin
 
 bool head_is_exl3(const sz_session* s) { return s->head_type >= 1021 && s->head_type <= 1028; }
 
-// LDS of a workgroup of head_exl3_K for m rows: the four waves' 4-row rings (static; a row is 64 lanes x 4 words at K = 3 and
-// 4, x K words otherwise) and the A rows, 4 KiB for every 512 inputs and every two rows (dynamic).
+// What bounds the rows a call of an EXL3 head takes (kept from when its A rows lay in LDS: callers size their batches by it): the bytes of
+// four 4-row rings (a row is 64 lanes x 4 words at K = 3 and 4, x K words otherwise) and 4 KiB of A rows for every 512 inputs and
+// every two rows, against a compute unit's.
 uint32_t exl3_head_lds_dynamic(uint32_t hidden, uint32_t m) { return 4 * ((hidden / 128 + 3) / 4) * ((m + 1) / 2) * 1024; }
 uint32_t exl3_head_lds(uint32_t bits, uint32_t hidden, uint32_t m) {
     const uint32_t stride = (bits == 3 || bits == 4) ? 4 : bits;
@@ -745,19 +746,24 @@ int head_check(sz_session* s, uint32_t m, uint64_t u, const char* who) {
 // buffer for them).
 bool head_argmax_fused(const sz_session* s) { return s->head_type == SZ_TYPE_Q8_0 || head_is_exl3(s); }
 
+// The product launch of an EXL3 head over n output blocks (sel: a list of them, 0: all).
+int head_exl3_blocks(sz_session* s, uint32_t n, uint32_t m, uint64_t logits, uint32_t ls, uint64_t sel, uint64_t stream) {
+    const sz_session_config& c = s->cfg;
+    const sz_arg a[] = {P(s->head_w), P(s->head_xa.ptr), P(s->head_inv.ptr), P(logits), U32(ls), P(s->head_part.ptr), U32(c.hidden), U32(c.vocab), U32(m), P(sel)};
+    return launch(("head_exl3_" + std::to_string(s->head_type - 1020)).c_str(), n, 1, 1, 256, 0, stream, a);
+}
+
 // An EXL3 head (kernels/exl3.cu:349-461, 610-625 of the reference: rotate the rows once, then one pass over the matrix for all
 // m <= 8 rows): the arg-max ids (0: not wanted) and / or the logits (0: not written).
 int head_exl3(sz_session* s, uint32_t m, uint64_t u, uint64_t logits, uint64_t ids, uint64_t stream, const Accept* accept = nullptr) {
     const sz_session_config& c = s->cfg;
-    const uint32_t kbs = c.hidden / 128, bits = (uint32_t) s->head_type - 1020;
+    const uint32_t kbs = c.hidden / 128;
     {
         const sz_arg a[] = {P(s->head_w), P(u), U32(c.hidden), P(s->head_xa.ptr), P(s->head_inv.ptr), U32(c.hidden)};
         if (launch("exl3_head_rotate", m, 1, 1, 64 * std::min<uint32_t>(16, kbs), 0, stream, a)) return 1;
     }
-    const uint32_t nparts = c.vocab / 128, lds = exl3_head_lds_dynamic(c.hidden, m);
-    const std::string kn = "head_exl3_" + std::to_string(bits);
-    const sz_arg a[] = {P(s->head_w), P(s->head_xa.ptr), P(s->head_inv.ptr), P(logits), U32(c.vocab), P(s->head_part.ptr), U32(c.hidden), U32(c.vocab), U32(m), P(0)};
-    if (launch(kn.c_str(), nparts, 1, 1, 256, lds, stream, a)) return 1;
+    const uint32_t nparts = c.vocab / 128;
+    if (head_exl3_blocks(s, nparts, m, logits, c.vocab, 0, stream)) return 1;
     if (!ids) return 0;
     return merge_parts(s, nparts, 8, m, ids, accept, stream);
 }
@@ -774,7 +780,7 @@ uint32_t head_proxy_k_use(const sz_session* s, uint32_t need_k) {
 // Leaves the list in hp.sel and the packed logits (rows max_sel * 128 apart) in hp.logits; *max_sel_out = the list's bound.
 int head_proxy_sparse(sz_session* s, uint32_t m, uint64_t u, uint32_t need_k, uint32_t* max_sel_out, uint64_t stream) {
     const sz_session_config& c = s->cfg;
-    const uint32_t kbs = c.hidden / 128, n_ob = c.vocab / 128, bits = (uint32_t) s->head_type - 1020;
+    const uint32_t kbs = c.hidden / 128, n_ob = c.vocab / 128;
     const uint32_t k_use = head_proxy_k_use(s, need_k), max_sel = std::min(m * k_use, n_ob);
     {
         const sz_arg a[] = {P(s->head_w), P(u), U32(c.hidden), P(s->head_xa.ptr), P(s->head_inv.ptr), U32(c.hidden)};
@@ -797,11 +803,7 @@ int head_proxy_sparse(sz_session* s, uint32_t m, uint64_t u, uint32_t need_k, ui
         const sz_arg a[] = {P(s->hp.seen.ptr), U32(n_ob), U32(max_sel), P(s->hp.sel.ptr)};
         if (launch("proxy_compact_seen", 1, 1, 1, 64, 0, stream, a)) return 1;
     }
-    const uint32_t lds = exl3_head_lds_dynamic(c.hidden, m);
-    const std::string kn = "head_exl3_" + std::to_string(bits);
-    const sz_arg a[] = {P(s->head_w), P(s->head_xa.ptr), P(s->head_inv.ptr), P(s->hp.logits.ptr), U32(max_sel * 128), P(s->head_part.ptr),
-                        U32(c.hidden), U32(c.vocab), U32(m), P(s->hp.sel.ptr)};
-    if (launch(kn.c_str(), max_sel, 1, 1, 256, lds, stream, a)) return 1;
+    if (head_exl3_blocks(s, max_sel, m, s->hp.logits.ptr, max_sel * 128, s->hp.sel.ptr, stream)) return 1;
     *max_sel_out = max_sel;
     return 0;
 }

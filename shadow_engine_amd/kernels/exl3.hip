@@ -1044,7 +1044,8 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 // Launch 1 of the head: token j = blockIdx.x.  Wave w rotates the 128-blocks w, w + waves, .. of x_j (x * suh, the
 // transform), the largest magnitude over the row gives the token's scale, and the scaled values go out as f16 high and
-// low parts: xa[(kb * 16 + 2 j + part) * 128 + 16 t8 + slot] for tile row t8 of block kb; inv[j] undoes the scale.
+// low parts, as the lanes take them: xa[((kb * 4 + t8 / 2) * 64 + 16 (slot / 4) + 2 j + part) * 8 + 4 (t8 % 2) + slot % 4] for tile row t8 of block
+// kb; inv[j] undoes the scale.
 // grid = m, block = 64 * min(16, in / 128).
 #define EXL3_HEAD_NB 4   /* 128-blocks a wave rotates at most: in <= 8192 */
 extern "C" __global__ void __launch_bounds__(1024) exl3_head_rotate(const u8* blob, const float* x, u32 xs, u16* xa, float* inv, u32 in_f) {
@@ -1079,101 +1080,72 @@ extern "C" __global__ void __launch_bounds__(1024) exl3_head_rotate(const u8* bl
     for (int q = 0; q < EXL3_HEAD_NB; q++) {
         const u32 kb = wave + nw * q;
         if (kb < kbs) {
-            u16* blk = xa + ((u64) kb * 16 + 2 * j) * 128;
+            u16* blk = xa + (u64) kb * 2048 + 2 * j * 8;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const u32 i = lane + 64 * h;
                 const float v = rot[q][h] * scale;
                 const _Float16 hi = (_Float16) v;
                 const _Float16 lo = (_Float16) (v - (float) hi);
-                const u32 at = 16 * (i >> 4) + exl3_aslot(i & 15);
+                const u32 t8 = i >> 4, slot = exl3_aslot(i & 15), at = ((t8 >> 1) * 64 + 16 * (slot >> 2)) * 8 + 4 * (t8 & 1) + (slot & 3);
                 blk[at] = __builtin_bit_cast(u16, hi);
-                blk[128 + at] = __builtin_bit_cast(u16, lo);
+                blk[at + 8] = __builtin_bit_cast(u16, lo);
             }
         }
     }
 }
 
-// Launch 2 of the head: output block ob = blockIdx.x (128 columns of the vocabulary).  Wave w of 4 takes the 128-blocks
-// w, w + 4, .. of the input (8 tile rows each) through a ring of 4 rows; its A rows (2 m rows of 128 f16 a block, copied
-// from xa once, in units of 4 rows) sit in LDS.  The four waves' sums are added in wave order, scaled back, taken through
-// the output-side transform and scales, optionally stored as logits[j * ls + column], and the block's best column of every
-// row goes to part[(ob * 8 + j) * 2] = {value bits, column} (a NaN counts as -inf, ties to the lower column).
+// Launch 2 of the head: output block ob = blockIdx.x (128 columns of the vocabulary).  Wave w of 4 takes the 128-blocks w, w + 4, .. of the
+// input, in units of two tile rows: the trellis and the A rows of a unit come through a ring of two slots.  The four waves' sums
+// are added in wave order, scaled back, taken through the output-side transform and scales, optionally stored as logits[j * ls +
+// column], and the block's best column of every row goes to part[(ob * 8 + j) * 2] = {value bits, column} (a NaN counts as -inf, ties
+// to the lower column).
 // With a block list (sel[0] = n, sel[1 ..] = blocks; matvec_cols_exl3_pre_sparse of the reference, exl3.cu tail) workgroup
 // i < n takes block sel[1 + i] and its logits and best go to place i instead of ob: logits[j * ls + 128 i + column in block];
 // the arithmetic of a block does not depend on which workgroup runs it, so these are the bits the full pass gives.
-// grid = out / 128 (or the list's bound), block 256, dynamic LDS = 4 * ceil(in / 512) * ceil(m / 2) KiB.
+// Bound by the decode (60 vector cycles for four weights a lane: 41 us of 151936 x 2048 at 4 bits).  Five workgroups a compute unit
+// (24 KiB of LDS and 102 registers each), so that the 1187 blocks of that size are one round: 51 us; with all of a wave's A rows in
+// LDS three fitted, 1.55 rounds that took two: 57.8 (8 rows of 4096 inputs: the hand-off of the 64 best 199 -> 132 us).  Tried: a workgroup of 16 waves a compute unit with its A rows in registers, block
+// after block: 57.8 too, the ends of a block are nobody else's time there.
+// grid = out / 128 (or the list's bound), block 256.
+#define EXL3_HEAD_OCC(K) ((K) <= 5 ? 5 : 3)
 template <int K>
 __device__ __forceinline__ void exl3_head_kernel(const u8* __restrict__ blob, const u16* __restrict__ xa, const float* __restrict__ inv,
                                                  float* __restrict__ logits, u32 ls, u32* __restrict__ part, u32 in_f, u32 out_f, u32 m,
                                                  const u32* __restrict__ sel) {
-    constexpr int D = 4;
-    typedef Exl3Rows<K, D> R;
-    constexpr int stride = R::stride, ur = R::unit_rows;
+    typedef VerifyRing<K, false, 8, 2> R;
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    constexpr int D = R::D, SLOT = R::UW + 256;                             // words of a slot: the unit's tiles, its A rows
     constexpr bool one_shift = 16 + 3 * K <= 32;
-    extern __shared__ __attribute__((aligned(16))) u16 a_sh[];            // [wave][its blocks][4 nq A rows][128]; afterwards the waves' sums
-    __shared__ __attribute__((aligned(16))) u32 wb_all[4][R::words];
+    __shared__ __attribute__((aligned(16))) u32 lds[4 * D * SLOT > 4096 ? 4 * D * SLOT : 4096];   // the rings; afterwards the waves' sums [wave][row][128]
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, at = blockIdx.x;
     if (sel && at >= sel[0]) return;                                       // a list shorter than the grid
     const u32 ob = sel ? sel[1 + at] : at;
-    const u32 kbs = in_f / 128, nkbw = (kbs + 3) / 4, nq = (m + 1) / 2;
-    const u32 nkb = wave < kbs ? (kbs - wave + 3) / 4 : 0;                 // this wave's blocks: wave, wave + 4, ..
-    const u32 nr = nkb * 8;
-    const u32 nt = out_f / 16;
-    const u64 pitch = (u64) nt * EXL3_TILE_WORDS(K, false);
-    const u32* tr = (const u32*) (blob + 2 * (u64) in_f + 2 * (u64) out_f + 4) + (u64) ob * 8 * EXL3_TILE_WORDS(K, false);
-    const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wb_all[wave]));
-    u16* aw = a_sh + (u64) wave * nkbw * nq * 512;                        // 512 f16 = 1 KiB = 4 A rows
-    const u32 aw_lds = __builtin_amdgcn_readfirstlane(lds_offset(aw));
-    // relative row i of the wave is tile row (wave + 4 (i / 8)) * 8 + i % 8 of the matrix
-    auto row_ptr = [&](u32 i) -> const u32* { return tr + (u64) ((wave + 4 * (i >> 3)) * 8 + (i & 7)) * pitch; };
-    auto issue = [&](u32 i) {                   // the unit that starts at relative row i (a multiple of ur) into its ring slot
-        const u32 slot = i & (D - 1);
-        if constexpr (K == 4 || K == 3) {
-            lds_load<4 * K>(row_ptr(i) + lane * K, wb_lds + slot * 1024);
-        } else if constexpr (K == 2) {
-            lds_load<16>(row_ptr(i + (lane >> 5)) + (lane & 31) * 4, wb_lds + slot * 512);
-        } else {
+    const u32 kbs = in_f / 128, total = wave < kbs ? (kbs - wave + 3) / 4 * 4 : 0u;   // this wave's units: four of each of the 128-blocks wave, wave + 4, ..
+    const u32 row = lane & 15, a = lane >> 4;
+    u32* wb = lds + wave * (D * SLOT);
+    const u32 wb_lds = __builtin_amdgcn_readfirstlane(lds_offset(wb));
+    const u32 pitch = out_f / 16 * (4 * R::TW);
+    const u64 base = uniform_u64((u64) (blob + 2 * (u64) in_f + 2 * (u64) out_f + 4) + (u64) ob * (8 * 4 * R::TW));
+    R ring;
+    ring.init((const u8*) base, pitch, total, wb_lds, lane);
+    auto request = [&](u32 unit, u32 slot) {
+        const u32 pair = (wave + (unit & ~3u)) * 4 + (unit & 3);           // of tile rows: 4 (wave + 4 (unit / 4)) + unit % 4
+        const u64 from = base + (u64) (2 * pair) * pitch;
 #pragma unroll
-            for (int d = 0; d < K; d++) lds_load<4>(row_ptr(i) + d * 64 + lane, wb_lds + slot * 256 * K + d * 256);
-        }
+        for (int i = 0; i < R::NI; i++)
+            if (64 * (i + 1) <= 16 * R::CH || 64 * i + lane < 16 * R::CH) lds_load_at(from, ring.off[i], wb_lds + (slot * SLOT + i * 256) * 4);
+        lds_load<16>((const u8*) xa + (u64) pair * 1024 + lane * 16, wb_lds + (slot * SLOT + R::UW) * 4);
     };
-    // the wave's A rows first (nq KiB a block), then its first rows
-    for (u32 kbl = 0; kbl < nkb; kbl++)
-        for (u32 qi = 0; qi < nq; qi++)
-            lds_load<16>((const u8*) xa + ((u64) (wave + 4 * kbl) * 16 + 4 * qi) * 256 + lane * 16, aw_lds + (kbl * nq + qi) * 1024);
-    u32 nring = 0;
-    for (u32 i = 0; i < (u32) D && i < nr; i += ur) {
-        issue(i);
-        nring += R::unit_loads;
-    }
-    // the A rows have landed once only the ring's loads are in flight (at most 4 K of them: K <= 8)
-    switch (nring) {
-        case 0: wait_vm<0>(); break;
-        case 1: wait_vm<1>(); break;
-        case 2: wait_vm<2>(); break;
-        case 3: wait_vm<3>(); break;
-        case 4: wait_vm<4>(); break;
-        case 5: wait_vm<5>(); break;
-        case 6: wait_vm<6>(); break;
-        case 7: wait_vm<7>(); break;
-        case 8: wait_vm<8>(); break;
-        case 12: wait_vm<12>(); break;
-        case 16: wait_vm<16>(); break;
-        case 20: wait_vm<20>(); break;
-        case 24: wait_vm<24>(); break;
-        case 28: wait_vm<28>(); break;
-        case 32: wait_vm<32>(); break;
-        default: wait_vm<0>(); break;
-    }
-    const u32 n = lane & 15, a = lane >> 4;
-    const u32 t0 = 32 * (n & 7) + 8 * a + 4 * (n >> 3);
-    // the 32 stream bits that end at bit e (exclusive) of the tile's ring: word jp holds the last of them, word jm the rest
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if ((u32) d < total) request(d, d);                                // four units at least, if any
+    const u32 t0 = 32 * (row & 7) + 8 * a + 4 * (row >> 3);
+    // the 32 stream bits that end at bit e (exclusive) of the tile's ring: word op holds the last of them, word om the rest
     auto window = [&](u32 e, u32& om, u32& op, u32& sh) {
-        const u32 jp = (e - 1) >> 5, jm = (jp + 8 * K - 1) % (8 * K);
+        op = (e - 1) >> 5;
+        om = op == 0 ? R::TW - 1 : op - 1;
         sh = 31 - ((e - 1) & 31);
-        om = (jm / K) * stride + jm % K;   // a tile's word j sits at decode lane j / K, word j % K of that lane
-        op = (jp / K) * stride + jp % K;
     };
     u32 om1, op1, sh1, om0 = 0, op0 = 0, sh0 = 0;
     window((t0 + 4) * K, om1, op1, sh1);
@@ -1181,116 +1153,75 @@ __device__ __forceinline__ void exl3_head_kernel(const u8* __restrict__ blob, co
     f32x4 acc[8];
 #pragma unroll
     for (int c = 0; c < 8; c++) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bool fed = n < 2 * m;                            // this lane supplies A row n
-    const u16* xa0 = aw + (fed ? n : 0) * 128 + 4 * a;
-    const u32* wb = wb_all[wave];
-    typedef u32 u32x2 __attribute__((ext_vector_type(2)));
-    if constexpr (one_shift && ur == 1) {
-        // Two tile rows a step on the 32-deep matrix instruction (a lane's 4 + 4 weights of the two rows' tiles against its 4 + 4
-        // A values: the contraction runs over both rows' inputs), half the matrix instructions.  nr is a multiple of 8.
-        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-        typedef u32 u32x4v __attribute__((ext_vector_type(4)));
+    const bool fed = row < 2 * m;                                          // this lane supplies A row `row`
 #pragma unroll 1
-        for (u32 i = 0; i < nr; i += 2) {
-            u32 w1[2][8][2];
-            u32x2 xv[2];
+    for (u32 unit = 0; unit < total; unit++) {
+        if (unit + 1 < total) wait_vm<R::NI + 1>();
+        else wait_vm<0>();
+        const u32* words = wb + (unit & 1) * SLOT;
+        u32 w1[16][2], w0[one_shift ? 1 : 16][2];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            w1[i][0] = words[i * R::TW + om1];
+            w1[i][1] = words[i * R::TW + op1];
+            if constexpr (!one_shift) {
+                w0[i][0] = words[i * R::TW + om0];
+                w0[i][1] = words[i * R::TW + op0];
+            }
+        }
+        u32x4 av = *(const u32x4*) (words + R::UW + lane * 4);
+        if (!fed) av = u32x4{0u, 0u, 0u, 0u};
+        if (unit + D < total) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the unit's words are in registers, its slot can take the unit D further on
+            request(unit + D, unit & 1);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            u32 b[2][2];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const u32 r = i + h;
-                exl3_rows_wait<K, D>(r + D > nr ? r + D - nr : 0);
-                const u32* row = wb + (r & (D - 1)) * R::row_words;
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    w1[h][c][0] = row[c * 8 * stride + om1];
-                    w1[h][c][1] = row[c * 8 * stride + op1];
+                const int i = 8 * h + c;
+                const u32 top = __builtin_amdgcn_alignbit(w1[i][0], w1[i][1], sh1);
+                u32 s0, s1;
+                if constexpr (one_shift) {
+                    s0 = __builtin_amdgcn_ubfe(top, 3 * K, 16);
+                    s1 = __builtin_amdgcn_ubfe(top, 2 * K, 16);
+                } else {
+                    const u32 low = __builtin_amdgcn_alignbit(w0[i][0], w0[i][1], sh0);
+                    s0 = __builtin_amdgcn_ubfe(low, K, 16);
+                    s1 = low & 0xffffu;
                 }
-                xv[h] = *(const u32x2*) (xa0 + (u64) (r >> 3) * nq * 512 + 16 * (r & 7));
-                if (!fed) xv[h] = u32x2{0u, 0u};
-                if (r + D < nr) {
-                    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the row's words are in registers, its slot can take the row D further on
-                    issue(r + D);
-                }
+                const u32 s2 = __builtin_amdgcn_ubfe(top, K, 16), s3 = top & 0xffffu;
+                b[h][0] = __builtin_bit_cast(u32, exl3_cb2_pair(s0, s1));
+                b[h][1] = __builtin_bit_cast(u32, exl3_cb2_pair(s2, s3));
             }
-            const f16x8 av = __builtin_bit_cast(f16x8, u32x4v{xv[0][0], xv[0][1], xv[1][0], xv[1][1]});
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                u32 b[2][2];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const u32 hi = __builtin_amdgcn_alignbit(w1[h][c][0], w1[h][c][1], sh1);
-                    const u32 s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16), s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
-                    const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
-                    b[h][0] = __builtin_bit_cast(u32, exl3_cb2_pair(s0, s1));
-                    b[h][1] = __builtin_bit_cast(u32, exl3_cb2_pair(s2, s3));
-                }
-                const f16x8 bv = __builtin_bit_cast(f16x8, u32x4v{b[0][0], b[0][1], b[1][0], b[1][1]});
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc[c], 0, 0, 0);
-            }
-        }
-    } else
-#pragma unroll 1
-    for (u32 i = 0; i < nr; i++) {
-        exl3_rows_wait<K, D>(i + D > nr ? i + D - nr : 0);
-        const u32* row = wb + (i & (D - 1)) * R::row_words;
-        u32 w1[8][2], w0[8][2];
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            w1[c][0] = row[c * 8 * stride + om1];
-            w1[c][1] = row[c * 8 * stride + op1];
-            if constexpr (!one_shift) {
-                w0[c][0] = row[c * 8 * stride + om0];
-                w0[c][1] = row[c * 8 * stride + op0];
-            }
-        }
-        u32x2 xv = *(const u32x2*) (xa0 + (u64) (i >> 3) * nq * 512 + 16 * (i & 7));
-        if (!fed) xv = u32x2{0u, 0u};
-        // the row's words are in registers once the reads have returned: its slot can take the row D further on
-        if ((i + 1) % ur == 0 && i + D + 1 - ur < nr) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-            issue(i + D + 1 - ur);
-        }
-        const f16x4 av = __builtin_bit_cast(f16x4, xv);
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const u32 hi = __builtin_amdgcn_alignbit(w1[c][0], w1[c][1], sh1);
-            u32 s0, s1;
-            if constexpr (one_shift) {
-                s0 = __builtin_amdgcn_ubfe(hi, 3 * K, 16);
-                s1 = __builtin_amdgcn_ubfe(hi, 2 * K, 16);
-            } else {
-                const u32 lo = __builtin_amdgcn_alignbit(w0[c][0], w0[c][1], sh0);
-                s0 = __builtin_amdgcn_ubfe(lo, K, 16);
-                s1 = lo & 0xffffu;
-            }
-            const u32 s2 = __builtin_amdgcn_ubfe(hi, K, 16), s3 = hi & 0xffffu;
-            const f16x2 b01 = exl3_cb2_pair(s0, s1), b23 = exl3_cb2_pair(s2, s3);
-            const f16x4 bv = {b01[0], b01[1], b23[0], b23[1]};
-            acc[c] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, acc[c], 0, 0, 0);
+            const f16x8 bv = __builtin_bit_cast(f16x8, u32x4{b[0][0], b[0][1], b[1][0], b[1][1]});
+            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, av), bv, acc[c], 0, 0, 0);
         }
     }
-    __syncthreads();                                       // every wave is done with its A rows: the space takes the sums
-    // D rows 4 a + i: lane group a holds tokens 2 a and 2 a + 1 (high part + low part each); red[wave][token][128]
-    float* red = (float*) a_sh;
+    __syncthreads();                                       // every wave is done with its ring: the space takes the sums
+    // D rows 4 a + i: lane group a holds tokens 2 a and 2 a + 1 (high part + low part each)
+    float* red = (float*) lds;
     {
         float* o = red + (u64) wave * m * 128;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
-            if (2 * a < m) o[(2 * a) * 128 + 16 * c + n] = acc[c][0] + acc[c][1];
-            if (2 * a + 1 < m) o[(2 * a + 1) * 128 + 16 * c + n] = acc[c][2] + acc[c][3];
+            if (2 * a < m) o[(2 * a) * 128 + 16 * c + row] = acc[c][0] + acc[c][1];
+            if (2 * a + 1 < m) o[(2 * a + 1) * 128 + 16 * c + row] = acc[c][2] + acc[c][3];
         }
     }
     __syncthreads();
-    const u16* svh = (const u16*) (blob + 2 * (u64) in_f) + ob * 128;
-    const float sv0 = f16_to_f32(svh[lane]), sv1 = f16_to_f32(svh[lane + 64]);
     for (u32 j = wave; j < m; j += 4) {
+        const u16* svh = (const u16*) (blob + 2 * (u64) in_f) + ob * 128;
+        const float sv0 = f16_to_f32(svh[lane]), sv1 = f16_to_f32(svh[lane + 64]);
         float v0 = 0.0f, v1 = 0.0f;
         for (u32 w = 0; w < 4; w++) {
             v0 += red[((u64) w * m + j) * 128 + lane];
             v1 += red[((u64) w * m + j) * 128 + lane + 64];
         }
-        const float iv = inv[j];
-        v0 *= iv;
-        v1 *= iv;
+        const float f = inv[j];
+        v0 *= f;
+        v1 *= f;
         wht128_wave(v0, v1, lane);
         v0 *= sv0;
         v1 *= sv1;
@@ -1439,13 +1370,12 @@ extern "C" __global__ void __launch_bounds__(64) proxy_q2_quant_x(const u8* blob
     }
 }
 
-#define EXL3_HEAD_ENTRIES(K)                                                                                                          \
-    extern "C" __global__ void __launch_bounds__(256) head_exl3_##K(const u8* blob, const u16* xa, const float* inv, float* logits, u32 ls, \
-                                                                     u32* part, u32 in_f, u32 out_f, u32 m, const u32* sel) {             \
-        exl3_head_kernel<K>(blob, xa, inv, logits, ls, part, in_f, out_f, m, sel);                                                    \
-    }                                                                                                                                 \
+#define EXL3_HEAD_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_HEAD_OCC(K)) head_exl3_##K(const u8* blob, const u16* xa, const float* inv, float* logits, u32 ls, u32* part, u32 in_f, u32 out_f, u32 m, const u32* sel) { \
+        exl3_head_kernel<K>(blob, xa, inv, logits, ls, part, in_f, out_f, m, sel); \
+    } \
     extern "C" __global__ void __launch_bounds__(256) exl3_build_q2_proxy_##K(const u8* blob, u32* w_q2, u16* w_sc, u32 in_f, u32 out_f) { \
-        exl3_q2_proxy_build<K>(blob, w_q2, w_sc, in_f, out_f);                                                                        \
+        exl3_q2_proxy_build<K>(blob, w_q2, w_sc, in_f, out_f); \
     }
 EXL3_HEAD_ENTRIES(1)
 EXL3_HEAD_ENTRIES(2)
