@@ -1426,7 +1426,9 @@ int32_t sz_hc_read(sz_hc* h, uint32_t m, uint64_t r, uint64_t u, uint64_t stream
     if (m == 0 || m > c.max_rows) return fail("sz_hc_read: " + std::to_string(m) + " rows (1.." + std::to_string(c.max_rows) + ")");
     if ((r & 15) || (u & 15)) return fail("sz_hc_read: rows must be 16-byte aligned");
     const DenseShape d = dense_shape((uint64_t) c.hidden * c.streams);
-    const uint32_t pass = d.block / 64 / d.waves;   // whole rows, a wave or more each
+    const uint32_t group = d.block / 64 / d.waves;   // whole rows, a wave or more each
+    const uint64_t ch = (uint64_t) c.hidden * c.streams;
+    const uint32_t groups = (c.rank + group - 1) / group + (c.inject_w ? (c.streams + group - 1) / group : 0);
     const DenseShape du = dense_shape(c.rank);
     const uint32_t per = 4 * std::max<uint32_t>(1, du.pass / (du.block / 64 / du.waves));   // 4 waves of 64 / G columns
     // LDS of the first launch: the sums of squares of every stream's spans (of at least 256 columns) and its scale; as many rows
@@ -1436,11 +1438,18 @@ int32_t sz_hc_read(sz_hc* h, uint32_t m, uint64_t r, uint64_t u, uint64_t stream
     const uint32_t lot = (uint32_t) std::min<uint64_t>(m, std::max<uint64_t>(1, 80000 / lds));
     for (uint32_t j = 0; j < m; j += lot) {
         const uint32_t n = std::min(lot, m - j);
+        // Rows one after the other in a workgroup of the first launch, as many (of its 4) as bring the launch down to a workgroup a
+        // compute unit: each normalises all inputs in f64 for itself, and two on one unit take turns at that.  A read and a write,
+        // bf16, rank 320: 4 rows of 8192 columns 19.1 us with 324 workgroups of a row, 17.0 with 162 of two (17.4 with three), 4 rows
+        // of 16384 28.3 and 24.9; rank 512: 6 rows of 6144 37.7 us with a row each, 24.9 with three.  One row of more than 8192
+        // columns, which has little to normalise and is bound by its loads' latency, is better off with two workgroups a unit: 17.6
+        // and 18.1 us.  A row each has kernels of its own (the loop over rows costs them 3 to 5%).
+        const uint32_t units = n == 1 && ch > 8192 ? 512 : 256, np = std::min(4u, (groups + units - 1) / units), pass = group * np;
         const uint64_t rj = r + (uint64_t) j * c.hidden * c.streams * 4, sc = h->scales.ptr + (uint64_t) j * c.streams * 8, dj = h->down.ptr + (uint64_t) j * c.rank * 4;
         const sz_arg a[] = {U32(dense_code(c.down_type)), P(c.down_w), U32(c.rank), U32(dense_code(c.inject_type)), P(c.inject_w), P(rj), P(c.norm_w), P(sc),
-                            P(dj), P(h->g.ptr + (uint64_t) j * c.streams * 4), U32(c.hidden), U32(c.streams), U32(n), F32(c.eps)};
-        if (launch((std::string("hc_down_m") + dense_m(n)).c_str(), (c.rank + pass - 1) / pass + (c.inject_w ? (c.streams + pass - 1) / pass : 0), 1, 1, d.block,
-                   (uint32_t) (n * lds), stream, a))
+                            P(dj), P(h->g.ptr + (uint64_t) j * c.streams * 4), U32(c.hidden), U32(c.streams), U32(n), F32(c.eps), U32(np)};
+        if (launch((std::string(np > 1 ? "hc_down_rows_m" : "hc_down_m") + dense_m(n)).c_str(),
+                   (c.rank + pass - 1) / pass + (c.inject_w ? (c.streams + pass - 1) / pass : 0), 1, 1, d.block, (uint32_t) (n * lds), stream, a))
             return 1;
         const sz_arg b[] = {U32(dense_code(c.up_type)), P(c.up_w), P(dj), P(rj), P(c.norm_w), P(sc), P(u + (uint64_t) j * c.hidden * 4), U32(c.hidden), U32(c.streams), U32(c.rank), U32(n)};
         if (launch((std::string("hc_up_m") + dense_m(n)).c_str(), (c.hidden + per - 1) / per, 1, 1, 256, 0, stream, b)) return 1;

@@ -1120,9 +1120,11 @@ extern "C" __global__ void __launch_bounds__(512) router_rows_m8(u32 type, const
 // The hyper-connection's read (forward.rs:797-812) in two launches.  The first: every stream of every row normalised, the mean
 // of squares and the scaling of every input in f64 as the CPU path has them, and the down and inject products of that.  A
 // workgroup owns `pass` rows of the two matrices (down's first) and normalises the inputs for itself: it has to read all of them
-// anyway, and the arithmetic is less than another launch costs.  Workgroup 0 leaves the scales 1/sqrt(ms + eps) for the second
-// launch.
-// r: [m][streams * h]; down, g: silu(t / streams), 2 sigmoid(t / streams).  grid = ceil(rank / pass) + ceil(streams / pass) (inject),
+// anyway, and the arithmetic is less than another launch costs.  That arithmetic, in f64, is what bounds it, not the weights: two
+// workgroups on a compute unit take nearly twice as long as one.  hc_down_rows_m* take np rows in each group of dense_waves(ch)
+// waves, one after the other, the next row's weights on their way, so that one workgroup a unit does (4 rows of 8192 bf16 columns,
+// rank 320: 11.9 us -> 9.2); hc_down_m* one row.  Workgroup 0 leaves the scales 1/sqrt(ms + eps) for the second launch.
+// r: [m][streams * h]; down, g: silu(t / streams), 2 sigmoid(t / streams).  grid = ceil(rank / pass) + ceil(streams / pass) (inject), np <= HC_NP (1 for hc_down_m*),
 // block 64 max(4, dense_waves(ch)), dynamic LDS = m * streams * (1 + chunks of ch) doubles.
 __device__ __forceinline__ double lane_xor_f64(double v, u32 lane, int h) {
     const u64 b = __builtin_bit_cast(u64, v);
@@ -1170,10 +1172,12 @@ __device__ __forceinline__ void hc_normalise(const DenseSlice<T>& sl, float (&xv
     }
 }
 
-template <class T, int M>
+#define HC_NP 4u   // rows of a wave at most
+template <class T, int M, bool MANY>
 __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows, u32 first, const float* __restrict__ r, const float* __restrict__ nw, double* __restrict__ scales,
-                                             u32 h, u32 cs, u32 m, float eps, float* red, u32 act, float* y, u32 ys) {
+                                             u32 h, u32 cs, u32 m, float eps, u32 np, float* red, u32 act, float* y, u32 ys) {
     typedef DenseSlice<T> S;
+    if constexpr (!MANY) np = 1;
     const u32 tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const u32 cols = h * cs, kwn = dense_waves(cols), rw = (blockDim.x >> 6) / kwn, rg = wave / kwn;
     const S sl{wave - rg * kwn, kwn, 64, lane, cols};
@@ -1182,16 +1186,16 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     const u32 wide = h / span + 2;
     double* scl = part + (u64) m * cs * wide;
     const bool live = rg < rw;
-    const u32 row = first + rg;
+    auto weights = [&](u32 q, u32 o, typename T::Raw (&raw)[S::NCH]) {   // of the wave's q-th row
+        const u32 row = first + q * rw + rg;
+        sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, o, live && o < outer && row < rows, raw);
+    };
     float xv[M][DENSE_LANE_COLS];
-    typename T::Raw wv[S::NCH];
-    sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, 0, live && row < rows, wv);
+    typename T::Raw wv[S::NCH], wn[S::NCH];
+    weights(0, 0, wv);
     sl.inputs(r, cols, m, 0, xv);
     for (u32 i = tid; i < m * cs * wide; i += blockDim.x) part[i] = 0.0;
     __syncthreads();
-    float acc[M];
-#pragma unroll
-    for (int j = 0; j < M; j++) acc[j] = 0.0f;
     // the spans' sums of squares first, then the products (of inputs that are still in registers where outer == 1)
     for (u32 o = 0; o < outer; o++) {
         if (o) sl.inputs(r, cols, m, o, xv);
@@ -1220,6 +1224,12 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     }
     float nv[1][DENSE_LANE_COLS];   // the norm weights come while the scales are made
     sl.inputs(nw, 0, 1, 0, nv);
+    u32 qn = 0, on = 0;   // the row and the columns that wn is of
+    auto next = [&]() {
+        if (++qn == np) qn = 0, on++;
+        weights(qn, on, wn);
+    };
+    if constexpr (MANY) next();
     __syncthreads();
     for (u32 i = tid; i < m * cs; i += blockDim.x) {
         double ss = 0.0;
@@ -1229,61 +1239,100 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
         if (blockIdx.x == 0) scales[i] = sc;
     }
     __syncthreads();
-    for (u32 o = 0; o < outer; o++) {
-        if (outer > 1) {
-            sl.weights(w + (u64) min(row, rows - 1) * cols * T::BYTES, o, live && row < rows, wv);
-            sl.inputs(r, cols, m, o, xv);
-            sl.inputs(nw, 0, 1, o, nv);
+    if constexpr (MANY) {
+        for (u32 o = 0; o < outer; o++) {
+            if (outer > 1) {
+                sl.inputs(r, cols, m, o, xv);
+                sl.inputs(nw, 0, 1, o, nv);
+            }
+            hc_normalise<T, M>(sl, xv, nv, scl, h, cs, m, o);
+            for (u32 q = 0; q < np; q++) {
+                float acc[M];
+#pragma unroll
+                for (int j = 0; j < M; j++) acc[j] = 0.0f;
+                sl.dot(wv, xv, acc);
+#pragma unroll
+                for (int i = 0; i < S::NCH; i++) wv[i] = wn[i];
+                next();
+                const float t = dense_reduce<M>(acc, 64, lane);
+                float* sum = red + (q * 8 + wave) * 8 + lane;   // the lane's own
+                if (live && lane < (u32) M) *sum = o ? *sum + t : t;
+            }
         }
-        hc_normalise<T, M>(sl, xv, nv, scl, h, cs, m, o);
-        sl.dot(wv, xv, acc);
+    } else {
+        float acc[M];
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[j] = 0.0f;
+        for (u32 o = 0; o < outer; o++) {
+            if (outer > 1) {
+                weights(0, o, wv);
+                sl.inputs(r, cols, m, o, xv);
+                sl.inputs(nw, 0, 1, o, nv);
+            }
+            hc_normalise<T, M>(sl, xv, nv, scl, h, cs, m, o);
+            sl.dot(wv, xv, acc);
+        }
+        const float t = dense_reduce<M>(acc, 64, lane);
+        if (live && lane < (u32) M) red[wave * 8 + lane] = t;
     }
-    const float t = dense_reduce<M>(acc, 64, lane);
-    if (live && lane < (u32) M) red[wave * 8 + lane] = t;
     __syncthreads();
-    const u32 q = tid / 8, j = tid & 7, orow = first + q;
-    if (q < rw && j < m && orow < rows) {
-        float s = red[q * kwn * 8 + j];
-        for (u32 v = 1; v < kwn; v++) s += red[(q * kwn + v) * 8 + j];
-        y[(u64) j * ys + orow] = dense_act(s, act, (float) cs);
+    const u32 orow = tid / 8, j = tid & 7, q = orow / rw, og = orow - q * rw;
+    if (q < np && j < m && first + orow < rows) {
+        const float* part8 = red + (q * 8 + og * kwn) * 8 + j;
+        float s = part8[0];
+        for (u32 v = 1; v < kwn; v++) s += part8[v * 8];
+        y[(u64) j * ys + first + orow] = dense_act(s, act, (float) cs);
     }
 }
-template <int M>
-__device__ __forceinline__ void hc_down_of(u32 type, const u8* w, u32 rows, u32 first, const float* r, const float* nw, double* scales, u32 h, u32 cs, u32 m, float eps, float* red,
+template <int M, bool MANY>
+__device__ __forceinline__ void hc_down_of(u32 type, const u8* w, u32 rows, u32 first, const float* r, const float* nw, double* scales, u32 h, u32 cs, u32 m, float eps, u32 np, float* red,
                                            u32 act, float* y, u32 ys) {
     // spans stay whole inside a stream's 4-column groups: 8 columns a load only where a stream is a multiple of 8
-    if (type == 0) hc_down_rows<DenseF32, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+    if (type == 0) hc_down_rows<DenseF32, M, MANY>(w, rows, first, r, nw, scales, h, cs, m, eps, np, red, act, y, ys);
     else if (type == 1) {
-        if (h % 8 == 0) hc_down_rows<Dense16<false, 8>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
-        else hc_down_rows<Dense16<false, 4>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+        if (h % 8 == 0) hc_down_rows<Dense16<false, 8>, M, MANY>(w, rows, first, r, nw, scales, h, cs, m, eps, np, red, act, y, ys);
+        else hc_down_rows<Dense16<false, 4>, M, MANY>(w, rows, first, r, nw, scales, h, cs, m, eps, np, red, act, y, ys);
     } else {
-        if (h % 8 == 0) hc_down_rows<Dense16<true, 8>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
-        else hc_down_rows<Dense16<true, 4>, M>(w, rows, first, r, nw, scales, h, cs, m, eps, red, act, y, ys);
+        if (h % 8 == 0) hc_down_rows<Dense16<true, 8>, M, MANY>(w, rows, first, r, nw, scales, h, cs, m, eps, np, red, act, y, ys);
+        else hc_down_rows<Dense16<true, 4>, M, MANY>(w, rows, first, r, nw, scales, h, cs, m, eps, np, red, act, y, ys);
     }
 }
-template <int M>
+template <int M, bool MANY>
 __device__ __forceinline__ void hc_down(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down, float* g, u32 h,
-                                        u32 cs, u32 m, float eps) {
-    __shared__ float red[64];
-    const u32 pass = (blockDim.x >> 6) / dense_waves(h * cs), groups = (rank + pass - 1) / pass;
-    if (blockIdx.x < groups) hc_down_of<M>(type, w, rank, blockIdx.x * pass, r, nw, (double*) scales, h, cs, m, eps, red, 1, down, rank);
-    else hc_down_of<M>(gate_type, gate_w, cs, (blockIdx.x - groups) * pass, r, nw, (double*) scales, h, cs, m, eps, red, 2, g, cs);
+                                        u32 cs, u32 m, float eps, u32 np) {
+    __shared__ float red[(MANY ? HC_NP : 1) * 64];
+    if constexpr (!MANY) np = 1;
+    const u32 pass = (blockDim.x >> 6) / dense_waves(h * cs) * np, groups = (rank + pass - 1) / pass;
+    if (blockIdx.x < groups) hc_down_of<M, MANY>(type, w, rank, blockIdx.x * pass, r, nw, (double*) scales, h, cs, m, eps, np, red, 1, down, rank);
+    else hc_down_of<M, MANY>(gate_type, gate_w, cs, (blockIdx.x - groups) * pass, r, nw, (double*) scales, h, cs, m, eps, np, red, 2, g, cs);
 }
 extern "C" __global__ void __launch_bounds__(512) hc_down_m1(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
-                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
-    hc_down<1>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<1, false>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
 }
 extern "C" __global__ void __launch_bounds__(512, 4) hc_down_m4(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
-                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
-    hc_down<4>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<4, false>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
 }
 extern "C" __global__ void __launch_bounds__(512) hc_down_m8(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
-                                                             float* g, u32 h, u32 cs, u32 m, float eps) {
-    hc_down<8>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps);
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<8, false>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_rows_m1(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<1, true>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_rows_m4(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<4, true>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
+}
+extern "C" __global__ void __launch_bounds__(512) hc_down_rows_m8(u32 type, const u8* w, u32 rank, u32 gate_type, const u8* gate_w, const float* r, const float* nw, u8* scales, float* down,
+                                                             float* g, u32 h, u32 cs, u32 m, float eps, u32 np) {
+    hc_down<8, true>(type, w, rank, gate_type, gate_w, r, nw, scales, down, g, h, cs, m, eps, np);
 }
 
 // The second: u[j][i] = (sum over the streams s, in order, of sigmoid(up row s h + i . down_j) * the normalised r[j][s h + i]) / streams.
-// A wave takes 64 / G columns i at a time and the streams' rows of them one after the other, the next row's weights on their
+// A wave takes 64 / G columns i at a time and the streams' rows of them one after the other, the next row's weights and terms on their
 // way, so that the sum over the streams needs nobody else.  grid = ceil(h / (4 * 64 / G)), block 256.
 template <class T, int M>
 __device__ __forceinline__ void hc_up_rows(const u8* __restrict__ w, const float* __restrict__ down, const float* __restrict__ r, const float* __restrict__ nw,
@@ -1304,11 +1353,18 @@ __device__ __forceinline__ void hc_up_rows(const u8* __restrict__ w, const float
     float a[M];
 #pragma unroll
     for (int j = 0; j < M; j++) a[j] = 0.0f;
+    float nn = nw[i], rn = r[(u64) j0 * cs * h + i];
+    double scn = scales[j0 * cs];
     for (u32 s = 0; s < cs; s++) {
         const u64 at = (u64) s * h + i;
-        if (s + 1 < cs) sl.weights(w + (at + h) * rank * T::BYTES, 0, true, wn);
-        const float n = nw[at], rv = r[(u64) j0 * cs * h + at];
-        const double sc = scales[j0 * cs + s];
+        const float n = nn, rv = rn;
+        const double sc = scn;
+        if (s + 1 < cs) {
+            sl.weights(w + (at + h) * rank * T::BYTES, 0, true, wn);
+            nn = nw[at + h];
+            rn = r[(u64) j0 * cs * h + at + h];
+            scn = scales[j0 * cs + s + 1];
+        }
         float acc[M];
 #pragma unroll
         for (int j = 0; j < M; j++) acc[j] = 0.0f;

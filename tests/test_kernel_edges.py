@@ -205,6 +205,16 @@ def test_hyper_connection_at_its_edges(gpu, ty, h, cs, rank, m, size):  # noqa: 
         assert np.allclose(g[j], wg_, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("ty,h,cs,rank,m", [
+    (sz.BF16, 2048, 4, 252, 4), (sz.BF16, 2048, 4, 256, 4),   # 256 workgroups of a row, and the first count with two
+    (sz.F32, 1536, 4, 764, 8), (sz.F16, 1600, 3, 516, 1),     # three rows each, the last workgroups not full
+    (sz.F16, 1152, 4, 2052, 3), (sz.BF16, 96, 4, 1028, 5),    # more than four each; four rows side by side, two of each after the other
+    (sz.F32, 2052, 4, 516, 2), (sz.BF16, 4096, 4, 516, 1)])   # inputs that do not stay in registers: three each, two for one input
+def test_hyper_connection_rows_of_a_workgroup(gpu, ty, h, cs, rank, m):  # noqa: F811
+    """The rows a workgroup takes one after the other, at the counts where their number changes."""
+    test_hyper_connection_at_its_edges(gpu, ty, h, cs, rank, m, 1.0)
+
+
 @pytest.mark.parametrize("ty", [sz.F32, sz.F16, sz.BF16])
 @pytest.mark.parametrize("rows,cols,m", [(9, 3072, 4), (5, 5000, 8), (6, 7168, 1), (17, 8192, 5), (3, 8196, 8), (1100, 9220, 3), (4, 20480, 4)])
 def test_unquantized_rows_of_several_waves_and_longer(gpu, ty, rows, cols, m):  # noqa: F811
