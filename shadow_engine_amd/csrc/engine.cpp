@@ -1306,10 +1306,11 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         }
         const uint32_t nt = ntl <= 2 ? ntl : ntl + ntl % 2, bits = (uint32_t) f.bits, wide_ring = bits <= 7 ? 3 : 2;
         {
-            // two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, where the items are few, fills the
-            // chip (3 bits, 512 experts of 2048 x 512, top-10: 45 tokens 102 and 120 us, 200 tokens 183 and 179, 512 262 and 256, 1024 381
-            // and 346; 600 tokens through 60 of 1024 x 256, top-8: 106 and 120; 1500 through 32 of 2048 x 512, top-4: 226 and 212)
-            const bool wide = rows * fbs >= 16000;
+            // two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, whose rings are deeper, where the
+            // work is little or where eight waves would leave compute units without a workgroup (3 bits, 512 experts of 2048 x 512, top-10:
+            // 45 tokens 102 us with four waves and 123 with eight, 200 tokens 178 and 176, 512 254 and 252, 1024 371 and 344; 600 tokens
+            // through 60 of 1024 x 256, top-8: 105 and 119; 2048 through 64 of 2048 x 512, top-4: 254 and 243; 1500 through 32: 177 and 188)
+            const bool wide = rows * fbs >= 16000 && max_items * fbs >= 512;
             const uint32_t ncb = wide ? 2 : 1;
             // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING, XPF_RING_N), afterwards the exchange of four tiles' sums
             uint32_t lds = ncb * 2 * std::min(4u, nt) * 8192;
@@ -1322,8 +1323,8 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         }
         {
             // shares of an item: one wave a column block in the end where items are few, all blocks on eight waves, whose start then counts
-            // once, where they fill the chip (1, 2 shares of 8 waves, 4 of 4: 45 tokens as above 138, 111, 102 us, 512 tokens 261, 256, 272,
-            // 4096 at 4 bits 968, 986, 1059)
+            // once, where they fill the chip (1, 2 shares of 8 waves, 4 of 4: 45 tokens as above 137, 109, 101 us, 512 tokens 257, 252, 267,
+            // 4096 at 4 bits 967, 988, 1071)
             const bool wide = rows >= 1800;
             const uint32_t waves = std::min(wide ? 8u : 4u, kbs), parts = std::max((kbs + 4 * waves - 1) / (4 * waves), std::min(rows >= 20000 ? 1u : wide ? 2u : 4u, kbs / waves)), nd = std::min(4u, nt);
             const uint32_t ring = wide ? wide_ring : bits <= 4 ? 8 : bits <= 6 ? 6 : 4;   // XPF_RING, XPF_RING_DOWN_N

@@ -1105,8 +1105,9 @@ extern "C" __global__ void __launch_bounds__(1024) exl3_head_rotate(const u8* bl
 // the arithmetic of a block does not depend on which workgroup runs it, so these are the bits the full pass gives.
 // Bound by the decode (60 vector cycles for four weights a lane: 41 us of 151936 x 2048 at 4 bits).  Five workgroups a compute unit
 // (24 KiB of LDS and 102 registers each), so that the 1187 blocks of that size are one round: 51 us; with all of a wave's A rows in
-// LDS three fitted, 1.55 rounds that took two: 57.8 (8 rows of 4096 inputs: the hand-off of the 64 best 199 -> 132 us).  Tried: a workgroup of 16 waves a compute unit with its A rows in registers, block
-// after block: 57.8 too, the ends of a block are nobody else's time there.
+// LDS three fitted, 1.55 rounds that took two: 57.8 (8 rows of 4096 inputs: the hand-off of the 64 best 199 -> 132 us).  Tried: a
+// workgroup of 16 waves a compute unit with its A rows in registers, block after block: 57.8 too, the ends of a block are nobody
+// else's time there.
 // grid = out / 128 (or the list's bound), block 256.
 #define EXL3_HEAD_OCC(K) ((K) <= 5 ? 5 : 3)
 template <int K>
@@ -1406,8 +1407,9 @@ EXL3_HEAD_ENTRIES(8)
 // What bounds it: the decode, 60 vector cycles for four weights a lane, an expert again for every item, and 9 more for each matrix instruction
 // (measured: of its 16 cycles a SIMD issues nothing else for 9, whichever wave it comes from), so few, large items; then the ends of a
 // workgroup, a third of launch 2's time.  4096 tokens through 512 experts of 2048 x 512 and the shared one at 4 bits, top-10: 130 + 385 +
-// 265 us, 456 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
-// and 738 MB of partial sums in between, took 674 + 213 + 285; the chunk 1288 -> 968 us, of 45 tokens at 3 bits 121 -> 102.
+// 265 us, 568 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
+// and 738 MB of partial sums in between, took 674 + 213 + 285.  The chunk on inputs that are not in a cache: 1290 -> 920 us, of 45 tokens at
+// 3 bits 121 -> 120 (there the launches' latencies and the weights' first trip count).
 // Tried: launch 2 by waves of 128 columns for 64 tokens (460 us), its matrix instructions placed among the decode (no change), its two
 // waves of a SIMD half a unit apart (2 %), an expert's items on one XCD (less traffic, same time); launch 3 in launch 2's form (272 to 312).
 

@@ -93,13 +93,13 @@ extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, 
 #define PF_TOK_D 32    // tokens of one work item of the down kernel: with half the activations in LDS twice the workgroups fit a CU
 
 // Groups the chunk's (token, rank) pairs by expert: offs[e] .. offs[e + 1] are the positions in list[] of expert e's pairs
-// (pair = token * k + rank; the shared expert, index ne, takes the pairs npairs + token when nshared = tokens).  The order of an expert's pairs in list[] is arbitrary; every pair owns its
-// output rows, so the results do not depend on it.  items[0] = the number of work items, items[1 + 2 i], items[2 + 2 i] =
+// (pair = token * k + rank; the shared expert, index ne, takes the pairs npairs + token when nshared = tokens).  The order of an expert's pairs in list[] is
+// arbitrary; every pair owns its output rows, so the results do not depend on it.  items[0] = the number of work items, items[1 + 2 i], items[2 + 2 i] =
 // (expert, first position) of item i: every run of up to unit_gu pairs of an expert is one item of the gate/up kernel (at most
 // ne + 1 + rows / unit_gu of them); items_d likewise with runs of up to unit_d pairs, for the down kernel.  The longest items come
 // first, so that the launches end on short ones, and all ahead of the workgroups launched for the rest of the bound (int8 chunk of 512
 // tokens: 239 -> 226 us with the order alone).  Bound by the round trips of its loads: 41 us for 40960 pairs when a thread had one in
-// flight, 37 with eight.  One workgroup.  grid 1, block 1024; ne <= 512.
+// flight, 37 with eight, 29 with 32.  One workgroup.  grid 1, block 1024; ne <= 512.
 extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list,
                                                                  u32* items, u32* items_d, u32 unit_gu, u32 unit_d) {
     __shared__ u32 s_cnt[513], s_off[514], s_fill[513], s_full[2][513], s_class[2][9];
