@@ -514,7 +514,6 @@ int verify_items(sz_session* s, const SzLayer& L, const std::string& tag, uint32
     std::string t;
     format_of(L.type, f, t);
     const uint64_t part = matrix_bytes(f, c.hidden, c.ff) + L.gap;   // from one projection of an expert to the next
-    if (part >> 32) return fail("sz_moe_layer_verify: a projection of 4 GiB or more");
     // The plan is a launch of 4.5 us: worth it where it saves the decode of about 30 M weights (expected, for independent choices).
     // Measured, us a layer with and without: 78.5 and 80.6 at 8 rows of top-10 of 512 Q8_0 experts of 2048 x 512 (17 M saved), 98.2
     // and 92.9 at 6 rows of top-8 of 256 of 3072 x 768 (25 M), 87.5 and 87.2 at 8 rows of top-8 of 128 of 2560 x 768 (73 M), 296
@@ -580,7 +579,8 @@ int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, ui
     const double pairs = (double) m * c.top_k, weights = 3.0 * c.hidden * c.ff;
     const bool small = (pairs + (shared ? m : 0)) * weights < (L.type == SZ_TYPE_Q8_0 ? 25e6 : 70e6) && c.ff <= 4096;
     const char* items = std::getenv("SHADOWZERO_GGUF_ITEMS");   // "plan" or "pairs": that form at any size
-    if (m > 1 && (!small || items) && !std::getenv("SHADOWZERO_GGUF_PLANNED")) return verify_items(s, L, tag, m, u, rl, sgl, y, plan, stream);
+    const bool apart = (matrix_bytes(f, c.hidden, c.ff) + L.gap) >> 32;   // projections further apart than these kernels' 32-bit offset reaches
+    if (m > 1 && (!small || items) && !apart && !std::getenv("SHADOWZERO_GGUF_PLANNED")) return verify_items(s, L, tag, m, u, rl, sgl, y, plan, stream);
     const uint64_t addr = plan + p.a0, rec = plan + p.r0, wts = plan + p.w_off, cnt = plan + p.counts_off;
     const uint64_t addr_d = addr + 2ull * p.GT * 8, rec_d = rec + 2ull * p.GT * 17 * 4;
     const std::string kn = "matvec_grouped_" + tag;
