@@ -1324,8 +1324,9 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         {
             // shares of an item: one wave a column block in the end where items are few, all blocks on eight waves, whose start then counts
             // once, where they fill the chip (1, 2 shares of 8 waves, 4 of 4: 45 tokens as above 137, 109, 101 us, 512 tokens 257, 252, 267,
-            // 4096 at 4 bits 967, 988, 1071)
-            const bool wide = rows >= 1800;
+            // 4096 at 4 bits 967, 988, 1071; 8 and 4 waves: 764 tokens, top-3 of 128 of 1792 x 256 and the shared one, 2 bits 142, 132,
+            // 700 through 64 of 1024 x 256, top-4, 97, 93, 380 through 256 of 3072 x 256, top-8, at 5 bits 230, 242, 190 as above 178, 182)
+            const bool wide = rows * fbs * kbs >= 115000;
             const uint32_t waves = std::min(wide ? 8u : 4u, kbs), parts = std::max((kbs + 4 * waves - 1) / (4 * waves), std::min(rows >= 20000 ? 1u : wide ? 2u : 4u, kbs / waves)), nd = std::min(4u, nt);
             const uint32_t ring = wide ? wide_ring : bits <= 4 ? 8 : bits <= 6 ? 6 : 4;   // XPF_RING, XPF_RING_DOWN_N
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(items_d), P(pb.drows.ptr), P(pb.dinv.ptr), P(pb.eo.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff),
