@@ -368,7 +368,7 @@ def test_gguf_layers_by_distinct_expert(gpu, monkeypatch, ty, hidden, ff, ne, k,
 
 
 @pytest.mark.parametrize("kb,tokens,hidden,ff", [(1, 129, 256, 256), (2, 40, 1024, 512), (4, 300, 256, 512), (5, 140, 512, 512), (6, 210, 256, 256), (7, 97, 256, 512),
-                                                 (8, 260, 256, 512), (3, 4100, 256, 512), (6, 4100, 256, 512)])
+                                                 (8, 260, 256, 512), (3, 5500, 256, 512), (6, 5500, 256, 512), (8, 5500, 256, 512)])
 def test_exl3_prefill_items_of_every_size(gpu, kb, tokens, hidden, ff):  # noqa: F811
     """Experts with few and many tokens (items of one tile to the most, the wide and the narrow form of the gate and up launch, the
     shortest streams), a token of zeros, one of very large inputs, and an expert whose gate is silent in one 128-block: that
