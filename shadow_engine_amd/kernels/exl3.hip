@@ -1774,6 +1774,22 @@ __device__ __forceinline__ void xpf_activate(f32x4 (&g)[8], f32x4 (&u)[8], const
     xpf_put_plain(rows, half_step, g, lane);
 }
 
+// A token's factors (what undoes its blocks' powers of two, `f[16 b]`) as launch 3 may take its sums from one block's power of two to the
+// next one's.  The sums of a block are below 2^25 in its own units (128 inputs of at most 2^15 times weights below 4), whatever follows
+// multiplies them by f[b - 1] / f[b], and what counts is the product of these steps from the largest factor before a block to its own: at
+// most 2^88 keeps four blocks' sums below 2^116.  A block beyond that is nothing beside the sums (its values are below 2^-80 of the
+// largest ones): drop(b) makes it zeros, and it takes the factor of the one before.
+template <class Drop>
+__device__ __forceinline__ void xpf_chain(float* f, u32 fbs, Drop drop) {
+    float most = f[0];
+    for (u32 b = 1; b < fbs; b++) {
+        if (most / f[16 * b] > 0x1p88f) {
+            f[16 * b] = f[16 * (b - 1)];
+            drop(b);
+        } else if (f[16 * b] > most) most = f[16 * b];
+    }
+}
+
 // A workgroup's sums through LDS (x: [block of 128 columns][of R tiles][register][lane]), so that a wave has all 128 columns of a
 // token tile: the wave of columns 64 half .. of block `at` leaves tile T in place R at + i.
 __device__ __forceinline__ void xpf_leave(f32x4* x, u32 place, u32 half, const f32x4 (&acc)[4], u32 lane) {
@@ -1900,17 +1916,12 @@ __device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__
             else wait_vm<0>();
         } else wait_vm<0>();
         lds_barrier();
-        // A block whose values are nothing beside the sums of the blocks before it (2^-88) would take the sums out of range with its power
-        // of two: zeros in its place, and the power of two of the one before.
+        // blocks that xpf_chain drops: zeros in their place
         if (threadIdx.x < 16 * it.tiles) {
             const u32 T = threadIdx.x / 16, t = threadIdx.x % 16;
-            for (u32 b = 1; b < fbs; b++) {
-                float* f = fac + (T * fbs + b) * 16 + t;
-                if (f[-16] / f[0] > 0x1p88f) {
-                    f[0] = f[-16];
-                    for (u32 i = 0; i < 16; i++) *(u32x4*) (xrows + (T * fbs + b) * XPF_ROWS_U16 + (16 * i + t) * 8) = u32x4{0, 0, 0, 0};
-                }
-            }
+            xpf_chain(fac + T * fbs * 16 + t, fbs, [&](u32 b) {
+                for (u32 i = 0; i < 16; i++) *(u32x4*) (xrows + (T * fbs + b) * XPF_ROWS_U16 + (16 * i + t) * 8) = u32x4{0, 0, 0, 0};
+            });
         }
         lds_barrier();
         if (!total) return;

@@ -400,3 +400,40 @@ def test_exl3_prefill_items_of_every_size(gpu, kb, tokens, hidden, ff):  # noqa:
             assert np.array_equal(np.isfinite(got[j]), np.isfinite(want[i])) and np.isfinite(want[i]).any() == np.isfinite(got[j]).any()
         else:
             assert rel_l2(got[j], want[i]) <= 1e-3, (j, rel_l2(got[j], want[i]))
+
+
+# What an expert's four 128-blocks of ff leave for the down product: the output scales of gate and up and the input scales of down
+# whose product sets a block's size.  0, and 1e-22 as three of f16's subnormals, are silent beside any other.
+BLOCK_SIZES = {"strong": (1, 45, 45), "huge": (3e4, 3e4, 3e4), "weak": (1, 1e-4, 1e-4), "weaker": (2e-7, 2e-7, 2e-7), "least": (6e-8, 6e-8, 6e-8), "ordinary": (1, 1, 1), "silent": (1, 0, 1)}
+
+
+@pytest.mark.parametrize("kb", [2, 4, 7])
+@pytest.mark.parametrize("tokens", [19, 700])
+def test_exl3_prefill_blocks_of_any_size_beside_each_other(gpu, kb, tokens):  # noqa: F811
+    """Every order of block sizes whose powers of two are far apart step by step, or only over several steps: the sums over ff stay
+    in range, and every token's row is within the chunk's 1e-3 of the oracle (one expert a token, so that none hides another)."""
+    rng = np.random.default_rng(kb * 1000 + tokens)
+    orders = [("strong", "weak", "silent", "ordinary"), ("strong", "weaker", "silent", "ordinary"), ("huge", "weak", "least", "ordinary"), ("huge", "ordinary", "weaker", "silent"),
+              ("least", "weak", "huge", "silent"), ("silent", "least", "ordinary", "strong"), ("strong", "silent", "weak", "silent"), ("weak", "silent", "silent", "weaker")]
+    hidden, ff, ne, ty = 256, 512, len(orders), sz.EXL3(kb)
+    dbuf, stride, blobs, _ = build_layer(gpu, rng, ty, hidden, ff, ne, False)
+    gb, ub, _ = synth.expert_bytes(ty, hidden, ff)
+    for e, order in enumerate(orders):
+        for b, size in enumerate(order):
+            for at, scale in zip((2 * hidden, gb + 2 * hidden, gb + ub), BLOCK_SIZES[size]):
+                part = blobs[e][at + 256 * b:at + 256 * (b + 1)].view(np.float16)
+                part[:] = (part.astype(np.float32) * scale).astype(np.float16)
+        dbuf[e * stride:e * stride + blobs[e].size] = dev(gpu, blobs[e])
+    s = sz.Session(hidden, ff, ne, 1, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, 0, 0)
+    x, logits = rng.normal(size=(tokens, hidden)).astype(np.float32), np.full((tokens, ne), -9.0, np.float32)
+    logits[np.arange(tokens), np.arange(tokens) % ne] = 9.0
+    y = gpu.zeros((tokens, hidden), dtype=gpu.float32, device="cuda")
+    dx, dl, dg = dev(gpu, x), dev(gpu, logits), dev(gpu, np.zeros(tokens, np.float32))
+    s.moe_prefill_chunk(0, tokens, dx.data_ptr(), dl.data_ptr(), dg.data_ptr(), y.data_ptr())
+    gpu.cuda.synchronize()
+    got, rows = y.cpu().numpy(), np.r_[:16, tokens - 3:tokens]
+    want, _, _ = oracle_layer(ty, hidden, ff, 1, blobs, None, logits[rows], np.zeros(rows.size, np.float32), x[rows])
+    for i, j in enumerate(rows):
+        assert rel_l2(got[j], want[i]) <= 1e-3, (orders[j % ne], rel_l2(got[j], want[i]))
+    assert np.isfinite(got).all()
