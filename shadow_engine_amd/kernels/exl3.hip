@@ -1692,7 +1692,7 @@ struct XpfStep {
 // The products of a wave (64 columns) over the `ring.units` 64-blocks of the inputs.  The operand rows (src: [64-block][tiles], whole
 // item) come through a ring of NB slots of NT tiles in LDS (`stage`, slots `slot_u16` apart) that the NW waves of one projection share, of
 // which this is number `part`: requested NB - 1 units ahead, each wave its share, a barrier a unit.  A step's words and
-// operand rows are read while the one before is multiplied. The whole workgroup calls this with the same number of units.  D + 1 >= NB; units >= D.
+// operand rows are read while the one before is multiplied. The whole workgroup calls this with the same number of units.  D + 1 >= NB.
 template <int K, int NT, int NB, int NW, class R>
 __device__ __forceinline__ void xpf_stream(const R& ring, const u32* wb, const u16* __restrict__ src, u16* stage, u32 slot_u16, u32 tiles, u32 part, u32 lane,
                                            f32x4 (&acc)[NT][4]) {
@@ -1709,8 +1709,9 @@ __device__ __forceinline__ void xpf_stream(const R& ring, const u32* wb, const u
         for (int c = 0; c < 4; c++) acc[T][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int i = -D; i < 0; i++) {
-        ring.issue(i + D, i + D, lane);
-        if (i + NB - 1 >= 0) request(i + NB - 1, i + NB - 1);
+        // a stream may be shorter than its ring (hidden = 256: four units)
+        if ((u32) (i + D) < ring.units) ring.issue(i + D, i + D, lane);
+        if (i + NB - 1 >= 0 && (u32) (i + NB - 1) < ring.units) request(i + NB - 1, i + NB - 1);
     }
     // this wave's share of a unit's operand rows has landed (behind it: NB - 2 times a unit's trellis rows and operand rows, but for the
     // stream's end); every wave's, and the slot of the unit before has been read
