@@ -1782,12 +1782,16 @@ __device__ __forceinline__ void xpf_activate(f32x4 (&g)[8], f32x4 (&u)[8], const
 // largest ones): drop(b) makes it zeros, and it takes the factor of the one before.
 template <class Drop>
 __device__ __forceinline__ void xpf_chain(float* f, u32 fbs, Drop drop) {
-    float most = f[0];
+    float most = f[0], last = most;
     for (u32 b = 1; b < fbs; b++) {
-        if (most / f[16 * b] > 0x1p88f) {
-            f[16 * b] = f[16 * (b - 1)];
+        const float here = f[16 * b];
+        if (most > here * 0x1p88f) {
+            f[16 * b] = last;
             drop(b);
-        } else if (f[16 * b] > most) most = f[16 * b];
+        } else {
+            last = here;
+            most = fmaxf(most, here);
+        }
     }
 }
 
