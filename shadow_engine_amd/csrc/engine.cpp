@@ -507,17 +507,55 @@ int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32
     return 0;
 }
 
-// A layer of GGUF experts for several tokens, by distinct expert on the matrix cores (verify_items_* in kernels/gguf.hip).
+// The two launches of a single token (decode_gate_up_*, decode_down_combine_*): rows a workgroup and their LDS, if the shape has them.
+struct DecodeShape {
+    bool ok = false;
+    uint32_t rp = 8, rd = 0, rs_gu = 0, rs_d = 0, pairs = 0;
+};
+DecodeShape decode_shape(const sz_session_config& c, const Format& f, bool shared) {
+    DecodeShape d;
+    const uint32_t uh = c.hidden / 32, uf = c.ff / 32;
+    if (c.hidden % 32 || c.ff % 32 || uh > 64 || 64 % uh || uf > 64 || 64 % uf || c.top_k > 16) return d;
+    d.rd = std::max(4u, 64 / uf);
+    d.rs_gu = (d.rp * (c.hidden / f.qk * f.bb) + 31) / 16 * 16;
+    d.rs_d = (d.rd * (c.ff / f.qk * f.bb) + 31) / 16 * 16;
+    d.pairs = c.top_k + (shared ? 1 : 0);
+    d.ok = c.ff % d.rp == 0 && c.hidden % d.rd == 0 && 2 * d.rs_gu <= 16384 && d.pairs * d.rs_d <= 16384 && d.pairs * c.ff <= 8192;
+    return d;
+}
+
+// Whether a layer of GGUF experts runs on the matrix cores (verify_items) or the vector unit.  Their sums are in another order, and a
+// token's bits must not depend on the other tokens of its batch (what a verify round accepts is what decoding token by token gives):
+// the layer's shape alone decides, for one row to eight.  The more weights a token takes the sooner the matrix cores win; IQ3_S holds
+// out longer where a single token has its two launches.  Measured, us of the router and the layer, four layers in a row, vector unit /
+// matrix cores at 1, 2, 4 and 8 rows, by millions of weights a token:
+//   Q8_0                       10.2: 17.9 20.3 28.7 43.1 / 19.2 23.0 31.1 53.2    11.0: 16.1 19.6 27.1 45.5 / 18.1 19.9 23.3 35.9
+//                              18.9: 19.9 25.1 38.1 65.4 / 20.2 22.4 31.4 52.5    47.2: 30.6 54.2 93.0 167 / 25.2 36.0 59.6 88.5
+//   IQ3_S with two launches    18.9: 17.6 25.5 30.9 50.7 / 20.8 23.9 33.4 57.1    34.6: 19.9 30.1 46.7 79.1 / 23.6 31.5 44.0 83.2
+//                              40.9: 25.7 36.6 53.0 90.5 / 24.1 32.7 46.7 96.5    50.3: 28.6 40.1 63.2 108 / 24.8 33.4 54.3 80.4
+//   IQ3_S without them         18.9: 20.2 24.2 36.4 59.5 / 22.3 24.3 36.5 57.5    20.6: 21.8 27.7 38.3 57.4 / 21.2 24.4 31.6 47.0
+//                              47.2: 31.4 48.7 81.5 149 / 27.4 35.7 60.2 93.7
+// A line in front of 34.6 would cost a single token a fifth; behind it layers of few experts lose what their tokens share (60 experts
+// at 34.6: 19.8 29.7 45.6 73.9 / 23.7 31.4 43.3 57.9).  More than 4096 inputs of a down product are more than the vector kernels
+// without a plan take; with one, 21.2 of Q8_0: 33.3 43.4 59.5 90.5 / 22.8 25.3 31.7 46.1.
+bool gguf_matrix_cores(const sz_session_config& c, int type, const Format& f, bool shared) {
+    if (c.ff > 4096) return true;
+    const double weights = 3.0 * c.hidden * c.ff * (c.top_k + (shared ? 1 : 0));
+    return weights >= (type == SZ_TYPE_Q8_0 ? 11e6 : decode_shape(c, f, shared).ok ? 40e6 : 20e6);
+}
+
+// A layer of GGUF experts by distinct expert on the matrix cores (verify_items_* in kernels/gguf.hip).
 int verify_items(sz_session* s, const SzLayer& L, const std::string& tag, uint32_t m, uint64_t u, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t plan, uint64_t stream) {
     const sz_session_config& c = s->cfg;
     Format f;
     std::string t;
     format_of(L.type, f, t);
     const uint64_t part = matrix_bytes(f, c.hidden, c.ff) + L.gap;   // from one projection of an expert to the next
-    // The plan is a launch of 4.5 us: worth it where it saves the decode of about 30 M weights (expected, for independent choices).
-    // Measured, us a layer with and without: 78.5 and 80.6 at 8 rows of top-10 of 512 Q8_0 experts of 2048 x 512 (17 M saved), 98.2
-    // and 92.9 at 6 rows of top-8 of 256 of 3072 x 768 (25 M), 87.5 and 87.2 at 8 rows of top-8 of 128 of 2560 x 768 (73 M), 296
-    // and 309 at 8 rows of top-12 of 512 of 3328 x 1536 (113 M), 55.6 and 85.5 at 8 rows of top-12 of 32 of 2048 x 512 (203 M).
+    // The plan is a launch of 4.5 us: worth it where it saves the decode of about 30 M weights (expected, for independent choices); the bits
+    // are the same either way.  Measured, us a layer with and without: 78.5 and 80.6 at 8 rows of top-10 of 512 Q8_0 experts of 2048 x 512
+    // (17 M saved), 98.2 and 92.9 at 6 rows of top-8 of 256 of 3072 x 768 (25 M), 87.5 and 87.2 at 8 rows of top-8 of 128 of 2560 x 768 (73
+    // M), 296 and 309 at 8 rows of top-12 of 512 of 3328 x 1536 (113 M), 55.6 and 85.5 at 8 rows of top-12 of 32 of 2048 x 512 (203 M): no
+    // line has all of these right, the first takes 3 % more than it could here.
     const double pairs = (double) m * c.top_k, distinct = c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) m));
     const char* form = std::getenv("SHADOWZERO_GGUF_ITEMS");
     const bool by_pair = form ? std::strcmp(form, "pairs") == 0 : (pairs - distinct) * 3.0 * c.hidden * c.ff < 30e6;
@@ -571,16 +609,9 @@ int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, ui
         s->last_fused = true;
         return verify_layers(s, L.vpos, L.vpos + 1, l, m, u, rl, sgl, y, plan, stream);
     }
-    // Several tokens: by distinct expert on the matrix cores (kernels/gguf.hip), unless the layer is so small that the vector kernels'
-    // shorter chains are over first.  Measured, us a layer of four in a row, vector kernels and matrix cores: Q8_0 at 31 M weights of
-    // (token, expert) pairs (128 experts of 2048 x 512, top-4, 2 rows) 22.4 and 21.3, at 19 M 18.6 and 22.7; IQ3_S at 71 M (60 of 3072 x
-    // 768, top-4, 2 rows) 35.3 and 29.1, at 69 M (512 of 2048 x 512, top-10, 2 rows) 30.3 and 31.6, at 104 M 40.1 and 32.7; 8 rows of
-    // top-8 of 128 Q8_0 experts of 2560 x 768 167 and 87.5.
-    const double pairs = (double) m * c.top_k, weights = 3.0 * c.hidden * c.ff;
-    const bool small = (pairs + (shared ? m : 0)) * weights < (L.type == SZ_TYPE_Q8_0 ? 25e6 : 70e6) && c.ff <= 4096;
-    const char* items = std::getenv("SHADOWZERO_GGUF_ITEMS");   // "plan" or "pairs": that form at any size
+    const char* items = std::getenv("SHADOWZERO_GGUF_ITEMS");   // "plan" or "pairs": that form of the matrix cores at any size
     const bool apart = (matrix_bytes(f, c.hidden, c.ff) + L.gap) >> 32;   // projections further apart than these kernels' 32-bit offset reaches
-    if (m > 1 && (!small || items) && !apart && !std::getenv("SHADOWZERO_GGUF_PLANNED")) return verify_items(s, L, tag, m, u, rl, sgl, y, plan, stream);
+    if ((items || gguf_matrix_cores(c, L.type, f, shared)) && !apart && !std::getenv("SHADOWZERO_GGUF_PLANNED")) return verify_items(s, L, tag, m, u, rl, sgl, y, plan, stream);
     const uint64_t addr = plan + p.a0, rec = plan + p.r0, wts = plan + p.w_off, cnt = plan + p.counts_off;
     const uint64_t addr_d = addr + 2ull * p.GT * 8, rec_d = rec + 2ull * p.GT * 17 * 4;
     const std::string kn = "matvec_grouped_" + tag;
@@ -597,23 +628,18 @@ int moe_layer(sz_session* s, uint32_t l, uint32_t m, uint64_t u, uint64_t rl, ui
         // One token: two launches.  Launch 1 hands over act = silu(gate) * up and the routing weights, launch 2 owns a row chunk
         // for all of the token's experts and adds them up itself (SHADOWZERO_GGUF_THREE_LAUNCH=1 keeps the general form).
         const bool three = std::getenv("SHADOWZERO_GGUF_THREE_LAUNCH") != nullptr;
-        const uint32_t uh = c.hidden / 32, uf = c.ff / 32;
-        if (m == 1 && !three && c.hidden % 32 == 0 && c.ff % 32 == 0 && uh <= 64 && 64 % uh == 0 && uf <= 64 && 64 % uf == 0 && c.top_k <= 16) {
-            const uint32_t rp = 8, rd = std::max(4u, 64 / uf);
-            const uint32_t rs_gu = (rp * rb_gu + 31) / 16 * 16, rs_d = (rd * rb_d + 31) / 16 * 16;
-            const uint32_t Sd = c.top_k + (shared ? 1 : 0);
-            if (c.ff % rp == 0 && c.hidden % rd == 0 && 2 * rs_gu <= 16384 && Sd * rs_d <= 16384 && Sd * c.ff <= 8192) {
-                const std::string d1 = "decode_gate_up_" + tag, d2 = "decode_down_combine_" + tag;
-                {
-                    const sz_arg a[] = {P(rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(u), P(plan), P(s->eg.ptr),
-                                        U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(rp)};
-                    if (launch(d1.c_str(), c.ff / rp, S, 1, 512, 2 * rs_gu, stream, a)) return 1;   // 8 waves: a gate row and an up row each at hidden 2048
-                }
-                s->last_fused = true;
-                const sz_arg a[] = {U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), P(s->eg.ptr), P(sgl), P(y),
-                                    U32(c.top_k), U32(c.hidden), U32(c.ff), U32(rd)};
-                return launch(d2.c_str(), c.hidden / rd, 1, 1, 64 * std::min(16u, std::max(4u, Sd)), Sd * rs_d + Sd * uf * 144, stream, a);   // a wave a pair
+        const DecodeShape d = decode_shape(c, f, shared);
+        if (m == 1 && !three && d.ok) {
+            const std::string d1 = "decode_gate_up_" + tag, d2 = "decode_down_combine_" + tag;
+            {
+                const sz_arg a[] = {P(rl), U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(u), P(plan), P(s->eg.ptr),
+                                    U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff), U32(d.rp)};
+                if (launch(d1.c_str(), c.ff / d.rp, S, 1, 512, 2 * d.rs_gu, stream, a)) return 1;   // 8 waves: a gate row and an up row each at hidden 2048
             }
+            s->last_fused = true;
+            const sz_arg a[] = {U64(L.experts), U64(L.stride), U64(L.shared), U32((uint32_t) part), P(plan), P(s->eg.ptr), P(sgl), P(y),
+                                U32(c.top_k), U32(c.hidden), U32(c.ff), U32(d.rd)};
+            return launch(d2.c_str(), c.hidden / d.rd, 1, 1, 64 * std::min(16u, std::max(4u, d.pairs)), d.pairs * d.rs_d + d.pairs * (c.ff / 32) * 144, stream, a);   // a wave a pair
         }
         const std::string k1 = "verify_gate_up_" + tag, k2 = "verify_down_" + tag;
         {

@@ -402,8 +402,8 @@ extern "C" __global__ void __launch_bounds__(1024, 4) matvec_cols_w_iq3_s(const 
     gg_cols<GgIq3, 2>(w, x, xs, y, ys, rows, cols, m);
 }
 
-// ------------------------------------------------------------------------------------- MoE layers for a batch, by distinct expert
-// The verify layer of GGUF experts for several tokens, on the products above: every distinct expert's weights are decoded once for
+// ------------------------------------------------------------------------------------- MoE layers, by distinct expert
+// The verify layer of GGUF experts for one to eight tokens, on the products above: every distinct expert's weights are decoded once for
 // the tokens that chose it (route_plan in route.hip.h lists them).  Expert e's gate, up and down lie at experts + e stride + {0, part,
 // 2 part}, the shared one's at shared + the same.  A workgroup takes 2 to 8 row tiles of one expert (the host's choice), a wave a
 // 256-column chunk; the first launch has the same rows of gate and up and leaves silu(gate) * up.  Measured, 8 tokens of top-8 of 128

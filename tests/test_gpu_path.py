@@ -354,7 +354,7 @@ def test_moe_layer_verify_planned_form_matches_the_oracle(gpu, monkeypatch, ty, 
     (sz.IQ3_S, 512, 256, 8, 3, False),             # no shared expert: rank 0's workgroup computes the weights; 8 units a down row
     (sz.Q8_0, 1024, 512, 12, 4, True),
     (sz.Q8_0, 512, 256, 16, 4, False),
-    (sz.Q8_0, 2048, 2048, 6, 2, True),             # too large for launch 2's staging: the call falls back to three launches
+    (sz.Q8_0, 2048, 2048, 6, 2, True),             # too large for launch 2's staging: three launches (of the matrix cores)
 ])
 def test_one_token_layer_in_two_launches(gpu, monkeypatch, ty, hidden, ff, ne, k, shared):
     """A single token takes the two-launch form (act and the routing weights out of launch 1, the down rows of all experts and

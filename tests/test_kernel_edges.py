@@ -367,6 +367,40 @@ def test_gguf_layers_by_distinct_expert(gpu, monkeypatch, ty, hidden, ff, ne, k,
     assert np.array_equal(bits(outs[0]), bits(outs[1]))
 
 
+@pytest.mark.parametrize("ty,hidden,ff,ne,k,shared", [
+    (sz.Q8_0, 1024, 256, 16, 4, False),         # the vector unit, a single token in two launches
+    (sz.Q8_0, 3072, 256, 12, 2, True),          # rows of 96 units: three launches for a single token too
+    (sz.Q8_0, 1280, 1024, 12, 2, True),         # just above the line: the matrix cores
+    (sz.Q8_0, 2560, 768, 24, 8, False),
+    (sz.IQ3_S, 2048, 512, 32, 10, True),        # below the line of the layers with two launches
+    (sz.IQ3_S, 2048, 512, 32, 13, True),        # above it
+    (sz.IQ3_S, 768, 1280, 8, 3, False),         # below the line of those without, rows of 24 and 40 units
+    (sz.IQ3_S, 1792, 768, 16, 4, True),         # above it
+    (sz.IQ3_S, 512, 4608, 6, 1, True),          # more than 4096 inputs of the down products
+])
+def test_a_gguf_layers_bits_do_not_depend_on_the_batch(gpu, ty, hidden, ff, ne, k, shared):  # noqa: F811
+    """On both sides of every line of the choice between vector unit and matrix cores: a token's row has the same bits in batches of
+    1 to 8 rows, within 2e-6 relative L2 of the oracle."""
+    rng = np.random.default_rng(ty + hidden + ff + k)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, shared)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty if shared else 0, dbuf.data_ptr() + ne * stride if shared else 0)
+    u, logits, sgl = rng.normal(size=(8, hidden)).astype(np.float32), rng.normal(size=(8, ne)).astype(np.float32), rng.normal(size=8).astype(np.float32)
+    du, dl, dg = dev(gpu, u), dev(gpu, logits), dev(gpu, sgl)
+    want, widx, _ = oracle_layer(ty, hidden, ff, k, blobs, sh, logits, sgl, u)
+    first = None
+    for m in range(8, 0, -1):
+        y = gpu.zeros((m, hidden), dtype=gpu.float32, device="cuda")
+        s.moe_layer_verify(0, m, du.data_ptr(), dl.data_ptr(), dg.data_ptr(), y.data_ptr())
+        gpu.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert np.array_equal(s.last_route(m)[0], widx[:m])
+        if first is None:
+            first = got
+            assert max(rel_l2(got[j], want[j]) for j in range(8)) <= 2e-6
+        assert np.array_equal(bits(got), bits(first[:m])), f"{m} rows"
+
+
 @pytest.mark.parametrize("kb,tokens,hidden,ff", [(1, 129, 256, 256), (2, 40, 1024, 512), (4, 300, 256, 512), (5, 140, 512, 512), (6, 210, 256, 256), (7, 97, 256, 512),
                                                  (8, 260, 256, 512), (3, 5500, 256, 512), (6, 5500, 256, 512), (8, 5500, 256, 512)])
 def test_exl3_prefill_items_of_every_size(gpu, kb, tokens, hidden, ff):  # noqa: F811
