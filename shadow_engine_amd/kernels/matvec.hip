@@ -1240,23 +1240,27 @@ __device__ __forceinline__ void hc_down_rows(const u8* __restrict__ w, u32 rows,
     }
     __syncthreads();
     if constexpr (MANY) {
+        float acc[HC_NP][M];   // a lane's own over all its columns, as below: a row's bits are the same in either form
+#pragma unroll
+        for (int q = 0; q < (int) HC_NP; q++)
+#pragma unroll
+            for (int j = 0; j < M; j++) acc[q][j] = 0.0f;
         for (u32 o = 0; o < outer; o++) {
             if (outer > 1) {
                 sl.inputs(r, cols, m, o, xv);
                 sl.inputs(nw, 0, 1, o, nv);
             }
             hc_normalise<T, M>(sl, xv, nv, scl, h, cs, m, o);
-            for (u32 q = 0; q < np; q++) {
-                float acc[M];
 #pragma unroll
-                for (int j = 0; j < M; j++) acc[j] = 0.0f;
-                sl.dot(wv, xv, acc);
+            for (u32 q = 0; q < HC_NP; q++) {
+                if (q >= np) break;
+                sl.dot(wv, xv, acc[q]);
 #pragma unroll
                 for (int i = 0; i < S::NCH; i++) wv[i] = wn[i];
                 next();
-                const float t = dense_reduce<M>(acc, 64, lane);
-                float* sum = red + (q * 8 + wave) * 8 + lane;   // the lane's own
-                if (live && lane < (u32) M) *sum = o ? *sum + t : t;
+                if (o + 1 < outer) continue;
+                const float t = dense_reduce<M>(acc[q], 64, lane);
+                if (live && lane < (u32) M) red[(q * 8 + wave) * 8 + lane] = t;
             }
         }
     } else {

@@ -215,6 +215,35 @@ def test_hyper_connection_rows_of_a_workgroup(gpu, ty, h, cs, rank, m):  # noqa:
     test_hyper_connection_at_its_edges(gpu, ty, h, cs, rank, m, 1.0)
 
 
+@pytest.mark.parametrize("ty,h,cs,rank,m", [
+    (sz.BF16, 4096, 4, 320, 5), (sz.F32, 2052, 4, 516, 8),    # more than 8192 columns: one row a workgroup for one input, several for more
+    (sz.F16, 2304, 4, 1028, 3), (sz.BF16, 2048, 4, 320, 8),   # several for both; inputs that stay in registers
+    (sz.F32, 4352, 64, 200, 8)])                              # inputs in lots: seven, then one
+def test_hyper_connection_bits_do_not_depend_on_the_batch(gpu, ty, h, cs, rank, m):  # noqa: F811
+    """hc_read of a row alone, in a batch of two and in one of m: the same bits."""
+    rng = np.random.default_rng(h + cs + m)
+    ch = h * cs
+    r = rng.normal(size=(m, ch)).astype(np.float32)
+    nw = (1 + 0.1 * rng.normal(size=ch)).astype(np.float32)
+    wd, wu, wi = dense_matrix(rng, ty, rank, ch), dense_matrix(rng, ty, ch, rank), dense_matrix(rng, ty, cs, ch)
+    dnw, dwd, dwu, dwi = dev(gpu, nw), dev(gpu, wd), dev(gpu, wu), dev(gpu, wi)
+    hc = sz.HyperConnection(h, cs, rank, 1e-6, dnw.data_ptr(), ty, dwd.data_ptr(), ty, dwu.data_ptr(), ty, dwi.data_ptr())
+
+    def read(rows):
+        dr, du = dev(gpu, rows), gpu.zeros((len(rows), h), dtype=gpu.float32, device="cuda")
+        hc.read(len(rows), dr.data_ptr(), du.data_ptr())
+        gpu.cuda.synchronize()
+        g = np.empty((len(rows), cs), np.float32)
+        sz.download(g, hc.gains)
+        return bits(du.cpu().numpy()), bits(g)
+
+    u, g = read(r)
+    for n in (1, 2):
+        for j in range(0, m - n + 1, n):
+            un, gn = read(r[j:j + n])
+            assert np.array_equal(un, u[j:j + n]) and np.array_equal(gn, g[j:j + n]), (n, j)
+
+
 @pytest.mark.parametrize("ty", [sz.F32, sz.F16, sz.BF16])
 @pytest.mark.parametrize("rows,cols,m", [(9, 3072, 4), (5, 5000, 8), (6, 7168, 1), (17, 8192, 5), (3, 8196, 8), (1100, 9220, 3), (4, 20480, 4)])
 def test_unquantized_rows_of_several_waves_and_longer(gpu, ty, rows, cols, m):  # noqa: F811
