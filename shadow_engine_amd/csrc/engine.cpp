@@ -387,7 +387,7 @@ struct sz_session {
             uint64_t ptr = 0;
         };
         DevBuf mem;
-        Part xq, xd, tidx, w, cnt, offs, list, items, hq, hd, eo, amax, arows, ainv, drows, dinv;
+        Part xq, xd, tidx, w, cnt, offs, list, items, hq, hd, eo, most, arows, ainv, drows, dinv;
         int lay(std::initializer_list<std::pair<Part*, uint64_t>> parts) {
             uint64_t n = 0;
             for (const auto& p : parts) n += (p.second + 255) & ~255ull;
@@ -1313,11 +1313,11 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1, max_items = some + rows / tok, max_down = some + rows / 64, tiles = rows / 16 + c.n_expert + 2;
         const uint32_t bound = (uint32_t) ((max_items + 7) / 8 * 8), bound_d = (uint32_t) ((max_down + 7) / 8 * 8);   // workgroups an item's part (xpf_place)
         if (pb.lay({{&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4}, {&pb.items, (2 + 2 * max_items + 2 * max_down) * 4},
-                    {&pb.eo, rows * c.hidden * 4}, {&pb.amax, T * 4}, {&pb.arows, tiles * 2 * kbs * 4096}, {&pb.ainv, tiles * 2 * 64}, {&pb.drows, tiles * fbs * 4096}, {&pb.dinv, tiles * fbs * 64}}))
+                    {&pb.eo, rows * c.hidden * 4}, {&pb.most, T * 8}, {&pb.arows, tiles * 2 * kbs * 4096}, {&pb.ainv, tiles * 2 * 64}, {&pb.drows, tiles * fbs * 4096}, {&pb.dinv, tiles * fbs * 64}}))
             return 1;
         const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0, items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
         {
-            const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens), P(x), P(pb.amax.ptr), U32(c.hidden)};
+            const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens), P(x), P(pb.most.ptr), U32(c.hidden)};
             if (launch("route_topk_rows", (tokens + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
         }
         {
@@ -1326,7 +1326,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
             if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
         }
         {
-            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(x), P(pb.amax.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), U32(c.n_expert),
+            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(x), P(pb.most.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), U32(c.n_expert),
                                 U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(tok), U32(ntl)};
             if (launch("prefill_rotate_exl3", bound * ntl, 1, 1, 256, 0, stream, a)) return 1;
         }

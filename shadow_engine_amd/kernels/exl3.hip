@@ -1562,13 +1562,18 @@ __device__ __forceinline__ void xpf_tiles(u32 tiles, F&& run) {
     run(XpfInt<4>());
 }
 
-// Launch 1: a tile (16 tokens) of an item; wave w takes the 128-blocks w, w + 4, .. of the inputs.  A token's power of
-// two takes the product of its largest input (amax, from the routing launch) and the projection's largest input scale to [2^7, 2^8):
-// no value passes 2^15 in the transform.  rows: an item's [gate, up][64-block][tile], inv: [gate, up][tile][16].
+// Launch 1: a tile (16 tokens) of an item; wave w takes the 128-blocks w, w + 4, .. of the inputs.  A token's power of two takes a bound
+// of its inputs times the projection's input scales to [2^7, 2^8): no value passes 2^15 in the transform.  Values 2^21 below the bound are
+// f16's subnormals, whose last bit is 2^31 below it.  The bound is the largest input (most, from the routing launch) times the largest
+// scale where all scales, or those of the four channels about that input, are within 2^10 of the largest, so that the bound is no further than
+// that from the largest product; else (a large input of a channel that the expert scales to next to nothing) the largest product, which
+// takes another pass over the inputs (such a pass for every token: 52 us of 4096 tokens' 920, 4 of 45 tokens' 121).
+// rows: an item's [gate, up][64-block][tile], inv: [gate, up][tile][16].
 // Bound by the rows it writes (8 bytes an input and pair).  grid = xpf_place's, of `tiles` parts, block 256.
 extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const float* x,
-                                                                      const float* amax, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles) {
-    __shared__ u32 s_scale[2][4];
+                                                                      const u32* most, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles) {
+    __shared__ u32 s_scale[2][4], s_least[2][4];
+    __shared__ float s_most[2][4][16];
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, kbs = hidden / 128;
     u32 T;
     const u32 item = xpf_place(tiles, T);
@@ -1576,43 +1581,98 @@ extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64*
     if (T >= it.tiles) return;
     const u32 e = it.e, pair = list[it.first + min(16 * T + (lane & 15), it.n - 1)];   // places past the item's end repeat its last pair: nothing reads them
     const u32 token = pair < npairs ? pair / k : pair - npairs;
-    const float am = amax[token];
+    const float am = bits_f32(most[2 * token]);
     const u16* suh[2] = {(const u16*) (e < ne ? eaddr[e] : sh_addr[0]), (const u16*) (e < ne ? eaddr[(u64) ne + e] : sh_addr[1])};
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-        u32 m = 0;
+        u32 m = 0, l = 0x7fffu;
         for (u32 i = threadIdx.x; i < hidden / 8; i += 256) {
             const u32x4a v = ((const u32x4a*) suh[s])[i];
 #pragma unroll
-            for (int q = 0; q < 4; q++) m = max(m, max(v[q] & 0x7fffu, (v[q] >> 16) & 0x7fffu));
+            for (int q = 0; q < 4; q++) {
+                m = max(m, max(v[q] & 0x7fffu, (v[q] >> 16) & 0x7fffu));
+                l = min(l, min(v[q] & 0x7fffu, (v[q] >> 16) & 0x7fffu));
+            }
         }
         m = wave_max_u32(m);
-        if (lane == 0) s_scale[s][wave] = m;
+        l = wave_min_u32(l);
+        if (lane == 0) {
+            s_scale[s][wave] = m;
+            s_least[s][wave] = l;
+        }
     }
+    const float* xr = x + (u64) token * hidden + 4 * (lane >> 4);
+    f32x4 xv[8];
+    auto inputs = [&](u32 kb) {
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) xv[ks] = *(const f32x4*) (xr + kb * 128 + 16 * ks);
+    };
+    inputs(min(wave, kbs - 1));   // on their way while the scales' maxima are made
     __syncthreads();
-    float scale[2];
+    // a block's inputs times their scales
+    auto scaled = [&](u32 s, u32 kb, f32x4 (&v)[8]) {
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) {
+            const u16x4 s4 = *(const u16x4*) (suh[s] + kb * 128 + 16 * ks + 4 * (lane >> 4));
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[ks][q] = xv[ks][q] * f16_to_f32(s4[q]);
+        }
+    };
+    float bound[2], scale[2], largest[2];
+    bool wide = false;   // scales further apart
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-        const u32 m = max(max(s_scale[s][0], s_scale[s][1]), max(s_scale[s][2], s_scale[s][3]));
+        largest[s] = f16_to_f32((u16) max(max(s_scale[s][0], s_scale[s][1]), max(s_scale[s][2], s_scale[s][3])));
+        wide = wide || f16_to_f32((u16) min(min(s_least[s][0], s_least[s][1]), min(s_least[s][2], s_least[s][3]))) * 0x1p10f < largest[s];
+        bound[s] = am * largest[s];
+    }
+    bool loose[2] = {false, false};
+    if (__builtin_amdgcn_ballot_w64(wide)) {
+        const u32 at = most[2 * token + 1];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const u16x4 own = *(const u16x4*) (suh[s] + at) & (u16) 0x7fff;
+            loose[s] = f16_to_f32(min(min(own[0], own[1]), min(own[2], own[3]))) * 0x1p10f < largest[s];
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(loose[0] || loose[1])) {   // the same in all four waves
+        float p[2] = {0.0f, 0.0f};
+#pragma unroll 1
+        for (u32 kb = wave; kb < kbs; kb += 4) {
+            f32x4 v[8];
+            inputs(kb);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                scaled(s, kb, v);
+                p[s] = fmaxf(p[s], xpf_token_max(v, lane));
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+            if (lane < 16) s_most[s][wave][lane] = p[s];
+        inputs(min(wave, kbs - 1));
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const u32 t = lane & 15;
+            if (loose[s]) bound[s] = fmaxf(fmaxf(s_most[s][0][t], s_most[s][1][t]), fmaxf(s_most[s][2][t], s_most[s][3][t]));
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
         float iv;
-        pow2_scale_of(f32_bits(am * f16_to_f32((u16) m)), scale[s], iv);
+        pow2_scale_of(f32_bits(bound[s]), scale[s], iv);
         scale[s] *= 0.0078125f;
         if (wave == 0 && lane < 16) inv[(it.base * 2 + s * it.tiles + T) * 16 + lane] = iv * XPF_UNSCALE;
     }
-    const float* xr = x + (u64) token * hidden + 4 * (lane >> 4);
     for (u32 kb = wave; kb < kbs; kb += 4) {
-        f32x4 xv[8];
-#pragma unroll
-        for (int ks = 0; ks < 8; ks++) xv[ks] = *(const f32x4*) (xr + kb * 128 + 16 * ks);
+        if (kb != wave) inputs(kb);
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             f32x4 v[8];
+            scaled(s, kb, v);
 #pragma unroll
-            for (int ks = 0; ks < 8; ks++) {
-                const u16x4 s4 = *(const u16x4*) (suh[s] + kb * 128 + 16 * ks + 4 * (lane >> 4));
-#pragma unroll
-                for (int q = 0; q < 4; q++) v[ks][q] = (xv[ks][q] * f16_to_f32(s4[q])) * scale[s];
-            }
+            for (int ks = 0; ks < 8; ks++) v[ks] *= scale[s];
             xpf_transform(v);
             xpf_put_transformed(rows + ((u64) it.base * 2 + s * it.tiles) * kbs * XPF_ROWS_U16 + (2 * kb * it.tiles + T) * XPF_HALF_U16, it.tiles * XPF_HALF_U16, v, lane);
         }

@@ -51,22 +51,31 @@ extern "C" __global__ void __launch_bounds__(256) moe_combine_qwen_rows(float* y
 // Routing alone: tidx[j*k + t], weights[j*k + t] (f32), cnt[j] experts chosen, one wave a token.  grid = ceil(m / 4), block 256; ne <= 512, k <= 16.
 // The weights are ex_t over the sum of the chosen ex (route_weights_chosen): a prefill chunk routes thousands of tokens, and
 // the sum over all experts that cancels out of them is 512 f64 exponentials a token.
-// amax (0: not wanted): the largest magnitude of every token's input row x[hidden].
-extern "C" __global__ void __launch_bounds__(256) route_topk_rows(const float* logits, u32* tidx, float* weights, u32* cnt, u32 ne, u32 k, u32 m, const float* x, float* amax, u32 hidden) {
+// most (0: not wanted): of every token's input row x[hidden] the largest magnitude (f32 bits) and the first four channels that have it.
+extern "C" __global__ void __launch_bounds__(256) route_topk_rows(const float* logits, u32* tidx, float* weights, u32* cnt, u32 ne, u32 k, u32 m, const float* x, u32* most, u32 hidden) {
     __shared__ double exs[4][512];
     __shared__ u32 tops[4][16];
     const u32 lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const u32 j = blockIdx.x * 4 + w;
     if (j >= m) return;
-    if (amax) {
+    if (most) {
         float mx = 0.0f;
+        u32 at = 0;
 #pragma unroll 8
         for (u32 i = lane; i < hidden / 4; i += 64) {
             const f32x4 v = ((const f32x4*) (x + (u64) j * hidden))[i];
-            mx = fmaxf(fmaxf(fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3]))), mx);
+            const float a = fmaxf(fmaxf(__builtin_fabsf(v[0]), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
+            if (a > mx) {
+                mx = a;
+                at = 4 * i;
+            }
         }
-        mx = wave_max_f32(mx);
-        if (lane == 0) amax[j] = mx;
+        const float all = wave_max_f32(mx);
+        at = wave_min_u32(mx == all ? at : 0xffffffffu);
+        if (lane == 0) {
+            most[2 * (u64) j] = f32_bits(all);
+            most[2 * (u64) j + 1] = at;
+        }
     }
     route_ids(logits + (u64) j * ne, ne, k, lane, exs[w], tops[w]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

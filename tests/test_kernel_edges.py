@@ -500,3 +500,35 @@ def test_exl3_prefill_blocks_of_any_size_beside_each_other(gpu, kb, tokens):  # 
     for i, j in enumerate(rows):
         assert rel_l2(got[j], want[i]) <= 1e-3, (orders[j % ne], rel_l2(got[j], want[i]))
     assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("kb", [3, 6])
+@pytest.mark.parametrize("tokens", [19, 700])
+def test_exl3_prefill_large_inputs_that_an_expert_scales_to_nothing(gpu, kb, tokens):  # noqa: F811
+    """Inputs far above the others in channels whose scale is zero, f16's least, or a thousandth of the largest: what counts is the product, and the other channels keep
+    their bits (within the chunk's 1e-3 of the oracle)."""
+    rng = np.random.default_rng(kb * 1000 + tokens)
+    hidden, ff, ne, k, ty = 512, 256, 4, 2, sz.EXL3(kb)
+    dbuf, stride, blobs, _ = build_layer(gpu, rng, ty, hidden, ff, ne, False)
+    gb, _, _ = synth.expert_bytes(ty, hidden, ff)
+    for e in range(ne):
+        for at in (0, gb):
+            suh = blobs[e][at:at + 2 * hidden].view(np.float16)
+            most = np.abs(suh.astype(np.float32)).max()
+            suh[[3, 300, 7, 9]] = 0.0, 6e-8, most / 1024, most / 1200      # both sides of the line where launch 1 takes a pass for the products
+        dbuf[e * stride:e * stride + blobs[e].size] = dev(gpu, blobs[e])
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, 0, 0)
+    x, logits = rng.normal(size=(tokens, hidden)).astype(np.float32), rng.normal(size=(tokens, ne)).astype(np.float32)
+    x[0::4, 3] = 1e12
+    x[1::4, 3] = -3.3e38
+    x[2::4, 300] = 3e8
+    x[3::8, 7], x[7::8, 9] = 2e5, 2e5
+    y = gpu.zeros((tokens, hidden), dtype=gpu.float32, device="cuda")
+    dx, dl, dg = dev(gpu, x), dev(gpu, logits), dev(gpu, np.zeros(tokens, np.float32))
+    s.moe_prefill_chunk(0, tokens, dx.data_ptr(), dl.data_ptr(), dg.data_ptr(), y.data_ptr())
+    gpu.cuda.synchronize()
+    got, rows = y.cpu().numpy(), np.r_[:12, tokens - 4:tokens]
+    want, _, _ = oracle_layer(ty, hidden, ff, k, blobs, None, logits[rows], np.zeros(rows.size, np.float32), x[rows])
+    for i, j in enumerate(rows):
+        assert rel_l2(got[j], want[i]) <= 1e-3, (j, rel_l2(got[j], want[i]))
