@@ -1318,7 +1318,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0, items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
         {
             const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens), P(x), P(pb.most.ptr), U32(c.hidden)};
-            if (launch("route_topk_rows", (tokens + 3) / 4, 1, 1, 256, 0, stream, a)) return 1;
+            if (launch("route_topk_rows", (tokens + 3) / 4 * 2, 1, 1, 256, 0, stream, a)) return 1;
         }
         {
             const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr),
