@@ -1309,8 +1309,33 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         // EXL3 experts: f16 activations on the columns of the matrix instruction, items of up to 128 pairs, of 64 for the down
         // products (kernels/exl3.hip, "the prefill chunk of an EXL3 layer": XPF_NT, XPF_DOWN_NT, XPF_ROWS_U16, XPF_RING)
         if (c.ff > 512) return fail("sz_moe_prefill_chunk: EXL3 experts of more than 512 intermediate features are not built (a workgroup keeps four 128-blocks of a token)");
-        const uint32_t most = f.bits <= 5 ? 8 : 6, tok = 16 * most, kbs = c.hidden / 128, fbs = c.ff / 128, ntl = std::min<uint32_t>(most, (tokens + 15) / 16);
-        const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1, max_items = some + rows / tok, max_down = some + rows / 64, tiles = rows / 16 + c.n_expert + 2;
+        const uint32_t kbs = c.hidden / 128, fbs = c.ff / 128, widest = f.bits <= 5 ? 8 : 6;
+        const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1;
+        // The gate and up launch: two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, whose rings are
+        // deeper, where the work is little or where eight waves would leave compute units without a workgroup (3 bits, 512 experts of
+        // 2048 x 512, top-10: 45 tokens 102 us with four waves and 123 with eight, 200 tokens 178 and 176, 512 254 and 252, 1024 371 and
+        // 344; 600 tokens through 60 of 1024 x 256, top-8: 105 and 119; 2048 through 64 of 2048 x 512, top-4: 254 and 243; 1500 through
+        // 32: 177 and 188).  By the bound on the items: how many experts the router reaches the host does not know.
+        const bool wide_gu = rows * fbs >= 16000 && (some + rows / (16 * widest)) * fbs >= 512;
+        // Of four waves, items so short that the chip is full: an item's chain over all inputs takes about 2.5 + its tiles, its workgroups a
+        // compute unit each, of a single tile half a unit (1.2 units' time for two of them).  Routers prefer some experts: 0.4 of those that
+        // independent choices would reach, the experts' last tiles and the rest of the pairs in whole items.  us with items of up to 128,
+        // 64, 32 and 16 pairs, router with Zipf's preferences and without: 45 tokens through 512 experts of 2048 x 512, top-10, and the
+        // shared one, 3 bits 115, 115, 127, 102 and 291, 291, 290, 215; 500 through 32 of 2048 x 512, top-2, 3 bits 113, 95, 83, 101 and 94,
+        // 90, 82, 101; 200 through 128 of 4096 x 512, top-8, and the shared one, 4 bits 216, 220, 226, 242 and 291, 288, 286, 242; 700
+        // through 64 of 3072 x 512, top-6, and the shared one, 4 bits 247, 252, 322, 356 and 253, 251, 298, 352.
+        const double reached = 0.4 * c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) T));
+        uint32_t most = widest;
+        if (!wide_gu) {
+            double best = 1e30;
+            for (uint32_t n : {widest, 4u, 2u, 1u}) {
+                const double chain = 2.5 + (double) std::min<uint64_t>(n, (T + 15) / 16), work = reached * 3.5 + (double) rows / (16 * n) * chain;
+                const double cost = n > 1 ? std::max(chain, 1.4 / 256 * fbs * work) : work * fbs <= 256 * chain ? chain : std::max(4.7, 0.83 / 256 * fbs * work);
+                if (cost < best) best = cost, most = n;
+            }
+        }
+        const uint32_t tok = 16 * most, ntl = std::min<uint32_t>(most, (tokens + 15) / 16), nt = ntl <= 2 ? ntl : ntl + ntl % 2, nd = std::min(4u, nt);
+        const uint64_t max_items = some + rows / tok, max_down = some + rows / (16 * nd), tiles = rows / 16 + c.n_expert + 2;
         const uint32_t bound = (uint32_t) ((max_items + 7) / 8 * 8), bound_d = (uint32_t) ((max_down + 7) / 8 * 8);   // workgroups an item's part (xpf_place)
         if (pb.lay({{&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4}, {&pb.items, (2 + 2 * max_items + 2 * max_down) * 4},
                     {&pb.eo, rows * c.hidden * 4}, {&pb.most, T * 8}, {&pb.arows, tiles * 2 * kbs * 4096}, {&pb.ainv, tiles * 2 * 64}, {&pb.drows, tiles * fbs * 4096}, {&pb.dinv, tiles * fbs * 64}}))
@@ -1322,39 +1347,39 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         }
         {
             const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr),
-                                P(pb.items.ptr), P(items_d), U32(tok), U32(64)};
+                                P(pb.items.ptr), P(items_d), U32(tok), U32(16 * nd)};
             if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
         }
         {
+            // shares of the inputs' 128-blocks, as many as make about 1200 workgroups of a few tiles (45 tokens through 512 experts of 2048 x 512
+            // as above 121, 118, 117, 115 us with 1 to 4, 250 as above 159, 152, 146, 150, 1200 through 128 of 4096 x 512, top-8, at 4 bits
+            // 574, 564, 563, 561)
+            const uint32_t shares = (uint32_t) std::max(1.0, std::min<double>(kbs / 4, std::floor(1200.0 / (reached + rows / 16) + 0.5)));
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(x), P(pb.most.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), U32(c.n_expert),
-                                U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(tok), U32(ntl)};
-            if (launch("prefill_rotate_exl3", bound * ntl, 1, 1, 256, 0, stream, a)) return 1;
+                                U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(tok), U32(ntl), U32(shares)};
+            if (launch("prefill_rotate_exl3", bound * ntl * shares, 1, 1, 256, 0, stream, a)) return 1;
         }
-        const uint32_t nt = ntl <= 2 ? ntl : ntl + ntl % 2, bits = (uint32_t) f.bits, wide_ring = bits <= 7 ? 3 : 2;
+        const uint32_t bits = (uint32_t) f.bits, wide_ring = bits <= 7 ? 3 : 2;
         {
-            // two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, whose rings are deeper, where the
-            // work is little or where eight waves would leave compute units without a workgroup (3 bits, 512 experts of 2048 x 512, top-10:
-            // 45 tokens 102 us with four waves and 123 with eight, 200 tokens 178 and 176, 512 254 and 252, 1024 371 and 344; 600 tokens
-            // through 60 of 1024 x 256, top-8: 105 and 119; 2048 through 64 of 2048 x 512, top-4: 254 and 243; 1500 through 32: 177 and 188)
-            const bool wide = rows * fbs >= 16000 && max_items * fbs >= 512;
-            const uint32_t ncb = wide ? 2 : 1;
+            const uint32_t ncb = wide_gu ? 2 : 1;
             // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING, XPF_RING_N), afterwards the exchange of four tiles' sums
             uint32_t lds = ncb * 2 * std::min(4u, nt) * 8192;
             for (uint32_t n = 1; n <= nt; n += n == 1 ? 1 : 2) {
-                const uint32_t deep = n <= 2 ? (bits <= 4 ? 8 : 12 - bits) : n == 4 ? (bits <= 5 ? 5 : 4) : wide_ring, ring = wide ? wide_ring : deep;
-                lds = std::max(lds, (wide ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
+                const uint32_t deep = n == 1 ? (bits <= 2 ? 8 : bits <= 5 ? 10 - bits : bits <= 7 ? 4 : 3) : n == 2 ? (bits <= 4 ? 8 : 12 - bits) : n == 4 ? (bits <= 5 ? 5 : 4) : wide_ring, ring = wide_gu ? wide_ring : deep;
+                lds = std::max(lds, (wide_gu ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
             }
-            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff)};
-            if (launch(((wide ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 256 * ncb, lds, stream, a)) return 1;
+            const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff), U32(tok)};
+            if (launch(((wide_gu ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 256 * ncb, lds, stream, a)) return 1;
         }
         {
-            // shares of an item: one wave a column block in the end where items are few, all blocks on eight waves, whose start then counts
-            // once, where they fill the chip (1, 2 shares of 8 waves, 4 of 4: 45 tokens as above 137, 109, 101 us, 512 tokens 257, 252, 267,
-            // 4096 at 4 bits 967, 988, 1071; 8 and 4 waves: 764 tokens, top-3 of 128 of 1792 x 256 and the shared one, 2 bits 142, 132,
-            // 700 through 64 of 1024 x 256, top-4, 97, 93, 380 through 256 of 3072 x 256, top-8, at 5 bits 230, 242, 190 as above 178, 182)
+            // shares of an item: a wave a column block, but all blocks on eight waves, whose start then counts once, where items fill the chip (1, 2
+            // shares of 8 waves, 4 of 4: 45 tokens as above 137, 109, 101 us, 512 tokens 257, 252, 267, 4096 at 4 bits 967, 988, 1071; 4 and
+            // 8 shares of 4: 64 tokens through 60 of 4096 x 512, top-4, 4 bits 167, 150; 8 and 4 waves: 764 tokens, top-3 of 128 of 1792 x 256
+            // and the shared one, 2 bits 142, 132, 700 through 64 of 1024 x 256, top-4, 97, 93, 380 through 256 of 3072 x 256, top-8, at 5
+            // bits 230, 242, 190 as above 178, 182)
             const bool wide = rows * fbs * kbs >= 115000;
-            const uint32_t waves = std::min(wide ? 8u : 4u, kbs), parts = std::max((kbs + 4 * waves - 1) / (4 * waves), std::min(rows >= 20000 ? 1u : wide ? 2u : 4u, kbs / waves)), nd = std::min(4u, nt);
-            const uint32_t ring = wide ? wide_ring : bits <= 4 ? 8 : bits <= 6 ? 6 : 4;   // XPF_RING, XPF_RING_DOWN_N
+            const uint32_t waves = std::min(wide ? 8u : 4u, kbs), parts = rows >= 20000 ? (kbs + 4 * waves - 1) / (4 * waves) : (kbs + waves - 1) / waves;
+            const uint32_t ring = wide ? wide_ring : bits <= 3 ? 8 : bits == 4 ? 7 : bits == 5 ? 5 : bits <= 7 ? 4 : 3;   // XPF_RING, XPF_RING_DOWN_N
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(items_d), P(pb.drows.ptr), P(pb.dinv.ptr), P(pb.eo.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff),
                                 U32(nd), U32(parts)};
             if (launch(((wide ? "prefill_down_" : "prefill_down_n_") + tag).c_str(), bound_d * parts, 1, 1, 64 * waves, 4 * (nd * fbs * 1040 + 256 * waves) + waves * ring * 512 * bits, stream, a)) return 1;

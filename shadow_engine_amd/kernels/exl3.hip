@@ -1416,10 +1416,11 @@ EXL3_HEAD_ENTRIES(8)
 // Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for.
 #define XPF_NT(K) ((K) <= 5 ? 8 : 6)
 // Units of a wave's ring of trellis rows: what eight waves have room for, and in workgroups of four waves (few items, whose weights come
-// from memory rather than a cache: their trip is what the launch waits for) as deep as the operand rows of NT tiles leave room.
+// from memory rather than a cache: their trip is what the launch waits for) as deep as the operand rows of NT tiles leave room, of one tile
+// in half a compute unit's LDS: then two workgroups share a unit.
 #define XPF_RING(K) ((K) <= 7 ? 3 : 2)
-#define XPF_RING_N(K, NT) ((NT) <= 2 ? ((K) <= 4 ? 8 : 12 - (K)) : (NT) == 4 ? ((K) <= 5 ? 5 : 4) : XPF_RING(K))
-#define XPF_RING_DOWN_N(K) ((K) <= 4 ? 8 : (K) <= 6 ? 6 : 4)
+#define XPF_RING_N(K, NT) ((NT) == 1 ? ((K) <= 2 ? 8 : (K) <= 5 ? 10 - (K) : (K) <= 7 ? 4 : 3) : (NT) == 2 ? ((K) <= 4 ? 8 : 12 - (K)) : (NT) == 4 ? ((K) <= 5 ? 5 : 4) : XPF_RING(K))
+#define XPF_RING_DOWN_N(K) ((K) <= 3 ? 8 : (K) == 4 ? 7 : (K) == 5 ? 5 : (K) <= 7 ? 4 : 3)
 // What undoes the 1 / 128 that the stored values carry and applies the transform's 1 / sqrt(128)
 #define XPF_UNSCALE 11.3137085f
 typedef u16 u16x4 __attribute__((ext_vector_type(4)));
@@ -1562,21 +1563,21 @@ __device__ __forceinline__ void xpf_tiles(u32 tiles, F&& run) {
     run(XpfInt<4>());
 }
 
-// Launch 1: a tile (16 tokens) of an item; wave w takes the 128-blocks w, w + 4, .. of the inputs.  A token's power of two takes a bound
+// Launch 1: a tile (16 tokens) of an item and one of `shares` of the inputs' 128-blocks: wave w takes 4 share + w, from there 4 shares on, ..  A token's power of two takes a bound
 // of its inputs times the projection's input scales to [2^7, 2^8): no value passes 2^15 in the transform.  Values 2^21 below the bound are
 // f16's subnormals, whose last bit is 2^31 below it.  The bound is the largest input (most, from the routing launch) times the largest
 // scale where all scales, or those of the four channels about that input, are within 2^10 of the largest, so that the bound is no further than
 // that from the largest product; else (a large input of a channel that the expert scales to next to nothing) the largest product, which
 // takes another pass over the inputs (such a pass for every token: 52 us of 4096 tokens' 920, 4 of 45 tokens' 121).
 // rows: an item's [gate, up][64-block][tile], inv: [gate, up][tile][16].
-// Bound by the rows it writes (8 bytes an input and pair).  grid = xpf_place's, of `tiles` parts, block 256.
+// Bound by the rows it writes (8 bytes an input and pair).  grid = xpf_place's, of `tiles * shares` parts, block 256.
 extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const float* x,
-                                                                      const u32* most, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles) {
+                                                                      const u32* most, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles, u32 shares) {
     __shared__ u32 s_scale[2][4], s_least[2][4];
     __shared__ float s_most[2][4][16];
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, kbs = hidden / 128;
-    u32 T;
-    const u32 item = xpf_place(tiles, T);
+    u32 part;
+    const u32 item = xpf_place(tiles * shares, part), T = part / shares, share = part - T * shares, first = share * 4 + wave;
     const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, tok);
     if (T >= it.tiles) return;
     const u32 e = it.e, pair = list[it.first + min(16 * T + (lane & 15), it.n - 1)];   // places past the item's end repeat its last pair: nothing reads them
@@ -1607,7 +1608,7 @@ extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64*
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) xv[ks] = *(const f32x4*) (xr + kb * 128 + 16 * ks);
     };
-    inputs(min(wave, kbs - 1));   // on their way while the scales' maxima are made
+    inputs(min(first, kbs - 1));   // on their way while the scales' maxima are made
     __syncthreads();
     // a block's inputs times their scales
     auto scaled = [&](u32 s, u32 kb, f32x4 (&v)[8]) {
@@ -1650,7 +1651,7 @@ extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64*
 #pragma unroll
         for (int s = 0; s < 2; s++)
             if (lane < 16) s_most[s][wave][lane] = p[s];
-        inputs(min(wave, kbs - 1));
+        inputs(min(first, kbs - 1));
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < 2; s++) {
@@ -1663,10 +1664,10 @@ extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64*
         float iv;
         pow2_scale_of(f32_bits(bound[s]), scale[s], iv);
         scale[s] *= 0.0078125f;
-        if (wave == 0 && lane < 16) inv[(it.base * 2 + s * it.tiles + T) * 16 + lane] = iv * XPF_UNSCALE;
+        if (first == 0 && lane < 16) inv[(it.base * 2 + s * it.tiles + T) * 16 + lane] = iv * XPF_UNSCALE;
     }
-    for (u32 kb = wave; kb < kbs; kb += 4) {
-        if (kb != wave) inputs(kb);
+    for (u32 kb = first; kb < kbs; kb += 4 * shares) {
+        if (kb != first) inputs(kb);
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             f32x4 v[8];
@@ -1866,21 +1867,21 @@ __device__ __forceinline__ void xpf_take(const f32x4* x, u32 place, f32x4 (&v)[8
     for (u32 c = 0; c < 8; c++) v[c] = x[(place * 8 + c) * 64 + lane];
 }
 
-// Launch 2: an item and NCB 128-column blocks of ff, four waves a block (gate's two halves, up's).  rows2:
+// Launch 2: an item (of up to tok pairs) and NCB 128-column blocks of ff, four waves a block (gate's two halves, up's).  rows2:
 // [tile][128-block of ff], inv2: [tile][128-block][16].  grid = xpf_place's, of ff / 128 / NCB parts, block 256 NCB; dynamic LDS: NB
 // slots of two projections' NT tiles and the waves' rings (for the NT of 1, 2, 4, 6, 8 that takes most), or the exchange of the sums, 64
 // KiB NCB for four tiles.
 template <int K, int NCB>
 __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs, const u32* __restrict__ items,
                                                             const u16* __restrict__ rows, const float* __restrict__ inv, u16* __restrict__ rows2, float* __restrict__ inv2, u32 ne, u32 hidden,
-                                                            u32 ff) {
+                                                            u32 ff, u32 tok) {
     extern __shared__ __attribute__((aligned(16))) u32 dyn[];
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const u32 sel = wave / (2 * NCB), part = wave % (2 * NCB), b = part / 2, half = part & 1;
     const u32 kbs = hidden / 128, fbs = ff / 128;
     u32 group;
     const u32 item = xpf_place(fbs / NCB, group), cb = group * NCB + b;
-    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, 16 * XPF_NT(K));
+    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, tok);
     if (it.n == 0) return;
     const u32 e = it.e;
     const u8* bg = (const u8*) (e < ne ? eaddr[e] : sh_addr[0]);
@@ -1923,10 +1924,10 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
     });
 }
 
-// Launch 3: an item of up to XPF_DOWN_NT tiles and one of `parts` shares of the 128-column blocks of hidden, a wave a block at a time: the
+// Launch 3: an item of up to ntl (at most XPF_DOWN_NT) tiles and one of `parts` shares of the 128-column blocks of hidden, a wave a block at a time: the
 // products of the item's operand rows over ff and the output side: eo[pair][hidden].  The rows, their factors and the output scales are copied
 // to LDS once; from then on every wave goes its own way, its ring of trellis rows filled from one block to the next.
-// grid = xpf_place's, block 64 W; dynamic LDS in words: NTL tiles' rows (fbs * 1024 each), factors (fbs * 16 each), 64
+// grid = xpf_place's, block 64 W; dynamic LDS in words: ntl tiles' rows (fbs * 1024 each), factors (fbs * 16 each), 64
 // XPF_DOWN_BLOCKS a wave for the output scales, the waves' rings.
 #define XPF_DOWN_NT 4
 #define XPF_DOWN_BLOCKS 4   /* most column blocks of a wave: parts * W * 4 >= hidden / 128 */
@@ -1941,7 +1942,7 @@ __device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__
     const u32 fbs = ff / 128, cbs = hidden / 128, U = 4 * fbs;   // U: units a column block
     u32 share;
     const u32 item = xpf_place(parts, share);
-    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, 16 * XPF_DOWN_NT);
+    const XpfItem it = xpf_item(offs, items, item, ne, sh_addr != nullptr, 16 * ntl);
     if (it.n == 0) return;
     const u8* down = (const u8*) uniform_u64(it.e < ne ? eaddr[2ull * ne + it.e] : sh_addr[2]);
     const u32 cb0 = share * W + wave, stride = parts * W;        // the wave's column blocks: cb0, cb0 + stride, ..
@@ -2068,12 +2069,12 @@ __device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__
 
 #define EXL3_PREFILL_ENTRIES(K) \
     extern "C" __global__ void __launch_bounds__(512, 2) prefill_gate_up_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
-                                                                                  float* inv2, u32 ne, u32 hidden, u32 ff) { \
-        prefill_gate_up_exl3_kernel<K, 2>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff); \
+                                                                                  float* inv2, u32 ne, u32 hidden, u32 ff, u32 tok) { \
+        prefill_gate_up_exl3_kernel<K, 2>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff, tok); \
     } \
     extern "C" __global__ void __launch_bounds__(256, 2) prefill_gate_up_n_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
-                                                                                    float* inv2, u32 ne, u32 hidden, u32 ff) { \
-        prefill_gate_up_exl3_kernel<K, 1>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff); \
+                                                                                    float* inv2, u32 ne, u32 hidden, u32 ff, u32 tok) { \
+        prefill_gate_up_exl3_kernel<K, 1>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff, tok); \
     } \
     extern "C" __global__ void __launch_bounds__(512, 2) prefill_down_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const u16* rows, const float* inv, \
                                                                                float* eo, u32 ne, u32 hidden, u32 ff, u32 ntl, u32 parts) { \

@@ -532,3 +532,37 @@ def test_exl3_prefill_large_inputs_that_an_expert_scales_to_nothing(gpu, kb, tok
     want, _, _ = oracle_layer(ty, hidden, ff, k, blobs, None, logits[rows], np.zeros(rows.size, np.float32), x[rows])
     for i, j in enumerate(rows):
         assert rel_l2(got[j], want[i]) <= 1e-3, (j, rel_l2(got[j], want[i]))
+
+
+@pytest.mark.parametrize("kb,hidden,ff,ne,k,shared,chunks", [
+    (3, 1280, 512, 32, 2, False, (1400, 500, 60, 17)),        # items of up to 128 pairs, 32, 16; ten 128-blocks of hidden
+    (2, 512, 256, 60, 8, False, (1300, 900, 100)),            # 128, 64, 16
+    (4, 4096, 512, 16, 2, False, (260, 120, 20)),             # 32 blocks: shares of the rotation and of the down products
+    (1, 256, 256, 40, 3, True, (1030, 200, 33, 1)),           # two blocks
+    (2, 512, 512, 300, 8, False, (560, 130, 48)),             # two launches of eight waves, then four
+    (5, 1024, 512, 140, 8, True, (500, 90)), (7, 1024, 512, 140, 8, True, (500, 90)),
+    (6, 768, 256, 32, 6, True, (400, 40)), (8, 768, 512, 32, 6, False, (400, 40))])
+def test_exl3_prefill_bits_do_not_depend_on_the_chunk(gpu, kb, hidden, ff, ne, k, shared, chunks):  # noqa: F811
+    """The first tokens of a chunk in chunks of their own, through the other forms and item lengths: the same bits, within the chunk's
+    1e-3 of the oracle."""
+    rng = np.random.default_rng(kb * 1000 + hidden)
+    ty, most = sz.EXL3(kb), max(chunks)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, shared)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty if shared else 0, dbuf.data_ptr() + ne * stride if shared else 0)
+    x, logits = rng.normal(size=(most, hidden)).astype(np.float32), synth.zipf_router_logits(rng, most, ne)
+    sgl = rng.normal(size=most).astype(np.float32)
+    dx, dl, dg = dev(gpu, x), dev(gpu, logits), dev(gpu, sgl)
+    first = None
+    for tokens in chunks:
+        y = gpu.zeros((tokens, hidden), dtype=gpu.float32, device="cuda")
+        s.moe_prefill_chunk(0, tokens, dx.data_ptr(), dl.data_ptr(), dg.data_ptr(), y.data_ptr())
+        gpu.cuda.synchronize()
+        got = y.cpu().numpy()
+        if first is None:
+            first = got
+            rows = np.unique(np.r_[0, rng.integers(0, tokens, 10), tokens - 1])
+            want, _, _ = oracle_layer(ty, hidden, ff, k, blobs, sh, logits[rows], sgl[rows], x[rows])
+            for i, j in enumerate(rows):
+                assert rel_l2(got[j], want[i]) <= 1e-3, (j, rel_l2(got[j], want[i]))
+        assert np.array_equal(bits(got), bits(first[:tokens])), tokens
