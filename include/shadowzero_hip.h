@@ -170,9 +170,9 @@ void sz_layer_spacing(int32_t expert_type, uint64_t hidden, uint64_t ff, uint32_
  * sz_verify_round) is fused into the product for Q8_0 and EXL3; the other types go through their logits, kept in a buffer
  * this call allocates (max_rows x vocab floats), as the reference's mv_cols + topk_rows_at do (session.rs:7034-7052). */
 int32_t sz_session_set_head(sz_session*, int32_t ggml_type, uint64_t w);
-/* LDS a workgroup of the EXL3 head's kernel takes for m rows (0 for another type): the head entry points refuse a call
- * whose need is above a compute unit's 160 KiB (hidden 4096 takes all 8 rows at any rate, hidden 8192 up to 4), and
- * sz_session_set_head a head that cannot take one row.  No counterpart in the reference (its kernels take 64 rows in registers). */
+/* What limits the rows of a call on an EXL3 head: the head entry points refuse m rows where this is above 160 KiB (hidden 4096
+ * takes all 8 rows at any rate, hidden 8192 up to 4); 0 for another type.  The bytes of LDS that the rows and the trellis of a
+ * workgroup would take together; the kernel takes less.  No counterpart in the reference (its kernels take 64 rows in registers). */
 uint32_t sz_exl3_head_lds_bytes(int32_t type, uint32_t hidden, uint32_t m);
 /* The optional, INEXACT 2-bit screen of an EXL3 head for the top-64 hand-off (HeadProxy, session.rs:428-441, built at
  * session.rs:2631-2674 by exl3_build_q2_proxy_K, kernels/exl3.cu:916-996; used by head_top_at, session.rs:5952-6022): off by
@@ -249,7 +249,8 @@ int32_t sz_copy_ranges(const uint64_t* ranges, uint32_t n, uint64_t stream);
  * block maxima f32[m][vocab / 128], 11 the list of chosen blocks (count, then the blocks ascending), 12 the packed logits of the
  * listed blocks (rows 128 * min(m * k_use, vocab / 128) apart); of the prefill chunk of EXL3 experts: 13 the operand rows
  * of the gate and up launch, 14 the pairs' down rows, 15 the operand rows of the down launch, 16 their factors, 17 the work items.  0 for any
- * other `which`. */
+ * other `which`.  13 to 17 are parts of one allocation that every chunk lays out anew: an address is that of the last chunk and
+ * stale after the next one. */
 uint64_t sz_session_buffer(sz_session*, int32_t which);
 
 /* A whole verify round over device-resident inputs: for every layer l the MoE block on u[l][m][hidden] with rl[l][m][ne]

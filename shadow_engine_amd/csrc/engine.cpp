@@ -748,13 +748,12 @@ int head_argmax_mfma(sz_session* s, uint32_t m, uint64_t u, uint64_t logits, uin
 
 bool head_is_exl3(const sz_session* s) { return s->head_type >= 1021 && s->head_type <= 1028; }
 
-// What bounds the rows a call of an EXL3 head takes (kept from when its A rows lay in LDS: callers size their batches by it): the bytes of
-// four 4-row rings (a row is 64 lanes x 4 words at K = 3 and 4, x K words otherwise) and 4 KiB of A rows for every 512 inputs and
-// every two rows, against a compute unit's.
-uint32_t exl3_head_lds_dynamic(uint32_t hidden, uint32_t m) { return 4 * ((hidden / 128 + 3) / 4) * ((m + 1) / 2) * 1024; }
+// The rows a call of an EXL3 head may bring are a limit of this interface, which callers size their batches by (sz_exl3_head_lds_bytes
+// against CU_LDS_BYTES): the LDS of a workgroup that keeps its A rows there, four 4-row rings (a row is 64 lanes x 4 words at K = 3 and
+// 4, x K words otherwise) and 4 KiB for every 512 inputs and every two rows.  head_exl3_K itself takes 24 KiB whatever the rows.
 uint32_t exl3_head_lds(uint32_t bits, uint32_t hidden, uint32_t m) {
     const uint32_t stride = (bits == 3 || bits == 4) ? 4 : bits;
-    return 4 * (4 * 64 * stride) * 4 + exl3_head_lds_dynamic(hidden, m);
+    return 4 * (4 * 64 * stride) * 4 + 4 * ((hidden / 128 + 3) / 4) * ((m + 1) / 2) * 1024;
 }
 
 int head_check(sz_session* s, uint32_t m, uint64_t u, const char* who) {
@@ -762,9 +761,8 @@ int head_check(sz_session* s, uint32_t m, uint64_t u, const char* who) {
     if (m == 0 || m > s->cfg.max_rows) return fail(std::string(who) + ": " + std::to_string(m) + " rows");
     if (u & 15) return fail(std::string(who) + ": activations must be 16-byte aligned");
     if (head_is_exl3(s) && exl3_head_lds((uint32_t) s->head_type - 1020, s->cfg.hidden, m) > CU_LDS_BYTES)
-        return fail(std::string(who) + ": an EXL3 head of hidden " + std::to_string(s->cfg.hidden) + " at " + std::to_string(s->head_type - 1020) + " bits takes " +
-                    std::to_string(exl3_head_lds((uint32_t) s->head_type - 1020, s->cfg.hidden, m)) + " bytes of LDS for " + std::to_string(m) +
-                    " rows, a compute unit has " + std::to_string(CU_LDS_BYTES) + ": fewer rows a call");
+        return fail(std::string(who) + ": " + std::to_string(m) + " rows are above the limit of an EXL3 head of hidden " + std::to_string(s->cfg.hidden) + " at " +
+                    std::to_string(s->head_type - 1020) + " bits (sz_exl3_head_lds_bytes above " + std::to_string(CU_LDS_BYTES) + "): fewer rows a call");
     return 0;
 }
 
@@ -1062,9 +1060,7 @@ int32_t sz_session_set_head(sz_session* s, int32_t ty, uint64_t w) {
     if (exl3) {
         const sz_session_config& c = s->cfg;
         if (c.vocab == 0 || c.vocab % 128 || c.hidden % 128 || c.hidden > 8192) return fail("sz_session_set_head: an EXL3 head needs hidden (<= 8192) and the vocabulary to be multiples of 128");
-        // a head that cannot take even one row is refused here; how many rows a call may bring is checked call by call
-        if (exl3_head_lds((uint32_t) ty - 1020, c.hidden, 1) > CU_LDS_BYTES)
-            return fail("sz_session_set_head: an EXL3 head of hidden " + std::to_string(c.hidden) + " does not fit a compute unit's LDS");
+        // one row is within the limit of every such head; how many a call may bring is checked call by call
         if (s->head_xa.need((uint64_t) c.hidden / 128 * 16 * 256) || s->head_inv.need(64)) return 1;
     }
     s->head_type = ty;

@@ -127,9 +127,9 @@ def test_grid_table_copies_are_identical():
     assert len(a) == 512 and a == b
 
 
-def test_the_exl3_heads_lds_bound_is_what_the_kernel_takes():
-    """head_exl3_K: four 4-row rings (static) + 4 KiB of A rows for every 512 inputs and two rows (dynamic), against the 160 KiB of
-    a compute unit: hidden 4096 takes 8 rows at every rate (exactly 160 KiB at K = 8), hidden 8192 at most 4."""
+def test_the_limit_on_the_rows_of_an_exl3_head():
+    """Four 4-row rings and 4 KiB of A rows for every 512 inputs and two rows, against the 160 KiB of a compute unit: hidden 4096
+    takes 8 rows at every rate (exactly 160 KiB at K = 8), hidden 8192 at most 4."""
     L = sz.lib()
     ring = lambda k: 4 * 4 * 64 * (4 if k in (3, 4) else k) * 4
     for k in range(1, 9):
