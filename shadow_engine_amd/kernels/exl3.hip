@@ -176,75 +176,6 @@ __device__ __forceinline__ void wht128_wave(float& v0, float& v1, u32 lane) {
     v1 *= 0.08838835f;
 }
 
-// ------------------------------------------------------------------------------------- trellis rows through the LDS
-// A wave's whole share of a projection (the 8 tile rows of its 128 x 128 block, 2 K KiB) is requested in one burst of
-// global-to-LDS loads before it does anything else with the block: the loads need no registers, all of them are in
-// flight while the wave rotates its input and decodes the first rows, and the decode loop stays rolled.  The loads are
-// written as inline assembly on purpose: the compiler then keeps no count of them, so it does not hold back the first LDS
-// read until every one of them has landed; exl3_rows_wait is the only thing that orders them.  Consequences for the
-// caller: every ordinary global load whose value is still needed must have been consumed before exl3_rows_issue (a load
-// the compiler waits for later would wait for the whole burst), and a wave must pass exl3_rows_wait<K>(7) before it ends.
-// LDS layout of a tile row: decode lane L's K words start at word L * stride; K = 3 and 4 use the 16-byte lane pitch of
-// the wide loads, the others are packed.  A wave's buffer is a ring of D rows (8, or fewer where more waves must fit a CU).  Rows are requested in units: one row by
-// one load (K = 3, 4), two rows by one load (K = 2: a 512-byte row is half a load), one row by K one-word loads (the rest).
-template <int K, int D = 8, bool H = false>
-struct Exl3Rows {
-    static_assert(D == 4 || D == 6 || D == 8, "ring depths in use");
-    static constexpr int depth = D;                              // rows of the ring
-    static constexpr int stride = (K == 3 || K == 4) ? 4 : K;
-    static constexpr int src_words = 8 * EXL3_TILE_WORDS(K, H);  // words of a tile row of the block in memory
-    // a half rate's row is copied as it lies, 64 words a load, the last load partly: 96, 160, 224 words in 128, 192, 256
-    static constexpr int unit_rows = (!H && K == 2) ? 2 : 1;
-    static constexpr int unit_loads = H ? (src_words + 63) / 64 : (K == 2 || K == 3 || K == 4) ? 1 : K;
-    static constexpr int row_words = H ? 64 * unit_loads : 64 * stride;
-    static constexpr int words = D * row_words;
-    static constexpr int loads = D / unit_rows * unit_loads;   // of a full ring
-    // loads that may still be in flight once the row t places behind the oldest requested one has landed
-    static constexpr int after(int t) { return t >= D - 1 ? 0 : (D - 1 - t) / unit_rows * unit_loads; }
-};
-
-// Requests the unit that starts at row r (a multiple of unit_rows) of the wave's row stream into its ring slot r % D.
-// row0 = the stream's first tile row (of the wave's 128-column block), pitch = words between tile rows, lds = the ring.
-template <int K, int D = 8, bool H = false>
-__device__ __forceinline__ void exl3_unit_issue(const u32* __restrict__ row0, u64 pitch, u32 r, u32 lane, u32 lds) {
-    const u32 slot = r % D;
-    if constexpr (H) {
-        typedef Exl3Rows<K, D, H> R;
-#pragma unroll
-        for (int d = 0; d < R::unit_loads; d++)   // at least 32 lanes of every load are active: the wave always issues it
-            if (d * 64 + lane < (u32) R::src_words) lds_load<4>(row0 + r * pitch + d * 64 + lane, lds + slot * 4 * R::row_words + d * 256);
-    } else if constexpr (K == 4 || K == 3) {
-        lds_load<4 * K>(row0 + r * pitch + lane * K, lds + slot * 1024);
-    } else if constexpr (K == 2) {
-        lds_load<16>(row0 + (r + (lane >> 5)) * pitch + (lane & 31) * 4, lds + slot * 512);   // lanes 0..31 row r, 32..63 row r + 1
-    } else {
-#pragma unroll
-        for (int d = 0; d < K; d++) lds_load<4>(row0 + r * pitch + d * 64 + lane, lds + slot * 256 * K + d * 256);
-    }
-}
-
-// The first D rows of a stream (every stream is a whole number of 8-row blocks).
-template <int K, int D = 8, bool H = false>
-__device__ __forceinline__ void exl3_rows_issue(const u32* __restrict__ row0, u64 pitch, u32 lane, u32 lds) {
-#pragma unroll
-    for (int r = 0; r < D; r += Exl3Rows<K, D, H>::unit_rows) exl3_unit_issue<K, D, H>(row0, pitch, r, lane, lds);
-}
-
-// Returns once the row t places behind the oldest request in flight has landed (with everything requested before it).
-template <int K, int D = 8, bool H = false>
-__device__ __forceinline__ void exl3_rows_wait(u32 t) {
-    switch (t) {
-        case 0: wait_vm<Exl3Rows<K, D, H>::after(0)>(); break;
-        case 1: wait_vm<Exl3Rows<K, D, H>::after(1)>(); break;
-        case 2: wait_vm<Exl3Rows<K, D, H>::after(2)>(); break;
-        case 3: wait_vm<Exl3Rows<K, D, H>::after(3)>(); break;
-        case 4: wait_vm<Exl3Rows<K, D, H>::after(4)>(); break;
-        case 5: wait_vm<Exl3Rows<K, D, H>::after(5)>(); break;
-        case 6: wait_vm<Exl3Rows<K, D, H>::after(6)>(); break;
-        default: wait_vm<0>(); break;
-    }
-}
-
 // ------------------------------------------------------------------------------------------- the verify layer
 // Resident EXL3 layers for a verify batch (m <= 8 rows): a plan, gate and up, down, the rank-order sum, each launch for one
 // layer (sz_moe_layer_verify, sz_moe_block_verify) or for all layers of one type of a round at once (sz_verify_round is
