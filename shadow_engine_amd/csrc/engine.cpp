@@ -1332,8 +1332,9 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         }
         const uint32_t tok = 16 * most, ntl = std::min<uint32_t>(most, (tokens + 15) / 16), nt = ntl <= 2 ? ntl : ntl + ntl % 2, nd = std::min(4u, nt);
         const uint64_t max_items = some + rows / tok, max_down = some + rows / (16 * nd), tiles = rows / 16 + c.n_expert + 2;
+        // (room for items of one tile whatever their length: a chunk never takes more than a longer one)
         const uint32_t bound = (uint32_t) ((max_items + 7) / 8 * 8), bound_d = (uint32_t) ((max_down + 7) / 8 * 8);   // workgroups an item's part (xpf_place)
-        if (pb.lay({{&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4}, {&pb.items, (2 + 2 * max_items + 2 * max_down) * 4},
+        if (pb.lay({{&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4}, {&pb.items, (2 + 4 * (some + rows / 16)) * 4},
                     {&pb.eo, rows * c.hidden * 4}, {&pb.most, T * 8}, {&pb.arows, tiles * 2 * kbs * 4096}, {&pb.ainv, tiles * 2 * 64}, {&pb.drows, tiles * fbs * 4096}, {&pb.dinv, tiles * fbs * 64}}))
             return 1;
         const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0, items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
