@@ -1339,8 +1339,10 @@ EXL3_HEAD_ENTRIES(8)
 // (measured: of its 16 cycles a SIMD issues nothing else for 9, whichever wave it comes from), so few, large items; then the ends of a
 // workgroup, a third of launch 2's time.  4096 tokens through 512 experts of 2048 x 512 and the shared one at 4 bits, top-10: 130 + 385 +
 // 265 us, 568 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
-// and 738 MB of partial sums in between, took 674 + 213 + 285.  The chunk on inputs that are not in a cache: 1290 -> 920 us, of 45 tokens at
-// 3 bits 121 -> 120 (there the launches' latencies and the weights' first trip count).
+// and 738 MB of partial sums in between, took 674 + 213 + 285.  The chunk on inputs that are not in a cache: 1290 -> 914 us.
+// Of few items launch 2 is as long as the longest item's chain over all inputs, and the chip is not full: the host makes items shorter, down
+// to one tile, splits launch 1 and 3 over the 128-blocks, and lets two workgroups share a compute unit (45 tokens at 3 bits 121 -> 101 us,
+// 250 tokens through 32 experts of 3072 x 256, top-3, at 2 bits 104 -> 88 and 159 with items of 128).
 // Tried: launch 2 by waves of 128 columns for 64 tokens (460 us), its matrix instructions placed among the decode (no change), its two
 // waves of a SIMD half a unit apart (2 %), an expert's items on one XCD (less traffic, same time); launch 3 in launch 2's form (272 to 312).
 
