@@ -1307,26 +1307,25 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         if (c.ff > 512) return fail("sz_moe_prefill_chunk: EXL3 experts of more than 512 intermediate features are not built (a workgroup keeps four 128-blocks of a token)");
         const uint32_t kbs = c.hidden / 128, fbs = c.ff / 128, widest = f.bits <= 5 ? 8 : 6;
         const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1;
-        // The gate and up launch: two 128-blocks of ff a workgroup of eight waves share the operand rows; one of four waves, whose rings are
-        // deeper, where the work is little or where eight waves would leave compute units without a workgroup (3 bits, 512 experts of
-        // 2048 x 512, top-10: 45 tokens 102 us with four waves and 123 with eight, 200 tokens 178 and 176, 512 254 and 252, 1024 371 and
-        // 344; 600 tokens through 60 of 1024 x 256, top-8: 105 and 119; 2048 through 64 of 2048 x 512, top-4: 254 and 243; 1500 through
-        // 32: 177 and 188).  By the bound on the items: how many experts the router reaches the host does not know.
-        const bool wide_gu = rows * fbs >= 16000 && (some + rows / (16 * widest)) * fbs >= 512;
-        // Of four waves, items so short that the chip is full: an item's chain over all inputs takes about 2.5 + its tiles, its workgroups a
-        // compute unit each, of a single tile half a unit (1.2 units' time for two of them).  Routers prefer some experts: 0.4 of those that
-        // independent choices would reach, the experts' last tiles and the rest of the pairs in whole items.  us with items of up to 128,
-        // 64, 32 and 16 pairs, router with Zipf's preferences and without: 45 tokens through 512 experts of 2048 x 512, top-10, and the
-        // shared one, 3 bits 115, 115, 127, 102 and 291, 291, 290, 215; 500 through 32 of 2048 x 512, top-2, 3 bits 113, 95, 83, 101 and 94,
-        // 90, 82, 101; 200 through 128 of 4096 x 512, top-8, and the shared one, 4 bits 216, 220, 226, 242 and 291, 288, 286, 242; 700
-        // through 64 of 3072 x 512, top-6, and the shared one, 4 bits 247, 252, 322, 356 and 253, 251, 298, 352.
-        const double reached = 0.4 * c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) T));
-        uint32_t most = widest;
+        // The gate and up launch: workgroups of four waves, two of which share a compute unit, with items of up to 64 pairs; for long chunks of
+        // eight waves, which take two 128-blocks of ff and items of up to 128 pairs: an expert is decoded less often, but a workgroup has a
+        // unit for itself (4096 tokens through 512 experts of 2048 x 512, top-10, and the shared one, 4 bits, four waves and eight, a
+        // router with Zipf's preferences: 941 and 915 us, without: 1110 and 1019; 3500 through 64 of 3072 x 512, top-6: 727 and 681;
+        // 2048 as the first 556 and 550, 601 and 669; 4000 through 256 of 3072 x 256, top-6, 2 bits 611 and 624).
+        const bool wide_gu = rows * fbs >= 95000;
+        // Of four waves, items so short that the chip is full: an item's chain over all inputs takes about 4 + its tiles; two workgroups that share
+        // a unit 1.6 times that.  Routers prefer some experts: 0.3 of those that independent choices would reach, the experts' last tiles
+        // and the rest of the pairs in whole items.  us with items of 16, 32 and 64 pairs, router with Zipf's preferences and without: 45 tokens
+        // as above at 3 bits 100, 112, 106 and 213, 240, 240; 200 tokens 179, 160, 140 and 354, 335, 347; 512 tokens 328, 260, 227 and
+        // 384, 395, 395; 200 through 128 of 4096 x 512, top-8, and the shared one, 4 bits 244, 196, 206 and 243, 244, 246; 300 through 160
+        // of 2560 x 256, top-6, 121, 105, 132 and 123, 127, 141; 500 through 32 of 2048 x 512, top-2, 3 bits 101, 82, 99.
+        const double reached = 0.3 * c.n_expert * (1.0 - std::pow(1.0 - (double) c.top_k / c.n_expert, (double) T));
+        uint32_t most = f.bits <= 5 ? 8 : 6;   // XPF_NT
         if (!wide_gu) {
             double best = 1e30;
-            for (uint32_t n : {widest, 4u, 2u, 1u}) {
-                const double chain = 2.5 + (double) std::min<uint64_t>(n, (T + 15) / 16), work = reached * 3.5 + (double) rows / (16 * n) * chain;
-                const double cost = n > 1 ? std::max(chain, 1.4 / 256 * fbs * work) : work * fbs <= 256 * chain ? chain : std::max(4.7, 0.83 / 256 * fbs * work);
+            for (uint32_t n : {4u, 2u, 1u}) {
+                const double chain = 4 + (double) std::min<uint64_t>(n, (T + 15) / 16), rest = (double) rows / (16 * n);
+                const double cost = (reached + rest) * fbs <= 256 ? chain : std::max(1.6 * chain, 0.95 / 256 * fbs * (reached * 5 + rest * chain));
                 if (cost < best) best = cost, most = n;
             }
         }
@@ -1362,7 +1361,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
             // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING, XPF_RING_N), afterwards the exchange of four tiles' sums
             uint32_t lds = ncb * 2 * std::min(4u, nt) * 8192;
             for (uint32_t n = 1; n <= nt; n += n == 1 ? 1 : 2) {
-                const uint32_t deep = n == 1 ? (bits <= 2 ? 8 : bits <= 5 ? 10 - bits : bits <= 7 ? 4 : 3) : n == 2 ? (bits <= 4 ? 8 : 12 - bits) : n == 4 ? (bits <= 5 ? 5 : 4) : wide_ring, ring = wide_gu ? wide_ring : deep;
+                const uint32_t ring = wide_gu ? wide_ring : std::min(8u, (40 - 2 * n) / (2 * n + bits));
                 lds = std::max(lds, (wide_gu ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
             }
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff), U32(tok)};

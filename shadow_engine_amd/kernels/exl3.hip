@@ -1340,19 +1340,21 @@ EXL3_HEAD_ENTRIES(8)
 // workgroup, a third of launch 2's time.  4096 tokens through 512 experts of 2048 x 512 and the shared one at 4 bits, top-10: 130 + 385 +
 // 265 us, 568 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
 // and 738 MB of partial sums in between, took 674 + 213 + 285.  The chunk on inputs that are not in a cache: 1290 -> 914 us.
-// Of few items launch 2 is as long as the longest item's chain over all inputs, and the chip is not full: the host makes items shorter, down
-// to one tile, splits launch 1 and 3 over the 128-blocks, and lets two workgroups share a compute unit (45 tokens at 3 bits 121 -> 101 us,
-// 250 tokens through 32 experts of 3072 x 256, top-3, at 2 bits 104 -> 88 and 159 with items of 128).
+// Of few items launch 2 is as long as the longest item's chain over all inputs, and the chip is not full: the host takes workgroups of four
+// waves, two a compute unit, and shorter items, down to one tile, and splits launch 1 and 3 over the 128-blocks (45 tokens at 3 bits 121 -> 100
+// us, 512 tokens 273 -> 227, 250 through 32 experts of 3072 x 256, top-3, at 2 bits 104 -> 93 and 159 with items of 128).
 // Tried: launch 2 by waves of 128 columns for 64 tokens (460 us), its matrix instructions placed among the decode (no change), its two
 // waves of a SIMD half a unit apart (2 %), an expert's items on one XCD (less traffic, same time); launch 3 in launch 2's form (272 to 312).
 
-// Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for.
+// Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for; in workgroups of four waves 4.
 #define XPF_NT(K) ((K) <= 5 ? 8 : 6)
-// Units of a wave's ring of trellis rows: what eight waves have room for, and in workgroups of four waves (few items, whose weights come
-// from memory rather than a cache: their trip is what the launch waits for) as deep as the operand rows of NT tiles leave room, of one tile
-// in half a compute unit's LDS: then two workgroups share a unit.
+#define XPF_NT_N 4
+// Units of a wave's ring of trellis rows: what eight waves have room for, and in workgroups of four waves as deep as leaves two of them room on a
+// compute unit, with the operand rows of NT tiles and no more than 8 (rings of 5 units for four tiles and one workgroup a unit: 200
+// tokens of 512 experts of 2048 x 512, top-10, 3 bits 160 us, with rings of 2 and two workgroups 140; with a router without preferences 432
+// and 347).
 #define XPF_RING(K) ((K) <= 7 ? 3 : 2)
-#define XPF_RING_N(K, NT) ((NT) == 1 ? ((K) <= 2 ? 8 : (K) <= 5 ? 10 - (K) : (K) <= 7 ? 4 : 3) : (NT) == 2 ? ((K) <= 4 ? 8 : 12 - (K)) : (NT) == 4 ? ((K) <= 5 ? 5 : 4) : XPF_RING(K))
+#define XPF_RING_N(K, NT) ((40 - 2 * (NT)) / (2 * (NT) + (K)) < 8 ? (40 - 2 * (NT)) / (2 * (NT) + (K)) : 8)   /* (D + 1) 4096 NT + 2048 K D bytes, at most 80 KiB */
 #define XPF_RING_DOWN_N(K) ((K) <= 3 ? 8 : (K) == 4 ? 7 : (K) == 5 ? 5 : (K) <= 7 ? 4 : 3)
 // What undoes the 1 / 128 that the stored values carry and applies the transform's 1 / sqrt(128)
 #define XPF_UNSCALE 11.3137085f
@@ -1820,7 +1822,7 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
     const u8* bg = (const u8*) (e < ne ? eaddr[e] : sh_addr[0]);
     const u8* bu = (const u8*) (e < ne ? eaddr[(u64) ne + e] : sh_addr[1]);
     const u8* bd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
-    xpf_tiles<XPF_NT(K)>(it.tiles, [&](auto n) {
+    xpf_tiles<NCB == 2 ? XPF_NT(K) : XPF_NT_N>(it.tiles, [&](auto n) {
         constexpr int NT = decltype(n)::value, G = NT < 4 ? NT : 4;
         typedef VerifyRing<K, false, 4, NCB == 2 ? XPF_RING(K) : XPF_RING_N(K, NT)> R;
         constexpr int NB = NCB == 2 ? 3 : R::D + 1;

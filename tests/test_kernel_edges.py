@@ -431,7 +431,7 @@ def test_a_gguf_layers_bits_do_not_depend_on_the_batch(gpu, ty, hidden, ff, ne, 
 
 
 @pytest.mark.parametrize("kb,tokens,hidden,ff", [(1, 129, 256, 256), (2, 40, 1024, 512), (4, 300, 256, 512), (5, 140, 512, 512), (6, 210, 256, 256), (7, 97, 256, 512),
-                                                 (8, 260, 256, 512)] + [(kb, 5500, 256, 512) for kb in range(1, 9)])
+                                                 (8, 260, 256, 512)] + [(kb, 8000, 256, 512) for kb in range(1, 9)])
 def test_exl3_prefill_items_of_every_size(gpu, kb, tokens, hidden, ff):  # noqa: F811
     """Experts with few and many tokens (items of one tile to the most, the wide and the narrow form of the gate and up launch, the
     shortest streams) at every bit rate, a token of zeros, one of very large inputs, one whose products pass f32's range, and an
@@ -536,12 +536,12 @@ def test_exl3_prefill_large_inputs_that_an_expert_scales_to_nothing(gpu, kb, tok
 
 
 @pytest.mark.parametrize("kb,hidden,ff,ne,k,shared,chunks", [
-    (3, 1280, 512, 32, 2, False, (1400, 500, 60, 17)),        # items of up to 128 pairs, 32, 16; ten 128-blocks of hidden
-    (2, 512, 256, 60, 8, False, (1300, 900, 100)),            # 128, 64, 16
+    (3, 1280, 512, 32, 2, False, (1400, 500, 60, 17)),        # items of up to 64 pairs, 32, 16; ten 128-blocks of hidden
+    (2, 512, 256, 60, 8, False, (1300, 700, 100)),            # the same
     (4, 4096, 512, 16, 2, False, (260, 120, 20)),             # 32 blocks: shares of the rotation and of the down products
     (1, 256, 256, 40, 3, True, (1030, 200, 33, 1)),           # two blocks
-    (2, 512, 512, 300, 8, False, (560, 130, 48)),             # two launches of eight waves, then four
-    (5, 1024, 512, 140, 8, True, (500, 90)), (7, 1024, 512, 140, 8, True, (500, 90)),
+    (2, 512, 512, 300, 8, False, (3000, 560, 130, 48)),       # both launches of eight waves, then of four
+    (5, 512, 512, 140, 8, True, (2700, 500, 90)), (7, 512, 512, 140, 8, True, (2700, 500, 90)), (4, 256, 512, 16, 10, True, (2400, 250, 40)),
     (6, 768, 256, 32, 6, True, (400, 40)), (8, 768, 512, 32, 6, False, (400, 40))])
 def test_exl3_prefill_bits_do_not_depend_on_the_chunk(gpu, kb, hidden, ff, ne, k, shared, chunks):  # noqa: F811
     """The first tokens of a chunk in chunks of their own, through the other forms and item lengths: the same bits, within the chunk's

@@ -92,7 +92,7 @@ template <int K, int NT, int NB, int NW, int D> static void stream(const char* n
 template <int K, int NT> static void both() {
     if constexpr (NT <= XPF_NT(K)) {
         stream<K, NT, 3, 4, XPF_RING(K)>("eight waves");
-        stream<K, NT, XPF_RING_N(K, NT) + 1, 2, XPF_RING_N(K, NT)>("four waves");
+        if constexpr (NT <= XPF_NT_N) stream<K, NT, XPF_RING_N(K, NT) + 1, 2, XPF_RING_N(K, NT)>("four waves");
     }
 }
 template <int K> static void rate() { both<K, 1>(); both<K, 2>(); both<K, 4>(); both<K, 6>(); both<K, 8>(); }
@@ -104,7 +104,7 @@ def test_prefill_streams_stay_inside_their_item_and_wait_for_what_they_read(tmp_
     """Every bit rate, number of token tiles and shape of the gate and up launch, from the shortest stream (hidden = 256: shorter than the
     ring of four waves) on: no request past the stream's end, no slot filled before it was read, no read before it has landed."""
     src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
-    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_RING", "XPF_RING_N", "XPF_HALF_U16"))
+    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_N", "XPF_HALF_U16"))
     start = src.index("template <int K, int NT, int NB, int NW, class R>")
     stream = src[start:src.index("\n}\n", start) + 3]
     path = tmp_path / "stream.cpp"
