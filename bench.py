@@ -274,8 +274,10 @@ def exl3_prefill(torch, sz, synth, synth_device, stream, tokens=512, bits=3):
     w.step_bytes = distinct * (gu + dn) + tokens * (2 * HIDDEN + NE) * 4
     # rotate: the rows of x in, f16 operand rows of every pair for gate and up out; gate/up: the experts' two matrices and those
     # rows in, down's operand rows out; down: the experts' third matrix and its operand rows in, the pairs' rows of the result out
-    w.kernel_bytes = {"prefill_rotate_exl3": tokens * HIDDEN * 4 + pairs * 2 * HIDDEN * 2, "prefill_gate_up_exl3_%d" % bits: distinct * gu + pairs * (2 * HIDDEN + FF) * 2,
-                      "prefill_down_exl3_%d" % bits: distinct * dn + pairs * FF * 2 + pairs * HIDDEN * 4}
+    w.kernel_bytes = {"prefill_rotate_exl3": tokens * HIDDEN * 4 + pairs * 2 * HIDDEN * 2}
+    for form in ("", "n_"):   # workgroups of eight waves, of four
+        w.kernel_bytes["prefill_gate_up_%sexl3_%d" % (form, bits)] = distinct * gu + pairs * (2 * HIDDEN + FF) * 2
+        w.kernel_bytes["prefill_down_%sexl3_%d" % (form, bits)] = distinct * dn + pairs * FF * 2 + pairs * HIDDEN * 4
     w.dtype = "f32 accumulate over EXL3 f16 codebook weights x f16 activations (matrix cores)"
     w.describe = {"workload": "prefill chunk, %d tokens x hidden 2048 through 512 EXL3 K=%d experts + the shared one (top-10, Zipf-skewed routing, "
                               "%d distinct experts hit), f16 activations" % (tokens, bits, distinct), "rows": tokens, "resident_GB": round(buf.numel() / 1e9, 2)}
