@@ -1355,6 +1355,7 @@ EXL3_HEAD_ENTRIES(8)
 // and 347).
 #define XPF_RING(K) ((K) <= 7 ? 3 : 2)
 #define XPF_RING_N(K, NT) ((40 - 2 * (NT)) / (2 * (NT) + (K)) < 8 ? (40 - 2 * (NT)) / (2 * (NT) + (K)) : 8)   /* (D + 1) 4096 NT + 2048 K D bytes, at most 80 KiB */
+// Launch 3's, of four waves: as deep as leaves two workgroups room with the rows of one tile.
 #define XPF_RING_DOWN_N(K) ((K) <= 3 ? 8 : (K) == 4 ? 7 : (K) == 5 ? 5 : (K) <= 7 ? 4 : 3)
 // What undoes the 1 / 128 that the stored values carry and applies the transform's 1 / sqrt(128)
 #define XPF_UNSCALE 11.3137085f
