@@ -387,7 +387,7 @@ struct sz_session {
             uint64_t ptr = 0;
         };
         DevBuf mem;
-        Part xq, xd, tidx, w, cnt, offs, list, items, hq, hd, eo, most, arows, ainv, drows, dinv;
+        Part xq, xd, xh, tidx, w, cnt, offs, list, items, hq, hh, hd, eo, most, arows, ainv, drows, dinv;
         int lay(std::initializer_list<std::pair<Part*, uint64_t>> parts) {
             uint64_t n = 0;
             for (const auto& p : parts) n += (p.second + 255) & ~255ull;
@@ -1383,34 +1383,35 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden), U32(c.top_k)};
         return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, tokens, 1, 256, 0, stream, a);
     }
-    const uint64_t max_items = c.n_expert + 1 + rows / 64, max_items_d = c.n_expert + 1 + rows / 32;   // every expert's runs of up to 64 (32) pairs: PF_TOK, PF_TOK_D in kernels/prefill.hip
+    const uint64_t max_items = c.n_expert + 1 + rows / 64;   // every expert's runs of up to 64 pairs: PF_TOK in kernels/prefill.hip
     if (pb.lay({{&pb.xq, T * c.hidden}, {&pb.xd, T * c.hidden / 32 * 4}, {&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4},
-                {&pb.items, (2 + 2 * max_items + 2 * max_items_d) * 4}, {&pb.hq, rows * c.ff}, {&pb.hd, rows * (c.ff / 32) * 4}, {&pb.eo, rows * c.hidden * 4}}))
+                {&pb.items, (2 + 4 * max_items) * 4}, {&pb.hq, rows * c.ff}, {&pb.xh, T * c.hidden * 2}, {&pb.hh, rows * c.ff * 2}, {&pb.hd, rows * (c.ff / 32) * 4}, {&pb.eo, rows * c.hidden * 4}}))
         return 1;
     const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0;
     {
         // routing and quantization do not depend on each other: one launch
         const uint64_t n = T * c.hidden;
-        const sz_arg a[] = {P(x), U64(n), P(pb.xq.ptr), P(pb.xd.ptr), P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
+        const sz_arg a[] = {P(x), U64(n), P(pb.xq.ptr), P(pb.xd.ptr), P(pb.xh.ptr), P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
         if (launch("prefill_front", (tokens + 3) / 4 + (uint32_t) ((n / 32 + 255) / 256), 1, 1, 256, 0, stream, a)) return 1;
     }
-    const uint64_t items_d = pb.items.ptr + (1 + 2 * max_items) * 4;   // the down kernel's items: runs of up to 32 pairs (PF_TOK_D)
+    const uint64_t items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
     {
-        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(items_d), U32(64), U32(32)};
+        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(items_d), U32(64), U32(64)};
         if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
     }
     {
-        const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.xq.ptr), P(pb.xd.ptr), P(pb.hq.ptr), P(pb.hd.ptr),
+        const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.xh.ptr), P(pb.xd.ptr), P(pb.hq.ptr), P(pb.hh.ptr), P(pb.hd.ptr),
                             U32(c.n_expert), U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(c.ff)};
-        static const bool w4 = std::getenv("SHADOWZERO_PREFILL_FOUR_WAVES") != nullptr;   // the four-wave form, for comparisons
-        if (launch(w4 ? "prefill_gate_up_iq3_s_w4" : "prefill_gate_up_iq3_s", c.ff / 64, (uint32_t) max_items, 1, w4 ? 256 : 512, 0, stream, a)) return 1;
+        if (launch("prefill_gate_up_iq3_s", c.ff / 64, (uint32_t) max_items, 1, 512, 0, stream, a)) return 1;
     }
     {
-        // a workgroup takes 4 (else 2, else 1) blocks of 64 rows in turn: the two chunks of one block are too little work for its set-up
-        const uint32_t blocks = c.hidden / 64, per = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1;
-        const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(items_d), P(pb.hq.ptr), P(pb.hd.ptr), P(pb.eo.ptr), U32(c.n_expert),
+        // 128 rows a workgroup; in long chunks, which fill the chip many times over, four lots in turn, whose set-up counts once (1, 2 and 4 lots:
+        // 4096 tokens through 512 experts of 2048 x 512, top-10, and the shared one 861, 851, 847 us; 512 tokens 174, 174, 178, 150 through
+        // 128 of 2560 x 768, top-8, 120, 125, 128, 40 through 64 of 1024 x 256, top-4, 30, 33, 38)
+        const uint32_t blocks = c.hidden / 128, per = rows >= 20000 && blocks % 4 == 0 ? 4 : 1;
+        const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.hh.ptr), P(pb.hd.ptr), P(pb.eo.ptr), U32(c.n_expert),
                             U32(c.hidden), U32(c.ff)};
-        if (launch("prefill_down_iq3_s", blocks / per, (uint32_t) max_items_d, 1, 256, 0, stream, a)) return 1;
+        if (launch("prefill_down_iq3_s", blocks / per, (uint32_t) max_items, 1, 512, 0, stream, a)) return 1;
     }
     const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden), U32(c.top_k)};
     return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, tokens, 1, 256, 0, stream, a);

@@ -1,27 +1,38 @@
-// The prefill chunk of one MoE layer on int8 activations: tokens grouped by expert, IQ3_S weights decoded to signed int8
-// in registers, int8 MFMA tiles (v_mfma_i32_16x16x32_i8: 16 tokens x 16 weight rows x one 32-weight sub-block), exact int32
-// sub-block dots scaled by (weight scale x activation scale) in f32, SwiGLU, H re-quantized per 32, down into pair rows.
+// The prefill chunk of one MoE layer on int8 activations: tokens grouped by expert, IQ3_S weights decoded to whole numbers in f16, f16 MFMA
+// tiles (v_mfma_f32_16x16x32_f16: 16 weight rows x 16 tokens x one 32-weight sub-block), a sub-block's exact sums scaled by the
+// activations' scale in f32, SwiGLU, H re-quantized per 32, down into pair rows.
 //
 // Arithmetic follows the reference's CPU statement of the int8-activation expert (crates/shadowzero-model/src/cpu_expert.rs:99-110,
 // 144-155, 217, 298-339 and cpu_expert_avx512.rs:25-42) with activation blocks of 32: d_x = amax / 127,
-// q = clamp(round-half-away(v / d_x)); weights grid * sign as int8 with s_w = d (1 + 2 scale) per 32; a row's product is
-// the sum over sub-blocks, in order, of (s_w * d_x) * (float) (int32 dot) in f32, each added with one fused multiply-add
-// (the CPU statement rounds the product first: a last-bit difference now and then).  The launch structure is the
-// native fused path's (native/fused/shadowzero_fused.cu:5-9: quantize, group, experts), re-made for wave64 MFMA.
+// q = clamp(round-half-away(v / d_x)); weights grid * sign with s_w = d (1 + 2 scale) per 32.  Codes (up to 127) and
+// grid * sign * (1 + 2 scale) (up to 465) are whole numbers, exact in f16, and 32 products of theirs stay below 2^24: the matrix
+// instruction's f32 sum of a sub-block is exact.  A row's product is, per 256 weights, d times the sum over the sub-blocks of
+// d_x * sum, both steps fused multiply-adds in f32 (the CPU statement adds (s_w * d_x) * sum sub-block by sub-block: other
+// roundings of the last bits).  Codes are multiplied by 2^-6 and weights by 2^-14, exactly, and d by 2^20: sums of the largest finite
+// activations then stay finite until d is in.  The launch structure is the native fused path's (native/fused/shadowzero_fused.cu:5-9: quantize,
+// group, experts), re-made for wave64 MFMA.
 //
-// MFMA operand layout (16x16x32 i8): A (tokens x k) lane l holds row l % 16, k = 8 (l / 16) .. +8 as 8 bytes; B (k x rows)
-// lane l holds column l % 16, the same k; C lane l holds column l % 16, rows 4 (l / 16) + r in acc[r].
+// Why f16 and not the int8 instruction: int8 weights leave the scale 1 + 2 s out, and every sum then takes a conversion, a product of
+// scales and a multiply-add, 12 vector instructions a tile and sub-block where this form takes 4 (and a matrix instruction of
+// the same length).
+//
+// MFMA operand layout: A (weight rows x k) lane l holds row l % 16, k = 8 (l / 16) .. +8; B (k x tokens) lane l holds token l % 16, the
+// same k; C lane l holds token l % 16, weight rows 4 (l / 16) + r in element r.
 
 //
 // The ahead-of-time build has the matrix instructions write to ordinary vector registers: every tile's 4 sums a lane are
-// converted and scaled at once, and out of the accumulation registers each would first cost a move (8 of 40 vector
-// instructions a tile pair).
+// scaled at once, and out of the accumulation registers each would first cost a move.
 // hipcc: -mllvm -amdgpu-mfma-vgpr-form=1
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// q[i] = clamp(round(x[i] / d)), d[b] = amax / 127 over each 32 values (cpu_expert_avx512.rs:25-42).  One thread a block of 32.
-__device__ __forceinline__ void quant_block_q8(const float* x, u64 b, i8* q, float* d) {
+__device__ __forceinline__ u32 f16_pair(float a, float b) { return __builtin_bit_cast(u32, f16x2{(_Float16) a, (_Float16) b}); }
+
+// q[i] = clamp(round(x[i] / d)), d[b] = amax / 127 over each 32 values (cpu_expert_avx512.rs:25-42); h (where not null): the codes
+// again, times 2^-6, as f16.  One thread a block of 32.
+__device__ __forceinline__ void quant_block_q8(const float* x, u64 b, i8* q, float* d, u16* h) {
     const f32x4* p = (const f32x4*) (x + b * 32);
     float v[32];
 #pragma unroll
@@ -39,38 +50,45 @@ __device__ __forceinline__ void quant_block_q8(const float* x, u64 b, i8* q, flo
     const float id = dd > 0.0f ? 1.0f / dd : 0.0f;
     u32 w[8];
 #pragma unroll
+    for (int i = 0; i < 32; i++) v[i] = fminf(127.0f, fmaxf(-127.0f, roundf(v[i] * id)));
+#pragma unroll
     for (int i = 0; i < 8; i++) {
         u32 pack = 0;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float r = fminf(127.0f, fmaxf(-127.0f, roundf(v[4 * i + k] * id)));
-            pack |= ((u32) (int) r & 0xffu) << (8 * k);
-        }
+        for (int k = 0; k < 4; k++) pack |= ((u32) (int) v[4 * i + k] & 0xffu) << (8 * k);
         w[i] = pack;
     }
     u32x4* o = (u32x4*) (q + b * 32);
     o[0] = u32x4{w[0], w[1], w[2], w[3]};
     o[1] = u32x4{w[4], w[5], w[6], w[7]};
+    if (h) {
+        u32x4* oh = (u32x4*) (h + b * 32);
+#pragma unroll
+        for (int i = 0; i < 32; i++) v[i] *= 0x1p-6f;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            oh[i] = u32x4{f16_pair(v[8 * i], v[8 * i + 1]), f16_pair(v[8 * i + 2], v[8 * i + 3]), f16_pair(v[8 * i + 4], v[8 * i + 5]), f16_pair(v[8 * i + 6], v[8 * i + 7])};
+    }
     d[b] = dd;
 }
 
 // grid = ceil(n / 32 / 256), block 256.
 extern "C" __global__ void __launch_bounds__(256) quant_act_q8(const float* x, u64 n, i8* q, float* d) {
     const u64 b = (u64) blockIdx.x * 256 + threadIdx.x;
-    if (b < n / 32) quant_block_q8(x, b, q, d);
+    if (b < n / 32) quant_block_q8(x, b, q, d, nullptr);
 }
 
 // The two things a chunk needs before its tokens can be grouped, in one launch (they do not depend on each other): the
 // routing of its m tokens (workgroups [0, ceil(m / 4)): a wave a token, as route_topk_rows) and the quantization of its
 // activations (the workgroups after them, as quant_act_q8).  grid = ceil(m / 4) + ceil(n / 32 / 256), block 256.
-extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, u64 n, i8* q, float* d, const float* logits, u32* tidx, float* weights, u32* cnt,
+extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, u64 n, i8* q, float* d, u16* h, const float* logits, u32* tidx, float* weights, u32* cnt,
                                                                 u32 ne, u32 k, u32 m) {
     __shared__ double exs[4][512];
     __shared__ u32 tops[4][16];
     const u32 nr = (m + 3) / 4;
     if (blockIdx.x >= nr) {
         const u64 b = (u64) (blockIdx.x - nr) * 256 + threadIdx.x;
-        if (b < n / 32) quant_block_q8(x, b, q, d);
+        if (b < n / 32) quant_block_q8(x, b, q, d, h);
         return;
     }
     const u32 lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -90,7 +108,6 @@ extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, 
 
 #define PF_TOK 64      // tokens of one work item: PF_TOK / 16 MFMA tiles of 16
 #define PF_TILES (PF_TOK / 16)
-#define PF_TOK_D 32    // tokens of one work item of the down kernel: with half the activations in LDS twice the workgroups fit a CU
 
 // Groups the chunk's (token, rank) pairs by expert: offs[e] .. offs[e + 1] are the positions in list[] of expert e's pairs
 // (pair = token * k + rank; the shared expert, index ne, takes the pairs npairs + token when nshared = tokens).  The order of an expert's pairs in list[] is
@@ -204,360 +221,372 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
     for (u32 j = tid; j < nshared; j += 1024) list[s_off[ne] + j] = npairs + j;
 }
 
-__shared__ u32 pf_grid[512];
-__shared__ u64 pf_sign[256];   // a sign byte as eight byte masks: 0xff where the bit is set
+__shared__ u32x2 pf_grid[512];   // the codebook grid, a weight's magnitude as f16
 
-// Fills the two tables; every thread of the workgroup (256) calls it, and a barrier must follow before they are read.
+// Fills the table; every thread of the workgroup (512) calls it, and a barrier must follow before it is read.
 __device__ __forceinline__ void pf_tables(u32 tid) {
-    for (u32 i = tid; i < 512; i += 256) pf_grid[i] = IQ3S_GRID[i];
-    u64 m = 0;
-#pragma unroll
-    for (int b = 0; b < 8; b++) m |= ((tid >> b) & 1u) ? (0xffull << (8 * b)) : 0ull;
-    pf_sign[tid] = m;
+    const u32 g = IQ3S_GRID[tid];
+    pf_grid[tid] = u32x2{f16_pair((float) (g & 0xff), (float) ((g >> 8) & 0xff)), f16_pair((float) ((g >> 16) & 0xff), (float) (g >> 24))};
 }
 
-// Eight consecutive weights (k = 8 kq .. 8 kq + 7 of sub-block g) of one IQ3_S block at `blk` (LDS, 2-byte aligned) as
-// signed int8 (cpu_expert.rs:99-110).
-__device__ __forceinline__ u64 iq3s_int8x8(const u8* blk, u32 g, u32 kq) {
-    const u32 j = 8 * g + 2 * kq;                       // index of the first of the two 4-weight groups
-    const u32 qs = *(const u16*) (blk + 2 + j);
-    const u32 qh = blk[66 + g] >> (2 * kq);
+// Eight consecutive weights (k = 8 kq .. 8 kq + 7 of sub-block g) of one IQ3_S block at `blk` (LDS, 2-byte aligned) as f16: grid * sign
+// (cpu_expert.rs:99-110) * (1 + 2 scale), `scale` holding the last factor twice; qh: bits 0 and 1 the ninth bits of the two grid indexes.  The two
+// signs of a pair are moved to the sign bits of its halves by one multiplication (the two copies of the sign byte that it
+// makes do not overlap).
+__device__ __forceinline__ f16x8 iq3s_f16x8(const u8* blk, u32 g, u32 kq, u32 qh, f16x2 scale) {
+    const u32 qs = *(const u16*) (blk + 2 + 8 * g + 2 * kq);   // the low bytes of the two 4-weight groups' grid indexes
     const u32 signs = blk[74 + 4 * g + kq];
-    const u32 g0 = pf_grid[(qs & 0xff) | ((qh & 1u) << 8)], g1 = pf_grid[(qs >> 8) | ((qh & 2u) << 7)];
-    // negate the bytes whose sign bit is set: (m ^ mask) + (mask & 1) per byte, magnitudes are at most 15 so nothing carries
-    const u64 mask = pf_sign[signs];
-    const u32 m0 = (u32) mask, m1 = (u32) (mask >> 32);
-    const u32 w0 = (g0 ^ m0) + (m0 & 0x01010101u), w1 = (g1 ^ m1) + (m1 & 0x01010101u);
-    return ((u64) w1 << 32) | w0;
+    u32 at0 = (qs & 0xff) << 3 | ((qh << 11) & 0x800u), at1 = (qs >> 8) << 3 | ((qh << 10) & 0x800u);
+    asm("" : "+v"(at0), "+v"(at1));   // bytes into the table, whose own address then is the loads' constant offset
+    const u32x2 g0 = *(const u32x2*) ((const u8*) pf_grid + at0), g1 = *(const u32x2*) ((const u8*) pf_grid + at1);
+    auto pair = [&](u32 grid, u32 spread) {
+        return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, grid) * __builtin_bit_cast(f16x2, ((signs * spread) & 0x80008000u) ^ __builtin_bit_cast(u32, scale)));
+    };
+    return __builtin_bit_cast(f16x8, u32x4{pair(g0.x, 0x40008000u), pair(g0.y, 0x10002000u), pair(g1.x, 0x04000800u), pair(g1.y, 0x01000200u)});
 }
 
-// The sub-block scales d (1 + 2 s) of a block: the four lanes that share a row (kq = 0..3) would each work out all eight;
-// instead lane (n, kq) works out the two of the byte it is handed (sub-blocks 2 kq and 2 kq + 1) and leaves them in the wave's
-// own strip sw[8][16] (LDS), where the products read them back (a quarter of the arithmetic, conflict-free reads).
-// A wavefront fence must follow before the strip is read.
-__device__ __forceinline__ void iq3s_scales_to_strip(const u8* blk, u32 n, u32 kq, float* sw) {
-    const float d = f16_to_f32(*(const u16*) blk);
-    const u32 sc = blk[106 + kq];
-    sw[(2 * kq) * 16 + n] = d * (float) (1 + 2 * (sc & 0x0f));
-    sw[(2 * kq + 1) * 16 + n] = d * (float) (1 + 2 * (sc >> 4));
+// (1 + 2 s) 2^-14 twice, s the four bits from `bit` on.
+__device__ __forceinline__ f16x2 iq3s_scale_pair(u32 sc, u32 bit) {
+    const f16x2 v = __builtin_bit_cast(f16x2, __builtin_amdgcn_ubfe(sc, bit, 4) * 0x20002u + 0x2c012c01u);   // 2^-4 + (1 + 2 s) 2^-14
+    return v - f16x2{(_Float16) 0x1p-4f, (_Float16) 0x1p-4f};
 }
 
-#define PF_KC 256      // k of one staged chunk: one IQ3_S block a row
-#define PF_AB(TOK) ((TOK) * 256)   // a chunk's activations in LDS: [tokens][16 columns of 16 bytes], column c of token t at slot c ^ (t & 15)
-#define PF_DB(TOK) ((TOK) * 32)    // a chunk's activation scales in LDS: [8 sub-blocks][tokens]
-#define PF_WB 7168     // a chunk's 64 blocks of one matrix in LDS: 28 words a row
-#define PF_WS 112      // bytes between rows there
+#define PF_WB 7168             // 64 rows' blocks of one matrix in LDS: 28 words a row
+#define PF_WS 112              // bytes between rows there
 
-// A chunk is brought into LDS by global-to-LDS loads (no registers in between), every wave a quarter of them, one chunk
-// ahead of the products: while the matrix and vector units work on chunk c the loads of chunk c + 1 are in flight into the
-// other buffer.  A wave's load instruction fills 64 consecutive slots of LDS from 64 addresses of its choosing, so the
-// layout is made by choosing the addresses.
-
-// The int8 activations and their scales of TOK pairs (32 or 64) for k in [k0, k0 + 256).  Token t's 16-byte column c lands at
-// slot c ^ (t & 15) of its row: the 16 tokens of an MFMA tile then read the same column from 16 different bank groups.
-// `rows` (LDS): the row of q and d every pair reads; a pair past the item's end names row 0, whose products are dropped.
-template <int TOK, int NWV = 4>   // NWV: the waves that share the chunk's loads
-__device__ __forceinline__ void pf_issue_a(const i8* __restrict__ q, const float* __restrict__ d, const u32* rows, u32 cols, u32 k0, u32 lds_a,
-                                           u32 lds_d, u32 wave, u32 lane) {
-    static_assert((TOK / 8) % NWV == 0, "every wave the same number of load instructions");
-#pragma unroll
-    for (int it = 0; it < TOK / 4 / NWV; it++) {          // TOK / 4 instructions a chunk: 4 tokens each
-        const u32 j = wave * (TOK / 4 / NWV) + it, t = 4 * j + (lane >> 4), c = (lane & 15) ^ (t & 15);
-        lds_load<16>(q + (u64) rows[t] * cols + k0 + 16 * c, lds_a + j * 1024);
-    }
-#pragma unroll
-    for (int it = 0; it < TOK / 8 / NWV; it++) {          // TOK / 8 instructions: 64 of the 8 x TOK scales each
-        const u32 j = wave * (TOK / 8 / NWV) + it, i = j * 64 + lane, g = i / TOK, t = i % TOK;
-        lds_load<4>(d + (u64) rows[t] * (cols / 32) + k0 / 32 + g, lds_d + j * 256);
-    }
+__device__ __forceinline__ u64 uniform_u64(u64 v) {
+    return ((u64) (u32) __builtin_amdgcn_readfirstlane((u32) (v >> 32)) << 32) | (u32) __builtin_amdgcn_readfirstlane((u32) v);
+}
+// lds_load_at's 4-byte form
+__device__ __forceinline__ void pf_load4_at(u64 base, u32 off, u32 lds) {
+    u32 keep;
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %3\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(lds), "s"(base) : "memory");
 }
 
-// Block `c` (the 256 weights k in [256 c, 256 c + 256)) of 64 consecutive rows of a row-major IQ3_S matrix: 28 words a
-// row.  Blocks are only 2-byte aligned: a row's words start at the word that holds the block's first byte, and the block
-// begins pf_shift (0 or 2) bytes into its slot.  The words of a row never leave the matrix: its first block starts on a
-// word and its last one ends on one (a row is a multiple of 4 bytes, or rows come in even numbers).
-// w = the first of the 64 rows, rb = bytes a row.
-__device__ __forceinline__ u32 pf_shift(const u8* w, u32 rb, u32 c, u32 row) { return (u32) ((u64) (w + (u64) row * rb + c * 110) & 2); }
-template <int NWV = 4>
-__device__ __forceinline__ void pf_issue_w(const u8* __restrict__ w, u32 rb, u32 c, u32 lds_w, u32 wave, u32 lane) {
+// The same block (256 weights) of 64 consecutive rows of a row-major IQ3_S matrix: 28 words a row.  Blocks are only 2-byte
+// aligned: a row's words start at the word that holds the block's first byte, and the block begins pf_shift (0 or 2) bytes
+// into its slot.  The words of a row never leave the matrix: its first block starts on a word and its last one ends on one (a
+// row is a multiple of 4 bytes, or rows come in even numbers).  at = the first of the 64 rows' block, rb = bytes a row.
+__device__ __forceinline__ u32 pf_shift(u64 at, u32 rb, u32 row) { return ((u32) at + row * rb) & 2; }
+struct PfRows {
+    u32 off[4];   // the lane's word in the wave's load instructions, of 28: 64 rows x 28 words
+    static __device__ __forceinline__ u32 place(u32 it, u32 wave) { return it < 3 ? wave + 8 * it : 24 + (wave & 3); }
+    __device__ __forceinline__ void init(u32 rb, u32 wave, u32 lane) {
 #pragma unroll
-    for (int it = 0; it < (28 + NWV - 1) / NWV; it++) {   // 28 instructions a chunk and matrix: 64 rows x 28 words
-        const u32 j = NWV == 4 ? wave * 7 + it : wave + NWV * it;
-        if (j < 28) {                                     // (wave-uniform)
-            const u32 i = j * 64 + lane, row = i / 28, dw = i % 28;
-            const u8* a = w + (u64) row * rb + c * 110;
-            lds_load<4>(a - ((u64) a & 2) + 4 * dw, lds_w + j * 256);
+        for (u32 it = 0; it < 4; it++) {
+            const u32 i = place(it, wave) * 64 + lane;
+            off[it] = i / 28 * rb + i % 28 * 4;
         }
     }
+    // the wave's share of the instructions, 3 or 4 of 8 waves' 28; with `mirrored` 4 or 3: of two calls 7
+    template <bool mirrored>
+    __device__ __forceinline__ void issue(u64 at, u32 lds_w, u32 wave) const {
+#pragma unroll
+        for (u32 it = 0; it < 4; it++)
+            if (it < 3 || (mirrored ? wave >= 4 : wave < 4))   // (wave-uniform)
+                pf_load4_at(at & ~3ull, (off[it] + ((u32) at & 3)) & ~3u, lds_w + place(it, wave) * 256);
+    }
+};
+
+// Half a block's products (128 weights, 4 sub-blocks) with the first T token tiles: acc += d_x * a sub-block's exact sum, in sub-block order.
+// xs, ds: the half's activations and their scales ([sub-block][64 tokens]); blk: the lane's row's block in LDS.
+template <int T>
+__device__ __forceinline__ void pf_products(f32x4 (&acc)[T], const u8* xs, const float* ds, const u8* blk, u32 half, u32 n, u32 kq) {
+    f16x8 w[4];
+    const u32 qh = ((u32) *(const u16*) (blk + 66 + 4 * half) | (u32) *(const u16*) (blk + 68 + 4 * half) << 16) >> (2 * kq);
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = iq3s_f16x8(blk, 4 * half + j, kq, qh >> (8 * j), iq3s_scale_pair(blk[106 + 2 * half + j / 2], 4 * (j % 2)));
+    __builtin_amdgcn_sched_barrier(0);
+    // a step is a tile and sub-block: its operands are read a step ahead, its sums scaled while the next one's are made
+    auto read = [&](int step, f16x8& x, float& dx) {
+        const u32 a = step / 4, g = step % 4;
+        x = *(const f16x8*) (xs + (16 * a + n) * 256 + ((4 * g + kq) ^ n) * 16);
+        dx = ds[g * PF_TOK + 16 * a + n];
+    };
+    f16x8 x[2];
+    float dx[3];
+    f32x4 c[2];
+    read(0, x[0], dx[0]);
+#pragma unroll
+    for (int step = 0; step <= 4 * T; step++) {
+        if (step + 1 < 4 * T) read(step + 1, x[(step + 1) % 2], dx[(step + 1) % 3]);
+        if (step < 4 * T) c[step % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[step % 4], x[step % 2], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        if (step > 0) {
+            f32x4& sum = acc[(step - 1) / 4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[r] = __builtin_fmaf(dx[(step - 1) % 3], c[(step - 1) % 2][r], sum[r]);
+            asm volatile("" : "+v"(sum));   // here, and not where the sums are next used: the products' registers are needed
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
-// One staged chunk's products: for each of its 8 sub-blocks the lane's 8 weights of its row (gate and up, or down) against
-// the first T token tiles, every tile's exact int32 sums scaled and added in f32 (a fused multiply-add a sum, in sub-block
-// order).  aq, ad: the chunk's activations and their scales; bg, bu, bd: the lane's row's block in LDS.
-template <int V> struct pf_int { static constexpr int value = V; };
-
-// NG sub-blocks from G0 on (8 from 0: the whole block; 4 from 0 or 4: a wave's half where two waves share a row group).
-template <int T, int TOK, int NG = 8, int G0 = 0>
-__device__ __forceinline__ void pf_products_gu(float (&accg)[PF_TILES][4], float (&accu)[PF_TILES][4], const u8* aq, const float* ad, const u8* bg, const u8* bu,
-                                               u32 n, u32 kq, float* sw) {
-    constexpr u32 g0 = G0;
-    iq3s_scales_to_strip(bg, n, kq, sw);
-    iq3s_scales_to_strip(bu, n, kq, sw + 128);
+// A block is complete: total += 2^20 d * acc, d the f16 scale of the block of each of the lane's four rows, which the lanes of the rows hand over
+// through the wave's own strip of LDS (a wave's LDS operations are in order).
+template <int T>
+__device__ __forceinline__ void pf_fold(f32x4 (&total)[T], f32x4 (&acc)[T], const u8* blk, float* strip, u32 n, u32 kq) {
+    if (kq == 0) strip[n] = f16_to_f32(*(const u16*) blk) * 0x1p20f;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    const f32x4 d = *(const f32x4*) (strip + 4 * kq);
 #pragma unroll
-    for (u32 gg = 0; gg < NG; gg++) {
-        const u32 g = g0 + gg;
-        const float swg = sw[g * 16 + n], swu = sw[128 + g * 16 + n];
-        const u64 b_g = iq3s_int8x8(bg, g, kq), b_u = iq3s_int8x8(bu, g, kq);
-        const u32 col = ((2 * g + (kq >> 1)) ^ n) * 16 + 8 * (kq & 1);   // where this lane's 8 activations of a token lie in its row
+    for (int a = 0; a < T; a++) {
 #pragma unroll
-        for (int a = 0; a < T; a++) {
-            const u64 av = *(const u64*) (aq + (16 * a + n) * 256 + col);
-            const f32x4 dx = *(const f32x4*) (ad + g * TOK + 16 * a + 4 * kq);
-            const i32x4 z = {0, 0, 0, 0};
-            const i32x4 cg = __builtin_amdgcn_mfma_i32_16x16x32_i8((long) av, (long) b_g, z, 0, 0, 0);
-            const i32x4 cu = __builtin_amdgcn_mfma_i32_16x16x32_i8((long) av, (long) b_u, z, 0, 0, 0);
+        for (int r = 0; r < 4; r++) total[a][r] = __builtin_fmaf(d[r], acc[a][r], total[a][r]);
+        acc[a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+
+// The products of a workgroup of 8 waves: T tiles of an item's tokens with 128 rows, waves 0 .. 3 the 64 that begin at w0, waves 4 .. 7 the
+// 64 at w1, 16 each; `blocks` IQ3_S blocks of every row, nc of them (the whole row) for one lot of 128 rows, whose sums go to
+// finish(lot, total), then nc of the rows `lot` bytes further on.  x, d: the codes and scales of `cols` inputs a row, s_rows (LDS): the
+// row of every token.
+//
+// Blocks and activations come into LDS by global-to-LDS loads, a wave's load instruction filling 64 consecutive slots from 64 addresses of
+// its choosing: the layout is made by choosing the addresses.  Token t's 16-byte column c lands at slot c ^ (t & 15) of its row, so
+// that the 16 tokens of an MFMA tile read the same column from 16 different bank groups.  For one or two tiles a whole block of
+// the rows with its activations is a stage, three or two of them in flight (an item of one tile has little to multiply while it
+// waits); for three and four the activations come a half block at a time, one ahead, the rows a block ahead.  Two workgroups a
+// compute unit by the stage's LDS.
+//
+// What bounds it: the decode, about 27 vector instructions for a lane's 8 weights, for every item of an expert again, then LDS (the grid
+// look-ups' bank conflicts) and the waits of items of one tile.  512 tokens through 512 experts of 2048 x 512, top-10, router with
+// Zipf's preferences: gate and up 138 -> 112 us, down 82 -> 61, the chunk 229 -> 173; 4096 tokens and the shared expert 1092 -> 847; 700
+// through 60 of 4096 x 1536, top-4, 582 -> 420.  Gate and up of 16 rows in one wave, which reads the activations half as often,
+// spilled registers (230 us).
+#define PF_STAGE 73728
+template <int T, class F>
+__device__ __forceinline__ void pf_stream(u8* stage, u64 w0, u64 w1, u64 lot, u32 rb, u32 nc, u32 blocks, const u16* __restrict__ x, const float* __restrict__ d, const u32* s_rows, u32 cols,
+                                          float* strip, u32 wave, u32 lane, F&& finish) {
+    constexpr u32 XB = T * 4096;   // half a block's activations: [16 T tokens][16 columns of 8 codes]
+    const u32 n = lane & 15, kq = lane >> 4, lrow = (wave & 3) * 16 + n, mine = wave >> 2, lds0 = __builtin_amdgcn_readfirstlane(lds_offset(stage));
+    PfRows rows;
+    rows.init(rb, wave, lane);
+    auto input = [&](u32 j) {   // the lane's part of an instruction of 4 tokens
+        const u32 t = 4 * j + (lane >> 4);
+        return x + (u64) s_rows[t] * cols + 8 * ((lane & 15) ^ (t & 15));
+    };
+    f32x4 acc[T], total[T];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                accg[a][r] = __builtin_fmaf(swg * dx[r], (float) cg[r], accg[a][r]);
-                accu[a][r] = __builtin_fmaf(swu * dx[r], (float) cu[r], accu[a][r]);
+    for (int a = 0; a < T; a++) acc[a] = total[a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    u32 ahead = 0;             // blocks asked for; of these in the current lot, and its number
+    u32 ac = 0, ab = 0;
+    u64 a0 = w0, a1 = w1;
+    auto next = [&] {
+        ahead++;
+        a0 += 110;
+        a1 += 110;
+        if (++ac == nc) {
+            ac = 0;
+            ab++;
+            a0 = w0 + ab * lot;
+            a1 = w1 + ab * lot;
+        }
+    };
+    u64 at = mine ? w1 : w0;   // the wave's block
+    u32 c = 0, done = 0;
+    auto fold = [&](const u8* blk) {
+        pf_fold<T>(total, acc, blk, strip, n, kq);
+        at += 110;
+        if (++c == nc) {
+            finish(done, total);
+#pragma unroll
+            for (int a = 0; a < T; a++) total[a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            c = 0;
+            done++;
+            at = (mine ? w1 : w0) + done * lot;
+        }
+    };
+    if constexpr (T <= 2) {
+        constexpr u32 D = T == 1 ? 3 : 2, WO = 2 * XB, DO = WO + 2 * PF_WB, SB = DO + 2048, A = 7 + T + 1;   // A: a wave's loads a stage
+        static_assert(D * SB <= PF_STAGE, "the stages' LDS");
+        const u16* xp = input(T == 1 ? wave & 3 : wave);
+        const float* dp = d + (u64) s_rows[lane] * (cols / 32) + wave;
+        auto request = [&](u32 slot) {
+            const u32 to = lds0 + slot * SB;
+            if constexpr (T == 1) lds_load<16>(xp + ac * 256 + (wave >> 2) * 128, to + wave * 1024);
+            else {
+                lds_load<16>(xp + ac * 256, to + wave * 1024);
+                lds_load<16>(xp + ac * 256 + 128, to + XB + wave * 1024);
             }
+            rows.issue<false>(a0, to + WO, wave);
+            rows.issue<true>(a1, to + WO + PF_WB, wave);
+            lds_load<4>(dp + ac * 8, to + DO + wave * 256);   // a sub-block's 64
+            next();
+        };
+#pragma unroll
+        for (u32 i = 0; i + 1 < D; i++)
+            if (i < blocks) request(i);
+        u32 slot = 0;
+#pragma unroll 1
+        for (u32 b = 0; b < blocks; b++) {
+            if (D == 3 && ahead > b + 1) wait_vm<(D - 2) * A>();
+            else wait_vm<0>();
+            __syncthreads();   // block b is in LDS, from every wave; the products of block b - 1 are done, so its slot is free
+            const u8* s = stage + slot * SB;
+            if (ahead < blocks) request(slot == 0 ? D - 1 : slot - 1);
+            slot = slot + 1 == D ? 0u : slot + 1;
+            const u8* blk = s + WO + mine * PF_WB + lrow * PF_WS + pf_shift(at, rb, lrow);
+            pf_products<T>(acc, s, (const float*) (s + DO), blk, 0, n, kq);
+            pf_products<T>(acc, s + XB, (const float*) (s + DO + 1024), blk, 1, n, kq);
+            fold(blk);
+        }
+    } else {
+        constexpr u32 WO = 2 * XB, DO = WO + 4 * PF_WB;
+        static_assert(DO + 2048 <= PF_STAGE, "the stages' LDS");
+        const u16* xp[2] = {input(wave), input(wave + 8)};
+        const float* dp = d + (u64) s_rows[lane] * (cols / 32) + (wave & 3);
+        auto inputs = [&](u32 u, u32 slot) {   // half u of a row's inputs
+            lds_load<16>(xp[0] + u * 128, lds0 + slot * XB + wave * 1024);
+            if (T == 4 || wave < 4) lds_load<16>(xp[1] + u * 128, lds0 + slot * XB + (wave + 8) * 1024);
+            if (wave < 4) lds_load<4>(dp + u * 4, lds0 + DO + slot * 1024 + wave * 256);
+        };
+        rows.issue<false>(a0, lds0 + WO, wave);
+        rows.issue<true>(a1, lds0 + WO + PF_WB, wave);
+        next();
+        inputs(0, 0);
+#pragma unroll 1
+        for (u32 b = 0; b < blocks; b++) {
+            const u8* blk = stage + WO + ((b & 1) * 2 + mine) * PF_WB + lrow * PF_WS + pf_shift(at, rb, lrow);
+            const u32 to = lds0 + WO + ((b + 1) & 1) * 2 * PF_WB;
+            wait_vm<0>();
+            __syncthreads();   // the block and its first half's activations are in LDS, from every wave; block b - 1 is done with
+            inputs(2 * c + 1, 1);
+            if (b + 1 < blocks) rows.issue<false>(a0, to, wave);
+            pf_products<T>(acc, stage, (const float*) (stage + DO), blk, 0, n, kq);
+            wait_vm<0>();
+            __syncthreads();
+            if (b + 1 < blocks) {
+                inputs(c + 1 == nc ? 0 : 2 * c + 2, 0);
+                rows.issue<true>(a1, to + PF_WB, wave);
+                next();
+            }
+            pf_products<T>(acc, stage + XB, (const float*) (stage + DO + 1024), blk, 1, n, kq);
+            fold(blk);
         }
     }
 }
-template <int T, int TOK>
-__device__ __forceinline__ void pf_products_d(float (&acc)[TOK / 16][4], const u8* aq, const float* ad, const u8* bd, u32 n, u32 kq, float* sws) {
-    iq3s_scales_to_strip(bd, n, kq, sws);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (u32 g = 0; g < 8; g++) {
-        const float sw = sws[g * 16 + n];
-        const u64 b = iq3s_int8x8(bd, g, kq);
-        const u32 col = ((2 * g + (kq >> 1)) ^ n) * 16 + 8 * (kq & 1);
-#pragma unroll
-        for (int a = 0; a < T; a++) {
-            const u64 av = *(const u64*) (aq + (16 * a + n) * 256 + col);
-            const f32x4 dx = *(const f32x4*) (ad + g * TOK + 16 * a + 4 * kq);
-            const i32x4 z = {0, 0, 0, 0};
-            const i32x4 cc = __builtin_amdgcn_mfma_i32_16x16x32_i8((long) av, (long) b, z, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[a][r] = __builtin_fmaf(sw * dx[r], (float) cc[r], acc[a][r]);
-        }
+template <int V> struct pf_int { static constexpr int value = V; };
+// Straight-line products for the item's number of token tiles: only that many tiles' sums are live in the loop.
+template <class F>
+__device__ __forceinline__ void pf_tiles(u32 nt, F&& run) {
+    switch ((nt + 15) / 16) {
+        case 1: return run(pf_int<1>{});
+        case 2: return run(pf_int<2>{});
+        case 3: return run(pf_int<3>{});
+        default: return run(pf_int<PF_TILES>{});
     }
 }
 
-// Work item blockIdx.y = (expert, first position) from prefill_group: gate and up rows [64 blockIdx.x + 16 (wave & 3), +16) of
+// Work item blockIdx.y = (expert, first position) from prefill_group: gate and up rows [64 blockIdx.x, +64) of
 // the expert against up to 64 of its pairs' tokens, SwiGLU (silu in f32, cpu_expert.rs:217), and H re-quantized per 32
-// features: hq[pair][ff], hd[pair][ff / 32].  eaddr[part * ne + e] / sh_addr[part] as in the planner's kernels.
-// grid = (ff / 64, the bound on the number of items), block 64 NWV.
-// NWV = 4: wave w rows 16 w .. 16 w + 15, all 8 sub-blocks of a chunk's block.  NWV = 8 (block 512): waves w and w + 4 share
-// the rows 16 (w & 3) .. and take sub-blocks 0..3 and 4..7 of every block; their partial sums are added at the end (the same
-// LDS a workgroup, twice the waves a SIMD to cover the LDS reads and the barriers of a chunk).
-template <int NWV>
-__device__ __forceinline__ void prefill_gate_up_iq3_s_body(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items,
-                                                           const i8* xq, const float* xd, i8* hq, float* hd, u32 ne, u32 k, u32 npairs, u32 hidden, u32 ff) {
-    // two buffers of a chunk: activations | gate rows | up rows | activation scales; afterwards the item's 64 x 64 block of H
-    constexpr u32 AB = PF_AB(PF_TOK), BUF = AB + 2 * PF_WB + PF_DB(PF_TOK);
-    __shared__ __attribute__((aligned(16))) u8 stage[2 * BUF];
+// features: hq[pair][ff], hh the same codes times 2^-6 as f16, hd[pair][ff / 32].  eaddr[part * ne + e] / sh_addr[part] as in the planner's kernels.
+// grid = (ff / 64, the bound on the number of items), block 512.
+extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
+                                                                        const u32* items, const u16* xh, const float* xd, i8* hq, u16* hh, float* hd, u32 ne,
+                                                                        u32 k, u32 npairs, u32 hidden, u32 ff) {
+    constexpr u32 HP = 68;
+    __shared__ __attribute__((aligned(16))) u8 stage[PF_STAGE];   // afterwards the item's 64 x 64 block of H
     __shared__ u32 s_rows[PF_TOK], s_pairs[PF_TOK];
-    __shared__ float s_sw[NWV][256];   // a wave's strip of sub-block scales: gate [8][16], up [8][16]
-    static_assert(sizeof(stage) >= 3 * PF_TOK * 65 * sizeof(float), "H and the second half's partial sums reuse the staging area");
-    float (*hs)[65] = (float (*)[65]) stage;
-    const u32 tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const u32 n = lane & 15, kq = lane >> 4;
-    const u32 rw = wave & 3, kh = wave >> 2;             // the wave's row group; which half of the sub-blocks (NWV = 8)
-    const u32 lrow = rw * 16 + n;                        // the lane's weight row inside the workgroup's 64
-    const u32 rb = hidden / 256 * 110, rbx = blockIdx.x;
-    const u32 lds0 = __builtin_amdgcn_readfirstlane(lds_offset(stage));
+    __shared__ __attribute__((aligned(16))) float s_strip[8][16];
+    static_assert(sizeof(stage) >= 2 * PF_TOK * HP * sizeof(float), "H and the up sums reuse the staging area");
+    const u32 tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const u32 n = lane & 15, kq = lane >> 4, rbx = blockIdx.x;
+    const u32 rb = hidden / 256 * 110;
     if (blockIdx.y >= items[0]) return;
     const u32 e = items[1 + 2 * blockIdx.y], t0 = items[2 + 2 * blockIdx.y];
     if (e == ne && !sh_addr) return;
     const u32 first = offs[e], nt = min((u32) PF_TOK, offs[e + 1] - first - t0);
-    if (tid < 256) pf_tables(tid);
-    const u8* wg = (const u8*) (e < ne ? eaddr[e] : sh_addr[0]) + (u64) rbx * 64 * rb;
-    const u8* wu = (const u8*) (e < ne ? eaddr[(u64) ne + e] : sh_addr[1]) + (u64) rbx * 64 * rb;
-    if (tid < PF_TOK) {
+    pf_tables(tid);
+    const u64 wg = uniform_u64(e < ne ? eaddr[e] : sh_addr[0]) + (u64) rbx * 64 * rb, wu = uniform_u64(e < ne ? eaddr[(u64) ne + e] : sh_addr[1]) + (u64) rbx * 64 * rb;
+    if (tid < PF_TOK) {   // a place past the item's end has row 0, whose products are dropped
         const u32 p = tid < nt ? list[first + t0 + tid] : 0;
         s_pairs[tid] = p;
         s_rows[tid] = p < npairs ? p / k : p - npairs;
     }
-    float accg[PF_TILES][4], accu[PF_TILES][4];
+    __syncthreads();   // s_rows and the table are written
+    float (*hs)[HP] = (float (*)[HP]) stage;
+    float (*us)[HP] = (float (*)[HP]) (stage + PF_TOK * HP * sizeof(float));
+    pf_tiles(nt, [&](auto tiles) {
+        constexpr int T = decltype(tiles)::value;
+        pf_stream<T>(stage, wg, wu, 0, rb, hidden / 256, hidden / 256, xh, xd, s_rows, hidden, s_strip[wave], wave, lane, [&](u32, f32x4 (&sums)[T]) {
+            // the staging area becomes H [token][feature]: up's sums go to the waves that hold gate's
+            __syncthreads();
+            if (wave >= 4) {
 #pragma unroll
-    for (int a = 0; a < PF_TILES; a++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) accg[a][r] = accu[a][r] = 0.0f;
-    __syncthreads();   // s_rows and the tables are written
-    auto issue = [&](u32 c) {
-        const u32 base = lds0 + (c & 1) * BUF;
-        pf_issue_a<PF_TOK, NWV>(xq, xd, s_rows, hidden, c * PF_KC, base, base + AB + 2 * PF_WB, wave, lane);
-        pf_issue_w<NWV>(wg, rb, c, base + AB, wave, lane);
-        pf_issue_w<NWV>(wu, rb, c, base + AB + PF_WB, wave, lane);
-    };
-    const u32 nc = hidden / PF_KC;
-    constexpr int NG = NWV == 8 ? 4 : 8;
-    // The loop over the chunks, straight-line code for the item's number of token tiles T (the scheduler overlaps one tile's
-    // loads and matrix instructions with the scaling of the tile before it) and, with 8 waves, for the wave's half of the
-    // sub-blocks: chosen once, outside the loop, so that only T tiles' sums are live in it.
-    auto chunks = [&](auto tiles, auto half) {
-        constexpr int T = decltype(tiles)::value, G0 = decltype(half)::value;
-        float ag[PF_TILES][4], au[PF_TILES][4];
-#pragma unroll
-        for (int a = 0; a < T; a++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) ag[a][r] = au[a][r] = 0.0f;
-        issue(0);
-        for (u32 c = 0; c < nc; c++) {
-            wait_vm<0>();
-            __syncthreads();   // chunk c is in LDS, from every wave; the products of chunk c - 1 are done, so its buffer is free
-            if (c + 1 < nc) issue(c + 1);
-            const u8* buf = stage + (c & 1) * BUF;
-            const u8* aq = buf;
-            const float* ad = (const float*) (buf + AB + 2 * PF_WB);
-            const u8* bg = buf + AB + lrow * PF_WS + pf_shift(wg, rb, c, lrow);
-            const u8* bu = buf + AB + PF_WB + lrow * PF_WS + pf_shift(wu, rb, c, lrow);
-            pf_products_gu<T, PF_TOK, NG, G0>(ag, au, aq, ad, bg, bu, n, kq, s_sw[wave]);
-        }
-#pragma unroll
-        for (int a = 0; a < T; a++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                accg[a][r] = ag[a][r];
-                accu[a][r] = au[a][r];
+                for (int a = 0; a < T; a++) *(f32x4*) &us[16 * a + n][16 * (wave - 4) + 4 * kq] = sums[a];
             }
-    };
-    auto halves = [&](auto tiles) {
-        if (NWV == 8 && kh == 1) chunks(tiles, pf_int<4>{});
-        else chunks(tiles, pf_int<0>{});
-    };
-    switch ((nt + 15) / 16) {
-        case 1: halves(pf_int<1>{}); break;
-#if PF_TILES > 2
-        case 2: halves(pf_int<2>{}); break;
-        case 3: halves(pf_int<3>{}); break;
-#endif
-        default: halves(pf_int<PF_TILES>{}); break;
-    }
-    __syncthreads();   // the staging area becomes H
-    if constexpr (NWV == 8) {
-        // the second half's partial sums go through LDS to the wave that holds the first half's
-        float (*pg)[65] = (float (*)[65]) (stage + PF_TOK * 65 * sizeof(float));
-        float (*pu)[65] = (float (*)[65]) (stage + 2 * PF_TOK * 65 * sizeof(float));
-        if (kh == 1) {
+            __syncthreads();
+            // H = silu(gate) * up for (token 16 a + n, features 16 wave + 4 kq + r)
+            if (wave < 4) {
 #pragma unroll
-            for (int a = 0; a < PF_TILES; a++)
+                for (int a = 0; a < T; a++) {
+                    const f32x4 u = *(const f32x4*) &us[16 * a + n][16 * wave + 4 * kq];
+                    f32x4 h;
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    pg[16 * a + 4 * kq + r][16 * rw + n] = accg[a][r];
-                    pu[16 * a + 4 * kq + r][16 * rw + n] = accu[a][r];
+                    for (int r = 0; r < 4; r++) h[r] = (sums[a][r] / (1.0f + expf(-sums[a][r]))) * u[r];
+                    *(f32x4*) &hs[16 * a + n][16 * wave + 4 * kq] = h;
                 }
+            }
+            __syncthreads();
+        });
+    });
+    // per-32 quantization over features: a thread 8 of them, the four threads of a 32-block side by side
+    const u32 t = tid >> 3, f = 8 * (tid & 7);
+    if (t < nt) {
+        float v[8], amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            v[i] = hs[t][f + i];
+            amax = fmaxf(amax, fabsf(v[i]));
         }
-        __syncthreads();
-        if (kh == 0) {
+        amax = fmaxf(amax, lane_xor<1>(amax, lane));
+        amax = fmaxf(amax, lane_xor<2>(amax, lane));
+        const float dd = amax / 127.0f;
+        const float id = dd > 0.0f ? 1.0f / dd : 0.0f;
+        u32 q[2] = {0, 0};
 #pragma unroll
-            for (int a = 0; a < PF_TILES; a++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    accg[a][r] += pg[16 * a + 4 * kq + r][16 * rw + n];
-                    accu[a][r] += pu[16 * a + 4 * kq + r][16 * rw + n];
-                }
+        for (int i = 0; i < 8; i++) {
+            v[i] = fminf(127.0f, fmaxf(-127.0f, roundf(v[i] * id)));
+            q[i / 4] |= ((u32) (int) v[i] & 0xffu) << (8 * (i % 4));
+            v[i] *= 0x1p-6f;
         }
+        const u64 at = (u64) s_pairs[t] * ff + rbx * 64 + f;
+        *(u32x2*) (hq + at) = u32x2{q[0], q[1]};
+        *(u32x4*) (hh + at) = u32x4{f16_pair(v[0], v[1]), f16_pair(v[2], v[3]), f16_pair(v[4], v[5]), f16_pair(v[6], v[7])};
+        if ((tid & 3) == 0) hd[at / 32] = dd;
     }
-    // H = silu(gate) * up for (token 16 a + 4 kq + r, feature 16 rw + n), then per-32 quantization over features
-    if (kh == 0) {
-#pragma unroll
-        for (int a = 0; a < PF_TILES; a++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) hs[16 * a + 4 * kq + r][16 * rw + n] = (accg[a][r] / (1.0f + expf(-accg[a][r]))) * accu[a][r];
-    }
-    __syncthreads();
-    if (tid < 2 * PF_TOK) {
-        const u32 t = tid >> 1, half = tid & 1;
-        if (t < nt) {
-            float amax = 0.0f;
-            for (u32 i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(hs[t][32 * half + i]));
-            const float dd = amax / 127.0f;
-            const float id = dd > 0.0f ? 1.0f / dd : 0.0f;
-            const u32 p = s_pairs[t];
-            i8* o = hq + (u64) p * ff + rbx * 64 + 32 * half;
-            for (u32 i = 0; i < 32; i++) o[i] = (i8) (int) fminf(127.0f, fmaxf(-127.0f, roundf(hs[t][32 * half + i] * id)));
-            hd[(u64) p * (ff / 32) + rbx * 2 + half] = dd;
-        }
-    }
-}
-
-extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
-                                                                        const u32* items, const i8* xq, const float* xd, i8* hq, float* hd, u32 ne,
-                                                                        u32 k, u32 npairs, u32 hidden, u32 ff) {
-    prefill_gate_up_iq3_s_body<8>(eaddr, sh_addr, offs, list, items, xq, xd, hq, hd, ne, k, npairs, hidden, ff);
-}
-// The same with four waves a workgroup (block 256), every wave the whole of its rows' blocks: kept for comparisons.
-extern "C" __global__ void __launch_bounds__(256, 2) prefill_gate_up_iq3_s_w4(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
-                                                                           const u32* items, const i8* xq, const float* xd, i8* hq, float* hd, u32 ne,
-                                                                           u32 k, u32 npairs, u32 hidden, u32 ff) {
-    prefill_gate_up_iq3_s_body<4>(eaddr, sh_addr, offs, list, items, xq, xd, hq, hd, ne, k, npairs, hidden, ff);
 }
 
 // Work item blockIdx.y: down rows of the expert against its pairs' H: eo[pair][hidden], unweighted (cpu_expert.rs:316-339).
-// A workgroup takes hidden / 64 / gridDim.x blocks of 64 rows one after the other (wave w rows 16 w .. 16 w + 15 of each):
-// its set-up is paid once, and the loads of a block's first chunk are in flight while the block before it is multiplied.
-// items: prefill_group's list of runs of up to PF_TOK_D pairs.
-// grid = (a divisor of hidden / 64, the bound on the number of those items), block 256.
-extern "C" __global__ void __launch_bounds__(256, 4) prefill_down_iq3_s(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
-                                                                     const u32* items, const i8* hq, const float* hd, float* eo, u32 ne, u32 hidden,
+// A workgroup takes hidden / 128 / gridDim.x lots of 128 rows one after the other: its set-up is paid once, and the loads of a
+// lot's first blocks are in flight while the lot before it is multiplied.
+// grid = (a divisor of hidden / 128, the bound on the number of items), block 512.
+extern "C" __global__ void __launch_bounds__(512, 4) prefill_down_iq3_s(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
+                                                                     const u32* items, const u16* hh, const float* hd, float* eo, u32 ne, u32 hidden,
                                                                      u32 ff) {
-    constexpr u32 TOK = PF_TOK_D, AB = PF_AB(TOK), BUF = AB + PF_WB + PF_DB(TOK);   // two buffers of a chunk: activations | rows | activation scales
-    __shared__ __attribute__((aligned(16))) u8 stage[2 * BUF];
-    __shared__ u32 s_pairs[TOK];
-    __shared__ float s_sw[4][128];   // a wave's strip of sub-block scales [8][16]
-    const u32 tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    __shared__ __attribute__((aligned(16))) u8 stage[PF_STAGE];
+    __shared__ u32 s_pairs[PF_TOK];
+    __shared__ __attribute__((aligned(16))) float s_strip[8][16];
+    const u32 tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const u32 n = lane & 15, kq = lane >> 4;
-    const u32 lrow = wave * 16 + n;
-    const u32 rb = ff / 256 * 110;
-    const u32 per = hidden / 64 / gridDim.x, rb0 = blockIdx.x * per;     // this workgroup's row blocks: rb0 .. rb0 + per - 1
-    const u32 lds0 = __builtin_amdgcn_readfirstlane(lds_offset(stage));
+    const u32 rb = ff / 256 * 110, per = hidden / 128 / gridDim.x, lot0 = blockIdx.x * per;
     if (blockIdx.y >= items[0]) return;
     const u32 e = items[1 + 2 * blockIdx.y], t0 = items[2 + 2 * blockIdx.y];
     if (e == ne && !sh_addr) return;
-    const u32 first = offs[e], nt = min((u32) TOK, offs[e + 1] - first - t0);
+    const u32 first = offs[e], nt = min((u32) PF_TOK, offs[e + 1] - first - t0);
     pf_tables(tid);
-    const u8* wd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]) + (u64) rb0 * 64 * rb;
-    if (tid < TOK) s_pairs[tid] = tid < nt ? list[first + t0 + tid] : 0;
-    float acc[TOK / 16][4];
+    const u64 wd = uniform_u64(e < ne ? eaddr[2ull * ne + e] : sh_addr[2]) + (u64) lot0 * 128 * rb;
+    if (tid < PF_TOK) s_pairs[tid] = tid < nt ? list[first + t0 + tid] : 0;
+    __syncthreads();   // s_pairs and the table are written
+    pf_tiles(nt, [&](auto tiles) {
+        constexpr int T = decltype(tiles)::value;
+        pf_stream<T>(stage, wd, wd + 64ull * rb, 128ull * rb, rb, ff / 256, per * (ff / 256), hh, hd, s_pairs, ff, s_strip[wave], wave, lane, [&](u32 lot, f32x4 (&sums)[T]) {
+            const u32 row = (lot0 + lot) * 128 + wave * 16 + 4 * kq;
 #pragma unroll
-    for (int a = 0; a < TOK / 16; a++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[a][r] = 0.0f;
-    __syncthreads();   // s_pairs and the tables are written
-    const u32 nc = ff / PF_KC, units = per * nc;   // a unit: one chunk of one row block
-    auto issue = [&](u32 u) {
-        const u32 base = lds0 + (u & 1) * BUF, c = u % nc;
-        pf_issue_a<TOK>(hq, hd, s_pairs, ff, c * PF_KC, base, base + AB + PF_WB, wave, lane);
-        pf_issue_w(wd + (u64) (u / nc) * 64 * rb, rb, c, base + AB, wave, lane);
-    };
-    issue(0);
-    for (u32 u = 0; u < units; u++) {
-        wait_vm<0>();
-        __syncthreads();   // unit u is in LDS, from every wave; the products of unit u - 1 are done, so its buffer is free
-        if (u + 1 < units) issue(u + 1);
-        const u32 c = u % nc, rbi = u / nc;
-        const u8* buf = stage + (u & 1) * BUF;
-        const u8* aq = buf;
-        const float* ad = (const float*) (buf + AB + PF_WB);
-        const u8* bd = buf + AB + lrow * PF_WS + pf_shift(wd + (u64) rbi * 64 * rb, rb, c, lrow);
-        if (nt <= 16) pf_products_d<1, TOK>(acc, aq, ad, bd, n, kq, s_sw[wave]);
-        else pf_products_d<2, TOK>(acc, aq, ad, bd, n, kq, s_sw[wave]);
-        if (c + 1 == nc) {   // the row block is complete
-            const u32 row = (rb0 + rbi) * 64 + lrow;
-#pragma unroll
-            for (int a = 0; a < TOK / 16; a++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const u32 t = 16 * a + 4 * kq + r;
-                    if (t < nt) eo[(u64) s_pairs[t] * hidden + row] = acc[a][r];
-                    acc[a][r] = 0.0f;
-                }
-        }
-    }
+            for (int a = 0; a < T; a++)
+                if (16 * a + n < nt) *(f32x4*) (eo + (u64) s_pairs[16 * a + n] * hidden + row) = sums[a];
+        });
+    });
 }

@@ -567,3 +567,47 @@ def test_exl3_prefill_bits_do_not_depend_on_the_chunk(gpu, kb, hidden, ff, ne, k
             for i, j in enumerate(rows):
                 assert rel_l2(got[j], want[i]) <= 1e-3, (j, rel_l2(got[j], want[i]))
         assert np.array_equal(bits(got), bits(first[:tokens])), tokens
+
+
+@pytest.mark.parametrize("hidden,ff", [(256, 256), (512, 768), (1024, 512)])
+def test_iq3s_prefill_items_of_every_size(gpu, hidden, ff):  # noqa: F811
+    """Experts with 1 to 130 tokens, at the edges of the tiles of 16 and the items of 64, over rows of one block (shorter than the
+    stages in flight) and more; a token of zeros and one whose activations are close to f32's largest.  Every row within the chunk's
+    1e-3 of the int8 oracle and, whatever the items' tiles, with the bits the token has in a chunk of its own; so has a chunk
+    of the same tokens over and over, in which a workgroup takes several lots of rows."""
+    rng = np.random.default_rng(hidden + ff)
+    counts, ty = [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 80, 130], sz.IQ3_S
+    ne = k = len(counts)
+    tokens = max(counts)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, True)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty, dbuf.data_ptr() + ne * stride)
+    x = rng.normal(size=(tokens, hidden)).astype(np.float32)
+    x[2], x[4] = 0.0, x[4] / np.abs(x[4]).max() * np.float32(3e38)
+    logits = rng.normal(size=(tokens, ne)).astype(np.float32)
+    logits[np.arange(tokens)[:, None] >= np.array(counts)[None]] = -np.inf
+    sgl = rng.normal(size=tokens).astype(np.float32)
+
+    def chunk(x, logits, sgl):
+        dx, dl, dg = dev(gpu, x), dev(gpu, logits), dev(gpu, sgl)
+        y = gpu.zeros(x.shape, dtype=gpu.float32, device="cuda")
+        s.moe_prefill_chunk(0, x.shape[0], dx.data_ptr(), dl.data_ptr(), dg.data_ptr(), y.data_ptr())
+        gpu.cuda.synchronize()
+        return y.cpu().numpy()
+
+    got = chunk(x, logits, sgl)
+    assert not got[2].any()
+    for j in (0, 1, 3, 14, 15, 16, 40, 64, 100, tokens - 1):
+        oi, ow = O.route(logits[j], k)
+        wq, wd, _ = O.quantize_act(x[j], 32)
+        want = np.zeros(hidden, np.float32)
+        for e, w in zip(oi, ow):
+            if e < ne:
+                want = want + np.float32(w) * O.expert_int8(blobs[e], hidden, ff, wq, wd)[0]
+        want = want + np.float32(O.lib().orc_sigmoid(float(sgl[j]))) * O.expert_int8(sh, hidden, ff, wq, wd)[0]
+        assert rel_l2(got[j], want) <= REL_L2, (j, rel_l2(got[j], want))
+    for j in (0, 2, 4, 15, 63, 64, 129):
+        assert np.array_equal(bits(chunk(x[j:j + 1], logits[j:j + 1], sgl[j:j + 1])[0]), bits(got[j])), j
+    reps = 1500                                              # long enough for several lots a workgroup
+    big = chunk(np.resize(x, (reps, hidden)), np.resize(logits, (reps, ne)), np.resize(sgl, reps))
+    assert np.array_equal(bits(big), bits(np.resize(got, (reps, hidden))))
