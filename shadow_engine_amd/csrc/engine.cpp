@@ -1358,11 +1358,11 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         const uint32_t bits = (uint32_t) f.bits, wide_ring = bits <= 7 ? 3 : 2;
         {
             const uint32_t ncb = wide_gu ? 2 : 1;
-            // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING, XPF_RING_N), afterwards the exchange of four tiles' sums
+            // LDS: slots of a unit's operand rows and the rings of trellis rows (XPF_RING_W, XPF_RING_N), afterwards the exchange of four tiles' sums
             uint32_t lds = ncb * 2 * std::min(4u, nt) * 8192;
             for (uint32_t n = 1; n <= nt; n += n == 1 ? 1 : 2) {
-                const uint32_t ring = wide_gu ? wide_ring : std::min(8u, (40 - 2 * n) / (2 * n + bits));
-                lds = std::max(lds, (wide_gu ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
+                const uint32_t ring = !wide_gu ? std::min(8u, (40 - 2 * n) / (2 * n + bits)) : n >= 6 ? wide_ring : std::min(8u, (39 - n) / (n + bits));
+                lds = std::max(lds, (wide_gu && n >= 6 ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
             }
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff), U32(tok)};
             if (launch(((wide_gu ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 256 * ncb, lds, stream, a)) return 1;

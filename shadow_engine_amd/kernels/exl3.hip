@@ -1349,12 +1349,16 @@ EXL3_HEAD_ENTRIES(8)
 // Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for; in workgroups of four waves 4.
 #define XPF_NT(K) ((K) <= 5 ? 8 : 6)
 #define XPF_NT_N 4
-// Units of a wave's ring of trellis rows: what eight waves have room for, and in workgroups of four waves as deep as leaves two of them room on a
-// compute unit, with the operand rows of NT tiles and no more than 8 (rings of 5 units for four tiles and one workgroup a unit: 200
-// tokens of 512 experts of 2048 x 512, top-10, 3 bits 160 us, with rings of 2 and two workgroups 140; with a router without preferences 432
-// and 347).
+// Units of a wave's ring of trellis rows.  Launch 2, eight waves a workgroup: with six and eight tiles what a compute unit's LDS has room
+// for beside three slots of operand rows (XPF_RING); with fewer as many as fit with one slot more, at most 8: an item of one or
+// two tiles multiplies little while it waits.  4096 tokens of 512 experts of 2048 x 512, top-10, and the shared one, 4 bits: 916 -> 892 us (an item of one tile had waited half its time with rings of 3).
+// Four waves: as deep as leaves two workgroups room on a compute unit (rings of 5 units for four tiles and one workgroup a
+// unit: 200 tokens of 512 experts of 2048 x 512, top-10, 3 bits 160 us, with rings of 2 and two workgroups 140; with a router without
+// preferences 432 and 347).
 #define XPF_RING(K) ((K) <= 7 ? 3 : 2)
-#define XPF_RING_N(K, NT) ((40 - 2 * (NT)) / (2 * (NT) + (K)) < 8 ? (40 - 2 * (NT)) / (2 * (NT) + (K)) : 8)   /* (D + 1) 4096 NT + 2048 K D bytes, at most 80 KiB */
+// (D + 1) 4096 NT + 4096 K D bytes, at most 156 KiB; with four waves (D + 1) 4096 NT + 2048 K D, at most 80 KiB
+#define XPF_RING_W(K, NT) ((NT) >= 6 ? XPF_RING(K) : (39 - (NT)) / ((NT) + (K)) < 8 ? (39 - (NT)) / ((NT) + (K)) : 8)
+#define XPF_RING_N(K, NT) ((40 - 2 * (NT)) / (2 * (NT) + (K)) < 8 ? (40 - 2 * (NT)) / (2 * (NT) + (K)) : 8)
 // Launch 3's, of four waves: as deep as leaves two workgroups room with the rows of one tile.
 #define XPF_RING_DOWN_N(K) ((K) <= 3 ? 8 : (K) == 4 ? 7 : (K) == 5 ? 5 : (K) <= 7 ? 4 : 3)
 // What undoes the 1 / 128 that the stored values carry and applies the transform's 1 / sqrt(128)
@@ -1825,8 +1829,8 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
     const u8* bd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
     xpf_tiles<NCB == 2 ? XPF_NT(K) : XPF_NT_N>(it.tiles, [&](auto n) {
         constexpr int NT = decltype(n)::value, G = NT < 4 ? NT : 4;
-        typedef VerifyRing<K, false, 4, NCB == 2 ? XPF_RING(K) : XPF_RING_N(K, NT)> R;
-        constexpr int NB = NCB == 2 ? 3 : R::D + 1;
+        typedef VerifyRing<K, false, 4, NCB == 2 ? XPF_RING_W(K, NT) : XPF_RING_N(K, NT)> R;
+        constexpr int NB = NCB == 2 && NT >= 6 ? 3 : R::D + 1;
         u32* wb = dyn + NB * 2 * NT * (XPF_HALF_U16 / 2) + wave * (R::D * R::UW);
         R ring;
         ring.init((sel ? bu : bg) + 2 * (u64) hidden + 2 * (u64) ff + 4 + (u64) (cb * 8 + half * 4) * (4 * R::TW), (ff / 16) * (4 * R::TW), 2 * kbs,

@@ -112,3 +112,19 @@ def test_prefill_streams_stay_inside_their_item_and_wait_for_what_they_read(tmp_
     subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
     r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_prefill_streams_of_eight_waves_as_deep_as_their_tiles_leave_room(tmp_path):
+    """The same for the rings of workgroups of eight waves: the fewer the tiles the deeper, and within a compute unit's LDS."""
+    src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
+    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_W", "XPF_RING_N", "XPF_HALF_U16"))
+    start = src.index("template <int K, int NT, int NB, int NW, class R>")
+    stream = src[start:src.index("\n}\n", start) + 3]
+    of_four, of_eight = "stream<K, NT, 3, 4, XPF_RING(K)>", "stream<K, NT, NT >= 6 ? 3 : XPF_RING_W(K, NT) + 1, 4, XPF_RING_W(K, NT)>"
+    room = "static_assert((NT >= 6 ? 3 : XPF_RING_W(K, NT) + 1) * NT + K * XPF_RING_W(K, NT) <= 39, \"LDS\"); "
+    assert of_four in HARNESS
+    path = tmp_path / "stream.cpp"
+    path.write_text(HARNESS.replace(of_four, room + of_eight) % {"macros": macros, "stream": stream})
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
+    r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
