@@ -1301,6 +1301,14 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
     const bool shared = L.shared != 0;
     const uint64_t T = tokens, k = c.top_k, np = T * k, rows = np + (shared ? T : 0);
     auto& pb = s->pf;
+    // prefill_group: one workgroup up to 4096 pairs, beyond them one for the items and up to 16 that list 2048 pairs or more each
+    auto group = [&](uint64_t items_d, uint32_t unit, uint32_t unit_d) -> int {
+        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(items_d), U32(unit), U32(unit_d)};
+        if (np <= 4096) return launch("prefill_group", 1, 1, 1, 1024, 0, stream, a);
+        const uint32_t share = (uint32_t) std::max<uint64_t>(2048, (np + 15) / 16);
+        const sz_arg b[] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], U32(share)};
+        return launch("prefill_group_many", 1 + (uint32_t) ((np + share - 1) / share), 1, 1, 1024, 0, stream, b);
+    };
     if (exl3) {
         // EXL3 experts: f16 activations on the columns of the matrix instruction, items of up to 128 pairs, of 64 for the down
         // products (kernels/exl3.hip, "the prefill chunk of an EXL3 layer": XPF_NT, XPF_DOWN_NT, XPF_ROWS_U16, XPF_RING)
@@ -1341,11 +1349,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
             const sz_arg a[] = {P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens), P(x), P(pb.most.ptr), U32(c.hidden)};
             if (launch("route_topk_rows", (tokens + 3) / 4 * 2, 1, 1, 256, 0, stream, a)) return 1;
         }
-        {
-            const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr),
-                                P(pb.items.ptr), P(items_d), U32(tok), U32(16 * nd)};
-            if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
-        }
+        if (group(items_d, tok, 16 * nd)) return 1;
         {
             // shares of the inputs' 128-blocks, as many as make about 1200 workgroups of a few tiles (45 tokens through 512 experts of 2048 x 512
             // as above 121, 118, 117, 115 us with 1 to 4, 250 as above 159, 152, 146, 150, 1200 through 128 of 4096 x 512, top-8, at 4 bits
@@ -1385,7 +1389,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
     }
     const uint64_t max_items = c.n_expert + 1 + rows / 64;   // every expert's runs of up to 64 pairs: PF_TOK in kernels/prefill.hip
     if (pb.lay({{&pb.xq, T * c.hidden}, {&pb.xd, T * c.hidden / 32 * 4}, {&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4},
-                {&pb.items, (2 + 4 * max_items) * 4}, {&pb.hq, rows * c.ff}, {&pb.xh, T * c.hidden * 2}, {&pb.hh, rows * c.ff * 2}, {&pb.hd, rows * (c.ff / 32) * 4}, {&pb.eo, rows * c.hidden * 4}}))
+                {&pb.items, (1 + 2 * max_items) * 4}, {&pb.hq, rows * c.ff}, {&pb.xh, T * c.hidden * 2}, {&pb.hh, rows * c.ff * 2}, {&pb.hd, rows * (c.ff / 32) * 4}, {&pb.eo, rows * c.hidden * 4}}))
         return 1;
     const uint64_t sh = shared ? L.eaddr.ptr + 3ull * c.n_expert * 8 : 0;
     {
@@ -1394,11 +1398,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         const sz_arg a[] = {P(x), U64(n), P(pb.xq.ptr), P(pb.xd.ptr), P(pb.xh.ptr), P(rl), P(pb.tidx.ptr), P(pb.w.ptr), P(pb.cnt.ptr), U32(c.n_expert), U32(c.top_k), U32(tokens)};
         if (launch("prefill_front", (tokens + 3) / 4 + (uint32_t) ((n / 32 + 255) / 256), 1, 1, 256, 0, stream, a)) return 1;
     }
-    const uint64_t items_d = pb.items.ptr + (1 + 2 * max_items) * 4;
-    {
-        const sz_arg a[] = {P(pb.tidx.ptr), U32(tokens), U32(c.top_k), U32(c.n_expert), U32(shared ? tokens : 0), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(items_d), U32(64), U32(64)};
-        if (launch("prefill_group", 1, 1, 1, 1024, 0, stream, a)) return 1;
-    }
+    if (group(0, 64, 64)) return 1;
     {
         const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.list.ptr), P(pb.items.ptr), P(pb.xh.ptr), P(pb.xd.ptr), P(pb.hq.ptr), P(pb.hh.ptr), P(pb.hd.ptr),
                             U32(c.n_expert), U32(c.top_k), U32((uint32_t) np), U32(c.hidden), U32(c.ff)};

@@ -115,42 +115,51 @@ extern "C" __global__ void __launch_bounds__(256) prefill_front(const float* x, 
 // (expert, first position) of item i: every run of up to unit_gu pairs of an expert is one item of the gate/up kernel (at most
 // ne + 1 + rows / unit_gu of them); items_d likewise with runs of up to unit_d pairs, for the down kernel.  The longest items come
 // first, so that the launches end on short ones, and all ahead of the workgroups launched for the rest of the bound (int8 chunk of 512
-// tokens: 239 -> 226 us with the order alone).  Bound by the round trips of its loads: 41 us for 40960 pairs when a thread had one in
-// flight, 37 with eight, 29 with 32.  One workgroup.  grid 1, block 1024; ne <= 512.
-extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list,
-                                                                 u32* items, u32* items_d, u32 unit_gu, u32 unit_d) {
-    __shared__ u32 s_cnt[513], s_off[514], s_fill[513], s_full[2][513], s_class[2][9];
+// tokens: 239 -> 226 us with the order alone).  items_d may be null.
+// Up to 4096 pairs one workgroup does it all (prefill_group).  For more (prefill_group_many) every workgroup counts all pairs; the first then writes offs and the
+// items, the others list `share` pairs each, whose places in an expert's run the count of the pairs ahead of them tells: nothing passes between workgroups.
+// Bound by the counting, lots of loads and the LDS additions of popular experts.  40960 pairs 29.5 -> 16.8 us, 5120 9.6 -> 6.5, where one
+// workgroup did it all; 450 pairs 4.6 either way, which the common form would make 4.9.
+template <bool many>
+__device__ __forceinline__ void prefill_group_body(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list, u32* items, u32* items_d, u32 unit_gu, u32 unit_d, u32 share) {
+    __shared__ u32 s_cnt[513], s_off[514], s_ahead[513], s_full[2][513], s_class[2][9];
     const u32 tid = threadIdx.x, npairs = tokens * k, nexp = ne + 1;
+    const u32 b = many ? blockIdx.x : 0u, from = !many ? 0u : b ? min((b - 1) * share, npairs) : npairs, to = many ? min(from + share, npairs) : npairs;   // the pairs it lists
     for (u32 i = tid; i < nexp; i += 1024) {
         s_cnt[i] = 0;
-        s_fill[i] = 0;
+        s_ahead[i] = 0;
     }
     if (tid < 18) s_class[tid / 9][tid % 9] = 0;
     __syncthreads();
     // 32 pairs of a thread in flight at a time: the loads' round trips are what this launch is made of; as many as there are where those are few
     // (1200 pairs 8.0 us with 32, 5.0 with four)
-    auto lot = [&](auto depth, u32 p0, auto each) {
+    auto lot = [&](auto depth, u32 p0, u32 end, auto use) {
         constexpr int N = sizeof(depth);
         u32 e[N];
 #pragma unroll
         for (int q = 0; q < N; q++) e[q] = tidx[min(p0 + 1024 * q, npairs - 1)];
 #pragma unroll
         for (int q = 0; q < N; q++)
-            if (p0 + 1024 * q < npairs && e[q] < ne) each(p0 + 1024 * q, e[q]);
+            if (p0 + 1024 * q < end && e[q] < ne) use(p0 + 1024 * q, e[q]);
     };
     struct Many {
         u8 of[32];
     };
-    auto pairs = [&](auto each) {
-        if (npairs <= 1024) {
-            if (tid < npairs) lot(u8(), tid, each);
-        } else if (npairs <= 4096) lot(u32(), tid, each);
-        else
-            for (u32 p0 = tid; p0 < npairs; p0 += 32 * 1024) lot(Many(), p0, each);
+    auto few = [&](u32 p0, u32 end, auto use) {
+        if (!many && npairs <= 1024) {
+            if (tid < npairs) lot(u8(), tid, npairs, use);
+        } else
+            for (; p0 < end; p0 += 4 * 1024) lot(u32(), p0, end, use);
     };
-    pairs([&](u32, u32 e) { atomicAdd(&s_cnt[e], 1u); });
+    if (many)
+        for (u32 p0 = tid; p0 < npairs; p0 += 32 * 1024) lot(Many(), p0, npairs, [&](u32 p, u32 e) { atomicAdd(p < from ? &s_ahead[e] : &s_cnt[e], 1u); });
+    else few(tid, npairs, [&](u32, u32 e) { atomicAdd(&s_cnt[e], 1u); });
     if (tid == 0) s_cnt[ne] = nshared;
     __syncthreads();
+    if (from) {   // (uniform)
+        for (u32 i = tid; i < nexp; i += 1024) s_cnt[i] += s_ahead[i];
+        __syncthreads();
+    }
     // three running sums over the experts, each by a wave of its own: lane L takes the experts [9 L, 9 L + 9) (ne <= 512), the
     // lanes' totals are scanned across the wave, and every lane writes its experts' starts: of the pairs, of the full items of
     // either list
@@ -185,14 +194,19 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
             }
         } else {
             // the items that are not full, by the number of their tiles of 16 pairs
-            for (u32 i = tid - 192; i < 2 * nexp; i += 1024 - 192) {
+            for (u32 i = tid - 192; b == 0 && i < (items_d ? 2 : 1) * nexp; i += 1024 - 192) {
                 const u32 l = i >= nexp ? 1u : 0u, unit = l ? unit_d : unit_gu, rest = s_cnt[i - l * nexp] % unit;
                 if (rest) atomicAdd(&s_class[l][1 + min((unit - rest) / 16, 7u)], 1u);
             }
         }
     }
     __syncthreads();
-    if (tid < 2) {   // where the full ones end and each class begins, the longest first
+    auto lists = [&] {
+        few(from + tid, to, [&](u32 p, u32 e) { list[s_off[e] + atomicAdd(&s_ahead[e], 1u)] = p; });
+        for (u32 j = b * 1024 + tid; j < nshared; j += (many ? gridDim.x : 1u) * 1024) list[s_off[ne] + j] = npairs + j;
+    };
+    if (b) return lists();
+    if (tid < (items_d ? 2u : 1u)) {   // where the full ones end and each class begins, the longest first
         u32 run = 0;
         for (u32 c = 0; c < 9; c++) {
             const u32 n = s_class[tid][c];
@@ -202,7 +216,7 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
         (tid ? items_d : items)[0] = run;
     }
     __syncthreads();
-    for (u32 i = tid; i < 2 * nexp; i += 1024) {
+    for (u32 i = tid; i < (items_d ? 2 : 1) * nexp; i += 1024) {
         const u32 l = i >= nexp ? 1u : 0u, e = i - l * nexp, unit = l ? unit_d : unit_gu, n = s_cnt[e], rest = n % unit;
         u32* to = l ? items_d : items;
         u32 at = s_full[l][e], t0 = 0;
@@ -217,8 +231,17 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx
         }
     }
     for (u32 i = tid; i <= nexp; i += 1024) offs[i] = s_off[i];
-    pairs([&](u32 p, u32 e) { list[s_off[e] + atomicAdd(&s_fill[e], 1u)] = p; });
-    for (u32 j = tid; j < nshared; j += 1024) list[s_off[ne] + j] = npairs + j;
+    lists();
+}
+// At most 4096 pairs.  grid 1, block 1024; ne <= 512.
+extern "C" __global__ void __launch_bounds__(1024) prefill_group(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list,
+                                                                 u32* items, u32* items_d, u32 unit_gu, u32 unit_d) {
+    prefill_group_body<false>(tidx, tokens, k, ne, nshared, offs, list, items, items_d, unit_gu, unit_d, 0);
+}
+// grid = 1 + ceil(pairs / share), block 1024; ne <= 512.
+extern "C" __global__ void __launch_bounds__(1024) prefill_group_many(const u32* tidx, u32 tokens, u32 k, u32 ne, u32 nshared, u32* offs, u32* list,
+                                                                      u32* items, u32* items_d, u32 unit_gu, u32 unit_d, u32 share) {
+    prefill_group_body<true>(tidx, tokens, k, ne, nshared, offs, list, items, items_d, unit_gu, unit_d, share);
 }
 
 __shared__ u32x2 pf_grid[512];   // the codebook grid, a weight's magnitude as f16

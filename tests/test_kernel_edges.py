@@ -611,3 +611,23 @@ def test_iq3s_prefill_items_of_every_size(gpu, hidden, ff):  # noqa: F811
     reps = 1500                                              # long enough for several lots a workgroup
     big = chunk(np.resize(x, (reps, hidden)), np.resize(logits, (reps, ne)), np.resize(sgl, reps))
     assert np.array_equal(bits(big), bits(np.resize(got, (reps, hidden))))
+
+
+@pytest.mark.parametrize("tokens,k", [(1024, 4), (1025, 4), (2049, 2), (1366, 3), (2731, 12), (16384, 2)])
+def test_grouping_of_more_pairs_than_one_workgroup_lists(gpu, tokens, k):  # noqa: F811
+    """4096 pairs, the first numbers beyond (a share of one run of 1024 pairs and a ragged one), some masked, and many: every token has
+    the bits it has in chunks that one workgroup groups."""
+    rng = np.random.default_rng(tokens + k)
+    hidden, ff, ne, ty = 256, 256, 16, sz.IQ3_S
+    dbuf, stride, _, _ = build_layer(gpu, rng, ty, hidden, ff, ne, True)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty, dbuf.data_ptr() + ne * stride)
+    logits = synth.zipf_router_logits(rng, tokens, ne)
+    logits[::7, :-k + 1] = -np.inf                           # fewer experts than k
+    dx, dl, dg = dev(gpu, rng.normal(size=(tokens, hidden)).astype(np.float32)), dev(gpu, logits), dev(gpu, rng.normal(size=tokens).astype(np.float32))
+    whole, cut = (gpu.zeros((tokens, hidden), dtype=gpu.float32, device="cuda") for _ in range(2))
+    s.moe_prefill_chunk(0, tokens, dx.data_ptr(), dl.data_ptr(), dg.data_ptr(), whole.data_ptr())
+    for t0 in range(0, tokens, 300):
+        s.moe_prefill_chunk(0, min(300, tokens - t0), dx[t0:].data_ptr(), dl[t0:].data_ptr(), dg[t0:].data_ptr(), cut[t0:].data_ptr())
+    gpu.cuda.synchronize()
+    assert gpu.isfinite(whole).all() and np.array_equal(bits(whole.cpu().numpy()), bits(cut.cpu().numpy()))
