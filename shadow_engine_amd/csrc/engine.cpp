@@ -1313,15 +1313,16 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
         // EXL3 experts: f16 activations on the columns of the matrix instruction, items of up to 128 pairs, of 64 for the down
         // products (kernels/exl3.hip, "the prefill chunk of an EXL3 layer": XPF_NT, XPF_DOWN_NT, XPF_ROWS_U16, XPF_RING)
         if (c.ff > 512) return fail("sz_moe_prefill_chunk: EXL3 experts of more than 512 intermediate features are not built (a workgroup keeps four 128-blocks of a token)");
-        const uint32_t kbs = c.hidden / 128, fbs = c.ff / 128, widest = f.bits <= 5 ? 8 : 6;
+        const uint32_t kbs = c.hidden / 128, fbs = c.ff / 128;
         const uint64_t some = std::min<uint64_t>(c.n_expert, np) + 1;
-        // The gate and up launch: workgroups of four waves, two of which share a compute unit, with items of up to 64 pairs; for long chunks of
-        // eight waves, which take two 128-blocks of ff and items of up to 128 pairs: an expert is decoded less often, but a workgroup has a
-        // unit for itself (4096 tokens through 512 experts of 2048 x 512, top-10, and the shared one, 4 bits, four waves and eight, a
-        // router with Zipf's preferences: 941 and 915 us, without: 1110 and 1019; 3500 through 64 of 3072 x 512, top-6: 727 and 681;
-        // 2048 as the first 556 and 550, 601 and 669; 4000 through 256 of 3072 x 256, top-6, 2 bits 611 and 624).
+        // The gate and up launch: workgroups of one 128-block of ff, two of which share a compute unit, with items of up to 64 pairs; for long
+        // chunks of two 128-blocks and items of up to 128 pairs: an expert is decoded less often, but a workgroup has a unit for
+        // itself (4096 tokens through 512 experts of 2048 x 512, top-10, and the shared one, 4 bits, one block and two, a router with
+        // Zipf's preferences: 941 and 915 us, without: 1110 and 1019; 3500 through 64 of 3072 x 512, top-6: 727 and 681; 2048 as the first
+        // 556 and 550, 601 and 669; 4000 through 256 of 3072 x 256, top-6, 2 bits 611 and 624; measured again since both gained: 1500 as the
+        // first 433, 433, 512 of them 221, 218, 200 140, 172).
         const bool wide_gu = rows * fbs >= 95000;
-        // Of four waves, items so short that the chip is full: an item's chain over all inputs takes about 4 + its tiles; two workgroups that share
+        // Of one block, items so short that the chip is full: an item's chain over all inputs takes about 4 + its tiles; two workgroups that share
         // a unit 1.6 times that.  Routers prefer some experts: 0.3 of those that independent choices would reach, the experts' last tiles
         // and the rest of the pairs in whole items.  us with items of 16, 32 and 64 pairs, router with Zipf's preferences and without: 45 tokens
         // as above at 3 bits 100, 112, 106 and 213, 240, 240; 200 tokens 179, 160, 140 and 354, 335, 347; 512 tokens 328, 260, 227 and
@@ -1369,7 +1370,7 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
                 lds = std::max(lds, (wide_gu && n >= 6 ? 3 : ring + 1) * 2 * n * 2048 + 4 * ncb * ring * 512 * bits);
             }
             const sz_arg a[] = {P(L.eaddr.ptr), P(sh), P(pb.offs.ptr), P(pb.items.ptr), P(pb.arows.ptr), P(pb.ainv.ptr), P(pb.drows.ptr), P(pb.dinv.ptr), U32(c.n_expert), U32(c.hidden), U32(c.ff), U32(tok)};
-            if (launch(((wide_gu ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 256 * ncb, lds, stream, a)) return 1;
+            if (launch(((wide_gu ? "prefill_gate_up_" : "prefill_gate_up_n_") + tag).c_str(), bound * (fbs / ncb), 1, 1, 512, lds, stream, a)) return 1;
         }
         {
             // shares of an item: a wave a column block, but all blocks on eight waves, whose start then counts once, where items fill the chip (1, 2

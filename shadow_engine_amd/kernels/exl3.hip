@@ -236,15 +236,15 @@ __device__ __forceinline__ u64 uniform_u64(u64 v) {
     return ((u64) (u32) __builtin_amdgcn_readfirstlane((u32) (v >> 32)) << 32) | (u32) __builtin_amdgcn_readfirstlane((u32) v);
 }
 
-// A wave's stream of trellis rows for CT column tiles: units of 16 tiles (16 / CT tile rows, 512 K bytes), each brought
+// A wave's stream of trellis rows for CT column tiles: units of UT tiles (UT / CT tile rows, 32 K UT bytes), each brought
 // into one of D ring slots by NI global-to-LDS loads of 16 bytes a lane.  In LDS a unit lies packed in the order of the
 // bit stream: tile row, column tile, tile word.
-template <int K, bool H, int CT, int DEPTH = 0>
+template <int K, bool H, int CT, int DEPTH = 0, int UT = 16>
 struct VerifyRing {
     static constexpr int TW = EXL3_TILE_WORDS(K, H), CH = TW / 4;   // words and 16-byte chunks a tile
-    static constexpr int UR = 16 / CT;                              // tile rows a unit
-    static constexpr int NI = (CH + 3) / 4;                         // loads a unit: 16 CH chunks, 64 a load, the last load perhaps partly
-    static constexpr int UW = 64 * CH;                              // words a unit
+    static constexpr int UR = UT / CT;                              // tile rows a unit
+    static constexpr int NI = (UT * CH + 63) / 64;                  // loads a unit: UT CH chunks, 64 a load, the last load perhaps partly
+    static constexpr int UW = UT * TW;                              // words a unit
     static constexpr int D = DEPTH ? DEPTH : CH <= 8 ? 3 : 2;
     u64 row0;         // the wave's first tile row, at its first column tile (uniform)
     u32 pitch;        // bytes between tile rows
@@ -265,7 +265,7 @@ struct VerifyRing {
         const u64 at = row0 + (u64) unit * ((u64) UR * pitch);
 #pragma unroll
         for (int i = 0; i < NI; i++)
-            if (64 * (i + 1) <= 16 * CH || 64 * i + lane < 16 * CH) lds_load_at(at, off[i], lds + (slot * UW + i * 256) * 4);
+            if (64 * (i + 1) <= UT * CH || 64 * i + lane < (u32) (UT * CH)) lds_load_at(at, off[i], lds + (slot * UW + i * 256) * 4);
     }
     // requests the first D units and returns once everything requested before them has landed
     __device__ __forceinline__ void fill(u32 lane) const {
@@ -1340,23 +1340,27 @@ EXL3_HEAD_ENTRIES(8)
 // workgroup, a third of launch 2's time.  4096 tokens through 512 experts of 2048 x 512 and the shared one at 4 bits, top-10: 130 + 385 +
 // 265 us, 568 items and 907 of the down launch, where items of 48 tokens, with every workgroup rotating a quarter of the inputs for itself
 // and 738 MB of partial sums in between, took 674 + 213 + 285.  The chunk on inputs that are not in a cache: 1290 -> 914 us.
-// Of few items launch 2 is as long as the longest item's chain over all inputs, and the chip is not full: the host takes workgroups of four
-// waves, two a compute unit, and shorter items, down to one tile, and splits launch 1 and 3 over the 128-blocks (45 tokens at 3 bits 121 -> 100
-// us, 512 tokens 273 -> 227, 250 through 32 experts of 3072 x 256, top-3, at 2 bits 104 -> 93 and 159 with items of 128).
+// Of few items launch 2 is as long as the longest item's chain over all inputs, and the chip is not full: the host takes workgroups of one
+// 128-block, two a compute unit, and shorter items, down to one tile, and splits launch 1 and 3 over the 128-blocks (45 tokens at 3 bits 121 -> 100
+// us, 512 tokens 273 -> 221, 250 through 32 experts of 3072 x 256, top-3, at 2 bits 104 -> 91 and 159 with items of 128).  Their waves take 32
+// columns: with 64 a SIMD had one or two waves, and a wave alone gets a vector instruction in five to eight cycles (16 tokens through 60
+// experts of 4096 x 512, top-4, 98 -> 91 us, 64 113 -> 107, 100 through 512 of 2048 x 512, top-10, 122 -> 119; 45 101, 101: 292 such
+// workgroups on 256 units, of which some have two and work at the decode's rate).
 // Tried: launch 2 by waves of 128 columns for 64 tokens (460 us), its matrix instructions placed among the decode (no change), its two
 // waves of a SIMD half a unit apart (2 %), an expert's items on one XCD (less traffic, same time); launch 3 in launch 2's form (272 to 312).
 
-// Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for; in workgroups of four waves 4.
+// Most tiles of 16 tokens of a work item: what a wave of 64 columns can keep sums and operands for; in workgroups of one 128-block 4.
 #define XPF_NT(K) ((K) <= 5 ? 8 : 6)
 #define XPF_NT_N 4
-// Units of a wave's ring of trellis rows.  Launch 2, eight waves a workgroup: with six and eight tiles what a compute unit's LDS has room
-// for beside three slots of operand rows (XPF_RING); with fewer as many as fit with one slot more, at most 8: an item of one or
-// two tiles multiplies little while it waits.  4096 tokens of 512 experts of 2048 x 512, top-10, and the shared one, 4 bits: 916 -> 892 us (an item of one tile had waited half its time with rings of 3).
-// Four waves: as deep as leaves two workgroups room on a compute unit (rings of 5 units for four tiles and one workgroup a
+// Units of a wave's ring of trellis rows (64 inputs).  Launch 2, two 128-blocks a workgroup: with six and eight tiles what a compute unit's LDS has
+// room for beside three slots of operand rows (XPF_RING); with fewer as many as fit with one slot more, at most 8: an item of one or
+// two tiles multiplies little while it waits.  4096 tokens of 512 experts of 2048 x 512, top-10, and the shared one, 4 bits: 916 -> 892
+// us (an item of one tile had waited half its time with rings of 3).
+// One 128-block: as deep as leaves two workgroups room on a compute unit (rings of 5 units for four tiles and one workgroup a
 // unit: 200 tokens of 512 experts of 2048 x 512, top-10, 3 bits 160 us, with rings of 2 and two workgroups 140; with a router without
 // preferences 432 and 347).
 #define XPF_RING(K) ((K) <= 7 ? 3 : 2)
-// (D + 1) 4096 NT + 4096 K D bytes, at most 156 KiB; with four waves (D + 1) 4096 NT + 2048 K D, at most 80 KiB
+// (D + 1) 4096 NT + 4096 K D bytes, at most 156 KiB; of one 128-block (D + 1) 4096 NT + 2048 K D, at most 80 KiB
 #define XPF_RING_W(K, NT) ((NT) >= 6 ? XPF_RING(K) : (39 - (NT)) / ((NT) + (K)) < 8 ? (39 - (NT)) / ((NT) + (K)) : 8)
 #define XPF_RING_N(K, NT) ((40 - 2 * (NT)) / (2 * (NT) + (K)) < 8 ? (40 - 2 * (NT)) / (2 * (NT) + (K)) : 8)
 // Launch 3's, of four waves: as deep as leaves two workgroups room with the rows of one tile.
@@ -1620,35 +1624,36 @@ extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64*
     }
 }
 
-// What a wave multiplies at a time: two tile rows of four column tiles (the words of their windows) with the operand rows of NT token
+// What a wave multiplies at a time: two tile rows of four (CT = 2: two) column tiles (the words of their windows) with the operand rows of NT token
 // tiles, `step` u16 from one to the next.  read() and rows() ask LDS for them, products() adds acc[T][c][q] = output 16 c + 4 a + q of token 16 T + n.
 template <int K, int CT, int NT>
 struct XpfStep {
     static constexpr int TW = EXL3_TILE_WORDS(K, false);
     static constexpr bool one_shift = 16 + 3 * K <= 32;
-    u32 w1[8][2], w0[one_shift ? 1 : 8][2];
+    static constexpr int W = CT < 4 ? CT : 4;   // column tiles of a step
+    u32 w1[2 * W][2], w0[one_shift ? 1 : 2 * W][2];
     static __device__ __forceinline__ void window(u32 e, u32& om, u32& op, u32& sh) {
         op = (e - 1) >> 5;
         om = op == 0 ? TW - 1 : op - 1;
         sh = 31 - ((e - 1) & 31);
     }
     static __device__ __forceinline__ u32 first(u32 lane) { return 32 * (lane & 7) + 8 * (lane >> 4) + 4 * ((lane & 15) >> 3); }   // the lane's first weight
-    // step s of the unit at `row`: its tile rows 2 s and 2 s + 1 (CT = 4: the unit has four), or their column tiles 4 s .. 4 s + 3 (CT = 8)
+    // step s of the unit at `row`: its tile rows 2 s and 2 s + 1 (CT = 4, 2: the unit has four), or their column tiles 4 s .. 4 s + 3 (CT = 8)
     __device__ __forceinline__ void read(const u32* row, u32 s, u32 lane) {
         u32 om, op, sh;
-        row += s * (CT == 4 ? 8 : 4) * TW;
+        row += s * (CT == 8 ? 4 : 2 * CT) * TW;
         window((first(lane) + 4) * K, om, op, sh);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            w1[i][0] = row[(i / 4 * CT + i % 4) * TW + om];
-            w1[i][1] = row[(i / 4 * CT + i % 4) * TW + op];
+        for (int i = 0; i < 2 * W; i++) {
+            w1[i][0] = row[(i / W * CT + i % W) * TW + om];
+            w1[i][1] = row[(i / W * CT + i % W) * TW + op];
         }
         if constexpr (!one_shift) {
             window((first(lane) + 2) * K, om, op, sh);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                w0[i][0] = row[(i / 4 * CT + i % 4) * TW + om];
-                w0[i][1] = row[(i / 4 * CT + i % 4) * TW + op];
+            for (int i = 0; i < 2 * W; i++) {
+                w0[i][0] = row[(i / W * CT + i % W) * TW + om];
+                w0[i][1] = row[(i / W * CT + i % W) * TW + op];
             }
         }
     }
@@ -1663,11 +1668,11 @@ struct XpfStep {
         window((first(lane) + 4) * K, om, op, sh1);
         if constexpr (!one_shift) window((first(lane) + 2) * K, om, op, sh0);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < W; c++) {
             u32 b[2][2];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const int i = 4 * h + c;
+                const int i = W * h + c;
                 const u32 hi = __builtin_amdgcn_alignbit(w1[i][0], w1[i][1], sh1);
                 u32 s0, s1;
                 if constexpr (one_shift) {
@@ -1749,6 +1754,57 @@ __device__ __forceinline__ void xpf_stream(const R& ring, const u32* wb, const u
     }
 }
 
+// The same for waves of 32 columns, four to a projection: a unit has half the tiles and the waves of a compute unit are twice as many.  For short
+// chunks, whose items leave a SIMD one or two waves of 64 columns: such a wave spends half of its time on what comes between the decodes.
+template <int K, int NT, int NB, class R>
+__device__ __forceinline__ void xpf_stream_n(const R& ring, const u32* wb, const u16* __restrict__ src, u16* stage, u32 slot_u16, u32 tiles, u32 part, u32 lane, f32x4 (&acc)[NT][2]) {
+    constexpr int D = R::D, LEAST = NT <= 2 ? NT : NT - 1, A = 2 * LEAST / 4;   // A: loads of a unit's operand rows that every wave makes at least
+    static_assert(D + 1 >= NB && R::UR == 4, "operand rows are requested no earlier than the trellis rows of their unit");
+    auto request = [&](u32 unit, u32 slot) {
+        const u8* from = (const u8*) (src + (u64) unit * tiles * XPF_HALF_U16) + lane * 16;
+        const u32 to = __builtin_amdgcn_readfirstlane(lds_offset(stage + slot * slot_u16));
+        for (u32 i = part; i < 2 * tiles; i += 4) lds_load<16>(from + i * 1024, to + i * 1024);
+    };
+#pragma unroll
+    for (int T = 0; T < NT; T++) acc[T][0] = acc[T][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = -D; i < 0; i++) {
+        if ((u32) (i + D) < ring.units) ring.issue(i + D, i + D, lane);
+        if (i + NB - 1 >= 0 && (u32) (i + NB - 1) < ring.units) request(i + NB - 1, i + NB - 1);
+    }
+    auto ready = [&](u32 unit) {
+        if (unit + D <= ring.units) wait_vm<(NB - 2) * (R::NI + A)>();
+        else wait_vm<0>();
+        lds_barrier();
+    };
+    typedef XpfStep<K, 2, NT> Step;
+    Step s0, s1;
+    u32x4 x0[NT], x1[NT];
+    ready(0);
+    s0.read(wb, 0, lane);
+    Step::rows(x0, stage + lane * 8, XPF_HALF_U16);
+    u32 slot = 0, at = 0;
+#pragma unroll 1
+    for (u32 unit = 0; unit < ring.units; unit++) {
+        s1.read(wb + slot * R::UW, 1, lane);
+        Step::rows(x1, stage + at * slot_u16 + 512 + lane * 8, XPF_HALF_U16);
+        __builtin_amdgcn_sched_barrier(0);
+        s0.template products<0>(x0, acc, lane);
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the unit's words are in registers, its slot can take the unit D further on
+        if (unit + D < ring.units) ring.issue(unit + D, slot, lane);
+        if (unit + NB - 1 < ring.units) request(unit + NB - 1, at == 0 ? NB - 1 : at - 1);
+        slot = slot + 1 == (u32) D ? 0u : slot + 1;
+        at = at + 1 == (u32) NB ? 0u : at + 1;
+        if (unit + 1 < ring.units) {
+            ready(unit + 1);
+            s0.read(wb + slot * R::UW, 0, lane);
+            Step::rows(x0, stage + at * slot_u16 + lane * 8, XPF_HALF_U16);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        s1.template products<0>(x1, acc, lane);
+    }
+}
+
 // What launch 2 makes of a token tile's sums over the inputs (g, u: gate and up of a 128-block, in true units but for the output side):
 // output sides, act = silu(gate) * up times the down projection's input scales, its rotation, as operand rows.  The token's power of
 // two for this block is a multiple of 8 in the exponent, so that blocks mostly share one; inv undoes it.
@@ -1796,19 +1852,15 @@ __device__ __forceinline__ void xpf_chain(float* f, u32 fbs, Drop drop) {
     }
 }
 
-// A workgroup's sums through LDS (x: [block of 128 columns][of R tiles][register][lane]), so that a wave has all 128 columns of a
-// token tile: the wave of columns 64 half .. of block `at` leaves tile T in place R at + i.
-__device__ __forceinline__ void xpf_leave(f32x4* x, u32 place, u32 half, const f32x4 (&acc)[4], u32 lane) {
-#pragma unroll
-    for (u32 c = 0; c < 4; c++) x[(place * 8 + half * 4 + c) * 64 + lane] = acc[c];
-}
+// A workgroup's sums came through LDS (x: [block of 128 columns][of R tiles][register][lane]), so that a wave has all 128 columns of a
+// token tile.
 __device__ __forceinline__ void xpf_take(const f32x4* x, u32 place, f32x4 (&v)[8], u32 lane) {
 #pragma unroll
     for (u32 c = 0; c < 8; c++) v[c] = x[(place * 8 + c) * 64 + lane];
 }
 
-// Launch 2: an item (of up to tok pairs) and NCB 128-column blocks of ff, four waves a block (gate's two halves, up's).  rows2:
-// [tile][128-block of ff], inv2: [tile][128-block][16].  grid = xpf_place's, of ff / 128 / NCB parts, block 256 NCB; dynamic LDS: NB
+// Launch 2: an item (of up to tok pairs) and NCB 128-column blocks of ff: two, with two waves a projection and block (NCB = 2), or one, with four.  rows2:
+// [tile][128-block of ff], inv2: [tile][128-block][16].  grid = xpf_place's, of ff / 128 / NCB parts, block 512; dynamic LDS: NB
 // slots of two projections' NT tiles and the waves' rings (for the NT of 1, 2, 4, 6, 8 that takes most), or the exchange of the sums, 64
 // KiB NCB for four tiles.
 template <int K, int NCB>
@@ -1816,8 +1868,9 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
                                                             const u16* __restrict__ rows, const float* __restrict__ inv, u16* __restrict__ rows2, float* __restrict__ inv2, u32 ne, u32 hidden,
                                                             u32 ff, u32 tok) {
     extern __shared__ __attribute__((aligned(16))) u32 dyn[];
+    constexpr int CT = NCB == 2 ? 4 : 2;   // column tiles a wave
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const u32 sel = wave / (2 * NCB), part = wave % (2 * NCB), b = part / 2, half = part & 1;
+    const u32 sel = wave / 4, part = wave % 4, b = NCB == 2 ? part / 2 : 0, at = NCB == 2 ? part & 1 : part;   // at: which of the block's waves
     const u32 kbs = hidden / 128, fbs = ff / 128;
     u32 group;
     const u32 item = xpf_place(fbs / NCB, group), cb = group * NCB + b;
@@ -1829,15 +1882,17 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
     const u8* bd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
     xpf_tiles<NCB == 2 ? XPF_NT(K) : XPF_NT_N>(it.tiles, [&](auto n) {
         constexpr int NT = decltype(n)::value, G = NT < 4 ? NT : 4;
-        typedef VerifyRing<K, false, 4, NCB == 2 ? XPF_RING_W(K, NT) : XPF_RING_N(K, NT)> R;
+        typedef VerifyRing<K, false, CT, NCB == 2 ? XPF_RING_W(K, NT) : XPF_RING_N(K, NT), 4 * CT> R;
         constexpr int NB = NCB == 2 && NT >= 6 ? 3 : R::D + 1;
         u32* wb = dyn + NB * 2 * NT * (XPF_HALF_U16 / 2) + wave * (R::D * R::UW);
         R ring;
-        ring.init((sel ? bu : bg) + 2 * (u64) hidden + 2 * (u64) ff + 4 + (u64) (cb * 8 + half * 4) * (4 * R::TW), (ff / 16) * (4 * R::TW), 2 * kbs,
+        ring.init((sel ? bu : bg) + 2 * (u64) hidden + 2 * (u64) ff + 4 + (u64) (cb * 8 + at * CT) * (4 * R::TW), (ff / 16) * (4 * R::TW), 2 * kbs,
                   __builtin_amdgcn_readfirstlane(lds_offset(wb)), lane);
-        f32x4 acc[NT][4];
-        xpf_stream<K, NT, NB, 2 * NCB>(ring, wb, rows + ((u64) it.base * 2 + sel * it.tiles) * kbs * XPF_ROWS_U16, (u16*) dyn + sel * NT * XPF_HALF_U16, 2 * NT * XPF_HALF_U16, it.tiles, part, lane,
-                                       acc);
+        f32x4 acc[NT][CT];
+        const u16* src = rows + ((u64) it.base * 2 + sel * it.tiles) * kbs * XPF_ROWS_U16;
+        u16* stage = (u16*) dyn + sel * NT * XPF_HALF_U16;
+        if constexpr (NCB == 2) xpf_stream<K, NT, NB, 4>(ring, wb, src, stage, 2 * NT * XPF_HALF_U16, it.tiles, part, lane, acc);
+        else xpf_stream_n<K, NT, NB>(ring, wb, src, stage, 2 * NT * XPF_HALF_U16, it.tiles, part, lane, acc);
         const float* iv = inv + (it.base * 2 + sel * it.tiles) * 16 + (lane & 15);
         f32x4* x = (f32x4*) dyn;
 #pragma unroll
@@ -1847,12 +1902,14 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
             for (int i = 0; i < G && T0 + i < NT; i++) {
                 const float f = iv[16 * min((u32) (T0 + i), it.tiles - 1)];
 #pragma unroll
-                for (int c = 0; c < 4; c++) acc[T0 + i][c] *= f;
-                xpf_leave(x, (b * 2 + sel) * G + i, half, acc[T0 + i], lane);
+                for (int c = 0; c < CT; c++) {
+                    acc[T0 + i][c] *= f;
+                    x[(((b * 2 + sel) * G + i) * 8 + at * CT + c) * 64 + lane] = acc[T0 + i][c];
+                }
             }
             lds_barrier();
-            // four waves a block: one a tile
-            const u32 i = part - 2 * b + 2 * sel, T = T0 + i;
+            // a wave a tile and block
+            const u32 i = NCB == 2 ? part - 2 * b + 2 * sel : wave, T = T0 + i;
             if (i < (u32) G && T < it.tiles) {
                 f32x4 g[8], u[8];
                 xpf_take(x, (b * 2) * G + i, g, lane);
@@ -2012,7 +2069,7 @@ __device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__
                                                                                   float* inv2, u32 ne, u32 hidden, u32 ff, u32 tok) { \
         prefill_gate_up_exl3_kernel<K, 2>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff, tok); \
     } \
-    extern "C" __global__ void __launch_bounds__(256, 2) prefill_gate_up_n_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
+    extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_n_exl3_##K(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* items, const u16* rows, const float* inv, u16* rows2, \
                                                                                     float* inv2, u32 ne, u32 hidden, u32 ff, u32 tok) { \
         prefill_gate_up_exl3_kernel<K, 1>(eaddr, sh_addr, offs, items, rows, inv, rows2, inv2, ne, hidden, ff, tok); \
     } \

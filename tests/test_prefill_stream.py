@@ -128,3 +128,19 @@ def test_prefill_streams_of_eight_waves_as_deep_as_their_tiles_leave_room(tmp_pa
     subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
     r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_prefill_streams_of_narrow_waves(tmp_path):
+    """The same for the workgroups of one 128-block, whose waves take 32 columns, four to a projection."""
+    src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
+    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_N", "XPF_HALF_U16"))
+    start = src.index("template <int K, int NT, int NB, class R>")
+    stream = src[start:src.index("\n}\n", start) + 3]
+    harness = HARNESS.replace("xpf_stream<K, NT, NB, NW>(", "xpf_stream_n<K, NT, NB>(").replace("f32x4 acc[NT][4];", "f32x4 acc[NT][2];").replace("Ring<D, (2 * K + 3) / 4> R;", "Ring<D, (K + 3) / 4> R;")
+    harness = harness.replace("stream<K, NT, 3, 4, XPF_RING(K)>(\"eight waves\");", "").replace("XPF_RING_N(K, NT) + 1, 2, XPF_RING_N(K, NT)", "XPF_RING_N(K, NT) + 1, 4, XPF_RING_N(K, NT)")
+    assert harness.count("xpf_stream_n<") == 1 and harness.count("eight waves") == 0 and "+ 1, 4, XPF_RING_N" in harness
+    path = tmp_path / "stream.cpp"
+    path.write_text(harness % {"macros": macros, "stream": stream})
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
+    r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
