@@ -1185,10 +1185,14 @@ int32_t sz_head_top(sz_session* s, uint32_t m, uint64_t u, uint32_t* top_host, u
         if (launch("topk_merge", m, 1, 1, 1024, 0, stream, b)) return 1;
         return top_finish(s, m, top_host, stream);
     }
-    if (s->logits.need((uint64_t) c.max_rows * c.vocab * 4) || s->topv.need((uint64_t) c.max_rows * nb * 64 * 4) ||
-        s->topi.need((uint64_t) c.max_rows * nb * 64 * 4))
-        return 1;
+    if (s->logits.need((uint64_t) c.max_rows * c.vocab * 4)) return 1;
     if (head_logits(s, m, u, s->logits.ptr, stream)) return 1;
+    if (head_is_exl3(s)) {   // its blocks' largest logits say which blocks hold the 64
+        const sz_arg a[] = {P(s->logits.ptr), U32(c.vocab), P(s->head_part.ptr), U32(c.vocab / 128), P(topo)};
+        if (launch("topk_blocks", m, 1, 1, 1024, 0, stream, a)) return 1;
+        return top_finish(s, m, top_host, stream);
+    }
+    if (s->topv.need((uint64_t) c.max_rows * nb * 64 * 4) || s->topi.need((uint64_t) c.max_rows * nb * 64 * 4)) return 1;
     const sz_arg a[] = {P(s->logits.ptr), U32(c.vocab), U32(c.vocab), U32(nb), P(s->topv.ptr), P(s->topi.ptr)};
     if (launch("topk_slices", m * nb, 1, 1, 1024, 0, stream, a)) return 1;
     const sz_arg b[] = {P(s->topv.ptr), P(s->topi.ptr), U32(nb), P(topo)};

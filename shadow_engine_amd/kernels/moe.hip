@@ -336,6 +336,77 @@ __device__ __forceinline__ u64 tk_best_of_4096(u32 n, F key, u64* sh) {
     return (blockDim.x >> 6) == 16 ? tk_best_of<64, 4>(n, key, sh) : tk_best_of<64, 16>(n, key, sh);
 }
 
+// Row r = blockIdx.x of a head that left the largest logit of every block of 128 and its id in part[(block * 8 + r) * 2 ..]: the 64 best of its
+// nob * 128 logits (nob <= 2048) into out[r*128 .. +64) (value bits) and out[r*128 + 64 .. +64) (ids).  Whatever is among them is at least
+// as good as the 64th best of the blocks' largest, and lies in one of those 64 blocks: the blocks' keys are sorted, those blocks' logits
+// read, and what is as good, 64 and a few as a rule, sorted.  Up to 128 such keys a wave sorts alone, up to 2048 the workgroup; where
+// there are more (equal logits) it sorts all 8192.  Bound by its chain of dependent steps, four rows of 151 936 logits 8.3 us, where topk_slices, which sorts all of them, and topk_merge
+// take 9.9 + 7.1.  grid = rows, block 1024.
+extern "C" __global__ void __launch_bounds__(1024) topk_blocks(const float* logits, u32 stride, const u32* part, u32 nob, u32* out) {
+    __shared__ u64 sh[1024], s_key[2048], s_least;
+    __shared__ u32 s_block[64], s_n;
+    const u32 r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float* row = logits + (u64) r * stride;
+    u64 best = tk_best_of<32, 2>(nob, [&](u32 t) { return tk_key(bits_f32(part[((u64) t * 8 + r) * 2]), part[((u64) t * 8 + r) * 2 + 1]); }, sh);
+    if (tid < 64) {
+        float x;
+        u32 id;
+        tk_unkey(best, x, id);
+        s_block[tid] = id / 128;                       // of nothing (fewer than 64 blocks): past every block
+        if (tid == 63) s_least = best;
+        if (tid == 0) s_n = 0;
+    }
+    __syncthreads();
+    const u64 least = s_least;
+    {
+        // four blocks a wave, every load out before the first is waited for
+        float v[8];
+        u64 k[8];
+        u32 base[8], found = 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = row[min(s_block[4 * wave + i / 2], nob - 1) * 128 + 64 * (i & 1) + lane];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const u32 b = s_block[4 * wave + i / 2];
+            k[i] = tk_key(v[i], b * 128 + 64 * (i & 1) + lane);
+            if (k[i] < least || b >= nob) k[i] = 0;
+            const u64 in = __builtin_amdgcn_ballot_w64(k[i] != 0);
+            base[i] = found + __builtin_popcountll(in & ((1ull << lane) - 1));
+            found += __builtin_popcountll(in);
+        }
+        u32 at = 0;
+        if (lane == 0) at = atomicAdd(&s_n, found);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (k[i] != 0 && at + base[i] < 2048) s_key[at + base[i]] = k[i];
+    }
+    __syncthreads();
+    const u32 n = s_n;
+    if (n <= 128) {
+        if (wave) return;
+        u64 a = lane < n ? s_key[lane] : TK_NOTHING, b = lane + 64 < n ? s_key[lane + 64] : TK_NOTHING;
+        tk_sort64<false>(a, lane);
+        tk_sort64<true>(b, lane);
+        best = tk_larger(a, b);
+        tk_merge<64, true>(best, lane);
+    } else if (n <= 2048) {
+        best = tk_best_of<32, 2>(n, [&](u32 t) { return s_key[t]; }, sh);
+    } else {
+        best = tk_best_of<128, 8>(8192, [&](u32 t) {
+            const u32 b = s_block[t / 128];
+            return b < nob ? tk_key(row[b * 128 + t % 128], b * 128 + t % 128) : TK_NOTHING;
+        }, sh);
+    }
+    if (tid < 64) {
+        float x;
+        u32 id;
+        tk_unkey(best, x, id);
+        out[r * 128 + tid] = f32_bits(x);
+        out[r * 128 + 64 + tid] = id;
+    }
+}
+
 // Slice b of row r (blockIdx.x = r * nb + b): the 64 best of logits[r*stride + 4096 b .. +4096) into sv/si[(r*nb + b)*64 ..].
 // Slots past the vocabulary hold (-inf, 0xffffffff).  grid = rows * nb, block 1024 or 256.
 extern "C" __global__ void __launch_bounds__(1024) topk_slices(const float* logits, u32 vocab, u32 stride, u32 nb, float* sv, u32* si) {

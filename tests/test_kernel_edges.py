@@ -631,3 +631,38 @@ def test_grouping_of_more_pairs_than_one_workgroup_lists(gpu, tokens, k):  # noq
         s.moe_prefill_chunk(0, min(300, tokens - t0), dx[t0:].data_ptr(), dl[t0:].data_ptr(), dg[t0:].data_ptr(), cut[t0:].data_ptr())
     gpu.cuda.synchronize()
     assert gpu.isfinite(whole).all() and np.array_equal(bits(whole.cpu().numpy()), bits(cut.cpu().numpy()))
+
+
+@pytest.mark.parametrize("nob", [1, 2, 63, 64, 65, 130, 1187, 2048])
+def test_the_64_best_from_the_blocks_largest(gpu, nob):  # noqa: F811
+    """Fewer than 64 blocks of 128 logits to the most: random rows, rows whose best lie in few blocks (128 to 2048 as good as the 64th block's
+    largest, and more), equal logits, zeros of both signs, infinities, NaN and nothing but -inf: values and ids as the
+    oracle's sort gives them."""
+    rng = np.random.default_rng(nob)
+    n, rows = nob * 128, np.empty((8, nob * 128), np.float32)
+    rows[0] = rng.normal(size=n)
+    rows[1] = rng.normal(size=n) + 8 * (np.arange(n) // 128 % 97 == 5)
+    rows[2] = rng.normal(size=n) * (1 + 30 * (np.arange(n) // 128 >= nob - 20))
+    rows[3] = 1.25
+    rows[4] = rng.integers(-3, 1, n) * 0.5
+    rows[4, 3::11] = -0.0
+    rows[5] = np.where(rng.random(n) < 0.01, np.nan, rng.normal(size=n))
+    rows[5, rng.integers(0, n, 3)] = np.inf, -np.inf, np.inf
+    rows[6] = -np.inf
+    rows[6, rng.integers(0, n, 40)] = rng.normal(size=40)
+    rows[7] = np.where(rng.random(n) < 0.5, np.nan, -np.inf)
+    part = np.zeros((nob, 8, 2), np.uint32)
+    clean = np.where(np.isnan(rows), -np.inf, rows).astype(np.float32).reshape(8, nob, 128)
+    best = clean.argmax(axis=2)                              # the lowest id on ties
+    part[:, :, 0] = bits(np.take_along_axis(clean, best[:, :, None], 2)[:, :, 0]).T
+    part[:, :, 1] = (best + np.arange(nob) * 128).T
+    dl, dp = dev(gpu, rows), dev(gpu, part.view(np.int32))
+    out = gpu.zeros(8 * 128, dtype=gpu.int32, device="cuda")
+    A = sz.Arg
+    sz.launch("topk_blocks", (8, 1, 1), (1024, 1, 1), 0, 0, [A.ptr(dl.data_ptr()), A.u32(n), A.ptr(dp.data_ptr()), A.u32(nob), A.ptr(out.data_ptr())])
+    gpu.cuda.synchronize()
+    words = out.cpu().numpy().view(np.uint32).reshape(8, 128)
+    for r in range(8):
+        vals, ids = O.topk(rows[r], 64)
+        assert np.array_equal(words[r, 64:], ids), f"row {r}"
+        assert np.array_equal(words[r, :64], bits(vals)), f"row {r}"
