@@ -244,26 +244,33 @@ extern "C" __global__ void __launch_bounds__(1024) prefill_group_many(const u32*
     prefill_group_body<true>(tidx, tokens, k, ne, nshared, offs, list, items, items_d, unit_gu, unit_d, share);
 }
 
-__shared__ u32x2 pf_grid[512];   // the codebook grid, a weight's magnitude as f16
+// A workgroup's LDS.  The grid comes first: its address fits the look-ups' constant offset.
+#define PF_STAGE 73728
+struct PfLds {
+    u32x2 grid[512];   // the codebook grid, a weight's magnitude as f16
+    u8 stage[PF_STAGE];
+    u32 rows[PF_TOK], pairs[PF_TOK];
+    float strip[8][16];
+};
 
 // Fills the table; every thread of the workgroup (512) calls it, and a barrier must follow before it is read.
-__device__ __forceinline__ void pf_tables(u32 tid) {
+__device__ __forceinline__ void pf_tables(u32x2* grid, u32 tid) {
     const u32 g = IQ3S_GRID[tid];
-    pf_grid[tid] = u32x2{f16_pair((float) (g & 0xff), (float) ((g >> 8) & 0xff)), f16_pair((float) ((g >> 16) & 0xff), (float) (g >> 24))};
+    grid[tid] = u32x2{f16_pair((float) (g & 0xff), (float) ((g >> 8) & 0xff)), f16_pair((float) ((g >> 16) & 0xff), (float) (g >> 24))};
 }
 
 // Eight consecutive weights (k = 8 kq .. 8 kq + 7 of sub-block g) of one IQ3_S block at `blk` (LDS, 2-byte aligned) as f16: grid * sign
 // (cpu_expert.rs:99-110) * (1 + 2 scale), `scale` holding the last factor twice; qh: bits 0 and 1 the ninth bits of the two grid indexes.  The two
 // signs of a pair are moved to the sign bits of its halves by one multiplication (the two copies of the sign byte that it
 // makes do not overlap).
-__device__ __forceinline__ f16x8 iq3s_f16x8(const u8* blk, u32 g, u32 kq, u32 qh, f16x2 scale) {
+__device__ __forceinline__ f16x8 iq3s_f16x8(const u32x2* grid, const u8* blk, u32 g, u32 kq, u32 qh, f16x2 scale) {
     const u32 qs = *(const u16*) (blk + 2 + 8 * g + 2 * kq);   // the low bytes of the two 4-weight groups' grid indexes
     const u32 signs = blk[74 + 4 * g + kq];
     u32 at0 = (qs & 0xff) << 3 | ((qh << 11) & 0x800u), at1 = (qs >> 8) << 3 | ((qh << 10) & 0x800u);
     asm("" : "+v"(at0), "+v"(at1));   // bytes into the table, whose own address then is the loads' constant offset
-    const u32x2 g0 = *(const u32x2*) ((const u8*) pf_grid + at0), g1 = *(const u32x2*) ((const u8*) pf_grid + at1);
-    auto pair = [&](u32 grid, u32 spread) {
-        return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, grid) * __builtin_bit_cast(f16x2, ((signs * spread) & 0x80008000u) ^ __builtin_bit_cast(u32, scale)));
+    const u32x2 g0 = *(const u32x2*) ((const u8*) grid + at0), g1 = *(const u32x2*) ((const u8*) grid + at1);
+    auto pair = [&](u32 of, u32 spread) {
+        return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, of) * __builtin_bit_cast(f16x2, ((signs * spread) & 0x80008000u) ^ __builtin_bit_cast(u32, scale)));
     };
     return __builtin_bit_cast(f16x8, u32x4{pair(g0.x, 0x40008000u), pair(g0.y, 0x10002000u), pair(g1.x, 0x04000800u), pair(g1.y, 0x01000200u)});
 }
@@ -315,11 +322,11 @@ struct PfRows {
 // Half a block's products (128 weights, 4 sub-blocks) with the first T token tiles: acc += d_x * a sub-block's exact sum, in sub-block order.
 // xs, ds: the half's activations and their scales ([sub-block][64 tokens]); blk: the lane's row's block in LDS.
 template <int T>
-__device__ __forceinline__ void pf_products(f32x4 (&acc)[T], const u8* xs, const float* ds, const u8* blk, u32 half, u32 n, u32 kq) {
+__device__ __forceinline__ void pf_products(f32x4 (&acc)[T], const u32x2* grid, const u8* xs, const float* ds, const u8* blk, u32 half, u32 n, u32 kq) {
     f16x8 w[4];
     const u32 qh = ((u32) *(const u16*) (blk + 66 + 4 * half) | (u32) *(const u16*) (blk + 68 + 4 * half) << 16) >> (2 * kq);
 #pragma unroll
-    for (int j = 0; j < 4; j++) w[j] = iq3s_f16x8(blk, 4 * half + j, kq, qh >> (8 * j), iq3s_scale_pair(blk[106 + 2 * half + j / 2], 4 * (j % 2)));
+    for (int j = 0; j < 4; j++) w[j] = iq3s_f16x8(grid, blk, 4 * half + j, kq, qh >> (8 * j), iq3s_scale_pair(blk[106 + 2 * half + j / 2], 4 * (j % 2)));
     __builtin_amdgcn_sched_barrier(0);
     // a step is a tile and sub-block: its operands are read a step ahead, its sums scaled while the next one's are made
     auto read = [&](int step, f16x8& x, float& dx) {
@@ -373,16 +380,17 @@ __device__ __forceinline__ void pf_fold(f32x4 (&total)[T], f32x4 (&acc)[T], cons
 // waits); for three and four the activations come a half block at a time, one ahead, the rows a block ahead.  Two workgroups a
 // compute unit by the stage's LDS.
 //
-// What bounds it: the decode, about 27 vector instructions for a lane's 8 weights, for every item of an expert again, then LDS (the grid
-// look-ups' bank conflicts) and the waits of items of one tile.  512 tokens through 512 experts of 2048 x 512, top-10, router with
-// Zipf's preferences: gate and up 138 -> 112 us, down 82 -> 61, the chunk 229 -> 173; 4096 tokens and the shared expert 1092 -> 847; 700
-// through 60 of 4096 x 1536, top-4, 582 -> 420.  Gate and up of 16 rows in one wave, which reads the activations half as often,
-// spilled registers (230 us).
-#define PF_STAGE 73728
+// What bounds it: the decode, about 24 vector instructions for a lane's 8 weights, for every item of an expert again, then LDS, busy half the time
+// (the grid look-ups' bank conflicts), and the waits of items of one tile.  512 tokens through 512 experts of 2048 x 512, top-10, router
+// with Zipf's preferences: gate and up 138 -> 111 us, down 82 -> 61, the chunk 229 -> 169; 4096 tokens and the shared expert 1092 ->
+// 843; 700 through 60 of 4096 x 1536, top-4, 582 -> 418.  Tried: 16 rows of either matrix and half the sub-blocks a wave, which reads
+// the activations half as often (gate and up 112, down 78).
 template <int T, class F>
-__device__ __forceinline__ void pf_stream(u8* stage, u64 w0, u64 w1, u64 lot, u32 rb, u32 nc, u32 blocks, const u16* __restrict__ x, const float* __restrict__ d, const u32* s_rows, u32 cols,
-                                          float* strip, u32 wave, u32 lane, F&& finish) {
+__device__ __forceinline__ void pf_stream(PfLds& lds, u64 w0, u64 w1, u64 lot, u32 rb, u32 nc, u32 blocks, const u16* __restrict__ x, const float* __restrict__ d, const u32* s_rows, u32 cols,
+                                          u32 wave, u32 lane, F&& finish) {
     constexpr u32 XB = T * 4096;   // half a block's activations: [16 T tokens][16 columns of 8 codes]
+    u8* stage = lds.stage;
+    float* strip = lds.strip[wave];
     const u32 n = lane & 15, kq = lane >> 4, lrow = (wave & 3) * 16 + n, mine = wave >> 2, lds0 = __builtin_amdgcn_readfirstlane(lds_offset(stage));
     PfRows rows;
     rows.init(rb, wave, lane);
@@ -451,8 +459,8 @@ __device__ __forceinline__ void pf_stream(u8* stage, u64 w0, u64 w1, u64 lot, u3
             if (ahead < blocks) request(slot == 0 ? D - 1 : slot - 1);
             slot = slot + 1 == D ? 0u : slot + 1;
             const u8* blk = s + WO + mine * PF_WB + lrow * PF_WS + pf_shift(at, rb, lrow);
-            pf_products<T>(acc, s, (const float*) (s + DO), blk, 0, n, kq);
-            pf_products<T>(acc, s + XB, (const float*) (s + DO + 1024), blk, 1, n, kq);
+            pf_products<T>(acc, lds.grid, s, (const float*) (s + DO), blk, 0, n, kq);
+            pf_products<T>(acc, lds.grid, s + XB, (const float*) (s + DO + 1024), blk, 1, n, kq);
             fold(blk);
         }
     } else {
@@ -477,7 +485,7 @@ __device__ __forceinline__ void pf_stream(u8* stage, u64 w0, u64 w1, u64 lot, u3
             __syncthreads();   // the block and its first half's activations are in LDS, from every wave; block b - 1 is done with
             inputs(2 * c + 1, 1);
             if (b + 1 < blocks) rows.issue<false>(a0, to, wave);
-            pf_products<T>(acc, stage, (const float*) (stage + DO), blk, 0, n, kq);
+            pf_products<T>(acc, lds.grid, stage, (const float*) (stage + DO), blk, 0, n, kq);
             wait_vm<0>();
             __syncthreads();
             if (b + 1 < blocks) {
@@ -485,7 +493,7 @@ __device__ __forceinline__ void pf_stream(u8* stage, u64 w0, u64 w1, u64 lot, u3
                 rows.issue<true>(a1, to + PF_WB, wave);
                 next();
             }
-            pf_products<T>(acc, stage + XB, (const float*) (stage + DO + 1024), blk, 1, n, kq);
+            pf_products<T>(acc, lds.grid, stage + XB, (const float*) (stage + DO + 1024), blk, 1, n, kq);
             fold(blk);
         }
     }
@@ -510,10 +518,10 @@ extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const
                                                                         const u32* items, const u16* xh, const float* xd, i8* hq, u16* hh, float* hd, u32 ne,
                                                                         u32 k, u32 npairs, u32 hidden, u32 ff) {
     constexpr u32 HP = 68;
-    __shared__ __attribute__((aligned(16))) u8 stage[PF_STAGE];   // afterwards the item's 64 x 64 block of H
-    __shared__ u32 s_rows[PF_TOK], s_pairs[PF_TOK];
-    __shared__ __attribute__((aligned(16))) float s_strip[8][16];
-    static_assert(sizeof(stage) >= 2 * PF_TOK * HP * sizeof(float), "H and the up sums reuse the staging area");
+    __shared__ __attribute__((aligned(16))) PfLds lds;   // the stages are afterwards the item's 64 x 64 block of H
+    u8* stage = lds.stage;
+    u32 *s_rows = lds.rows, *s_pairs = lds.pairs;
+    static_assert(sizeof(lds.stage) >= 2 * PF_TOK * HP * sizeof(float), "H and the up sums reuse the staging area");
     const u32 tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const u32 n = lane & 15, kq = lane >> 4, rbx = blockIdx.x;
     const u32 rb = hidden / 256 * 110;
@@ -521,7 +529,7 @@ extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const
     const u32 e = items[1 + 2 * blockIdx.y], t0 = items[2 + 2 * blockIdx.y];
     if (e == ne && !sh_addr) return;
     const u32 first = offs[e], nt = min((u32) PF_TOK, offs[e + 1] - first - t0);
-    pf_tables(tid);
+    pf_tables(lds.grid, tid);
     const u64 wg = uniform_u64(e < ne ? eaddr[e] : sh_addr[0]) + (u64) rbx * 64 * rb, wu = uniform_u64(e < ne ? eaddr[(u64) ne + e] : sh_addr[1]) + (u64) rbx * 64 * rb;
     if (tid < PF_TOK) {   // a place past the item's end has row 0, whose products are dropped
         const u32 p = tid < nt ? list[first + t0 + tid] : 0;
@@ -533,7 +541,7 @@ extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const
     float (*us)[HP] = (float (*)[HP]) (stage + PF_TOK * HP * sizeof(float));
     pf_tiles(nt, [&](auto tiles) {
         constexpr int T = decltype(tiles)::value;
-        pf_stream<T>(stage, wg, wu, 0, rb, hidden / 256, hidden / 256, xh, xd, s_rows, hidden, s_strip[wave], wave, lane, [&](u32, f32x4 (&sums)[T]) {
+        pf_stream<T>(lds, wg, wu, 0, rb, hidden / 256, hidden / 256, xh, xd, s_rows, hidden, wave, lane, [&](u32, f32x4 (&sums)[T]) {
             // the staging area becomes H [token][feature]: up's sums go to the waves that hold gate's
             __syncthreads();
             if (wave >= 4) {
@@ -589,9 +597,8 @@ extern "C" __global__ void __launch_bounds__(512, 4) prefill_gate_up_iq3_s(const
 extern "C" __global__ void __launch_bounds__(512, 4) prefill_down_iq3_s(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list,
                                                                      const u32* items, const u16* hh, const float* hd, float* eo, u32 ne, u32 hidden,
                                                                      u32 ff) {
-    __shared__ __attribute__((aligned(16))) u8 stage[PF_STAGE];
-    __shared__ u32 s_pairs[PF_TOK];
-    __shared__ __attribute__((aligned(16))) float s_strip[8][16];
+    __shared__ __attribute__((aligned(16))) PfLds lds;
+    u32* s_pairs = lds.pairs;
     const u32 tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const u32 n = lane & 15, kq = lane >> 4;
     const u32 rb = ff / 256 * 110, per = hidden / 128 / gridDim.x, lot0 = blockIdx.x * per;
@@ -599,13 +606,13 @@ extern "C" __global__ void __launch_bounds__(512, 4) prefill_down_iq3_s(const u6
     const u32 e = items[1 + 2 * blockIdx.y], t0 = items[2 + 2 * blockIdx.y];
     if (e == ne && !sh_addr) return;
     const u32 first = offs[e], nt = min((u32) PF_TOK, offs[e + 1] - first - t0);
-    pf_tables(tid);
+    pf_tables(lds.grid, tid);
     const u64 wd = uniform_u64(e < ne ? eaddr[2ull * ne + e] : sh_addr[2]) + (u64) lot0 * 128 * rb;
     if (tid < PF_TOK) s_pairs[tid] = tid < nt ? list[first + t0 + tid] : 0;
     __syncthreads();   // s_pairs and the table are written
     pf_tiles(nt, [&](auto tiles) {
         constexpr int T = decltype(tiles)::value;
-        pf_stream<T>(stage, wd, wd + 64ull * rb, 128ull * rb, rb, ff / 256, per * (ff / 256), hh, hd, s_pairs, ff, s_strip[wave], wave, lane, [&](u32 lot, f32x4 (&sums)[T]) {
+        pf_stream<T>(lds, wd, wd + 64ull * rb, 128ull * rb, rb, ff / 256, per * (ff / 256), hh, hd, s_pairs, ff, wave, lane, [&](u32 lot, f32x4 (&sums)[T]) {
             const u32 row = (lot0 + lot) * 128 + wave * 16 + 4 * kq;
 #pragma unroll
             for (int a = 0; a < T; a++)
