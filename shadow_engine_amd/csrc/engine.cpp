@@ -1389,8 +1389,8 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
                                 U32(nd), U32(parts)};
             if (launch(((wide ? "prefill_down_" : "prefill_down_n_") + tag).c_str(), bound_d * parts, 1, 1, 64 * waves, 4 * (nd * fbs * 1040 + 256 * waves) + waves * ring * 512 * bits, stream, a)) return 1;
         }
-        const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden), U32(c.top_k)};
-        return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, tokens, 1, 256, 0, stream, a);
+        const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden / 4), U32(c.top_k)};
+        return launch("prefill_combine", c.hidden / 256, tokens, 1, 64, 0, stream, a);
     }
     const uint64_t max_items = c.n_expert + 1 + rows / 64;   // every expert's runs of up to 64 pairs: PF_TOK in kernels/prefill.hip
     if (pb.lay({{&pb.xq, T * c.hidden}, {&pb.xd, T * c.hidden / 32 * 4}, {&pb.tidx, np * 4}, {&pb.w, np * 4}, {&pb.cnt, T * 4}, {&pb.offs, (c.n_expert + 2) * 4ull}, {&pb.list, rows * 4},
@@ -1418,8 +1418,8 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
                             U32(c.hidden), U32(c.ff)};
         if (launch("prefill_down_iq3_s", blocks / per, (uint32_t) max_items, 1, 512, 0, stream, a)) return 1;
     }
-    const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden), U32(c.top_k)};
-    return launch("moe_combine_qwen_rows", (c.hidden + 255) / 256, tokens, 1, 256, 0, stream, a);
+    const sz_arg a[] = {P(y), P(pb.eo.ptr), P(pb.w.ptr), P(shared ? pb.eo.ptr + np * c.hidden * 4 : 0), P(sgl), P(pb.cnt.ptr), U32(c.hidden / 4), U32(c.top_k)};
+    return launch("prefill_combine", c.hidden / 256, tokens, 1, 64, 0, stream, a);
 }
 
 // The chunk's intermediate buffers, for tests: which = 0 xq (int8), 1 xd (f32), 2 tidx (u32), 3 w (f32), 4 hq (int8), 5 hd (f32),

@@ -666,3 +666,26 @@ def test_the_64_best_from_the_blocks_largest(gpu, nob):  # noqa: F811
         vals, ids = O.topk(rows[r], 64)
         assert np.array_equal(words[r, 64:], ids), f"row {r}"
         assert np.array_equal(words[r, :64], bits(vals)), f"row {r}"
+
+
+@pytest.mark.parametrize("k,n,shared", [(1, 256, False), (3, 260, True), (10, 2048, True), (16, 1028, False)])
+def test_chunk_combine_is_the_rows_combine(gpu, k, n, shared):  # noqa: F811
+    """Four outputs a lane, the same bits: widths that leave the last workgroup part empty, tokens with fewer experts than k
+    (whose other rows hold NaN), with and without the shared expert's row."""
+    rng = np.random.default_rng(n + k)
+    tokens = 7
+    cnt = rng.integers(0, k + 1, tokens).astype(np.int32)
+    cnt[0] = k
+    eo = rng.normal(size=(tokens, k, n)).astype(np.float32)
+    eo[np.arange(k)[None] >= cnt[:, None]] = np.nan
+    bufs = [dev(gpu, a) for a in (eo, rng.random((tokens, k)).astype(np.float32), rng.normal(size=(tokens, n)).astype(np.float32), rng.normal(size=tokens).astype(np.float32), cnt)]
+    A = sz.Arg
+    ys = []
+    for name, width, grid, block in (("moe_combine_qwen_rows", n, -(-n // 256), 256), ("prefill_combine", n // 4, -(-n // 256), 64)):
+        y = gpu.full((tokens + 1, n), 7.0, dtype=gpu.float32, device="cuda")
+        e, w, s, g, c = (b.data_ptr() for b in bufs)
+        sz.launch(name, (grid, tokens, 1), (block, 1, 1), 0, 0, [A.ptr(y.data_ptr()), A.ptr(e), A.ptr(w), A.ptr(s if shared else 0), A.ptr(g), A.ptr(c), A.u32(width), A.u32(k)])
+        gpu.cuda.synchronize()
+        ys.append(y.cpu().numpy())
+    assert np.isfinite(ys[0]).all() and (ys[0][tokens] == 7.0).all()
+    assert np.array_equal(bits(ys[0]), bits(ys[1]))
