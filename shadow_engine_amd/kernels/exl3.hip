@@ -1446,7 +1446,8 @@ __device__ __forceinline__ void xpf_put_transformed(u16* rows, u32 half_step, co
                 w[0][j] = r[0];
                 w[1][j] = r[1];
             }
-            *(u32x4*) (rows + h * half_step + ((b4 * 4 + a + 2 * b5) * 16 + n) * 8) = u32x4{w[0][0], w[0][1], w[1][0], w[1][1]};
+            const u32x4 o = {w[0][0], w[0][1], w[1][0], w[1][1]};
+            __builtin_nontemporal_store(o, (u32x4*) (rows + h * half_step + ((b4 * 4 + a + 2 * b5) * 16 + n) * 8));
         }
 }
 // The values as they lie before a transform or after two.
@@ -1514,7 +1515,9 @@ __device__ __forceinline__ void xpf_tiles(u32 tiles, F&& run) {
 // that from the largest product; else (a large input of a channel that the expert scales to next to nothing) the largest product, which
 // takes another pass over the inputs (such a pass for every token: 52 us of 4096 tokens' 920, 4 of 45 tokens' 121).
 // rows: an item's [gate, up][64-block][tile], inv: [gate, up][tile][16].
-// Bound by the rows it writes (8 bytes an input and pair).  grid = xpf_place's, of `tiles * shares` parts, block 256.
+// Bound by the rows it writes (8 bytes an input and pair), past the caches: the next launch begins with rows that were written long before (kept there:
+// 4096 tokens as above 857 us for the chunk, 844, 512 tokens 220, 218.5, 100 tokens 119, 118, 250 through 32 experts 84, 83).
+// grid = xpf_place's, of `tiles * shares` parts, block 256.
 extern "C" __global__ void __launch_bounds__(256) prefill_rotate_exl3(const u64* eaddr, const u64* sh_addr, const u32* offs, const u32* list, const u32* items, const float* x,
                                                                       const u32* most, u16* rows, float* inv, u32 ne, u32 k, u32 npairs, u32 hidden, u32 tok, u32 tiles, u32 shares) {
     __shared__ u32 s_scale[2][4], s_least[2][4];
