@@ -884,26 +884,39 @@ __device__ __forceinline__ void exl3_cols_kernel(const u8* __restrict__ w, const
                                s_mx, s_iv);
 }
 
-// y_j's 128-output block ob: the partial sums added up, the output-side transform, the scales.  grid = (out / 128, m), block 64.
+template <int N>
+struct ConstInt {
+    static constexpr int value = N;
+};
+// y_j's 128-output block ob: the partial sums added up, the output-side transform, the scales.  A chain of round trips, few waves: of many
+// partials sixteen are asked for at once (four at once: a call of 8192 x 16384 at 3 bits for 4 inputs 28.2 us, 26.5, for one 25.9, 23.8; 8192 x
+// 2048 at 2 bits 10.4, 9.5; two of 8192 x 32768 at 4 bits 46.6, 45.4).  grid = (out / 128, m), block 64.
 extern "C" __global__ void __launch_bounds__(64) exl3_finish_rows(const float* part, const u8* w, float* y, u32 ys, u32 in_f, u32 out_f) {
     const u32 lane = threadIdx.x, ob = blockIdx.x, j = blockIdx.y, zs = (in_f / 128 + 3) / 4;
     const u16* svh = (const u16*) (w + 2 * (u64) in_f) + ob * 128;
     const float s0 = f16_to_f32(svh[lane]), s1 = f16_to_f32(svh[lane + 64]);
     float v0 = 0.0f, v1 = 0.0f;
-    for (u32 z0 = 0; z0 < zs; z0 += 4) {
-        float a[4][2];   // four partials' loads in flight together
+    // `count` partials' loads in flight together, the last one's again past the end
+    auto add = [&](auto count, u32 z0) {
+        constexpr int N = decltype(count)::value;
+        float a[N][2];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < N; q++) {
             const float* p = part + ((u64) j * zs + min(z0 + q, zs - 1)) * out_f + ob * 128;
             a[q][0] = p[lane];
             a[q][1] = p[lane + 64];
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < N; q++)
             if (z0 + q < zs) {
                 v0 += a[q][0];
                 v1 += a[q][1];
             }
+    };
+    for (u32 z0 = 0; z0 < zs; z0 += 16) {
+        if (zs - z0 > 8) add(ConstInt<16>(), z0);
+        else if (zs - z0 > 4) add(ConstInt<8>(), z0);
+        else add(ConstInt<4>(), z0);
     }
     wht128_wave(v0, v1, lane);
     float* o = y + (u64) j * ys + ob * 128;
@@ -1491,21 +1504,17 @@ __device__ __forceinline__ u32 xpf_place(u32 parts, u32& part) {
 }
 // The products are compiled for 1, 2, 4, 6 and 8 token tiles: an item of 3, 5 or 7 has the next one's do for it, the last tile's
 // operand rows being whatever lies there.
-template <int N>
-struct XpfInt {
-    static constexpr int value = N;
-};
 template <int MOST, class F>
 __device__ __forceinline__ void xpf_tiles(u32 tiles, F&& run) {
-    if (tiles == 1) return run(XpfInt<1>());
-    if (tiles == 2) return run(XpfInt<2>());
+    if (tiles == 1) return run(ConstInt<1>());
+    if (tiles == 2) return run(ConstInt<2>());
     if constexpr (MOST > 6) {
-        if (tiles > 6) return run(XpfInt<8>());
+        if (tiles > 6) return run(ConstInt<8>());
     }
     if constexpr (MOST > 4) {
-        if (tiles > 4) return run(XpfInt<6>());
+        if (tiles > 4) return run(ConstInt<6>());
     }
-    run(XpfInt<4>());
+    run(ConstInt<4>());
 }
 
 // Launch 1: a tile (16 tokens) of an item and one of `shares` of the inputs' 128-blocks: wave w takes 4 share + w, from there 4 shares on, ..  A token's power of two takes a bound

@@ -689,3 +689,27 @@ def test_chunk_combine_is_the_rows_combine(gpu, k, n, shared):  # noqa: F811
         ys.append(y.cpu().numpy())
     assert np.isfinite(ys[0]).all() and (ys[0][tokens] == 7.0).all()
     assert np.array_equal(bits(ys[0]), bits(ys[1]))
+
+
+@pytest.mark.parametrize("zs", [1, 4, 5, 8, 9, 16, 17, 21, 33])
+def test_finish_adds_any_number_of_partials(gpu, zs):  # noqa: F811
+    """exl3_finish_rows: sums of 1 to 33 partials (an input's 512 and a rest of 128), three rows of two output blocks, against
+    64 bits.  zs - 1 additions, seven levels of the transform and its factor, a product: no more than zs + 9 roundings of 2^-24 of the
+    magnitudes that go in."""
+    rng = np.random.default_rng(zs)
+    in_f, out_f, m = 512 * (zs - 1) + 128, 256, 3
+    part = rng.normal(size=(m, zs, out_f)).astype(np.float32)
+    svh = rng.normal(size=out_f).astype(np.float16)
+    w = np.concatenate([rng.integers(0, 256, 2 * in_f).astype(np.uint8), svh.view(np.uint8)])
+    dp, dw = dev(gpu, part), dev(gpu, w)
+    y = gpu.zeros((m, out_f + 4), dtype=gpu.float32, device="cuda")
+    A = sz.Arg
+    sz.launch("exl3_finish_rows", (out_f // 128, m, 1), (64, 1, 1), 0, 0, [A.ptr(dp.data_ptr()), A.ptr(dw.data_ptr()), A.ptr(y.data_ptr()), A.u32(out_f + 4), A.u32(in_f), A.u32(out_f)])
+    gpu.cuda.synchronize()
+    h = np.ones((1, 1))
+    while len(h) < 128:
+        h = np.block([[h, h], [h, -h]])
+    sums, mags = part.astype(np.float64).sum(1).reshape(m, 2, 128), np.abs(part.astype(np.float64)).sum((1,)).reshape(m, 2, 128).sum(2, keepdims=True)
+    want = (sums @ h / np.sqrt(128)).reshape(m, out_f) * svh
+    bound = np.broadcast_to((zs + 9) * 2.0**-24 * mags / np.sqrt(128), (m, 2, 128)).reshape(m, out_f) * np.abs(svh.astype(np.float64))
+    assert (np.abs(y.cpu().numpy()[:, :out_f] - want) <= bound).all()
