@@ -238,8 +238,11 @@ __device__ __forceinline__ u64 uniform_u64(u64 v) {
 
 // A wave's stream of trellis rows for CT column tiles: units of UT tiles (UT / CT tile rows, 32 K UT bytes), each brought
 // into one of D ring slots by NI global-to-LDS loads of 16 bytes a lane.  In LDS a unit lies packed in the order of the
-// bit stream: tile row, column tile, tile word.
-template <int K, bool H, int CT, int DEPTH = 0, int UT = 16>
+// bit stream: tile row, column tile, tile word.  ONCE: past the caches, for streams that no other workgroup reads (six layers of 512 experts of 2048 x
+// 512, top-10, 4 rows, at 3 bits 250 us, 241; a round of 48 at 2, 3 and 4 bits 906, 901; a projection of 4096 x 2048 for four inputs at 4 bits
+// 9.2, 8.8, of 6144 x 16384 at 3 bits 23.6, 22.7; of 8192 x 32768, with 8 MB of partial sums behind it, 45.4, 46.3).  A prefill chunk's items
+// share their expert's rows (4096 tokens 857 us, past the caches 893).
+template <int K, bool H, int CT, int DEPTH = 0, int UT = 16, bool ONCE = true>
 struct VerifyRing {
     static constexpr int TW = EXL3_TILE_WORDS(K, H), CH = TW / 4;   // words and 16-byte chunks a tile
     static constexpr int UR = UT / CT;                              // tile rows a unit
@@ -265,7 +268,7 @@ struct VerifyRing {
         const u64 at = row0 + (u64) unit * ((u64) UR * pitch);
 #pragma unroll
         for (int i = 0; i < NI; i++)
-            if (64 * (i + 1) <= UT * CH || 64 * i + lane < (u32) (UT * CH)) lds_load_at(at, off[i], lds + (slot * UW + i * 256) * 4);
+            if (64 * (i + 1) <= UT * CH || 64 * i + lane < (u32) (UT * CH)) lds_load_at<ONCE>(at, off[i], lds + (slot * UW + i * 256) * 4);
     }
     // requests the first D units and returns once everything requested before them has landed
     __device__ __forceinline__ void fill(u32 lane) const {
@@ -1079,7 +1082,7 @@ __device__ __forceinline__ void exl3_head_kernel(const u8* __restrict__ blob, co
         const u64 from = base + (u64) (2 * pair) * pitch;
 #pragma unroll
         for (int i = 0; i < R::NI; i++)
-            if (64 * (i + 1) <= 16 * R::CH || 64 * i + lane < 16 * R::CH) lds_load_at(from, ring.off[i], wb_lds + (slot * SLOT + i * 256) * 4);
+            if (64 * (i + 1) <= 16 * R::CH || 64 * i + lane < 16 * R::CH) lds_load_at<true>(from, ring.off[i], wb_lds + (slot * SLOT + i * 256) * 4);
         lds_load<16>((const u8*) xa + (u64) pair * 1024 + lane * 16, wb_lds + (slot * SLOT + R::UW) * 4);
     };
 #pragma unroll
@@ -1894,7 +1897,7 @@ __device__ __forceinline__ void prefill_gate_up_exl3_kernel(const u64* __restric
     const u8* bd = (const u8*) (e < ne ? eaddr[2ull * ne + e] : sh_addr[2]);
     xpf_tiles<NCB == 2 ? XPF_NT(K) : XPF_NT_N>(it.tiles, [&](auto n) {
         constexpr int NT = decltype(n)::value, G = NT < 4 ? NT : 4;
-        typedef VerifyRing<K, false, CT, NCB == 2 ? XPF_RING_W(K, NT) : XPF_RING_N(K, NT), 4 * CT> R;
+        typedef VerifyRing<K, false, CT, NCB == 2 ? XPF_RING_W(K, NT) : XPF_RING_N(K, NT), 4 * CT, false> R;
         constexpr int NB = NCB == 2 && NT >= 6 ? 3 : R::D + 1;
         u32* wb = dyn + NB * 2 * NT * (XPF_HALF_U16 / 2) + wave * (R::D * R::UW);
         R ring;
@@ -1944,7 +1947,7 @@ template <int K, int DEPTH>
 __device__ __forceinline__ void prefill_down_exl3_kernel(const u64* __restrict__ eaddr, const u64* __restrict__ sh_addr, const u32* __restrict__ offs, const u32* __restrict__ list,
                                                          const u32* __restrict__ items, const u16* __restrict__ rows, const float* __restrict__ inv, float* __restrict__ eo, u32 ne, u32 hidden,
                                                          u32 ff, u32 ntl, u32 parts) {
-    typedef VerifyRing<K, false, 8, DEPTH> R;
+    typedef VerifyRing<K, false, 8, DEPTH, 16, false> R;
     constexpr int D = R::D;
     extern __shared__ __attribute__((aligned(16))) u32 dyn[];
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, W = blockDim.x >> 6;

@@ -101,25 +101,31 @@ __device__ __forceinline__ void pow2_scale_of(u32 mx_bits, float& scale, float& 
 __device__ __forceinline__ u32 lds_offset(const void* p) { return (u32) (u64) (const __attribute__((address_space(3))) void*) p; }
 
 // One load instruction: every lane moves B bytes from its own global address to LDS address `lds` + 16 * lane (B = 16 and
-// 12) or `lds` + 4 * lane (B = 4); `lds` must be wave-uniform.  A 4-byte-aligned source is enough.
-template <int B>
+// 12) or `lds` + 4 * lane (B = 4); `lds` must be wave-uniform.  A 4-byte-aligned source is enough.  once: data that nobody reads
+// again, which goes past the caches (nontemporal).
+template <int B, bool once = false>
 __device__ __forceinline__ void lds_load(const void* g, u32 lds) {
     static_assert(B == 16 || B == 12 || B == 4, "sizes the chip has");
     // m0 carries the LDS address; it is put back afterwards, so the statement leaves no register changed
     u32 keep;
     lds = __builtin_amdgcn_readfirstlane(lds);   // uniform by contract; this tells the compiler so
-#define SZ_LDS_LOAD(op) asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t" op " %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(g), "s"(lds) : "memory")
-    if constexpr (B == 16) SZ_LDS_LOAD("global_load_lds_dwordx4");
-    if constexpr (B == 12) SZ_LDS_LOAD("global_load_lds_dwordx3");
-    if constexpr (B == 4) SZ_LDS_LOAD("global_load_lds_dword");
+#define SZ_LDS_LOAD(op, past) asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t" op " %1, off" past "\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(g), "s"(lds) : "memory")
+    if constexpr (B == 16 && once) SZ_LDS_LOAD("global_load_lds_dwordx4", " nt");
+    if constexpr (B == 16 && !once) SZ_LDS_LOAD("global_load_lds_dwordx4", "");
+    if constexpr (B == 12) SZ_LDS_LOAD("global_load_lds_dwordx3", "");
+    if constexpr (B == 4) SZ_LDS_LOAD("global_load_lds_dword", "");
 #undef SZ_LDS_LOAD
 }
 
 // The 16-byte form from a wave-uniform address plus the lane's 32-bit offset: no 64-bit address arithmetic a lane.
+template <bool once = false>
 __device__ __forceinline__ void lds_load_at(u64 base, u32 off, u32 lds) {
     u32 keep;
     lds = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(lds), "s"(base) : "memory");
+#define SZ_LDS_LOAD(past) asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3" past "\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(lds), "s"(base) : "memory")
+    if constexpr (once) SZ_LDS_LOAD(" nt");
+    else SZ_LDS_LOAD("");
+#undef SZ_LDS_LOAD
 }
 
 // A 4-byte global load the compiler keeps no count of (as lds_load's): the caller orders it with wait_vm and must pass the
