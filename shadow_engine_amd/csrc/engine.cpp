@@ -495,7 +495,7 @@ int verify_layers(sz_session* s, uint32_t p0, uint32_t p1, uint32_t base, uint32
                 if (launch(kn.c_str(), c.ff / (64 * ct), 2 * slots, nl * zs, 256, 0, stream, a)) return 1;
             }
             {
-                const std::string kn = std::string("verify_down_") + verify_variant(c.hidden, (uint64_t) nl * slots * zd * (c.hidden / 128), m, &ct) + tag;
+                const std::string kn = std::string(zs > 4 ? "verify_down_x_" : "verify_down_") + verify_variant(c.hidden, (uint64_t) nl * slots * zd * (c.hidden / 128), m, &ct) + tag;
                 const sz_arg a[] = {P(rl), P(table(r0)), U64(V.experts), U64(V.stride), U64(V.shared), U32(V.part), U32(base), P(plans), P(plans), U32(s->plan_stride), U32(ioff), P(part), P(dn),
                                     U32(c.n_expert), U32(c.top_k), U32(m), U32(c.hidden), U32(c.ff)};
                 if (launch(kn.c_str(), c.hidden / (64 * ct), slots, nl * zd, 256, 0, stream, a)) return 1;

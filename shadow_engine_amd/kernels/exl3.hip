@@ -565,12 +565,15 @@ __device__ __forceinline__ void verify_gate_up_kernel(const float* __restrict__ 
 
 // Launch 3: act = silu(gate) * up of every token of the item out of launch 2's sums (partials added, output side of the two
 // projections), rotated into the down projection's basis as A rows, then its products: dn[((layer * S + pair) * zd + z) *
-// hidden + column], zd = ceil(ff / 512).  grid = (hidden / (64 CT), slots, layers zd), block 256.
-template <int K, bool H, int CT, int NG>
+// hidden + column], zd = ceil(ff / 512).  grid = (hidden / (64 CT), slots, layers zd), block 256.  WIDE: gate and up have more than four
+// partials (inputs of more than 2048 features), which are asked for eight at once (four layers of 32 experts of 4096 x 1536, top-2, 8 rows, at 4 bits 350 us, 324;
+// of 64 of 4096 x 512, top-4, 2 rows 120.5, 116.5; six of 160 of 3584 x 768, top-12, 6 rows, at 3 bits 725, 712).  Kernels of their own: as a
+// branch, 10 KB of code more, the others lose (a round of 16 layers of 1024 x 768 at 8 rows 232 us, 237).
+template <int K, bool H, int CT, int NG, bool WIDE = false>
 __device__ __forceinline__ void verify_down_kernel(const float* __restrict__ logits, const u8* __restrict__ table, u64 experts, u64 stride, u64 shared, u32 part0, u32 base,
                                                    const u8* __restrict__ plans, u8* __restrict__ weights, u32 plan_stride, u32 ioff, const float* __restrict__ gup, float* __restrict__ dn,
                                                    u32 ne, u32 k, u32 m, u32 hidden, u32 ff) {
-    constexpr int NMAX = 4 * NG;
+    constexpr int NMAX = 4 * NG, TOKENS = WIDE ? 1 : 2, PARTS = WIDE ? 8 : 4;
     typedef VerifyRing<K, H, CT> R;
     __shared__ __attribute__((aligned(16))) u32 wb_all[4][R::D * R::UW];
     __shared__ __attribute__((aligned(16))) u16 a_sh[16 * 3 * NMAX * 32];
@@ -636,18 +639,19 @@ __device__ __forceinline__ void verify_down_kernel(const float* __restrict__ log
         sc[4] = load_u16_uncounted(sud);
         sc[5] = load_u16_uncounted(sud + 64);
 #pragma unroll
-        for (int r0 = 0; r0 < NMAX; r0 += 2) {
+        for (int r0 = 0; r0 < NMAX; r0 += TOKENS) {
             if ((u32) r0 < n) {
-                // two tokens at a time, the first four partials of each requested together; the first lot goes out ahead of the rows
-                float pv[2][4][4];
+                // two tokens at a time, the first four partials of each requested together (WIDE: one, its first eight); the first lot goes out
+                // ahead of the rows
+                float pv[TOKENS][PARTS][4];
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
+                for (int q = 0; q < TOKENS; q++) {
                     // (a lot's second token past the item's: its first again, so that no load stands behind a branch)
-                    const u32 pair = ((u32) (r0 + q) < n ? pairs[r0 / 2] >> (16 * q) : pairs[r0 / 2]) & 0xffffu;
+                    const u32 pair = ((u32) (r0 + q) < n ? pairs[r0 / 2] >> (16 * ((r0 + q) & 1)) : pairs[r0 / 2]) & 0xffffu;
                     const float* pg = g0 + (u64) pair * zs * ff;
                     const float* pu = g0 + (u64) (S + pair) * zs * ff;
 #pragma unroll
-                    for (int zz = 0; zz < 4; zz++) {
+                    for (int zz = 0; zz < PARTS; zz++) {
                         const u64 o = (u64) min((u32) zz, zs - 1) * ff;
                         pv[q][zz][0] = load_f32_uncounted(pg + o);
                         pv[q][zz][1] = load_f32_uncounted(pg + o + 64);
@@ -663,23 +667,23 @@ __device__ __forceinline__ void verify_down_kernel(const float* __restrict__ log
                     wait_vm<0>();
                 }
 #pragma unroll
-                for (int q = 0; q < 2; q++)
+                for (int q = 0; q < TOKENS; q++)
 #pragma unroll
-                    for (int zz = 0; zz < 4; zz++)
+                    for (int zz = 0; zz < PARTS; zz++)
 #pragma unroll
                         for (int c = 0; c < 4; c++) load_landed(pv[q][zz][c]);
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
+                for (int q = 0; q < TOKENS; q++) {
                     const int r = r0 + q;
                     if ((u32) r < n) {
                         float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                        for (int zz = 0; zz < 4; zz++)
+                        for (int zz = 0; zz < PARTS; zz++)
 #pragma unroll
                             for (int c = 0; c < 4; c++) t[c] += (u32) zz < zs ? pv[q][zz][c] : 0.0f;
-                        if (zs > 4) {
+                        if (zs > (u32) PARTS) {
                             const u32 pair = (pairs[r / 2] >> (16 * (r & 1))) & 0xffffu;
-                            for (u32 zz = 4; zz < zs; zz++) {
+                            for (u32 zz = PARTS; zz < zs; zz++) {
                                 const float* pg = g0 + ((u64) pair * zs + zz) * ff;
                                 const float* pu = g0 + ((u64) (S + pair) * zs + zz) * ff;
                                 t[0] += pg[0];
@@ -808,6 +812,57 @@ __device__ __forceinline__ void verify_down_kernel(const float* __restrict__ log
         const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
         verify_down_kernel<K, true, 2, 2>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
     }
+// x: inputs of more than 2048 features
+#define EXL3_VERIFY_WIDE_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_x_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 8, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_x_t4_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 4, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) verify_down_x_t2_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 2, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_x_w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 8, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_x_t4w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 4, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) verify_down_x_t2w_exl3_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, false, 2, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    }
+#define EXL3_VERIFY_WIDE_HALF_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_x_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 8, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_x_t4_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 4, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 1)) verify_down_x_t2_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 2, 1, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_x_w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 8, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_x_t4w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 4, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) verify_down_x_t2w_exl3h_##K(const float* logits, const u8* table, u64 experts, u64 stride, u64 shared, u32 part, u32 base, \
+        const u8* plans, u8* weights, u32 plan_stride, u32 ioff, const float* gup, float* dn, u32 ne, u32 k, u32 m, u32 hidden, u32 ff) { \
+        verify_down_kernel<K, true, 2, 2, true>(logits, table, experts, stride, shared, part, base, plans, weights, plan_stride, ioff, gup, dn, ne, k, m, hidden, ff); \
+    }
 EXL3_VERIFY_ENTRIES(1)
 EXL3_VERIFY_ENTRIES(2)
 EXL3_VERIFY_ENTRIES(3)
@@ -819,6 +874,17 @@ EXL3_VERIFY_ENTRIES(8)
 EXL3_VERIFY_HALF_ENTRIES(1)
 EXL3_VERIFY_HALF_ENTRIES(2)
 EXL3_VERIFY_HALF_ENTRIES(3)
+EXL3_VERIFY_WIDE_ENTRIES(1)
+EXL3_VERIFY_WIDE_ENTRIES(2)
+EXL3_VERIFY_WIDE_ENTRIES(3)
+EXL3_VERIFY_WIDE_ENTRIES(4)
+EXL3_VERIFY_WIDE_ENTRIES(5)
+EXL3_VERIFY_WIDE_ENTRIES(6)
+EXL3_VERIFY_WIDE_ENTRIES(7)
+EXL3_VERIFY_WIDE_ENTRIES(8)
+EXL3_VERIFY_WIDE_HALF_ENTRIES(1)
+EXL3_VERIFY_WIDE_HALF_ENTRIES(2)
+EXL3_VERIFY_WIDE_HALF_ENTRIES(3)
 
 // Launch 4: token j = blockIdx.y of layer blockIdx.z, output block blockIdx.x: y[j] = sum over its cnt[j] experts t, in rank order,
 // of w[j,t] * (the down product of pair j k + t) + sigmoid(gl[j]) * (the shared expert's).  Wave t finishes expert t (partials

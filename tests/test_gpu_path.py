@@ -335,6 +335,12 @@ def test_moe_layer_verify_matches_the_oracle(gpu, ty, hidden, ff, ne, k, m, shar
     run_moe_layer_case(gpu, ty, hidden, ff, ne, k, m, shared)
 
 
+@pytest.mark.parametrize("ty,hidden,m", [(sz.EXL3(3), 2304, 2), (sz.EXL3(3), 4096, 5), (sz.EXL3(2), 4352, 3), (sz.EXL3(6), 5120, 8)])
+def test_moe_layer_of_more_than_four_partials(gpu, ty, hidden, m):
+    """Gate and up sums of 5, 8, 9 and 10 partials (512 inputs each, the last of 256 or 512): what the down launch asks for at once and what is behind it."""
+    run_moe_layer_case(gpu, ty, hidden, 256, 6, 3, m, True)
+
+
 @pytest.mark.parametrize("ty,hidden,ff,ne,k,m,shared", [
     (sz.IQ3_S, 2048, 512, 32, 10, 4, True),        # tokens share experts: groups of several inputs
     (sz.Q8_0, 512, 256, 16, 4, 8, False),
