@@ -713,3 +713,27 @@ def test_finish_adds_any_number_of_partials(gpu, zs):  # noqa: F811
     want = (sums @ h / np.sqrt(128)).reshape(m, out_f) * svh
     bound = np.broadcast_to((zs + 9) * 2.0**-24 * mags / np.sqrt(128), (m, 2, 128)).reshape(m, out_f) * np.abs(svh.astype(np.float64))
     assert (np.abs(y.cpu().numpy()[:, :out_f] - want) <= bound).all()
+
+
+def cols_call(gpu, ty, dw, cols, rows, x):  # noqa: F811
+    m, dx = len(x), dev(gpu, x)
+    y = gpu.full((m, rows), float("nan"), dtype=gpu.float32, device="cuda")
+    n = sz.matvec_cols_scratch(ty, cols, rows, m)
+    scratch = gpu.empty(n, dtype=gpu.uint8, device="cuda")
+    sz.matvec_cols(ty, dw.data_ptr(), cols, rows, dx.data_ptr(), cols, y.data_ptr(), rows, m, scratch.data_ptr(), n)
+    gpu.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("cols,rows", [(2048, 24576), (2048, 24704), (2048, 25088), (4096, 16384), (4096, 16512), (4096, 20480), (4096, 28672), (4096, 32768), (4096, 33280), (8192, 22528)])
+def test_large_projections_for_more_than_four_inputs(gpu, cols, rows):  # noqa: F811
+    """The sizes at which a projection's tile count changes for more than four inputs, and rows that fill no wider workgroup: a row's bits are those of the calls
+    of up to four, which choose by another rule; a sample of the outputs in the magnitude of the inputs."""
+    g = gpu.Generator(device="cuda")
+    g.manual_seed(cols + rows)
+    dw = synth_device.exl3_matrix(gpu, cols + rows, cols, rows, 2)
+    x = gpu.randn((8, cols), device="cuda", generator=g).cpu().numpy()
+    few = np.concatenate([cols_call(gpu, sz.EXL3(2), dw, cols, rows, x[j:j + 4]) for j in (0, 4)])
+    assert np.isfinite(few).all() and (np.abs(few).max(axis=1) > 0).all()
+    for m in (5, 8):
+        assert np.array_equal(bits(cols_call(gpu, sz.EXL3(2), dw, cols, rows, x[:m])), bits(few[:m])), m
