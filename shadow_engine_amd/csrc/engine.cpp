@@ -149,11 +149,12 @@ static uint32_t gguf_lds(uint32_t waves, uint32_t tiles, uint32_t ng) { return w
 // compute unit, so a launch runs 512 of them at once, w / 2 of four tiles and w / 4 of eight, and a few left over cost as much as 512.  us a call of 8
 // inputs at 4 bits by two, four and eight tiles: w = 768 19.3, 20.9, 22.9; 896 24.0, 21.3, 23.3; 1024 23.9, 21.8, 23.5; 1152 27.9, 27.1, 31.3 (5 inputs at
 // 2 bits 22.6, 23.7, 28.7); 1280 28.7, 27.5, 31.7; 1536 32.9, 28.8, 32.3; 1792 37.0, 35.6, 33.2; 2048 40.6, 36.1, 33.3; 2304 45.5, 42.0, 42.9; 3072
-// 58.2, 49.3, 44.8; 4096 73.8, 59.7, 53.0.
-static const char* cols_variant(uint64_t cols, uint64_t rows, uint32_t m, uint32_t* ct) {
+// 58.2, 49.3, 44.8; 4096 73.8, 59.7, 53.0.  Above 5 bits one tile where its workgroups (2 w) do not outnumber the compute units (EXL3_COLS_NARROW_ENTRIES).
+static const char* cols_variant(const Format& f, uint64_t cols, uint64_t rows, uint32_t m, uint32_t* ct) {
     const uint64_t w = rows / 128 * exl3_ksplit((uint32_t) cols);
     if (m > 4 && rows % 512 == 0 && ((w >= 1792 && w <= 2048) || w >= 2816)) { *ct = 8; return "w_"; }
     if (m > 4 && rows % 256 == 0 && ((w > 768 && w <= 1024) || w >= 1280)) { *ct = 4; return "t4w_"; }
+    if (!f.half && f.bits >= 6 && cols % 256 == 0 && w <= 128) { *ct = 1; return m > 4 ? "t1w_" : "t1_"; }
     return verify_variant(rows, w, m, ct);
 }
 
@@ -171,7 +172,7 @@ int matvec_cols_dev(int ty, uint64_t w, uint64_t cols, uint64_t rows, uint64_t x
         if (scratch_bytes < cols_scratch_bytes(f, cols, rows, m) || !scratch) return fail("matvec_cols: workspace too small for EXL3");
         const uint32_t zs = exl3_ksplit((uint32_t) cols);
         uint32_t ct;
-        const std::string kn = std::string("matvec_grouped_") + cols_variant(cols, rows, m, &ct) + tag;
+        const std::string kn = std::string("matvec_grouped_") + cols_variant(f, cols, rows, m, &ct) + tag;
         const sz_arg a0[] = {P(w), P(x), U32(xs), P(scratch), U32((uint32_t) cols), U32((uint32_t) rows), U32(m)};
         if (launch(kn.c_str(), (uint32_t) rows / (64 * ct), zs, 1, 256, 0, stream, a0)) return 1;
         const sz_arg a1[] = {P(scratch), P(w), P(y), U32(ys), U32((uint32_t) cols), U32((uint32_t) rows)};

@@ -1030,6 +1030,16 @@ extern "C" __global__ void __launch_bounds__(64) exl3_finish_rows(const float* p
     extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K + 1, 2)) matvec_grouped_t2w_exl3h_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
         exl3_cols_kernel<K, true, 2, 2>(w, x, xs, part, in_f, out_f, m); \
     }
+// One column tile a wave, for inputs in 256s (a unit is 16 tile rows).  Above 5 bits a ring holds two units and a weight takes two windows: half the chain
+// for a wave of a matrix whose workgroups fill half the chip (a call of 2048 x 4096 at 6 bits for 1, 4 and 8 inputs 8.8, 10.0 and 12.3 us by two tiles, 7.8, 9.1
+// and 11.0 by one; at 3 and 4 bits 7.8, 9.0 and 11.3 by either).
+#define EXL3_COLS_NARROW_ENTRIES(K) \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 1)) matvec_grouped_t1_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 1, 1>(w, x, xs, part, in_f, out_f, m); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_VERIFY_OCC(K, 2)) matvec_grouped_t1w_exl3_##K(const u8* w, const float* x, u32 xs, float* part, u32 in_f, u32 out_f, u32 m) { \
+        exl3_cols_kernel<K, false, 1, 2>(w, x, xs, part, in_f, out_f, m); \
+    }
 EXL3_COLS_ENTRIES(1)
 EXL3_COLS_ENTRIES(2)
 EXL3_COLS_ENTRIES(3)
@@ -1038,6 +1048,9 @@ EXL3_COLS_ENTRIES(5)
 EXL3_COLS_ENTRIES(6)
 EXL3_COLS_ENTRIES(7)
 EXL3_COLS_ENTRIES(8)
+EXL3_COLS_NARROW_ENTRIES(6)
+EXL3_COLS_NARROW_ENTRIES(7)
+EXL3_COLS_NARROW_ENTRIES(8)
 EXL3_COLS_HALF_ENTRIES(1)
 EXL3_COLS_HALF_ENTRIES(2)
 EXL3_COLS_HALF_ENTRIES(3)

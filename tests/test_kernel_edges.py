@@ -715,6 +715,24 @@ def test_finish_adds_any_number_of_partials(gpu, zs):  # noqa: F811
     assert (np.abs(y.cpu().numpy()[:, :out_f] - want) <= bound).all()
 
 
+@pytest.mark.parametrize("kb,half", [(6, False), (7, False), (8, False), (3, True)])
+@pytest.mark.parametrize("cols", [256, 640, 768, 2048])
+def test_small_projections_above_five_bits(gpu, kb, half, cols):  # noqa: F811
+    """One column tile a wave where the inputs come in 256s, two elsewhere (and at half rates): blocks of 512 inputs that are whole, a half and a quarter.  The oracle's
+    values, and a row's bits whatever the rows beside it."""
+    rng = np.random.default_rng(cols + kb)
+    rows = 384
+    ty = sz.EXL3_HALF(kb) if half else sz.EXL3(kb)
+    w, x = synth.exl3_blob(rng, cols, rows, kb, half), rng.normal(size=(8, cols)).astype(np.float32)
+    first = None
+    for m in (1, 4, 5, 8):
+        got = cols_call(gpu, ty, dev(gpu, w), cols, rows, x[:m])
+        first = got if first is None else first
+        assert np.array_equal(bits(got[:1]), bits(first[:1])), m
+    for j in range(8):
+        assert rel_l2(got[j], O.exl3_matvec(cols, rows, kb, w, x[j], half=half)) <= 2e-6, j
+
+
 def cols_call(gpu, ty, dw, cols, rows, x):  # noqa: F811
     m, dx = len(x), dev(gpu, x)
     y = gpu.full((m, rows), float("nan"), dtype=gpu.float32, device="cuda")
