@@ -145,11 +145,11 @@ static uint32_t gguf_waves(uint64_t cols) {
 }
 static uint32_t gguf_lds(uint32_t waves, uint32_t tiles, uint32_t ng) { return waves * (1584 * 4 + tiles * ng * 64 * 4); }
 
-// The column tiles of a projection alone.  For more than four inputs by the 64-column strips of 512 inputs, w of them two at a time: two workgroups share a
-// compute unit, so a launch runs 512 of them at once, w / 2 of four tiles and w / 4 of eight, and a few left over cost as much as 512.  us a call of 8
+// The column tiles of a projection alone, by its w blocks of 128 columns and 512 inputs.  For more than four inputs: a launch of two tiles a wave has w workgroups,
+// of four w / 2, of eight w / 4; two share a compute unit, so 512 run at once, and a few left over cost as much as 512.  us a call of 8
 // inputs at 4 bits by two, four and eight tiles: w = 768 19.3, 20.9, 22.9; 896 24.0, 21.3, 23.3; 1024 23.9, 21.8, 23.5; 1152 27.9, 27.1, 31.3 (5 inputs at
 // 2 bits 22.6, 23.7, 28.7); 1280 28.7, 27.5, 31.7; 1536 32.9, 28.8, 32.3; 1792 37.0, 35.6, 33.2; 2048 40.6, 36.1, 33.3; 2304 45.5, 42.0, 42.9; 3072
-// 58.2, 49.3, 44.8; 4096 73.8, 59.7, 53.0.  Above 5 bits one tile where its workgroups (2 w) do not outnumber the compute units (EXL3_COLS_NARROW_ENTRIES).
+// 58.2, 49.3, 44.8; 4096 73.8, 59.7, 53.0.  Above 5 bits one tile where its 2 w workgroups do not outnumber the compute units (EXL3_COLS_NARROW_ENTRIES).
 static const char* cols_variant(const Format& f, uint64_t cols, uint64_t rows, uint32_t m, uint32_t* ct) {
     const uint64_t w = rows / 128 * exl3_ksplit((uint32_t) cols);
     if (m > 4 && rows % 512 == 0 && ((w >= 1792 && w <= 2048) || w >= 2816)) { *ct = 8; return "w_"; }
