@@ -12,7 +12,7 @@ lines carry the same fields):
     config1  one Q8_0 1024 x 2048 matrix-vector product
     config2  one IQ3_S MoE layer for one token (512 experts + shared, top-10); a step walks through 8 different layers
     config3  one EXL3 K=3 MoE layer for 4 tokens + head + acceptance (weights of the one layer stay warm in cache)
-    config4  one prefill chunk: 512 tokens through the 512 IQ3_S experts of a layer on int8 activations (int8 MFMA)
+    config4  one prefill chunk: 512 tokens through the 512 IQ3_S experts of a layer on int8 activations (whole numbers, f16 MFMA)
     exl3head the 151,936 x 2048 lm_head of an EXL3 checkpoint (--bits K, default 4) for the batch, arg-max fused in
     exl3top  the same head's top-64 hand-off to the host; --screen N goes through the inexact 2-bit screen, N blocks a row
     stage    one EXL3 layer of a safetensors checkpoint staged into HBM (the loader beside the path; PCIe-inclusive)
@@ -37,7 +37,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBPS = 8000.0
-INT8_MFMA_PEAK_TOPS = 5000.0
+F16_MFMA_PEAK_TFLOPS = 2500.0
 HIDDEN, FF, NE, TOPK, VOCAB, ROWS = 2048, 512, 512, 10, 151936, 4
 COUNTERS = os.path.join(ROOT, "profiles", "counters.json")
 SIMDS = 256 * 4                                  # 256 compute units x 4 SIMDs; a wave64 vector instruction takes one for 4 cycles
@@ -236,12 +236,12 @@ def iq3s_prefill(torch, sz, synth, synth_device, stream, tokens=512):
     distinct = int(np.unique(ids).size)
     gu, _, dn = synth.expert_bytes(sz.IQ3_S, HIDDEN, FF)
     w.step_bytes = distinct * (2 * gu + dn) + tokens * (2 * HIDDEN + NE) * 4
-    # gate/up: the experts' two matrices, the tokens' int8 codes and scales in, H's codes and scales out; down: the experts' third
+    # gate/up: the experts' two matrices, the tokens' codes (as f16) and scales in, H's codes (int8 and f16) and scales out; down: the experts' third
     # matrix, H in, the pairs' rows of the result out (f32, summed by the combine launch: counted as the EXL3 launches' are)
-    w.kernel_bytes = {"prefill_gate_up_iq3_s": distinct * 2 * gu + tokens * HIDDEN * 9 // 8 + tokens * TOPK * FF * 9 // 8,
-                      "prefill_down_iq3_s": distinct * dn + tokens * TOPK * FF * 9 // 8 + tokens * TOPK * HIDDEN * 4}
+    w.kernel_bytes = {"prefill_gate_up_iq3_s": distinct * 2 * gu + tokens * HIDDEN * 17 // 8 + tokens * TOPK * FF * 25 // 8,
+                      "prefill_down_iq3_s": distinct * dn + tokens * TOPK * FF * 17 // 8 + tokens * TOPK * HIDDEN * 4}
     w.kernel_ops = {"prefill_gate_up_iq3_s": 2.0 * tokens * TOPK * 2 * FF * HIDDEN, "prefill_down_iq3_s": 2.0 * tokens * TOPK * FF * HIDDEN}
-    w.dtype = "int8 x int8 -> int32 MFMA, f32 scales"
+    w.dtype = "int8 codes as f16 x f16 whole-number weights -> f32 MFMA, f32 scales"
     w.describe = {"workload": "config 4: prefill chunk, %d tokens x hidden 2048 through 512 IQ3_S experts (top-10, Zipf-skewed routing, "
                               "%d distinct experts hit) on per-32 int8 activations" % (tokens, distinct), "rows": tokens,
                   "resident_GB": round(buf.numel() / 1e9, 2)}
@@ -448,7 +448,7 @@ def kernel_times(w, stream, sz, reps):
             per_kernel[name]["bytes_per_launch"] = int(w.kernel_bytes[name])
             per_kernel[name]["GBps"] = w.kernel_bytes[name] / (us * 1e-6) / 1e9
         if name in w.kernel_ops:
-            per_kernel[name]["int8_TOPs"] = w.kernel_ops[name] / (us * 1e-6) / 1e12
+            per_kernel[name]["mfma_TFLOPs"] = w.kernel_ops[name] / (us * 1e-6) / 1e12
     return per_kernel
 
 
@@ -480,9 +480,9 @@ def roofline_of(w, per_kernel, counters, stale):
         r["counters"] = "profiles/counters.json"
     else:
         r["counters"] = stale.get(dom, "none on file for this workload") if key else "none on file for this workload"
-    if "int8_TOPs" in per_kernel[dom]:
-        t = per_kernel[dom]["int8_TOPs"]
-        r["mfma"] = {"achieved": round(t, 2), "peak": INT8_MFMA_PEAK_TOPS, "unit": "TOP/s", "frac": round(t / INT8_MFMA_PEAK_TOPS, 5)}
+    if "mfma_TFLOPs" in per_kernel[dom]:
+        t = per_kernel[dom]["mfma_TFLOPs"]
+        r["mfma"] = {"achieved": round(t, 2), "peak": F16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(t / F16_MFMA_PEAK_TFLOPS, 5)}
     return r
 
 

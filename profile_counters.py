@@ -36,7 +36,7 @@ NAMES = {"config5": ("verify_round_config5", "the default benchmark workload (co
          "config3": ("verify_layer_and_head_config3", "bench.py --workload config3 (one EXL3 K=3 MoE layer for 4 tokens + Q8_0 head + acceptance)", " --workload config3"),
          "config1": ("matvec_q8_0_config1", "bench.py --workload config1 (one Q8_0 1024 x 2048 matrix-vector product)", " --workload config1"),
          "config2": ("iq3s_decode_layer_config2", "bench.py --workload config2 (IQ3_S MoE layer for one token, 8 different layers a step)", " --workload config2"),
-         "config4": ("prefill_chunk_config4", "bench.py --workload config4 (prefill chunk: 512 tokens through 512 IQ3_S experts, int8 matrix cores)", " --workload config4"),
+         "config4": ("prefill_chunk_config4", "bench.py --workload config4 (prefill chunk: 512 tokens through 512 IQ3_S experts, int8 activations, f16 matrix cores)", " --workload config4"),
          "exl3head": ("head_exl3_k4_lm_head", "bench.py --workload exl3head (EXL3 K=4 lm_head 151936 x 2048, 4-row batch, arg-max fused in)", " --workload exl3head"),
          "exl3top": ("head_exl3_k4_top64", "bench.py --workload exl3top (top-64 hand-off of the EXL3 K=4 lm_head 151936 x 2048 for 4 rows, exact)", " --workload exl3top"),
          "exl3top_screen": ("head_exl3_k4_top64_screened", "bench.py --workload exl3top --screen 128 (the same hand-off through the inexact 2-bit screen, 128 blocks a row)",
