@@ -45,11 +45,6 @@ __device__ __forceinline__ void gg_order() {
 
 // 16 rows x 256 columns of a wave: load() requests them, stage() makes them readable, products() adds
 // sum of the chunk for token 4 G + lane / 16 and row lane % 16 to out[G], in units of the inputs' scale.
-// ONCE: Q8_0 weights past the caches, for the items of a layer of more than four rows, whose experts nobody reads again and which push out what the
-// launches share (four layers of 128 experts of 2560 x 768, top-8, 8 rows 359 us, 350; three of 128 of 2560 x 1024 331, 319, of 32 of 3072 x 1536,
-// top-4, 6 rows 232, 225).  Few rows of few layers are read again from the last level (three layers of 64 of 2048 x 512, 4 rows 123, past
-// the caches 124.5; two of 32 of 2560 x 1024, one row 47.9, 49.5), a projection's chunks share lines (8201 x 3072 for five inputs, twice, 21.4, 21.6),
-// and so do the six loads of an IQ3_S block (the last two layers 317, 358 and 227, 254): ordinary loads.
 struct GgQ8 {
     static constexpr u32 QK = 32, BB = 34, CHUNK = 272;   // bytes of a 256-column chunk: 17 pieces of 16
     static constexpr u32 PITCH = 72;                      // words of a row in the strip: 68 and a shift of four banks
@@ -67,7 +62,6 @@ struct GgQ8 {
     }
     __device__ __forceinline__ u32 place(int i) const { return __builtin_amdgcn_ubfe(at[i / 3], 10 * (i % 3), 5); }
     __device__ __forceinline__ u32 row(int i) const { return __builtin_amdgcn_ubfe(at[i / 3], 10 * (i % 3) + 5, 5); }
-    template <bool ONCE>
     __device__ __forceinline__ void load(const u8* __restrict__ w, u32 rb, u32 first, u32 rows, u32 col, u32 lane) {
         if (rb < CHUNK) return;
         const u8* base = w + (u64) first * rb + col / 32 * 34;
@@ -76,10 +70,7 @@ struct GgQ8 {
         for (int i = 0; i < 2; i++) asm volatile("" : "+v"(at[i]));   // the addresses are a few operations: not kept
 #pragma unroll
         for (int i = 0; i < 5; i++)
-            if (i < 4 || lane < 16) {
-                const u32x4b* p = (const u32x4b*) (base + (u64) min(row(i), rmost) * rb + place(i) * 16);
-                v[i] = ONCE ? __builtin_nontemporal_load(p) : *p;
-            }
+            if (i < 4 || lane < 16) v[i] = *(const u32x4b*) (base + (u64) min(row(i), rmost) * rb + place(i) * 16);
     }
     __device__ __forceinline__ void stage(u32* strip, const u8* __restrict__ w, u32 rb, u32 first, u32 rows, u32 lane) const {
         if (rb < CHUNK) {
@@ -154,7 +145,6 @@ struct GgIq3 {
     static constexpr u32 part_at(u32 q, u32 g) { return 64 * g + 8 * q; }
     u32 qs[4], sg[2], qh, sc, d;
     __device__ __forceinline__ void init(u32) {}
-    template <bool>
     __device__ __forceinline__ void load(const u8* __restrict__ w, u32 rb, u32 first, u32 rows, u32 col, u32 lane) {
         const u32 g = lane >> 4;
         const u8* p = w + (u64) min(first + (lane & 15), rows - 1) * rb + col / 256 * BB;
@@ -318,7 +308,7 @@ extern __shared__ __attribute__((aligned(16))) u32 sz_dyn_lds[];
 // order, so the bits, do not depend on m).  A row's last chunk, where it is short, is its last 256 columns, the inputs of the ones
 // that the chunk before has taken as zeros.  Ends with the waves' sums in LDS behind a barrier; gg_total adds them up.
 // Dynamic LDS: GG_STRIP and nt * NG * 64 words a wave; table: 512 words of a format with a grid.
-template <class F, int NG, bool ONCE, class Tile, class Input>
+template <class F, int NG, class Tile, class Input>
 __device__ __forceinline__ void gg_sums(Tile tile, u32 nt, u32 rows, Input input, u32 m, u32 cols, u32* table) {
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, W = blockDim.x >> 6;
     const u32 rb = cols / F::QK * F::BB, nc = (cols + 255) / 256;
@@ -339,7 +329,7 @@ __device__ __forceinline__ void gg_sums(Tile tile, u32 nt, u32 rows, Input input
         }
         if (c == wave) {
             const GgTile t0 = tile(0);
-            cur.template load<ONCE>(t0.w, rb, t0.first, rows, start(c), lane);   // W <= nc
+            cur.load(t0.w, rb, t0.first, rows, start(c), lane);   // W <= nc
             if constexpr (F::grid) {
                 for (u32 i = threadIdx.x; i < 512; i += blockDim.x) table[i] = IQ3S_GRID[i];
                 __syncthreads();
@@ -356,7 +346,7 @@ __device__ __forceinline__ void gg_sums(Tile tile, u32 nt, u32 rows, Input input
             now.stage(strip, tt.w, rb, tt.first, rows, lane);
             if (t + 1 < nt || c + W < nc) {
                 const GgTile next = tile(t + 1 < nt ? t + 1 : 0);
-                cur.template load<ONCE>(next.w, rb, next.first, rows, start(t + 1 < nt ? c : c + W), lane);
+                cur.load(next.w, rb, next.first, rows, start(t + 1 < nt ? c : c + W), lane);
             }
             float out[NG];
 #pragma unroll
@@ -392,7 +382,7 @@ template <class F, int NG>
 __device__ __forceinline__ void gg_cols(const u8* __restrict__ w, const float* __restrict__ x, u32 xs, float* __restrict__ y, u32 ys, u32 rows, u32 cols, u32 m) {
     __shared__ u32 table[F::grid ? 512 : 1];
     const u32 n16 = (rows + 15) / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
-    gg_sums<F, NG, false>([&](u32 t) { return GgTile{w, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, rows, [&](u32 j) { return x + (u64) j * xs; }, m, cols, table);
+    gg_sums<F, NG>([&](u32 t) { return GgTile{w, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, rows, [&](u32 j) { return x + (u64) j * xs; }, m, cols, table);
     for (u32 i = threadIdx.x; i < nt * NG * 64; i += blockDim.x) {
         const u32 t = i / (NG * 64), G = i / 64 % NG, l = i & 63;
         const u32 r = 16 * (blockIdx.x + t * gridDim.x) + (l & 15), j = 4 * G + (l >> 4);
@@ -507,7 +497,7 @@ __device__ __forceinline__ void gg_gate_up(const float* __restrict__ logits, u64
     const u32 n16 = ff / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
     auto run = [&](auto ng) {
         constexpr int N = decltype(ng)::value;
-        gg_sums<F, N, (NG > 1)>([&](u32 t) { return GgTile{it.w + (t & 1 ? part : 0u), 16 * (blockIdx.x + (t >> 1) * gridDim.x)}; }, 2 * nt, ff,
+        gg_sums<F, N>([&](u32 t) { return GgTile{it.w + (t & 1 ? part : 0u), 16 * (blockIdx.x + (t >> 1) * gridDim.x)}; }, 2 * nt, ff,
                       [&](u32 r) { return u + (u64) it.token(r) * hidden; }, it.n, hidden, table);
         for (u32 i = threadIdx.x; i < nt * N * 64; i += blockDim.x) {
             const u32 t = i / (N * 64), l = i % (N * 64), r = l >> 4;
@@ -537,7 +527,7 @@ __device__ __forceinline__ void gg_down(const float* __restrict__ logits, u64 ex
     const u32 n16 = hidden / 16, nt = (n16 - blockIdx.x + gridDim.x - 1) / gridDim.x;
     auto run = [&](auto ng) {
         constexpr int N = decltype(ng)::value;
-        gg_sums<F, N, (NG > 1)>([&](u32 t) { return GgTile{it.w + 2 * (u64) part, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, hidden,
+        gg_sums<F, N>([&](u32 t) { return GgTile{it.w + 2 * (u64) part, 16 * (blockIdx.x + t * gridDim.x)}; }, nt, hidden,
                       [&](u32 r) { return act + (u64) it.pair(r) * ff; }, it.n, ff, table);
         for (u32 i = threadIdx.x; i < nt * N * 64; i += blockDim.x) {
             const u32 t = i / (N * 64), l = i % (N * 64), r = l >> 4;
