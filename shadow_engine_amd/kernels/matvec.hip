@@ -1490,13 +1490,10 @@ __device__ __forceinline__ f16x4 head_codes_f16(u32 q) {
 }
 
 // Requests tile `t` (rows 16 t .. 16 t + 15, clamped to the last row) into the LDS buffer at byte offset `lds`: wave w of W
-// brings rows w, w + W, .., each as 16-byte pieces (ceil(row bytes / 1024) instructions a row).  A head of 64 MiB or more goes past the caches, out of which
-// it would push everything else (the 64 best of 4 rows of 151 936 x 2048 107 us, 98.7; of 8 of 65 536 x 4096 121, 117.5; a round of 4 layers with the
-// first 155, 152, with 32 000 x 2048 and one row 52.6, 51.9); a smaller one the last level keeps from call to call (32 000 x 1024, one row 48.5, 50.3).
-template <int W>
-__device__ __forceinline__ void head_tile_issue(const u8* __restrict__ w, u32 rows, u32 rb, u32 t, u32 lds, u32 wave, u32 lane) {
+// brings rows w, w + W, .., each as 16-byte pieces (ceil(row bytes / 1024) instructions a row).  once: past the caches.
+template <int W, bool once>
+__device__ __forceinline__ void head_tile_rows(const u8* __restrict__ w, u32 rows, u32 rb, u32 t, u32 lds, u32 wave, u32 lane) {
     const u32 pieces = rb / 16;                           // rb is a multiple of 16 here
-    const bool once = (u64) rows * rb >= 64u << 20;
 #pragma unroll
     for (int rr = 0; rr < (16 + W - 1) / W; rr++) {
         const u32 lr = wave + W * rr;
@@ -1506,12 +1503,19 @@ __device__ __forceinline__ void head_tile_issue(const u8* __restrict__ w, u32 ro
 #pragma unroll
             for (int c = 0; c < 5; c++)
                 if (c * 64 < pieces)
-                    if (c * 64 + lane < pieces) {
-                        if (once) lds_load<16, true>(src + (c * 64 + lane) * 16, dst + c * 1024);
-                        else lds_load<16>(src + (c * 64 + lane) * 16, dst + c * 1024);
-                    }
+                    if (c * 64 + lane < pieces) lds_load<16, once>(src + (c * 64 + lane) * 16, dst + c * 1024);
         }
     }
+}
+// A head of 256 MiB or more, what the last level holds, goes past the caches, out of which it would push everything else (the 64 best of 4
+// rows of 151 936 x 2048, 315 MiB, 107 us, 98.7; of 8 of 65 536 x 4096, 272 MiB, 121, 117.5; a round of 2 layers with the first 96, 90, of 4 with
+// four rows 134, 132).  A smaller one is there again at the next call, also with layers in between (4 rows of 151 936 x 1024, 158 MiB, 86 and past
+// the caches 91; rounds of 1 to 16 layers with 65 536 x 2560, 170 MiB, 85, 104, 129, 173, 257 and 88, 108, 135, 178, 262; with 249 MiB 0 to 2 %
+// apart).  The choice stands outside the loops: at every load it cost those heads 1 to 2 %.
+template <int W>
+__device__ __forceinline__ void head_tile_issue(const u8* __restrict__ w, u32 rows, u32 rb, u32 t, u32 lds, u32 wave, u32 lane) {
+    if ((u64) rows * rb >= 256u << 20) head_tile_rows<W, true>(w, rows, rb, t, lds, wave, lane);
+    else head_tile_rows<W, false>(w, rows, rb, t, lds, wave, lane);
 }
 
 // W waves (4, 6 or 8), cols = CMAX (512 W unless a narrower row is given more waves) at most and a multiple of 64 W.

@@ -755,3 +755,30 @@ def test_large_projections_for_more_than_four_inputs(gpu, cols, rows):  # noqa: 
     assert np.isfinite(few).all() and (np.abs(few).max(axis=1) > 0).all()
     for m in (5, 8):
         assert np.array_equal(bits(cols_call(gpu, sz.EXL3(2), dw, cols, rows, x[:m])), bits(few[:m])), m
+
+
+@pytest.mark.parametrize("hidden,over", [(1024, 246724), (2048, 123362), (4096, 61681)])
+@pytest.mark.parametrize("m", [1, 8])
+def test_a_q8_0_head_about_as_large_as_the_last_level(gpu, hidden, over, m):  # noqa: F811
+    """256 MiB, from where on a head is read past the caches, and a row less, which is not: the logits' bits are those of the head's two parts, and the ids
+    their arg-max."""
+    x = gpu.randn((m, hidden), device="cuda", generator=gpu.Generator(device="cuda").manual_seed(hidden))
+    w = synth_device.q8_0_head(gpu, hidden, over, hidden)
+    rb = hidden // 32 * 34
+    assert over * rb >= 256 << 20 > (over - 1) * rb
+
+    def logits(first, rows):
+        s = sz.Session(hidden, 256, 8, 2, 0, rows, 8)
+        s.set_head(sz.Q8_0, w.data_ptr() + first * rb)
+        out, ids = gpu.full((m, rows), float("nan"), device="cuda"), gpu.zeros(m, dtype=gpu.int32, device="cuda")
+        s.head_logits(m, x.data_ptr(), out.data_ptr())
+        s.head_argmax(m, x.data_ptr(), ids.data_ptr())
+        gpu.cuda.synchronize()
+        assert gpu.equal(out.argmax(dim=1).int(), ids)
+        return out
+
+    cut = over // 2 // 16 * 16                               # 16-byte aligned, as a head has to be
+    parts = gpu.cat([logits(0, cut), logits(cut, over - cut)], dim=1)
+    assert gpu.isfinite(parts).all()
+    for rows in (over, over - 1):
+        assert gpu.equal(logits(0, rows), parts[:, :rows]), rows
