@@ -119,8 +119,7 @@ struct DevBuf {
 // 768 (top-8) and 32 of 1536 (top-4), and rounds of 4 and 16 of them: this choice is within 1.5 % of the best (at 8 rows of 4
 // layers of 512: 3 %).  E.g. 4 layers alone at 1, 4 and 8 rows of 512 experts: 97, 167 and 289 us with 2, 115, 172 and 274 with 4,
 // 162, 204 and 282 with 8, 97, 166 and 272 here; a round of 16 at 8 rows 734, 658, 617, 617 here; of 32 experts of 1536 1418,
-// 1214, 1100, 1095 here.  A projection alone (EXL3 at 4 bits) wants 2 tiles up to 8192 x 2048; at 8 inputs of 16384 x 4096 or 32768
-// x 2048 4 tiles would take 22 us a call where this takes 26.
+// 1214, 1100, 1095 here.  A projection alone for more than four inputs: cols_variant.
 static const char* verify_variant(uint64_t cols, uint64_t waves8, uint32_t m, uint32_t* ct) {
     *ct = cols % 512 == 0 && waves8 >= 8192 ? 8 : cols % 256 == 0 && waves8 >= 2048 ? 4 : 2;
     if (m > 4) return *ct == 8 ? "w_" : *ct == 4 ? "t4w_" : "t2w_";
@@ -145,15 +144,30 @@ static uint32_t gguf_waves(uint64_t cols) {
 }
 static uint32_t gguf_lds(uint32_t waves, uint32_t tiles, uint32_t ng) { return waves * (1584 * 4 + tiles * ng * 64 * 4); }
 
-// The column tiles of a projection alone, by its w blocks of 128 columns and 512 inputs.  For more than four inputs: a launch of two tiles a wave has w workgroups,
-// of four w / 2, of eight w / 4; two share a compute unit, so 512 run at once, and a few left over cost as much as 512.  us a call of 8
-// inputs at 4 bits by two, four and eight tiles: w = 768 19.3, 20.9, 22.9; 896 24.0, 21.3, 23.3; 1024 23.9, 21.8, 23.5; 1152 27.9, 27.1, 31.3 (5 inputs at
-// 2 bits 22.6, 23.7, 28.7); 1280 28.7, 27.5, 31.7; 1536 32.9, 28.8, 32.3; 1792 37.0, 35.6, 33.2; 2048 40.6, 36.1, 33.3; 2304 45.5, 42.0, 42.9; 3072
-// 58.2, 49.3, 44.8; 4096 73.8, 59.7, 53.0.  Above 5 bits one tile where its 2 w workgroups do not outnumber the compute units (EXL3_COLS_NARROW_ENTRIES).
+// The column tiles of a projection alone, by its w blocks of 128 columns and 512 inputs.  Up to four inputs as a verify launch's, but above 5 bits
+// one tile where its 2 w workgroups do not outnumber the compute units (EXL3_COLS_NARROW_ENTRIES).
+// For more than four inputs a launch has w workgroups of two tiles a wave, w / 2 of four or w / 4 of eight, and lasts as long as the compute units
+// that have one more than the others: a unit has n2, n4 or n8 of them at most, and twice the tiles cost 1.6 to 1.9 times as much a workgroup.
+// They win where that halves the number, and where it only nearly does the higher the rate and the number of inputs the sooner.  us a call by two, four and eight tiles:
+//   w            768              1024             1280             1792             2048             2816             3584             4224
+//   n2 n4 n8     3 2 1            4 2 1            5 3 2            7 4 2            8 4 2            11 6 3           14 7 4           17 9 5
+//   1 bit,  m 5  16.3 18.3 19.3   19.2 18.9 19.8   22.2 23.8 27.9   28.0 29.1 28.8   30.8 29.7 29.5   40.4 40.2 39.1   49.4 46.2 47.9   57.7 56.1 57.7
+//   2 bits, m 5  16.4 18.4 21.2   19.8 19.3 21.8   23.3 23.9 28.8   29.0 29.0 29.7   32.2 29.8 30.2   42.2 40.5 39.6   51.7 46.7 48.6   60.4 56.6 57.9
+//           m 8  19.4 20.6 22.9   22.9 21.6 23.6   26.9 26.8 31.1   34.3 32.7 32.5   38.8 34.0 33.3   49.7 45.9 43.8   61.0 52.8 53.4   71.3 62.1 62.8
+//   4 bits, m 5  17.4 19.1 21.2   21.5 19.9 21.8   25.1 24.4 29.1   32.1 30.9 30.3   35.9 32.1 30.6   46.5 43.1 40.3   57.5 50.6 51.0   66.9 59.8 59.2
+//           m 8  19.9 21.0 23.0   24.3 22.0 23.5   28.5 27.3 31.5   36.6 35.2 33.0   40.7 36.3 33.5   53.1 48.7 44.3   66.0 56.1 55.4   77.7 64.4 62.8
+//   8 bits, m 8  22.8 22.0 21.3   27.9 22.8 22.0   33.4 31.7 32.5   44.0 39.0 33.7   49.2 40.9 35.5   65.0 56.1 49.9   80.8 67.0 62.0   95.3 77.7 72.6
+// Over all rates, the half ones among them, 5 and 8 inputs and 43 values of w from 512 to 6144 the choice is 0.4 % above the best of the three on the
+// average and nowhere more than 1.5 % above that of a verify launch, which is 5.7 % above the best.
 static const char* cols_variant(const Format& f, uint64_t cols, uint64_t rows, uint32_t m, uint32_t* ct) {
-    const uint64_t w = rows / 128 * exl3_ksplit((uint32_t) cols);
-    if (m > 4 && rows % 512 == 0 && ((w >= 1792 && w <= 2048) || w >= 2816)) { *ct = 8; return "w_"; }
-    if (m > 4 && rows % 256 == 0 && ((w > 768 && w <= 1024) || w >= 1280)) { *ct = 4; return "t4w_"; }
+    const uint64_t w = rows / 128 * exl3_ksplit((uint32_t) cols), n2 = (w + 255) / 256, n4 = (w + 511) / 512, n8 = (w + 1023) / 1024;
+    if (m > 4 && w > 768) {
+        const bool low = f.bits < 3;
+        const bool eight = w >= 2816 && (f.bits >= 5 || (m > 6 && !low));
+        if (rows % 512 == 0 && (eight || (n4 == 2 * n8 && (n8 > 2 || (n8 == 2 && (m > 6 || !low)))))) { *ct = 8; return "w_"; }
+        const uint64_t four = !low ? 1280 : f.bits == 1 && !f.half ? 2048 : 1281;
+        if (rows % 256 == 0 && (n2 == 2 * n4 || w >= four)) { *ct = 4; return "t4w_"; }
+    }
     if (!f.half && f.bits >= 6 && cols % 256 == 0 && w <= 128) { *ct = 1; return m > 4 ? "t1w_" : "t1_"; }
     return verify_variant(rows, w, m, ct);
 }

@@ -190,3 +190,25 @@ sz.matvec_cols({ty}, 256, 0, 100, 512, 0, 1024, 128, 3, 0, 0, 16)
 got = taken()
 assert [g[0] for g in got] == ["matvec_q8_0"] * 3 and [g[2][2:] for g in got] == [[1024 + 512 * j, 100, 0] for j in range(3)], got
 """)
+
+
+# bits (0.5 more: a half rate), inputs, columns, rows, the tiles a wave that are within 1.5 % of the fastest there
+TILES = [(1, 5, 4096, 20480, 2), (1, 8, 2048, 40960, 2), (2, 5, 4096, 20480, 2), (2.5, 5, 2048, 40960, 2), (3, 5, 4096, 20480, 4), (4, 8, 2048, 40960, 4),
+         (4, 5, 2048, 24576, 2), (1, 5, 4096, 14336, 4), (6, 8, 2048, 32768, 4), (4, 5, 4096, 18432, 2), (1, 5, 4096, 28672, 2), (2, 8, 4096, 28672, 8), (4, 5, 4096, 28672, 8),
+         (2, 5, 2048, 65536, 4), (2, 8, 2048, 65536, 8), (4, 5, 8192, 16384, 8), (3, 8, 4096, 36864, 4), (1, 5, 8192, 22528, 8), (1, 5, 8192, 28672, 4), (4, 5, 8192, 28672, 4),
+         (6, 5, 8192, 28672, 8), (4, 8, 4096, 67584, 8), (2, 5, 4096, 67584, 4), (4, 5, 8192, 32768, 8), (4, 8, 4096, 16512, 2), (4, 8, 2048, 65792, 4),
+         (6, 8, 2048, 4096, 1), (6, 4, 2048, 4096, 1), (6, 8, 640, 4096, 2), (3.5, 8, 2048, 4096, 2), (4, 4, 4096, 20480, 2), (4, 1, 8192, 32768, 4)]
+
+
+def test_the_tiles_of_a_projection(stub):
+    """At the edges of the rule: what a call launches is what was fastest there."""
+    stub(f"""
+for bits, m, cols, rows, want in {TILES}:
+    half, kb = bits % 1 > 0, int(bits)
+    ty = sz.EXL3_HALF(kb) if half else sz.EXL3(kb)
+    sz.matvec_cols(ty, 256, cols, rows, 512, cols, 1024, rows, m, 4096, sz.matvec_cols_scratch(ty, cols, rows, m), 16)
+    (name, shape, _), finish = taken()
+    kind = {{8: "", 4: "t4", 2: "t2", 1: "t1"}}[want] + ("w_" if m > 4 else "" if want == 8 else "_")
+    assert name == "matvec_grouped_" + kind + ("exl3h_" if half else "exl3_") + str(kb), (bits, m, cols, rows, name)
+    assert shape[:3] == (rows // (64 * want), -(-cols // 512), 1) and finish[0] == "exl3_finish_rows", (bits, m, cols, rows, shape)
+""")
