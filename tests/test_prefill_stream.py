@@ -1,5 +1,5 @@
-"""The order of requests, waits and reads of the EXL3 prefill chunk's product streams, on the CPU: xpf_stream's own source, compiled for the
-host with its loads, waits and LDS reads replaced by checks."""
+"""The order of requests, waits and reads of the EXL3 prefill chunk's product streams, on the CPU: the streams' own source, compiled for the
+host with their loads, waits and LDS reads replaced by checks, in the forms that the gate and up kernel instantiates."""
 import os
 import re
 import subprocess
@@ -70,77 +70,84 @@ template <int K, int CT, int NT> struct XpfStep {
 };
 %(stream)s
 
-template <int K, int NT, int NB, int NW, int D> static void stream(const char* name) {
-    typedef Ring<D, (2 * K + 3) / 4> R;
+template <int K, int NT, int NCB> static void stream(const char* name) {
+    constexpr int CT = NCB == 2 ? 4 : 2, WAVES = 4;                      // column tiles a wave, waves a projection
+    typedef Ring<%(depth)s, (4 * CT * 2 * K + 63) / 64> R;               // a tile is 2 K times 16 bytes, a load 64 times
+    constexpr int NB = %(slots)s;
+    // bytes of LDS: the slots of two projections' operand rows and the waves' rings
+    static_assert(NB * 2 * NT * 2048 + 2 * WAVES * R::D * 4 * CT * 32 * K <= (NCB == 2 ? 156 : 80) * 1024, "LDS");
     static u16 src[64 * 8 * 1024], rows[9 * 2 * 8 * 1024];
     static u32 wb[16 * 64];
     for (u32 n : {4u, 8u, 12u, 16u, 64u})
         for (u32 t = NT <= 2 ? NT : NT - 1; t <= (u32) NT; t++)
-            for (u32 p = 0; p < (u32) NW; p++) {
+            for (u32 p = 0; p < (u32) WAVES; p++) {
                 issued = landed = 0;
                 trellis.clear();
                 operands.clear();
-                what = name, units = n, tiles = t, part = p, parts = NW, step = 0, slot_halves = 2 * NT * XPF_HALF_U16, source = src, lds_rows = rows, lds_words = wb;
-                f32x4 acc[NT][4];
+                what = name, units = n, tiles = t, part = p, parts = WAVES, step = 0, slot_halves = 2 * NT * XPF_HALF_U16, source = src, lds_rows = rows, lds_words = wb;
+                f32x4 acc[NT][CT];
                 R ring;
                 ring.units = n;
-                xpf_stream<K, NT, NB, NW>(ring, wb, src, rows, slot_halves, t, p, 0u, acc);
+                if constexpr (NCB == 2) %(wide)s(ring, wb, src, rows, slot_halves, t, p, 0u, acc);
+                else %(narrow)s(ring, wb, src, rows, slot_halves, t, p, 0u, acc);
                 check(step == 2 * n, "the stream ended early");
                 check(landed == issued, "loads in flight at the end");
             }
 }
-template <int K, int NT> static void both() {
-    if constexpr (NT <= XPF_NT(K)) {
-        stream<K, NT, 3, 4, XPF_RING(K)>("eight waves");
-        if constexpr (NT <= XPF_NT_N) stream<K, NT, XPF_RING_N(K, NT) + 1, 2, XPF_RING_N(K, NT)>("four waves");
-    }
+template <int K, int NT> static void tiles_of() {
+    if constexpr (NCB_ == 2 && NT <= XPF_NT(K)) stream<K, NT, 2>("two blocks");
+    if constexpr (NCB_ == 1 && NT <= XPF_NT_N) stream<K, NT, 1>("one block");
 }
-template <int K> static void rate() { both<K, 1>(); both<K, 2>(); both<K, 4>(); both<K, 6>(); both<K, 8>(); }
+template <int K> static void rate() { tiles_of<K, 1>(); tiles_of<K, 2>(); tiles_of<K, 4>(); tiles_of<K, 6>(); tiles_of<K, 8>(); }
 int main() { rate<1>(); rate<2>(); rate<3>(); rate<4>(); rate<5>(); rate<6>(); rate<7>(); rate<8>(); }
 """
 
 
-def test_prefill_streams_stay_inside_their_item_and_wait_for_what_they_read(tmp_path):
-    """Every bit rate, number of token tiles and shape of the gate and up launch, from the shortest stream (hidden = 256: shorter than the
-    ring of four waves) on: no request past the stream's end, no slot filled before it was read, no read before it has landed."""
+def run_streams(tmp_path, blocks):
     src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
-    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_N", "XPF_HALF_U16"))
-    start = src.index("template <int K, int NT, int NB, int NW, class R>")
-    stream = src[start:src.index("\n}\n", start) + 3]
+    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_W", "XPF_RING_N", "XPF_HALF_U16"))
+    kernel = src[src.index("void prefill_gate_up_exl3_kernel("):]
+
+    def of_kernel(pattern):
+        return re.search(pattern, kernel[:kernel.index("\n}\n")]).group(1)
+
+    def function(head):
+        start = src.index(head)
+        return src[start:src.index("\n}\n", start) + 3]
+
+    fills = {"macros": f"#define NCB_ {blocks}\n" + macros, "stream": function("template <int K, int NT, int NB, int NW, class R>") + function("template <int K, int NT, int NB, class R>"),
+             "depth": of_kernel(r"typedef VerifyRing<K, false, CT, (.*), 4 \* CT, false> R;"), "slots": of_kernel(r"constexpr int NB = (.*);"),
+             "wide": of_kernel(r"if constexpr \(NCB == 2\) (xpf_stream<.*>)\(ring"), "narrow": of_kernel(r"else (xpf_stream_n<.*>)\(ring")}
+    assert of_kernel(r"constexpr int CT = (.*);") == "NCB == 2 ? 4 : 2"
     path = tmp_path / "stream.cpp"
-    path.write_text(HARNESS % {"macros": macros, "stream": stream})
+    path.write_text(HARNESS % fills)
     subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
     r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_prefill_streams_stay_inside_their_item_and_wait_for_what_they_read(tmp_path):
+    """Every bit rate and number of token tiles of the workgroups of two 128-blocks, from the shortest stream (hidden = 256: shorter than most
+    rings) on: no request past the stream's end, no slot filled before it was read, no read before it has landed, and rings that a compute unit's
+    LDS has room for."""
+    run_streams(tmp_path, 2)
 
 
 def test_prefill_streams_of_eight_waves_as_deep_as_their_tiles_leave_room(tmp_path):
-    """The same for the rings of workgroups of eight waves: the fewer the tiles the deeper, and within a compute unit's LDS."""
+    """The rings of up to four tiles: the fewer the tiles the deeper, at most 8 units, and one unit more would not fit."""
     src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
-    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_W", "XPF_RING_N", "XPF_HALF_U16"))
-    start = src.index("template <int K, int NT, int NB, int NW, class R>")
-    stream = src[start:src.index("\n}\n", start) + 3]
-    of_four, of_eight = "stream<K, NT, 3, 4, XPF_RING(K)>", "stream<K, NT, NT >= 6 ? 3 : XPF_RING_W(K, NT) + 1, 4, XPF_RING_W(K, NT)>"
-    room = "static_assert((NT >= 6 ? 3 : XPF_RING_W(K, NT) + 1) * NT + K * XPF_RING_W(K, NT) <= 39, \"LDS\"); "
-    assert of_four in HARNESS
-    path = tmp_path / "stream.cpp"
-    path.write_text(HARNESS.replace(of_four, room + of_eight) % {"macros": macros, "stream": stream})
-    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
-    r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
-    assert r.returncode == 0, r.stdout
+    macros = "\n".join(re.search(r"^#define %s\b.*$" % n, src, re.M).group(0) for n in ("XPF_RING", "XPF_RING_W", "XPF_RING_N"))
+    path = tmp_path / "rings.cpp"
+    path.write_text("#include <cstdio>\n" + macros + "\nint main() { for (int k = 1; k <= 8; k++) for (int nt = 1; nt <= 4; nt *= 2) printf(\"%d %d %d %d\\n\", k, nt, XPF_RING_W(k, nt), XPF_RING_N(k, nt)); }\n")
+    subprocess.run(["g++", "-o", tmp_path / "rings", path], check=True)
+    rings = {tuple(map(int, line.split()[:2])): tuple(map(int, line.split()[2:])) for line in subprocess.run([tmp_path / "rings"], capture_output=True, text=True).stdout.splitlines()}
+    for (k, nt), (two, one) in rings.items():
+        assert 2 <= two <= 8 and 2 <= one <= 8
+        assert two == 8 or (two + 2) * 4096 * nt + 4096 * k * (two + 1) > 156 * 1024
+        assert one == 8 or (one + 2) * 4096 * nt + 2048 * k * (one + 1) > 80 * 1024
+        assert nt == 4 or (two >= rings[k, 2 * nt][0] and one >= rings[k, 2 * nt][1])
 
 
 def test_prefill_streams_of_narrow_waves(tmp_path):
-    """The same for the workgroups of one 128-block, whose waves take 32 columns, four to a projection."""
-    src = open(os.path.join(build.KERNELS, "exl3.hip")).read()
-    macros = "\n".join(re.search(r"^#define %s\b.*$" % re.escape(n), src, re.M).group(0) for n in ("XPF_NT", "XPF_NT_N", "XPF_RING", "XPF_RING_N", "XPF_HALF_U16"))
-    start = src.index("template <int K, int NT, int NB, class R>")
-    stream = src[start:src.index("\n}\n", start) + 3]
-    harness = HARNESS.replace("xpf_stream<K, NT, NB, NW>(", "xpf_stream_n<K, NT, NB>(").replace("f32x4 acc[NT][4];", "f32x4 acc[NT][2];").replace("Ring<D, (2 * K + 3) / 4> R;", "Ring<D, (K + 3) / 4> R;")
-    harness = harness.replace("stream<K, NT, 3, 4, XPF_RING(K)>(\"eight waves\");", "").replace("XPF_RING_N(K, NT) + 1, 2, XPF_RING_N(K, NT)", "XPF_RING_N(K, NT) + 1, 4, XPF_RING_N(K, NT)")
-    assert harness.count("xpf_stream_n<") == 1 and harness.count("eight waves") == 0 and "+ 1, 4, XPF_RING_N" in harness
-    path = tmp_path / "stream.cpp"
-    path.write_text(harness % {"macros": macros, "stream": stream})
-    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-o", tmp_path / "stream", path], check=True)
-    r = subprocess.run([tmp_path / "stream"], capture_output=True, text=True)
-    assert r.returncode == 0, r.stdout
+    """The same for the workgroups of one 128-block, whose waves take 32 columns, four to a projection, and two of which share a unit."""
+    run_streams(tmp_path, 1)
