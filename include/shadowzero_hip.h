@@ -284,12 +284,12 @@ int32_t sz_hc_write(uint64_t r, uint64_t g, uint64_t y, uint32_t m, uint32_t hid
 /* Per-32 int8 activations: q[n], d[n/32] with d = amax/127, q = round-half-away(v/d) (cpu_expert_avx512.rs:25-42). */
 int32_t sz_quantize_act(uint64_t x_f32, uint64_t n, uint64_t q_i8, uint64_t d_f32, uint64_t stream);
 /* One prefill chunk through layer l (IQ3_S experts): tokens x[t][hidden] f32, routing from rl[t][n_expert], tokens grouped by
- * expert, int8 MFMA products, SwiGLU, int8 H, down, weighted combine in rank order (+ the shared expert gated by sgl[t])
+ * expert, exact products of the int8 codes on the f16 matrix cores, SwiGLU, int8 codes of H, down, weighted combine in rank order (+ the shared expert gated by sgl[t])
  * into y[t][hidden]. */
 int32_t sz_moe_prefill_chunk(sz_session*, uint32_t layer, uint32_t tokens, uint64_t x, uint64_t rl, uint64_t sgl, uint64_t y, uint64_t stream);
 /* The last chunk's intermediate device buffers, for parity tests: 0 xq int8[t][hidden], 1 xd f32[t][hidden/32], 2 tidx u32[t][k],
  * 3 w f32[t][k], 4 hq int8[pair][ff], 5 hd f32[pair][ff/32], 6 eo f32[pair][hidden] (pair = token * k + rank, then the shared
- * expert's t rows).  0 when nothing has run. */
+ * expert's t rows), 7 xh and 8 hh, the codes of 0 and 4 times 2^-6 as f16, which the products read.  0 when nothing has run. */
 uint64_t sz_prefill_buffer(sz_session*, int32_t which);
 
 /* ---- B5: the checkpoint formats either side of the path (host code; no GPU is needed up to the two staging calls) ---- */

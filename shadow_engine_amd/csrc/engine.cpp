@@ -1450,12 +1450,12 @@ int32_t sz_moe_prefill_chunk(sz_session* s, uint32_t l, uint32_t tokens, uint64_
 }
 
 // The chunk's intermediate buffers, for tests: which = 0 xq (int8), 1 xd (f32), 2 tidx (u32), 3 w (f32), 4 hq (int8), 5 hd (f32),
-// 6 eo (f32).  Returns the device address (0 if the session has not run a chunk).
+// 6 eo (f32), 7 xh and 8 hh (f16, the codes the products read).  Returns the device address (0 if the session has not run a chunk).
 uint64_t sz_prefill_buffer(sz_session* s, int32_t which) {
     if (!s) return 0;
     auto& pb = s->pf;
-    const uint64_t ptrs[] = {pb.xq.ptr, pb.xd.ptr, pb.tidx.ptr, pb.w.ptr, pb.hq.ptr, pb.hd.ptr, pb.eo.ptr};
-    return which >= 0 && which < 7 ? ptrs[which] : 0;
+    const uint64_t ptrs[] = {pb.xq.ptr, pb.xd.ptr, pb.tidx.ptr, pb.w.ptr, pb.hq.ptr, pb.hd.ptr, pb.eo.ptr, pb.xh.ptr, pb.hh.ptr};
+    return which >= 0 && which < (int32_t) (sizeof ptrs / sizeof ptrs[0]) ? ptrs[which] : 0;
 }
 
 }   // extern "C"

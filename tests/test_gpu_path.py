@@ -1276,11 +1276,11 @@ def test_activation_quantization_on_the_gpu_is_bit_exact(gpu):
 @pytest.mark.parametrize("tokens,hidden,ff,ne,k,shared,skew", [(48, 512, 256, 16, 4, True, True), (130, 256, 256, 8, 3, False, True),
                                                                  (5, 2048, 512, 40, 10, True, False)])
 def test_prefill_chunk_matches_the_int8_oracle(gpu, tokens, hidden, ff, ne, k, shared, skew):
-    """Routing ids and the int8 codes of the input activations bit-exact; the layer output within 1e-3 relative L2 of the oracle
-    that runs the same int8 arithmetic (cpu_expert.rs:243-339 with per-32 activation blocks).  The codes of H = silu(gate) * up,
-    quantized again between the two products, are held to a relaxed bar on purpose: at most 1e-3 of them may differ from the
-    oracle's (by one step each), because the device's expf and the fused multiply-add that folds a sub-block's int32 sum into
-    the f32 total leave H a last bit or two away from the oracle's, which now and then crosses a rounding boundary."""
+    """Routing ids and the int8 codes of the input activations bit-exact, as bytes and as the f16 values that the products read; the layer
+    output within 1e-3 relative L2 of the oracle that runs the same int8 arithmetic (cpu_expert.rs:243-339 with per-32 activation blocks).
+    The codes of H = silu(gate) * up, quantized again between the two products, are held to a relaxed bar on purpose: at most 1e-3 of them
+    may differ from the oracle's (by one step each), because the device's expf and the order in which a sub-block's exact sum and its
+    scales are folded into the f32 total leave H a last bit or two away from the oracle's, which now and then crosses a rounding boundary."""
     rng = np.random.default_rng(tokens * 3 + ne)
     ty = sz.IQ3_S
     dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, shared)
@@ -1303,7 +1303,12 @@ def test_prefill_chunk_matches_the_int8_oracle(gpu, tokens, hidden, ff, ne, k, s
     tidx = fetch(2, np.uint32, tokens * k).reshape(tokens, k)
     xq = fetch(0, np.int8, tokens * hidden).reshape(tokens, hidden)
     xd = fetch(1, np.float32, tokens * hidden // 32).reshape(tokens, hidden // 32)
-    hq = fetch(4, np.int8, tokens * k * ff).reshape(tokens, k, ff)
+    pairs = tokens * k + (tokens if shared else 0)
+    hq = fetch(4, np.int8, pairs * ff).reshape(pairs, ff)
+    # what the products read: the same codes times 2^-6 in f16, exactly
+    assert np.array_equal(fetch(7, np.float16, xq.size).astype(np.float32).reshape(xq.shape) * 64, xq)
+    assert np.array_equal(fetch(8, np.float16, hq.size).astype(np.float32).reshape(hq.shape) * 64, hq)
+    hq = hq[:tokens * k].reshape(tokens, k, ff)
     code_total = code_diff = 0
     for j in range(tokens):
         oi, ow = O.route(logits[j], k)
@@ -1368,6 +1373,9 @@ def test_config4_prefill_chunk_full_size(gpu):
     sz.check(sz.lib().sz_download(xq.ctypes.data, s.prefill_buffer(0), xq.nbytes))
     wq_all, wd_all, _ = O.quantize_act(x, 32)
     assert np.array_equal(xq.ravel(), wq_all)
+    xh = np.empty((tokens, hidden), np.float16)
+    sz.check(sz.lib().sz_download(xh.ctypes.data, s.prefill_buffer(7), xh.nbytes))
+    assert np.array_equal(xh.astype(np.float32).ravel() * 64, wq_all)
     wts = np.empty((tokens, k), np.float32)
     sz.check(sz.lib().sz_download(wts.ctypes.data, s.prefill_buffer(3), wts.nbytes))
     for j in range(tokens):

@@ -743,18 +743,105 @@ def cols_call(gpu, ty, dw, cols, rows, x):  # noqa: F811
     return y.cpu().numpy()
 
 
+def exl3_columns(w, cols, rows, kb, at):
+    """The blob of the 128 outputs from `at` on of an EXL3 matrix (host bytes): their scales and, of every 16 inputs, their eight tiles."""
+    tiles = w[2 * (cols + rows) + 4:].reshape(cols // 16, rows // 16, 32 * kb)[:, at // 16:at // 16 + 8]
+    return np.concatenate([w[:2 * cols], w[2 * (cols + at):2 * (cols + at + 128)], w[2 * (cols + rows):2 * (cols + rows) + 4], tiles.ravel()])
+
+
+@pytest.mark.parametrize("kb", [2, 6])
 @pytest.mark.parametrize("cols,rows", [(2048, 24576), (2048, 24704), (2048, 25088), (4096, 16384), (4096, 16512), (4096, 20480), (4096, 28672), (4096, 32768), (4096, 33280), (8192, 22528)])
-def test_large_projections_for_more_than_four_inputs(gpu, cols, rows):  # noqa: F811
+def test_large_projections_for_more_than_four_inputs(gpu, cols, rows, kb):  # noqa: F811
     """The sizes at which a projection's tile count changes for more than four inputs, and rows that fill no wider workgroup: a row's bits are those of the calls
-    of up to four, which choose by another rule; a sample of the outputs in the magnitude of the inputs."""
+    of up to four, which choose by another rule; the first, a middle and the last block of 128 outputs are the oracle's, at a rate whose weights take one window and at
+    one of two."""
     g = gpu.Generator(device="cuda")
     g.manual_seed(cols + rows)
-    dw = synth_device.exl3_matrix(gpu, cols + rows, cols, rows, 2)
+    ty, dw = sz.EXL3(kb), synth_device.exl3_matrix(gpu, cols + rows, cols, rows, kb)
     x = gpu.randn((8, cols), device="cuda", generator=g).cpu().numpy()
-    few = np.concatenate([cols_call(gpu, sz.EXL3(2), dw, cols, rows, x[j:j + 4]) for j in (0, 4)])
+    few = np.concatenate([cols_call(gpu, ty, dw, cols, rows, x[j:j + 4]) for j in (0, 4)])
     assert np.isfinite(few).all() and (np.abs(few).max(axis=1) > 0).all()
     for m in (5, 8):
-        assert np.array_equal(bits(cols_call(gpu, sz.EXL3(2), dw, cols, rows, x[:m])), bits(few[:m])), m
+        assert np.array_equal(bits(cols_call(gpu, ty, dw, cols, rows, x[:m])), bits(few[:m])), m
+    w = dw.cpu().numpy()
+    for at in (0, rows // 256 * 128, rows - 128):
+        block = exl3_columns(w, cols, rows, kb, at)
+        for j in (0, 7):
+            assert rel_l2(few[j, at:at + 128], O.exl3_matvec(cols, 128, kb, block, x[j])) <= 2e-6, (at, j)
+
+
+DOWN_FORMS = {4: (("t2_", 2), ("t4_", 4), ("", 8)), 8: (("t2w_", 2), ("t4w_", 4), ("w_", 8))}
+
+
+@pytest.mark.parametrize("kb,half", [(k, False) for k in range(1, 9)] + [(k, True) for k in range(1, 4)])
+@pytest.mark.parametrize("hidden,m", [(2560, 4), (4608, 8), (4608, 3), (2560, 6)])
+def test_every_form_of_the_down_launch_of_more_than_four_partials(gpu, kb, half, hidden, m):  # noqa: F811
+    """Gate and up sums of 5 and 9 partials through the kernels that ask for eight at once and those that ask for four, every tile count, launched by name on what
+    a layer's call left behind (its plan and its sums): the same additions in the same order, so the same bits, in every pair's row.  The
+    layer's own output is the oracle's."""
+    rng = np.random.default_rng(100 * kb + hidden + m + half)
+    ff, ne, k = 768, 6, 3
+    ty = sz.EXL3_HALF(kb) if half else sz.EXL3(kb)
+    tag = ("exl3h_%d" if half else "exl3_%d") % kb
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, True)
+    s = sz.Session(hidden, ff, ne, k, 1, 0, 8)
+    shared = dbuf.data_ptr() + ne * stride
+    s.set_layer(0, ty, dbuf.data_ptr(), stride, ty, shared)
+    u, rl, sgl = rng.normal(size=(m, hidden)).astype(np.float32), rng.normal(size=(m, ne)).astype(np.float32), rng.normal(size=m).astype(np.float32)
+    du, drl, dsgl, y = dev(gpu, u), dev(gpu, rl), dev(gpu, sgl), gpu.zeros((m, hidden), dtype=gpu.float32, device="cuda")
+    sz.ktime_begin("verify_")
+    s.moe_layer_verify(0, m, du.data_ptr(), drl.data_ptr(), dsgl.data_ptr(), y.data_ptr())
+    gpu.cuda.synchronize()
+    names = sz.ktime_end()
+    assert "verify_plan_exl3" in names and "verify_down_x_" + ("t2w_" if m > 4 else "t2_") + tag in names, names
+    want, _, _ = oracle_layer(ty, hidden, ff, k, blobs, sh, rl, sgl, u)
+    assert all(rel_l2(y[j].cpu().numpy(), want[j]) <= 2e-6 for j in range(m))
+
+    plan, sums = sz.lib().sz_session_buffer(s._h, 0), sz.lib().sz_session_buffer(s._h, 1)
+    zd, part = -(-ff // 512), synth.expert_bytes(ty, hidden, ff)[0]
+    ioff = -(-(2 * m * k * 4 + m * 4) // 16) * 16              # the items behind [ids | weights | counts]
+    P, U, U64 = sz.Arg.ptr, sz.Arg.u32, sz.Arg.u64
+    first = None
+    for kind in ("verify_down_", "verify_down_x_"):
+        for form, ct in DOWN_FORMS[8 if m > 4 else 4]:
+            dn = gpu.full((m * (k + 1), zd, hidden), float("nan"), dtype=gpu.float32, device="cuda")
+            sz.launch(kind + form + tag, (hidden // (64 * ct), m * k + 2, zd), (256, 1, 1), 0, 0,
+                      [P(drl.data_ptr()), P(0), U64(dbuf.data_ptr()), U64(stride), U64(shared), U(part), U(0), P(plan), P(plan), U(0), U(ioff), P(sums), P(dn.data_ptr()),
+                       U(ne), U(k), U(m), U(hidden), U(ff)])
+            gpu.cuda.synchronize()
+            got = bits(dn.cpu().numpy())
+            first = got if first is None else first
+            assert np.isfinite(dn.cpu().numpy()).all() and np.array_equal(got, first), (kind, form)
+
+
+@pytest.mark.parametrize("ty", [sz.EXL3(3), sz.EXL3_HALF(2)])
+@pytest.mark.parametrize("m,L,form", [(4, 8, "t4_"), (4, 32, ""), (8, 4, "t4w_"), (8, 16, "w_")])
+def test_rounds_of_more_than_four_partials_take_wider_tiles(gpu, ty, m, L, form):  # noqa: F811
+    """Layers of 2560 inputs, one run as a round's launch takes them: enough workgroups for 4 and 8 column tiles a wave of the down products.  A sample
+    of the layers with the oracle."""
+    rng = np.random.default_rng(m + L)
+    hidden, ff, ne, k = 2560, 256, 6, 3
+    s = sz.Session(hidden, ff, ne, k, L, 1024, 8)
+    s.set_graph(False)
+    dbuf, stride, blobs, sh = build_layer(gpu, rng, ty, hidden, ff, ne, True)      # the layers differ by their inputs
+    for l in range(L):
+        s.set_layer(l, ty, dbuf.data_ptr(), stride, ty, dbuf.data_ptr() + ne * stride)
+    dhead = dev(gpu, synth.q8_0_matrix(rng, 1024, hidden))
+    s.set_head(sz.Q8_0, dhead.data_ptr())
+    u, rl = rng.normal(size=(L, m, hidden)).astype(np.float32), rng.normal(size=(L, m, ne)).astype(np.float32)
+    sgl, hu = rng.normal(size=(L, m)).astype(np.float32), rng.normal(size=(m, hidden)).astype(np.float32)
+    du, drl, dsgl, dhu = dev(gpu, u), dev(gpu, rl), dev(gpu, sgl), dev(gpu, hu)
+    y = gpu.zeros((L, m, hidden), dtype=gpu.float32, device="cuda")
+    drafts, out = gpu.zeros(8, dtype=gpu.int32, device="cuda"), gpu.zeros(10, dtype=gpu.int32, device="cuda")
+    sz.ktime_begin("verify_down_")
+    s.verify_round(m, du.data_ptr(), drl.data_ptr(), dsgl.data_ptr(), y.data_ptr(), dhu.data_ptr(), drafts.data_ptr(), out.data_ptr())
+    gpu.cuda.synchronize()
+    names = sz.ktime_end()
+    assert list(names) == ["verify_down_x_" + form + ("exl3h_2" if ty == sz.EXL3_HALF(2) else "exl3_3")], names
+    got = y.cpu().numpy()
+    for l in (0, L // 2, L - 1):
+        want, _, _ = oracle_layer(ty, hidden, ff, k, blobs, sh, rl[l], sgl[l], u[l])
+        assert all(rel_l2(got[l, j], want[j]) <= 2e-6 for j in range(m)), l
 
 
 @pytest.mark.parametrize("hidden,over", [(1024, 246724), (2048, 123362), (4096, 61681)])
