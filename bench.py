@@ -236,9 +236,9 @@ def iq3s_prefill(torch, sz, synth, synth_device, stream, tokens=512):
     distinct = int(np.unique(ids).size)
     gu, _, dn = synth.expert_bytes(sz.IQ3_S, HIDDEN, FF)
     w.step_bytes = distinct * (2 * gu + dn) + tokens * (2 * HIDDEN + NE) * 4
-    # gate/up: the experts' two matrices, the tokens' codes (as f16) and scales in, H's codes (int8 and f16) and scales out; down: the experts' third
+    # gate/up: the experts' two matrices, the tokens' codes (as f16) and scales in, H's codes (as f16) and scales out; down: the experts' third
     # matrix, H in, the pairs' rows of the result out (f32, summed by the combine launch: counted as the EXL3 launches' are)
-    w.kernel_bytes = {"prefill_gate_up_iq3_s": distinct * 2 * gu + tokens * HIDDEN * 17 // 8 + tokens * TOPK * FF * 25 // 8,
+    w.kernel_bytes = {"prefill_gate_up_iq3_s": distinct * 2 * gu + tokens * HIDDEN * 17 // 8 + tokens * TOPK * FF * 17 // 8,
                       "prefill_down_iq3_s": distinct * dn + tokens * TOPK * FF * 17 // 8 + tokens * TOPK * HIDDEN * 4}
     w.kernel_ops = {"prefill_gate_up_iq3_s": 2.0 * tokens * TOPK * 2 * FF * HIDDEN, "prefill_down_iq3_s": 2.0 * tokens * TOPK * FF * HIDDEN}
     w.dtype = "int8 codes as f16 x f16 whole-number weights -> f32 MFMA, f32 scales"
@@ -275,7 +275,7 @@ def exl3_prefill(torch, sz, synth, synth_device, stream, tokens=512, bits=3):
     # rotate: the rows of x in, f16 operand rows of every pair for gate and up out; gate/up: the experts' two matrices and those
     # rows in, down's operand rows out; down: the experts' third matrix and its operand rows in, the pairs' rows of the result out
     w.kernel_bytes = {"prefill_rotate_exl3": tokens * HIDDEN * 4 + pairs * 2 * HIDDEN * 2}
-    for form in ("", "n_"):   # workgroups of eight waves, of four
+    for form in ("", "n_"):   # gate and up: workgroups of two 128-blocks, of one; down: of eight waves, of four
         w.kernel_bytes["prefill_gate_up_%sexl3_%d" % (form, bits)] = distinct * gu + pairs * (2 * HIDDEN + FF) * 2
         w.kernel_bytes["prefill_down_%sexl3_%d" % (form, bits)] = distinct * dn + pairs * FF * 2 + pairs * HIDDEN * 4
     w.dtype = "f32 accumulate over EXL3 f16 codebook weights x f16 activations (matrix cores)"

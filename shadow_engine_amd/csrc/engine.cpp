@@ -797,11 +797,17 @@ int head_check(sz_session* s, uint32_t m, uint64_t u, const char* who) {
 // buffer for them).
 bool head_argmax_fused(const sz_session* s) { return s->head_type == SZ_TYPE_Q8_0 || head_is_exl3(s); }
 
-// The product launch of an EXL3 head over n output blocks (sel: a list of them, 0: all).
+// The product launch of an EXL3 head over n output blocks (sel: a list of them, 0: all).  A head of more than 256 MiB, what the last level holds, is read past
+// the caches (384 MiB at 6 bits, us of a round of 1 and 4 layers for one row 122 -> 118, 135 -> 132; 297 MiB at 4 bits 124 -> 121, 151 -> 149).  A smaller one is there
+// again at the next call, also with layers in between (past the caches rounds of 1, 4 and 16 layers for four rows with 223 MiB 96 -> 102, 134 -> 136, 245 -> 255,
+// with 111 MiB 89 -> 90, 125 -> 127, 231 -> 234, of 48 layers 1 % either way; a call alone with 223 MiB 79 -> 83; one that finds none of its 148 MiB 75.2 -> 74.0).
+// A list's blocks are few.
 int head_exl3_blocks(sz_session* s, uint32_t n, uint32_t m, uint64_t logits, uint32_t ls, uint64_t sel, uint64_t stream) {
     const sz_session_config& c = s->cfg;
     const sz_arg a[] = {P(s->head_w), P(s->head_xa.ptr), P(s->head_inv.ptr), P(logits), U32(ls), P(s->head_part.ptr), U32(c.hidden), U32(c.vocab), U32(m), P(sel)};
-    return launch(("head_exl3_" + std::to_string(s->head_type - 1020)).c_str(), n, 1, 1, 256, 0, stream, a);
+    const uint32_t bits = (uint32_t) s->head_type - 1020;
+    const bool past = !sel && (uint64_t) c.hidden * c.vocab * bits / 8 > 256ull << 20;
+    return launch(((past ? "head_exl3_past_" : "head_exl3_") + std::to_string(bits)).c_str(), n, 1, 1, 256, 0, stream, a);
 }
 
 // An EXL3 head (kernels/exl3.cu:349-461, 610-625 of the reference: rotate the rows once, then one pass over the matrix for all

@@ -238,10 +238,13 @@ __device__ __forceinline__ u64 uniform_u64(u64 v) {
 
 // A wave's stream of trellis rows for CT column tiles: units of UT tiles (UT / CT tile rows, 32 K UT bytes), each brought
 // into one of D ring slots by NI global-to-LDS loads of 16 bytes a lane.  In LDS a unit lies packed in the order of the
-// bit stream: tile row, column tile, tile word.  ONCE: past the caches, for streams that no other workgroup reads (six layers of 512 experts of 2048 x
-// 512, top-10, 4 rows, at 3 bits 250 us, 241; a round of 48 at 2, 3 and 4 bits 906, 901; a projection of 4096 x 2048 for four inputs at 4 bits
-// 9.2, 8.8, of 6144 x 16384 at 3 bits 23.6, 22.7; of 8192 x 32768, with 8 MB of partial sums behind it, 45.4, 46.3).  A prefill chunk's items
-// share their expert's rows (4096 tokens 857 us, past the caches 893).
+// bit stream: tile row, column tile, tile word.  ONCE: past the caches, for trellises that the caches would not have at the next call either, and that push
+// out what the launches share: the experts of a verify layer change with the tokens, and where the pairs are its items at most a fifth of them shares one.
+// Calls with other inputs each time: layers of seven shapes at 2 to 4 bits, 1 to 8 of them alone and rounds of up to 32, 1.5 to 2 % faster whatever
+// they touch, 16 MiB to 4 GiB (six of 512 experts of 2048 x 512, top-10, 4 rows, at 3 bits 250 us, 241; pairs of which 5 to 20 % repeat 1.2 %); where all
+// experts together fit the last level, 256 MB, no slower.  The same inputs again and again, up to what it holds, are 0.7 % slower, at most 4.
+// Projections win either way (4096 x 2048 for four inputs at 4 bits 9.2, 8.8, 6144 x 16384 at 3 bits 23.6, 22.7; 8192 x 32768, with 8 MB of partial
+// sums behind it, 45.4, 46.3).  A prefill chunk's items share their expert's rows (4096 tokens 857 us, past the caches 893).
 template <int K, bool H, int CT, int DEPTH = 0, int UT = 16, bool ONCE = true>
 struct VerifyRing {
     static constexpr int TW = EXL3_TILE_WORDS(K, H), CH = TW / 4;   // words and 16-byte chunks a tile
@@ -1134,9 +1137,11 @@ extern "C" __global__ void __launch_bounds__(1024) exl3_head_rotate(const u8* bl
 // LDS three fitted, 1.55 rounds that took two: 57.8 (8 rows of 4096 inputs: the hand-off of the 64 best 199 -> 132 us).  Tried: a
 // workgroup of 16 waves a compute unit with its A rows in registers, block after block: 57.8 too, the ends of a block are nobody
 // else's time there.
+// ONCE: the trellis past the caches, for a head that the last level cannot hold (head_exl3_blocks has the line).  A kernel of its own: the choice
+// at every unit cost 1 to 2 %.
 // grid = out / 128 (or the list's bound), block 256.
 #define EXL3_HEAD_OCC(K) ((K) <= 5 ? 5 : 3)
-template <int K>
+template <int K, bool ONCE>
 __device__ __forceinline__ void exl3_head_kernel(const u8* __restrict__ blob, const u16* __restrict__ xa, const float* __restrict__ inv,
                                                  float* __restrict__ logits, u32 ls, u32* __restrict__ part, u32 in_f, u32 out_f, u32 m,
                                                  const u32* __restrict__ sel) {
@@ -1161,7 +1166,7 @@ __device__ __forceinline__ void exl3_head_kernel(const u8* __restrict__ blob, co
         const u64 from = base + (u64) (2 * pair) * pitch;
 #pragma unroll
         for (int i = 0; i < R::NI; i++)
-            if (64 * (i + 1) <= 16 * R::CH || 64 * i + lane < 16 * R::CH) lds_load_at<true>(from, ring.off[i], wb_lds + (slot * SLOT + i * 256) * 4);
+            if (64 * (i + 1) <= 16 * R::CH || 64 * i + lane < 16 * R::CH) lds_load_at<ONCE>(from, ring.off[i], wb_lds + (slot * SLOT + i * 256) * 4);
         lds_load<16>((const u8*) xa + (u64) pair * 1024 + lane * 16, wb_lds + (slot * SLOT + R::UW) * 4);
     };
 #pragma unroll
@@ -1399,7 +1404,10 @@ extern "C" __global__ void __launch_bounds__(64) proxy_q2_quant_x(const u8* blob
 
 #define EXL3_HEAD_ENTRIES(K) \
     extern "C" __global__ void __launch_bounds__(256, EXL3_HEAD_OCC(K)) head_exl3_##K(const u8* blob, const u16* xa, const float* inv, float* logits, u32 ls, u32* part, u32 in_f, u32 out_f, u32 m, const u32* sel) { \
-        exl3_head_kernel<K>(blob, xa, inv, logits, ls, part, in_f, out_f, m, sel); \
+        exl3_head_kernel<K, false>(blob, xa, inv, logits, ls, part, in_f, out_f, m, sel); \
+    } \
+    extern "C" __global__ void __launch_bounds__(256, EXL3_HEAD_OCC(K)) head_exl3_past_##K(const u8* blob, const u16* xa, const float* inv, float* logits, u32 ls, u32* part, u32 in_f, u32 out_f, u32 m, const u32* sel) { \
+        exl3_head_kernel<K, true>(blob, xa, inv, logits, ls, part, in_f, out_f, m, sel); \
     } \
     extern "C" __global__ void __launch_bounds__(256) exl3_build_q2_proxy_##K(const u8* blob, u32* w_q2, u16* w_sc, u32 in_f, u32 out_f) { \
         exl3_q2_proxy_build<K>(blob, w_q2, w_sc, in_f, out_f); \
@@ -1791,7 +1799,9 @@ struct XpfStep {
 
 // The products of a wave (64 columns) over the `ring.units` 64-blocks of the inputs.  The operand rows (src: [64-block][tiles], whole
 // item) come through a ring of NB slots of NT tiles in LDS (`stage`, slots `slot_u16` apart) that the NW waves of one projection share, of
-// which this is number `part`: requested NB - 1 units ahead, each wave its share, a barrier a unit.  A step's words and
+// which this is number `part`: requested NB - 1 units ahead, each wave its share, a barrier a unit.  The waits count the loads that every wave makes of a
+// unit: where its operand rows do not divide evenly (one tile: two loads for four waves) a wave that makes one more waits for as many loads as units are in
+// flight sooner than it would have to, and the others with it at the barrier.  A step's words and
 // operand rows are read while the one before is multiplied. The whole workgroup calls this with the same number of units.  D + 1 >= NB.
 template <int K, int NT, int NB, int NW, class R>
 __device__ __forceinline__ void xpf_stream(const R& ring, const u32* wb, const u16* __restrict__ src, u16* stage, u32 slot_u16, u32 tiles, u32 part, u32 lane,

@@ -869,3 +869,35 @@ def test_a_q8_0_head_about_as_large_as_the_last_level(gpu, hidden, over, m):  # 
     assert gpu.isfinite(parts).all()
     for rows in (over, over - 1):
         assert gpu.equal(logits(0, rows), parts[:, :rows]), rows
+
+
+@pytest.mark.parametrize("kb,hidden,blocks", [(3, 2048, 2731), (4, 2048, 2049), (8, 4096, 513)])
+def test_an_exl3_head_about_as_large_as_the_last_level(gpu, kb, hidden, blocks):  # noqa: F811
+    """A head just above 256 MiB, which is read past the caches, and one of the same blocks but the last, which is not: the same bits and ids; the last
+    block is the oracle's."""
+    m, rows = 5, 128 * blocks
+    assert hidden * rows * kb // 8 > 256 << 20 >= hidden * (rows - 128) * kb // 8
+    blob = synth_device.exl3_matrix(gpu, kb, hidden, rows, kb)
+    x = gpu.randn((m, hidden), device="cuda", generator=gpu.Generator(device="cuda").manual_seed(kb))
+    at, tiles = 2 * (hidden + rows), blob[2 * (hidden + rows) + 4:].view(hidden // 16, rows // 16, 32 * kb)
+    smaller = gpu.cat([blob[:at - 256], blob[at:at + 4], tiles[:, :rows // 16 - 8].reshape(-1)])
+
+    def run(w, n):
+        s = sz.Session(hidden, 256, 8, 2, 0, n, 8)
+        s.set_head(sz.EXL3(kb), w.data_ptr())
+        out, ids = gpu.full((m, n), float("nan"), device="cuda"), gpu.zeros(m, dtype=gpu.int32, device="cuda")
+        sz.ktime_begin("head_exl3_")
+        s.head_logits(m, x.data_ptr(), out.data_ptr())
+        s.head_argmax(m, x.data_ptr(), ids.data_ptr())
+        gpu.cuda.synchronize()
+        names = sz.ktime_end()
+        assert list(names) == ["head_exl3_" + ("past_" if n == rows else "") + str(kb)], names
+        assert gpu.isfinite(out).all() and gpu.equal(out.argmax(dim=1).int(), ids)
+        return out
+
+    whole = run(blob, rows)
+    assert gpu.equal(run(smaller, rows - 128), whole[:, :rows - 128])
+    w = blob.cpu().numpy()
+    last = exl3_columns(w, hidden, rows, kb, rows - 128)
+    for j in (0, m - 1):
+        assert rel_l2(whole[j, rows - 128:].cpu().numpy(), O.exl3_matvec(hidden, 128, kb, last, x[j].cpu().numpy())) <= REL_L2
