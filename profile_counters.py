@@ -47,6 +47,8 @@ NAMES = {"config5": ("verify_round_config5", "the default benchmark workload (co
          "cols-exl3_4-4rows": ("matvec_cols_exl3_k4_4rows", "the case cols-exl3_4-4rows of perf/cases.py (four EXL3 K=4 projections of 4096 x 2048 for 4 inputs a pass)", None),
          "block-q8_0-8rows": ("moe_block_q8_0_8rows", "the case block-q8_0-8rows of perf/cases.py (router and MoE block of four Q8_0 layers for 8 tokens a pass)", None),
          "block-exl3_3-4rows": ("moe_block_exl3_k3_4rows", "the case block-exl3_3-4rows of perf/cases.py (router and MoE block of six EXL3 K=3 layers for 4 tokens a pass)", None),
+         "prefill-exl3_3-45": ("prefill_chunk_exl3_k3_45", "the case prefill-exl3_3-45 of perf/cases.py (a chunk of 45 tokens through 512 EXL3 K=3 experts and the shared one)", None),
+         "prefill-exl3_4-4096": ("prefill_chunk_exl3_k4_4096", "the case prefill-exl3_4-4096 of perf/cases.py (a chunk of 4096 tokens through 512 EXL3 K=4 experts and the shared one)", None),
          "hyper-bf16-4rows": ("hyper_connection_bf16_4rows", "the case hyper-bf16-4rows of perf/cases.py (hyper-connection read and write, BF16, 4 streams of 2048, rank 320, 4 rows)", None)}
 SQ1 = "SQ_INSTS_VALU SQ_ACTIVE_INST_VALU SQ_BUSY_CYCLES SQ_WAVES SQ_WAVE_CYCLES SQ_WAIT_INST_ANY SQ_INSTS_SALU SQ_INSTS_LDS"
 SQ2 = "SQ_INSTS_MFMA SQ_VALU_MFMA_BUSY_CYCLES SQ_LDS_BANK_CONFLICT SQ_ACTIVE_INST_LDS SQ_INSTS_VMEM_RD SQ_WAIT_ANY SQ_ACTIVE_INST_ANY SQ_INSTS_VMEM_WR"

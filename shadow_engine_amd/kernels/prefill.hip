@@ -380,7 +380,7 @@ __device__ __forceinline__ void pf_fold(f32x4 (&total)[T], f32x4 (&acc)[T], cons
 // waits); for three and four the activations come a half block at a time, one ahead, the rows a block ahead.  Two workgroups a
 // compute unit by the stage's LDS.
 //
-// What bounds it: the decode, about 24 vector instructions for a lane's 8 weights, for every item of an expert again, then LDS, busy half the time
+// What bounds it: the decode, about 25 vector instructions for a lane's 8 weights, for every item of an expert again, then LDS, busy half the time
 // (the grid look-ups' bank conflicts), and the waits of items of one tile.  512 tokens through 512 experts of 2048 x 512, top-10, router
 // with Zipf's preferences: gate and up 138 -> 111 us, down 82 -> 61, the chunk 229 -> 169; 4096 tokens and the shared expert 1092 ->
 // 843; 700 through 60 of 4096 x 1536, top-4, 582 -> 418.  Tried: 16 rows of either matrix and half the sub-blocks a wave, which reads
