@@ -1191,7 +1191,7 @@ int32_t sz_head_logits(sz_session* s, uint32_t m, uint64_t u, uint64_t logits, u
 }
 
 // The merge kernel's output goes straight into pinned host memory (device-visible, coherent): once the stream has drained the
-// 2 KiB a row are there, and no copy from device memory (a blocking driver call of its own) is needed.
+// 512 bytes a row are there, and no copy from device memory (a blocking driver call of its own) is needed.
 static int top_finish(sz_session* s, uint32_t m, uint32_t* top_host, uint64_t stream) {
     if (sz_stream_synchronize(stream)) return 1;
     std::memcpy(top_host, s->top_host, (size_t) m * 128 * 4);
